@@ -260,6 +260,7 @@ struct MoveStrided {
   uint32_t dim_s, dim_d;      // the dim each side stores contiguously
   uint32_t tiles_s, tiles_d;  // 64-element tiles along them
   uint64_t count;
+  FastDiv by_shape[MOVE_MAX_RANK];   // by shape[order[o]], for k_move_rows (a tensor has fewer than 2^31 elements)
 };
 
 // Both sides contiguous along the same dim: consecutive threads take consecutive elements of
@@ -270,26 +271,11 @@ __global__ __launch_bounds__(256) void k_move_rows(MoveStrided p) {
   uint32_t rem = uint32_t(i);  // a tensor has fewer than 2^31 elements
   int64_t so = 0, d_o = 0;
   for (int o = int(p.rank) - 1; o >= 0; o--) {
-    const uint32_t d = p.order[o], c = rem % p.shape[d];
-    rem /= p.shape[d];
+    const uint32_t d = p.order[o], rest = p.by_shape[o].div(rem), c = rem - rest * p.shape[d];
+    rem = rest;
     so += int64_t(c) * p.ss[d], d_o += int64_t(c) * p.ds[d];
   }
   store_u32(p.dst, p.ddt, d_o, move_bits(p.src, p.sdt, so, p.ddt));
-}
-
-// The same when nothing is converted and every run along the shared contiguous dim is whole
-// 16-byte vectors on both sides: shapes and strides count vectors.
-__global__ __launch_bounds__(256) void k_move_rows16(MoveStrided p) {
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= p.count) return;
-  uint32_t rem = uint32_t(i);
-  int64_t so = 0, d_o = 0;
-  for (int o = int(p.rank) - 1; o >= 0; o--) {
-    const uint32_t d = p.order[o], c = rem % p.shape[d];
-    rem /= p.shape[d];
-    so += int64_t(c) * p.ss[d], d_o += int64_t(c) * p.ds[d];
-  }
-  MRL_STORE_ONCE(static_cast<const v4u_t *>(p.src)[so], static_cast<v4u_t *>(p.dst) + d_o);
 }
 
 // The two sides are contiguous along different dims: a 64 x 64 tile of (dim_d, dim_s) goes
@@ -591,23 +577,23 @@ __global__ __launch_bounds__(256) void k_move_tiled32(MoveStrided p) {
   }
 }
 
-// Any other pair of contiguous dims (a Packed(8) digit on one side, say, too short for the
-// 64 x 64 transpose): a tile of up to 4096 elements, `ext[d]` along each digit, chosen on the host
-// so that it holds runs of 64 contiguous elements on both sides.  Read in source order into LDS,
-// written in destination order.  Element t of the tile in source order has digit
-// (t / tstride_s[d]) % ext[d] along d, likewise tstride_d in destination order; the divisions are
-// multiplications by precomputed reciprocals (exact for operands below 2^16).
+// A tile of a Move over a common strided view: `ext[d]` elements along each digit, as many tiles along
+// it as `chunks[d]`.  Element t of the tile in source order has digit (t / tstride_s[d]) % ext[d]
+// along d, likewise tstride_d in destination order; the divisions are multiplications by
+// precomputed reciprocals (exact for operands below 2^16).  The digits the tile extends along come
+// first.
 struct MoveTile {
-  MoveStrided m;
+  const void *src;
+  void *dst;
+  int sdt, ddt;
+  uint32_t shape[MOVE_MAX_RANK];
+  int64_t ss[MOVE_MAX_RANK], ds[MOVE_MAX_RANK];
   uint32_t ext[MOVE_MAX_RANK], chunks[MOVE_MAX_RANK];
   uint32_t tstride_s[MOVE_MAX_RANK], tstride_d[MOVE_MAX_RANK];
   uint32_t inv_s[MOVE_MAX_RANK], inv_d[MOVE_MAX_RANK], inv_ext[MOVE_MAX_RANK];  // ceil(2^32 / x)
-  uint32_t tile;  // elements per tile
+  uint32_t tile;  // elements (k_move_runs: vectors) per tile
   FastDiv by_chunks[MOVE_MAX_RANK];   // a block number into tile coordinates without dividing (blocks number below 2^31)
-  // Runs of V > 1 elements per thread: the LDS distance between neighbours along the
-  // destination's fastest digit, and whether whole runs may be loaded / stored as one vector.
-  uint32_t lds_step;
-  bool vec_s, vec_d;
+  uint32_t lds_step[4];  // k_move_gather: where the elements of a destination run of four lie in source order, from its first
 };
 constexpr uint32_t MOVE_TILE_MAX = 4096;
 
@@ -615,97 +601,169 @@ __device__ inline uint32_t div_small(uint32_t n, uint32_t d, uint32_t inv) {
   return d == 1 ? n : __umulhi(n, inv);
 }
 
-// E: the element type when nothing is converted (typed loads and stores), void when the dtypes
-// differ (conversion per element).  Offsets fit 32 bits: a tensor has fewer than 2^31 elements.
-// V: elements per thread and step, a run along the fastest digit of the side being walked (the
-// host picks V > 1 only when those digits, their tile extents and their sizes are multiples of
-// V): one digit extraction serves V elements.
-// NACT: the digits along which the tile extends come first (the host orders them so) and number
-// at most NACT; the per-element digit loops run over exactly those, unrolled, with no test of
-// which digits matter.
-// E void: elements are converted, SSIZE and DSIZE their sizes in bytes on the two sides.
-template <class E, int V, int NACT, int SSIZE = 0, int DSIZE = 0>
-__global__ __launch_bounds__(256) void k_move_gather(MoveTile p) {
-  constexpr bool CONVERT = std::is_void<E>::value;
-  typedef typename std::conditional<CONVERT, uint32_t, E>::type Cell;
-  static_assert(V == 1 || !CONVERT, "runs are for elements that are not converted");
-  typedef Cell Run __attribute__((ext_vector_type(V == 1 ? 2 : V)));  // used only when V > 1
-  __shared__ Cell lds[MOVE_TILE_MAX + MOVE_TILE_MAX / 64];
+// Coordinates of this workgroup's tile: the offsets of its origin on the two sides, and how much of
+// each digit is left from there on.
+__device__ inline void tile_origin(const MoveTile &p, int64_t &base_s, int64_t &base_d, uint32_t (&room)[MOVE_MAX_RANK]) {
   uint32_t blk = blockIdx.x;
-  int64_t base_s = 0, base_d = 0;
-  uint32_t room[MOVE_MAX_RANK];  // how much of each digit is left from this tile's origin on
+  base_s = base_d = 0;
 #pragma unroll
   for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) {
-    room[d] = 1;
-    if (d < p.m.rank) {
-      const uint32_t rest = p.by_chunks[d].div(blk);
-      const uint32_t origin = (blk - rest * p.chunks[d]) * p.ext[d];
-      blk = rest;
-      room[d] = p.m.shape[d] - origin;
-      base_s += int64_t(origin) * p.m.ss[d], base_d += int64_t(origin) * p.m.ds[d];
-    }
+    const uint32_t rest = p.by_chunks[d].div(blk);
+    const uint32_t origin = (blk - rest * p.chunks[d]) * p.ext[d];
+    blk = rest;
+    room[d] = p.shape[d] - origin;
+    base_s += int64_t(origin) * p.ss[d], base_d += int64_t(origin) * p.ds[d];
   }
-#pragma unroll 4
-  for (uint32_t t = threadIdx.x * V; t < p.tile; t += 256 * V) {
-    uint32_t so = 0;
-    bool inside = true;
+}
+
+// V elements of `size` bytes as zero-extended values <-> memory, one access of V * size bytes.
+template <int SIZE, int V>
+__device__ inline void load_run(const void *p, int64_t off, uint32_t (&raw)[V]) {
+  constexpr int BYTES = SIZE * V;
+  if constexpr (V == 1 || BYTES < 4) {
 #pragma unroll
-    for (uint32_t d = 0; d < uint32_t(NACT); d++) {
-      const uint32_t q = div_small(t, p.tstride_s[d], p.inv_s[d]);
-      const uint32_t c = q - div_small(q, p.ext[d], p.inv_ext[d]) * p.ext[d];
-      inside = inside && c < room[d];
-      so += c * uint32_t(p.m.ss[d]);
+    for (int e = 0; e < V; e++) raw[e] = load_sized<SIZE>(p, off + e);
+  } else {
+    typedef uint32_t W __attribute__((ext_vector_type(BYTES / 4 == 1 ? 2 : BYTES / 4)));
+    const uint8_t *at = static_cast<const uint8_t *>(p) + off * SIZE;
+    uint32_t w[BYTES / 4];
+    if constexpr (BYTES == 4) w[0] = *reinterpret_cast<const uint32_t *>(at);
+    else {
+      const W v = *reinterpret_cast<const W *>(at);
+#pragma unroll
+      for (int i = 0; i < BYTES / 4; i++) w[i] = v[i];
     }
-    if (inside) {
-      if constexpr (CONVERT) {
-        lds[t + t / 64] = load_sized<SSIZE ? SSIZE : 4>(p.m.src, base_s + so);
-      } else if constexpr (V == 1) {
-        lds[t + t / 64] = static_cast<const E *>(p.m.src)[base_s + so];
-      } else {
-        const E *from = static_cast<const E *>(p.m.src) + base_s + so;
-        Run run;
-        if (p.vec_s) run = *reinterpret_cast<const Run *>(from);
-        else
 #pragma unroll
-          for (int e = 0; e < V; e++) run[e] = from[e];
+    for (int e = 0; e < V; e++)
+      raw[e] = SIZE == 4 ? w[e] : (w[e * SIZE / 4] >> (8 * (e * SIZE % 4))) & (SIZE == 1 ? 0xffu : 0xffffu);
+  }
+}
+template <int SIZE, int V>
+__device__ inline void store_run(void *p, int64_t off, const uint32_t (&v)[V]) {
+  constexpr int BYTES = SIZE * V;
+  if constexpr (V == 1 || BYTES < 4) {
 #pragma unroll
-        for (int e = 0; e < V; e++) lds[t + t / 64 + e] = run[e];
+    for (int e = 0; e < V; e++) store_sized<SIZE>(p, off + e, v[e]);
+  } else {
+    uint32_t w[BYTES / 4];
+#pragma unroll
+    for (int i = 0; i < BYTES / 4; i++) w[i] = 0;
+#pragma unroll
+    for (int e = 0; e < V; e++) {
+      if constexpr (SIZE == 4) w[e] = v[e];
+      else w[e * SIZE / 4] |= (v[e] & (SIZE == 1 ? 0xffu : 0xffffu)) << (8 * (e * SIZE % 4));
+    }
+    uint8_t *at = static_cast<uint8_t *>(p) + off * SIZE;
+    if constexpr (BYTES == 4) MRL_STORE_ONCE(w[0], reinterpret_cast<uint32_t *>(at));
+    else if constexpr (BYTES == 8) MRL_STORE_ONCE((v2u{w[0], w[1]}), reinterpret_cast<v2u *>(at));
+    else MRL_STORE_ONCE((v4u_t{w[0], w[1], w[2], w[3]}), reinterpret_cast<v4u_t *>(at));
+  }
+}
+
+// Both sides contiguous along the same digit, in whole vectors of V elements (shape, strides and
+// extents count vectors; the wider side of a vector is 16, 8 or 4 bytes), converted or not.  Bound
+// by memory, so what matters is the order: a workgroup's tile is long along the digit that
+// continues the destination's runs AND along the one that continues the source's, so that both
+// sides see whole cache lines (f32 2048 x 16384 into bf16 strips of 16 columns, runs of 64 and
+// 32 bytes: an element per thread in destination order 133 us, this 44).  UNROLL vectors a
+// thread, their loads in flight together.
+constexpr int MOVE_RUNS_ACT = 4;   // digits a tile extends along at most
+template <int SE, int DE, int V, int UNROLL>
+__global__ __launch_bounds__(256) void k_move_runs(MoveTile p) {
+  int64_t base_s, base_d;
+  uint32_t room[MOVE_MAX_RANK];
+  tile_origin(p, base_s, base_d, room);
+  uint32_t raw[UNROLL][V], to[UNROLL];
+  bool inside[UNROLL];
+#pragma unroll
+  for (int u = 0; u < UNROLL; u++) {
+    uint32_t rem = threadIdx.x + u * 256, so = 0;
+    inside[u] = rem < p.tile;
+    to[u] = 0;
+#pragma unroll
+    for (int d = 0; d < MOVE_RUNS_ACT; d++) {
+      const uint32_t rest = div_small(rem, p.ext[d], p.inv_ext[d]), c = rem - rest * p.ext[d];
+      rem = rest;
+      inside[u] = inside[u] && c < room[d];
+      so += c * uint32_t(p.ss[d]), to[u] += c * uint32_t(p.ds[d]);
+    }
+    // (a vector outside the tensor loads the tile's first one instead: no branch between the loads)
+    load_run<SE, V>(p.src, (base_s + (inside[u] ? so : 0u)) * V, raw[u]);
+  }
+  with_dtypes<SE, DE>(p.sdt, p.ddt, [&](auto sd, auto dd) {
+#pragma unroll
+    for (int u = 0; u < UNROLL; u++)
+#pragma unroll
+      for (int e = 0; e < V; e++) raw[u][e] = convert_raw(raw[u][e], decltype(sd)::value, decltype(dd)::value);
+  });
+#pragma unroll
+  for (int u = 0; u < UNROLL; u++)
+    if (inside[u]) store_run<DE, V>(p.dst, (base_d + to[u]) * V, raw[u]);
+}
+
+// Any other pair of contiguous digits (an OddEven digit on one side, a Packed digit of rows: too
+// short for the 64 x 64 transpose): a tile of up to 4096 elements, chosen on the host so that it
+// holds long runs on both sides, is read in source order, converted in registers, and written
+// in destination order out of LDS.  VS, VD: elements per access on the two sides, 4 where the
+// element's neighbours in the tile are its neighbours in memory, else 1.  The loads of a batch of
+// four accesses are in flight together, and their digits are worked out once per access, not per
+// element: that arithmetic is what bounds the kernel.
+template <int SE, int DE, int VS, int VD, int NACT>
+__global__ __launch_bounds__(256) void k_move_gather(MoveTile p) {
+  __shared__ uint32_t lds[MOVE_TILE_MAX + MOVE_TILE_MAX / 32];
+  int64_t base_s, base_d;
+  uint32_t room[MOVE_MAX_RANK];
+  tile_origin(p, base_s, base_d, room);
+  auto cell = [](uint32_t t) { return t + t / 32; };
+  constexpr int BATCH = 4;
+  for (uint32_t t0 = 0; t0 < p.tile; t0 += 256 * VS * BATCH) {
+    uint32_t raw[BATCH][VS];
+#pragma unroll
+    for (int u = 0; u < BATCH; u++) {
+      const uint32_t t = t0 + (u * 256 + threadIdx.x) * VS;
+      uint32_t so = 0;
+      bool inside = t < p.tile;
+#pragma unroll
+      for (int d = 0; d < NACT; d++) {
+        const uint32_t q = div_small(t, p.tstride_s[d], p.inv_s[d]);
+        const uint32_t c = q - div_small(q, p.ext[d], p.inv_ext[d]) * p.ext[d];
+        inside = inside && c < room[d];
+        so += c * uint32_t(p.ss[d]);
+      }
+      load_run<SE, VS>(p.src, base_s + (inside ? so : 0u), raw[u]);
+    }
+    with_dtypes<SE, DE>(p.sdt, p.ddt, [&](auto sd, auto dd) {
+#pragma unroll
+      for (int u = 0; u < BATCH; u++)
+#pragma unroll
+        for (int e = 0; e < VS; e++) raw[u][e] = convert_raw(raw[u][e], decltype(sd)::value, decltype(dd)::value);
+    });
+#pragma unroll
+    for (int u = 0; u < BATCH; u++) {
+      const uint32_t t = t0 + (u * 256 + threadIdx.x) * VS;
+      if (t < p.tile) {
+#pragma unroll
+        for (int e = 0; e < VS; e++) lds[cell(t) + e] = raw[u][e];  // a run of four never crosses a multiple of 32
       }
     }
   }
   __syncthreads();
 #pragma unroll 4
-  for (uint32_t t = threadIdx.x * V; t < p.tile; t += 256 * V) {
+  for (uint32_t t = threadIdx.x * VD; t < p.tile; t += 256 * VD) {
     uint32_t d_o = 0, at = 0;
     bool inside = true;
 #pragma unroll
-    for (uint32_t d = 0; d < uint32_t(NACT); d++) {
+    for (int d = 0; d < NACT; d++) {
       const uint32_t q = div_small(t, p.tstride_d[d], p.inv_d[d]);
       const uint32_t c = q - div_small(q, p.ext[d], p.inv_ext[d]) * p.ext[d];
       inside = inside && c < room[d];
-      d_o += c * uint32_t(p.m.ds[d]);
+      d_o += c * uint32_t(p.ds[d]);
       at += c * p.tstride_s[d];
     }
-    if (inside) {
-      if constexpr (CONVERT) {
-        const uint32_t v = convert_raw(lds[at + at / 64], p.m.sdt, p.m.ddt);
-        store_sized<DSIZE ? DSIZE : 4>(p.m.dst, base_d + d_o, v);
-      } else if constexpr (V == 1) {
-        static_cast<E *>(p.m.dst)[base_d + d_o] = lds[at + at / 64];
-      } else {
-        Run run;
+    uint32_t v[VD];
 #pragma unroll
-        for (int e = 0; e < V; e++) {
-          const uint32_t from = at + e * p.lds_step;  // the next element along the destination's fastest digit
-          run[e] = lds[from + from / 64];
-        }
-        E *to = static_cast<E *>(p.m.dst) + base_d + d_o;
-        if (p.vec_d) *reinterpret_cast<Run *>(to) = run;
-        else
-#pragma unroll
-          for (int e = 0; e < V; e++) to[e] = run[e];
-      }
-    }
+    for (int e = 0; e < VD; e++) v[e] = lds[cell(at + (VD == 1 ? 0 : p.lds_step[e]))];
+    if (inside) store_run<DE, VD>(p.dst, base_d + d_o, v);
   }
 }
 
@@ -1205,6 +1263,105 @@ hipError_t launch_copy(const void *src, void *dst, uint64_t bytes, hipStream_t s
   return mrl::plan::last_error();
 }
 
+namespace {
+// Up to this many elements a Move with nothing to vectorise runs an element per thread: one round
+// of workgroups whatever the layouts, where the tiled kernels' loops over a handful of tiles take
+// three times as long.
+constexpr uint64_t MOVE_TINY = 65536;
+
+// A MoveTile's per-digit arrays from a view and the tile's extents.  `first`: digits in the order a
+// vector's number counts them (k_move_runs), nullptr for any order with the extended digits first.
+void fill_tile(MoveTile *t, const MoveStrided &p, const uint32_t *ext, const uint32_t *tstride_s, const uint32_t *tstride_d,
+               const uint32_t *first, uint32_t *n_act, uint64_t *blocks) {
+  auto inverse = [](uint32_t x) { return x <= 1 ? 0u : uint32_t(((uint64_t(1) << 32) + x - 1) / x); };
+  t->src = p.src, t->dst = p.dst, t->sdt = p.sdt, t->ddt = p.ddt;
+  uint32_t perm[MOVE_MAX_RANK], n = 0;
+  bool taken[MOVE_MAX_RANK] = {};
+  for (uint32_t i = 0; first && i < *n_act; i++) perm[n++] = first[i], taken[first[i]] = true;
+  for (int extended = 1; extended >= 0; extended--) {
+    for (uint32_t d = 0; d < MOVE_MAX_RANK; d++)
+      if (!taken[d] && (ext[d] > 1) == bool(extended)) perm[n++] = d, taken[d] = true;
+    if (extended && !first) *n_act = n;
+  }
+  *blocks = 1;
+  for (uint32_t i = 0; i < MOVE_MAX_RANK; i++) {
+    const uint32_t d = perm[i];
+    t->shape[i] = p.shape[d], t->ss[i] = p.ss[d], t->ds[i] = p.ds[d], t->ext[i] = ext[d];
+    t->chunks[i] = (p.shape[d] + ext[d] - 1) / ext[d], t->by_chunks[i] = FastDiv(t->chunks[i]);
+    t->inv_ext[i] = inverse(ext[d]);
+    t->tstride_s[i] = tstride_s ? tstride_s[d] : 1, t->tstride_d[i] = tstride_d ? tstride_d[d] : 1;
+    t->inv_s[i] = inverse(t->tstride_s[i]), t->inv_d[i] = inverse(t->tstride_d[i]);
+    *blocks *= t->chunks[i];
+  }
+}
+
+// k_move_runs: `shared` is the digit both sides store contiguously, in vectors of `vec` elements.
+hipError_t launch_move_runs(MoveStrided p, uint32_t shared, uint32_t vec, hipStream_t stream) {
+  const uint32_t se = uint32_t(mrl_dtype_size(p.sdt)), de = uint32_t(mrl_dtype_size(p.ddt)), rank = p.rank;
+  for (uint32_t d = 0; d < rank; d++) {
+    if (d == shared) p.shape[d] /= vec;
+    else p.ss[d] /= vec, p.ds[d] /= vec;
+  }
+  p.count /= vec;
+  // Four vectors a thread once every compute unit gets two such workgroups.
+  const uint32_t tile_cap = p.count >= 1024ull * 2 * g_compute_units ? 1024 : 256;
+  uint32_t ext[MOVE_MAX_RANK], first[MOVE_RUNS_ACT], n_first = 0, tile = 1;
+  for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) ext[d] = 1;
+  auto take = [&](uint32_t d, uint32_t most) {
+    const uint32_t e = std::min({p.shape[d], most, tile_cap / tile});
+    bool known = false;
+    for (uint32_t i = 0; i < n_first; i++) known = known || first[i] == d;
+    if (e <= 1 || known || n_first == MOVE_RUNS_ACT) return;
+    first[n_first++] = d, ext[d] = e, tile *= e;
+  };
+  // (a shared digit longer than 256 vectors is cut into even pieces)
+  take(shared, p.shape[shared] <= 256 ? 256u : (p.shape[shared] + (p.shape[shared] + 255) / 256 - 1) / ((p.shape[shared] + 255) / 256));
+  auto fastest = [&](const int64_t *stride) {   // the digit that continues the runs of one side
+    int best = -1;
+    for (uint32_t d = 0; d < rank; d++)
+      if (d != shared && p.shape[d] > 1 && (best < 0 || stride[d] < stride[best])) best = int(d);
+    return best;
+  };
+  const int next_d = fastest(p.ds), next_s = fastest(p.ss);
+  if (next_d >= 0 && next_s >= 0 && next_s != next_d) {
+    // 512 bytes of the source side, the rest of the tile along the destination's
+    const uint32_t want_s = std::max(1u, 512u / (ext[shared] * vec * se));
+    const uint32_t keep = std::min({want_s, p.shape[next_s], std::max(1u, tile_cap / tile)});
+    take(uint32_t(next_d), std::max(1u, tile_cap / tile / keep));
+    take(uint32_t(next_s), p.shape[next_s]);
+  } else if (next_d >= 0) {
+    take(uint32_t(next_d), p.shape[next_d]);
+  }
+  for (int o = int(rank) - 1; o >= 0; o--) take(p.order[o], p.shape[p.order[o]]);
+  MoveTile t;
+  uint64_t blocks = 0;
+  uint32_t n_act = n_first;
+  fill_tile(&t, p, ext, nullptr, nullptr, first, &n_act, &blocks);
+  t.tile = tile;
+  for (uint32_t e = 0; e < 4; e++) t.lds_step[e] = 0;
+  if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
+  const dim3 grid{uint32_t(blocks)};
+#define MRL_RUNS_V(SE, DE, V)                                                                                       \
+  if (vec == V) {                                                                                                  \
+    if (tile > 256) MRL_LAUNCH((k_move_runs<SE, DE, V, 4>), grid, dim3(256), 0, stream, t);                         \
+    else MRL_LAUNCH((k_move_runs<SE, DE, V, 1>), grid, dim3(256), 0, stream, t);                                    \
+  }
+#define MRL_RUNS(SE, DE)                                                                                            \
+  if (se == SE && de == DE) {                                                                                      \
+    constexpr int WIDE = 16 / (SE > DE ? SE : DE);                                                                  \
+    MRL_RUNS_V(SE, DE, WIDE)                                                                                        \
+    else MRL_RUNS_V(SE, DE, WIDE / 2)                                                                               \
+    else if constexpr (WIDE >= 8) MRL_RUNS_V(SE, DE, WIDE / 4)                                                      \
+  }
+  MRL_RUNS(1, 1) MRL_RUNS(1, 2) MRL_RUNS(1, 4)
+  MRL_RUNS(2, 1) MRL_RUNS(2, 2) MRL_RUNS(2, 4)
+  MRL_RUNS(4, 1) MRL_RUNS(4, 2) MRL_RUNS(4, 4)
+#undef MRL_RUNS
+#undef MRL_RUNS_V
+  return mrl::plan::last_error();
+}
+}  // namespace
+
 // Move over a common strided view of the two sides (layout_factor.h).  Returns
 // hipErrorInvalidValue when the view does not fit the kernels' index ranges (the caller then
 // takes the generic path).
@@ -1262,24 +1419,14 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
   for (uint32_t i = 0; i < p.rank; i++)
     for (uint32_t j = i + 1; j < p.rank; j++)
       if (p.ds[p.order[j]] > p.ds[p.order[i]]) std::swap(p.order[i], p.order[j]);
-  // A shared contiguous dim serves both sides when its runs are at least 64 bytes long.
-  const bool shared_runs = dim_s >= 0 && dim_s == dim_d &&
-                           (rank == 1 || uint64_t(p.shape[dim_s]) * mrl_dtype_size(src_dtype) >= 64);
-  // A tensor this small is one round of workgroups either way: an element per thread finishes
-  // in a third of the time the tiled kernels' loops over a handful of tiles take.
-  const bool tiny = p.count <= 65536;
-  if (dim_s < 0 || dim_d < 0 || shared_runs || tiny) {
-    // Whole 16-byte vectors along the shared dim, everywhere: move vectors, not elements.
-    const int64_t per = 16 / int64_t(mrl_dtype_size(src_dtype));
-    bool vectors = dim_s >= 0 && dim_s == dim_d && src_dtype == dst_dtype && p.shape[dim_s] % per == 0 &&
-                   (reinterpret_cast<uintptr_t>(src) & 15) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0;
-    for (uint32_t d = 0; vectors && d < rank; d++)
-      vectors = int(d) == dim_s || (p.ss[d] % per == 0 && p.ds[d] % per == 0);
-    if (vectors && rank == 1)
-      return launch_copy(src, dst, p.count * mrl_dtype_size(src_dtype), stream);
+  const size_t se = mrl_dtype_size(src_dtype), de = mrl_dtype_size(dst_dtype);
+  const bool shared = dim_s >= 0 && dim_s == dim_d;
+  if (shared && rank == 1) {
+    if (src_dtype == dst_dtype && p.count % (16 / se) == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0 &&
+        (reinterpret_cast<uintptr_t>(dst) & 15) == 0)
+      return launch_copy(src, dst, p.count * se, stream);
     // One contiguous run with a conversion: four elements per thread.
-    const size_t se = mrl_dtype_size(src_dtype), de = mrl_dtype_size(dst_dtype);
-    if (rank == 1 && dim_s == 0 && dim_d == 0 && src_dtype != dst_dtype && p.count >= 1024 &&
+    if (src_dtype != dst_dtype && p.count >= 1024 &&
         (reinterpret_cast<uintptr_t>(src) % (4 * se)) == 0 && (reinterpret_cast<uintptr_t>(dst) % (4 * de)) == 0) {
       // sixteen bytes a thread on the wider side where both buffers are aligned for it
       // (two-byte to one-byte elements: sixteen, two 16-byte loads and a 16-byte store)
@@ -1299,17 +1446,27 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
 #undef MRL_CONVERT
       return mrl::plan::last_error();
     }
-    if (vectors) {
-      for (uint32_t d = 0; d < rank; d++) {
-        if (int(d) == dim_s) p.shape[d] /= uint32_t(per);
-        else p.ss[d] /= per, p.ds[d] /= per;
-      }
-      p.count /= uint64_t(per);
+  }
+  // A shared contiguous digit in whole vectors on both sides: 16, 8 or 4 bytes on the wider side.
+  const size_t widest = std::max(se, de);
+  uint32_t vec = 0;
+  if (shared && rank > 1)
+    for (uint32_t v = uint32_t(16 / widest); vec == 0 && v >= 1 && v * widest >= 4; v /= 2) {
+      bool fits = v > 1 && p.shape[dim_s] % v == 0 && (reinterpret_cast<uintptr_t>(src) % (v * se)) == 0 &&
+                  (reinterpret_cast<uintptr_t>(dst) % (v * de)) == 0;
+      for (uint32_t d = 0; fits && d < rank; d++) fits = int(d) == dim_s || (p.ss[d] % v == 0 && p.ds[d] % v == 0);
+      if (fits) vec = v;
     }
+  if (vec) return launch_move_runs(p, uint32_t(dim_s), vec, stream);
+  // Runs of at least 64 bytes that are not whole vectors (odd rows), a tensor of one round of
+  // workgroups either way, or one with no contiguous digit: an element per thread.
+  const bool shared_runs = shared && (rank == 1 || uint64_t(p.shape[dim_s]) * se >= 64);
+  const bool tiny = p.count <= MOVE_TINY;
+  if (dim_s < 0 || dim_d < 0 || shared_runs || tiny) {
     const uint64_t blocks = (p.count + 255) / 256;
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-    if (vectors) MRL_LAUNCH(k_move_rows16, dim3(uint32_t(blocks)), dim3(256), 0, stream, p);
-    else MRL_LAUNCH(k_move_rows, dim3(uint32_t(blocks)), dim3(256), 0, stream, p);
+    for (uint32_t o = 0; o < rank; o++) p.by_shape[o] = FastDiv(p.shape[p.order[o]]);
+    MRL_LAUNCH(k_move_rows, dim3(uint32_t(blocks)), dim3(256), 0, stream, p);
     return mrl::plan::last_error();
   }
   // Two long contiguous dims: the 64 x 64 transpose.
@@ -1360,19 +1517,14 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
     else MRL_LAUNCH(k_move_tiled_as<uint32_t>, dim3(uint32_t(blocks)), dim3(256), 0, stream, p);
     return mrl::plan::last_error();
   }
-  // Neither pattern above, up to a million elements: an element per thread again (a [45, 1963, 4]
-  // tensor turned to [45, 4, 1963] took 20 us through the tile below, 4 us this way).
-  if (p.count <= (1u << 20)) {
-    MRL_LAUNCH(k_move_rows, dim3(uint32_t((p.count + 255) / 256)), dim3(256), 0, stream, p);
-    return mrl::plan::last_error();
-  }
   // Otherwise a tile grown digit by digit: along the destination's fastest digits until they
   // make a run of 64, along the source's fastest until they do, then along the destination's
-  // again while the tile stays within MOVE_TILE_MAX.
-  MoveTile t;
-  t.m = p;
+  // again while the tile stays within `cap`: 4096 elements, fewer where that would leave compute
+  // units without a workgroup.
+  const uint32_t cap = p.count >= 4096ull * 2 * g_compute_units ? MOVE_TILE_MAX : 1024;
+  uint32_t ext[MOVE_MAX_RANK];
   uint32_t by_ss[MOVE_MAX_RANK], by_ds[MOVE_MAX_RANK];  // digits, fastest first
-  for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) by_ss[d] = by_ds[d] = d, t.ext[d] = 1;
+  for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) by_ss[d] = by_ds[d] = d, ext[d] = 1;
   std::sort(by_ss, by_ss + rank, [&](uint32_t x, uint32_t y) { return p.ss[x] < p.ss[y]; });
   std::sort(by_ds, by_ds + rank, [&](uint32_t x, uint32_t y) { return p.ds[x] < p.ds[y]; });
   uint32_t tile = 1;
@@ -1380,102 +1532,93 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
     uint32_t run = 1;
     for (uint32_t i = 0; i < rank && run < run_target; i++) {
       const uint32_t d = order[i];
-      run *= t.ext[d];
-      if (t.ext[d] == p.shape[d] || run >= run_target) continue;
-      const uint32_t want = std::min<uint32_t>({p.shape[d] / t.ext[d], (run_target + run - 1) / run,
+      run *= ext[d];
+      if (ext[d] == p.shape[d] || run >= run_target) continue;
+      const uint32_t want = std::min<uint32_t>({p.shape[d] / ext[d], (run_target + run - 1) / run,
                                                 std::max<uint32_t>(1, tile_cap / tile)});
       if (want <= 1) break;
-      tile = tile / t.ext[d] * (t.ext[d] * want), run *= want, t.ext[d] *= want;
-      if (t.ext[d] != p.shape[d]) break;  // a partly covered digit ends the contiguous run
+      tile = tile / ext[d] * (ext[d] * want), run *= want, ext[d] *= want;
+      if (ext[d] != p.shape[d]) break;  // a partly covered digit ends the contiguous run
     }
   };
-  grow(by_ds, 64, MOVE_TILE_MAX / 64);
-  grow(by_ss, 64, MOVE_TILE_MAX);
-  grow(by_ds, MOVE_TILE_MAX, MOVE_TILE_MAX);
+  grow(by_ds, 64, cap / 64);
+  grow(by_ss, 64, cap);
+  grow(by_ds, cap, cap);
   // The runs are as long as they get; a tile still far below the cap (a digit covered in part
   // ends the growth above: 4 of 6 strips of an OddEven(16) dim left a tile of 64 elements, 20000
   // workgroups for 5 MB) is filled along whatever digits have room, more runs per workgroup.
-  for (uint32_t i = 0; i < rank && tile < MOVE_TILE_MAX; i++) {
+  for (uint32_t i = 0; i < rank && tile < cap; i++) {
     const uint32_t d = by_ds[i];
-    const uint32_t grown = std::min<uint32_t>(p.shape[d], uint32_t(uint64_t(t.ext[d]) * (MOVE_TILE_MAX / tile)));
-    if (grown > t.ext[d]) tile = tile / t.ext[d] * grown, t.ext[d] = grown;
+    const uint32_t grown = std::min<uint32_t>(p.shape[d], uint32_t(uint64_t(ext[d]) * (cap / tile)));
+    if (grown > ext[d]) tile = tile / ext[d] * grown, ext[d] = grown;
   }
-  t.tile = tile;
-  uint64_t blocks = 1;
-  uint32_t stride_s = 1, stride_d = 1;
-  auto inverse = [](uint32_t x) { return x <= 1 ? 0u : uint32_t(((uint64_t(1) << 32) + x - 1) / x); };
-  for (uint32_t i = 0; i < rank; i++) {
-    t.tstride_s[by_ss[i]] = stride_s, stride_s *= t.ext[by_ss[i]];
-    t.tstride_d[by_ds[i]] = stride_d, stride_d *= t.ext[by_ds[i]];
-  }
-  for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) {
-    if (d >= rank) t.tstride_s[d] = t.tstride_d[d] = 1;
-    t.chunks[d] = d < rank ? (p.shape[d] + t.ext[d] - 1) / t.ext[d] : 1;
-    t.inv_s[d] = inverse(t.tstride_s[d]), t.inv_d[d] = inverse(t.tstride_d[d]), t.inv_ext[d] = inverse(t.ext[d]);
-    blocks *= t.chunks[d];
-  }
-  if (blocks > 0x7fffffffull || tile > MOVE_TILE_MAX) return hipErrorInvalidValue;
-  const dim3 grid{uint32_t(blocks)};
-  const size_t elem = mrl_dtype_size(src_dtype);
-  // Runs of 4 or 2 elements per thread (any element size) where both sides' fastest digits allow.
-  const uint32_t fs = by_ss[0], fd = by_ds[0];
-  uint32_t run = 1;
-  if (src_dtype == dst_dtype && p.ss[fs] == 1 && p.ds[fd] == 1)
-    for (uint32_t v : {4u, 2u})
-      if (run == 1 && t.ext[fs] % v == 0 && p.shape[fs] % v == 0 && t.ext[fd] % v == 0 && p.shape[fd] % v == 0) run = v;
-  t.lds_step = t.tstride_s[fd];
-  if (elem == 1 && run == 2) run = 1;  // bytes travel in fours or alone
-  t.vec_s = (reinterpret_cast<uintptr_t>(src) % (elem * run)) == 0;
-  t.vec_d = (reinterpret_cast<uintptr_t>(dst) % (elem * run)) == 0;
-  for (uint32_t d = 0; d < rank; d++) {
-    if (d != fs && p.ss[d] % run != 0) t.vec_s = false;
-    if (d != fd && p.ds[d] % run != 0) t.vec_d = false;
-  }
-  // Digits the tile extends along first (any order of the digits serves the kernel, as long as
-  // every per-digit array follows it).
-  uint32_t perm[MOVE_MAX_RANK], n_act = 0, n_rest = 0;
-  for (uint32_t d = 0; d < MOVE_MAX_RANK; d++)
-    if (t.ext[d] > 1) perm[n_act++] = d;
-  for (uint32_t d = 0; d < MOVE_MAX_RANK; d++)
-    if (t.ext[d] <= 1) perm[n_act + n_rest++] = d;
+  if (tile > MOVE_TILE_MAX) return hipErrorInvalidValue;
+  uint32_t tstride_s[MOVE_MAX_RANK], tstride_d[MOVE_MAX_RANK];
   {
-    const MoveTile o = t;
-    for (uint32_t i = 0; i < MOVE_MAX_RANK; i++) {
-      const uint32_t d = perm[i];
-      t.m.shape[i] = o.m.shape[d], t.m.ss[i] = o.m.ss[d], t.m.ds[i] = o.m.ds[d];
-      t.ext[i] = o.ext[d], t.chunks[i] = o.chunks[d], t.by_chunks[i] = FastDiv(o.chunks[d]);
-      t.tstride_s[i] = o.tstride_s[d], t.tstride_d[i] = o.tstride_d[d];
-      t.inv_s[i] = o.inv_s[d], t.inv_d[i] = o.inv_d[d], t.inv_ext[i] = o.inv_ext[d];
+    uint32_t run_s = 1, run_d = 1;
+    for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) tstride_s[d] = tstride_d[d] = 1;
+    for (uint32_t i = 0; i < rank; i++) {
+      tstride_s[by_ss[i]] = run_s, run_s *= ext[by_ss[i]];
+      tstride_d[by_ds[i]] = run_d, run_d *= ext[by_ds[i]];
     }
-    t.m.rank = MOVE_MAX_RANK;  // size-one digits fill the tail: shape 1, one chunk
   }
-#define MRL_GATHER(E, V)                                                                              \
-  do {                                                                                                \
-    if (n_act <= 3) MRL_LAUNCH((k_move_gather<E, V, 3>), grid, dim3(256), 0, stream, t);              \
-    else if (n_act <= 5) MRL_LAUNCH((k_move_gather<E, V, 5>), grid, dim3(256), 0, stream, t);         \
-    else MRL_LAUNCH((k_move_gather<E, V, int(MOVE_MAX_RANK)>), grid, dim3(256), 0, stream, t);        \
+  // Whether the tile's elements, taken in one side's order, lie there in whole runs of four: the
+  // fastest digits continue each other (1, ext, ...) up to a multiple of four, inside the tensor as
+  // well as inside the tile, and everything else is a multiple of four apart.  in_run: how many
+  // of the fastest digits make up the four; on the destination side, whose runs are gathered from
+  // LDS at fixed distances, no run of four may carry into a further digit.
+  auto fours = [&](const uint32_t *order, const int64_t *stride, const void *base, size_t size, bool gathered, uint32_t *in_run) {
+    if ((reinterpret_cast<uintptr_t>(base) % (4 * size)) != 0) return false;
+    int64_t run = 1;
+    for (uint32_t i = 0; i < rank; i++) {
+      const uint32_t d = order[i];
+      if (stride[d] != run || (gathered && 4 % run != 0)) return false;
+      const bool whole = (run * ext[d]) % 4 == 0 && (run * p.shape[d]) % 4 == 0;
+      if (whole) {
+        for (uint32_t j = i + 1; j < rank; j++)
+          if (stride[order[j]] % 4 != 0) return false;
+        *in_run = i + 1;
+        return true;
+      }
+      if (ext[d] != p.shape[d]) return false;
+      run *= ext[d];
+    }
+    return false;
+  };
+  uint32_t digits_s = 0, digits_d = 0;
+  const bool fours_s = fours(by_ss, p.ss, src, se, false, &digits_s), fours_d = fours(by_ds, p.ds, dst, de, true, &digits_d);
+  MoveTile t;
+  for (uint32_t e = 0; e < 4; e++) {
+    uint32_t rem = e;
+    t.lds_step[e] = 0;
+    for (uint32_t i = 0; fours_d && i < digits_d; i++) {
+      const uint32_t d = by_ds[i], size = i + 1 == digits_d ? 4 : ext[d];
+      t.lds_step[e] += rem % size * tstride_s[d], rem /= size;
+    }
+  }
+  uint32_t n_act = 0;
+  uint64_t blocks = 0;
+  fill_tile(&t, p, ext, tstride_s, tstride_d, nullptr, &n_act, &blocks);
+  t.tile = tile;
+  if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
+  const dim3 grid{uint32_t(blocks)};
+#define MRL_GATHER_V(SE, DE, VS, VD)                                                                                 \
+  do {                                                                                                               \
+    if (n_act <= 4) MRL_LAUNCH((k_move_gather<SE, DE, VS, VD, 4>), grid, dim3(256), 0, stream, t);                   \
+    else MRL_LAUNCH((k_move_gather<SE, DE, VS, VD, int(MOVE_MAX_RANK)>), grid, dim3(256), 0, stream, t);             \
   } while (0)
-  if (src_dtype != dst_dtype) {
-    const int se = int(elem), de = int(mrl_dtype_size(dst_dtype));
-#define MRL_GATHER_CV(SE, DE)                                                                                      \
-  if (se == SE && de == DE) {                                                                                      \
-    if (n_act <= 5) MRL_LAUNCH((k_move_gather<void, 1, 5, SE, DE>), grid, dim3(256), 0, stream, t);                \
-    else MRL_LAUNCH((k_move_gather<void, 1, int(MOVE_MAX_RANK), SE, DE>), grid, dim3(256), 0, stream, t);          \
+#define MRL_GATHER(SE, DE)                                  \
+  if (se == SE && de == DE) {                               \
+    if (fours_s && fours_d) MRL_GATHER_V(SE, DE, 4, 4);     \
+    else if (fours_s) MRL_GATHER_V(SE, DE, 4, 1);           \
+    else if (fours_d) MRL_GATHER_V(SE, DE, 1, 4);           \
+    else MRL_GATHER_V(SE, DE, 1, 1);                        \
   }
-    MRL_GATHER_CV(1, 1) MRL_GATHER_CV(1, 2) MRL_GATHER_CV(1, 4)
-    MRL_GATHER_CV(2, 1) MRL_GATHER_CV(2, 2) MRL_GATHER_CV(2, 4)
-    MRL_GATHER_CV(4, 1) MRL_GATHER_CV(4, 2) MRL_GATHER_CV(4, 4)
-#undef MRL_GATHER_CV
-  }
-  else if (elem == 4 && run == 4) MRL_GATHER(uint32_t, 4);
-  else if (elem == 4 && run == 2) MRL_GATHER(uint32_t, 2);
-  else if (elem == 4) MRL_GATHER(uint32_t, 1);
-  else if (elem == 2 && run == 4) MRL_GATHER(uint16_t, 4);
-  else if (elem == 2 && run == 2) MRL_GATHER(uint16_t, 2);
-  else if (elem == 2) MRL_GATHER(uint16_t, 1);
-  else if (run == 4) MRL_GATHER(uint8_t, 4);
-  else MRL_GATHER(uint8_t, 1);
+  MRL_GATHER(1, 1) MRL_GATHER(1, 2) MRL_GATHER(1, 4)
+  MRL_GATHER(2, 1) MRL_GATHER(2, 2) MRL_GATHER(2, 4)
+  MRL_GATHER(4, 1) MRL_GATHER(4, 2) MRL_GATHER(4, 4)
 #undef MRL_GATHER
+#undef MRL_GATHER_V
   return mrl::plan::last_error();
 }
 

@@ -103,8 +103,12 @@ struct FastDiv {
   uint32_t mul = 0, shift = 0;
   FastDiv() = default;
   explicit FastDiv(uint32_t d) {
-    uint32_t s = 0;
-    while ((1ull << s) < d) s++;
+    if ((d & (d - 1)) == 0) {  // a power of two (most digits of a Move are 1): the same constants without the division
+      shift = 31 + (d ? uint32_t(__builtin_ctz(d)) : 0);
+      mul = (1u << 31) + 1;
+      return;
+    }
+    const uint32_t s = 32 - uint32_t(__builtin_clz(d));
     mul = uint32_t((1ull << (31 + s)) / d + 1);
     shift = 31 + s;
   }
