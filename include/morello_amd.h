@@ -246,7 +246,10 @@ int mrl_run_noalloc(const mrl_spec *spec, void *const *params, void *stream);
 
 /* Literal stand-in for calling the emitted kernel from the emitted main
  * (codegen/cpu.rs:284-409): `params` are HOST pointers; inputs (and the output, when it
- * is read) are copied to the device, the Spec is run, written parameters are copied back. */
+ * is read) are copied to the device, the Spec is run, written parameters are copied back.
+ * Device and pinned memory for it stay with the library between calls (at most two sets of up to 1 GiB
+ * on the device and 32 MiB pinned; calls from several threads use a set each);
+ * mrl_stream_release(NULL) gives them back. */
 int mrl_run_host(const mrl_spec *spec, void *const *params);
 
 /* Per-kind conveniences that build the descriptor themselves.  NULL layouts mean
@@ -400,7 +403,8 @@ int mrl_device_mem_free(size_t *free_bytes);
  * handle is what mrl_run_async, mrl_run_compose and the per-kind conveniences take.
  * mrl_stream_destroy waits for the stream's work, then frees the stream and its scratch arena.
  * mrl_stream_release waits for the work of a stream the CALLER owns (any hipStream_t that was
- * passed to mrl_run_async, NULL included) and frees only the arena the library kept for it:
+ * passed to mrl_run_async, NULL included) and frees only the arena the library kept for it (with NULL
+ * also what mrl_run_host keeps between calls):
  * call it before hipStreamDestroy, or to give the memory back; the stream stays usable and its
  * next call starts a new arena. */
 int mrl_stream_create(void **stream);

@@ -236,6 +236,7 @@ class Spec:
                 l = nhwc(shp) if self.kind == SpecKind.Conv else row_major(shp)
             self.layouts.append(l)
             self._c.layouts[i] = l.to_c()
+        self._nbytes = None   # bytes of each parameter, once run_host has asked for them
 
     # -- reference-named accessors ---------------------------------------------------
     def parameter_shape(self, idx: int):
@@ -291,9 +292,11 @@ class Spec:
         parameter's layout; the output array is written in place."""
         if len(arrays) != len(self.dtypes):
             raise ValueError("one array per parameter")
+        if self._nbytes is None:
+            self._nbytes = [self.bytes_used(i) for i in range(len(self.dtypes))]
         for i, a in enumerate(arrays):
-            if not a.flags["C_CONTIGUOUS"] or a.nbytes != self.bytes_used(i):
-                raise ValueError(f"parameter {i}: need a contiguous buffer of {self.bytes_used(i)} bytes")
+            if not a.flags["C_CONTIGUOUS"] or a.nbytes != self._nbytes[i]:
+                raise ValueError(f"parameter {i}: need a contiguous buffer of {self._nbytes[i]} bytes")
         arr = (C.c_void_p * len(arrays))(*[a.ctypes.data for a in arrays])
         _check(B.load().mrl_run_host(C.byref(self._c), arr), "mrl_run_host")
 

@@ -13,6 +13,7 @@
 #include <string>
 #include <vector>
 
+#include "host_stage.h"
 #include "kernels.h"
 #include "layout_factor.h"
 
@@ -1432,6 +1433,7 @@ int mrl_init(int device) {
     if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) == hipSuccess) g_scratch_ptr[device] = ptr;
     else (void)hipGetLastError();
   }
+  mrl::on_host_stage_stream_end(drop_arena);
   g_device = device;
   mrl::g_compute_units = prop.multiProcessorCount > 0 ? uint32_t(prop.multiProcessorCount) : 256u;
   return MRL_OK;
@@ -1780,37 +1782,36 @@ int mrl_run_host(const mrl_spec *spec, void *const *params) {
   if (rc != MRL_OK) return rc;
   if (!params) return MRL_ERR_NULL;
   if (g_device < 0 && (rc = mrl_init(0)) != MRL_OK) return rc;
+  // The stage holds what is only read first, then what is read and written, then what is only
+  // written: one contiguous range goes in and one comes out.
+  mrl::HostStage::Piece pieces[MRL_MAX_PARAMS];
   void *dev[MRL_MAX_PARAMS] = {nullptr, nullptr, nullptr, nullptr};
-  auto cleanup = [&]() {
-    for (void *p : dev)
-      if (p) (void)hipFree(p);
-  };
-  for (uint32_t i = 0; i < spec->n_params; i++) {
-    if (!params[i]) {
-      cleanup();
-      return MRL_ERR_NULL;
-    }
-    const size_t bytes = mrl_spec_parameter_bytes(spec, i);
-    hipError_t e = hipMalloc(&dev[i], bytes ? bytes : 4);
-    if (e == hipSuccess && parameter_direction(*spec, i) != 1)
-      e = hipMemcpy(dev[i], params[i], bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      cleanup();
-      return hip_fail(e, "staging parameter to device");
-    }
-  }
-  rc = mrl_run(spec, dev);
-  if (rc == MRL_OK) {
+  size_t offset[MRL_MAX_PARAMS], total = 0;
+  int n = 0, n_in = 0, first_out = 0;
+  for (int direction : {0, 2, 1}) {
+    if (direction == 2) first_out = n;
+    if (direction == 1) n_in = n;
     for (uint32_t i = 0; i < spec->n_params; i++) {
-      if (parameter_direction(*spec, i) == 0) continue;
-      hipError_t e = hipMemcpy(params[i], dev[i], mrl_spec_parameter_bytes(spec, i), hipMemcpyDeviceToHost);
-      if (e != hipSuccess) {
-        cleanup();
-        return hip_fail(e, "copying output to host");
-      }
+      if (parameter_direction(*spec, i) != direction) continue;
+      if (!params[i]) return MRL_ERR_NULL;
+      const size_t bytes = mrl_spec_parameter_bytes(spec, i);
+      pieces[n++] = {params[i], total, bytes};
+      offset[i] = total;
+      total += (std::max<size_t>(bytes, 4) + 255) & ~size_t(255);
     }
   }
-  cleanup();
+  hipError_t e = hipSuccess;
+  mrl::HostStage *stage = mrl::HostStage::acquire(total, &e);
+  if (!stage) return hip_fail(e, "staging parameters to device");
+  for (uint32_t i = 0; i < spec->n_params; i++) dev[i] = stage->device() + offset[i];
+  if ((e = stage->upload(pieces, n_in)) != hipSuccess) {
+    rc = hip_fail(e, "staging parameters to device");
+  } else {
+    Workspace ws(stage->stream());
+    rc = dispatch(*spec, dev, ws);
+  }
+  if (rc == MRL_OK && (e = stage->download(pieces + first_out, n - first_out)) != hipSuccess) rc = hip_fail(e, "copying output to host");
+  mrl::HostStage::release(stage, rc == MRL_OK);
   return rc;
 }
 
@@ -2534,6 +2535,7 @@ int mrl_stream_synchronize(void *stream) {
 int mrl_stream_release(void *stream) {
   HIP_TRY(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
   drop_arena(static_cast<hipStream_t>(stream));
+  if (!stream) mrl::HostStage::drop_idle();
   return MRL_OK;
 }
 
