@@ -19,11 +19,11 @@ namespace {
 
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
-// `vecs` 16-byte vectors across PCIe, either way.  16 workgroups keep the link full (55 GB/s; 256 of
+// `vecs` 16-byte vectors across PCIe, either way (no Spec's kernel: it is in no plan).  16 workgroups keep the link full (55 GB/s; 256 of
 // them reach 50: the link wants long runs more than many requests).  The last workgroup to finish
 // resets the counter and raises the flag on the host.
 constexpr int COPY_BLOCKS = 16;
-__global__ __launch_bounds__(256) void k_host_copy(const v4u *__restrict__ src, v4u *__restrict__ dst, uint32_t vecs, uint32_t *counter,
+__global__ __launch_bounds__(256) void pcie_copy(const v4u *__restrict__ src, v4u *__restrict__ dst, uint32_t vecs, uint32_t *counter,
                                                    uint32_t *flag, uint32_t ticket) {
   const uint32_t step = gridDim.x * 256;
   for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < vecs; i += step * 4) {
@@ -204,7 +204,7 @@ void HostStage::drop_idle() {
 hipError_t HostStage::copy(void *dst, const void *src, size_t bytes, uint32_t slot, uint32_t ticket, hipStream_t stream) {
   const uint32_t vecs = uint32_t((bytes + 15) / 16);   // both sides are padded to 256 bytes
   const uint32_t blocks = std::min<uint32_t>(COPY_BLOCKS, (vecs + 255) / 256);
-  k_host_copy<<<dim3(blocks), dim3(256), 0, stream>>>(static_cast<const v4u *>(src), static_cast<v4u *>(dst), vecs, counters_ + slot * 16,
+  pcie_copy<<<dim3(blocks), dim3(256), 0, stream>>>(static_cast<const v4u *>(src), static_cast<v4u *>(dst), vecs, counters_ + slot * 16,
                                                        flags_ + slot * 16, ticket);
   return hipGetLastError();
 }
