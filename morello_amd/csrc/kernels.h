@@ -128,6 +128,8 @@ struct GemmArgs {
   // false: B rows run along N (`ldb` = elements between k rows); true: B rows run along K
   // (`ldb` = elements between n rows), as col_major / layout![0,2,1] store it.
   bool b_kmajor = false;
+  // C is bf16 (bf16 operands only): the f32 sum, the old value included, is rounded once.
+  bool c_bf16 = false;
   // Conv as an implicit Matmul (the CONV build of the kernel): `a` is a channels-last image
   // [batch][h][w][c], row p of the left operand is the window of output pixel p (fh runs of
   // fw * c contiguous elements), never materialised.  m = batch * oh * ow, k = fh * fw * c.
@@ -173,6 +175,11 @@ hipError_t launch_gemm_big(const GemmArgs &g, int kind, hipStream_t stream, uint
 // ---- gemv.hip: at most four rows of A against a k-fastest B, as dot products (a stream over B) ----
 bool gemv_applicable(const GemmArgs &g, int kind);
 hipError_t launch_gemv(const GemmArgs &g, int kind, hipStream_t stream);
+
+// ---- gemm_skinny.hip: few rows of A or a small problem, operands straight from memory into the
+// matrix cores, rows of any alignment ----
+bool gemm_skinny_applicable(const GemmArgs &g, int kind);
+hipError_t launch_gemm_skinny(const GemmArgs &g, int kind, hipStream_t stream);
 
 // ---- gemm_sched.hip: the same kernel under a caller-chosen tile_out / split schedule -----
 uint32_t gemm_schedule_count();
