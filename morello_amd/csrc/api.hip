@@ -450,9 +450,10 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   // -1: no matrix-core kernel for these dtypes.
   const int kind = (da == MRL_I8 && db == MRL_I8 && dc == MRL_I32)       ? 0
                    : (da == MRL_U8 && db == MRL_I8 && dc == MRL_I32)     ? 1
-                   : (da == MRL_BF16 && db == MRL_BF16 && dc == MRL_F32) ? 2
+                   : (da == MRL_BF16 && db == MRL_BF16 && (dc == MRL_F32 || dc == MRL_BF16)) ? 2
                    : (da == MRL_F32 && db == MRL_F32 && dc == MRL_F32)   ? 3
                                                                          : -1;
+  g.c_bf16 = dc == MRL_BF16;
   // Few rows, or a small problem: read in place whatever the rows' alignment.
   if (!sched && kind >= 0 && rows && mrl::gemm_skinny_applicable(g, kind)) {
     HIP_TRY(mrl::launch_gemm_skinny(g, kind, ws.stream));
@@ -476,57 +477,51 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
       int64_t ld, bs;
       return as_rows(t, &ld, &bs) && ld % per16 == 0 && bs % per16 == 0;
     };
-    auto densify = [&](Prepared &p, bool read, bool pad) -> int {
-      mrl::Strided dense = p.t;
-      const int64_t cols = p.t.shape[2], ld = pad ? (cols + per16 - 1) / per16 * per16 : cols;
-      dense.stride[2] = 1, dense.stride[1] = ld, dense.stride[0] = int64_t(p.t.shape[1]) * ld;
-      const size_t bytes = size_t(p.t.shape[0]) * dense.stride[0] * p.elem;
+    auto transposed = [](mrl::Strided t) {   // [b, k, n] viewed as [b, n, k]
+      std::swap(t.shape[1], t.shape[2]);
+      std::swap(t.stride[1], t.stride[2]);
+      return t;
+    };
+    // Rows of another tensor in memory: dense, each padded to whole chunks.
+    auto rows_of = [&](const mrl::Strided &t) {
+      mrl::Strided d = t;
+      d.stride[2] = 1, d.stride[1] = (int64_t(t.shape[2]) + per16 - 1) / per16 * per16, d.stride[0] = int64_t(t.shape[1]) * d.stride[1];
+      return d;
+    };
+    int64_t any_ld, any_bs;
+    // A and B as rows, whichever way B's run; an operand with no rows at all is turned by a Move.
+    mrl::PadRows pads[2];
+    int n_pads = 0;
+    auto make_rows = [&](Prepared &p, mrl::Strided &t) -> int {
+      if (walkable(t)) return MRL_OK;
+      mrl::Strided dense = rows_of(t);
+      const size_t bytes = size_t(t.shape[0]) * dense.stride[0] * p.elem;
       HIP_TRY(ws.alloc(&dense.ptr, bytes));
-      int64_t old_ld, old_bs;
-      if (read && as_rows(p.t, &old_ld, &old_bs)) {  // rows stay rows: one pass, padding included
-        HIP_TRY(mrl::launch_pad_rows(p.t, dense.ptr, uint32_t(ld), p.elem, ws.stream));
-      } else if (read) {
-        if (ld != cols) HIP_TRY(mrl::launch_fill_zero(dense.ptr, bytes, ws.stream));
-        HIP_TRY(mrl::launch_move_strided(p.t, dense, ws.stream));
+      if (as_rows(t, &any_ld, &any_bs)) {
+        pads[n_pads++] = {t, dense.ptr, uint32_t(dense.stride[1]), t.shape[1], p.elem};
+      } else {
+        if (dense.stride[1] != int64_t(t.shape[2])) HIP_TRY(mrl::launch_fill_zero(dense.ptr, bytes, ws.stream));
+        HIP_TRY(mrl::launch_move_strided(t, dense, ws.stream));
       }
-      p.t = dense;
+      t = dense;
       return MRL_OK;
     };
-    bool b_walkable = walkable(b.t);
-    if (!b_walkable) {
-      mrl::Strided bt = b.t;  // [b, n, k] view: B with k fastest needs whole chunks along K
-      std::swap(bt.shape[1], bt.shape[2]);
-      std::swap(bt.stride[1], bt.stride[2]);
-      b_walkable = walkable(bt);
+    if ((rc = make_rows(a, a.t)) != MRL_OK) return rc;
+    mrl::Strided b_rows = g.b_kmajor ? transposed(b.t) : b.t;
+    if ((rc = make_rows(b, b_rows)) != MRL_OK) return rc;
+    b.t = g.b_kmajor ? transposed(b_rows) : b_rows;
+    if (n_pads == 2) HIP_TRY(mrl::launch_pad_rows_pair(pads[0], pads[1], ws.stream));
+    else if (n_pads == 1) HIP_TRY(mrl::launch_pad_rows(pads[0], ws.stream));
+    c_densified = !as_rows(c.t, &any_ld, &any_bs);
+    if (c_densified) {
+      mrl::Strided dense = c.t;
+      dense.stride[2] = 1, dense.stride[1] = c.t.shape[2], dense.stride[0] = int64_t(c.t.shape[1]) * c.t.shape[2];
+      HIP_TRY(ws.alloc(&dense.ptr, size_t(c.t.shape[0]) * dense.stride[0] * c.elem));
+      if (s.accum) HIP_TRY(mrl::launch_move_strided(c.t, dense, ws.stream));
+      c.t = dense;
     }
-    int64_t any_ld, any_bs;
-    if (!walkable(a.t) && !b_walkable && a.elem == b.elem && as_rows(a.t, &any_ld, &any_bs) && as_rows(b.t, &any_ld, &any_bs)) {
-      // Both operands keep their rows and only need them padded: the two copies in one launch.
-      Prepared *both[2] = {&a, &b};
-      mrl::Strided dense[2];
-      for (int i = 0; i < 2; i++) {
-        const Prepared &p = *both[i];
-        dense[i] = p.t;
-        const int64_t cols = p.t.shape[2], ld = (cols + per16 - 1) / per16 * per16;
-        dense[i].stride[2] = 1, dense[i].stride[1] = ld, dense[i].stride[0] = int64_t(p.t.shape[1]) * ld;
-        HIP_TRY(ws.alloc(&dense[i].ptr, size_t(p.t.shape[0]) * dense[i].stride[0] * p.elem));
-      }
-      HIP_TRY(mrl::launch_pad_rows_pair(a.t, dense[0].ptr, uint32_t(dense[0].stride[1]), b.t, dense[1].ptr,
-                                        uint32_t(dense[1].stride[1]), a.elem, ws.stream));
-      a.t = dense[0], b.t = dense[1];
-      g.b_kmajor = false;
-    } else {
-      if (!walkable(a.t) && (rc = densify(a, true, true)) != MRL_OK) return rc;
-      if (!b_walkable) {
-        if ((rc = densify(b, true, true)) != MRL_OK) return rc;
-        g.b_kmajor = false;
-      }
-    }
-    int64_t ld, bs;
-    c_densified = !as_rows(c.t, &ld, &bs);
-    if (c_densified && (rc = densify(c, s.accum != 0, false)) != MRL_OK) return rc;
     g.a = a.t.ptr, g.b = b.t.ptr, g.c = c.t.ptr;
-    b_ok = g.b_kmajor || as_rows(b.t, &g.ldb, &g.sb);
+    b_ok = as_rows(b_rows, &g.ldb, &g.sb);
     rows = as_rows(a.t, &g.lda, &g.sa) && b_ok && as_rows(c.t, &g.ldc, &g.sc);
   }
   auto finish = [&]() -> int {
@@ -536,7 +531,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   };
   if (sched) {
     // A manual schedule is honoured wherever the kernel can run, whatever the size model says.
-    if (kind < 0 || !rows || g.b_kmajor || !mrl::gemm_possible(g, kind)) return MRL_ERR_UNSUPPORTED;
+    if (kind < 0 || g.c_bf16 || !rows || g.b_kmajor || !mrl::gemm_possible(g, kind)) return MRL_ERR_UNSUPPORTED;
     hipError_t e = mrl::launch_gemm_scheduled(g, kind, sched->tile_m, sched->tile_n, sched->split_k, ws.stream, sched->staging);
     if (e == hipErrorInvalidValue) return MRL_ERR_UNSUPPORTED;
     HIP_TRY(e);
@@ -553,7 +548,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
       mrl::GemmArgs slices = g;
       slices.batch = splits, slices.k = (g.k - left) / splits;
       slices.sa = slices.k, slices.sb = g.b_kmajor ? int64_t(slices.k) : int64_t(slices.k) * g.ldb;
-      slices.c = partial, slices.ldc = g.n, slices.sc = int64_t(g.m) * g.n, slices.accum = 0;
+      slices.c = partial, slices.ldc = g.n, slices.sc = int64_t(g.m) * g.n, slices.accum = 0, slices.c_bf16 = false;
       HIP_TRY(mrl::launch_gemm(slices, kind, ws.stream));
       if (left) {
         mrl::GemmArgs rest = slices;
@@ -564,10 +559,19 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
         rest.c = (char *)partial + size_t(splits) * g.m * g.n * 4;
         HIP_TRY(mrl::launch_gemm(rest, kind, ws.stream));
       }
-      HIP_TRY(mrl::launch_sum_splits(partial, g.c, splits + (left ? 1 : 0), g.m, g.n, g.ldc, g.accum != 0, kind <= 1, ws.stream));
+      HIP_TRY(mrl::launch_sum_splits(partial, g.c, splits + (left ? 1 : 0), g.m, g.n, g.ldc, g.accum != 0, kind <= 1, g.c_bf16, ws.stream));
     } else {
       HIP_TRY(mrl::launch_gemm(g, kind, ws.stream));
     }
+  } else if (dc == MRL_BF16) {
+    // The generic kernel works in the output's dtype: an f32 result first, rounded once.
+    mrl::Strided wide = c.t;
+    wide.dtype = MRL_F32;
+    wide.stride[2] = 1, wide.stride[1] = c.t.shape[2], wide.stride[0] = int64_t(c.t.shape[1]) * c.t.shape[2];
+    HIP_TRY(ws.alloc(&wide.ptr, c.count * sizeof(float)));
+    if (s.accum) HIP_TRY(mrl::launch_move_strided(c.t, wide, ws.stream));
+    HIP_TRY(mrl::launch_matmul_generic(a.t, b.t, wide, s.accum, ws.stream));
+    HIP_TRY(mrl::launch_move_strided(wide, c.t, ws.stream));
   } else
     HIP_TRY(mrl::launch_matmul_generic(a.t, b.t, c.t, s.accum, ws.stream));
   return finish();
@@ -746,7 +750,7 @@ int run_conv(const mrl_spec &s, void *const *params, Workspace &ws) {
       slices.c = partial, slices.ldc = conv_args.n, slices.sc = int64_t(conv_args.m) * conv_args.n, slices.accum = 0;
       HIP_TRY(mrl::launch_conv_gemm(slices, kind, ws.stream, 64));
       HIP_TRY(mrl::launch_sum_splits(partial, conv_args.c, splits, conv_args.m, conv_args.n, conv_args.ldc,
-                                     s.accum != 0, kind <= 1, ws.stream));
+                                     s.accum != 0, kind <= 1, false, ws.stream));
     } else {
       HIP_TRY(mrl::launch_conv_gemm(conv_args, kind, ws.stream, forced == 2 ? g_forced->conv_tile : 0));
     }
@@ -760,7 +764,7 @@ int run_conv(const mrl_spec &s, void *const *params, Workspace &ws) {
       flat.ptr = filt.t.ptr, flat.dtype = filt.t.dtype, flat.rank = 3;
       flat.shape[0] = 1, flat.shape[1] = cv.f, flat.shape[2] = uint32_t(window);
       flat.stride[0] = 0, flat.stride[1] = int64_t(window), flat.stride[2] = 1;
-      HIP_TRY(mrl::launch_pad_rows(flat, padded, uint32_t(row_elems), filt.elem, ws.stream));
+      HIP_TRY(mrl::launch_pad_rows({flat, padded, uint32_t(row_elems), cv.f, filt.elem}, ws.stream));
       weights = padded;
     }
     // A 1x1 filter over whole chunks of channels: the image is U already.
@@ -939,7 +943,7 @@ int run_compose_msm(const mrl_spec &s, void *const *params, Workspace &ws) {
         flat.ptr = const_cast<void *>(dense), flat.dtype = MRL_BF16, flat.rank = 3;
         flat.shape[0] = 1, flat.shape[1] = b * rows, flat.shape[2] = cols;
         flat.stride[0] = 0, flat.stride[1] = cols, flat.stride[2] = 1;
-        HIP_TRY(mrl::launch_pad_rows(flat, buf, dp, 2, ws.stream));
+        HIP_TRY(mrl::launch_pad_rows({flat, buf, dp, flat.shape[1], 2}, ws.stream));
         dense = buf;
       }
       *result = dense;
@@ -1208,13 +1212,17 @@ int run_bf16_output(const mrl_spec &s, void *const *params, Workspace &ws) {
     if ((rc = move(i, s.dtypes[i], s.layouts[i], params[i], MRL_BF16, t.layouts[i], buf)) != MRL_OK) return rc;
     t.dtypes[i] = MRL_BF16, p[i] = buf;
   }
+  if (s.kind == MRL_SPEC_MATMUL) {  // rounded where the sums are stored
+    p[2] = params[2];
+    return run_matmul(t, p, ws);
+  }
   uint32_t shape[MRL_MAX_RANK], rank;
   parameter_shape(s, 2, shape, &rank);
   HIP_TRY(ws.alloc(&p[2], size_t(volume(shape, rank)) * 4));
   t.dtypes[2] = MRL_F32;
   mrl_layout_row_major(shape, rank, &t.layouts[2]);
   if (s.accum && (rc = move(2, MRL_BF16, s.layouts[2], params[2], MRL_F32, t.layouts[2], p[2])) != MRL_OK) return rc;
-  if ((rc = s.kind == MRL_SPEC_MATMUL ? run_matmul(t, p, ws) : run_conv(t, p, ws)) != MRL_OK) return rc;
+  if ((rc = run_conv(t, p, ws)) != MRL_OK) return rc;
   return move(2, MRL_F32, t.layouts[2], p[2], MRL_BF16, s.layouts[2], params[2]);
 }
 
@@ -1703,7 +1711,7 @@ uint32_t mrl_target_kernels(const char **names, uint32_t cap) {
       "k_softmax_cols",
       "k_softmax_generic", "k_softmax_cols_short", "k_parts", "k_parts_block", "k_parts_rows", "k_parts_cols", "k_broadcast", "k_broadcast_rows", "k_broadcast_fill_rows", "k_fill", "k_fill16", "k_fill_zero", "k_move_rows", "k_move_runs",
       "k_move_tiled", "k_move_tiled_as", "k_move_tiled8v", "k_move_tiled16", "k_move_tiled16v", "k_move_tiled32", "k_move_gather", "k_move_generic", "k_relayout", "k_convert4", "k_copy1",
-      "k_copy16", "k_pad_rows", "k_pad_rows_pair", "k_pad_rows16", "k_widen_bf16"};
+      "k_copy16", "k_pad_rows", "k_pad_rows_pair", "k_widen_bf16"};
   const uint32_t n = sizeof families / sizeof families[0];
   for (uint32_t i = 0; i < n && i < cap && names; i++) names[i] = families[i];
   return n;

@@ -63,7 +63,6 @@ __global__ __launch_bounds__(512) void k_gemm_big(MRL_WALK_PARAMS, GemmArgs g) {
   constexpr int K_SLAB = 32 / ES;
   static_assert(TM == 4 && TN == 2, "the assembly loop is written for 4 x 2 MFMA blocks per wave");
   typedef typename T::Acc Acc;
-  typedef typename T::Out Out;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -77,7 +76,6 @@ __global__ __launch_bounds__(512) void k_gemm_big(MRL_WALK_PARAMS, GemmArgs g) {
 
   const uint8_t *A = (const uint8_t *)g.a + (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES;
   const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + n0) * ES;
-  Out *C = (Out *)g.c + int64_t(blockIdx.y) * g.sc + m0 * g.ldc + n0;
   const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = uint32_t(g.ldb) * ES;
   const uint32_t lds0 = uint32_t(uintptr_t(lds));  // LDS byte address of the dynamic allocation
 
@@ -142,8 +140,7 @@ __global__ __launch_bounds__(512) void k_gemm_big(MRL_WALK_PARAMS, GemmArgs g) {
   acc[2][0] = __builtin_bit_cast(Acc, c4), acc[2][1] = __builtin_bit_cast(Acc, c5);
   acc[3][0] = __builtin_bit_cast(Acc, c6), acc[3][1] = __builtin_bit_cast(Acc, c7);
   int colsum[TN] = {sums[0], sums[1]};
-  epilogue<T, A_UNSIGNED, false, BN, WAVES_M, TM, TN>(g, C, lds, acc, colsum, lane, wm, wm * WM, wn * WN,
-                                                      int(g.m - m0), int(g.n - n0));
+  epilogue<T, A_UNSIGNED, false, BN, WAVES_M, TM, TN>(g, blockIdx.y, m0, n0, lds, acc, colsum, lane, wm, wm * WM, wn * WN);
 }
 
 // Whole tiles, an even number of k steps, and offsets the loop's 32-bit arithmetic can hold.
@@ -165,7 +162,7 @@ hipError_t launch_big(const GemmArgs &g, hipStream_t stream) {
   const int tiles_m = int(g.m / 256), tiles_n = int(g.n / 256);
   const double mn = double(g.m) * g.n * g.batch;
   plan::work(T::ES == 1 ? plan::UNIT_MFMA_I8 : plan::UNIT_MFMA_BF16, 2.0 * mn * g.k,
-             (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * 4 * (g.accum ? 2 : 1),
+             (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * (g.c_bf16 ? 2 : 4) * (g.accum ? 2 : 1),
              2.0 * 256 * 256 * double(g.k), 500.0 + 1200.0 * double(g.k * T::ES / 128),
              T::ES == 1 ? 1.25 : 1.08);  // measured: 1800 TOPS int8 at 4096^3
   const TileWalk walk = tile_walk(tiles_m, tiles_n);

@@ -200,11 +200,14 @@ struct F32 {
 // and, for an accumulating Spec, the previous contents).  `colsum` holds this wave's partial
 // column sums of B; the partials of the PARTS waves that share the columns (and of the two
 // lane halves) are combined through LDS, which every wave must be done reading.
-template <class T, bool A_UNSIGNED, bool EDGE, int BN, int PARTS, int TM, int TN>
-__device__ inline void epilogue(const GemmArgs &g, typename T::Out *C, uint8_t *lds,
-                                typename T::Acc (&acc)[TM][TN], int (&colsum)[TN], int lane,
-                                int part_idx, int row0, int col0, int rows_left, int cols_left) {
+// Stored: the type of C in memory, the accumulators' or bf16 (a bf16 Matmul that hands on bf16: the
+// f32 sum, the old value included, is rounded once).
+template <class T, bool A_UNSIGNED, bool EDGE, int BN, int PARTS, int TM, int TN, class Stored>
+__device__ inline void epilogue_as(const GemmArgs &g, Stored *C, uint8_t *lds,
+                                   typename T::Acc (&acc)[TM][TN], int (&colsum)[TN], int lane,
+                                   int part_idx, int row0, int col0, int rows_left, int cols_left) {
   typedef typename T::Out Out;
+  constexpr bool NARROW = sizeof(Stored) == 2;
   constexpr int WAVES_M = PARTS;
   const int wm = part_idx;
   // Epilogue.  Column sums: combine the partials of the WAVES_M waves and two lane halves.
@@ -237,14 +240,15 @@ __device__ inline void epilogue(const GemmArgs &g, typename T::Out *C, uint8_t *
   // output: 14.0 against 15.0 us); a large one, or rows that straddle lines, is written faster
   // through the cache, which joins the parts of a line (268 MB: 60 against 73 us; rows of 4425
   // floats: 28 against 43 us).
-  const bool stream_c = double(g.m) * g.n * g.batch * sizeof(Out) <= 32.0 * 1024 * 1024 && (g.ldc * sizeof(Out)) % 128 == 0;
+  // bf16 rows leave in pieces of 64 bytes, half a line: always through the cache.
+  const bool stream_c = !NARROW && double(g.m) * g.n * g.batch * sizeof(Out) <= 32.0 * 1024 * 1024 && (g.ldc * sizeof(Out)) % 128 == 0;
   const int lane_row = row0 + (lane >> 5) * 4, lane_col = col0 + (lane & 31);
-  Out *c_lane = C + int64_t(lane_row) * g.ldc + lane_col;
-  const uint32_t ldc_b = uint32_t(g.ldc) * sizeof(Out);
-  const auto c_buf = buffer_of(C, EDGE ? int64_t(rows_left - 1) * ldc_b + int64_t(cols_left) * sizeof(Out) : 0);
-  const uint32_t lane_off = uint32_t(lane_row) * ldc_b + uint32_t(lane_col) * sizeof(Out);
+  Stored *c_lane = C + int64_t(lane_row) * g.ldc + lane_col;
+  const uint32_t ldc_b = uint32_t(g.ldc) * sizeof(Stored);
+  const auto c_buf = buffer_of(C, EDGE ? int64_t(rows_left - 1) * ldc_b + int64_t(cols_left) * sizeof(Stored) : 0);
+  const uint32_t lane_off = uint32_t(lane_row) * ldc_b + uint32_t(lane_col) * sizeof(Stored);
   auto offset_of = [&](int tm, int tn, int r) -> uint32_t {
-    const uint32_t off = lane_off + uint32_t(tm * 32 + (r >> 2) * 8 + (r & 3)) * ldc_b + tn * 32 * sizeof(Out);
+    const uint32_t off = lane_off + uint32_t(tm * 32 + (r >> 2) * 8 + (r & 3)) * ldc_b + tn * 32 * sizeof(Stored);
     return lane_col + tn * 32 < cols_left ? off : OUT_OF_RANGE;
   };
 #pragma unroll
@@ -255,10 +259,12 @@ __device__ inline void epilogue(const GemmArgs &g, typename T::Out *C, uint8_t *
       for (int tn = 0; tn < TN; tn++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-          if constexpr (EDGE)
+          if constexpr (EDGE && NARROW)
+            prev[tn][r] = Out(__builtin_bit_cast(Stored, __builtin_amdgcn_raw_buffer_load_b16(c_buf, offset_of(tm, tn, r), 0, 0)));
+          else if constexpr (EDGE)
             prev[tn][r] = __builtin_bit_cast(Out, __builtin_amdgcn_raw_buffer_load_b32(c_buf, offset_of(tm, tn, r), 0, 0));
           else
-            prev[tn][r] = c_lane[int64_t(tm * 32 + (r >> 2) * 8 + (r & 3)) * g.ldc + tn * 32];
+            prev[tn][r] = Out(c_lane[int64_t(tm * 32 + (r >> 2) * 8 + (r & 3)) * g.ldc + tn * 32]);
         }
     }
     // A row's TN segments of 128 bytes one after the other: when rows of C are not whole cache
@@ -272,19 +278,35 @@ __device__ inline void epilogue(const GemmArgs &g, typename T::Out *C, uint8_t *
           Out v = acc[tm][tn][r];
           if (A_UNSIGNED) v += Out(corr[tn]);
           if (g.accum) v += prev[tn][r];
-          if constexpr (EDGE) {
+          if constexpr (EDGE && NARROW) {
+            __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, Stored(v)), c_buf, offset_of(tm, tn, r), 0, 0);
+          } else if constexpr (EDGE) {
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), c_buf, offset_of(tm, tn, r), 0,
                                                   decltype(streaming)::value ? 2 : 0);
           } else {
-            Out *to = &c_lane[int64_t(tm * 32 + (r >> 2) * 8 + (r & 3)) * g.ldc + tn * 32];
+            Stored *to = &c_lane[int64_t(tm * 32 + (r >> 2) * 8 + (r & 3)) * g.ldc + tn * 32];
             if constexpr (decltype(streaming)::value) __builtin_nontemporal_store(v, to);
-            else *to = v;
+            else *to = Stored(v);
           }
         }
     };
-    if (stream_c) store_rows(std::true_type{});
+    if constexpr (NARROW) store_rows(std::false_type{});
+    else if (stream_c) store_rows(std::true_type{});
     else store_rows(std::false_type{});
   }
+}
+
+// The tile at row m0, column n0 of batch entry `entry`.
+template <class T, bool A_UNSIGNED, bool EDGE, int BN, int PARTS, int TM, int TN>
+__device__ inline void epilogue(const GemmArgs &g, int64_t entry, int64_t m0, int64_t n0, uint8_t *lds,
+                                typename T::Acc (&acc)[TM][TN], int (&colsum)[TN], int lane, int part_idx, int row0, int col0) {
+  const int64_t at = entry * g.sc + m0 * g.ldc + n0;
+  if constexpr (std::is_same<T, BF16>::value)
+    if (g.c_bf16)
+      return epilogue_as<T, A_UNSIGNED, EDGE, BN, PARTS, TM, TN>(g, (__bf16 *)g.c + at, lds, acc, colsum, lane, part_idx, row0, col0,
+                                                                 int(g.m - m0), int(g.n - n0));
+  epilogue_as<T, A_UNSIGNED, EDGE, BN, PARTS, TM, TN>(g, (typename T::Out *)g.c + at, lds, acc, colsum, lane, part_idx, row0, col0,
+                                                      int(g.m - m0), int(g.n - n0));
 }
 
 // Pins the instruction order of one k step: slot I of N issues MFMA_PER MFMAs, then its even
@@ -336,7 +358,6 @@ __global__ __launch_bounds__(TL::NT) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
   constexpr int SLABS = BKB / 32;                 // MFMA k steps per tile (32 bytes each)
   constexpr int K_SLAB = 32 / ES;                 // elements of K per MFMA
   typedef typename T::Acc Acc;
-  typedef typename T::Out Out;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, lives in an SGPR
@@ -347,7 +368,6 @@ __global__ __launch_bounds__(TL::NT) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
 
   const uint8_t *A = (const uint8_t *)g.a + (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES;
   const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : n0)) * ES;
-  Out *C = (Out *)g.c + int64_t(blockIdx.y) * g.sc + m0 * g.ldc + n0;
   const int64_t lda_b = g.lda * ES, ldb_b = g.ldb * ES;
 
   // Per-thread staging assignments for one k step.  Thread `tid` moves 16-byte chunk
@@ -594,8 +614,7 @@ __global__ __launch_bounds__(TL::NT) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
     }
   }
 
-  epilogue<T, A_UNSIGNED, EDGE, BN, WAVES_M, TM, TN>(g, C, lds, acc, colsum, lane, wm, wm * WM, wn * WN,
-                                                     int(g.m - m0), int(g.n - n0));
+  epilogue<T, A_UNSIGNED, EDGE, BN, WAVES_M, TM, TN>(g, blockIdx.y, m0, n0, lds, acc, colsum, lane, wm, wm * WM, wn * WN);
 }
 
 // Whether the 32-bit offsets of the EDGE kernels reach every row of a tile.
@@ -621,7 +640,7 @@ hipError_t launch(const GemmArgs &g, hipStream_t stream) {
     const double k_steps = double((g.k * T::ES + TL::BKB - 1) / TL::BKB) * (TL::BKB / T::ES);  // k, padded to steps
     const double mn = double(g.m) * g.n * g.batch;
     plan::work(T::ES == 1 ? plan::UNIT_MFMA_I8 : T::ES == 2 ? plan::UNIT_MFMA_BF16 : plan::UNIT_MFMA_F32,
-               2.0 * mn * g.k, (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * 4 * (g.accum ? 2 : 1),
+               2.0 * mn * g.k, (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * (g.c_bf16 ? 2 : 4) * (g.accum ? 2 : 1),
                2.0 * BM * BN * k_steps,
                // prologue and epilogue, then one barrier-to-barrier trip per step of K, longer for a
                // larger tile (measured 0.4-0.55 us at 64 x 64, 0.6-1.0 at 128 x 128, 1.4-2.0 at 256 x 256)

@@ -8,6 +8,7 @@
 // meet in LDS once.  Rows may start at any element.
 //   semantics: morello/src/spec.rs:480-485; integers exact, bf16 and f32 summed in f32.
 #include "gemm_mfma_kernel.h"
+#include "row_chunks.h"
 
 namespace mrl {
 namespace {
@@ -39,23 +40,6 @@ __device__ inline typename Kind<KIND>::Acc mfma(v4i a, v4i b, typename Kind<KIND
   }
 }
 
-// The sixteen bytes from byte `shift` (0 .. 15) of two chunks on.
-__device__ inline v4i cut(v4i lo, v4i hi, uint32_t shift) {
-  // by one and by two words as bit selects (as conditional copies the compiler moves the words
-  // through LDS), then by bytes
-  const uint32_t by1 = 0u - (shift >> 2 & 1), by2 = 0u - (shift >> 3 & 1);
-  uint32_t t[8] = {uint32_t(lo[0]), uint32_t(lo[1]), uint32_t(lo[2]), uint32_t(lo[3]),
-                   uint32_t(hi[0]), uint32_t(hi[1]), uint32_t(hi[2]), uint32_t(hi[3])};
-#pragma unroll
-  for (int i = 0; i < 7; i++) t[i] = (t[i + 1] & by1) | (t[i] & ~by1);
-#pragma unroll
-  for (int i = 0; i < 5; i++) t[i] = (t[i + 2] & by2) | (t[i] & ~by2);
-  v4i v;
-#pragma unroll
-  for (int i = 0; i < 4; i++) v[i] = int(__builtin_amdgcn_alignbyte(t[i + 1], t[i], shift & 3));
-  return v;
-}
-
 // Sixteen bytes of a row of k_bytes, from a multiple of 16 on.  ALIGNED: rows start on 16-byte chunks
 // and K ends on one.  Otherwise they are cut out of the two aligned chunks they lie in: an access
 // that is not aligned runs at a fraction of the rate, and an aligned chunk that holds a valid byte
@@ -79,24 +63,17 @@ struct Row {
   }
   __device__ v4i value(const Raw &r) const {
     if constexpr (ALIGNED) return r.lo;
-    return cut(r.lo, r.hi, uint32_t(shift));
+    return cut_chunk(r.lo, r.hi, uint32_t(shift));
   }
   // those behind the row's end are zeros
   __device__ v4i tail(int kb) const {
     const int left = k_bytes - kb;
-    v4i v = {0, 0, 0, 0};
-    if (left <= 0) return v;
+    if (left <= 0) return v4i{0, 0, 0, 0};
     Raw r;
     r.lo = *(const v4i *)(first + kb);
     if constexpr (ALIGNED) return r.lo;
     r.hi = *(const v4i *)(first + kb + (shift + min(left, 16) > 16 ? 16 : 0));
-    v = value(r);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int n = left - 4 * i;
-      v[i] &= n >= 4 ? -1 : n <= 0 ? 0 : int((1u << (8 * n)) - 1);
-    }
-    return v;
+    return keep_bytes(value(r), left);
   }
 };
 

@@ -210,7 +210,7 @@ inline bool wide_applicable(const GemmArgs &g, int elem_size) {
   const int64_t bk = 128 / elem_size;
   const bool long_k = g.k >= WIDE_LONG_K_STEPS * bk;
   const bool one_round = uint64_t(g.m / 256) * (g.n / 256) * g.batch <= g_compute_units;
-  return !g.b_kmajor && g.m % 256 == 0 && g.n % 256 == 0 && g.k % (2 * bk) == 0 &&
+  return !g.b_kmajor && !g.c_bf16 && g.m % 256 == 0 && g.n % 256 == 0 && g.k % (2 * bk) == 0 &&
          (long_k || (one_round && g.k >= (g.accum ? WIDE_MIN_STEPS : 4) * bk)) &&
          g.lda * elem_size * 256 < (int64_t(1) << 32) && g.ldb * elem_size * (bk + 1) < (int64_t(1) << 31) &&
          g.ldc * 4 * 32 < (int64_t(1) << 31);

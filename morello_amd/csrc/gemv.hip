@@ -119,7 +119,6 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemv(GemmArgs g) {
     }
   }
   // Lane r * COLS + c stores C[r][col0 + c].
-  acc_t *C = (acc_t *)g.c + int64_t(blockIdx.y) * g.sc;
 #pragma unroll
   for (int r = 0; r < ROWS; r++)
 #pragma unroll
@@ -127,9 +126,16 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemv(GemmArgs g) {
       if (lane == r * COLS + c && r < int(g.m) && col0 + c < int64_t(g.n)) {
         acc_t v = acc[r][c];
         if (KIND == 1) v += acc_t(colsum[c] * 128);
-        acc_t *out = C + int64_t(r) * g.ldc + col0 + c;
-        if (g.accum) v += *out;
-        *out = v;
+        const int64_t at = int64_t(blockIdx.y) * g.sc + int64_t(r) * g.ldc + col0 + c;
+        if (KIND == 2 && g.c_bf16) {
+          __bf16 *out = (__bf16 *)g.c + at;
+          if (g.accum) v += acc_t(float(*out));
+          *out = __bf16(float(v));
+        } else {
+          acc_t *out = (acc_t *)g.c + at;
+          if (g.accum) v += *out;
+          *out = v;
+        }
       }
 }
 

@@ -12,6 +12,7 @@
 
 #include "kernels.h"
 #include "layout_factor.h"
+#include "row_chunks.h"
 
 namespace mrl {
 namespace {
@@ -793,68 +794,47 @@ __global__ __launch_bounds__(256) void k_widen_bf16(const uint16_t *__restrict__
     dst[i] = uint32_t(src[i]) << 16;
 }
 
-// Copies [batch][rows][cols] with contiguous rows into rows of `dst_ld` elements (a whole number
-// of dwords), writing zeros from the end of each row to its leading dimension.  One thread per
-// destination dword, assembled from element-sized loads (the source rows need not be aligned
-// beyond their element size).
-template <class E>
-__global__ __launch_bounds__(256) void k_pad_rows(const E *__restrict__ src, uint32_t *__restrict__ dst,
-                                                  uint32_t rows, uint32_t cols, int64_t src_batch,
-                                                  int64_t src_ld, uint32_t dst_ld, uint64_t dwords) {
-  constexpr uint32_t PER = 4 / sizeof(E);
-  const uint32_t row_dwords = dst_ld / PER;
-  const uint64_t step = uint64_t(gridDim.x) * blockDim.x;
-  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < dwords; i += step) {
-    const uint64_t line = i / row_dwords;
-    const uint32_t col0 = uint32_t(i % row_dwords) * PER;
-    const E *from = src + int64_t(line / rows) * src_batch + int64_t(line % rows) * src_ld;
-    uint32_t word = 0;
+// Copies [batch][rows][cols] with contiguous rows, starting on any element, into `dst_rows` rows of whole
+// 16-byte chunks, zeros from each row's end on and in the rows past the last.  A thread makes four
+// chunks, each out of the two aligned chunks of the source it lies in (with a load per element, u8
+// 5440 x 1683 x 2556 took 62.9 us in all; 46.7 now).
+struct PadJob {
+  const uint8_t *src;
+  chunk_t *dst;
+  uint32_t rows, dst_rows, row_bytes, row_chunks;   // row_chunks: of a destination row
+  uint32_t chunks;                                  // destination chunks in all
+  int64_t src_batch, src_ld;                        // bytes
+  FastDiv by_row_chunks, by_dst_rows;
+};
+constexpr int PAD_UNROLL = 4;
+__device__ inline void pad_chunks(const PadJob &j) {
+  const uint32_t first = blockIdx.x * (256 * PAD_UNROLL) + threadIdx.x;
+  chunk_t lo[PAD_UNROLL], hi[PAD_UNROLL];
+  int left[PAD_UNROLL];
+  uint32_t shift[PAD_UNROLL];
 #pragma unroll
-    for (uint32_t e = 0; e < PER; e++)
-      if (col0 + e < cols) word |= uint32_t(from[col0 + e]) << (8 * sizeof(E) * e);
-    dst[i] = word;
+  for (int u = 0; u < PAD_UNROLL; u++) {
+    const uint32_t i = min(first + u * 256, j.chunks - 1);
+    const uint32_t line = j.by_row_chunks.div(i), entry = j.by_dst_rows.div(line), row = line - entry * j.dst_rows;
+    const int at = int(i - line * j.row_chunks) * 16;
+    left[u] = row < j.rows ? int(j.row_bytes) - at : 0;
+    // (a chunk with nothing in it reads the row's first instead)
+    const uint8_t *from = j.src + int64_t(entry) * j.src_batch + int64_t(min(row, j.rows - 1)) * j.src_ld + (left[u] > 0 ? at : 0);
+    shift[u] = uint32_t(uintptr_t(from) & 15);
+    from -= shift[u];
+    lo[u] = *(const chunk_t *)from;
+    hi[u] = *(const chunk_t *)(from + (int(shift[u]) + min(left[u], 16) > 16 ? 16 : 0));
   }
+#pragma unroll
+  for (int u = 0; u < PAD_UNROLL; u++)
+    if (first + u * 256 < j.chunks) j.dst[first + u * 256] = keep_bytes(cut_chunk(lo[u], hi[u], shift[u]), left[u]);
 }
-
+__global__ __launch_bounds__(256) void k_pad_rows(PadJob j) { pad_chunks(j); }
 // Two such copies in one launch (blockIdx.y names the copy): the two operands of a Matmul whose rows
 // are not whole 16-byte chunks each took a launch of about 2.4 us for their padded copy (int8 1000^3).
-struct PadJob {
-  const void *src;
-  uint32_t *dst;
-  uint32_t rows, cols, dst_ld;
-  int64_t src_batch, src_ld;
-  uint64_t dwords;
-};
-template <class E>
 __global__ __launch_bounds__(256) void k_pad_rows_pair(PadJob j0, PadJob j1) {
   const PadJob &j = blockIdx.y ? j1 : j0;
-  constexpr uint32_t PER = 4 / sizeof(E);
-  const uint32_t row_dwords = j.dst_ld / PER;
-  const uint64_t step = uint64_t(gridDim.x) * blockDim.x;
-  for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < j.dwords; i += step) {
-    const uint64_t line = i / row_dwords;
-    const uint32_t col0 = uint32_t(i % row_dwords) * PER;
-    const E *from = static_cast<const E *>(j.src) + int64_t(line / j.rows) * j.src_batch + int64_t(line % j.rows) * j.src_ld;
-    uint32_t word = 0;
-#pragma unroll
-    for (uint32_t e = 0; e < PER; e++)
-      if (col0 + e < j.cols) word |= uint32_t(from[col0 + e]) << (8 * sizeof(E) * e);
-    j.dst[i] = word;
-  }
-}
-
-// The same when rows start on 16 bytes on both sides and `cols` is whole 16-byte vectors: one
-// thread per destination vector (sizes and strides here count vectors).
-__global__ __launch_bounds__(256) void k_pad_rows16(const v4u *__restrict__ src, v4u *__restrict__ dst, uint32_t rows,
-                                                    uint32_t cols, int64_t src_batch, int64_t src_ld, uint32_t dst_ld,
-                                                    uint64_t vectors) {
-  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= vectors) return;
-  const uint64_t line = i / dst_ld;
-  const uint32_t col = uint32_t(i % dst_ld);
-  v4u v{0, 0, 0, 0};
-  if (col < cols) v = MRL_LOAD_ONCE(src + int64_t(line / rows) * src_batch + int64_t(line % rows) * src_ld + col);
-  __builtin_nontemporal_store(v, dst + i);
+  if (blockIdx.x * (256 * PAD_UNROLL) < j.chunks) pad_chunks(j);
 }
 
 __global__ void k_copy1(const uint8_t *src, uint8_t *dst, uint64_t bytes) {
@@ -1642,67 +1622,40 @@ hipError_t launch_move_strided(const Strided &src, const Strided &dst, hipStream
   return launch_move_view(src.ptr, src.dtype, dst.ptr, dst.dtype, dims, n, stream);
 }
 
-hipError_t launch_pad_rows(const Strided &src, void *dst, uint32_t dst_ld, uint32_t elem_size,
-                           hipStream_t stream) {
-  if (src.rank != 3 || (src.shape[2] != 1 && src.stride[2] != 1) || dst_ld * elem_size % 4 != 0 ||
-      dst_ld < src.shape[2])
-    return hipErrorInvalidValue;
-  const uint32_t batch = src.shape[0], rows = src.shape[1], cols = src.shape[2];
-  const uint64_t dwords = uint64_t(batch) * rows * (dst_ld * elem_size / 4);
-  if (dwords == 0) return hipSuccess;
-  const uint32_t blocks = uint32_t(std::min<uint64_t>((dwords + 255) / 256, 65536));
-  const int64_t sb = batch == 1 ? 0 : src.stride[0], sl = rows == 1 ? 0 : src.stride[1];
-  plan::work(plan::UNIT_STREAM, 0, double(batch) * rows * cols * elem_size + 4.0 * dwords);
-  const uint32_t per16 = 16 / elem_size;
-  if (cols % per16 == 0 && dst_ld % per16 == 0 && sb % per16 == 0 && sl % per16 == 0 &&
-      (reinterpret_cast<uintptr_t>(src.ptr) & 15) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0 &&
-      dwords / 4 <= 0x7fffffffull * 256) {
-    const uint64_t vectors = dwords / 4;
-    MRL_LAUNCH(k_pad_rows16, dim3(uint32_t((vectors + 255) / 256)), dim3(256), 0, stream, (const v4u *)src.ptr, (v4u *)dst,
-               rows, cols / per16, sb / per16, sl / per16, dst_ld / per16, vectors);
-    return mrl::plan::last_error();
-  }
-  if (elem_size == 1)
-    MRL_LAUNCH(k_pad_rows<uint8_t>, dim3(blocks), dim3(256), 0, stream, (const uint8_t *)src.ptr,
-                       (uint32_t *)dst, rows, cols, sb, sl, dst_ld, dwords);
-  else if (elem_size == 2)
-    MRL_LAUNCH(k_pad_rows<uint16_t>, dim3(blocks), dim3(256), 0, stream, (const uint16_t *)src.ptr,
-                       (uint32_t *)dst, rows, cols, sb, sl, dst_ld, dwords);
-  else if (elem_size == 4)
-    MRL_LAUNCH(k_pad_rows<uint32_t>, dim3(blocks), dim3(256), 0, stream, (const uint32_t *)src.ptr,
-                       (uint32_t *)dst, rows, cols, sb, sl, dst_ld, dwords);
-  else
-    return hipErrorInvalidValue;
+namespace {
+bool pad_job(const PadRows &p, PadJob *j) {
+  const Strided &src = p.src;
+  const uint32_t es = p.elem_size;
+  if (src.rank != 3 || (src.shape[2] != 1 && src.stride[2] != 1) || uint64_t(p.dst_ld) * es % 16 != 0 || p.dst_ld < src.shape[2] ||
+      p.dst_rows < src.shape[1] || (reinterpret_cast<uintptr_t>(p.dst) & 15) != 0)
+    return false;
+  const uint32_t batch = src.shape[0], rows = src.shape[1];
+  j->src = static_cast<const uint8_t *>(src.ptr), j->dst = static_cast<chunk_t *>(p.dst);
+  j->rows = rows, j->dst_rows = p.dst_rows, j->row_bytes = src.shape[2] * es, j->row_chunks = uint32_t(uint64_t(p.dst_ld) * es / 16);
+  const uint64_t chunks = uint64_t(batch) * p.dst_rows * j->row_chunks;
+  if (chunks >= (1ull << 31) || chunks == 0) return false;
+  j->chunks = uint32_t(chunks);
+  j->src_batch = (batch == 1 ? 0 : src.stride[0]) * int64_t(es), j->src_ld = (rows == 1 ? 0 : src.stride[1]) * int64_t(es);
+  j->by_row_chunks = FastDiv(j->row_chunks), j->by_dst_rows = FastDiv(j->dst_rows);
+  return true;
+}
+double pad_bytes(const PadJob &j) { return double(j.chunks) / j.row_chunks / j.dst_rows * j.rows * j.row_bytes + 16.0 * j.chunks; }
+}  // namespace
+
+hipError_t launch_pad_rows(const PadRows &p, hipStream_t stream) {
+  PadJob j;
+  if (!pad_job(p, &j)) return hipErrorInvalidValue;
+  plan::work(plan::UNIT_STREAM, 0, pad_bytes(j));
+  MRL_LAUNCH(k_pad_rows, dim3((j.chunks + 256 * PAD_UNROLL - 1) / (256 * PAD_UNROLL)), dim3(256), 0, stream, j);
   return mrl::plan::last_error();
 }
 
-hipError_t launch_pad_rows_pair(const Strided &src0, void *dst0, uint32_t dst_ld0, const Strided &src1, void *dst1,
-                                uint32_t dst_ld1, uint32_t elem_size, hipStream_t stream) {
-  PadJob jobs[2];
-  const Strided *srcs[2] = {&src0, &src1};
-  void *dsts[2] = {dst0, dst1};
-  const uint32_t lds[2] = {dst_ld0, dst_ld1};
-  uint64_t most = 0;
-  double bytes = 0;
-  for (int i = 0; i < 2; i++) {
-    const Strided &src = *srcs[i];
-    if (src.rank != 3 || (src.shape[2] != 1 && src.stride[2] != 1) || lds[i] * elem_size % 4 != 0 || lds[i] < src.shape[2])
-      return hipErrorInvalidValue;
-    const uint32_t batch = src.shape[0], rows = src.shape[1], cols = src.shape[2];
-    jobs[i].src = src.ptr, jobs[i].dst = static_cast<uint32_t *>(dsts[i]);
-    jobs[i].rows = rows, jobs[i].cols = cols, jobs[i].dst_ld = lds[i];
-    jobs[i].src_batch = batch == 1 ? 0 : src.stride[0], jobs[i].src_ld = rows == 1 ? 0 : src.stride[1];
-    jobs[i].dwords = uint64_t(batch) * rows * (lds[i] * elem_size / 4);
-    most = std::max(most, jobs[i].dwords);
-    bytes += double(batch) * rows * cols * elem_size + 4.0 * jobs[i].dwords;
-  }
-  if (most == 0) return hipSuccess;
-  plan::work(plan::UNIT_STREAM, 0, bytes);
-  const dim3 grid(uint32_t(std::min<uint64_t>((most + 255) / 256, 65536)), 2);
-  if (elem_size == 1) MRL_LAUNCH(k_pad_rows_pair<uint8_t>, grid, dim3(256), 0, stream, jobs[0], jobs[1]);
-  else if (elem_size == 2) MRL_LAUNCH(k_pad_rows_pair<uint16_t>, grid, dim3(256), 0, stream, jobs[0], jobs[1]);
-  else if (elem_size == 4) MRL_LAUNCH(k_pad_rows_pair<uint32_t>, grid, dim3(256), 0, stream, jobs[0], jobs[1]);
-  else return hipErrorInvalidValue;
+hipError_t launch_pad_rows_pair(const PadRows &p0, const PadRows &p1, hipStream_t stream) {
+  PadJob j0, j1;
+  if (!pad_job(p0, &j0) || !pad_job(p1, &j1)) return hipErrorInvalidValue;
+  plan::work(plan::UNIT_STREAM, 0, pad_bytes(j0) + pad_bytes(j1));
+  const uint32_t most = std::max(j0.chunks, j1.chunks);
+  MRL_LAUNCH(k_pad_rows_pair, dim3((most + 256 * PAD_UNROLL - 1) / (256 * PAD_UNROLL), 2), dim3(256), 0, stream, j0, j1);
   return mrl::plan::last_error();
 }
 
@@ -1831,13 +1784,13 @@ hipError_t launch_softmax_generic(const Strided &in, const Strided &out, uint32_
 
 namespace {
 // One thread per 32-bit element of C.
-template <class T>
-__global__ __launch_bounds__(256) void k_sum_splits(const T *__restrict__ partial, T *__restrict__ c, uint32_t splits,
+template <class T, class Stored = T>
+__global__ __launch_bounds__(256) void k_sum_splits(const T *__restrict__ partial, Stored *__restrict__ c, uint32_t splits,
                                                     uint32_t n, uint64_t count, int64_t ldc, int accum) {
   const uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= count) return;
-  T *to = c + int64_t(i / n) * ldc + int64_t(i % n);
-  T sum = accum ? *to : T(0);
+  Stored *to = c + int64_t(i / n) * ldc + int64_t(i % n);
+  T sum = accum ? T(*to) : T(0);
   constexpr uint32_t U = 8;  // loads in flight together
   for (uint32_t s0 = 0; s0 < splits; s0 += U) {
     T v[U];
@@ -1846,12 +1799,12 @@ __global__ __launch_bounds__(256) void k_sum_splits(const T *__restrict__ partia
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) sum += s0 + u < splits ? v[u] : T(0);
   }
-  *to = sum;
+  *to = Stored(sum);
 }
 }  // namespace
 
 hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint32_t m, uint32_t n, int64_t ldc,
-                             bool accum, bool integers, hipStream_t stream) {
+                             bool accum, bool integers, bool c_bf16, hipStream_t stream) {
   const uint64_t count = uint64_t(m) * n;
   if (count == 0) return hipSuccess;
   const uint64_t blocks = (count + 255) / 256;
@@ -1860,6 +1813,9 @@ hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint
   if (integers)
     MRL_LAUNCH(k_sum_splits<int>, dim3(uint32_t(blocks)), dim3(256), 0, stream, (const int *)partial, (int *)c, splits, n,
                count, ldc, int(accum));
+  else if (c_bf16)
+    MRL_LAUNCH((k_sum_splits<float, __bf16>), dim3(uint32_t(blocks)), dim3(256), 0, stream, (const float *)partial, (__bf16 *)c, splits,
+               n, count, ldc, int(accum));
   else
     MRL_LAUNCH(k_sum_splits<float>, dim3(uint32_t(blocks)), dim3(256), 0, stream, (const float *)partial, (float *)c, splits,
                n, count, ldc, int(accum));

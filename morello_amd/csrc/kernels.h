@@ -82,13 +82,17 @@ hipError_t launch_move_strided(const Strided &src, const Strided &dst, hipStream
 struct MoveDim;
 hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_dtype,
                             const MoveDim *dims, uint32_t rank, hipStream_t stream);
-// Copy of a [batch][rows][cols] tensor with contiguous rows into dense rows of `dst_ld` elements
-// (a whole number of dwords), zeros from each row's end to `dst_ld`.
-hipError_t launch_pad_rows(const Strided &src, void *dst, uint32_t dst_ld, uint32_t elem_size,
-                           hipStream_t stream);
-// Two such copies (elements of the same size) in one launch.
-hipError_t launch_pad_rows_pair(const Strided &src0, void *dst0, uint32_t dst_ld0, const Strided &src1, void *dst1,
-                                uint32_t dst_ld1, uint32_t elem_size, hipStream_t stream);
+// Copy of a [batch][rows][cols] tensor with contiguous rows (starting on any element) into dense rows of
+// `dst_ld` elements (whole 16-byte chunks), `dst_rows` per batch entry; zeros from each row's end to
+// `dst_ld` and in the rows past the source's.
+struct PadRows {
+  Strided src;
+  void *dst;
+  uint32_t dst_ld, dst_rows, elem_size;
+};
+hipError_t launch_pad_rows(const PadRows &p, hipStream_t stream);
+// Two such copies in one launch.
+hipError_t launch_pad_rows_pair(const PadRows &p0, const PadRows &p1, hipStream_t stream);
 // bf16 -> f32 of a whole buffer, position by position.
 hipError_t launch_widen_bf16(const void *src, void *dst, uint64_t count, hipStream_t stream);
 // Move Spec fast path: same bytes on both sides (16-byte aligned buffers).
@@ -164,9 +168,9 @@ uint32_t gemm_tile_side(const GemmArgs &g, int kind);
 // of K whose partial results are summed afterwards (1: as it is).  The slices are whole k steps.
 uint32_t gemm_k_splits(const GemmArgs &g, int kind, uint32_t *remainder = nullptr);
 // c[r][col] (+)= sum over s of partial[s][r][col]; partial is dense [splits][m][n], 32-bit
-// elements (int32 when `integers`, else f32), summed in order of s.
+// elements (int32 when `integers`, else f32), summed in order of s; c holds the same, or bf16.
 hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint32_t m, uint32_t n, int64_t ldc,
-                             bool accum, bool integers, hipStream_t stream);
+                             bool accum, bool integers, bool c_bf16, hipStream_t stream);
 // Always the 256 x 256 tile, 128 bytes of K per step.
 // staging: 0 = whichever of the 256 x 256 kernels applies (four waves, eight waves, compiler-scheduled),
 // 1 / 2 / 3 = mrl_staging's REGISTERS / DIRECT_B / DIRECT_B_WIDE only (hipErrorInvalidValue where that one does not apply).
