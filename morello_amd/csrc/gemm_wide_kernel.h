@@ -57,28 +57,37 @@ constexpr int WIDE_MIN_STEPS = GEMM_WIDE_MIN_STEPS;
       MRL_WIDE_10("a", 22), MRL_WIDE_10("a", 23), MRL_WIDE_10("a", 24), "a250", "a251", "a252", "a253",     \
       "a254", "a255", "s60", "s61", "s62", "s63", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71",   \
       "s72", "s73", "s74", "s75", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89", "s90",     \
-      "s91", "s92", "s93", "s94", "s95", "scc", "memory"
+      "s91", "s92", "s93", "s94", "s95", "vcc", "scc", "memory"
 
-#define MRL_WIDE_RUN(TEXT)                                                                                         \
-  asm volatile(TEXT                                                                                                \
-               :                                                                                                   \
-               : [a_off0] "v"(a_off[0]), [a_off1] "v"(a_off[1]), [a_off2] "v"(a_off[2]), [a_off3] "v"(a_off[3]),   \
-                 [a_off4] "v"(a_off[4]), [a_off5] "v"(a_off[5]), [a_off6] "v"(a_off[6]), [a_off7] "v"(a_off[7]),   \
-                 [b_off0] "v"(b_off[0]), [b_off1] "v"(b_off[1]), [b_off2] "v"(b_off[2]), [b_off3] "v"(b_off[3]),   \
-                 [b_off4] "v"(b_off[4]), [b_off5] "v"(b_off[5]), [b_off6] "v"(b_off[6]), [b_off7] "v"(b_off[7]),   \
-                 [a_wr] "v"(a_wr), [a_rd0] "v"(a_rd[0]), [a_rd1] "v"(a_rd[1]), [b_rd0] "v"(b_rd[0]),               \
-                 [b_rd1] "v"(b_rd[1]), [b_rd2] "v"(b_rd[2]), [b_rd3] "v"(b_rd[3]), [b_rd4] "v"(b_rd[4]),           \
-                 [b_rd5] "v"(b_rd[5]), [b_rd6] "v"(b_rd[6]), [b_rd7] "v"(b_rd[7]), [c_lo0] "v"(c_lo[0]),           \
-                 [c_lo1] "v"(c_lo[1]), [c_lo2] "v"(c_lo[2]), [c_lo3] "v"(c_lo[3]), [c_hi0] "v"(c_hi[0]),           \
-                 [c_hi1] "v"(c_hi[1]), [c_hi2] "v"(c_hi[2]), [c_hi3] "v"(c_hi[3]), [part_wr] "v"(part_wr),         \
-                 [part_rd_lo] "v"(part_rd_lo), [part_rd_hi] "v"(part_rd_hi), [abase] "s"(A), [bbase] "s"(B),       \
-                 [bstep] "s"(b_step), [nk] "s"(nk), [dma_base] "s"(dma_base), [cbase] "s"(c_base),                 \
-                 [ldc16] "s"(ldc16), [k32] "s"(k32)                                                                \
-               : MRL_WIDE_CLOBBERS)
+#define MRL_WIDE_VGPRS                                                                                             \
+  [a_off0] "v"(a_off[0]), [a_off1] "v"(a_off[1]), [a_off2] "v"(a_off[2]), [a_off3] "v"(a_off[3]),                   \
+      [a_off4] "v"(a_off[4]), [a_off5] "v"(a_off[5]), [a_off6] "v"(a_off[6]), [a_off7] "v"(a_off[7]),              \
+      [b_off0] "v"(b_off[0]), [b_off1] "v"(b_off[1]), [b_off2] "v"(b_off[2]), [b_off3] "v"(b_off[3]),              \
+      [b_off4] "v"(b_off[4]), [b_off5] "v"(b_off[5]), [b_off6] "v"(b_off[6]), [b_off7] "v"(b_off[7]),              \
+      [a_wr] "v"(a_wr), [a_rd0] "v"(a_rd[0]), [a_rd1] "v"(a_rd[1]), [b_rd0] "v"(b_rd[0]), [b_rd1] "v"(b_rd[1]),    \
+      [b_rd2] "v"(b_rd[2]), [b_rd3] "v"(b_rd[3]), [c_lo0] "v"(c_lo[0]), [c_lo1] "v"(c_lo[1]),                      \
+      [c_lo2] "v"(c_lo[2]), [c_lo3] "v"(c_lo[3]), [c_hi0] "v"(c_hi[0]), [c_hi1] "v"(c_hi[1]),                      \
+      [c_hi2] "v"(c_hi[2]), [c_hi3] "v"(c_hi[3]), [part_wr] "v"(part_wr), [part_rd_lo] "v"(part_rd_lo),            \
+      [part_rd_hi] "v"(part_rd_hi)
+#define MRL_WIDE_VGPRS_NN , [b_rd4] "v"(b_rd[4]), [b_rd5] "v"(b_rd[5]), [b_rd6] "v"(b_rd[6]), [b_rd7] "v"(b_rd[7])
+#define MRL_WIDE_SGPRS                                                                                             \
+  [abase] "s"(A), [bbase] "s"(B), [bstep] "s"(b_step), [nk] "s"(nk), [dma_base] "s"(dma_base),                      \
+      [cbase] "s"(c_base), [ldc16] "s"(ldc16), [k32] "s"(k32)
+#define MRL_WIDE_RUN(TEXT) asm volatile(TEXT : : MRL_WIDE_VGPRS MRL_WIDE_VGPRS_NN, MRL_WIDE_SGPRS : MRL_WIDE_CLOBBERS)
+#define MRL_WIDE_EDGE                                                                                              \
+  [b_k0] "v"(b_k[0]), [b_zero] "v"(b_zero), [atail] "s"(a_tail), [btail] "s"(b_tail), [skip] "s"(skip),             \
+      [crec] "s"(c_records), [cm0] "s"(cols[0]), [cm1] "s"(cols[1]), [cm2] "s"(cols[2]), [cm3] "s"(cols[3]),       \
+      [cm4] "s"(cols[4]), [cm5] "s"(cols[5]), [cm6] "s"(cols[6]), [cm7] "s"(cols[7])
+#define MRL_WIDE_RUN_NN_EDGE(TEXT)                                                                                 \
+  asm volatile(TEXT : : MRL_WIDE_VGPRS MRL_WIDE_VGPRS_NN, [a_keep] "v"(a_keep), MRL_WIDE_SGPRS, MRL_WIDE_EDGE : MRL_WIDE_CLOBBERS)
+#define MRL_WIDE_RUN_NT_EDGE(TEXT)                                                                                 \
+  asm volatile(TEXT : : MRL_WIDE_VGPRS, [a_keep] "v"(a_keep), [b_k1] "v"(b_k[1]), MRL_WIDE_SGPRS, MRL_WIDE_EDGE : MRL_WIDE_CLOBBERS)
 
 // M, N multiples of 256; K an even number of k steps: GEMM_WIDE_MIN_STEPS at least for an accumulating
 // Spec (whose first eight steps carry the loads of C's old values), four otherwise; see wide_applicable().
-template <class T, bool A_UNSIGNED>
+// EDGE: any M and N, K of whole 16-byte chunks (at least WIDE_EDGE_MIN_STEPS of 128 bytes), either
+// orientation of B: see wide_edge_applicable().
+template <class T, bool A_UNSIGNED, bool B_KMAJOR = false, bool EDGE = false>
 __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int BM = 256, BN = 256, BKB = 128, WM = 128, WN = 128, TN = 8;
@@ -87,6 +96,7 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   constexpr int ROWS_PER_DMA = 1024 / B_ROWB;  // k rows one direct-to-LDS instruction fills: 4 (i8), 2 (bf16)
   constexpr int GROUP_K = 16 / ES;             // k rows a lane group of an MFMA operand holds: 16 (i8), 8 (bf16)
   typedef typename T::Out Out;
+  static_assert(EDGE || !B_KMAJOR, "a k-fastest B has the ragged form only");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -109,11 +119,13 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb) * ES;
 #else
   const uint8_t *A = (const uint8_t *)g.a + (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES;
-  const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + n0) * ES;
+  const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : n0)) * ES;
 #endif
   Out *C = (Out *)g.c + int64_t(blockIdx.y) * g.sc + m0 * g.ldc + n0;
   const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = uint32_t(g.ldb) * ES, ldc_b = uint32_t(g.ldc) * 4;
   const uint32_t lds0 = uint32_t(uintptr_t(lds));
+  // Rows and columns of C from the tile's first on; operand rows past the end repeat the last one.
+  const int m_left = EDGE ? min(BM, int(g.m - m0)) : BM, n_left = EDGE ? min(BN, int(g.n - n0)) : BN;
 
   // A staging: thread `tid` moves 16-byte chunk tid + i * 256 of a tile (rows 32 apart); chunks of
   // a row are XOR-ed with (row / 2) & 7 in LDS, as in k_gemm.
@@ -121,7 +133,7 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   {
     const int row = tid / 8, ch = tid % 8;
 #pragma unroll
-    for (int i = 0; i < 8; i++) a_off[i] = uint32_t(row + i * 32) * lda_b + ch * 16;
+    for (int i = 0; i < 8; i++) a_off[i] = uint32_t(min(row + i * 32, m_left - 1)) * lda_b + ch * 16;
     a_wr = lds0 + row * BKB + ((ch ^ ((row / 2) & 7)) << 4);
   }
   // B staging: instruction j of this wave fills LDS bytes [(8 * wave + j) * 1024, +1024) of the slot,
@@ -130,8 +142,16 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   uint32_t b_off[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    const int r = (wave * 8 + j) * ROWS_PER_DMA + (lane * 16) / B_ROWB;
-    b_off[j] = uint32_t(r) * ldb_b + wide_b_swizzle<T>((lane * 16) % B_ROWB, r) + 4096 - j * 1024;
+    if constexpr (B_KMAJOR) {
+      // eight rows of 128 bytes to an instruction, chunks XOR-ed with row / 2 as A's are
+      const int r = (wave * 8 + j) * 8 + (lane >> 3);
+      b_off[j] = uint32_t(min(r, n_left - 1)) * ldb_b + (((lane & 7) ^ ((r / 2) & 7)) << 4) + 4096 - j * 1024;
+    } else {
+      const int r = (wave * 8 + j) * ROWS_PER_DMA + (lane * 16) / B_ROWB;
+      int byte = wide_b_swizzle<T>((lane * 16) % B_ROWB, r);
+      if (EDGE) byte = min(byte, (n_left * ES + 15) / 16 * 16 - 16);
+      b_off[j] = uint32_t(r) * ldb_b + byte + 4096 - j * 1024;
+    }
   }
   const uint32_t dma_base = lds0 + WIDE_B_BASE + wave * 8192;
   // Operand reads.  A: lane (l % 16, l / 16) of block row tm reads 16 bytes of row
@@ -147,7 +167,15 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   // the k rows GROUP_K * g on of the slab (a second read takes the other half of them) for the
   // 16 columns of block column tn.
   uint32_t b_rd[TN];
-  {
+  if constexpr (B_KMAJOR) {
+    // as A's, per slab, once for block columns 0 .. 3 and once for 4 .. 7 (the rotated ones wrap round)
+    const int sw = ((lane & 15) / 2) & 7, group = lane >> 4;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const uint32_t at = lds0 + WIDE_B_BASE + (wn * WN + (lane & 15)) * BKB + (((4 * s + group) ^ sw) << 4);
+      b_rd[s] = at + (rot ? 4 * 16 * BKB : 0), b_rd[2 + s] = at - (rot ? 4 * 16 * BKB : 0);
+    }
+  } else {
     constexpr int LANES_PER_ROW = 16 / (8 / ES);
     const int p = lane & 15;
     const int k = GROUP_K * (lane >> 4) + p / LANES_PER_ROW;
@@ -175,8 +203,8 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   const uint32_t part_wr = part + (lane >> 4) * (BN * 4) + (rot ? 256 : 0);
   const uint32_t part_rd_lo = part + (rot ? 256 : 0), part_rd_hi = part - (rot ? 256 : 0);
 
-  const uint32_t b_step = uint32_t(BK) * ldb_b;
-  const uint32_t nk = g.k / BK, k32 = 32 * g.k;
+  const uint32_t b_step = B_KMAJOR ? uint32_t(BKB) : uint32_t(BK) * ldb_b;
+  const uint32_t nk = (g.k + BK - 1) / BK, k32 = 32 * nk * BK;   // (k32: what of K is zeroed counts in the sums of b + 128)
 
   // An accumulating Spec loads C's old values in nine of its first steps and adds them to the
   // accumulators a step later: one step after the other when K is short, with two or eleven steps
@@ -185,16 +213,45 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   // cycles longer (bf16 8192^3, cycle stamps), and close together they also ask HBM for all it
   // delivers (int8 4096^3: 64 MiB of C in the first quarter of the launch).
   const int spacing = !g.accum ? -1 : nk >= GEMM_WIDE_G11_MIN_STEPS ? 11 : nk >= GEMM_WIDE_G2_MIN_STEPS ? 2 : 0;
-#define MRL_WIDE_PICK(KIND)                                           \
-  do {                                                                \
-    if (spacing < 0) MRL_WIDE_RUN(GEMM_WIDE_##KIND);                  \
-    else if (spacing == 11) MRL_WIDE_RUN(GEMM_WIDE_##KIND##_ACC_G11); \
-    else if (spacing == 2) MRL_WIDE_RUN(GEMM_WIDE_##KIND##_ACC_G2);   \
-    else MRL_WIDE_RUN(GEMM_WIDE_##KIND##_ACC);                        \
+  if constexpr (EDGE) {
+    // Tile 0 is the last BK values of K; what the other tiles hold too, `skip` from its start, is zeroed.
+    const uint32_t skip_k = nk * BK - g.k;
+    const uint8_t *a_tail = A + int64_t(g.k - BK) * ES;
+    const uint8_t *b_tail = B + int64_t(g.k - BK) * (B_KMAJOR ? int64_t(ES) : int64_t(ldb_b));
+    const uint32_t a_keep = uint32_t(tid % 8) * 16 >= skip_k * ES ? ~0u : 0u;
+    // Where the lane's piece of B lies in K: for a k-fastest B in bytes, for even and odd instructions;
+    // else its k row for the first one.
+    const uint32_t skip = B_KMAJOR ? skip_k * ES : skip_k;
+    const uint32_t b_k[2] = {B_KMAJOR ? uint32_t((lane & 7) ^ (lane >> 4)) * 16 : uint32_t(wave * 8 * ROWS_PER_DMA + (lane * 16) / B_ROWB),
+                             uint32_t((lane & 7) ^ (lane >> 4 | 4)) * 16};
+    const uint32_t b_zero = dma_base + lane * 16;
+    // C: the resource ends with the last column of the wave's last row; a mask of lanes per block column.
+    const int rows = max(0, min(WM, m_left - wm * WM)), n_cols = max(0, min(WN, n_left - wn * WN));
+    const uint32_t c_records = __builtin_amdgcn_readfirstlane(rows && n_cols ? uint32_t(rows - 1) * ldc_b + n_cols * 4 + (rot ? 256 : 0) : 0);
+    uint64_t cols[TN];
+#pragma unroll
+    for (int t = 0; t < TN; t++) cols[t] = __ballot((t + rot) % TN * 16 + (lane & 15) < n_cols);
+#define MRL_WIDE_PICK(RUN, KIND)                        \
+  do {                                                  \
+    if (spacing < 0) RUN(GEMM_WIDE_##KIND);             \
+    else if (spacing == 11) RUN(GEMM_WIDE_##KIND##_ACC_G11); \
+    else if (spacing == 2) RUN(GEMM_WIDE_##KIND##_ACC_G2);   \
+    else RUN(GEMM_WIDE_##KIND##_ACC);                   \
   } while (0)
-  if constexpr (std::is_same<T, BF16>::value) MRL_WIDE_PICK(BF16);
-  else if constexpr (!A_UNSIGNED) MRL_WIDE_PICK(I8);
-  else MRL_WIDE_PICK(U8);
+    if constexpr (B_KMAJOR) {
+      if constexpr (std::is_same<T, BF16>::value) MRL_WIDE_PICK(MRL_WIDE_RUN_NT_EDGE, NT_EDGE_BF16);
+      else if constexpr (!A_UNSIGNED) MRL_WIDE_PICK(MRL_WIDE_RUN_NT_EDGE, NT_EDGE_I8);
+      else MRL_WIDE_PICK(MRL_WIDE_RUN_NT_EDGE, NT_EDGE_U8);
+    } else {
+      if constexpr (std::is_same<T, BF16>::value) MRL_WIDE_PICK(MRL_WIDE_RUN_NN_EDGE, EDGE_BF16);
+      else if constexpr (!A_UNSIGNED) MRL_WIDE_PICK(MRL_WIDE_RUN_NN_EDGE, EDGE_I8);
+      else MRL_WIDE_PICK(MRL_WIDE_RUN_NN_EDGE, EDGE_U8);
+    }
+  } else {
+    if constexpr (std::is_same<T, BF16>::value) MRL_WIDE_PICK(MRL_WIDE_RUN, BF16);
+    else if constexpr (!A_UNSIGNED) MRL_WIDE_PICK(MRL_WIDE_RUN, I8);
+    else MRL_WIDE_PICK(MRL_WIDE_RUN, U8);
+  }
 #undef MRL_WIDE_PICK
 }
 
@@ -216,22 +273,32 @@ inline bool wide_applicable(const GemmArgs &g, int elem_size) {
          g.ldc * 4 * 32 < (int64_t(1) << 31);
 }
 
-template <class T, bool A_UNSIGNED>
+// The ragged form: rows of whole 16-byte chunks, a K as long as the whole-tile form asks for (an
+// accumulating Spec's first steps carry C's old values here too).
+inline bool wide_edge_applicable(const GemmArgs &g, int elem_size) {
+  const int64_t per16 = 16 / elem_size, bk = 128 / elem_size;
+  auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  return !g.c_bf16 && al16(g.a) && al16(g.b) && g.k % per16 == 0 && g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 &&
+         g.sb % per16 == 0 && g.k >= WIDE_LONG_K_STEPS * bk && edge_addressable(g, elem_size) &&
+         g.ldb * elem_size * (bk + 1) < (int64_t(1) << 31);
+}
+
+template <class T, bool A_UNSIGNED, bool B_KMAJOR = false, bool EDGE = false>
 hipError_t launch_wide(const GemmArgs &g, hipStream_t stream) {
-  constexpr auto kern = k_gemm_wide<T, A_UNSIGNED>;
+  constexpr auto kern = k_gemm_wide<T, A_UNSIGNED, B_KMAJOR, EDGE>;
   static std::atomic<uint64_t> lds_limit_set{0};
   if (!plan::recording()) {
     hipError_t e = raise_lds_limit(lds_limit_set, (const void *)kern, WIDE_LDS_BYTES);
     if (e != hipSuccess) return e;
   }
-  const int tiles_m = int(g.m / 256), tiles_n = int(g.n / 256);
+  const int tiles_m = int((g.m + 255) / 256), tiles_n = int((g.n + 255) / 256);
   const double mn = double(g.m) * g.n * g.batch;
   plan::work(T::ES == 1 ? plan::UNIT_MFMA_I8 : plan::UNIT_MFMA_BF16, 2.0 * mn * g.k,
              (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * 4 * (g.accum ? 2 : 1),
              2.0 * 256 * 256 * double(g.k), 500.0 + 1200.0 * double(g.k * T::ES / 128),
              T::ES == 1 ? 1.62 : 1.18);  // measured: 2230-2330 TOPS int8 at 4096^3, 1360 TFLOPS bf16 at 8192^3
   const TileWalk walk = tile_walk(tiles_m, tiles_n);
-  MRL_LAUNCH((k_gemm_wide<T, A_UNSIGNED>), dim3(tiles_m * tiles_n, g.batch), dim3(256), WIDE_LDS_BYTES, stream,
+  MRL_LAUNCH((k_gemm_wide<T, A_UNSIGNED, B_KMAJOR, EDGE>), dim3(tiles_m * tiles_n, g.batch), dim3(256), WIDE_LDS_BYTES, stream,
              MRL_WALK_ARGS(walk), g);
   return mrl::plan::last_error();
 }

@@ -45,6 +45,18 @@ free as long as both operands agree, and here both hold bytes 16 g .. 16 g + 15 
     64 KB instruction cache: a body that does not fit is fetched anew by every launch, which cost
     100 to 350 cycles a step when the unrolled steps numbered eighteen.
 
+Two more forms of the same tile, each its own text (gen's nt and edge):
+  * nt: B is stored with k fastest.  Its tile is 256 rows of 128 bytes like A's, chunks XOR-ed with
+    (row / 2) & 7 on the source side of the direct-to-LDS loads, and an operand is one ds_read_b128
+    instead of two transposing reads.
+  * edge: any M and N, and any K of whole 16-byte chunks.  Rows and columns past the end are loaded as
+    copies of the last one (the kernel clamps the offsets); C is addressed through a buffer resource
+    whose end cuts off the rows, and a mask per block column cuts off the columns.  The tile that K
+    is not a whole number of is taken FIRST: tile 0 is the last 128 bytes of K, and what of it the
+    other tiles hold as well (%[skip] k from its start) is zeroed, in A's registers for bf16 (a NaN
+    times zero is no zero) and in B's LDS slot; the other tiles then count from the start of K.  Nothing in the
+    k loop knows of it.  The loop is left after any step.
+
 Register map (all named in the clobber list of the asm statement):
   a[0:255]    accumulators, block (tm, tn) at 4 * (8 * tm + tn); register i of lane l holds row
               4 * (l / 16) + i, column l % 16 of the block
@@ -58,6 +70,8 @@ Register map (all named in the clobber list of the asm statement):
   v[180:211]  old values of a block row of C
   s[60:61] A tile pointer   s[62:63] B tile pointer   s64 loop counter   s67 index of the next
   A tile to fetch, s68 of the next B tile   s[72:73] C block row pointer   s74 0x80808080   s69, s[78:79] scratch
+  edge: s[84:87] the buffer resource of C's block row, v[96:99] zeros before the loop; nt: v[160:163] the
+  lane's B operand addresses in the third slot, per slab and half of the block columns
 """
 import os
 import sys
@@ -182,7 +196,7 @@ class Item:
         self.gap = None
 
 
-def gen(kind, accum, opts=None, gap=0):
+def gen(kind, accum, opts=None, gap=0, nt=False, edge=False):
     """kind: 'u8' (A unsigned bytes), 'i8', 'bf16'.
     accum: the Spec accumulates into C (its old contents are read).
     gap: k steps of the loop run between two steps that load C's old values (0: those steps follow
@@ -198,6 +212,7 @@ def gen(kind, accum, opts=None, gap=0):
     add_in_memory = bool(accum and opts.get("atomic_c"))
     if add_in_memory:
         accum, gap = False, 0
+    assert not (edge and opts), "the experiments are written for whole tiles"
     unsigned = kind == "u8" and not opts.get("no_valu")
     is_float = kind == "bf16"
     mfma = "v_mfma_f32_16x16x32_bf16" if is_float else "v_mfma_i32_16x16x64_i8"
@@ -290,38 +305,89 @@ def gen(kind, accum, opts=None, gap=0):
         reg = bf(buf, tn, half)
         if opts.get("no_reads"):
             return lambda: None
+        if nt:
+            # one read for the whole operand, where the first half's stands
+            if half:
+                return lambda: None
+            # (block columns 4 .. 7 have addresses of their own: see the rotated columns below)
+            n = slab + (SLABS if tn >= TN // 2 else 0)
+            base = f"%[b_rd{n}]" if slot < 2 else f"v{B_ADDR + n}"
+            whole = bf(buf, tn)
+            off = (slot % 2) * B_SLOT + tn * 2048
+
+            def read():
+                e.lds_read(reg, f"ds_read_b128 {whole}, {base} offset:{off}")
+                e.producer[bf(buf, tn, 1)] = e.producer[reg]
+            return read
         base = f"%[b_rd{tn}]" if slot < 2 else f"v{B_ADDR + tn}"
         off = (slot % 2) * B_SLOT + slab * SLAB_BYTES + half * HI_BYTES
         return lambda: e.lds_read(reg, f"{tr} {reg}, {base} offset:{off}")
 
     # ---- prologue -------------------------------------------------------------------------
     E("s_mov_b32 s74, 0x80808080")      # in a register: a literal would double the size of every xor
-    E("s_mov_b64 s[60:61], %[abase]")
-    E("s_mov_b64 s[62:63], %[bbase]")
+    E("s_mov_b64 s[60:61], %[atail]" if edge else "s_mov_b64 s[60:61], %[abase]")
+    E("s_mov_b64 s[62:63], %[btail]" if edge else "s_mov_b64 s[62:63], %[bbase]")
     E("s_mov_b32 s67, 0")
     E("s_mov_b32 s68, 0")
+
+    def after_first(base, ptr, idx, advance):
+        """Behind tile 0: tile 1 is the first one of K when tile 0 was the last."""
+        if edge:
+            E(f"s_mov_b64 {ptr}, {base}")
+            E(f"s_mov_b32 {idx}, 1")
+        else:
+            advance()
+
     # A tiles 0 and 1 into the two register sets, B tiles 0 and 1 into slots 0 and 1
     for p in range(2):
         for i in range(8):
             load_a(p, i)
-        advance_a()
+        if p == 0:
+            after_first("%[abase]", "s[60:61]", "s67", advance_a)
+        else:
+            advance_a()
     for slot in range(2):
         set_m0(slot)
         for j in range(8):
             dma_b(j)
-        advance_b()
+        if slot == 0:
+            after_first("%[bbase]", "s[62:63]", "s68", advance_b)
+        else:
+            advance_b()
     for tn in range(TN):
         E(f"v_mov_b32 v{COL_SUM + tn}, 0")
     for i in range(8):
+        if edge and is_float:
+            e.vm_need(areg(0, i))
+            for w in range(4):
+                E(f"v_and_b32 {areg(0, i, w)}, %[a_keep], {areg(0, i, w)}")
         store_a(0, i, 0)            # waits for A tile 0 only
     for i in range(8):
         load_a(0, i)                # A tile 2
     advance_a()
     e.vm_wait_index(e.vm_issued - 9)  # all but A tile 2: B tiles 0 and 1 have landed
+    if edge:
+        # What of tile 0 belongs to other tiles too: zeros over the lane's piece j of it where its k lies
+        # before %[skip].  A wave writes over its own pieces, which have landed.
+        E("s_cmp_eq_u32 %[skip], 0")
+        E("s_cbranch_scc1 50f")
+        for w in range(4):
+            E(f"v_mov_b32 v{96 + w}, 0")
+        for j in range(8):
+            if nt:
+                E(f"v_cmp_gt_u32 vcc, %[skip], %[b_k{j % 2}]")
+            else:
+                rows = 2 if is_float else 4
+                E(f"v_add_u32 v{TMP0}, {j * rows}, %[b_k0]")
+                E(f"v_cmp_gt_u32 vcc, %[skip], v{TMP0}")
+            E("s_mov_b64 exec, vcc")
+            e.lds_write(f"ds_write_b128 %[b_zero], v[96:99] offset:{j * 1024}")
+            E("s_mov_b64 exec, -1")
+        E("50:")
     E("s_waitcnt lgkmcnt(0)")
     e.all_lds_done()
     E("s_barrier")
-    for tn in range(TN):
+    for tn in range(2 * SLABS if nt else TN):
         E(f"v_add_u32 v{B_ADDR + tn}, {2 * B_SLOT}, %[b_rd{tn}]")
     # What a step expects to find: slab 0's B operands in set 0 and its A operands but the last,
     # which every step reads behind its first MFMA.
@@ -461,6 +527,18 @@ def gen(kind, accum, opts=None, gap=0):
         if ptr_tm[0] == tm:
             return
         ptr_tm[0] = tm
+        if edge:
+            # the buffer resource: what is left of C from the block row on
+            E("s_mov_b64 s[84:85], %[cbase]")
+            E("s_mov_b32 s86, %[crec]")
+            if tm:
+                E(f"s_mul_i32 s78, %[ldc16], {tm}")
+                E("s_add_u32 s84, s84, s78")
+                E("s_addc_u32 s85, s85, 0")
+                E("s_sub_u32 s86, s86, s78")
+                E("s_cselect_b32 s86, 0, s86")
+            E("s_mov_b32 s87, 0x00020000")
+            return
         E("s_mov_b64 s[72:73], %[cbase]")
         if tm:
             E(f"s_mul_i32 s78, %[ldc16], {tm}")
@@ -523,6 +601,9 @@ def gen(kind, accum, opts=None, gap=0):
             if j < C_STEPS:
                 def ld(tn=tn, i=i, reg=reg):
                     c_ptr(j)
+                    if edge:
+                        e.vm(f"buffer_load_dword {reg}, {c_addr(tn, i)}, s[84:87], 0 offen offset:{tn * 64}", dst=reg)
+                        return
                     e.vm(f"global_load_dword {reg}, {c_addr(tn, i)}, s[72:73] offset:{tn * 64}{c_load_hint}", dst=reg)
                 out.append(Item(ld, 1, g, GAPS - 1, after=add_item))
         return out
@@ -532,6 +613,14 @@ def gen(kind, accum, opts=None, gap=0):
         `first` (the number of unrolled steps before it, modulo six)."""
         if first % 6:
             E(f"s_branch 1{first % 6}f")
+        if edge:
+            for pos in range(6):
+                E(f"1{pos}:")
+                step(pos)
+                E("s_sub_u32 s64, s64, 1")
+                E("s_cmp_lg_u32 s64, 0")
+                E("s_cbranch_scc1 10b" if pos == 5 else "s_cbranch_scc0 2f")
+            return
         for pos in (0, 2, 4):
             E(f"1{pos}:")
             step(pos)
@@ -675,6 +764,15 @@ def gen(kind, accum, opts=None, gap=0):
         for q in range(early, 256):
             tm, tn, i = where(q)
             c_ptr(tm)
+            if edge:
+                if i == 0:
+                    E(f"s_mov_b64 exec, %[cm{tn}]")
+                t = f"v{16 + q % 32}"
+                E(f"v_accvgpr_read_b32 {t}, a{q}")
+                if unsigned:
+                    E(f"v_add_u32 {t}, {t}, v{COL_SUM + tn}")
+                E(f"buffer_store_dword {t}, {c_addr(tn, i)}, s[84:87], 0 offen offset:{tn * 64}")
+                continue
             out = "global_store_dword"
             if add_in_memory:
                 out = "global_atomic_add_f32" if is_float else "global_atomic_add"
@@ -685,6 +783,8 @@ def gen(kind, accum, opts=None, gap=0):
                 E(f"v_accvgpr_read_b32 {t}, a{q}")
                 E(f"v_add_u32 {t}, {t}, v{COL_SUM + tn}")
                 E(f"{out} {c_addr(tn, i)}, {t}, s[72:73] offset:{tn * 64}{st_flags}")
+    if edge:
+        E("s_mov_b64 exec, -1")
     if trace:
         # The stamps replace the first rows of the wave's block of C (a timing build: its results are
         # not looked at): value j at row j % 4, columns 16 * (j / 4) .. + 15 of the block.
@@ -722,6 +822,14 @@ def variants():
         yield f"GEMM_WIDE_{kind.upper()}_ACC", kind, True, 0
         for gap in SPACED_GAPS:
             yield f"GEMM_WIDE_{kind.upper()}_ACC_G{gap}", kind, True, gap
+    # Ragged tiles, either orientation of B (whole tiles of a k-fastest B among them).
+    for kind in ("u8", "i8", "bf16"):
+        for nt in (False, True):
+            name = f"GEMM_WIDE_{'NT_' if nt else ''}EDGE_{kind.upper()}"
+            yield name, kind, False, 0, nt, True
+            yield name + "_ACC", kind, True, 0, nt, True
+            for gap in SPACED_GAPS:
+                yield f"{name}_ACC_G{gap}", kind, True, gap, nt, True
 
 
 def main():
@@ -742,8 +850,8 @@ def main():
              f"#define GEMM_WIDE_MIN_STEPS {MIN_STEPS}\n"]
     for gap in SPACED_GAPS:
         parts.append(f"#define GEMM_WIDE_G{gap}_MIN_STEPS {spaced_min_steps(gap)}\n")
-    for name, kind, accum, gap in variants():
-        lines = gen(kind, accum, opts, gap)
+    for name, kind, accum, gap, *form in variants():
+        lines = gen(kind, accum, None if form else opts, gap, *form)
         body = " \\\n".join('  "' + l + '\\n"' for l in lines)
         parts.append(f"#define {name} \\\n{body}\n")
     with open(out_path, "w") as f:

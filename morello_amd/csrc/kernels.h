@@ -174,6 +174,8 @@ hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint
 // Always the 256 x 256 tile, 128 bytes of K per step.
 // staging: 0 = whichever of the 256 x 256 kernels applies (four waves, eight waves, compiler-scheduled),
 // 1 / 2 / 3 = mrl_staging's REGISTERS / DIRECT_B / DIRECT_B_WIDE only (hipErrorInvalidValue where that one does not apply).
+// gemm_wide_edge.hip: the four-wave tile on ragged shapes and against a k-fastest B.
+hipError_t launch_gemm_wide_edge(const GemmArgs &g, int kind, hipStream_t stream);
 hipError_t launch_gemm_big(const GemmArgs &g, int kind, hipStream_t stream, uint32_t staging = 0);
 
 // ---- gemv.hip: at most four rows of A against a k-fastest B, as dot products (a stream over B) ----
