@@ -1,0 +1,336 @@
+// Conv NHWC u8|i8 x KRSC i8 -> i32 and bf16 x bf16 -> f32 for pixels of three or four channels (a first
+// layer), channels-last (morello/src/spec.rs:486-494: no stride, no padding): the form of
+// conv_windows.hip's kernel that needs no windows in LDS.
+//
+// What bounds such a layer is its output (16 x 109 x 109 x 64 floats: 49 MB against 1 MB of image) as long as
+// nothing else takes time; the other form's chain of patch, barrier, copied windows, barrier, MFMAs per
+// 128 pixels did (that layer in bf16, 7 x 7: 27.5 us).  Here a pixel takes four elements in LDS,
+// the fourth zero if there are three, so a window's row is a run of whole pixels at an address a
+// multiple of the pixel apart and MFMA operands are read where they lie:
+//   - a row of a window is 1, 2 or 4 chunks of 16 bytes (cpr; three are taken as four), a k step of 64
+//     bytes is 4 / cpr rows, and what a lane reads for step s lies s * 4 / cpr patch rows below what it
+//     reads for step 0: one address per lane, whatever the filter's size;
+//   - a wave works alone on 16 x 2 output pixels, its patch in LDS of its own: no barrier after the
+//     filters are staged.  The next item's pixels are fetched while this one is multiplied;
+//   - filters lie in the same order, zeros wherever no pixel is.  Floats: window positions
+//     past the filter's width or height are zeroed as well (a NaN there times zero is not zero).
+// A lane holds four consecutive filters of a pixel: 16 bytes, four lanes 64 contiguous ones, and two
+// such stores fill a cache line: they go through the L2 (past it, 32 x 3 -> 96 x 224 x 224 took 209 us).
+// Measured, the other form / this (us, TB/s of image, filters and output): bf16 7 x 7 16 x 3 -> 64 x 109^2 28.1 / 17.0,
+// 2.9; 32 x 3 -> 96 x 224^2 298 / 146, 4.3; 1 x 3 -> 64 x 109^2 10.4 / 5.4; 3 x 3 32 x 4 -> 16 x 224^2 80 / 23, 5.0; u8 7 x 7
+// 16 x 3 -> 64 x 109^2 23.0 / 15.1.  Items of four rows: 1 x 3 -> 64 x 109^2 6.9, 3 x 3 22.1, the others within 3 %.
+#include <algorithm>
+
+#include "kernels.h"
+#include "plan.h"
+
+namespace mrl {
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+enum { IMG_I8 = 0, IMG_U8 = 1, IMG_BF16 = 2 };
+
+constexpr int WAVES = 8, ITEM_W = 16, ITEM_H = 2;
+constexpr int HELD = 4;   // patch pixels a lane holds in flight
+constexpr int FB = 2;     // blocks of 16 filters multiplied at a time
+
+struct PixelsArgs {
+  const uint8_t *image, *filters;
+  int32_t *out;
+  uint32_t f, oh, ow, h, w, fh, fw;
+  uint32_t group;               // filters a workgroup takes, a multiple of 32
+  uint32_t pixel_bytes;         // of a pixel in memory: 3 or 4 elements
+  int accum;
+  uint32_t items, steps;        // 16 x 2 pieces of the output; k steps (KS whole ones and perhaps a tail)
+  uint32_t chunks_log2;         // log2 of cpr
+  uint32_t slots;               // pixels of a filter's row in LDS: steps * 64 / PB
+  uint32_t patch_w, patch_h;    // pixels
+  uint32_t patch_bytes;         // of LDS, rows that only a tail step's masked lanes read included
+  FastDiv by_image, by_row, by_slots, by_patch_w;   // items of an image, of an image's row of them
+};
+
+// KS: whole k steps of 64 bytes (a window's chunks / 4); the rest is a tail whose lanes past the
+// filter's last row count for nothing.
+template <int KS, int KIND>
+__global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
+  constexpr bool HALVES = KIND == IMG_BF16;
+  constexpr int ES = HALVES ? 2 : 1, PB = 4 * ES, PIXELS = 16 / PB;   // bytes of a pixel in LDS, pixels of a chunk
+  typedef typename std::conditional<HALVES, v4f, v4i>::type Acc;
+  auto mfma = [](v4i a, v4i b, Acc c) {
+    if constexpr (HALVES) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
+  };
+  struct Pixel { uint32_t v[ES]; };
+  struct Raw { uint32_t v[ES + 1]; uint32_t shift; };
+  // A pixel out of the aligned dwords it lies in (a dword without a byte of it is not read).
+  auto fetch = [&](const uint8_t *at) {
+    Raw r;
+    r.shift = uint32_t(reinterpret_cast<uintptr_t>(at)) & 3;
+    const uint32_t *from = reinterpret_cast<const uint32_t *>(at - r.shift);
+#pragma unroll
+    for (int i = 0; i < ES; i++) r.v[i] = from[i];
+    r.v[ES] = from[r.shift + p.pixel_bytes > 4 * ES ? ES : ES - 1];
+    return r;
+  };
+  const uint32_t last_mask = p.pixel_bytes == PB ? 0xffffffffu : HALVES ? 0xffffu : 0xffffffu;
+  auto pixel = [&](const Raw &r) {
+    Pixel x;
+#pragma unroll
+    for (int i = 0; i < ES; i++) x.v[i] = __builtin_amdgcn_alignbyte(r.v[i + 1], r.v[i], r.shift);
+    x.v[ES - 1] &= last_mask;
+    return x;
+  };
+  auto put = [&](uint8_t *to, const Pixel &x) {
+    if constexpr (HALVES) *(v2u *)to = v2u{x.v[0], x.v[ES - 1]};
+    else *(uint32_t *)to = x.v[0];
+  };
+  extern __shared__ __attribute__((aligned(16))) uint8_t pix_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t filter_row = p.steps * 64 + 16;   // 16 bytes more than the length: spreads an operand read over the banks
+  uint8_t *filt = pix_lds;
+  uint8_t *patch = pix_lds + p.group * filter_row + wave * p.patch_bytes;
+  const uint32_t f0 = blockIdx.y * p.group, nf = min(p.group, p.f - f0);   // this workgroup's filters (a multiple of 16)
+
+  // Where in a patch a lane's held pixels are does not depend on the item.
+  uint32_t held_y[HELD], held_x[HELD];
+  const uint32_t patch_pixels = p.patch_w * p.patch_h;
+#pragma unroll
+  for (int j = 0; j < HELD; j++) {
+    const uint32_t i = lane + j * 64;
+    held_y[j] = p.by_patch_w.div(i), held_x[j] = i - held_y[j] * p.patch_w;
+  }
+  struct Corner { uint32_t img, y0, x0; };
+  const uint32_t tiles_x = (p.ow + ITEM_W - 1) / ITEM_W, per_image = tiles_x * ((p.oh + ITEM_H - 1) / ITEM_H);
+  auto corner_of = [&](uint32_t item) {
+    const uint32_t img = p.by_image.div(item), in_img = item - img * per_image, ty = p.by_row.div(in_img);
+    return Corner{img, ty * ITEM_H, (in_img - ty * tiles_x) * ITEM_W};
+  };
+  // (past the image's edge, its last row or pixel again: those reach only results that are not
+  // stored, or positions past the filter's width)
+  auto source = [&](const Corner &at, uint32_t r, uint32_t x) {
+    return p.image + ((uint64_t(at.img) * p.h + min(at.y0 + r, p.h - 1)) * p.w + min(at.x0 + x, p.w - 1)) * p.pixel_bytes;
+  };
+  Raw held[HELD];
+  auto fetch_patch = [&](const Corner &at) {
+#pragma unroll
+    for (int j = 0; j < HELD; j++)
+      if (lane + j * 64 < int(patch_pixels)) held[j] = fetch(source(at, held_y[j], held_x[j]));
+  };
+  const uint32_t stride = gridDim.x * WAVES;
+  uint32_t item = blockIdx.x * WAVES + wave;
+  if (item < p.items) fetch_patch(corner_of(item));   // in flight while the filters are staged
+  // The filters: their bytes are one contiguous piece of memory, fetched in whole chunks with the loads in
+  // flight together (into what will be the patches), then spread out pixel by pixel.
+  {
+    const uint32_t filter_bytes = p.fh * p.fw * p.pixel_bytes;
+    const uint8_t *from = p.filters + uint64_t(f0) * filter_bytes;
+    const uint32_t head = uint32_t(reinterpret_cast<uintptr_t>(from)) & 15, chunks = (head + nf * filter_bytes + 15) / 16;
+    const v4i *first = reinterpret_cast<const v4i *>(from - head);
+    v4i *raw = reinterpret_cast<v4i *>(filt + p.group * filter_row);
+    constexpr uint32_t BATCH = 3;
+    for (uint32_t c0 = 0; c0 < chunks; c0 += BATCH * 64 * WAVES) {
+      v4i got[BATCH];
+#pragma unroll
+      for (uint32_t j = 0; j < BATCH; j++) got[j] = first[min(c0 + j * 64 * WAVES + tid, chunks - 1)];
+#pragma unroll
+      for (uint32_t j = 0; j < BATCH; j++)
+        if (c0 + j * 64 * WAVES + tid < chunks) raw[c0 + j * 64 * WAVES + tid] = got[j];
+    }
+    __syncthreads();
+    const uint32_t *words = reinterpret_cast<const uint32_t *>(raw);
+    const uint32_t per_row = uint32_t(PIXELS) << p.chunks_log2;   // pixels a window's row takes
+#pragma unroll 2
+    for (uint32_t i = tid; i < p.group * p.slots; i += 64 * WAVES) {
+      const uint32_t fi = p.by_slots.div(i), s = i - fi * p.slots;
+      const uint32_t r = s / PIXELS >> p.chunks_log2, x = s & (per_row - 1);
+      const bool real = fi < nf && r < p.fh && x < p.fw;
+      const uint32_t at = real ? head + ((fi * p.fh + r) * p.fw + x) * p.pixel_bytes : head;
+      Raw px;
+#pragma unroll
+      for (int w = 0; w <= ES; w++) px.v[w] = words[at / 4 + w];
+      px.shift = at & 3;
+      put(filt + fi * filter_row + s * PB, real ? pixel(px) : Pixel{});
+    }
+    __syncthreads();   // the raw bytes are no longer needed
+  }
+  const uint8_t *my_filt = filt + li * filter_row + lg * 16;
+  // u8 pixels are multiplied as a - 128: 128 times a filter's sum comes on top (kept in LDS, in the
+  // 16 bytes between the filters' rows).
+  if constexpr (KIND == IMG_U8) {
+    const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    for (uint32_t fb = wave; fb < p.group / 16; fb += WAVES) {
+      Acc sum = {};
+      for (uint32_t ks = 0; ks < p.steps; ks++) sum = mfma(*(const v4i *)(my_filt + fb * 16 * filter_row + ks * 64), ones, sum);
+      if (li == 0) *(v4i *)(filt + (fb * 16 + lg) * filter_row + p.steps * 64) = sum * 128;
+    }
+    __syncthreads();
+  }
+  // This lane's chunk of a step: row lg / cpr of the step's, chunk lg % cpr of the row.
+  const uint32_t row_bytes = p.patch_w * PB, chunk = lg & ((1u << p.chunks_log2) - 1), row_of = uint32_t(lg) >> p.chunks_log2;
+  const uint32_t step_bytes = (4u >> p.chunks_log2) * row_bytes;
+  const uint8_t *my_patch = patch + row_of * row_bytes + li * PB + chunk * 16;
+  const uint32_t keep_lo = chunk * PIXELS < p.fw ? 0xffffffffu : 0u, keep_hi = chunk * PIXELS + 1 < p.fw ? 0xffffffffu : 0u;
+  auto window = [&](uint32_t ks, int pb) {
+    const uint8_t *at = my_patch + ks * step_bytes + pb * row_bytes;
+    if constexpr (HALVES) {
+      const v2u lo = *(const v2u *)at & keep_lo, hi = *(const v2u *)(at + 8) & keep_hi;
+      return v4i{int(lo[0]), int(lo[1]), int(hi[0]), int(hi[1])};
+    } else {
+      const uint32_t *w = (const uint32_t *)at;
+      return v4i{int(w[0]), int(w[1]), int(w[2]), int(w[3])};
+    }
+  };
+  for (; item < p.items; item += stride) {
+    const Corner at = corner_of(item);
+#pragma unroll
+    for (int j = 0; j < HELD; j++)
+      if (lane + j * 64 < int(patch_pixels)) {
+        Pixel x = pixel(held[j]);
+        if (KIND == IMG_U8) x.v[0] ^= 0x80808080u;
+        put(patch + (lane + j * 64) * PB, x);
+      }
+    for (uint32_t i = lane + HELD * 64; i < patch_pixels; i += 64) {
+      const uint32_t r = p.by_patch_w.div(i);
+      Pixel x = pixel(fetch(source(at, r, i - r * p.patch_w)));
+      if (KIND == IMG_U8) x.v[0] ^= 0x80808080u;
+      put(patch + i * PB, x);
+    }
+    // The wave's LDS accesses complete in order: what is left is that the compiler keeps them so.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (item + stride < p.items) fetch_patch(corner_of(item + stride));
+    // Two blocks of filters at a time: with four at once the registers of half as many waves.
+#pragma unroll 1
+    for (uint32_t fb0 = 0; fb0 < nf; fb0 += 16 * FB) {
+      asm volatile("" : : : "memory");   // (else the window operands of all steps are kept from pass to pass, and spill)
+      Acc acc[ITEM_H][FB];
+#pragma unroll
+      for (int fb = 0; fb < FB; fb++) {
+        Acc from = {};
+        if constexpr (KIND == IMG_U8) from = *(const v4i *)(filt + (fb0 + fb * 16 + lg) * filter_row + p.steps * 64);
+#pragma unroll
+        for (int pb = 0; pb < ITEM_H; pb++) acc[pb][fb] = from;
+      }
+      const uint8_t *block = my_filt + fb0 * filter_row;
+      auto step = [&](uint32_t ks, bool inside) {
+        v4i a[FB], bop[ITEM_H];
+#pragma unroll
+        for (int fb = 0; fb < FB; fb++) a[fb] = *(const v4i *)(block + fb * 16 * filter_row + ks * 64);
+#pragma unroll
+        for (int pb = 0; pb < ITEM_H; pb++) {
+          bop[pb] = window(ks, pb);
+          if (HALVES && !inside) bop[pb] = v4i{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int pb = 0; pb < ITEM_H; pb++)
+#pragma unroll
+          for (int fb = 0; fb < FB; fb++) acc[pb][fb] = mfma(a[fb], bop[pb], acc[pb][fb]);
+      };
+#pragma unroll 2
+      for (int ks = 0; ks < KS; ks++) step(ks, true);
+      if (p.steps > KS) step(KS, KS * (4u >> p.chunks_log2) + row_of < p.fh);
+      const uint32_t x = at.x0 + li;
+#pragma unroll
+      for (int pb = 0; pb < ITEM_H; pb++) {
+        const uint32_t y = at.y0 + pb;
+        if (y < p.oh && x < p.ow) {
+          Acc *d = (Acc *)(p.out + ((uint64_t(at.img) * p.oh + y) * p.ow + x) * p.f + f0 + fb0 + 4 * lg);
+#pragma unroll
+          for (int fb = 0; fb < FB; fb++)
+            if (fb0 + fb * 16 < nf) {
+              Acc v = acc[pb][fb];
+              if (p.accum) v += d[4 * fb];
+              d[4 * fb] = v;
+            }
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <int KS, int KIND>
+hipError_t launch(const PixelsArgs &p, dim3 grid, size_t lds, hipStream_t stream) {
+  static std::atomic<uint64_t> limit{0};
+  if (!plan::recording() && lds > 65536) {
+    hipError_t e = raise_lds_limit(limit, (const void *)k_conv_windows<KS, KIND>, int(lds));
+    if (e != hipSuccess) return e;
+  }
+  MRL_LAUNCH((k_conv_windows<KS, KIND>), grid, dim3(64 * WAVES), lds, stream, p);
+  return plan::last_error();
+}
+template <int KS>
+hipError_t launch_ks(const PixelsArgs &p, int kind, dim3 grid, size_t lds, hipStream_t stream) {
+  switch (kind) {
+    case IMG_I8: return launch<KS, IMG_I8>(p, grid, lds, stream);
+    case IMG_U8: return launch<KS, IMG_U8>(p, grid, lds, stream);
+    default: return launch<KS, IMG_BF16>(p, grid, lds, stream);
+  }
+}
+
+constexpr uint32_t MAX_KS = 7;
+
+uint32_t chunks_log2_of(const ConvArgs &c, int kind) {   // chunks of 16 bytes of a window's row, as 1, 2 or 4
+  const uint32_t pixels = kind == IMG_BF16 ? 2 : 4, chunks = (c.fw + pixels - 1) / pixels;
+  return chunks <= 1 ? 0 : chunks <= 2 ? 1 : chunks <= 4 ? 2 : 3;
+}
+
+}  // namespace
+
+bool conv_pixels_applicable(const ConvArgs &c, int kind) {
+  if (kind < 0 || kind > 2 || c.in_planes || c.out_planes || c.c < 3 || c.c > 4 || c.f % 16 != 0) return false;
+  const uint32_t log2 = chunks_log2_of(c, kind), es = kind == IMG_BF16 ? 2 : 1;
+  if (log2 > 2 || ((uint64_t(c.fh) << log2) + 3) / 4 > MAX_KS) return false;
+  const uint64_t items = uint64_t(c.b) * ((c.oh + ITEM_H - 1) / ITEM_H) * ((c.ow + ITEM_W - 1) / ITEM_W);
+  return items < (1ull << 30) && (c.f + 31) / 32 < 65535 && (reinterpret_cast<uintptr_t>(c.out) & 15) == 0 &&
+         ((reinterpret_cast<uintptr_t>(c.image) | reinterpret_cast<uintptr_t>(c.filters)) & (es - 1)) == 0;
+}
+
+hipError_t launch_conv_pixels(const ConvArgs &c, int kind, hipStream_t stream) {
+  if (!conv_pixels_applicable(c, kind)) return hipErrorInvalidValue;
+  const uint32_t es = kind == IMG_BF16 ? 2 : 1, pb = 4 * es;
+  PixelsArgs p;
+  p.image = (const uint8_t *)c.image, p.filters = (const uint8_t *)c.filters, p.out = (int32_t *)c.out;
+  p.f = c.f, p.oh = c.oh, p.ow = c.ow, p.fh = c.fh, p.fw = c.fw, p.h = c.oh + c.fh - 1, p.w = c.ow + c.fw - 1;
+  p.pixel_bytes = c.c * es, p.accum = c.accum;
+  p.chunks_log2 = chunks_log2_of(c, kind);
+  const uint32_t rows_per_step = 4u >> p.chunks_log2, whole = c.fh / rows_per_step;
+  p.steps = (c.fh + rows_per_step - 1) / rows_per_step;
+  p.slots = p.steps * 64 / pb;
+  p.patch_w = ITEM_W - 1 + ((16 / pb) << p.chunks_log2), p.patch_h = ITEM_H + c.fh - 1;
+  p.patch_bytes = ((ITEM_H + p.steps * rows_per_step - 1) * p.patch_w * pb + 15) & ~15u;
+  const uint32_t tiles_x = (c.ow + ITEM_W - 1) / ITEM_W, per_image = tiles_x * ((c.oh + ITEM_H - 1) / ITEM_H);
+  p.items = c.b * per_image;
+  p.by_image = FastDiv(per_image), p.by_row = FastDiv(tiles_x), p.by_slots = FastDiv(p.slots), p.by_patch_w = FastDiv(p.patch_w);
+  // All filters of up to 128 in one workgroup, so that a pixel is staged once; 32 at a time where that
+  // would leave compute units without work.
+  const uint64_t wanted = (uint64_t(p.items) + WAVES - 1) / WAVES;
+  p.group = c.f <= 32 || wanted * 2 <= g_compute_units ? 32 : c.f <= 128 ? (c.f + 31) & ~31u : 64;
+  const uint32_t groups = (c.f + p.group - 1) / p.group;
+  // behind the filters the patches, and before them the filters as they lie in memory (16 bytes more on either side)
+  const size_t raw = size_t(std::min(c.f, p.group)) * c.fh * c.fw * p.pixel_bytes + 32;
+  const size_t lds = p.group * (p.steps * 64 + 16) + std::max(raw, WAVES * size_t(p.patch_bytes));
+  // Two workgroups to a compute unit walk the items, so that the filters are staged once each.
+  const uint32_t wgs = std::min<uint32_t>((p.items + WAVES - 1) / WAVES, std::max(1u, 2 * g_compute_units / groups));
+  const double pixels = double(c.b) * c.oh * c.ow;
+  plan::work(plan::UNIT_STREAM, 0, 1.5 * (pixels * c.f * 4 * (c.accum ? 2 : 1) + double(c.b) * p.h * p.w * p.pixel_bytes), 0,
+             4000.0 + (1000.0 + 200.0 * p.steps) * double((p.items + wgs * WAVES - 1) / (wgs * WAVES)));   // staging the filters; an item
+  const dim3 grid(wgs, groups);
+  switch (whole) {
+    case 0: return launch_ks<0>(p, kind, grid, lds, stream);
+    case 1: return launch_ks<1>(p, kind, grid, lds, stream);
+    case 2: return launch_ks<2>(p, kind, grid, lds, stream);
+    case 3: return launch_ks<3>(p, kind, grid, lds, stream);
+    case 4: return launch_ks<4>(p, kind, grid, lds, stream);
+    case 5: return launch_ks<5>(p, kind, grid, lds, stream);
+    case 6: return launch_ks<6>(p, kind, grid, lds, stream);
+    default: return launch_ks<7>(p, kind, grid, lds, stream);
+  }
+}
+
+}  // namespace mrl

@@ -335,6 +335,7 @@ bool conv_windows_applicable(const ConvArgs &c, int kind) {
 
 hipError_t launch_conv_windows(const ConvArgs &c, int kind, hipStream_t stream) {
   if (!conv_windows_applicable(c, kind)) return hipErrorInvalidValue;
+  if (conv_pixels_applicable(c, kind)) return launch_conv_pixels(c, kind, stream);
   const uint32_t es = kind == 3 ? 4 : kind == 2 ? 2 : 1;
   WindowsArgs p;
   p.image = (const uint8_t *)c.image, p.filters = (const uint8_t *)c.filters, p.out = (int32_t *)c.out;

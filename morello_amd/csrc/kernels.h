@@ -222,6 +222,9 @@ bool conv_small_applicable(const ConvArgs &c, int kind);
 hipError_t launch_conv_small(const ConvArgs &c, int kind, hipStream_t stream);
 bool conv_windows_applicable(const ConvArgs &c, int kind);
 hipError_t launch_conv_windows(const ConvArgs &c, int kind, hipStream_t stream);
+// conv_pixels.hip: the form of it for three or four channels, int8 or bf16, channels-last (launch_conv_windows goes there).
+bool conv_pixels_applicable(const ConvArgs &c, int kind);
+hipError_t launch_conv_pixels(const ConvArgs &c, int kind, hipStream_t stream);
 
 // ---- unfold.hip: the windows of a channels-last image as rows, for Conv as a Matmul ---------
 // image: [batch][oh+fh-1][ow+fw-1][c]; rows: [batch*oh*ow][row_elems], each row the fh*fw*c

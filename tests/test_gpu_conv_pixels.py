@@ -1,0 +1,70 @@
+"""First-layer Conv on pixels of three or four channels (conv_pixels.hip) against the oracle."""
+import numpy as np
+import pytest
+
+import morello_amd as M
+import orc
+from morello_amd import synth
+from gpu_util import run_spec
+
+pytestmark = pytest.mark.gpu
+NHWC = orc.make_layout([0, 2, 3, 1])
+TYPES = {"u8": ((M.u8, M.i8, M.i32), [0, 1, 5]), "i8": ((M.i8, M.i8, M.i32), [1, 1, 5]), "bf16": ((M.bf16, M.bf16, M.f32), [7, 7, 6])}
+
+
+@pytest.mark.parametrize("types", ["u8", "i8", "bf16"])
+@pytest.mark.parametrize("shape,accum", [
+    ((1, 16, 3, 1, 1, 1, 1), False),        # (times 4e5 images below: a single pixel each)
+    ((3, 32, 4, 5, 17, 1, 4), True),        # one row of a window, a pixel past an item's edge both ways
+    ((2, 48, 3, 4, 16, 2, 3), False),       # whole items, blocks of filters that end inside a group
+    ((2, 80, 4, 7, 33, 5, 2), True),        # a second group of one block
+    ((1, 96, 3, 30, 31, 3, 8), False),      # eight pixels a row: the widest of bf16
+    ((2, 64, 4, 19, 18, 7, 5), True),
+    ((1, 16, 3, 21, 15, 6, 6), False),
+    ((5, 16, 3, 230, 250, 3, 3), False),    # several items a wave
+    ((2, 112, 3, 101, 130, 3, 3), True),    # 112 filters in one group, the last pair half empty
+    ((2, 144, 3, 101, 130, 2, 2), False),   # groups of 64, the last of one block
+    ((1, 64, 3, 9, 20, 14, 7), False),      # int8: a patch of more pixels than a wave holds in flight
+    ((1, 32, 3, 12, 12, 4, 13), True),      # int8: four chunks a row
+])
+def test_three_and_four_channels(gpu, shape, accum, types):
+    """Integers bit for bit, bf16 to 1e-5 of the largest (f32 sums of at most 400 products in another order), from
+    operands one element into their buffers; NaN and infinity in a bf16 image reach the outputs whose
+    windows hold them and no others."""
+    dts, codes = TYPES[types]
+    b, f, c, oh, ow, fh, fw = shape
+    if (oh, ow) == (1, 1):
+        b = 2500
+        shape = (b,) + shape[1:]
+    gen = {M.u8: synth.uniform_u8, M.i8: synth.uniform_i8, M.bf16: synth.normal_bf16}
+    img, filt = gen[dts[0]](160, 0, (b, oh + fh - 1, ow + fw - 1, c)), gen[dts[1]](160, 1, (f, fh, fw, c))
+    out0 = synth.uniform_u8(160, 2, (b, oh, ow, f)).astype(np.float32 if types == "bf16" else np.int32) - 100
+    spec = M.Conv(list(shape), dts, accum=accum)
+    if types != "bf16" or fw <= 8 and fh * fw <= 49:   # (beyond that, another kernel's)
+        assert spec.plan().kernels == ["k_conv_windows"] and spec.plan().steps[0].block[0] == 512
+
+    def run(image, shift):
+        held = [np.zeros(x.size + shift, x.dtype) for x in (image, filt)]
+        held[0][shift:], held[1][shift:] = image.reshape(-1), filt.reshape(-1)
+        bufs = [M.DeviceBuffer.from_numpy(x) for x in held + [out0]]
+        spec.run_device([bufs[0].ptr + shift * img.itemsize, bufs[1].ptr + shift * filt.itemsize, bufs[2].ptr])
+        got = bufs[2].to_numpy(out0.dtype, out0.shape)
+        for x in bufs:
+            x.free()
+        return got
+
+    want = orc.conv(list(shape), codes, img, filt, out0.copy(), accum, layouts=[NHWC] * 3)
+    for shift in (0, 1):
+        got = run(img, shift)
+        if types != "bf16":
+            assert np.array_equal(got, want)
+        else:
+            assert float(np.abs(got.astype(np.float64) - want).max() / np.abs(want).max()) < 1e-5
+    if types == "bf16":
+        img = img.copy()
+        img[0, 0, 0, 0], img[b - 1, oh + fh - 2, ow + fw - 2, c - 1], img[0, (oh + fh - 1) // 2, (ow + fw - 1) // 2, 1] = 0x7fc0, 0x7f80, 0xff80
+        want = orc.conv(list(shape), codes, img, filt, out0.copy(), accum, layouts=[NHWC] * 3)
+        got = run(img, 0)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        ok = np.isfinite(want)
+        assert not ok.any() or float(np.abs(got[ok].astype(np.float64) - want[ok]).max() / np.abs(want[ok]).max()) < 1e-5
