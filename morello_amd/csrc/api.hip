@@ -485,7 +485,10 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     // Rows of another tensor in memory: dense, each padded to whole chunks.
     auto rows_of = [&](const mrl::Strided &t) {
       mrl::Strided d = t;
-      d.stride[2] = 1, d.stride[1] = (int64_t(t.shape[2]) + per16 - 1) / per16 * per16, d.stride[0] = int64_t(t.shape[1]) * d.stride[1];
+      // whole cache lines where that adds little: the 128 bytes of K (or of a row of B) that a tile takes
+      // from a row at a time then lie in one line, not two
+      const int64_t unit = t.shape[2] >= 32 * per16 ? 8 * per16 : per16;
+      d.stride[2] = 1, d.stride[1] = (int64_t(t.shape[2]) + unit - 1) / unit * unit, d.stride[0] = int64_t(t.shape[1]) * d.stride[1];
       return d;
     };
     int64_t any_ld, any_bs;
