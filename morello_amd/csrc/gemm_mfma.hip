@@ -152,6 +152,7 @@ hipError_t launch_gemm(const GemmArgs &g, int kind, hipStream_t stream) {
   // Only the 256 tile has a build without the EDGE kernels' limit on leading dimensions.
   const uint32_t side = edge_addressable(g, es) ? tile_side(g, es) : 256;
   if (side == 256) return launch_gemm_big(g, kind, stream);
+  if (const uint32_t bn = gemm_ring_columns(g, kind)) return launch_gemm_ring(g, kind, bn, stream);
   if (g.b_kmajor) return launch_gemm_nt(g, kind, side, stream);
   return launch_gemm_scheduled(g, kind, side, side, 128 / es, stream);
 }

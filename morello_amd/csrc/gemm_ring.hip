@@ -1,0 +1,400 @@
+// Matmul tiles of 128 rows by 64 to 192 columns for problems that do not fill the chip with 256 x 256 ones: operands
+// straight from memory into a ring of LDS slots of 128 bytes of K.
+//
+// What bounds a middling Matmul is less the MFMAs than everything around them: k_gemm's waves spend two
+// thirds of a step issuing what is not an MFMA, in one go, or waiting for a step's trip through registers (bf16
+// 1984 x 5120 x 1536, counters: MFMAs 33 % of the cycles), and tiles of 128 x 128 often come to a little over one per
+// compute unit.  Here:
+//   - operands go straight to LDS, and up to SLOTS steps are on their way at once.  Step k: wait until step
+//     k + 1 has landed, barrier; then, dealt out between step k's MFMAs, the reads of step k + 1's operands and the
+//     requests of step k + SLOTS, into the slot that step k's operands were read from (they are in registers
+//     before the barrier);
+//   - eight waves: four blocks of 64 x BN / 2 outputs, each once for the first and once for the second 64 bytes of
+//     every step, whose sums meet in LDS at the end: two waves on a SIMD, one issuing while the other's MFMAs
+//     run, and an operand read still serves BN / 32 or four MFMAs;
+//   - widths chosen so that the tiles fill one round (gemm_ring_columns).
+// The loads are buffer loads: rows past M or N and chunks past K come as zeros, without a branch.
+//
+// LDS: A as [row][128 bytes], 16-byte chunks XOR-ed with (row / 2) & 7; a k-fastest B likewise; a
+// row-major B as [k][columns], the pieces that transposing reads take (16 columns) XOR-ed so that the
+// rows that one half of a wave reads at once lie in different banks.  Loads fill LDS in order, so
+// the swizzles are applied to the addresses in memory.
+// Semantics: morello/src/spec.rs:480-485; integers exact, bf16 summed in f32.
+#include <algorithm>
+
+#include "gemm_mfma_kernel.h"
+
+namespace mrl {
+namespace {
+using gemm::BF16;
+using gemm::I8;
+using gemm::v2i;
+using gemm::v4i;
+using gemm::v8bf;
+using gemm::TileWalk;
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
+
+constexpr uint32_t OUTSIDE = 0x80000000u;   // an offset no resource here holds
+constexpr int BM = 128, STEP = 128, WAVES = 8;   // bytes of K a step: two MFMAs deep, one for each half of the waves
+
+template <class T> struct Ring;
+template <> struct Ring<I8> {
+  typedef v4i Acc;
+  __device__ static Acc mfma(v4i a, v4i b, Acc c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }
+};
+template <> struct Ring<BF16> {
+  typedef v4f Acc;
+  __device__ static Acc mfma(v4i a, v4i b, Acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+  }
+};
+
+// Byte position of a row-major B's piece-and-rest `byte` of k row r <-> in memory (an involution).  Rows
+// of BN elements; a row's place relative to the 256 bytes of a bank line repeats every 256 / (pitch % 256).
+template <class T, int BN>
+__device__ inline int swizzle(int byte, int r) {
+  constexpr int PITCH = BN * T::ES, PIECE = 16 * T::ES;
+  // the bits of the row number that tell apart the rows half a wave reads at once: bf16 r & 3 and bit 3, int8 r & 7 and bit 4
+  const int rows = T::ES == 2 ? (r & 3) | ((r >> 3) & 1) << 2 : (r & 7) | ((r >> 4) & 1) << 3;
+  constexpr int OFF = PITCH % 256;   // 0: all rows start in the same bank; 128 (64, 192): the low bit (two bits) of the row already moves it
+  constexpr int MOVED = OFF == 0 ? 0 : OFF % 128 == 0 ? 1 : OFF % 64 == 0 ? 2 : 3;
+  constexpr int PIECES = (256 >> MOVED) / PIECE;   // of a group to exchange within
+  const int x = (rows >> MOVED) & (PIECES - 1);
+  return ((byte / PIECE) ^ x) * PIECE + byte % PIECE;
+}
+
+// One load of 64 lanes x 16 bytes into the KiB at LDS address m0 + AT (wave-uniform), lane l to the l-th
+// 16 bytes; the instruction's offset AT is added to the address in memory too, so callers take it off
+// there.  An offset outside the resource brings zeros.  Assembly, so that the compiler does not wait for it.
+template <int AT>
+__device__ inline void dma16(__amdgpu_buffer_rsrc_t from, uint32_t off) {
+  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" : : "v"(off), "s"(from), "n"(AT) : "memory");
+}
+__device__ inline void dma_to(uint32_t lds_addr) { asm volatile("s_mov_b32 m0, %0" : : "s"(lds_addr) : "memory"); }
+__device__ inline __amdgpu_buffer_rsrc_t resource(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, int(bytes), 0x00020000);
+}
+// All but the newest N loads have landed, and every LDS read is done.
+template <int N>
+__device__ inline void wait_for_all_but() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
+}
+
+constexpr int min_of(int a, int b) { return a < b ? a : b; }
+// f(0), ..., f(N - 1) with the number as a type
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void each(F &&f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    each<N, I + 1>(f);
+  }
+}
+
+template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RB, int SLOTS>
+__global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_WALK_PARAMS, GemmArgs g) {
+  typedef typename Ring<T>::Acc Acc;
+  typedef typename T::Out Out;
+  constexpr int ES = T::ES, BK = STEP / ES, RA = 4, BN = 32 * RB, WM = 64, WN = 16 * RB;
+  constexpr int A_BYTES = BM * STEP, B_BYTES = BN * STEP, SLOT = A_BYTES + B_BYTES;
+  constexpr int A_LOADS = A_BYTES / (1024 * WAVES), B_LOADS = (B_BYTES / 1024 + WAVES - 1) / WAVES, LOADS = A_LOADS + B_LOADS;   // a wave's, per step
+  static_assert((SLOTS - 1) * LOADS < 64 && A_LOADS <= 4 && B_LOADS <= 4, "");
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kw = wave >> 2, wm = wave >> 1 & 1, wn = wave & 1;
+  MRL_WALK_TILE(tile_m, tile_n)
+  const int64_t m0 = int64_t(tile_m) * BM, n0 = int64_t(tile_n) * BN;
+  const uint8_t *A = (const uint8_t *)g.a + (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES;
+  const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : n0)) * ES;
+  const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = uint32_t(g.ldb) * ES;
+  // Bytes of the tile's rows (leading dimensions stay below 2^24 bytes); what of a row-major B's lies left of the tile.
+  const int a_end = min(BM, int(g.m - m0)) * int(lda_b), n0_b = int(n0) * ES;
+  const uint32_t b_end = uint32_t(min(BN, int(g.n - n0))) * ldb_b;
+  const int k_bytes = int(g.k) * ES, steps = (k_bytes + STEP - 1) / STEP;
+
+  // Where this lane's chunks of a step come from.  Rows of 64 bytes: sixteen to a load.
+  uint32_t a_off[A_LOADS], b_off[B_LOADS];
+  // Which of B's loads a wave's i-th one is: where they do not divide among the waves, the last few are made twice.
+  auto b_load = [&](int i) { return i * WAVES + wave - (i * WAVES + wave < B_BYTES / 1024 ? 0 : WAVES / 2); };
+  constexpr int CHUNKS = STEP / 16, ROWS_PER_LOAD = 64 / CHUNKS, ROWS_PER_LINE = 256 / STEP;
+  const int row16 = lane / CHUNKS, chunk = (lane % CHUNKS) ^ (row16 / ROWS_PER_LINE % CHUNKS);
+#pragma unroll
+  for (int i = 0; i < A_LOADS; i++) a_off[i] = uint32_t((wave * A_LOADS + i) * ROWS_PER_LOAD + row16) * lda_b + (chunk ^ ((wave * A_LOADS + i) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16;
+#pragma unroll
+  for (int i = 0; i < B_LOADS; i++) {
+    if constexpr (B_KMAJOR) b_off[i] = uint32_t((b_load(i)) * ROWS_PER_LOAD + row16) * ldb_b + (chunk ^ ((b_load(i)) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16;
+    else {
+      constexpr int PITCH = BN * ES;
+      const int at = (b_load(i)) * 1024 + lane * 16, r = at / PITCH;
+      b_off[i] = uint32_t(r) * ldb_b + swizzle<T, BN>(at % PITCH, r);
+    }
+  }
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((lds_void *)lds));
+  // (what the loads' instruction offsets add, taken off 4096 bytes that the resources start earlier)
+#pragma unroll
+  for (int i = 0; i < A_LOADS; i++) a_off[i] += 4096 - i * 1024;
+#pragma unroll
+  for (int i = 0; i < B_LOADS; i++) b_off[i] += 4096;
+  const uint8_t *a_tile = A - 4096, *b_tile = B - 4096;
+  int left = k_bytes;   // of K from the step to request on
+  uint32_t a_dst = lds0 + wave * (A_LOADS * 1024), b_dst = lds0 + A_BYTES;
+  const uint32_t a_dst_end = a_dst + SLOTS * SLOT;
+  __amdgpu_buffer_rsrc_t a_buf, b_buf;
+  const int64_t b_step = B_KMAJOR ? int64_t(STEP) : int64_t(BK) * ldb_b;
+  // The resources of the step to request, and its offsets: chunks past K, in the step that holds K's end,
+  // become ones outside (the steps behind it are empty, so for good).
+  auto prepare = [&]() {
+    const bool some = left > 0;
+    a_buf = resource(a_tile, some ? uint32_t(a_end - (k_bytes - left) + 4096) : 0u);
+    const uint32_t b_bytes = B_KMAJOR ? b_end - uint32_t(k_bytes - left) : uint32_t(min(left / ES, BK)) * ldb_b - n0_b;
+    b_buf = resource(b_tile, some ? b_bytes + 4096 : 0u);
+    if (some && left < STEP) {
+#pragma unroll
+      for (int i = 0; i < A_LOADS; i++)
+        if ((chunk ^ ((wave * A_LOADS + i) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16 >= left) a_off[i] = OUTSIDE;
+      if constexpr (B_KMAJOR)
+#pragma unroll
+        for (int i = 0; i < B_LOADS; i++)
+          if ((chunk ^ ((b_load(i)) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16 >= left) b_off[i] = OUTSIDE;
+    }
+  };
+  // Its i-th load of this wave.
+  auto load = [&](auto which) {
+    constexpr int I = decltype(which)::value;
+    if constexpr (I < A_LOADS) {
+      if constexpr (I == 0) dma_to(a_dst);
+      dma16<I * 1024>(a_buf, a_off[I]);
+    } else {
+      dma_to(b_dst + b_load(I - A_LOADS) * 1024);
+      dma16<0>(b_buf, b_off[I - A_LOADS]);
+    }
+  };
+  auto advance = [&]() {
+    left -= STEP;
+    a_tile += STEP, b_tile += b_step;
+    a_dst += SLOT, b_dst += SLOT;
+    if (a_dst == a_dst_end) a_dst -= SLOTS * SLOT, b_dst -= SLOTS * SLOT;
+  };
+
+  // Operand addresses within a slot: lane (l % 16, l / 16) takes the l / 16-th 16 bytes of row l % 16.
+  const int in_rows = li * STEP + (((4 * kw + lg) ^ (li / ROWS_PER_LINE % CHUNKS)) << 4);
+  int b_rd[RB];
+  if constexpr (!B_KMAJOR) {
+    constexpr int LANES_PER_ROW = 2 * ES;   // of a group of sixteen: 8 bytes each of a row's sixteen columns
+    const int r = (64 / ES) * kw + (16 / ES) * lg + li / LANES_PER_ROW;
+#pragma unroll
+    for (int c = 0; c < RB; c++) b_rd[c] = A_BYTES + r * (BN * ES) + swizzle<T, BN>((wn * WN + c * 16) * ES + 8 * (li % LANES_PER_ROW), r);
+  }
+  v4i af[2][RA], bf[2][RB];
+  int at_slot = 0;
+  const uint8_t *slot = lds;   // the one that operands are read from
+  // The i-th operand read of 64 bytes of K (RA of A, then RB of B).
+  auto read = [&](auto set, auto which) {
+    constexpr int S = decltype(set)::value, I = decltype(which)::value;
+    if constexpr (I < RA) af[S][I] = *(const v4i *)(slot + wm * WM * STEP + in_rows + I * 16 * STEP);
+    else if constexpr (B_KMAJOR) bf[S][I - RA] = *(const v4i *)(slot + A_BYTES + wn * WN * STEP + in_rows + (I - RA) * 16 * STEP);
+    else {
+      const uint8_t *at = slot + b_rd[I - RA];
+      const v2i lo = T::read_tr(at), hi = T::read_tr(at + T::K_PER_READ * (BN * ES));
+      bf[S][I - RA] = v4i{lo[0], lo[1], hi[0], hi[1]};
+    }
+  };
+  Acc acc[RA][RB];
+  int colsum[RB];
+#pragma unroll
+  for (int c = 0; c < RB; c++) {
+    colsum[c] = 0;
+#pragma unroll
+    for (int r = 0; r < RA; r++) acc[r][c] = Acc{0, 0, 0, 0};
+  }
+  auto multiply = [&](auto set, auto which) {   // the which-th block
+    constexpr int S = decltype(set)::value, I = decltype(which)::value, R = I / RB, C = I % RB;
+    if constexpr (A_UNSIGNED && C == 0) af[S][R] ^= v4i{int(0x80808080), int(0x80808080), int(0x80808080), int(0x80808080)};
+    acc[R][C] = Ring<T>::mfma(af[S][R], bf[S][C], acc[R][C]);
+    if constexpr (A_UNSIGNED && R == 0)   // a - 128 was multiplied: 128 times the column sums of B come on top
+#pragma unroll
+      for (int w = 0; w < 4; w++) colsum[C] = __builtin_amdgcn_sdot4(bf[S][C][w], 0x01010101, colsum[C], false);
+  };
+  std::integral_constant<int, 0> even;
+  std::integral_constant<int, 1> odd;
+  // One MFMA after the other with a read or a load, if there are any to issue, behind it: what a wave
+  // issues in one go its MFMAs wait for.
+  auto step = [&](auto multiplied, auto fetched) {
+    wait_for_all_but<(SLOTS - 2) * LOADS>();
+    at_slot = at_slot + 1 == SLOTS ? 0 : at_slot + 1;
+    slot = lds + at_slot * SLOT;
+    each<RA * RB>([&](auto q) {
+      constexpr int Q = decltype(q)::value, N = RA * RB, READS = RA + RB;
+      multiply(multiplied, q);
+      constexpr int R0 = min_of(READS, (Q * READS * 4 + N * 3 - 1) / (N * 3)), R1 = min_of(READS, ((Q + 1) * READS * 4 + N * 3 - 1) / (N * 3));   // in the first three quarters
+      each<R1 - R0>([&](auto i) { read(fetched, std::integral_constant<int, R0 + decltype(i)::value>{}); });   // (behind the last step: zeros)
+      constexpr int L0 = Q * LOADS / N, L1 = (Q + 1) * LOADS / N;
+      each<L1 - L0>([&](auto i) { load(std::integral_constant<int, L0 + decltype(i)::value>{}); });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    advance();
+    prepare();
+  };
+#pragma unroll 1
+  for (int s = 0; s < SLOTS; s++) {
+    prepare();
+    each<LOADS>([&](auto i) { load(i); });
+    advance();
+  }
+  wait_for_all_but<(SLOTS - 1) * LOADS>();
+  each<RA + RB>([&](auto i) { read(even, i); });
+  prepare();
+  for (int k = 0; k + 2 <= steps; k += 2) {
+    step(even, odd);
+    step(odd, even);
+  }
+  if (steps & 1) each<RA * RB>([&](auto q) { multiply(even, q); });
+  wait_for_all_but<0>();   // (requests past the last step write zeros)
+
+  // C.  Register i of a block: row 4 (l / 16) + i, column l % 16.  A wave's block row goes through its own
+  // piece of LDS and leaves in whole rows of WN columns.
+  if (A_UNSIGNED)
+#pragma unroll
+    for (int c = 0; c < RB; c++) {
+      colsum[c] += __shfl_xor(colsum[c], 16);
+      colsum[c] += __shfl_xor(colsum[c], 32);
+      colsum[c] *= 128;
+    }
+  constexpr int ROW = WN + 4, HALVES = RB > 6 ? 2 : 1, ROWS = WM / HALVES;   // (all of it, or half, fits the ring)
+  Out *piece = (Out *)lds + (wave & 3) * (ROWS * ROW);
+  const int64_t row_first = m0 + wm * WM, col_first = n0 + wn * WN;
+  const int cols = int(min(int64_t(WN), int64_t(g.n) - col_first));
+  // (The loops stay loops: code that a launch runs once is fetched from memory, and unrolled it took longer to
+  // fetch than to run.)
+  auto store = [&](auto *C, int half) {
+    typedef std::remove_pointer_t<decltype(C)> Stored;
+    typedef Stored four __attribute__((ext_vector_type(4)));
+    typedef Out out4 __attribute__((ext_vector_type(4)));
+    C += int64_t(blockIdx.y) * g.sc + (row_first + half * ROWS) * g.ldc + col_first;
+    const int rows = int(min(int64_t(ROWS), int64_t(g.m) - row_first - half * ROWS));
+    // four columns at a time where all of a row's are whole and aligned
+    if (cols % 4 == 0 && g.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % (4 * sizeof(Stored)) == 0) {
+#pragma unroll 4
+      for (int e = 0; e < ROWS * WN / 4 / 128; e++) {
+        const int at = (2 * e + kw) * 64 + lane, row = at / (WN / 4), col = at % (WN / 4) * 4;
+        if (row < rows && col < cols) {
+          out4 v = *(const out4 *)(piece + row * ROW + col);
+          four *d = (four *)(C + int64_t(row) * g.ldc + col);
+          if (g.accum) v += __builtin_convertvector(*d, out4);
+          *d = __builtin_convertvector(v, four);
+        }
+      }
+    } else {
+#pragma unroll 4
+      for (int e = 0; e < ROWS * WN / 128; e++) {
+        const int at = (2 * e + kw) * 64 + lane, row = at / WN, col = at % WN;
+        if (row < rows && col < cols) {
+          Out v = piece[row * ROW + col];
+          Stored *d = C + int64_t(row) * g.ldc + col;
+          if (g.accum) v += Out(*d);
+          *d = Stored(v);
+        }
+      }
+    }
+  };
+  // The two halves of K: the upper waves' sums through LDS onto the lower waves', and both store.
+#pragma unroll
+  for (int half = 0; half < HALVES; half++) {
+    auto for_each_of_half = [&](auto f) {
+#pragma unroll
+      for (int r = 0; r < RA / HALVES; r++)
+#pragma unroll
+        for (int c = 0; c < RB; c++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            Out v = acc[half * (RA / HALVES) + r][c][i];
+            if (A_UNSIGNED) v += Out(colsum[c]);
+            f(piece[(r * 16 + 4 * lg + i) * ROW + c * 16 + li], v);
+          }
+    };
+    if (kw) for_each_of_half([](Out &at, Out v) { at = v; });
+    __syncthreads();
+    if (!kw) for_each_of_half([](Out &at, Out v) { at = v + at; });
+    __syncthreads();
+    if (cols > 0 && row_first < int64_t(g.m)) {
+      if constexpr (std::is_same<T, BF16>::value) {
+        if (g.c_bf16) store((__bf16 *)g.c, half);
+        else store((Out *)g.c, half);
+      } else store((Out *)g.c, half);
+    }
+    if (half + 1 < HALVES) __syncthreads();
+  }
+}
+
+template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RB, int SLOTS>
+hipError_t launch_ring(const GemmArgs &g, hipStream_t stream) {
+  constexpr auto kern = k_gemm_ring<T, A_UNSIGNED, B_KMAJOR, RB, SLOTS>;
+  constexpr int BN = 32 * RB, LDS = SLOTS * (BM + BN) * STEP;
+  static_assert(LDS >= 4 * 64 * (16 * RB + 4) * 4, "the waves' pieces of C fit");
+  static std::atomic<uint64_t> lds_limit_set{0};
+  if (!plan::recording() && LDS > 65536) {
+    hipError_t e = raise_lds_limit(lds_limit_set, (const void *)kern, LDS);
+    if (e != hipSuccess) return e;
+  }
+  const int tiles_m = int((g.m + BM - 1) / BM), tiles_n = int((g.n + BN - 1) / BN);
+  const double mn = double(g.m) * g.n * g.batch, steps = double((uint64_t(g.k) * T::ES + STEP - 1) / STEP);
+  plan::work(T::ES == 1 ? plan::UNIT_MFMA_I8 : plan::UNIT_MFMA_BF16, 2.0 * mn * g.k,
+             (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * (g.c_bf16 ? 2 : 4) * (g.accum ? 2 : 1),
+             2.0 * BM * BN * steps * (STEP / T::ES), 2500.0 + 300.0 * steps);
+  const TileWalk walk = gemm::tile_walk(tiles_m, tiles_n);
+  MRL_LAUNCH((k_gemm_ring<T, A_UNSIGNED, B_KMAJOR, RB, SLOTS>), dim3(tiles_m * tiles_n, g.batch), dim3(64 * WAVES), LDS, stream, MRL_WALK_ARGS(walk), g);
+  return plan::last_error();
+}
+
+template <class T, bool A_UNSIGNED, int RB, int SLOTS>
+hipError_t launch_either(const GemmArgs &g, hipStream_t stream) {
+  return g.b_kmajor ? launch_ring<T, A_UNSIGNED, true, RB, SLOTS>(g, stream) : launch_ring<T, A_UNSIGNED, false, RB, SLOTS>(g, stream);
+}
+// As many slots as a compute unit's LDS holds of the wider ones, which run one to a unit (of the 64-wide tile's,
+// five instead of three measured within 4 % either way).
+template <class T, bool A_UNSIGNED>
+hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
+  switch (bn) {
+    case 64: return launch_either<T, A_UNSIGNED, 2, 3>(g, stream);
+    case 128:
+      if constexpr (T::ES == 2) return launch_either<T, A_UNSIGNED, 4, 4>(g, stream);
+      return hipErrorInvalidValue;
+    case 160: return launch_either<T, A_UNSIGNED, 5, 4>(g, stream);
+    case 192: return launch_either<T, A_UNSIGNED, 6, 4>(g, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
+
+// Measured against k_gemm's tiles (us, k_gemm / this), on rounds of one tile per compute unit:
+//   64 where k_gemm's 64 tile would go two to a unit (257 of them on) and this one at most one: bf16 1100 x 3001 x
+//     1100 35.1 / 28.0, 1280 x 1024 x 1600 11.2 / 10.6, u8 1408 x 3001 x 1408 23.6 / 20.9; two to a unit it loses (400 x
+//     3001 x 4400 35.7 / 46.4);
+//   160, else 192, where the 128 tile needs a second round and they do not: bf16 1001 x 2050 x 4425 47.2 / 38.9, 1800 x 2001
+//     x 3000 41.0 / 35.3, u8 1000 x 2001 x 4500 34.6 / 30.1;
+//   128, bf16, within one round: 1984 x 5171 x 1536 55.6 / 50.0, 2048^3 22.9 / 22.2 (u8 2048 x 2001 x 1792 20.0 / 22.1).
+// Short K leaves the start of the ring and the summing of the two halves of K dominant: bf16 1408 x 320 x 1408 5.9 /
+// 6.7, 2048 x 512 x 2560 12.0 / 13.2, 1500 x 512 x 2500 15.9 / 16.5.
+uint32_t gemm_ring_columns(const GemmArgs &g, int kind) {
+  if (kind < 0 || kind > 2) return 0;
+  const uint64_t es = kind == 2 ? 2 : 1, steps = (uint64_t(g.k) * es + STEP - 1) / STEP;
+  if (steps < 16 || g.m <= 128 || g.n <= 128) return 0;
+  auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
+  const uint64_t units = g_compute_units, small = tiles(64, 64);
+  if (small <= 512) return small > units && tiles(BM, 64) <= units ? 64 : 0;
+  const uint64_t whole = tiles(BM, 128);
+  if (whole <= units) return kind == 2 && steps >= 32 && 2 * whole > units ? 128 : 0;
+  return tiles(BM, 160) <= units ? 160 : tiles(BM, 192) <= units ? 192 : 0;
+}
+
+hipError_t launch_gemm_ring(const GemmArgs &g, int kind, uint32_t bn, hipStream_t stream) {
+  switch (kind) {
+    case 0: return launch_kind<I8, false>(g, bn, stream);
+    case 1: return launch_kind<I8, true>(g, bn, stream);
+    case 2: return launch_kind<BF16, false>(g, bn, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace mrl

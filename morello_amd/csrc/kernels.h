@@ -174,6 +174,10 @@ hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint
 // Always the 256 x 256 tile, 128 bytes of K per step.
 // staging: 0 = whichever of the 256 x 256 kernels applies (four waves, eight waves, compiler-scheduled),
 // 1 / 2 / 3 = mrl_staging's REGISTERS / DIRECT_B / DIRECT_B_WIDE only (hipErrorInvalidValue where that one does not apply).
+// gemm_ring.hip: tiles of 128 rows by `bn` (64, 128, 160 or 192) columns, operands straight into a ring of LDS slots; what
+// gemm_possible() takes with edge_addressable() leading dimensions.  gemm_ring_columns: the width for a problem, 0 for none.
+uint32_t gemm_ring_columns(const GemmArgs &g, int kind);
+hipError_t launch_gemm_ring(const GemmArgs &g, int kind, uint32_t bn, hipStream_t stream);
 // gemm_wide_edge.hip: the four-wave tile on ragged shapes and against a k-fastest B.
 hipError_t launch_gemm_wide_edge(const GemmArgs &g, int kind, hipStream_t stream);
 hipError_t launch_gemm_big(const GemmArgs &g, int kind, hipStream_t stream, uint32_t staging = 0);
