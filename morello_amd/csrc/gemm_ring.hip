@@ -71,7 +71,7 @@ template <int AT>
 __device__ inline void dma16(__amdgpu_buffer_rsrc_t from, uint32_t off) {
   asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" : : "v"(off), "s"(from), "n"(AT) : "memory");
 }
-__device__ inline void dma_to(uint32_t lds_addr) { asm volatile("s_mov_b32 m0, %0" : : "s"(lds_addr) : "memory"); }
+__device__ inline void dma_to(uint32_t lds_addr) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(lds_addr) : "memory"); }
 __device__ inline __amdgpu_buffer_rsrc_t resource(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, int(bytes), 0x00020000);
 }
