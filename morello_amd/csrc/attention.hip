@@ -83,6 +83,11 @@ constexpr float STALE_REFERENCE = 1.0e12f;  // ~2^40: an exponential beyond it m
 __device__ inline void dma16(const uint8_t *base, uint32_t voff, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(base));
 }
+// The same through a buffer resource: an offset past its end brings zeros.
+__device__ inline void dma16(__amdgpu_buffer_rsrc_t from, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(from));
+}
+constexpr uint32_t OUTSIDE = 0x80000000u;   // an offset no resource here holds, whatever block's is added
 __device__ inline uint32_t lds_address(const void *p) {
   return uint32_t(reinterpret_cast<uintptr_t>((lds_void *)p));
 }
@@ -104,9 +109,12 @@ __device__ inline v2i read_tr16(const uint8_t *p) {
 // is 2 * QG waves; with 2 groups the four waves share a compute unit's LDS and matrix cores between
 // them alone, which pays when 128-query blocks would leave half of the compute units without work
 // or pad a short query dimension.
-template <int D, bool RAGGED, bool KT_ROWS, int QG>
+// NARROW (with RAGGED): a head dim below D, in whole 16-byte chunks: rows of Q and K are `k_in` elements, rows of V
+// `n_out`, read in place; the chunks past a row's end, and the rows past n2, come as zeros.
+template <int D, bool RAGGED, bool KT_ROWS, int QG, bool NARROW>
 __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, const void *v, float *out, uint32_t b, uint32_t m,
-                                              uint32_t n2, uint32_t n_out, uint32_t key_splits, float *partials) {
+                                              uint32_t n2, uint32_t n_out, uint32_t key_splits, float *partials, uint32_t k_in) {
+  static_assert(!NARROW || (RAGGED && !KT_ROWS), "the narrow form is ragged and wants k fastest");
   // Scalar arguments (the file is built with kernel-argument preloading): the first fourteen
   // dwords arrive in SGPRs with the wave instead of through a load the prologue would wait for.
   struct {
@@ -159,10 +167,13 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
   const int steps = (my_blocks + 1) / 2;
   const int first_block = split_first + (half ? steps : 0);
   const int nblocks = half ? my_blocks - steps : steps;
+  const uint32_t k_row = NARROW ? k_in * 2 : ROW, v_row = NARROW ? n_out * 2 : ROW;   // bytes of a row in memory
   const uint32_t head_bytes = p.n2 * ROW;  // K or V of one batch entry
 
-  const uint8_t *K = (const uint8_t *)p.kt + head * p.n2 * ROW;
-  const uint8_t *V = (const uint8_t *)p.v + head * p.n2 * ROW;
+  const uint8_t *K = (const uint8_t *)p.kt + head * p.n2 * k_row;
+  const uint8_t *V = (const uint8_t *)p.v + head * p.n2 * v_row;
+  const auto k_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(K), 0, int(p.n2 * k_row), 0x00020000);
+  const auto v_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(V), 0, int(p.n2 * v_row), 0x00020000);
   uint8_t *my_lds = lds + half * HALF;
 
   // Q^T operands: block column qb (queries 16 qb + l % 16 of the wave's 32), chunk c of d:
@@ -175,9 +186,12 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
 #pragma unroll
     for (int qb = 0; qb < 2; qb++) {
       const int q_row = RAGGED ? min(q0 + 16 * qb + lr, int(p.m) - 1) : q0 + 16 * qb + lr;
-      const uint8_t *Q = (const uint8_t *)p.q + (head * p.m + q_row) * int64_t(ROW);
+      const uint8_t *Q = (const uint8_t *)p.q + (head * p.m + q_row) * int64_t(k_row);
 #pragma unroll
-      for (int c = 0; c < NC; c++) qf[qb][c] = *(const v4i *)(Q + c * 64 + lgp * 16);
+      for (int c = 0; c < NC; c++) {
+        if (NARROW && uint32_t(c * 64 + lgp * 16) >= k_row) qf[qb][c] = v4i{0, 0, 0, 0};
+        else qf[qb][c] = *(const v4i *)(Q + c * 64 + lgp * 16);
+      }
     }
   }
 
@@ -200,18 +214,25 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
       k_src[i] = row * ROW + ((ld_pc ^ DD::k_swizzle(row)) << 4);
     }
     v_src[i] = row * ROW + ((((ld_pc >> 1) ^ DD::v_swizzle(row)) << 5) | ((ld_pc & 1) << 4));
+    if constexpr (NARROW) {
+      const uint32_t k_at = k_src[i] % ROW, v_at = v_src[i] % ROW;
+      k_src[i] = k_at < k_row ? row * k_row + k_at : OUTSIDE;
+      v_src[i] = v_at < v_row ? row * v_row + v_at : OUTSIDE;
+    }
   }
   // Fetch of this lane's chunk i of K (V) block kb into the KiB at LDS address `dst`.  The block's
   // offset is wave-uniform and goes into the scalar base; only the ragged form, which clamps
   // each lane's address to the entry's last bytes, forms the offset per lane.
   auto fetch_k = [&](int kb, int i, uint32_t dst) {
-    const uint32_t block = uint32_t(first_block + kb) * (KT_ROWS ? BKV * 2 : TILE);
-    if constexpr (RAGGED) dma16(K, min(block + k_src[i], head_bytes - 16), dst);
+    const uint32_t block = uint32_t(first_block + kb) * (KT_ROWS ? BKV * 2 : NARROW ? BKV * k_row : TILE);
+    if constexpr (NARROW) dma16(k_buf, block + k_src[i], dst);
+    else if constexpr (RAGGED) dma16(K, min(block + k_src[i], head_bytes - 16), dst);
     else dma16(K + block, k_src[i], dst);
   };
   auto fetch_v = [&](int kb, int i, uint32_t dst) {
-    const uint32_t block = uint32_t(first_block + kb) * TILE;
-    if constexpr (RAGGED) dma16(V, min(block + v_src[i], head_bytes - 16), dst);
+    const uint32_t block = uint32_t(first_block + kb) * (NARROW ? BKV * v_row : TILE);
+    if constexpr (NARROW) dma16(v_buf, block + v_src[i], dst);
+    else if constexpr (RAGGED) dma16(V, min(block + v_src[i], head_bytes - 16), dst);
     else dma16(V + block, v_src[i], dst);
   };
   // O^T: block row db (d = 16 db + 4 (l / 16) + i in register i), block column qb.
@@ -579,6 +600,8 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
           const int col = db * 16 + 4 * lgp;
           if (whole_rows) {
             *(float4 *)(orow + col) = float4{v[0], v[1], v[2], v[3]};   // ordinary stores: non-temporal ones measured 33.0 against 32.5 us a launch
+          } else if (NARROW) {   // (rows are a multiple of eight floats)
+            if (col < int(p.n_out)) *(float4 *)(orow + col) = float4{v[0], v[1], v[2], v[3]};
           } else {
             if (col + 0 < int(p.n_out)) orow[col + 0] = v[0];
             if (col + 1 < int(p.n_out)) orow[col + 1] = v[1];
@@ -673,19 +696,19 @@ size_t attn_partial_bytes(const AttnArgs &a, uint32_t splits) {
 bool attn_applicable(const AttnArgs &a) {
   auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   return a.k == a.n && (a.k == 32 || a.k == 64 || a.k == 128) && a.n_out >= 1 && a.n_out <= a.n && a.m && a.n2 && a.b &&
-         (!a.kt_rows || a.n2 % 8 == 0) && (a.key_splits <= 1 || (a.partials && a.key_splits <= 65535)) &&
+         (!a.kt_rows || a.n2 % 8 == 0) && (a.k_in == 0 || (!a.kt_rows && a.k > 32 && a.k_in <= a.k && a.k_in % 8 == 0 && a.n_out % 8 == 0)) && (a.key_splits <= 1 || (a.partials && a.key_splits <= 65535)) &&
          uint64_t(a.n2) * a.k * 2 < (1ull << 31) && (a.query_block == 64 || a.query_block == 128) &&
          uint64_t((a.m + a.query_block - 1) / a.query_block) * a.b < (1u << 31) &&
          al16(a.q) && al16(a.kt) && al16(a.v) && al16(a.out);
 }
 
 namespace {
-template <int D, bool RAGGED, bool KT_ROWS, int QG>
+template <int D, bool RAGGED, bool KT_ROWS, int QG, bool NARROW = false>
 hipError_t launch_one(const AttnArgs &a, hipStream_t stream) {
   constexpr int LDS = Dims<D>::LDS_BYTES, BQ = 32 * QG;
   static std::atomic<uint64_t> lds_limit_set{0};
   if (!plan::recording()) {
-    hipError_t e = raise_lds_limit(lds_limit_set, (const void *)k_attn<D, RAGGED, KT_ROWS, QG>, LDS);
+    hipError_t e = raise_lds_limit(lds_limit_set, (const void *)k_attn<D, RAGGED, KT_ROWS, QG, NARROW>, LDS);
     if (e != hipSuccess) return e;
   }
   const dim3 grid(((a.m + BQ - 1) / BQ) * a.b, std::max(1u, a.key_splits));
@@ -698,8 +721,8 @@ hipError_t launch_one(const AttnArgs &a, hipStream_t stream) {
              // eight: 1.2 x that
              (QG == 2 ? 1.2 : 1.0) * 1.17 * 4.0 * BQ * D * (double((a.n2 + BKV - 1) / BKV) * BKV / std::max(1u, a.key_splits)),
              3000.0);
-  MRL_LAUNCH((k_attn<D, RAGGED, KT_ROWS, QG>), grid, dim3(128 * QG), LDS, stream, a.q, a.kt, a.v, a.out, a.b, a.m, a.n2, a.n_out,
-             a.key_splits, a.partials);
+  MRL_LAUNCH((k_attn<D, RAGGED, KT_ROWS, QG, NARROW>), grid, dim3(128 * QG), LDS, stream, a.q, a.kt, a.v, a.out, a.b, a.m, a.n2, a.n_out,
+             a.key_splits, a.partials, a.k_in);
   if (a.key_splits > 1) {
     const uint64_t rows = uint64_t(a.b) * a.m, total = rows * a.n_out;
     plan::work(plan::UNIT_STREAM, 0, double(attn_partial_bytes(a, a.key_splits)) + 4.0 * total);
@@ -711,6 +734,8 @@ hipError_t launch_one(const AttnArgs &a, hipStream_t stream) {
 
 template <int D, int QG>
 hipError_t launch_for(const AttnArgs &a, hipStream_t stream) {
+  if constexpr (D > 32)
+    if (a.k_in) return launch_one<D, true, false, QG, true>(a, stream);
   const bool whole = a.m % (32 * QG) == 0 && a.n2 % (2 * BKV) == 0;
   if (a.kt_rows) return whole ? launch_one<D, false, true, QG>(a, stream) : launch_one<D, true, true, QG>(a, stream);
   return whole ? launch_one<D, false, false, QG>(a, stream) : launch_one<D, true, false, QG>(a, stream);

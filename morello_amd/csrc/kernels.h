@@ -288,6 +288,9 @@ struct AttnArgs {
   // Columns of the result that exist in `out` (its rows are n_out floats): n, or fewer when V
   // was padded with zero columns up to a head dim the kernel is built for.
   uint32_t n_out;
+  // Not 0: q's and kt's rows are this many elements and v's n_out, multiples of eight (k, n > 32 the head dim they
+  // are taken as, zeros behind them).
+  uint32_t k_in = 0;
   bool kt_rows = false;  // KT stored row-major, n2 fastest (n2 a multiple of 8)
   // Queries per workgroup: 128 (eight waves) or 64 (four).
   uint32_t query_block = 128;
