@@ -114,7 +114,13 @@ hipError_t launch_gemm_big(const GemmArgs &g, int kind, hipStream_t stream, uint
   // A k-fastest B and ragged edges on the four-wave tile too, where K is long enough: against the compiler-scheduled
   // 256 tile, bf16 8192^3 with a k-fastest B 751 us (was 845), 1216 x 6016 x 7360 111 (was 131),
   // u8 2176 x 2816 x 3904 k-fastest 32 (was 42).
-  if (staging == 0 && kind <= 2 && (g.b_kmajor || !wide_applicable(g, elem_size_of(kind))) && wide_edge_applicable(g, elem_size_of(kind)))
+  // A bf16 result likewise (8192^3 804 us on the eight-wave tile, 737 here; k-fastest 837, 734), but for whole tiles that leave a
+  // quarter of the compute units idle: those are not short of power, and eight waves are as fast (4096 x 4096 x 2048 76.8,
+  // 77.6 here).
+  const uint64_t tiles = uint64_t((g.m + 255) / 256) * ((g.n + 255) / 256) * g.batch;
+  const bool eight_waves = g.c_bf16 && !g.b_kmajor && whole_tiles(g, 2) && big_applicable(g, 2) && 4 * tiles <= 3 * uint64_t(g_compute_units);
+  if (staging == 0 && kind <= 2 && !eight_waves && (g.b_kmajor || !wide_applicable(g, elem_size_of(kind))) &&
+      wide_edge_applicable(g, elem_size_of(kind)))
     return launch_gemm_wide_edge(g, kind, stream);
   if (g.b_kmajor) return launch_gemm_nt(g, kind, 256, stream);
   const bool whole = whole_tiles(g, elem_size_of(kind));

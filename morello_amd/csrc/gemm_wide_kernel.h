@@ -95,7 +95,6 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   constexpr int B_ROWB = BN * ES;              // bytes per k row of the B tile
   constexpr int ROWS_PER_DMA = 1024 / B_ROWB;  // k rows one direct-to-LDS instruction fills: 4 (i8), 2 (bf16)
   constexpr int GROUP_K = 16 / ES;             // k rows a lane group of an MFMA operand holds: 16 (i8), 8 (bf16)
-  typedef typename T::Out Out;
   static_assert(EDGE || !B_KMAJOR, "a k-fastest B has the ragged form only");
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -121,8 +120,9 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   const uint8_t *A = (const uint8_t *)g.a + (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES;
   const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : n0)) * ES;
 #endif
-  Out *C = (Out *)g.c + int64_t(blockIdx.y) * g.sc + m0 * g.ldc + n0;
-  const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = uint32_t(g.ldb) * ES, ldc_b = uint32_t(g.ldc) * 4;
+  const uint32_t c_es = EDGE && g.c_bf16 ? 2 : 4;   // bytes of an element of C
+  uint8_t *C = (uint8_t *)g.c + (int64_t(blockIdx.y) * g.sc + m0 * g.ldc + n0) * c_es;
+  const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = uint32_t(g.ldb) * ES, ldc_b = uint32_t(g.ldc) * c_es;
   const uint32_t lds0 = uint32_t(uintptr_t(lds));
   // Rows and columns of C from the tile's first on; operand rows past the end repeat the last one.
   const int m_left = EDGE ? min(BM, int(g.m - m0)) : BM, n_left = EDGE ? min(BN, int(g.n - n0)) : BN;
@@ -192,10 +192,10 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
   uint32_t c_lo[4], c_hi[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    c_hi[i] = uint32_t((lane >> 4) * 4 + i) * ldc_b + (lane & 15) * 4;
+    c_hi[i] = uint32_t((lane >> 4) * 4 + i) * ldc_b + (lane & 15) * c_es;
     c_lo[i] = c_hi[i] + (rot ? 512 : 0);
   }
-  const uint8_t *c_base = (const uint8_t *)(C + int64_t(wm * WM) * g.ldc + wn * WN) - (rot ? 256 : 0);
+  const uint8_t *c_base = C + (int64_t(wm * WM) * g.ldc + wn * WN) * c_es - (rot ? 256 : 0);
   const uint32_t ldc16 = 16 * ldc_b;
   // Column-sum partials [lane group][256 columns] of 4 bytes, 1 KiB into LDS once the loop is over:
   // a wave writes those of its block columns 0 .. 3 and reads all eight (rotated like C's).
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
     const uint32_t b_zero = dma_base + lane * 16;
     // C: the resource ends with the last column of the wave's last row; a mask of lanes per block column.
     const int rows = max(0, min(WM, m_left - wm * WM)), n_cols = max(0, min(WN, n_left - wn * WN));
-    const uint32_t c_records = __builtin_amdgcn_readfirstlane(rows && n_cols ? uint32_t(rows - 1) * ldc_b + n_cols * 4 + (rot ? 256 : 0) : 0);
+    const uint32_t c_records = __builtin_amdgcn_readfirstlane(rows && n_cols ? uint32_t(rows - 1) * ldc_b + n_cols * c_es + (rot ? 256 : 0) : 0);
     uint64_t cols[TN];
 #pragma unroll
     for (int t = 0; t < TN; t++) cols[t] = __ballot((t + rot) % TN * 16 + (lane & 15) < n_cols);
@@ -239,11 +239,17 @@ __global__ __launch_bounds__(256) void k_gemm_wide(MRL_WALK_PARAMS, GemmArgs g) 
     else RUN(GEMM_WIDE_##KIND##_ACC);                   \
   } while (0)
     if constexpr (B_KMAJOR) {
-      if constexpr (std::is_same<T, BF16>::value) MRL_WIDE_PICK(MRL_WIDE_RUN_NT_EDGE, NT_EDGE_BF16);
+      if constexpr (std::is_same<T, BF16>::value) {
+        if (g.c_bf16) MRL_WIDE_RUN_NT_EDGE(GEMM_WIDE_NT_EDGE_BF16_OUT16);
+        else MRL_WIDE_PICK(MRL_WIDE_RUN_NT_EDGE, NT_EDGE_BF16);
+      }
       else if constexpr (!A_UNSIGNED) MRL_WIDE_PICK(MRL_WIDE_RUN_NT_EDGE, NT_EDGE_I8);
       else MRL_WIDE_PICK(MRL_WIDE_RUN_NT_EDGE, NT_EDGE_U8);
     } else {
-      if constexpr (std::is_same<T, BF16>::value) MRL_WIDE_PICK(MRL_WIDE_RUN_NN_EDGE, EDGE_BF16);
+      if constexpr (std::is_same<T, BF16>::value) {
+        if (g.c_bf16) MRL_WIDE_RUN_NN_EDGE(GEMM_WIDE_EDGE_BF16_OUT16);
+        else MRL_WIDE_PICK(MRL_WIDE_RUN_NN_EDGE, EDGE_BF16);
+      }
       else if constexpr (!A_UNSIGNED) MRL_WIDE_PICK(MRL_WIDE_RUN_NN_EDGE, EDGE_I8);
       else MRL_WIDE_PICK(MRL_WIDE_RUN_NN_EDGE, EDGE_U8);
     }
@@ -274,11 +280,11 @@ inline bool wide_applicable(const GemmArgs &g, int elem_size) {
 }
 
 // The ragged form: rows of whole 16-byte chunks, a K as long as the whole-tile form asks for (an
-// accumulating Spec's first steps carry C's old values here too).
+// accumulating Spec's first steps carry C's old values here too; a bf16 C is written, not accumulated into).
 inline bool wide_edge_applicable(const GemmArgs &g, int elem_size) {
   const int64_t per16 = 16 / elem_size, bk = 128 / elem_size;
   auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  return !g.c_bf16 && al16(g.a) && al16(g.b) && g.k % per16 == 0 && g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 &&
+  return !(g.c_bf16 && g.accum) && al16(g.a) && al16(g.b) && g.k % per16 == 0 && g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 &&
          g.sb % per16 == 0 && g.k >= WIDE_LONG_K_STEPS * bk && edge_addressable(g, elem_size) &&
          g.ldb * elem_size * (bk + 1) < (int64_t(1) << 31);
 }

@@ -56,6 +56,7 @@ Two more forms of the same tile, each its own text (gen's nt and edge):
     other tiles hold as well (%[skip] k from its start) is zeroed, in A's registers for bf16 (a NaN
     times zero is no zero) and in B's LDS slot; the other tiles then count from the start of K.  Nothing in the
     k loop knows of it.  The loop is left after any step.
+  * out16 (an edge form that does not accumulate): the sums are rounded to bf16 on their way to C.
 
 Register map (all named in the clobber list of the asm statement):
   a[0:255]    accumulators, block (tm, tn) at 4 * (8 * tm + tn); register i of lane l holds row
@@ -196,7 +197,7 @@ class Item:
         self.gap = None
 
 
-def gen(kind, accum, opts=None, gap=0, nt=False, edge=False):
+def gen(kind, accum, opts=None, gap=0, nt=False, edge=False, out16=False):
     """kind: 'u8' (A unsigned bytes), 'i8', 'bf16'.
     accum: the Spec accumulates into C (its old contents are read).
     gap: k steps of the loop run between two steps that load C's old values (0: those steps follow
@@ -771,6 +772,10 @@ def gen(kind, accum, opts=None, gap=0, nt=False, edge=False):
                 E(f"v_accvgpr_read_b32 {t}, a{q}")
                 if unsigned:
                     E(f"v_add_u32 {t}, {t}, v{COL_SUM + tn}")
+                if out16:
+                    E(f"v_cvt_pk_bf16_f32 {t}, {t}, {t}")
+                    E(f"buffer_store_short {t}, {c_addr(tn, i)}, s[84:87], 0 offen offset:{tn * 32}")
+                    continue
                 E(f"buffer_store_dword {t}, {c_addr(tn, i)}, s[84:87], 0 offen offset:{tn * 64}")
                 continue
             out = "global_store_dword"
@@ -830,6 +835,8 @@ def variants():
             yield name + "_ACC", kind, True, 0, nt, True
             for gap in SPACED_GAPS:
                 yield f"{name}_ACC_G{gap}", kind, True, gap, nt, True
+            if kind == "bf16":
+                yield name + "_OUT16", kind, False, 0, nt, True, True
 
 
 def main():

@@ -70,3 +70,19 @@ def test_the_tail_of_k_is_counted_once_whatever_it_holds(gpu, k_fastest):
     row = Bm[:, :, k - 40] if k_fastest else Bm[:, k - 40, :]
     assert np.array_equal(got[:, 7], np.where(synth.bf16_bits_to_f32(row) > 0, np.inf, -np.inf))
     assert np.isfinite(np.delete(got, 7, axis=1)).all()
+
+
+@pytest.mark.parametrize("k_fastest", [False, True])
+@pytest.mark.parametrize("shape,steps,more", [((33, 300, 272), 20, 1), ((33, 257, 401), 21, 7), ((33, 512, 488), 24, 0)])
+def test_a_bf16_result_is_the_f32_sum_rounded(gpu, k_fastest, shape, steps, more):
+    """The same loop forms both; rows of an odd number of two-byte elements, tiles that end inside a block."""
+    b, m, n = shape
+    k = (steps * 128 + more * 16) // 2
+    A, Bm = operands((M.bf16,) * 3, (b, m, k), (b, n, k) if k_fastest else (b, k, (n + 7) // 8 * 8))
+    n = n if k_fastest else Bm.shape[2]
+    results = []
+    for out, zero in ((M.f32, np.float32), (M.bf16, np.uint16)):
+        spec = M.Matmul([b, m, k, n], (M.bf16, M.bf16, out), [None, M.layout(0, 2, 1) if k_fastest else None, None])
+        assert spec.plan().kernels[-1] == "k_gemm_wide" and "EDGE = true" in spec.plan().steps[-1].kernel, spec.plan()
+        results.append(run_spec(spec, [A, Bm, np.full((b, m, n), 7, zero)]))
+    assert np.array_equal(results[1], synth.f32_to_bf16_bits(results[0]))
