@@ -496,13 +496,16 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     // A and B as rows, whichever way B's run; an operand with no rows at all is turned by a Move.
     mrl::PadRows pads[2];
     int n_pads = 0;
-    auto make_rows = [&](Prepared &p, mrl::Strided &t) -> int {
+    auto make_rows = [&](Prepared &p, mrl::Strided &t, uint32_t rows, bool *padded) -> int {
+      *padded = false;
       if (walkable(t)) return MRL_OK;
       mrl::Strided dense = rows_of(t);
+      *padded = as_rows(t, &any_ld, &any_bs);
+      if (*padded) dense.stride[0] = int64_t(rows) * dense.stride[1];
       const size_t bytes = size_t(t.shape[0]) * dense.stride[0] * p.elem;
       HIP_TRY(ws.alloc(&dense.ptr, bytes));
-      if (as_rows(t, &any_ld, &any_bs)) {
-        pads[n_pads++] = {t, dense.ptr, uint32_t(dense.stride[1]), t.shape[1], p.elem};
+      if (*padded) {
+        pads[n_pads++] = {t, dense.ptr, uint32_t(dense.stride[1]), rows, p.elem};
       } else {
         if (dense.stride[1] != int64_t(t.shape[2])) HIP_TRY(mrl::launch_fill_zero(dense.ptr, bytes, ws.stream));
         HIP_TRY(mrl::launch_move_strided(t, dense, ws.stream));
@@ -510,9 +513,15 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
       t = dense;
       return MRL_OK;
     };
-    if ((rc = make_rows(a, a.t)) != MRL_OK) return rc;
+    bool a_padded, b_padded;
+    if ((rc = make_rows(a, a.t, a.t.shape[1], &a_padded)) != MRL_OK) return rc;
     mrl::Strided b_rows = g.b_kmajor ? transposed(b.t) : b.t;
-    if ((rc = make_rows(b, b_rows)) != MRL_OK) return rc;
+    // Where both are copied the copies hold zeros up to the next whole chunk of K (a row-major B in rows of
+    // its own), and K may as well end there: the four-wave 256 tile takes it then (4518 x 3787 x 4543 u8
+    // 138.3 -> 116.0 us, bf16 218.9 -> 187.0).
+    const uint32_t whole_k = uint32_t((g.k + per16 - 1) / per16 * per16);
+    if ((rc = make_rows(b, b_rows, g.b_kmajor ? b_rows.shape[1] : whole_k, &b_padded)) != MRL_OK) return rc;
+    if (a_padded && b_padded) g.k = whole_k;
     b.t = g.b_kmajor ? transposed(b_rows) : b_rows;
     if (n_pads == 2) HIP_TRY(mrl::launch_pad_rows_pair(pads[0], pads[1], ws.stream));
     else if (n_pads == 1) HIP_TRY(mrl::launch_pad_rows(pads[0], ws.stream));

@@ -86,3 +86,22 @@ def test_a_bf16_result_is_the_f32_sum_rounded(gpu, k_fastest, shape, steps, more
         assert spec.plan().kernels[-1] == "k_gemm_wide" and "EDGE = true" in spec.plan().steps[-1].kernel, spec.plan()
         results.append(run_spec(spec, [A, Bm, np.full((b, m, n), 7, zero)]))
     assert np.array_equal(results[1], synth.f32_to_bf16_bits(results[0]))
+
+
+@pytest.mark.parametrize("dts", KINDS)
+@pytest.mark.parametrize("k_fastest", [False, True])
+@pytest.mark.parametrize("shape,k_bytes,accum", [((33, 300, 271), 20 * 128 + 6, False), ((33, 257, 403), 24 * 128 - 2, True)])
+def test_a_k_of_no_whole_chunks_through_padded_copies(gpu, dts, k_fastest, shape, k_bytes, accum):
+    """Copies that hold zeros up to the next chunk of K, rows of them for a row-major B."""
+    b, m, n = shape
+    k = k_bytes // (2 if dts[0] == M.bf16 else 1)
+    A, Bm = operands(dts, (b, m, k), (b, n, k) if k_fastest else (b, k, n))
+    C0 = synth.uniform_i8(97, 2, (b, m, n)).astype(np.float32 if dts[2] == M.f32 else np.int32)
+    spec = M.Matmul([b, m, k, n], dts, [None, M.layout(0, 2, 1) if k_fastest else None, None], accum)
+    assert spec.plan().kernels == ["k_pad_rows_pair", "k_gemm_wide"], spec.plan()
+    got = run_spec(spec, [A, Bm, C0])
+    want = np.matmul(wide(A), wide(Bm).transpose(0, 2, 1) if k_fastest else wide(Bm)) + (C0 if accum else 0)
+    if dts[2] == M.i32:
+        assert np.array_equal(got, want.astype(np.int64).astype(np.int32))
+    else:
+        assert rel_err(got, want) < 1e-5
