@@ -12,6 +12,7 @@
 
 #include "kernels.h"
 #include "layout_factor.h"
+#include "pad_position.h"
 #include "row_chunks.h"
 
 namespace mrl {
@@ -801,8 +802,9 @@ __global__ __launch_bounds__(256) void k_widen_bf16(const uint16_t *__restrict__
 struct PadJob {
   const uint8_t *src;
   chunk_t *dst;
-  uint32_t rows, dst_rows, row_bytes, row_chunks;   // row_chunks: of a destination row
-  uint32_t chunks;                                  // destination chunks in all
+  uint64_t row_bytes;                     // of a source row
+  uint32_t rows, dst_rows, row_chunks;    // row_chunks: of a destination row
+  uint32_t chunks;                        // destination chunks in all
   int64_t src_batch, src_ld;                        // bytes
   FastDiv by_row_chunks, by_dst_rows;
 };
@@ -816,14 +818,14 @@ __device__ inline void pad_chunks(const PadJob &j) {
   for (int u = 0; u < PAD_UNROLL; u++) {
     const uint32_t i = min(first + u * 256, j.chunks - 1);
     const uint32_t line = j.by_row_chunks.div(i), entry = j.by_dst_rows.div(line), row = line - entry * j.dst_rows;
-    const int at = int(i - line * j.row_chunks) * 16;
-    left[u] = row < j.rows ? int(j.row_bytes) - at : 0;
+    const PadChunk c = pad_chunk(i - line * j.row_chunks, row < j.rows ? j.row_bytes : 0);
+    left[u] = c.left;
     // (a chunk with nothing in it reads the row's first instead)
-    const uint8_t *from = j.src + int64_t(entry) * j.src_batch + int64_t(min(row, j.rows - 1)) * j.src_ld + (left[u] > 0 ? at : 0);
+    const uint8_t *from = j.src + int64_t(entry) * j.src_batch + int64_t(min(row, j.rows - 1)) * j.src_ld + c.at;
     shift[u] = uint32_t(uintptr_t(from) & 15);
     from -= shift[u];
     lo[u] = *(const chunk_t *)from;
-    hi[u] = *(const chunk_t *)(from + (int(shift[u]) + min(left[u], 16) > 16 ? 16 : 0));
+    hi[u] = *(const chunk_t *)(from + (int(shift[u]) + left[u] > 16 ? 16 : 0));
   }
 #pragma unroll
   for (int u = 0; u < PAD_UNROLL; u++)
@@ -1631,7 +1633,7 @@ bool pad_job(const PadRows &p, PadJob *j) {
     return false;
   const uint32_t batch = src.shape[0], rows = src.shape[1];
   j->src = static_cast<const uint8_t *>(src.ptr), j->dst = static_cast<chunk_t *>(p.dst);
-  j->rows = rows, j->dst_rows = p.dst_rows, j->row_bytes = src.shape[2] * es, j->row_chunks = uint32_t(uint64_t(p.dst_ld) * es / 16);
+  j->rows = rows, j->dst_rows = p.dst_rows, j->row_bytes = uint64_t(src.shape[2]) * es, j->row_chunks = uint32_t(uint64_t(p.dst_ld) * es / 16);
   const uint64_t chunks = uint64_t(batch) * p.dst_rows * j->row_chunks;
   if (chunks >= (1ull << 31) || chunks == 0) return false;
   j->chunks = uint32_t(chunks);

@@ -29,3 +29,14 @@ def test_common_strided_view_of_two_layouts(tmp_path):
     assert res.returncode == 0, res.stderr
     run = subprocess.run([str(exe)], capture_output=True, text=True)
     assert run.returncode == 0 and "layout view ok" in run.stdout, run.stdout[-2000:] + run.stderr
+
+
+def test_positions_of_padded_copies(tmp_path):
+    """morello_amd/csrc/pad_position.h, the position arithmetic of k_pad_rows: rows on either side of 2^31 and
+    2^32 bytes (an f32 row of 600000001 elements is 2.4 GB)."""
+    exe = tmp_path / "pad_position_check"
+    cmd = ["g++", "-std=c++17", "-O1", "-Wall", "-Werror", os.path.join(ROOT, "tests", "pad_position_check.cpp"), "-o", str(exe)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    run = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert run.returncode == 0 and "pad positions ok" in run.stdout, run.stdout[-2000:] + run.stderr
