@@ -502,6 +502,11 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
       mrl::Strided dense = rows_of(t);
       *padded = as_rows(t, &any_ld, &any_bs);
       if (*padded) dense.stride[0] = int64_t(rows) * dense.stride[1];
+      // (a copy that cannot be: the operand stays as it is, for the generic kernel)
+      if (*padded && !mrl::pad_rows_possible({t, nullptr, uint32_t(dense.stride[1]), rows, p.elem})) {
+        *padded = false;
+        return MRL_OK;
+      }
       const size_t bytes = size_t(t.shape[0]) * dense.stride[0] * p.elem;
       HIP_TRY(ws.alloc(&dense.ptr, bytes));
       if (*padded) {

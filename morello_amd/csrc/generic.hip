@@ -1624,19 +1624,23 @@ hipError_t launch_move_strided(const Strided &src, const Strided &dst, hipStream
   return launch_move_view(src.ptr, src.dtype, dst.ptr, dst.dtype, dims, n, stream);
 }
 
+bool pad_rows_possible(const PadRows &p) {
+  const Strided &src = p.src;
+  if (src.rank != 3 || (src.shape[2] != 1 && src.stride[2] != 1) || uint64_t(p.dst_ld) * p.elem_size % 16 != 0 || p.dst_ld < src.shape[2] ||
+      p.dst_rows < src.shape[1])
+    return false;
+  const double chunks = double(src.shape[0]) * p.dst_rows * (uint64_t(p.dst_ld) * p.elem_size / 16);
+  return chunks >= 1 && chunks < double(1u << 31);
+}
+
 namespace {
 bool pad_job(const PadRows &p, PadJob *j) {
+  if (!pad_rows_possible(p) || (reinterpret_cast<uintptr_t>(p.dst) & 15) != 0) return false;
   const Strided &src = p.src;
-  const uint32_t es = p.elem_size;
-  if (src.rank != 3 || (src.shape[2] != 1 && src.stride[2] != 1) || uint64_t(p.dst_ld) * es % 16 != 0 || p.dst_ld < src.shape[2] ||
-      p.dst_rows < src.shape[1] || (reinterpret_cast<uintptr_t>(p.dst) & 15) != 0)
-    return false;
-  const uint32_t batch = src.shape[0], rows = src.shape[1];
+  const uint32_t es = p.elem_size, batch = src.shape[0], rows = src.shape[1];
   j->src = static_cast<const uint8_t *>(src.ptr), j->dst = static_cast<chunk_t *>(p.dst);
   j->rows = rows, j->dst_rows = p.dst_rows, j->row_bytes = uint64_t(src.shape[2]) * es, j->row_chunks = uint32_t(uint64_t(p.dst_ld) * es / 16);
-  const uint64_t chunks = uint64_t(batch) * p.dst_rows * j->row_chunks;
-  if (chunks >= (1ull << 31) || chunks == 0) return false;
-  j->chunks = uint32_t(chunks);
+  j->chunks = batch * p.dst_rows * j->row_chunks;
   j->src_batch = (batch == 1 ? 0 : src.stride[0]) * int64_t(es), j->src_ld = (rows == 1 ? 0 : src.stride[1]) * int64_t(es);
   j->by_row_chunks = FastDiv(j->row_chunks), j->by_dst_rows = FastDiv(j->dst_rows);
   return true;

@@ -90,6 +90,7 @@ struct PadRows {
   void *dst;
   uint32_t dst_ld, dst_rows, elem_size;
 };
+bool pad_rows_possible(const PadRows &p);   // (`dst` not looked at) fewer than 2^31 chunks, which the kernel numbers in 32 bits
 hipError_t launch_pad_rows(const PadRows &p, hipStream_t stream);
 // Two such copies in one launch.
 hipError_t launch_pad_rows_pair(const PadRows &p0, const PadRows &p1, hipStream_t stream);
