@@ -25,7 +25,7 @@ bool applicable(const GemmArgs &g, int es) {
   // read along with it, and are zeros wherever the caller padded the row.
   return g.m >= 1 && g.n >= 1 && g.k >= 1 &&
          g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 && g.sb % per16 == 0 &&
-         al16(g.a) && al16(g.b) && (reinterpret_cast<uintptr_t>(g.c) & 3) == 0 &&
+         al16(g.a) && al16(g.b) && reinterpret_cast<uintptr_t>(g.c) % (g.c_bf16 ? 2 : 4) == 0 &&   // stores of C are an element each
          g.batch <= 65535 && uint64_t((g.m + BM - 1) / BM) * ((g.n + BN - 1) / BN) < (1u << 30);
 }
 

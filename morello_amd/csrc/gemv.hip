@@ -183,7 +183,7 @@ bool gemv_applicable(const GemmArgs &g, int kind) {
   if (g.m > few && b_bytes > (g.m <= 2 * few ? (8ull << 20) : (4ull << 20))) return false;
   return g.b_kmajor && g.m >= 1 && g.m <= uint32_t(MRL_GEMV_MAX_M) && g.n >= 64 && int64_t(g.k) * es >= 1024 &&
          g.k % per16 == 0 && g.lda % per16 == 0 && g.ldb % per16 == 0 && g.sa % per16 == 0 && g.sb % per16 == 0 &&
-         al16(g.a) && al16(g.b) && (reinterpret_cast<uintptr_t>(g.c) & 3) == 0 && g.batch <= 65535 &&
+         al16(g.a) && al16(g.b) && reinterpret_cast<uintptr_t>(g.c) % (g.c_bf16 ? 2 : 4) == 0 && g.batch <= 65535 &&
          uint64_t(g.n) < (1ull << 31);
 }
 

@@ -40,3 +40,15 @@ def test_positions_of_padded_copies(tmp_path):
     assert res.returncode == 0, res.stderr
     run = subprocess.run([str(exe)], capture_output=True, text=True)
     assert run.returncode == 0 and "pad positions ok" in run.stdout, run.stdout[-2000:] + run.stderr
+
+
+def test_outputs_the_matrix_cores_take(tmp_path):
+    """C on any element of its own type: bf16 on two bytes, 32-bit results on four."""
+    exe = tmp_path / "dispatch_check"
+    lib_dir = os.path.join(ROOT, "morello_amd")
+    cmd = ["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-isystem", "/opt/rocm/include", os.path.join(ROOT, "tests", "dispatch_check.cpp"),
+           "-o", str(exe), "-L", lib_dir, "-lmorello_amd", f"-Wl,-rpath,{lib_dir}", "-Wl,-rpath,/opt/rocm/lib"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    run = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert run.returncode == 0 and "dispatch ok" in run.stdout, run.stdout[-2000:] + run.stderr

@@ -36,3 +36,27 @@ def test_bf16_result_is_the_f32_result_rounded(gpu, shape, accum, k_fastest):
     else:
         # another kernel's order of summing (at most 2^-15 of a sum of this size) may tip a tie: a step of bf16
         assert np.abs(got.view(np.int16).astype(np.int32) - want.view(np.int16).astype(np.int32)).max() <= 1
+
+
+@pytest.mark.parametrize("shape,k_fastest", [
+    ((1, 300, 520, 413), False), ((1, 1100, 264, 1300), True), ((1, 2900, 2600, 2100), False),  # 64, 128 and ragged 256 tile
+    ((1, 2560, 256, 2560), False), ((1, 2560, 2560, 2560), True),                               # whole 256 tiles
+    ((1, 1001, 2050, 4425), False), ((1, 130, 8256, 70), False), ((1, 1, 2048, 12000), True),   # ring, K in slices, dot products
+])
+@pytest.mark.parametrize("accum", [False, True])
+def test_bf16_result_on_any_element(gpu, shape, k_fastest, accum):
+    """An output that starts on an odd element goes through the same kernels as an aligned one: the same bits
+    (the generic kernel's order of summing gives others)."""
+    b, m, k, n = shape
+    A, Bm = synth.normal_bf16(80, 0, (b, m, k)), synth.normal_bf16(80, 1, (b, n, k) if k_fastest else (b, k, n))
+    old = synth.normal_bf16(80, 2, (b, m, n), 8.0)
+    spec = M.Matmul(list(shape), (M.bf16, M.bf16, M.bf16), [None, M.layout(0, 2, 1) if k_fastest else None, None], accum)
+    want = run_spec(spec, [A, Bm, old])
+    guarded = np.full(old.size + 2, 0x4242, np.uint16)
+    guarded[1:-1] = old.ravel()
+    bufs = [M.DeviceBuffer.from_numpy(x) for x in (A, Bm, guarded)]
+    spec.run_device([bufs[0].ptr, bufs[1].ptr, bufs[2].ptr + 2])
+    got = bufs[2].to_numpy(np.uint16, guarded.shape)
+    for x in bufs:
+        x.free()
+    assert np.array_equal(got[1:-1].reshape(old.shape), want) and got[0] == got[-1] == 0x4242
