@@ -247,9 +247,11 @@ int mrl_run_noalloc(const mrl_spec *spec, void *const *params, void *stream);
 /* Literal stand-in for calling the emitted kernel from the emitted main
  * (codegen/cpu.rs:284-409): `params` are HOST pointers; inputs (and the output, when it
  * is read) are copied to the device, the Spec is run, written parameters are copied back.
- * Device and pinned memory for it stay with the library between calls (at most two sets of up to 1 GiB
- * on the device and 32 MiB pinned; calls from several threads use a set each);
- * mrl_stream_release(NULL) gives them back. */
+ * Device and pinned memory for it stay with the library between calls: at most two sets, each of up to 1 GiB
+ * on the device for the parameters, 32 MiB pinned, and the scratch that its Specs took (64 MiB as for any stream
+ * that needs scratch, more, up to 16 GiB, after Specs that asked for more); calls from several threads use a
+ * set each.  Idle sets are given back when an allocation of this library finds too little device
+ * memory, and by mrl_stream_release(NULL). */
 int mrl_run_host(const mrl_spec *spec, void *const *params);
 
 /* Per-kind conveniences that build the descriptor themselves.  NULL layouts mean

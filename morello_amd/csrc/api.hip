@@ -306,7 +306,7 @@ struct Workspace {
       arena->in_use.lock();
     }
     requested += rounded;
-    if (!arena->base && rounded <= ARENA_BYTES && hipMalloc(&arena->base, ARENA_BYTES) == hipSuccess)
+    if (!arena->base && rounded <= ARENA_BYTES && mrl::device_malloc(&arena->base, ARENA_BYTES) == hipSuccess)
       arena->size = ARENA_BYTES;
     if (arena->base && rounded <= arena->size - arena_used) {
       *p = static_cast<uint8_t *>(arena->base) + arena_used;
@@ -314,6 +314,10 @@ struct Workspace {
       return hipSuccess;
     }
     hipError_t e = hipMallocAsync(p, rounded, stream);
+    if (e == hipErrorOutOfMemory && mrl::HostStage::drop_idle()) {
+      (void)hipGetLastError();   // (the first try's)
+      e = hipMallocAsync(p, rounded, stream);
+    }
     if (e == hipSuccess) allocs.push_back(*p);
     return e;
   }
@@ -328,7 +332,7 @@ struct Workspace {
       if (hipStreamSynchronize(stream) == hipSuccess) {
         if (arena->base) (void)hipFree(arena->base);
         arena->base = nullptr, arena->size = 0;
-        if (hipMalloc(&arena->base, grown) == hipSuccess) arena->size = grown;
+        if (mrl::device_malloc(&arena->base, grown) == hipSuccess) arena->size = grown;
         else arena->base = nullptr;
       }
     }
@@ -2535,7 +2539,7 @@ int mrl_device_malloc(void **ptr, size_t bytes) {
   if (!ptr) return MRL_ERR_NULL;
   int rc;
   if (g_device < 0 && (rc = mrl_init(0)) != MRL_OK) return rc;
-  HIP_TRY(hipMalloc(ptr, bytes ? bytes : 4));
+  HIP_TRY(mrl::device_malloc(ptr, bytes ? bytes : 4));
   return MRL_OK;
 }
 int mrl_device_free(void *ptr) {

@@ -26,8 +26,9 @@ class HostStage {
   // Idle stages stay for later calls (at most IDLE_MAX of them, each with at most KEEP_DEVICE_BYTES)
   // once their work is complete; a stage whose call failed (`good` false) does not.
   static void release(HostStage *stage, bool good);
-  // Frees the idle stages.
-  static void drop_idle();
+  // Frees the idle stages and the scratch kept for their streams; whether there were any.
+  static bool drop_idle();
+  static constexpr int IDLE_MAX = 2;
 
   struct Piece {      // a parameter: `bytes` at `offset` (a multiple of 256) of the device memory
     void *host;
@@ -43,7 +44,6 @@ class HostStage {
   hipStream_t stream() const { return stream_; }
 
  private:
-  static constexpr int IDLE_MAX = 2;
   static constexpr size_t KEEP_DEVICE_BYTES = size_t(1) << 30, PINNED_BYTES = size_t(32) << 20;
   static constexpr size_t PART_MAX = size_t(2) << 20;   // what one copy kernel takes at most: 37 us of PCIe against a launch's ~2
   static constexpr int SLOTS = int(PINNED_BYTES / PART_MAX);
@@ -63,6 +63,10 @@ class HostStage {
   uint32_t *counters_ = nullptr;  // device: workgroups of a copy that are done, per slot
   uint32_t ticket_ = 0;
 };
+
+// hipMalloc for all of the library's device memory: where there is not enough, what idle stages keep is given back
+// and tried for once more.
+hipError_t device_malloc(void **p, size_t bytes);
 
 // What to call with a stage's stream before it is destroyed (the scratch arena kept for it).
 void on_host_stage_stream_end(void (*f)(hipStream_t));

@@ -11,8 +11,8 @@
 #include <cstring>
 #include <functional>
 #include <mutex>
+#include <new>
 #include <thread>
-#include <vector>
 
 namespace mrl {
 namespace {
@@ -100,7 +100,8 @@ Helpers &helpers() {
 }
 
 std::mutex g_idle_mutex;
-std::vector<HostStage *> g_idle;
+HostStage *g_idle[HostStage::IDLE_MAX];   // the first g_n_idle
+int g_n_idle = 0;
 void (*g_stream_end)(hipStream_t) = nullptr;
 
 size_t round_up(size_t n, size_t to) { return (n + to - 1) / to * to; }
@@ -109,6 +110,15 @@ size_t round_up(size_t n, size_t to) { return (n + to - 1) / to * to; }
 
 void on_host_stage_stream_end(void (*f)(hipStream_t)) { g_stream_end = f; }
 
+hipError_t device_malloc(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && HostStage::drop_idle()) {
+    (void)hipGetLastError();   // (the first try's)
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 hipError_t HostStage::init() {
   hipError_t e = hipGetDevice(&device_id_);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking);
@@ -116,7 +126,7 @@ hipError_t HostStage::init() {
   if (e == hipSuccess) e = hipEventCreateWithFlags(&join_, hipEventDisableTiming);
   if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&pin_), PINNED_BYTES, hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&flags_), SLOTS * 64, hipHostMallocDefault);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&counters_), SLOTS * 64);
+  if (e == hipSuccess) e = device_malloc(reinterpret_cast<void **>(&counters_), SLOTS * 64);
   if (e != hipSuccess) return e;
   std::memset(flags_, 0, SLOTS * 64);
   return hipMemset(counters_, 0, SLOTS * 64);
@@ -143,11 +153,15 @@ HostStage *HostStage::acquire(size_t bytes, hipError_t *err) {
   HostStage *stage = nullptr;
   {
     std::lock_guard<std::mutex> lock(g_idle_mutex);
-    for (size_t i = 0; i < g_idle.size() && !stage; i++)
-      if (g_idle[i]->device_id_ == device) stage = g_idle[i], g_idle.erase(g_idle.begin() + i);
+    for (int i = 0; i < g_n_idle && !stage; i++)
+      if (g_idle[i]->device_id_ == device) stage = g_idle[i], g_idle[i] = g_idle[--g_n_idle];
   }
   if (!stage) {
-    stage = new HostStage;
+    stage = new (std::nothrow) HostStage;
+    if (!stage) {
+      *err = hipErrorOutOfMemory;
+      return nullptr;
+    }
     if ((*err = stage->init()) != hipSuccess) {
       delete stage;
       return nullptr;
@@ -157,7 +171,14 @@ HostStage *HostStage::acquire(size_t bytes, hipError_t *err) {
     if (stage->dev_) (void)hipFree(stage->dev_);
     stage->dev_ = nullptr, stage->dev_size_ = 0;
     const size_t want = round_up(bytes, size_t(2) << 20);
-    if ((*err = hipMalloc(reinterpret_cast<void **>(&stage->dev_), want)) != hipSuccess) {
+    *err = device_malloc(reinterpret_cast<void **>(&stage->dev_), want);
+    if (*err == hipErrorOutOfMemory && g_stream_end) {   // the scratch that earlier calls left on this stage's own stream
+      (void)hipGetLastError();
+      g_stream_end(stage->stream_);
+      *err = hipMalloc(reinterpret_cast<void **>(&stage->dev_), want);
+    }
+    if (*err != hipSuccess) {
+      stage->dev_ = nullptr;
       delete stage;
       return nullptr;
     }
@@ -178,27 +199,31 @@ void HostStage::release(HostStage *stage, bool good) {
   }
   {
     std::lock_guard<std::mutex> lock(g_idle_mutex);
-    if (g_idle.size() < size_t(IDLE_MAX)) {
-      g_idle.push_back(stage);
+    if (g_n_idle < IDLE_MAX) {
+      g_idle[g_n_idle++] = stage;
       return;
     }
   }
   delete stage;
 }
 
-void HostStage::drop_idle() {
-  std::vector<HostStage *> gone;
-  {
-    std::lock_guard<std::mutex> lock(g_idle_mutex);
-    gone.swap(g_idle);
-  }
+bool HostStage::drop_idle() {
   int device = 0;
   const bool known = hipGetDevice(&device) == hipSuccess;
-  for (HostStage *s : gone) {
+  bool any = false;
+  for (;;) {
+    HostStage *s = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(g_idle_mutex);
+      if (g_n_idle > 0) s = g_idle[--g_n_idle];
+    }
+    if (!s) break;
     (void)hipSetDevice(s->device_id_);
     delete s;
+    any = true;
   }
-  if (known) (void)hipSetDevice(device);
+  if (known && any) (void)hipSetDevice(device);
+  return any;
 }
 
 hipError_t HostStage::copy(void *dst, const void *src, size_t bytes, uint32_t slot, uint32_t ticket, hipStream_t stream) {
