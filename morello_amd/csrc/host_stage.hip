@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void pcie_copy(const v4u *__restrict__ src, v4
 
 // Helper threads for memcpy, started at the first large transfer and then asleep between transfers
 // for the life of the process.  One job at a time; others who want the helpers meanwhile do their
-// copies alone.
+// copies alone, as does a process that may have no more threads (it is asked again at the next transfer).
 class Helpers {
  public:
   static constexpr int COUNT = 3;
@@ -58,11 +58,11 @@ class Helpers {
     std::lock_guard<std::mutex> one_job(busy_, std::adopt_lock);
     {
       std::lock_guard<std::mutex> lock(m_);
-      if (!started_) {
-        for (int i = 0; i < COUNT; i++) std::thread([this] { work(); }).detach();
-        started_ = true;
+      try {
+        for (; started_ < COUNT; started_++) std::thread([this] { work(); }).detach();
+      } catch (const std::exception &) {   // (this is called from C)
       }
-      f_ = &f, n_ = n, next_ = 0, inside_ = COUNT, job_++;
+      f_ = &f, n_ = n, next_ = 0, inside_ = started_, job_++;
     }
     wake_.notify_all();
     for (int i; (i = next_.fetch_add(1)) < n;) f(i);
@@ -88,7 +88,7 @@ class Helpers {
   }
   std::mutex busy_, m_;
   std::condition_variable wake_, idle_;
-  bool started_ = false;
+  int started_ = 0;
   const std::function<void(int)> *f_ = nullptr;
   int n_ = 0, inside_ = 0;
   uint64_t job_ = 0;
@@ -286,7 +286,7 @@ struct HostStage::Parts {
   // megabyte's copy).
   template <class F>
   void for_each(F &&f) const {
-    if (total >= (size_t(2) << 20)) helpers().run(count, f);
+    if (total >= (size_t(2) << 20)) helpers().run(count, std::ref(f));   // (a reference: nothing to allocate)
     else for (int i = 0; i < count; i++) f(i);
   }
   // From four parts on every second one takes the stage's other stream: a copy then starts while the

@@ -96,8 +96,12 @@ static void drop_arena(hipStream_t s) {
 int main() {
   hipError_t e;
   mrl::on_host_stage_stream_end(drop_arena);
+  // No helper threads to be had, then some.
+  g_no_threads = true;
   HostStage *a = HostStage::acquire(9 * MB, &e);
   expect(a, "a stage");
+  round_trip(a, 9 * MB);
+  g_no_threads = false;
   round_trip(a, 9 * MB);
   round_trip(a, 3 * MB + 5);
   HostStage::release(a, true);
