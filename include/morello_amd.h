@@ -247,6 +247,7 @@ int mrl_run_noalloc(const mrl_spec *spec, void *const *params, void *stream);
 /* Literal stand-in for calling the emitted kernel from the emitted main
  * (codegen/cpu.rs:284-409): `params` are HOST pointers; inputs (and the output, when it
  * is read) are copied to the device, the Spec is run, written parameters are copied back.
+ * What the null stream and the streams that synchronise with it hold when the call is made comes first.
  * Device and pinned memory for it stay with the library between calls: at most two sets, each of up to 1 GiB
  * on the device for the parameters, 32 MiB pinned, and the scratch that its Specs took (64 MiB as for any stream
  * that needs scratch, more, up to 16 GiB, after Specs that asked for more); calls from several threads use a

@@ -1,12 +1,14 @@
 """Specs called on host buffers (mrl_run_host) through the pinned stage that stays between calls:
 transfers of one part and of many (more parts than the stage has slots), parameters that are read,
 read and written, and only written, stages shared out among threads, and given back."""
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
 
 import morello_amd as M
+import morello_amd._binding as B
 import orc
 from morello_amd import synth
 
@@ -67,3 +69,33 @@ def test_threads_use_a_stage_each_and_stages_are_given_back(gpu):
         M.release_stream()
         free.append(M.device_free_bytes())
     assert free[-1] >= free[1] and not bad
+
+
+@pytest.mark.parametrize("on_stream", [False, True])
+def test_host_buffers_that_earlier_work_still_fills(gpu, on_stream):
+    """The call comes behind what the null stream, and a stream that synchronises with it, hold: an input in
+    pinned memory that a Move writes behind some milliseconds of Matmul."""
+    n = 1 << 20
+    hip, pin = B.load(), C.c_void_p()
+    hip.hipHostMalloc.argtypes, hip.hipHostFree.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint], [C.c_void_p]
+    assert hip.hipHostMalloc(C.byref(pin), 4 * n, 0) == 0
+    x, out = np.ctypeslib.as_array(C.cast(pin, C.POINTER(C.c_float)), (n,)), np.zeros(n, np.float32)
+    long_one, move = M.Matmul([1, 8192, 8192, 8192], (M.f32, M.f32, M.f32)), M.Move([n], (M.f32, M.f32))
+    bufs = [M.DeviceBuffer(4 << 26) for _ in range(3)]
+    stream = M.Stream() if on_stream else None
+    enqueue = (lambda spec, ptrs: spec.run_async(ptrs, stream)) if on_stream else (lambda spec, ptrs: spec.run_noalloc(ptrs))
+    for value in (3.0, 4.0):
+        src = M.DeviceBuffer.from_numpy(np.full(n, value, np.float32))
+        x[:] = -1.0
+        M.synchronize()
+        enqueue(long_one, [b.ptr for b in bufs])
+        enqueue(move, [src.ptr, pin.value])
+        move.run_host(x, out)
+        assert (out == value).all()
+        M.synchronize()
+        src.free()
+    for b in bufs:
+        b.free()
+    if stream:
+        stream.destroy()
+    hip.hipHostFree(pin)
