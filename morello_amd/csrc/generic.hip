@@ -262,21 +262,26 @@ struct MoveStrided {
   uint32_t dim_s, dim_d;      // the dim each side stores contiguously
   uint32_t tiles_s, tiles_d;  // 64-element tiles along them
   uint64_t count;
-  FastDiv by_shape[MOVE_MAX_RANK];   // by shape[order[o]], for k_move_rows (a tensor has fewer than 2^31 elements)
+  FastDiv by_shape[MOVE_MAX_RANK];   // by shape[order[o]], for place_of (a tensor has fewer than 2^31 elements)
 };
+
+// Where the i-th element (or vector) in destination order lies on the two sides.
+__device__ inline void place_of(const MoveStrided &p, uint32_t i, int64_t &so, int64_t &d_o) {
+  so = d_o = 0;
+  for (int o = int(p.rank) - 1; o >= 0; o--) {
+    const uint32_t d = p.order[o], rest = p.by_shape[o].div(i), c = i - rest * p.shape[d];
+    i = rest;
+    so += int64_t(c) * p.ss[d], d_o += int64_t(c) * p.ds[d];
+  }
+}
 
 // Both sides contiguous along the same dim: consecutive threads take consecutive elements of
 // that dim, so reads and writes are both coalesced.
 __global__ __launch_bounds__(256) void k_move_rows(MoveStrided p) {
   const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= p.count) return;
-  uint32_t rem = uint32_t(i);  // a tensor has fewer than 2^31 elements
-  int64_t so = 0, d_o = 0;
-  for (int o = int(p.rank) - 1; o >= 0; o--) {
-    const uint32_t d = p.order[o], rest = p.by_shape[o].div(rem), c = rem - rest * p.shape[d];
-    rem = rest;
-    so += int64_t(c) * p.ss[d], d_o += int64_t(c) * p.ds[d];
-  }
+  int64_t so, d_o;
+  place_of(p, uint32_t(i), so, d_o);  // (a tensor has fewer than 2^31 elements)
   store_u32(p.dst, p.ddt, d_o, move_bits(p.src, p.sdt, so, p.ddt));
 }
 
@@ -702,6 +707,22 @@ __global__ __launch_bounds__(256) void k_move_runs(MoveTile p) {
   for (int u = 0; u < UNROLL; u++)
     if (inside[u]) store_run<DE, V>(p.dst, (base_d + to[u]) * V, raw[u]);
 }
+// Without tiles, a vector a thread in destination order: a tile's arithmetic, a dozen digits of its origin ahead
+// of the first load, is 1 to 3 us of a launch (launch_move_view says where they are earned back).
+template <int SE, int DE, int V>
+__global__ __launch_bounds__(256) void k_move_runs(MoveStrided p) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.count) return;
+  int64_t so, d_o;
+  place_of(p, i, so, d_o);
+  uint32_t raw[V];
+  load_run<SE, V>(p.src, so * V, raw);
+  with_dtypes<SE, DE>(p.sdt, p.ddt, [&](auto sd, auto dd) {
+#pragma unroll
+    for (int e = 0; e < V; e++) raw[e] = convert_raw(raw[e], decltype(sd)::value, decltype(dd)::value);
+  });
+  store_run<DE, V>(p.dst, d_o * V, raw);
+}
 
 // Any other pair of contiguous digits (an OddEven digit on one side, a Packed digit of rows: too
 // short for the 64 x 64 transpose): a tile of up to 4096 elements, chosen on the host so that it
@@ -767,6 +788,17 @@ __global__ __launch_bounds__(256) void k_move_gather(MoveTile p) {
     for (int e = 0; e < VD; e++) v[e] = lds[cell(at + (VD == 1 ? 0 : p.lds_step[e]))];
     if (inside) store_run<DE, VD>(p.dst, base_d + d_o, v);
   }
+}
+// Without a tile, an element a thread in destination order: small tensors, as above.
+template <int SE, int DE>
+__global__ __launch_bounds__(256) void k_move_gather(MoveStrided p) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.count) return;
+  int64_t so, d_o;
+  place_of(p, i, so, d_o);
+  uint32_t raw = load_sized<SE>(p.src, so);
+  with_dtypes<SE, DE>(p.sdt, p.ddt, [&](auto sd, auto dd) { raw = convert_raw(raw, decltype(sd)::value, decltype(dd)::value); });
+  store_sized<DE>(p.dst, d_o, raw);
 }
 
 // Four 16-byte vectors per thread in flight, streamed past the caches: 6.5 TB/s on a 256 MiB
@@ -1250,6 +1282,14 @@ namespace {
 // of workgroups whatever the layouts, where the tiled kernels' loops over a handful of tiles take
 // three times as long.
 constexpr uint64_t MOVE_TINY = 65536;
+// Up to this many an element or a vector a thread in destination order, no tiles: scattered reads come out of
+// the caches, and a tile's arithmetic is what is left.  Over 1200 random layouts of up to five dims (geometric means, tiles /
+// without): 64 to 128 thousand elements 4.8 / 3.2 us, 512 thousand to 1 Mi 6.4 / 4.8 (vectors 4.9 / 4.5), 2 to 4 Mi 9.7 / 12.6
+// (6.5 / 10.8); [45, 1963, 4] to [45, 4, 1963] f32 5.8 / 4.3, bf16 5.0 / 3.3.  Between 1 and 2 Mi it is either, by layout.
+constexpr uint64_t MOVE_SMALL = 1u << 20;
+// Whole 16-byte vectors in runs of 64 bytes or more, nothing converted: either side then reads and writes half a cache
+// line at least in any order, and tiles pay later (4 to 8 MB 5.8 / 3.8 us, 8 to 16 MB 5.4 / 4.5, 32 to 64 MB 15.4 / 17.7).
+constexpr uint64_t MOVE_DIRECT_BYTES = 16u << 20;
 
 // A MoveTile's per-digit arrays from a view and the tile's extents.  `first`: digits in the order a
 // vector's number counts them (k_move_runs), nullptr for any order with the extended digits first.
@@ -1277,22 +1317,17 @@ void fill_tile(MoveTile *t, const MoveStrided &p, const uint32_t *ext, const uin
   }
 }
 
-// k_move_runs: `shared` is the digit both sides store contiguously, in vectors of `vec` elements.
-hipError_t launch_move_runs(MoveStrided p, uint32_t shared, uint32_t vec, hipStream_t stream) {
-  const uint32_t se = uint32_t(mrl_dtype_size(p.sdt)), de = uint32_t(mrl_dtype_size(p.ddt)), rank = p.rank;
-  for (uint32_t d = 0; d < rank; d++) {
-    if (d == shared) p.shape[d] /= vec;
-    else p.ss[d] /= vec, p.ds[d] /= vec;
-  }
-  p.count /= vec;
+// k_move_runs' tile over a view whose shared digit counts vectors of `vec` elements: how many vectors it
+// holds, and how many tiles there are.
+uint32_t runs_tile(const MoveStrided &p, uint32_t shared, uint32_t vec, uint32_t se, MoveTile *t, uint64_t *blocks) {
+  const uint32_t rank = p.rank;
   // Four vectors a thread once every compute unit gets two such workgroups.
   const uint32_t tile_cap = p.count >= 1024ull * 2 * g_compute_units ? 1024 : 256;
   uint32_t ext[MOVE_MAX_RANK], first[MOVE_RUNS_ACT], n_first = 0, tile = 1;
   for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) ext[d] = 1;
   auto take = [&](uint32_t d, uint32_t most) {
     const uint32_t e = std::min({p.shape[d], most, tile_cap / tile});
-    bool known = false;
-    for (uint32_t i = 0; i < n_first; i++) known = known || first[i] == d;
+    const bool known = std::find(first, first + n_first, d) != first + n_first;
     if (e <= 1 || known || n_first == MOVE_RUNS_ACT) return;
     first[n_first++] = d, ext[d] = e, tile *= e;
   };
@@ -1315,17 +1350,33 @@ hipError_t launch_move_runs(MoveStrided p, uint32_t shared, uint32_t vec, hipStr
     take(uint32_t(next_d), p.shape[next_d]);
   }
   for (int o = int(rank) - 1; o >= 0; o--) take(p.order[o], p.shape[p.order[o]]);
+  uint32_t n_act = n_first;
+  fill_tile(t, p, ext, nullptr, nullptr, first, &n_act, blocks);
+  t->tile = tile;
+  for (uint32_t e = 0; e < 4; e++) t->lds_step[e] = 0;
+  return tile;
+}
+
+// k_move_runs: `shared` is the digit both sides store contiguously, in vectors of `vec` elements.
+hipError_t launch_move_runs(MoveStrided p, uint32_t shared, uint32_t vec, bool tiled, hipStream_t stream) {
+  const uint32_t se = uint32_t(mrl_dtype_size(p.sdt)), de = uint32_t(mrl_dtype_size(p.ddt));
+  for (uint32_t d = 0; d < p.rank; d++) {
+    if (d == shared) p.shape[d] /= vec;
+    else p.ss[d] /= vec, p.ds[d] /= vec;
+  }
+  p.count /= vec;
   MoveTile t;
   uint64_t blocks = 0;
-  uint32_t n_act = n_first;
-  fill_tile(&t, p, ext, nullptr, nullptr, first, &n_act, &blocks);
-  t.tile = tile;
-  for (uint32_t e = 0; e < 4; e++) t.lds_step[e] = 0;
-  if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
+  const uint32_t tile = tiled ? runs_tile(p, shared, vec, se, &t, &blocks) : 0;
+  if (!tiled) {
+    blocks = (p.count + 255) / 256;
+    for (uint32_t o = 0; o < p.rank; o++) p.by_shape[o] = FastDiv(p.shape[p.order[o]]);
+  }
   const dim3 grid{uint32_t(blocks)};
 #define MRL_RUNS_V(SE, DE, V)                                                                                       \
   if (vec == V) {                                                                                                  \
-    if (tile > 256) MRL_LAUNCH((k_move_runs<SE, DE, V, 4>), grid, dim3(256), 0, stream, t);                         \
+    if (!tiled) MRL_LAUNCH((k_move_runs<SE, DE, V>), grid, dim3(256), 0, stream, p);                            \
+    else if (tile > 256) MRL_LAUNCH((k_move_runs<SE, DE, V, 4>), grid, dim3(256), 0, stream, t);                    \
     else MRL_LAUNCH((k_move_runs<SE, DE, V, 1>), grid, dim3(256), 0, stream, t);                                    \
   }
 #define MRL_RUNS(SE, DE)                                                                                            \
@@ -1439,7 +1490,11 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
       for (uint32_t d = 0; fits && d < rank; d++) fits = int(d) == dim_s || (p.ss[d] % v == 0 && p.ds[d] % v == 0);
       if (fits) vec = v;
     }
-  if (vec) return launch_move_runs(p, uint32_t(dim_s), vec, stream);
+  const bool small = p.count <= MOVE_SMALL;
+  if (vec) {
+    const bool long_runs = vec == 16 / widest && se == de && uint64_t(p.shape[dim_s]) * se >= 64 && p.count * se <= MOVE_DIRECT_BYTES;
+    return launch_move_runs(p, uint32_t(dim_s), vec, !small && !long_runs, stream);
+  }
   // Runs of at least 64 bytes that are not whole vectors (odd rows), a tensor of one round of
   // workgroups either way, or one with no contiguous digit: an element per thread.
   const bool shared_runs = shared && (rank == 1 || uint64_t(p.shape[dim_s]) * se >= 64);
@@ -1497,6 +1552,16 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
     else if (mrl_dtype_size(src_dtype) == 1) MRL_LAUNCH(k_move_tiled_as<uint8_t>, dim3(uint32_t(blocks)), dim3(256), 0, stream, p);
     else if (mrl_dtype_size(src_dtype) == 2) MRL_LAUNCH(k_move_tiled_as<uint16_t>, dim3(uint32_t(blocks)), dim3(256), 0, stream, p);
     else MRL_LAUNCH(k_move_tiled_as<uint32_t>, dim3(uint32_t(blocks)), dim3(256), 0, stream, p);
+    return mrl::plan::last_error();
+  }
+  if (small) {
+    const dim3 grid{uint32_t((p.count + 255) / 256)};
+    for (uint32_t o = 0; o < rank; o++) p.by_shape[o] = FastDiv(p.shape[p.order[o]]);
+#define MRL_GATHER(SE, DE) if (se == SE && de == DE) MRL_LAUNCH((k_move_gather<SE, DE>), grid, dim3(256), 0, stream, p);
+    MRL_GATHER(1, 1) MRL_GATHER(1, 2) MRL_GATHER(1, 4)
+    MRL_GATHER(2, 1) MRL_GATHER(2, 2) MRL_GATHER(2, 4)
+    MRL_GATHER(4, 1) MRL_GATHER(4, 2) MRL_GATHER(4, 4)
+#undef MRL_GATHER
     return mrl::plan::last_error();
   }
   // Otherwise a tile grown digit by digit: along the destination's fastest digits until they

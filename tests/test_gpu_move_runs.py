@@ -86,3 +86,25 @@ def test_long_shared_digit_is_cut(gpu):
 def test_gathered_runs_of_four(gpu, sdt, ddt, rows, cols, dst):
     """Even and odd elements apart, strips of rows over odd widths: runs of four on one side, both or none."""
     _check(sdt, ddt, [1, rows, cols], None, dst, "k_move_gather")
+
+
+@pytest.mark.parametrize("sdt,ddt", [(M.f32, M.bf16), (M.f32, M.f32), (M.bf16, M.f32), (M.u8, M.f32), (M.u8, M.bf16),
+                                     (M.bf16, M.u8), (M.i32, M.u8)])
+@pytest.mark.parametrize("rows,cols", [(1030, 16 * 65), (1027, 16 * 129), (2049, 16 * 130)])
+def test_packing_strips_in_tiles(gpu, sdt, ddt, rows, cols):
+    """Past the 2^20 elements up to which a vector goes to a thread: tiles of one and of four vectors a thread,
+    ragged on both sides."""
+    _check(sdt, ddt, [1, rows, cols], None, STRIPS, "k_move_runs")
+    _check(ddt, sdt, [1, rows, cols], STRIPS, None, "k_move_runs")
+
+
+def test_long_runs_without_tiles(gpu):
+    """Whole vectors in runs of 64 bytes and more, up to 16 MB; and beyond, in tiles."""
+    _check(M.f32, M.f32, [7340, 12, 16], None, (1, 0, 2), "k_move_runs")
+    _check(M.u8, M.u8, [30, 14, 5, 8, 260], (0, 2, 1, 3, 4), (1, 2, 0, 3, 4), "k_move_runs")
+    _check(M.f32, M.f32, [29360, 12, 16], None, (1, 0, 2), "k_move_runs")
+
+
+@pytest.mark.parametrize("shift", [(1, 0), (0, 1), (2, 2), (4, 4), (8, 4)])
+def test_tiles_off_a_vector(gpu, shift):
+    _check(M.f32, M.bf16, [1, 1050, 1040], None, STRIPS, "k_move_runs", shift)

@@ -1,5 +1,7 @@
 """Which kernels a Spec goes to where two routes meet, by its plan (no GPU): Specs that one of them cannot
 take, or takes at many times the other's cost."""
+import math
+
 import pytest
 
 import morello_amd as M
@@ -12,3 +14,23 @@ def test_operands_too_many_for_padded_copies_stay_as_they_are(batch, k):
     """2^27 right operands of up to 16 rows of a chunk each are 2^31 chunks, more than the copy numbers."""
     p = M.Matmul([batch, 1, k, 1], (M.u8, M.i8, M.i32)).plan()
     assert p.kernels[-1] == "k_matmul_generic"
+
+
+@pytest.mark.parametrize("shape,dst,kernel,vec", [
+    ([45, 1963, 4], (0, 2, 1), "k_move_gather", 1), ([1, 1024, 1024], (0, 1, 2, (1, 16)), "k_move_gather", 1),
+    ([300, 200, 16], (1, 0, 2), "k_move_runs", 4), ([2, 64, 2050], (1, 0, 2), "k_move_runs", 2),
+    ([7340, 12, 16], (1, 0, 2), "k_move_runs", 4), ([8, 6, 5, 6212], (1, 2, 0, 3), "k_move_runs", 4),   # 5.6 MB in runs of 64 bytes and more
+])
+def test_small_moves_take_no_tiles(shape, dst, kernel, vec):
+    """An element (or vector) a thread up to 2^20 elements, and up to 16 MB in long runs: the tiles' arithmetic made
+    these 1.5 to 2 times as long."""
+    layout = M.layout(*[(d[0], M.Packed(d[1])) if isinstance(d, tuple) else d for d in dst])
+    p = M.Move(shape, (M.f32, M.f32), layouts=[None, layout]).plan()
+    threads = math.prod(shape) // vec
+    assert p.kernels == [kernel] and p.steps[0].grid == ((threads + 255) // 256, 1, 1)
+
+
+def test_large_moves_take_tiles():
+    for shape, dst in (([45, 19630, 4], (0, 2, 1)), ([1, 2048, 16384], (0, 2, 1, (2, M.Packed(16))))):
+        p = M.Move(shape, (M.f32, M.bf16), layouts=[None, M.layout(*dst)]).plan()
+        assert p.steps[0].grid[0] <= math.prod(shape) // 2048
