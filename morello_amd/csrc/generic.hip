@@ -1318,43 +1318,54 @@ void fill_tile(MoveTile *t, const MoveStrided &p, const uint32_t *ext, const uin
 }
 
 // k_move_runs' tile over a view whose shared digit counts vectors of `vec` elements: how many vectors it
-// holds, and how many tiles there are.
+// holds, and how many tiles there are.  0 where it would have more workgroups than a launch takes.
 uint32_t runs_tile(const MoveStrided &p, uint32_t shared, uint32_t vec, uint32_t se, MoveTile *t, uint64_t *blocks) {
   const uint32_t rank = p.rank;
   // Four vectors a thread once every compute unit gets two such workgroups.
   const uint32_t tile_cap = p.count >= 1024ull * 2 * g_compute_units ? 1024 : 256;
   uint32_t ext[MOVE_MAX_RANK], first[MOVE_RUNS_ACT], n_first = 0, tile = 1;
   for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) ext[d] = 1;
+  auto known = [&](uint32_t d) { return std::find(first, first + n_first, d) != first + n_first; };
   auto take = [&](uint32_t d, uint32_t most) {
     const uint32_t e = std::min({p.shape[d], most, tile_cap / tile});
-    const bool known = std::find(first, first + n_first, d) != first + n_first;
-    if (e <= 1 || known || n_first == MOVE_RUNS_ACT) return;
+    if (e <= 1 || known(d) || n_first == MOVE_RUNS_ACT) return;
     first[n_first++] = d, ext[d] = e, tile *= e;
   };
   // (a shared digit longer than 256 vectors is cut into even pieces)
   take(shared, p.shape[shared] <= 256 ? 256u : (p.shape[shared] + (p.shape[shared] + 255) / 256 - 1) / ((p.shape[shared] + 255) / 256));
-  auto fastest = [&](const int64_t *stride) {   // the digit that continues the runs of one side
+  auto next = [&](const int64_t *stride, int behind) {   // the digit that continues the runs of one side
     int best = -1;
     for (uint32_t d = 0; d < rank; d++)
-      if (d != shared && p.shape[d] > 1 && (best < 0 || stride[d] < stride[best])) best = int(d);
+      if (d != shared && int(d) != behind && p.shape[d] > 1 && (behind < 0 || stride[d] >= stride[behind]) &&
+          (best < 0 || stride[d] < stride[best]))
+        best = int(d);
     return best;
   };
-  const int next_d = fastest(p.ds), next_s = fastest(p.ss);
+  const int next_d = next(p.ds, -1), next_s = next(p.ss, -1);
   if (next_d >= 0 && next_s >= 0 && next_s != next_d) {
-    // 512 bytes of the source side, the rest of the tile along the destination's
-    const uint32_t want_s = std::max(1u, 512u / (ext[shared] * vec * se));
-    const uint32_t keep = std::min({want_s, p.shape[next_s], std::max(1u, tile_cap / tile)});
-    take(uint32_t(next_d), std::max(1u, tile_cap / tile / keep));
+    // 512 bytes of the source side, along two digits if need be, the rest of the tile along the destination's
+    const uint32_t want_s = std::min(std::max(1u, 512u / (ext[shared] * vec * se)), std::max(1u, tile_cap / tile));
+    const int further = p.shape[next_s] < want_s ? next(p.ss, next_s) : -1;
+    const bool two = further >= 0 && further != next_d;
+    const uint32_t s1 = std::min(want_s, p.shape[next_s]), s2 = two ? std::min(want_s / s1, p.shape[further]) : 1;
+    take(uint32_t(next_d), std::max(1u, tile_cap / tile / (s1 * s2)));
     take(uint32_t(next_s), p.shape[next_s]);
+    if (two) take(uint32_t(further), p.shape[further]);
   } else if (next_d >= 0) {
     take(uint32_t(next_d), p.shape[next_d]);
   }
-  for (int o = int(rank) - 1; o >= 0; o--) take(p.order[o], p.shape[p.order[o]]);
+  // What is left of the tile: along the destination's further digits, or, when they come to the tile's last
+  // digit, along the longest.
+  for (int o = int(rank) - 1; o >= 0 && n_first + 1 < uint32_t(MOVE_RUNS_ACT); o--) take(p.order[o], p.shape[p.order[o]]);
+  int longest = -1;
+  for (uint32_t d = 0; d < rank; d++)
+    if (!known(d) && (longest < 0 || p.shape[d] > p.shape[longest])) longest = int(d);
+  if (longest >= 0) take(uint32_t(longest), p.shape[longest]);
   uint32_t n_act = n_first;
   fill_tile(t, p, ext, nullptr, nullptr, first, &n_act, blocks);
   t->tile = tile;
   for (uint32_t e = 0; e < 4; e++) t->lds_step[e] = 0;
-  return tile;
+  return *blocks < (1u << 24) ? tile : 0;
 }
 
 // k_move_runs: `shared` is the digit both sides store contiguously, in vectors of `vec` elements.
@@ -1367,15 +1378,16 @@ hipError_t launch_move_runs(MoveStrided p, uint32_t shared, uint32_t vec, bool t
   p.count /= vec;
   MoveTile t;
   uint64_t blocks = 0;
+  // (a tile that leaves threads of its workgroup without a vector: four short digits, the rest of the tensor elsewhere)
   const uint32_t tile = tiled ? runs_tile(p, shared, vec, se, &t, &blocks) : 0;
-  if (!tiled) {
+  if (tile < 192) {
     blocks = (p.count + 255) / 256;
     for (uint32_t o = 0; o < p.rank; o++) p.by_shape[o] = FastDiv(p.shape[p.order[o]]);
   }
   const dim3 grid{uint32_t(blocks)};
 #define MRL_RUNS_V(SE, DE, V)                                                                                       \
   if (vec == V) {                                                                                                  \
-    if (!tiled) MRL_LAUNCH((k_move_runs<SE, DE, V>), grid, dim3(256), 0, stream, p);                            \
+    if (tile < 192) MRL_LAUNCH((k_move_runs<SE, DE, V>), grid, dim3(256), 0, stream, p);                            \
     else if (tile > 256) MRL_LAUNCH((k_move_runs<SE, DE, V, 4>), grid, dim3(256), 0, stream, t);                    \
     else MRL_LAUNCH((k_move_runs<SE, DE, V, 1>), grid, dim3(256), 0, stream, t);                                    \
   }

@@ -108,3 +108,13 @@ def test_long_runs_without_tiles(gpu):
 @pytest.mark.parametrize("shift", [(1, 0), (0, 1), (2, 2), (4, 4), (8, 4)])
 def test_tiles_off_a_vector(gpu, shift):
     _check(M.f32, M.bf16, [1, 1050, 1040], None, STRIPS, "k_move_runs", shift)
+
+
+@pytest.mark.parametrize("sdt,ddt", [(M.f32, M.f32), (M.f32, M.bf16), (M.bf16, M.bf16), (M.u8, M.f32)])
+def test_five_digits_short_and_long(gpu, sdt, ddt):
+    """More digits than a tile has: four of them short (no tile), and two on the source side before its runs are
+    long."""
+    _check(sdt, ddt, [20011, 2, 2, 2, 8], None, (0, 3, 2, 1, 4), "k_move_runs")
+    _check(sdt, ddt, [20011, 3, 2, 2, 16], None, (3, 0, 2, 1, 4), "k_move_runs")
+    _check(sdt, ddt, [107, 4, 696, 4, 4], None, (4, 3, 2, 1, 0, (4, "p", 2)), "k_move_runs" if max(np.dtype(NP[sdt]).itemsize, np.dtype(NP[ddt]).itemsize) == 4 else "k_move_gather")
+    _check(sdt, ddt, [2, 58566, 4, 3, 8], (0, 3, 1, 2, 4), (1, 0, 2, 3, 4), "k_move_runs")
