@@ -727,10 +727,12 @@ __global__ __launch_bounds__(256) void k_move_runs(MoveStrided p) {
 // Any other pair of contiguous digits (an OddEven digit on one side, a Packed digit of rows: too
 // short for the 64 x 64 transpose): a tile of up to 4096 elements, chosen on the host so that it
 // holds long runs on both sides, is read in source order, converted in registers, and written
-// in destination order out of LDS.  VS, VD: elements per access on the two sides, 4 where the
+// in destination order out of LDS.  VS, VD: elements per access on the two sides, 4 or 2 where the
 // element's neighbours in the tile are its neighbours in memory, else 1.  The loads of a batch of
 // four accesses are in flight together, and their digits are worked out once per access, not per
-// element: that arithmetic is what bounds the kernel.
+// element: that arithmetic is what bounds the kernel.  Runs of two: bf16 18 x 123556 transposed 8.0 us, element by element on
+// that side 11.7; f32 [16, 2, 5, 84558] to [0, 3, 2, 1] 23.3, 37.2.  NACT: digits that the tile extends along at most; f32
+// [1189, 5, 2, 4, 82] to [3, 4, 0, 2, 1, 3oe2], five of them, takes 26.1 us (16.4 with the runs of two) and 69.6 as any number.
 template <int SE, int DE, int VS, int VD, int NACT>
 __global__ __launch_bounds__(256) void k_move_gather(MoveTile p) {
   __shared__ uint32_t lds[MOVE_TILE_MAX + MOVE_TILE_MAX / 32];
@@ -1621,21 +1623,21 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
       tstride_d[by_ds[i]] = run_d, run_d *= ext[by_ds[i]];
     }
   }
-  // Whether the tile's elements, taken in one side's order, lie there in whole runs of four: the
-  // fastest digits continue each other (1, ext, ...) up to a multiple of four, inside the tensor as
-  // well as inside the tile, and everything else is a multiple of four apart.  in_run: how many
-  // of the fastest digits make up the four; on the destination side, whose runs are gathered from
-  // LDS at fixed distances, no run of four may carry into a further digit.
-  auto fours = [&](const uint32_t *order, const int64_t *stride, const void *base, size_t size, bool gathered, uint32_t *in_run) {
-    if ((reinterpret_cast<uintptr_t>(base) % (4 * size)) != 0) return false;
+  // Whether the tile's elements, taken in one side's order, lie there in whole runs of v (4 or 2): the
+  // fastest digits continue each other (1, ext, ...) up to a multiple of v, inside the tensor as
+  // well as inside the tile, and everything else is a multiple of v apart.  in_run: how many
+  // of the fastest digits make up the run; on the destination side, whose runs are gathered from
+  // LDS at fixed distances, no run may carry into a further digit.
+  auto runs_of = [&](uint32_t v, const uint32_t *order, const int64_t *stride, const void *base, size_t size, bool gathered, uint32_t *in_run) {
+    if ((reinterpret_cast<uintptr_t>(base) % (v * size)) != 0) return false;
     int64_t run = 1;
     for (uint32_t i = 0; i < rank; i++) {
       const uint32_t d = order[i];
-      if (stride[d] != run || (gathered && 4 % run != 0)) return false;
-      const bool whole = (run * ext[d]) % 4 == 0 && (run * p.shape[d]) % 4 == 0;
+      if (stride[d] != run || (gathered && v % run != 0)) return false;
+      const bool whole = (run * ext[d]) % v == 0 && (run * p.shape[d]) % v == 0;
       if (whole) {
         for (uint32_t j = i + 1; j < rank; j++)
-          if (stride[order[j]] % 4 != 0) return false;
+          if (stride[order[j]] % v != 0) return false;
         *in_run = i + 1;
         return true;
       }
@@ -1644,14 +1646,17 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
     }
     return false;
   };
-  uint32_t digits_s = 0, digits_d = 0;
-  const bool fours_s = fours(by_ss, p.ss, src, se, false, &digits_s), fours_d = fours(by_ds, p.ds, dst, de, true, &digits_d);
+  uint32_t digits_s = 0, digits_d = 0, run_s = 1, run_d = 1;
+  for (uint32_t v : {4u, 2u}) {   // (two bytes are no wider than one)
+    if (run_s == 1 && v * se >= 4 && runs_of(v, by_ss, p.ss, src, se, false, &digits_s)) run_s = v;
+    if (run_d == 1 && v * de >= 4 && runs_of(v, by_ds, p.ds, dst, de, true, &digits_d)) run_d = v;
+  }
   MoveTile t;
   for (uint32_t e = 0; e < 4; e++) {
     uint32_t rem = e;
     t.lds_step[e] = 0;
-    for (uint32_t i = 0; fours_d && i < digits_d; i++) {
-      const uint32_t d = by_ds[i], size = i + 1 == digits_d ? 4 : ext[d];
+    for (uint32_t i = 0; run_d > 1 && i < digits_d; i++) {
+      const uint32_t d = by_ds[i], size = i + 1 == digits_d ? run_d : ext[d];
       t.lds_step[e] += rem % size * tstride_s[d], rem /= size;
     }
   }
@@ -1664,19 +1669,26 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
 #define MRL_GATHER_V(SE, DE, VS, VD)                                                                                 \
   do {                                                                                                               \
     if (n_act <= 4) MRL_LAUNCH((k_move_gather<SE, DE, VS, VD, 4>), grid, dim3(256), 0, stream, t);                   \
+    else if (n_act <= 5) MRL_LAUNCH((k_move_gather<SE, DE, VS, VD, 5>), grid, dim3(256), 0, stream, t);              \
     else MRL_LAUNCH((k_move_gather<SE, DE, VS, VD, int(MOVE_MAX_RANK)>), grid, dim3(256), 0, stream, t);             \
+  } while (0)
+#define MRL_GATHER_S(SE, DE, VS)                            \
+  do {                                                      \
+    if (run_d == 4) MRL_GATHER_V(SE, DE, VS, 4);            \
+    else if (run_d == 2) MRL_GATHER_V(SE, DE, VS, (DE > 1 ? 2 : 1)); \
+    else MRL_GATHER_V(SE, DE, VS, 1);                       \
   } while (0)
 #define MRL_GATHER(SE, DE)                                  \
   if (se == SE && de == DE) {                               \
-    if (fours_s && fours_d) MRL_GATHER_V(SE, DE, 4, 4);     \
-    else if (fours_s) MRL_GATHER_V(SE, DE, 4, 1);           \
-    else if (fours_d) MRL_GATHER_V(SE, DE, 1, 4);           \
-    else MRL_GATHER_V(SE, DE, 1, 1);                        \
+    if (run_s == 4) MRL_GATHER_S(SE, DE, 4);                \
+    else if (run_s == 2) MRL_GATHER_S(SE, DE, (SE > 1 ? 2 : 1)); \
+    else MRL_GATHER_S(SE, DE, 1);                           \
   }
   MRL_GATHER(1, 1) MRL_GATHER(1, 2) MRL_GATHER(1, 4)
   MRL_GATHER(2, 1) MRL_GATHER(2, 2) MRL_GATHER(2, 4)
   MRL_GATHER(4, 1) MRL_GATHER(4, 2) MRL_GATHER(4, 4)
 #undef MRL_GATHER
+#undef MRL_GATHER_S
 #undef MRL_GATHER_V
   return mrl::plan::last_error();
 }

@@ -118,3 +118,20 @@ def test_five_digits_short_and_long(gpu, sdt, ddt):
     _check(sdt, ddt, [20011, 3, 2, 2, 16], None, (3, 0, 2, 1, 4), "k_move_runs")
     _check(sdt, ddt, [107, 4, 696, 4, 4], None, (4, 3, 2, 1, 0, (4, "p", 2)), "k_move_runs" if max(np.dtype(NP[sdt]).itemsize, np.dtype(NP[ddt]).itemsize) == 4 else "k_move_gather")
     _check(sdt, ddt, [2, 58566, 4, 3, 8], (0, 3, 1, 2, 4), (1, 0, 2, 3, 4), "k_move_runs")
+
+
+@pytest.mark.parametrize("sdt,ddt", [(M.u8, M.f32), (M.bf16, M.f32), (M.u8, M.u8), (M.f32, M.bf16), (M.bf16, M.bf16), (M.f32, M.f32)])
+@pytest.mark.parametrize("shape,src,dst", [
+    ([18, 60002], None, (1, 0)), ([18, 60004], None, (1, 0)), ([20, 60002], None, (1, 0)), ([17, 62003], None, (1, 0)),   # 2 and 2, 4 and 2, 2 and 4, none
+    ([1189, 5, 2, 4, 26], None, (3, 4, 0, 2, 1, (3, "oe", 2))),   # five digits
+    ([6, 7001, 5, 6], (2, 1, 3, 0), (0, 2, 3, 1)), ([3, 6, 30002, 2], (2, 3, 0, 1), (0, 1, 3, 2)),
+])
+def test_gathered_runs_of_four_and_of_two(gpu, sdt, ddt, shape, src, dst):
+    """Past the 2^20 elements up to which an element goes to a thread: every pair of run lengths."""
+    _check(sdt, ddt, shape, src, dst, "k_move_gather")
+
+
+@pytest.mark.parametrize("shift", [(1, 0), (0, 1), (2, 2), (2, 1)])
+def test_gathered_runs_off_an_element(gpu, shift):
+    _check(M.f32, M.f32, [20, 60004], None, (1, 0), "k_move_gather", shift)
+    _check(M.bf16, M.bf16, [20, 60004], None, (1, 0), "k_move_gather", shift)
