@@ -369,8 +369,19 @@ bool gemm_skinny_applicable(const GemmArgs &g, int kind) {
   const double macs = double(g.m) * g.n * g.k * g.batch;
   const bool chunks = k_bytes % 16 == 0 && g.lda * es % 16 == 0 && g.ldb * es % 16 == 0;
   if (g.b_kmajor) {
-    // Few columns and a long K: the tiled kernel with K shared out over workgroups.
-    if (g.m > 64 || ((uint64_t(g.n) + 15) / 16 * g.batch < 64 && macs > 8e6)) return false;
+    const uint64_t cols = (uint64_t(g.n) + 15) / 16 * g.batch;
+    // Few columns and a long K: the tiled kernel with K shared out over workgroups, or, for a row or a few of f32, the dot
+    // products.  One workgroup's eight waves take 0.26 us per KB of K (f32 0.4, more rows more), the others 6 to 20 us
+    // with their copies and the sum (us, this / the others: bf16 1 x 64000 x 14 36.4 / 17.4, 44 x 9600 x 16 15.5 / 7.9, 10 x
+    // 24416 x 16 15.6 / 20.8; f32 4 x 9792 x 64 16.9 / 7.0).
+    if (g.m > 64 || (cols < 64 && macs > 8e6)) return false;
+    if (g.batch == 1 && cols < 64 && macs >= 1e5 && k_bytes > (g.m > 16 ? 16384 : 40960)) return false;
+    if (kind == 3 && g.batch == 1 && cols < 32 && g.n >= 64 && g.m <= 4 && chunks && k_bytes >= 8192) return false;
+    // A short K keeps one to four of the eight waves: past two thousand blocks, which fill the chip several times over, the
+    // tiled kernel (us, this / that: f32 12 x (53 x 76 x 1533) 18.7 / 7.0, bf16 59 x 64 x 13690 6.3 / 3.0, u8 62 x (3 x 64 x 4096)
+    // 22.6 / 10.7; a thousand blocks or 512 bytes are even).
+    if (cols * ((g.m + 15) / 16) > 2048 && k_bytes < 512) return false;
+    if (kind == 3 && g.m > 32 && k_bytes < 256) return false;   // (f32 42 x 22 x 192 4.2 / 2.8)
     // One or two rows against a large B: the dot products (bf16 1 x 2048 x 16384 12.2 us, this 13.3; but
     // 1 x 4096 x 4096 9.5, 8.3).  More than 32 rows of whole chunks: past 8 MB of B the tiled kernel, which reads
     // A less often (bf16 64 x 2048 x 8192 11.5 us, this 12.0; 44 x 1280 x 1265 7.8, 4.9).
@@ -382,6 +393,11 @@ bool gemm_skinny_applicable(const GemmArgs &g, int kind) {
   // the rows are whole chunks and nothing has to be padded (f32 256^3 7.8 / 4.7, 300 x 100 x 3000 5.9 / 11.8; u8
   // 400^3 4.4 / 6.2; two k steps of the tiled kernel are as short as this).
   // (From sixteen of the tiled kernel's steps on it shares K out over workgroups.)
+  // A large C over a short K is stores, which the tiled kernel's larger blocks are better at (f32 794 x 27 x 2728 14.0 us,
+  // copies and that one 8.4; 1536 x 16 x 1585 24 / 10); a large B of bytes that needs no copy is read a byte at a time here (u8 21 x
+  // (1 x 1891 x 400) 22.2 / 13.7).
+  if (k_bytes < 512 && double(g.m) * g.n * g.batch > 4096.0 * double(k_bytes)) return false;
+  if (kind <= 1 && g.ldb % 16 == 0 && k_bytes >= 1024 && b_bytes > (4ull << 20)) return false;
   if (k_bytes > 4096 || (k_bytes >= 2048 && macs > 8e6)) return false;
   return chunks ? k_bytes > 256 && macs <= (kind == 3 ? 3e7 : 8e6) : macs <= (kind <= 1 ? 2e7 : 6e7);   // (a byte of B per load)
 }

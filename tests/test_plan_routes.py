@@ -46,3 +46,26 @@ def test_tiles_of_short_digits_fill_their_workgroups(types, inner):
         p = M.Move(shape, types, layouts=[None, M.layout(0, 3, 2, 1, 4)]).plan()
         assert p.kernels == ["k_move_runs"]
         assert p.steps[0].grid[0] * 192 <= math.prod(shape) // 4 + 256 and p.steps[0].grid[0] < 1 << 24
+
+
+@pytest.mark.parametrize("types,shape", [
+    ("bf16", [1, 1, 64000, 14]), ("bf16", [1, 44, 9600, 16]), ("f32", [1, 1, 64000, 64]), ("f32", [1, 4, 9792, 64]), ("u8", [1, 4, 320000, 3]),   # a long K, few columns
+    ("f32", [12, 53, 76, 1533]), ("bf16", [1, 59, 64, 13690]), ("u8", [62, 3, 64, 4096]),   # a short K, thousands of blocks
+])
+def test_few_rows_leave_k_gemm_skinny_where_it_is_the_slower_one(types, shape):
+    dts = {"bf16": (M.bf16, M.bf16, M.f32), "f32": (M.f32,) * 3, "u8": (M.u8, M.i8, M.i32)}[types]
+    kernels = M.Matmul(shape, dts, layouts=[None, KT, None]).plan().kernels
+    assert "k_gemm_skinny" not in kernels and "k_matmul_generic" not in kernels
+
+
+def test_few_rows_stay_with_k_gemm_skinny():
+    for dts, shape in (((M.bf16, M.bf16, M.f32), [1, 1, 4096, 4096]), ((M.u8, M.i8, M.i32), [1, 4, 32768, 30]), ((M.f32,) * 3, [2, 30, 64, 4000]),
+                       ((M.f32,) * 3, [1, 1, 4096, 1000]), ((M.bf16, M.bf16, M.f32), [60, 53, 256, 153])):
+        assert M.Matmul(shape, dts, layouts=[None, KT, None]).plan().kernels == ["k_gemm_skinny"], shape
+
+
+@pytest.mark.parametrize("types,shape", [("f32", [1, 794, 27, 2728]), ("f32", [1, 1536, 16, 1585]), ("bf16", [1, 370, 34, 2386]), ("u8", [21, 1, 1891, 400])])
+def test_small_problems_leave_k_gemm_tiny_where_it_is_the_slower_one(types, shape):
+    dts = {"bf16": (M.bf16, M.bf16, M.f32), "f32": (M.f32,) * 3, "u8": (M.u8, M.i8, M.i32)}[types]
+    kernels = M.Matmul(shape, dts).plan().kernels
+    assert "k_gemm_tiny" not in kernels and "k_matmul_generic" not in kernels
