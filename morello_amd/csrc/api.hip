@@ -527,10 +527,12 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     mrl::Strided b_rows = g.b_kmajor ? transposed(b.t) : b.t;
     // Where both are copied the copies hold zeros up to the next whole chunk of K (a row-major B in rows of
     // its own), and K may as well end there: the four-wave 256 tile takes it then (4518 x 3787 x 4543 u8
-    // 138.3 -> 116.0 us, bf16 218.9 -> 187.0).
+    // 138.3 -> 116.0 us, bf16 218.9 -> 187.0).  It wants twenty of its steps; a short K would only get a copy of many times its
+    // rows (u8 16 x 3 x 4825541: 77 MB for 14).
     const uint32_t whole_k = uint32_t((g.k + per16 - 1) / per16 * per16);
-    if ((rc = make_rows(b, b_rows, g.b_kmajor ? b_rows.shape[1] : whole_k, &b_padded)) != MRL_OK) return rc;
-    if (a_padded && b_padded) g.k = whole_k;
+    const bool end_whole = a_padded && uint64_t(g.k) * a.elem >= 20 * 128;
+    if ((rc = make_rows(b, b_rows, g.b_kmajor ? b_rows.shape[1] : end_whole ? whole_k : g.k, &b_padded)) != MRL_OK) return rc;
+    if (end_whole && b_padded) g.k = whole_k;
     b.t = g.b_kmajor ? transposed(b_rows) : b_rows;
     if (n_pads == 2) HIP_TRY(mrl::launch_pad_rows_pair(pads[0], pads[1], ws.stream));
     else if (n_pads == 1) HIP_TRY(mrl::launch_pad_rows(pads[0], ws.stream));

@@ -69,3 +69,12 @@ def test_small_problems_leave_k_gemm_tiny_where_it_is_the_slower_one(types, shap
     dts = {"bf16": (M.bf16, M.bf16, M.f32), "f32": (M.f32,) * 3, "u8": (M.u8, M.i8, M.i32)}[types]
     kernels = M.Matmul(shape, dts).plan().kernels
     assert "k_gemm_tiny" not in kernels and "k_matmul_generic" not in kernels
+
+
+def test_copies_of_a_short_k_are_no_taller_than_it():
+    """Right operands of one to three rows were copied into 16."""
+    for shape, most in (([1, 16, 3, 4825541], 16 << 20), ([1, 17, 1, 2111355], 4 << 20), ([47805, 1, 2, 187], 24 << 20)):
+        assert M.Matmul(shape, (M.u8, M.i8, M.i32)).plan().scratch_bytes <= most
+    p = M.Matmul([1, 1001, 2050, 4425], (M.bf16, M.bf16, M.bf16)).plan()   # a long one still ends on a whole chunk
+    assert p.kernels == ["k_pad_rows_pair", "k_gemm_ring"]
+    assert M.Matmul([1, 4518, 3787, 4543], (M.u8, M.i8, M.i32)).plan().kernels == ["k_pad_rows_pair", "k_gemm_wide"]
