@@ -474,7 +474,10 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   const double macs = double(g.m) * g.n * g.k * g.batch;
   const double generic_us = 2.5 + 0.04 * g.k + 2.0 * macs / 3e6;
   const double copies_us = 6.0 + 3.5 + 0.45 * double((uint64_t(g.k) * a.elem + 127) / 128);
-  const bool worth_two_more_passes = macs >= 256.0 * 256 * 256 || generic_us > copies_us;
+  // (thousands of dot products of a few dozen bytes, sixteen or fewer to an entry: a 64 x 64 tile each, bf16 50000 x (16 x 16 x 1)
+  // 141 us, generic 43)
+  const bool dots = g.n == 1 && g.m <= 16 && g.batch >= 1024 && uint64_t(g.k) * a.elem <= 128;
+  const bool worth_two_more_passes = !dots && (macs >= 256.0 * 256 * 256 || generic_us > copies_us);
   if (!sched && kind >= 0 && worth_two_more_passes) {
     const int64_t per16 = 16 / int64_t(a.elem);
     auto walkable = [&](const mrl::Strided &t) {
@@ -524,6 +527,13 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     };
     bool a_padded, b_padded;
     if ((rc = make_rows(a, a.t, a.t.shape[1], &a_padded)) != MRL_OK) return rc;
+    // A right operand of one column (or one row) has rows either way: read in place where one of them allows it, else
+    // copied as the fewer bytes (f32 20000 x (3 x 16 x 1): one row of K, or sixteen of an element each).
+    if (!g.b_kmajor && !walkable(b.t)) {
+      const mrl::Strided bt = transposed(b.t);
+      auto copied = [&](const mrl::Strided &t) { return double(t.shape[1]) * double(rows_of(t).stride[1]); };
+      if (walkable(bt) || (as_rows(bt, &any_ld, &any_bs) && copied(bt) < copied(b.t))) g.b_kmajor = true;
+    }
     mrl::Strided b_rows = g.b_kmajor ? transposed(b.t) : b.t;
     // Where both are copied the copies hold zeros up to the next whole chunk of K (a row-major B in rows of
     // its own), and K may as well end there: the four-wave 256 tile takes it then (4518 x 3787 x 4543 u8

@@ -78,3 +78,16 @@ def test_copies_of_a_short_k_are_no_taller_than_it():
     p = M.Matmul([1, 1001, 2050, 4425], (M.bf16, M.bf16, M.bf16)).plan()   # a long one still ends on a whole chunk
     assert p.kernels == ["k_pad_rows_pair", "k_gemm_ring"]
     assert M.Matmul([1, 4518, 3787, 4543], (M.u8, M.i8, M.i32)).plan().kernels == ["k_pad_rows_pair", "k_gemm_wide"]
+
+
+@pytest.mark.parametrize("layout", [None, KT])
+def test_a_right_operand_of_one_column_is_one_row(layout):
+    """It has rows along either dim; along K they are the shorter ones by far once padded to chunks."""
+    for dts, shape, scratch in (((M.f32,) * 3, [39287853, 3, 16, 1], 0), ((M.bf16, M.bf16, M.f32), [50000, 16, 16, 1], 0),
+                                ((M.u8, M.i8, M.i32), [50000, 16, 16, 1], 0), ((M.f32,) * 3, [1, 16, 33864, 1], 1 << 20)):
+        p = M.Matmul(shape, dts, layouts=[None, layout, None]).plan()
+        assert p.scratch_bytes <= scratch and not {"k_pad_rows", "k_pad_rows_pair"} & set(p.kernels), (shape, p)
+        assert ("k_matmul_generic" in p.kernels) == (shape[0] > 1), (shape, p)   # many short dot products: 64 x 64 tiles are mostly padding
+    # neither way whole chunks: a copy of one row, not of one row an element
+    p = M.Matmul([1, 300, 4001, 1], (M.bf16, M.bf16, M.f32), layouts=[None, layout, None]).plan()
+    assert p.scratch_bytes < 300 * 4096 * 2 + 4096 * 2 + (1 << 20)
