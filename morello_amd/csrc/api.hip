@@ -270,6 +270,10 @@ static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 constexpr int MAX_DEVICES = 64;
 void *g_scratch_ptr[MAX_DEVICES] = {};
 
+// Whether this thread's call makes the smallest copies there are (rows padded to 16 bytes and not to whole cache
+// lines, short columns turned): mrl_run_noalloc, for a Spec whose scratch does not fit otherwise.
+thread_local bool g_tight_scratch = false;
+
 struct Workspace {
   hipStream_t stream;
   std::vector<void *> allocs;
@@ -495,7 +499,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
       // whole cache lines where that adds little: the 128 bytes of K (or of a row of B) that a tile takes
       // from a row at a time then lie in one line, not two (bf16 1001 x 2050 x 4425 42.8 us, chunks only 50.7); an
       // f32 tile's MFMAs take longer than its lines (389 x 309 x 851 13.9, chunks only 13.7)
-      const int64_t unit = kind <= 2 && t.shape[2] >= 32 * per16 ? 8 * per16 : per16;
+      const int64_t unit = kind <= 2 && t.shape[2] >= 32 * per16 && !g_tight_scratch ? 8 * per16 : per16;
       d.stride[2] = 1, d.stride[1] = (int64_t(t.shape[2]) + unit - 1) / unit * unit, d.stride[0] = int64_t(t.shape[1]) * d.stride[1];
       return d;
     };
@@ -529,18 +533,19 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     if ((rc = make_rows(a, a.t, a.t.shape[1], &a_padded)) != MRL_OK) return rc;
     // A right operand of one column (or one row) has rows either way: read in place where one of them allows it, else
     // copied as the fewer bytes (f32 20000 x (3 x 16 x 1): one row of K, or sixteen of an element each).
-    if (!g.b_kmajor && !walkable(b.t)) {
-      const mrl::Strided bt = transposed(b.t);
-      auto copied = [&](const mrl::Strided &t) { return double(t.shape[1]) * double(rows_of(t).stride[1]); };
-      if (walkable(bt) || (as_rows(bt, &any_ld, &any_bs) && copied(bt) < copied(b.t))) g.b_kmajor = true;
-    }
+    auto copied = [&](const mrl::Strided &t) { return double(t.shape[1]) * double(rows_of(t).stride[1]); };
+    const mrl::Strided bt = transposed(b.t);
+    if (!g.b_kmajor && !walkable(b.t) && (walkable(bt) || (as_rows(bt, &any_ld, &any_bs) && copied(bt) < copied(b.t)))) g.b_kmajor = true;
+    // Columns of a few bytes grow to a chunk each when they are copied: turned into rows of N instead where that is less
+    // than a sixth (at a fifth the one pass is still the faster: u8 16 x 3 x 400000 23 us, turned 30), or where scratch is short.
+    if (g.b_kmajor && !walkable(bt) && copied(bt) > (g_tight_scratch ? 1 : 6) * copied(b.t)) g.b_kmajor = false;
     mrl::Strided b_rows = g.b_kmajor ? transposed(b.t) : b.t;
     // Where both are copied the copies hold zeros up to the next whole chunk of K (a row-major B in rows of
     // its own), and K may as well end there: the four-wave 256 tile takes it then (4518 x 3787 x 4543 u8
     // 138.3 -> 116.0 us, bf16 218.9 -> 187.0).  It wants twenty of its steps; a short K would only get a copy of many times its
     // rows (u8 16 x 3 x 4825541: 77 MB for 14).
     const uint32_t whole_k = uint32_t((g.k + per16 - 1) / per16 * per16);
-    const bool end_whole = a_padded && uint64_t(g.k) * a.elem >= 20 * 128;
+    const bool end_whole = a_padded && !g_tight_scratch && uint64_t(g.k) * a.elem >= 20 * 128;
     if ((rc = make_rows(b, b_rows, g.b_kmajor ? b_rows.shape[1] : end_whole ? whole_k : g.k, &b_padded)) != MRL_OK) return rc;
     if (end_whole && b_padded) g.k = whole_k;
     b.t = g.b_kmajor ? transposed(b_rows) : b_rows;
@@ -1806,8 +1811,15 @@ int mrl_run_noalloc(const mrl_spec *spec, void *const *params, void *stream) {
   }
   // What the call would take, from the plan (host arithmetic only), so that a Spec that does not
   // fit is turned down before anything is launched.
+  struct Tight {
+    ~Tight() { g_tight_scratch = false; }
+  } until_return;
   mrl_plan plan;
   if ((rc = mrl_spec_plan(spec, &plan, nullptr, 0)) != MRL_OK) return rc;
+  if (plan.scratch_bytes > NOALLOC_SCRATCH_BYTES) {   // with the smallest copies
+    g_tight_scratch = true;
+    if ((rc = mrl_spec_plan(spec, &plan, nullptr, 0)) != MRL_OK) return rc;
+  }
   const std::string too_large = "mrl_run_noalloc: the Spec needs " + std::to_string(plan.scratch_bytes) +
                                 " bytes of scratch, the fixed array holds " + std::to_string(NOALLOC_SCRATCH_BYTES);
   if (plan.scratch_bytes > NOALLOC_SCRATCH_BYTES) {

@@ -1,0 +1,38 @@
+"""mrl_run_noalloc near the end of its fixed scratch: copies that do not fit with their rows padded to cache
+lines, their K to whole chunks, or a right operand's short columns in chunks, are made smaller."""
+import numpy as np
+import pytest
+
+import morello_amd as M
+from gpu_util import run_spec
+from morello_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dts,shape,k_fastest", [
+    ((M.u8, M.i8, M.i32), [1, 56000, 515, 16], False),            # rows of 528 bytes fit, of 640 do not
+    ((M.bf16, M.bf16, M.f32), [1, 5900, 2817, 640], False),       # 5648, 5760
+    ((M.u8, M.i8, M.i32), [2, 40, 3, 1200000], True),             # 2.4 million columns of three bytes, as six rows
+])
+def test_copies_fit_that_did(gpu, dts, shape, k_fastest):
+    b, m, k, n = shape
+    spec = M.Matmul(shape, dts, layouts=[None, M.layout(0, 2, 1) if k_fastest else None, None])
+    assert spec.plan().scratch_bytes > M.NOALLOC_SCRATCH_BYTES
+    bt = (b, n, k) if k_fastest else (b, k, n)
+    if dts[0] == M.u8:
+        arrays = [synth.uniform_u8(950, 0, (b, m, k)), synth.uniform_i8(950, 1, bt), np.zeros((b, m, n), np.int32)]
+    else:
+        arrays = [synth.normal_bf16(950, 0, (b, m, k)), synth.normal_bf16(950, 1, bt), np.zeros((b, m, n), np.float32)]
+    want = run_spec(spec, arrays)
+    bufs = [M.DeviceBuffer.from_numpy(a) for a in arrays]
+    spec.run_noalloc([x.ptr for x in bufs])
+    M.synchronize()
+    got = bufs[2].to_numpy(arrays[2].dtype, arrays[2].shape)
+    for x in bufs:
+        x.free()
+    if dts[2] == M.i32:
+        assert np.array_equal(got, want)
+    else:
+        # the same kernel family over a K that ends elsewhere: f32 sums of 2817 products in another order
+        assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()

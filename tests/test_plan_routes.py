@@ -91,3 +91,8 @@ def test_a_right_operand_of_one_column_is_one_row(layout):
     # neither way whole chunks: a copy of one row, not of one row an element
     p = M.Matmul([1, 300, 4001, 1], (M.bf16, M.bf16, M.f32), layouts=[None, layout, None]).plan()
     assert p.scratch_bytes < 300 * 4096 * 2 + 4096 * 2 + (1 << 20)
+
+
+def test_columns_of_two_bytes_are_turned_not_padded():
+    assert M.Matmul([1, 17, 2, 12613142], (M.i8, M.i8, M.i32), layouts=[None, KT, None]).plan().scratch_bytes <= 32 << 20
+    assert M.Matmul([1, 16, 3, 400000], (M.u8, M.i8, M.i32), layouts=[None, KT, None]).plan().kernels == ["k_pad_rows_pair", "k_gemm"]   # a fifth: still one pass
