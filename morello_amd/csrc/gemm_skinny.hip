@@ -363,7 +363,7 @@ hipError_t launch_kind(const GemmArgs &g, hipStream_t stream) {
 
 bool gemm_skinny_applicable(const GemmArgs &g, int kind) {
   const uint64_t es = kind == 3 ? 4 : kind == 2 ? 2 : 1, k_bytes = uint64_t(g.k) * es, b_bytes = k_bytes * g.n * g.batch;
-  if (k_bytes < 64 || k_bytes >= (1ull << 31) || g.batch > 65535 || (g.m + 15) / 16 > 65535) return false;
+  if (k_bytes < 64 || k_bytes >= (1ull << 31) || g.batch > 65535 || (g.m + 15) / 16 > 65535 || g.n >= (1u << 26)) return false;
   // element-aligned operands
   if (reinterpret_cast<uintptr_t>(g.a) % es || reinterpret_cast<uintptr_t>(g.b) % es) return false;
   const double macs = double(g.m) * g.n * g.k * g.batch;
@@ -371,16 +371,21 @@ bool gemm_skinny_applicable(const GemmArgs &g, int kind) {
   if (g.b_kmajor) {
     const uint64_t cols = (uint64_t(g.n) + 15) / 16 * g.batch;
     // Few columns and a long K: the tiled kernel with K shared out over workgroups, or, for a row or a few of f32, the dot
-    // products.  One workgroup's eight waves take 0.26 us per KB of K (f32 0.4, more rows more), the others 6 to 20 us
-    // with their copies and the sum (us, this / the others: bf16 1 x 64000 x 14 36.4 / 17.4, 44 x 9600 x 16 15.5 / 7.9, 10 x
-    // 24416 x 16 15.6 / 20.8; f32 4 x 9792 x 64 16.9 / 7.0).
+    // products.  One workgroup's eight waves take 0.26 us per KB of K (f32 0.4, more rows more), the others 5 to 9 us
+    // where K falls into equal slices of rows read in place, and 10 to 20 with their copies or a slice left over (us, this / the
+    // others: bf16 1 x 64000 x 14 36.4 / 17.4, 1 x 16000 x 64 10.8 / 5.2, 4 x 10176 x 16 7.7 / 11.9, 10 x 24416 x 16 15.6 / 20.8, 44 x 9600 x 16
+    // 15.5 / 7.9; f32 4 x 9792 x 64 16.9 / 7.0).
     if (g.m > 64 || (cols < 64 && macs > 8e6)) return false;
-    if (g.batch == 1 && cols < 64 && macs >= 1e5 && k_bytes > (g.m > 16 ? 16384 : 40960)) return false;
+    if (g.batch == 1 && cols < 64 && macs >= 1e5 && k_bytes > 16384) {
+      uint32_t left = 0;
+      const bool slices = chunks && gemm_k_splits(g, kind, &left) > 1 && left == 0;
+      if (g.m > 16 || k_bytes > (slices ? 24576 : 40960)) return false;
+    }
     if (kind == 3 && g.batch == 1 && cols < 32 && g.n >= 64 && g.m <= 4 && chunks && k_bytes >= 8192) return false;
-    // A short K keeps one to four of the eight waves: past two thousand blocks, which fill the chip several times over, the
-    // tiled kernel (us, this / that: f32 12 x (53 x 76 x 1533) 18.7 / 7.0, bf16 59 x 64 x 13690 6.3 / 3.0, u8 62 x (3 x 64 x 4096)
+    // A short K keeps one to four of the eight waves: past two thousand blocks, which fill the chip several times over, and
+    // with columns for more than half of a tile (f32 18643 x (3 x 16 x 16) 36 / 73), the tiled kernel (us, this / that: f32 12 x (53 x 76 x 1533) 18.7 / 7.0, bf16 59 x 64 x 13690 6.3 / 3.0, u8 62 x (3 x 64 x 4096)
     // 22.6 / 10.7; a thousand blocks or 512 bytes are even).
-    if (cols * ((g.m + 15) / 16) > 2048 && k_bytes < 512) return false;
+    if (cols * ((g.m + 15) / 16) > 2048 && k_bytes < 512 && g.n > 32) return false;
     if (kind == 3 && g.m > 32 && k_bytes < 256) return false;   // (f32 42 x 22 x 192 4.2 / 2.8)
     // One or two rows against a large B: the dot products (bf16 1 x 2048 x 16384 12.2 us, this 13.3; but
     // 1 x 4096 x 4096 9.5, 8.3).  More than 32 rows of whole chunks: past 8 MB of B the tiled kernel, which reads

@@ -49,7 +49,7 @@ def test_tiles_of_short_digits_fill_their_workgroups(types, inner):
 
 
 @pytest.mark.parametrize("types,shape", [
-    ("bf16", [1, 1, 64000, 14]), ("bf16", [1, 44, 9600, 16]), ("f32", [1, 1, 64000, 64]), ("f32", [1, 4, 9792, 64]), ("u8", [1, 4, 320000, 3]),   # a long K, few columns
+    ("bf16", [1, 1, 64000, 14]), ("bf16", [1, 44, 9600, 16]), ("f32", [1, 1, 64000, 64]), ("f32", [1, 4, 9792, 64]), ("bf16", [1, 1, 16000, 64]), ("u8", [1, 4, 320000, 3]),   # a long K, few columns
     ("f32", [12, 53, 76, 1533]), ("bf16", [1, 59, 64, 13690]), ("u8", [62, 3, 64, 4096]),   # a short K, thousands of blocks
 ])
 def test_few_rows_leave_k_gemm_skinny_where_it_is_the_slower_one(types, shape):
@@ -59,7 +59,7 @@ def test_few_rows_leave_k_gemm_skinny_where_it_is_the_slower_one(types, shape):
 
 
 def test_few_rows_stay_with_k_gemm_skinny():
-    for dts, shape in (((M.bf16, M.bf16, M.f32), [1, 1, 4096, 4096]), ((M.u8, M.i8, M.i32), [1, 4, 32768, 30]), ((M.f32,) * 3, [2, 30, 64, 4000]),
+    for dts, shape in (((M.bf16, M.bf16, M.f32), [1, 1, 4096, 4096]), ((M.u8, M.i8, M.i32), [1, 4, 32767, 30]), ((M.bf16, M.bf16, M.f32), [1, 4, 10176, 16]), ((M.f32,) * 3, [18643, 3, 16, 16]), ((M.f32,) * 3, [2, 30, 64, 4000]),
                        ((M.f32,) * 3, [1, 1, 4096, 1000]), ((M.bf16, M.bf16, M.f32), [60, 53, 256, 153])):
         assert M.Matmul(shape, dts, layouts=[None, KT, None]).plan().kernels == ["k_gemm_skinny"], shape
 
