@@ -300,7 +300,7 @@ hipError_t launch_wide(const GemmArgs &g, hipStream_t stream) {
   const int tiles_m = int((g.m + 255) / 256), tiles_n = int((g.n + 255) / 256);
   const double mn = double(g.m) * g.n * g.batch;
   plan::work(T::ES == 1 ? plan::UNIT_MFMA_I8 : plan::UNIT_MFMA_BF16, 2.0 * mn * g.k,
-             (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * 4 * (g.accum ? 2 : 1),
+             (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * (g.c_bf16 ? 2 : 4) * (g.accum ? 2 : 1),
              2.0 * 256 * 256 * double(g.k), 500.0 + 1200.0 * double(g.k * T::ES / 128),
              T::ES == 1 ? 1.62 : 1.18);  // measured: 2230-2330 TOPS int8 at 4096^3, 1360 TFLOPS bf16 at 8192^3
   const TileWalk walk = tile_walk(tiles_m, tiles_n);

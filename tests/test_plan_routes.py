@@ -96,3 +96,12 @@ def test_a_right_operand_of_one_column_is_one_row(layout):
 def test_columns_of_two_bytes_are_turned_not_padded():
     assert M.Matmul([1, 17, 2, 12613142], (M.i8, M.i8, M.i32), layouts=[None, KT, None]).plan().scratch_bytes <= 32 << 20
     assert M.Matmul([1, 16, 3, 400000], (M.u8, M.i8, M.i32), layouts=[None, KT, None]).plan().kernels == ["k_pad_rows_pair", "k_gemm"]   # a fifth: still one pass
+
+
+@pytest.mark.parametrize("shape", [[1, 8192, 8192, 8192], [1, 2560, 2560, 2560], [1, 1001, 2050, 4425], [1, 300, 520, 416], [1, 2, 2048, 16384]])
+def test_plans_count_bf16_results_as_two_bytes(shape):
+    b, m, k, n = shape
+    for dt, es in ((M.bf16, 2), (M.f32, 4)):
+        step = M.Matmul(shape, (M.bf16, M.bf16, dt), layouts=[None, KT, None]).plan().steps[-1]
+        whole = 8 * ((k + 7) // 8)   # (a copied K ends on a whole chunk)
+        assert step.bytes in [2 * (m + n) * kk + es * m * n for kk in (k, whole)], (step, dt)
