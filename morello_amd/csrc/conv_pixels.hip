@@ -53,11 +53,11 @@ struct PixelsArgs {
 };
 
 // KS: whole k steps of 64 bytes (a window's chunks / 4); the rest is a tail whose lanes past the
-// filter's last row count for nothing.
-template <int KS, int KIND>
+// filter's last row count for nothing.  PIXELS: always true; tells this form from the other one in plans and profiles.
+template <int KS, int KIND, bool PIXELS>
 __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
   constexpr bool HALVES = KIND == IMG_BF16;
-  constexpr int ES = HALVES ? 2 : 1, PB = 4 * ES, PIXELS = 16 / PB;   // bytes of a pixel in LDS, pixels of a chunk
+  constexpr int ES = HALVES ? 2 : 1, PB = 4 * ES, PER_CHUNK = 16 / PB;   // bytes of a pixel in LDS, pixels of a chunk
   typedef typename std::conditional<HALVES, v4f, v4i>::type Acc;
   auto mfma = [](v4i a, v4i b, Acc c) {
     if constexpr (HALVES) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
@@ -142,11 +142,11 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
     }
     __syncthreads();
     const uint32_t *words = reinterpret_cast<const uint32_t *>(raw);
-    const uint32_t per_row = uint32_t(PIXELS) << p.chunks_log2;   // pixels a window's row takes
+    const uint32_t per_row = uint32_t(PER_CHUNK) << p.chunks_log2;   // pixels a window's row takes
 #pragma unroll 2
     for (uint32_t i = tid; i < p.group * p.slots; i += 64 * WAVES) {
       const uint32_t fi = p.by_slots.div(i), s = i - fi * p.slots;
-      const uint32_t r = s / PIXELS >> p.chunks_log2, x = s & (per_row - 1);
+      const uint32_t r = s / PER_CHUNK >> p.chunks_log2, x = s & (per_row - 1);
       const bool real = fi < nf && r < p.fh && x < p.fw;
       const uint32_t at = real ? head + ((fi * p.fh + r) * p.fw + x) * p.pixel_bytes : head;
       Raw px;
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
   const uint32_t row_bytes = p.patch_w * PB, chunk = lg & ((1u << p.chunks_log2) - 1), row_of = uint32_t(lg) >> p.chunks_log2;
   const uint32_t step_bytes = (4u >> p.chunks_log2) * row_bytes;
   const uint8_t *my_patch = patch + row_of * row_bytes + li * PB + chunk * 16;
-  const uint32_t keep_lo = chunk * PIXELS < p.fw ? 0xffffffffu : 0u, keep_hi = chunk * PIXELS + 1 < p.fw ? 0xffffffffu : 0u;
+  const uint32_t keep_lo = chunk * PER_CHUNK < p.fw ? 0xffffffffu : 0u, keep_hi = chunk * PER_CHUNK + 1 < p.fw ? 0xffffffffu : 0u;
   auto window = [&](uint32_t ks, int pb) {
     const uint8_t *at = my_patch + ks * step_bytes + pb * row_bytes;
     if constexpr (HALVES) {
@@ -254,14 +254,14 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
   }
 }
 
-template <int KS, int KIND>
+template <int KS, int KIND, bool PIXELS = true>
 hipError_t launch(const PixelsArgs &p, dim3 grid, size_t lds, hipStream_t stream) {
   static std::atomic<uint64_t> limit{0};
   if (!plan::recording() && lds > 65536) {
-    hipError_t e = raise_lds_limit(limit, (const void *)k_conv_windows<KS, KIND>, int(lds));
+    hipError_t e = raise_lds_limit(limit, (const void *)k_conv_windows<KS, KIND, PIXELS>, int(lds));
     if (e != hipSuccess) return e;
   }
-  MRL_LAUNCH((k_conv_windows<KS, KIND>), grid, dim3(64 * WAVES), lds, stream, p);
+  MRL_LAUNCH((k_conv_windows<KS, KIND, PIXELS>), grid, dim3(64 * WAVES), lds, stream, p);
   return plan::last_error();
 }
 template <int KS>

@@ -105,3 +105,9 @@ def test_plans_count_bf16_results_as_two_bytes(shape):
         step = M.Matmul(shape, (M.bf16, M.bf16, dt), layouts=[None, KT, None]).plan().steps[-1]
         whole = 8 * ((k + 7) // 8)   # (a copied K ends on a whole chunk)
         assert step.bytes in [2 * (m + n) * kk + es * m * n for kk in (k, whole)], (step, dt)
+
+
+def test_the_two_forms_of_k_conv_windows_are_told_apart():
+    pixels = M.Conv([32, 64, 3, 112, 112, 7, 7], (M.u8, M.i8, M.i32)).plan().steps[0].kernel
+    windows = M.Conv([8, 32, 3, 110, 110, 5, 5], (M.f32, M.f32, M.f32)).plan().steps[0].kernel
+    assert "PIXELS = true" in pixels and "PIXELS" not in windows
