@@ -64,14 +64,15 @@ __device__ inline int swizzle(int byte, int r) {
   return ((byte / PIECE) ^ x) * PIECE + byte % PIECE;
 }
 
-// One load of 64 lanes x 16 bytes into the KiB at LDS address m0 + AT (wave-uniform), lane l to the l-th
+// One load of 64 lanes x 16 bytes into the KiB at LDS address `lds_addr` + AT (wave-uniform), lane l to the l-th
 // 16 bytes; the instruction's offset AT is added to the address in memory too, so callers take it off
-// there.  An offset outside the resource brings zeros.  Assembly, so that the compiler does not wait for it.
+// there.  An offset outside the resource brings zeros.  Assembly, so that the compiler does not wait for it; M0 is set in
+// the same statement, with the wait state it needs: the compiler sets that reserved register right before its own
+// uses and keeps nothing in it, and may do so between any two statements.
 template <int AT>
-__device__ inline void dma16(__amdgpu_buffer_rsrc_t from, uint32_t off) {
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" : : "v"(off), "s"(from), "n"(AT) : "memory");
+__device__ inline void dma16(__amdgpu_buffer_rsrc_t from, uint32_t off, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen offset:%3 lds" : : "v"(off), "s"(from), "s"(lds_addr), "n"(AT) : "memory");
 }
-__device__ inline void dma_to(uint32_t lds_addr) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(lds_addr) : "memory"); }
 __device__ inline __amdgpu_buffer_rsrc_t resource(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, int(bytes), 0x00020000);
 }
@@ -161,13 +162,8 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
   // Its i-th load of this wave.
   auto load = [&](auto which) {
     constexpr int I = decltype(which)::value;
-    if constexpr (I < A_LOADS) {
-      if constexpr (I == 0) dma_to(a_dst);
-      dma16<I * 1024>(a_buf, a_off[I]);
-    } else {
-      dma_to(b_dst + b_load(I - A_LOADS) * 1024);
-      dma16<0>(b_buf, b_off[I - A_LOADS]);
-    }
+    if constexpr (I < A_LOADS) dma16<I * 1024>(a_buf, a_off[I], a_dst);
+    else dma16<0>(b_buf, b_off[I - A_LOADS], b_dst + b_load(I - A_LOADS) * 1024);
   };
   auto advance = [&]() {
     left -= STEP;
