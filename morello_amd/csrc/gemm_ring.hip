@@ -256,22 +256,22 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
       colsum[c] += __shfl_xor(colsum[c], 32);
       colsum[c] *= 128;
     }
-  constexpr int ROW = WN + 4, HALVES = RB > 6 ? 2 : 1, ROWS = WM / HALVES;   // (all of it, or half, fits the ring)
-  Out *piece = (Out *)lds + (wave & 3) * (ROWS * ROW);
+  constexpr int ROW = WN + 4;
+  Out *piece = (Out *)lds + (wave & 3) * (WM * ROW);
   const int64_t row_first = m0 + wm * WM, col_first = n0 + wn * WN;
   const int cols = int(min(int64_t(WN), int64_t(g.n) - col_first));
   // (The loops stay loops: code that a launch runs once is fetched from memory, and unrolled it took longer to
   // fetch than to run.)
-  auto store = [&](auto *C, int half) {
+  auto store = [&](auto *C) {
     typedef std::remove_pointer_t<decltype(C)> Stored;
     typedef Stored four __attribute__((ext_vector_type(4)));
     typedef Out out4 __attribute__((ext_vector_type(4)));
-    C += int64_t(blockIdx.y) * g.sc + (row_first + half * ROWS) * g.ldc + col_first;
-    const int rows = int(min(int64_t(ROWS), int64_t(g.m) - row_first - half * ROWS));
+    C += int64_t(blockIdx.y) * g.sc + row_first * g.ldc + col_first;
+    const int rows = int(min(int64_t(WM), int64_t(g.m) - row_first));
     // four columns at a time where all of a row's are whole and aligned
     if (cols % 4 == 0 && g.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % (4 * sizeof(Stored)) == 0) {
 #pragma unroll 4
-      for (int e = 0; e < ROWS * WN / 4 / 128; e++) {
+      for (int e = 0; e < WM * WN / 4 / 128; e++) {
         const int at = (2 * e + kw) * 64 + lane, row = at / (WN / 4), col = at % (WN / 4) * 4;
         if (row < rows && col < cols) {
           out4 v = *(const out4 *)(piece + row * ROW + col);
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
       }
     } else {
 #pragma unroll 4
-      for (int e = 0; e < ROWS * WN / 128; e++) {
+      for (int e = 0; e < WM * WN / 128; e++) {
         const int at = (2 * e + kw) * 64 + lane, row = at / WN, col = at % WN;
         if (row < rows && col < cols) {
           Out v = piece[row * ROW + col];
@@ -294,31 +294,27 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
     }
   };
   // The two halves of K: the upper waves' sums through LDS onto the lower waves', and both store.
+  auto for_each_sum = [&](auto f) {
 #pragma unroll
-  for (int half = 0; half < HALVES; half++) {
-    auto for_each_of_half = [&](auto f) {
+    for (int r = 0; r < RA; r++)
 #pragma unroll
-      for (int r = 0; r < RA / HALVES; r++)
+      for (int c = 0; c < RB; c++)
 #pragma unroll
-        for (int c = 0; c < RB; c++)
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            Out v = acc[half * (RA / HALVES) + r][c][i];
-            if (A_UNSIGNED) v += Out(colsum[c]);
-            f(piece[(r * 16 + 4 * lg + i) * ROW + c * 16 + li], v);
-          }
-    };
-    if (kw) for_each_of_half([](Out &at, Out v) { at = v; });
-    __syncthreads();
-    if (!kw) for_each_of_half([](Out &at, Out v) { at = v + at; });
-    __syncthreads();
-    if (cols > 0 && row_first < int64_t(g.m)) {
-      if constexpr (std::is_same<T, BF16>::value) {
-        if (g.c_bf16) store((__bf16 *)g.c, half);
-        else store((Out *)g.c, half);
-      } else store((Out *)g.c, half);
-    }
-    if (half + 1 < HALVES) __syncthreads();
+        for (int i = 0; i < 4; i++) {
+          Out v = acc[r][c][i];
+          if (A_UNSIGNED) v += Out(colsum[c]);
+          f(piece[(r * 16 + 4 * lg + i) * ROW + c * 16 + li], v);
+        }
+  };
+  if (kw) for_each_sum([](Out &at, Out v) { at = v; });
+  __syncthreads();
+  if (!kw) for_each_sum([](Out &at, Out v) { at = v + at; });
+  __syncthreads();
+  if (cols > 0 && row_first < int64_t(g.m)) {
+    if constexpr (std::is_same<T, BF16>::value) {
+      if (g.c_bf16) store((__bf16 *)g.c);
+      else store((Out *)g.c);
+    } else store((Out *)g.c);
   }
 }
 
