@@ -542,10 +542,10 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     mrl::Strided b_rows = g.b_kmajor ? transposed(b.t) : b.t;
     // Where both are copied the copies hold zeros up to the next whole chunk of K (a row-major B in rows of
     // its own), and K may as well end there: the four-wave 256 tile takes it then (4518 x 3787 x 4543 u8
-    // 138.3 -> 116.0 us, bf16 218.9 -> 187.0).  It wants twenty of its steps; a short K would only get a copy of many times its
-    // rows (u8 16 x 3 x 4825541: 77 MB for 14).
+    // 138.3 -> 116.0 us, bf16 218.9 -> 187.0), and K falls into equal slices (u8 384 x 2559 x 128 15.0 us, 12.5).  Both want sixteen
+    // steps or more; a short row-major operand would only get a copy of many times its rows (u8 16 x 3 x 4825541: 77 MB for 14).
     const uint32_t whole_k = uint32_t((g.k + per16 - 1) / per16 * per16);
-    const bool end_whole = a_padded && !g_tight_scratch && uint64_t(g.k) * a.elem >= 20 * 128;
+    const bool end_whole = a_padded && !g_tight_scratch && (g.b_kmajor || uint64_t(whole_k) * a.elem >= 16 * 128);
     if ((rc = make_rows(b, b_rows, g.b_kmajor ? b_rows.shape[1] : end_whole ? whole_k : g.k, &b_padded)) != MRL_OK) return rc;
     if (end_whole && b_padded) g.k = whole_k;
     b.t = g.b_kmajor ? transposed(b_rows) : b_rows;

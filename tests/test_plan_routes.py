@@ -78,6 +78,8 @@ def test_copies_of_a_short_k_are_no_taller_than_it():
     p = M.Matmul([1, 1001, 2050, 4425], (M.bf16, M.bf16, M.bf16)).plan()   # a long one still ends on a whole chunk
     assert p.kernels == ["k_pad_rows_pair", "k_gemm_ring"]
     assert M.Matmul([1, 4518, 3787, 4543], (M.u8, M.i8, M.i32)).plan().kernels == ["k_pad_rows_pair", "k_gemm_wide"]
+    for layout in (None, KT):   # ... which falls into equal slices
+        assert M.Matmul([1, 384, 2559, 120], (M.u8, M.i8, M.i32), layouts=[None, layout, None]).plan().kernels == ["k_pad_rows_pair", "k_gemm", "k_sum_splits"]
 
 
 @pytest.mark.parametrize("layout", [None, KT])
