@@ -830,7 +830,7 @@ __global__ __launch_bounds__(256) void k_widen_bf16(const uint16_t *__restrict__
 }
 
 // Copies [batch][rows][cols] with contiguous rows, starting on any element, into `dst_rows` rows of whole
-// 16-byte chunks, zeros from each row's end on and in the rows past the last.  A thread makes four
+// 16-byte chunks, zeros from each row's end on and in the rows past the last.  A thread makes one or four
 // chunks, each out of the two aligned chunks of the source it lies in (with a load per element, u8
 // 5440 x 1683 x 2556 took 62.9 us in all; 46.7 now).
 struct PadJob {
@@ -843,13 +843,14 @@ struct PadJob {
   FastDiv by_row_chunks, by_dst_rows;
 };
 constexpr int PAD_UNROLL = 4;
+template <int UNROLL>
 __device__ inline void pad_chunks(const PadJob &j) {
-  const uint32_t first = blockIdx.x * (256 * PAD_UNROLL) + threadIdx.x;
-  chunk_t lo[PAD_UNROLL], hi[PAD_UNROLL];
-  int left[PAD_UNROLL];
-  uint32_t shift[PAD_UNROLL];
+  const uint32_t first = blockIdx.x * (256 * UNROLL) + threadIdx.x;
+  chunk_t lo[UNROLL], hi[UNROLL];
+  int left[UNROLL];
+  uint32_t shift[UNROLL];
 #pragma unroll
-  for (int u = 0; u < PAD_UNROLL; u++) {
+  for (int u = 0; u < UNROLL; u++) {
     const uint32_t i = min(first + u * 256, j.chunks - 1);
     const uint32_t line = j.by_row_chunks.div(i), entry = j.by_dst_rows.div(line), row = line - entry * j.dst_rows;
     const PadChunk c = pad_chunk(i - line * j.row_chunks, row < j.rows ? j.row_bytes : 0);
@@ -862,15 +863,17 @@ __device__ inline void pad_chunks(const PadJob &j) {
     hi[u] = *(const chunk_t *)(from + (int(shift[u]) + left[u] > 16 ? 16 : 0));
   }
 #pragma unroll
-  for (int u = 0; u < PAD_UNROLL; u++)
+  for (int u = 0; u < UNROLL; u++)
     if (first + u * 256 < j.chunks) j.dst[first + u * 256] = keep_bytes(cut_chunk(lo[u], hi[u], shift[u]), left[u]);
 }
-__global__ __launch_bounds__(256) void k_pad_rows(PadJob j) { pad_chunks(j); }
+template <int UNROLL>
+__global__ __launch_bounds__(256) void k_pad_rows(PadJob j) { pad_chunks<UNROLL>(j); }
 // Two such copies in one launch (blockIdx.y names the copy): the two operands of a Matmul whose rows
 // are not whole 16-byte chunks each took a launch of about 2.4 us for their padded copy (int8 1000^3).
+template <int UNROLL>
 __global__ __launch_bounds__(256) void k_pad_rows_pair(PadJob j0, PadJob j1) {
   const PadJob &j = blockIdx.y ? j1 : j0;
-  if (blockIdx.x * (256 * PAD_UNROLL) < j.chunks) pad_chunks(j);
+  if (blockIdx.x * (256 * UNROLL) < j.chunks) pad_chunks<UNROLL>(j);
 }
 
 __global__ void k_copy1(const uint8_t *src, uint8_t *dst, uint64_t bytes) {
@@ -1734,6 +1737,10 @@ bool pad_job(const PadRows &p, PadJob *j) {
   j->by_row_chunks = FastDiv(j->row_chunks), j->by_dst_rows = FastDiv(j->dst_rows);
   return true;
 }
+// Four chunks a thread, their loads in flight together, for copies that fill the chip several times over; below, one a
+// thread, a shorter way to the first load (whole Matmuls of random sizes, four / one, geometric means by chunks of the larger
+// operand: 16 thousand 8.1 / 7.3 us, 256 thousand 20.6 / 19.8, 1 Mi 37.4 / 37.2, 4 Mi 97.0 / 100.6).
+bool pad_in_fours(uint32_t chunks) { return chunks >= 4096ull * g_compute_units; }
 double pad_bytes(const PadJob &j) { return double(j.chunks) / j.row_chunks / j.dst_rows * j.rows * j.row_bytes + 16.0 * j.chunks; }
 }  // namespace
 
@@ -1741,7 +1748,8 @@ hipError_t launch_pad_rows(const PadRows &p, hipStream_t stream) {
   PadJob j;
   if (!pad_job(p, &j)) return hipErrorInvalidValue;
   plan::work(plan::UNIT_STREAM, 0, pad_bytes(j));
-  MRL_LAUNCH(k_pad_rows, dim3((j.chunks + 256 * PAD_UNROLL - 1) / (256 * PAD_UNROLL)), dim3(256), 0, stream, j);
+  if (pad_in_fours(j.chunks)) MRL_LAUNCH((k_pad_rows<PAD_UNROLL>), dim3((j.chunks + 256 * PAD_UNROLL - 1) / (256 * PAD_UNROLL)), dim3(256), 0, stream, j);
+  else MRL_LAUNCH((k_pad_rows<1>), dim3((j.chunks + 255) / 256), dim3(256), 0, stream, j);
   return mrl::plan::last_error();
 }
 
@@ -1750,7 +1758,8 @@ hipError_t launch_pad_rows_pair(const PadRows &p0, const PadRows &p1, hipStream_
   if (!pad_job(p0, &j0) || !pad_job(p1, &j1)) return hipErrorInvalidValue;
   plan::work(plan::UNIT_STREAM, 0, pad_bytes(j0) + pad_bytes(j1));
   const uint32_t most = std::max(j0.chunks, j1.chunks);
-  MRL_LAUNCH(k_pad_rows_pair, dim3((most + 256 * PAD_UNROLL - 1) / (256 * PAD_UNROLL), 2), dim3(256), 0, stream, j0, j1);
+  if (pad_in_fours(most)) MRL_LAUNCH((k_pad_rows_pair<PAD_UNROLL>), dim3((most + 256 * PAD_UNROLL - 1) / (256 * PAD_UNROLL), 2), dim3(256), 0, stream, j0, j1);
+  else MRL_LAUNCH((k_pad_rows_pair<1>), dim3((most + 255) / 256, 2), dim3(256), 0, stream, j0, j1);
   return mrl::plan::last_error();
 }
 

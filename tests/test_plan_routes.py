@@ -113,3 +113,10 @@ def test_the_two_forms_of_k_conv_windows_are_told_apart():
     pixels = M.Conv([32, 64, 3, 112, 112, 7, 7], (M.u8, M.i8, M.i32)).plan().steps[0].kernel
     windows = M.Conv([8, 32, 3, 110, 110, 5, 5], (M.f32, M.f32, M.f32)).plan().steps[0].kernel
     assert "PIXELS = true" in pixels and "PIXELS" not in windows
+
+
+def test_padded_copies_of_up_to_a_million_chunks_go_one_to_a_thread():
+    step = M.Matmul([1, 1000, 1000, 1000], (M.u8, M.i8, M.i32)).plan().steps[0]
+    assert step.family == "k_pad_rows_pair" and step.grid[0] == (1000 * 64 + 255) // 256
+    step = M.Matmul([1, 5003, 4001, 5001], (M.bf16, M.bf16, M.f32)).plan().steps[0]
+    assert step.family == "k_pad_rows_pair" and step.grid[0] <= 5003 * 632 // 1024 + 1
