@@ -237,7 +237,8 @@ int mrl_run_async(const mrl_spec *spec, void *const *params, void *stream);
  * must be the calling thread's current one (MRL_ERR_NO_DEVICE otherwise).  Parameters are 256-byte
  * aligned, as device allocations are (MRL_ERR_UNSUPPORTED otherwise: the scratch need of a
  * misaligned call is not the plan's).  A Spec whose scratch need (mrl_spec_plan: scratch_bytes)
- * exceeds the array is turned down with MRL_ERR_TOO_LARGE before anything is launched.  All calls
+ * exceeds the array runs with smaller copies of its operands (rows padded to 16 bytes instead of whole
+ * cache lines) if it fits that way, and is otherwise turned down with MRL_ERR_TOO_LARGE before anything is launched.  All calls
  * on one GPU share the array: two that
  * overlap in time (different streams, or different host threads on one stream) race; the caller
  * serialises them. */

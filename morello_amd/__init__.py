@@ -283,7 +283,8 @@ class Spec:
 
     def run_noalloc(self, ptrs: Sequence[int], stream: "Stream | None" = None):
         """As run_async without any device allocation: scratch comes from the library's fixed
-        per-GPU array (NOALLOC_SCRATCH_BYTES); MorelloError (tensor too large) if the Spec needs more."""
+        per-GPU array (NOALLOC_SCRATCH_BYTES); MorelloError (tensor too large) if the Spec needs more
+        even with the smallest copies of its operands."""
         arr = (C.c_void_p * len(ptrs))(*ptrs)
         _check(B.load().mrl_run_noalloc(C.byref(self._c), arr, stream.handle if stream else None), "mrl_run_noalloc")
 
