@@ -11,6 +11,7 @@
 // theirs is the ceiling.
 #include <vector>
 
+#include "host_stage.h"
 #include "kernels.h"
 
 namespace mrl {
@@ -95,8 +96,8 @@ hipError_t measure_mfma_rate(int kind, bool random_operands, uint32_t iters, hip
     cleanup();              \
     return e;               \
   }
-  TRY(hipMalloc(&src, quads * sizeof(v4i)));
-  TRY(hipMalloc(&sink, size_t(cus) * 512 * sizeof(float)));
+  TRY(device_malloc(reinterpret_cast<void **>(&src), quads * sizeof(v4i)));
+  TRY(device_malloc(reinterpret_cast<void **>(&sink), size_t(cus) * 512 * sizeof(float)));
   TRY(hipMemcpyAsync(src, host.data(), quads * sizeof(v4i), hipMemcpyHostToDevice, stream));
   TRY(hipEventCreate(&e0));
   TRY(hipEventCreate(&e1));
