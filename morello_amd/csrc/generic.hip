@@ -12,23 +12,12 @@
 
 #include "kernels.h"
 #include "layout_factor.h"
+#include "move_device.h"
 #include "pad_position.h"
 #include "row_chunks.h"
 
 namespace mrl {
 namespace {
-
-__device__ inline float bf16_bits_to_f32(uint16_t v) { return __uint_as_float(uint32_t(v) << 16); }
-
-__device__ inline uint32_t narrow_int(int dtype, uint32_t v) {
-  switch (dtype) {
-    case MRL_U8: return v & 0xffu;
-    case MRL_I8: return uint32_t(int32_t(int8_t(uint8_t(v))));
-    case MRL_U16: return v & 0xffffu;
-    case MRL_I16: return uint32_t(int32_t(int16_t(uint16_t(v))));
-    default: return v;
-  }
-}
 
 __device__ inline float load_f32(const void *p, int dtype, int64_t off) {
   switch (dtype) {
@@ -41,22 +30,6 @@ __device__ inline float load_f32(const void *p, int dtype, int64_t off) {
     case MRL_F32: return ((const float *)p)[off];
     default: return bf16_bits_to_f32(((const uint16_t *)p)[off]);
   }
-}
-
-// Rust `as` for narrow integer targets saturates floats at the target's own bounds.
-__device__ inline uint32_t float_to_int(float f, int dt) {
-  if (f != f) return 0;
-  float lo, hi;
-  switch (dt) {
-    case MRL_U8: lo = 0.f, hi = 255.f; break;
-    case MRL_I8: lo = -128.f, hi = 127.f; break;
-    case MRL_U16: lo = 0.f, hi = 65535.f; break;
-    case MRL_I16: lo = -32768.f, hi = 32767.f; break;
-    case MRL_U32: return f <= 0.f ? 0u : f >= 4294967296.f ? 0xffffffffu : uint32_t(f);
-    default: return f <= -2147483648.f ? 0x80000000u : f >= 2147483648.f ? 0x7fffffffu : uint32_t(int32_t(f));
-  }
-  f = fminf(fmaxf(f, lo), hi);
-  return uint32_t(int32_t(f));
 }
 
 // Rust `as` semantics (verification.rs:547-569, `x.as_()` into the output dtype): integers wrap,
@@ -101,13 +74,6 @@ __global__ void k_relayout(const uint8_t *src, uint8_t *dst, LayoutEval sl, Layo
 }
 
 // ---------------------------------------------------------------------- move
-__device__ inline uint16_t f32_to_bf16_bits(float f) {
-  uint32_t bits = __float_as_uint(f);
-  if ((bits & 0x7fffffffu) > 0x7f800000u) return uint16_t((bits >> 16) | 0x40u);
-  bits += 0x7fffu + ((bits >> 16) & 1u);  // round to nearest even
-  return uint16_t(bits >> 16);
-}
-
 // One element: read as `sdt`, converted with Rust `as` semantics, returned as the bits of `ddt`.
 __device__ inline uint32_t move_bits(const void *src, int sdt, int64_t so, int ddt) {
   if (sdt == ddt) {  // bits as they are (a NaN keeps its payload)
@@ -121,70 +87,10 @@ __device__ inline uint32_t move_bits(const void *src, int sdt, int64_t so, int d
   return load_u32(src, sdt, so, MRL_U32);  // int -> int wraps
 }
 
-// An element's bits, zero-extended, by element size alone (no dtype switch around the load).
-template <int SIZE>
-__device__ inline uint32_t load_sized(const void *p, int64_t off) {
-  if constexpr (SIZE == 1) return static_cast<const uint8_t *>(p)[off];
-  else if constexpr (SIZE == 2) return static_cast<const uint16_t *>(p)[off];
-  else return static_cast<const uint32_t *>(p)[off];
-}
-template <int SIZE>
-__device__ inline void store_sized(void *p, int64_t off, uint32_t v) {
-  if constexpr (SIZE == 1) static_cast<uint8_t *>(p)[off] = uint8_t(v);
-  else if constexpr (SIZE == 2) static_cast<uint16_t *>(p)[off] = uint16_t(v);
-  else static_cast<uint32_t *>(p)[off] = v;
-}
-
-// The same conversions on an element already in a register (`raw`: its bits, zero-extended).
-__device__ inline float raw_to_f32(uint32_t raw, int dtype) {
-  switch (dtype) {
-    case MRL_U8: return float(raw & 0xffu);
-    case MRL_I8: return float(int8_t(uint8_t(raw)));
-    case MRL_U16: return float(raw & 0xffffu);
-    case MRL_I16: return float(int16_t(uint16_t(raw)));
-    case MRL_U32: return float(raw);
-    case MRL_I32: return float(int32_t(raw));
-    case MRL_F32: return __uint_as_float(raw);
-    default: return bf16_bits_to_f32(uint16_t(raw));
-  }
-}
-__device__ inline uint32_t convert_raw(uint32_t raw, int sdt, int ddt) {
-  if (sdt == ddt) return raw;
-  const bool src_float = sdt == MRL_F32 || sdt == MRL_BF16;
-  if (ddt == MRL_F32) return __float_as_uint(raw_to_f32(raw, sdt));
-  if (ddt == MRL_BF16) return f32_to_bf16_bits(raw_to_f32(raw, sdt));
-  if (src_float) return float_to_int(raw_to_f32(raw, sdt), ddt);
-  return narrow_int(sdt, raw);  // int -> int: extend by the source's sign, the store truncates
-}
-
-// Calls f(source dtype, destination dtype) with the two as compile-time constants
-// (std::integral_constant), chosen once by a switch over the dtypes of SE and of DE bytes: inside
-// f a conversion is the few instructions it needs, where a switch around every element costs more
-// than the conversion (u8 -> bf16 over 64 Mi elements: 60 us that way, 30 this way).
-template <int SE, int DE, class F>
-__device__ inline void with_dtypes(int sdt, int ddt, F &&f) {
-  // (u, i) of one and four bytes, (u, i, bf16) of two
-  constexpr int S0 = SE == 1 ? MRL_U8 : SE == 2 ? MRL_U16 : MRL_U32, S1 = S0 + 1, S2 = SE == 2 ? MRL_BF16 : MRL_F32;
-  constexpr int D0 = DE == 1 ? MRL_U8 : DE == 2 ? MRL_U16 : MRL_U32, D1 = D0 + 1, D2 = DE == 2 ? MRL_BF16 : MRL_F32;
-  const int si = sdt == S0 ? 0 : sdt == S1 ? 1 : 2, di = ddt == D0 ? 0 : ddt == D1 ? 1 : 2;
-#define MRL_CASE(A, B)                                                                   \
-  case A * 3 + B:                                                                        \
-    f(std::integral_constant<int, (A == 0 ? S0 : A == 1 ? S1 : S2)>{},                  \
-      std::integral_constant<int, (B == 0 ? D0 : B == 1 ? D1 : D2)>{});                 \
-    break;
-  switch (si * 3 + di) {
-    MRL_CASE(0, 0) MRL_CASE(0, 1) MRL_CASE(0, 2) MRL_CASE(1, 0) MRL_CASE(1, 1) MRL_CASE(1, 2)
-    MRL_CASE(2, 0) MRL_CASE(2, 1) MRL_CASE(2, 2)
-  }
-#undef MRL_CASE
-}
-
 // Move of a contiguous run with a dtype conversion: N elements per thread, one vector load
 // and one vector store (SE, DE: element sizes in bytes).  N = 4 where an element of four bytes is
 // involved, 8 or 16 between narrower ones, so that the wider side moves 16 bytes a thread (u8 ->
 // bf16 over 64 Mi elements: 68 us with four elements a thread).
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
-typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
 template <int SE, int DE, int N = 4>
 __global__ __launch_bounds__(256) void k_convert4(const void *__restrict__ src, void *__restrict__ dst, int sdt,
                                                   int ddt, uint64_t count) {
@@ -584,89 +490,6 @@ __global__ __launch_bounds__(256) void k_move_tiled32(MoveStrided p) {
   }
 }
 
-// A tile of a Move over a common strided view: `ext[d]` elements along each digit, as many tiles along
-// it as `chunks[d]`.  Element t of the tile in source order has digit (t / tstride_s[d]) % ext[d]
-// along d, likewise tstride_d in destination order; the divisions are multiplications by
-// precomputed reciprocals (exact for operands below 2^16).  The digits the tile extends along come
-// first.
-struct MoveTile {
-  const void *src;
-  void *dst;
-  int sdt, ddt;
-  uint32_t shape[MOVE_MAX_RANK];
-  int64_t ss[MOVE_MAX_RANK], ds[MOVE_MAX_RANK];
-  uint32_t ext[MOVE_MAX_RANK], chunks[MOVE_MAX_RANK];
-  uint32_t tstride_s[MOVE_MAX_RANK], tstride_d[MOVE_MAX_RANK];
-  uint32_t inv_s[MOVE_MAX_RANK], inv_d[MOVE_MAX_RANK], inv_ext[MOVE_MAX_RANK];  // ceil(2^32 / x)
-  uint32_t tile;  // elements (k_move_runs: vectors) per tile
-  FastDiv by_chunks[MOVE_MAX_RANK];   // a block number into tile coordinates without dividing (blocks number below 2^31)
-  uint32_t lds_step[4];  // k_move_gather: where the elements of a destination run of four lie in source order, from its first
-};
-constexpr uint32_t MOVE_TILE_MAX = 4096;
-
-__device__ inline uint32_t div_small(uint32_t n, uint32_t d, uint32_t inv) {
-  return d == 1 ? n : __umulhi(n, inv);
-}
-
-// Coordinates of this workgroup's tile: the offsets of its origin on the two sides, and how much of
-// each digit is left from there on.
-__device__ inline void tile_origin(const MoveTile &p, int64_t &base_s, int64_t &base_d, uint32_t (&room)[MOVE_MAX_RANK]) {
-  uint32_t blk = blockIdx.x;
-  base_s = base_d = 0;
-#pragma unroll
-  for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) {
-    const uint32_t rest = p.by_chunks[d].div(blk);
-    const uint32_t origin = (blk - rest * p.chunks[d]) * p.ext[d];
-    blk = rest;
-    room[d] = p.shape[d] - origin;
-    base_s += int64_t(origin) * p.ss[d], base_d += int64_t(origin) * p.ds[d];
-  }
-}
-
-// V elements of `size` bytes as zero-extended values <-> memory, one access of V * size bytes.
-template <int SIZE, int V>
-__device__ inline void load_run(const void *p, int64_t off, uint32_t (&raw)[V]) {
-  constexpr int BYTES = SIZE * V;
-  if constexpr (V == 1 || BYTES < 4) {
-#pragma unroll
-    for (int e = 0; e < V; e++) raw[e] = load_sized<SIZE>(p, off + e);
-  } else {
-    typedef uint32_t W __attribute__((ext_vector_type(BYTES / 4 == 1 ? 2 : BYTES / 4)));
-    const uint8_t *at = static_cast<const uint8_t *>(p) + off * SIZE;
-    uint32_t w[BYTES / 4];
-    if constexpr (BYTES == 4) w[0] = *reinterpret_cast<const uint32_t *>(at);
-    else {
-      const W v = *reinterpret_cast<const W *>(at);
-#pragma unroll
-      for (int i = 0; i < BYTES / 4; i++) w[i] = v[i];
-    }
-#pragma unroll
-    for (int e = 0; e < V; e++)
-      raw[e] = SIZE == 4 ? w[e] : (w[e * SIZE / 4] >> (8 * (e * SIZE % 4))) & (SIZE == 1 ? 0xffu : 0xffffu);
-  }
-}
-template <int SIZE, int V>
-__device__ inline void store_run(void *p, int64_t off, const uint32_t (&v)[V]) {
-  constexpr int BYTES = SIZE * V;
-  if constexpr (V == 1 || BYTES < 4) {
-#pragma unroll
-    for (int e = 0; e < V; e++) store_sized<SIZE>(p, off + e, v[e]);
-  } else {
-    uint32_t w[BYTES / 4];
-#pragma unroll
-    for (int i = 0; i < BYTES / 4; i++) w[i] = 0;
-#pragma unroll
-    for (int e = 0; e < V; e++) {
-      if constexpr (SIZE == 4) w[e] = v[e];
-      else w[e * SIZE / 4] |= (v[e] & (SIZE == 1 ? 0xffu : 0xffffu)) << (8 * (e * SIZE % 4));
-    }
-    uint8_t *at = static_cast<uint8_t *>(p) + off * SIZE;
-    if constexpr (BYTES == 4) MRL_STORE_ONCE(w[0], reinterpret_cast<uint32_t *>(at));
-    else if constexpr (BYTES == 8) MRL_STORE_ONCE((v2u{w[0], w[1]}), reinterpret_cast<v2u *>(at));
-    else MRL_STORE_ONCE((v4u_t{w[0], w[1], w[2], w[3]}), reinterpret_cast<v4u_t *>(at));
-  }
-}
-
 // Both sides contiguous along the same digit, in whole vectors of V elements (shape, strides and
 // extents count vectors; the wider side of a vector is 16, 8 or 4 bytes), converted or not.  Bound
 // by memory, so what matters is the order: a workgroup's tile is long along the digit that
@@ -724,73 +547,6 @@ __global__ __launch_bounds__(256) void k_move_runs(MoveStrided p) {
   store_run<DE, V>(p.dst, d_o * V, raw);
 }
 
-// Any other pair of contiguous digits (an OddEven digit on one side, a Packed digit of rows: too
-// short for the 64 x 64 transpose): a tile of up to 4096 elements, chosen on the host so that it
-// holds long runs on both sides, is read in source order, converted in registers, and written
-// in destination order out of LDS.  VS, VD: elements per access on the two sides, 4 or 2 where the
-// element's neighbours in the tile are its neighbours in memory, else 1.  The loads of a batch of
-// four accesses are in flight together, and their digits are worked out once per access, not per
-// element: that arithmetic is what bounds the kernel.  Runs of two: bf16 18 x 123556 transposed 8.0 us, element by element on
-// that side 11.7; f32 [16, 2, 5, 84558] to [0, 3, 2, 1] 23.3, 37.2.  NACT: digits that the tile extends along at most; f32
-// [1189, 5, 2, 4, 82] to [3, 4, 0, 2, 1, 3oe2], five of them, takes 26.1 us (16.4 with the runs of two) and 69.6 as any number.
-template <int SE, int DE, int VS, int VD, int NACT>
-__global__ __launch_bounds__(256) void k_move_gather(MoveTile p) {
-  __shared__ uint32_t lds[MOVE_TILE_MAX + MOVE_TILE_MAX / 32];
-  int64_t base_s, base_d;
-  uint32_t room[MOVE_MAX_RANK];
-  tile_origin(p, base_s, base_d, room);
-  auto cell = [](uint32_t t) { return t + t / 32; };
-  constexpr int BATCH = 4;
-  for (uint32_t t0 = 0; t0 < p.tile; t0 += 256 * VS * BATCH) {
-    uint32_t raw[BATCH][VS];
-#pragma unroll
-    for (int u = 0; u < BATCH; u++) {
-      const uint32_t t = t0 + (u * 256 + threadIdx.x) * VS;
-      uint32_t so = 0;
-      bool inside = t < p.tile;
-#pragma unroll
-      for (int d = 0; d < NACT; d++) {
-        const uint32_t q = div_small(t, p.tstride_s[d], p.inv_s[d]);
-        const uint32_t c = q - div_small(q, p.ext[d], p.inv_ext[d]) * p.ext[d];
-        inside = inside && c < room[d];
-        so += c * uint32_t(p.ss[d]);
-      }
-      load_run<SE, VS>(p.src, base_s + (inside ? so : 0u), raw[u]);
-    }
-    with_dtypes<SE, DE>(p.sdt, p.ddt, [&](auto sd, auto dd) {
-#pragma unroll
-      for (int u = 0; u < BATCH; u++)
-#pragma unroll
-        for (int e = 0; e < VS; e++) raw[u][e] = convert_raw(raw[u][e], decltype(sd)::value, decltype(dd)::value);
-    });
-#pragma unroll
-    for (int u = 0; u < BATCH; u++) {
-      const uint32_t t = t0 + (u * 256 + threadIdx.x) * VS;
-      if (t < p.tile) {
-#pragma unroll
-        for (int e = 0; e < VS; e++) lds[cell(t) + e] = raw[u][e];  // a run of four never crosses a multiple of 32
-      }
-    }
-  }
-  __syncthreads();
-#pragma unroll 4
-  for (uint32_t t = threadIdx.x * VD; t < p.tile; t += 256 * VD) {
-    uint32_t d_o = 0, at = 0;
-    bool inside = true;
-#pragma unroll
-    for (int d = 0; d < NACT; d++) {
-      const uint32_t q = div_small(t, p.tstride_d[d], p.inv_d[d]);
-      const uint32_t c = q - div_small(q, p.ext[d], p.inv_ext[d]) * p.ext[d];
-      inside = inside && c < room[d];
-      d_o += c * uint32_t(p.ds[d]);
-      at += c * p.tstride_s[d];
-    }
-    uint32_t v[VD];
-#pragma unroll
-    for (int e = 0; e < VD; e++) v[e] = lds[cell(at + (VD == 1 ? 0 : p.lds_step[e]))];
-    if (inside) store_run<DE, VD>(p.dst, base_d + d_o, v);
-  }
-}
 // Without a tile, an element a thread in destination order: small tensors, as above.
 template <int SE, int DE>
 __global__ __launch_bounds__(256) void k_move_gather(MoveStrided p) {
@@ -1293,7 +1049,7 @@ constexpr uint64_t MOVE_TINY = 65536;
 // (6.5 / 10.8); [45, 1963, 4] to [45, 4, 1963] f32 5.8 / 4.3, bf16 5.0 / 3.3.  Between 1 and 2 Mi it is either, by layout.
 constexpr uint64_t MOVE_SMALL = 1u << 20;
 // Whole 16-byte vectors in runs of 64 bytes or more, nothing converted: either side then reads and writes half a cache
-// line at least in any order, and tiles pay later (4 to 8 MB 5.8 / 3.8 us, 8 to 16 MB 5.4 / 4.5, 32 to 64 MB 15.4 / 17.7).
+// line at least in any order, and tiles pay later (4 to 8 MB 5.8 / 3.8 us, 8 to 16 MB 5.4 / 4.5, 16 to 32 MB 7.6 / 7.2 but up to 25 % either way, 32 to 64 MB 15.4 / 17.7).
 constexpr uint64_t MOVE_DIRECT_BYTES = 16u << 20;
 
 // A MoveTile's per-digit arrays from a view and the tile's extents.  `first`: digits in the order a
@@ -1668,32 +1424,9 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
   fill_tile(&t, p, ext, tstride_s, tstride_d, nullptr, &n_act, &blocks);
   t.tile = tile;
   if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-  const dim3 grid{uint32_t(blocks)};
-#define MRL_GATHER_V(SE, DE, VS, VD)                                                                                 \
-  do {                                                                                                               \
-    if (n_act <= 4) MRL_LAUNCH((k_move_gather<SE, DE, VS, VD, 4>), grid, dim3(256), 0, stream, t);                   \
-    else if (n_act <= 5) MRL_LAUNCH((k_move_gather<SE, DE, VS, VD, 5>), grid, dim3(256), 0, stream, t);              \
-    else MRL_LAUNCH((k_move_gather<SE, DE, VS, VD, int(MOVE_MAX_RANK)>), grid, dim3(256), 0, stream, t);             \
-  } while (0)
-#define MRL_GATHER_S(SE, DE, VS)                            \
-  do {                                                      \
-    if (run_d == 4) MRL_GATHER_V(SE, DE, VS, 4);            \
-    else if (run_d == 2) MRL_GATHER_V(SE, DE, VS, (DE > 1 ? 2 : 1)); \
-    else MRL_GATHER_V(SE, DE, VS, 1);                       \
-  } while (0)
-#define MRL_GATHER(SE, DE)                                  \
-  if (se == SE && de == DE) {                               \
-    if (run_s == 4) MRL_GATHER_S(SE, DE, 4);                \
-    else if (run_s == 2) MRL_GATHER_S(SE, DE, (SE > 1 ? 2 : 1)); \
-    else MRL_GATHER_S(SE, DE, 1);                           \
-  }
-  MRL_GATHER(1, 1) MRL_GATHER(1, 2) MRL_GATHER(1, 4)
-  MRL_GATHER(2, 1) MRL_GATHER(2, 2) MRL_GATHER(2, 4)
-  MRL_GATHER(4, 1) MRL_GATHER(4, 2) MRL_GATHER(4, 4)
-#undef MRL_GATHER
-#undef MRL_GATHER_S
-#undef MRL_GATHER_V
-  return mrl::plan::last_error();
+  if (se == 1) return launch_move_gather<1>(t, uint32_t(de), run_s, run_d, n_act, uint32_t(blocks), stream);
+  if (se == 2) return launch_move_gather<2>(t, uint32_t(de), run_s, run_d, n_act, uint32_t(blocks), stream);
+  return launch_move_gather<4>(t, uint32_t(de), run_s, run_d, n_act, uint32_t(blocks), stream);
 }
 
 // Move between two strided layouts of the same logical shape.

@@ -1,0 +1,6 @@
+// k_move_gather from elements of 2 bytes.
+#include "move_gather.h"
+
+namespace mrl {
+template hipError_t launch_move_gather<2>(const MoveTile &, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, hipStream_t);
+}  // namespace mrl
