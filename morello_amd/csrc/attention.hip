@@ -33,19 +33,12 @@
 // barriers per block.
 #include <algorithm>
 
-#include "kernels.h"
+#include "attention.h"
 
 namespace mrl {
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v2i __attribute__((ext_vector_type(2)));
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) v4s lds_v4s;
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void global_cvoid;
+using namespace attn;
 
 constexpr int BKV = 64;       // keys per block
 // Sizes that follow from the head dim D (k and n of the Compose; 32, 64 or 128).
@@ -72,30 +65,6 @@ __device__ constexpr int kt_swizzle(int d) { return ((d >> 1) & 1) | (((d >> 3) 
 // Wave priorities of the two kinds of slot: the matrix slot is the longer one and its MFMAs
 // should not queue behind the partner wave's vector instructions (worth ~0.5 % at 16 x 2048 x 128).
 constexpr int PRIO_A = 2, PRIO_B = 0;
-constexpr float LOG2E = 1.44269504088896340736f;
-constexpr float STALE_REFERENCE = 1.0e12f;  // ~2^40: an exponential beyond it moves the reference
-
-// One direct-to-LDS load: 64 lanes x 16 bytes from `base + voff` (voff per lane) to the 1 KiB at
-// LDS address `lds_addr` (wave-uniform), lane l to slot l.  Written as assembly so that the
-// compiler does not know of it: it would otherwise make every later LDS read wait for all such
-// loads in flight (it cannot tell the stages apart), which serialises a block's softmax behind
-// the next block's fetch.  The waits that matter are the explicit ones before the barriers.
-__device__ inline void dma16(const uint8_t *base, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(base));
-}
-// The same through a buffer resource: an offset past its end brings zeros.
-__device__ inline void dma16(__amdgpu_buffer_rsrc_t from, uint32_t voff, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(from));
-}
-constexpr uint32_t OUTSIDE = 0x80000000u;   // an offset no resource here holds, whatever block's is added
-__device__ inline uint32_t lds_address(const void *p) {
-  return uint32_t(reinterpret_cast<uintptr_t>((lds_void *)p));
-}
-
-__device__ inline v2i read_tr16(const uint8_t *p) {
-  const v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)p);
-  return __builtin_bit_cast(v2i, r);
-}
 
 // RAGGED: m need not be a multiple of 128 nor n2 of 128.  Query rows past m are computed on
 // a clamped (valid) row and not stored; the key blocks are dealt ceil/floor to the two halves,
@@ -143,12 +112,8 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
   const int qg = wave % QG, half = wave / QG;  // query group, key half
   constexpr int BQ = 32 * QG;
   const int lr = lane & 15, lgp = lane >> 4;   // position within a block's 16 rows / columns, lane group
-  // Workgroups go to the 8 XCDs round-robin.  All query blocks of a batch entry share its K
-  // and V, so a batch entry's blocks are kept on one XCD (one L2) whenever the counts allow:
-  // XCD x takes the x-th run of consecutive (entry, block) pairs.
-  const uint32_t nqb = (p.m + BQ - 1) / BQ, total = nqb * p.b;
-  uint32_t lin = blockIdx.x;
-  if (total % 8 == 0) lin = (lin % 8) * (total / 8) + lin / 8;
+  const uint32_t nqb = (p.m + BQ - 1) / BQ;
+  const uint32_t lin = xcd_run(blockIdx.x, nqb * p.b);
   const int64_t head = lin / nqb;
   const int q0 = int(lin % nqb) * BQ + qg * 32;
   // Key blocks of this half: [first_block, first_block + nblocks); both halves run `steps`
@@ -243,7 +208,7 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
     for (int qb = 0; qb < 2; qb++)
 #pragma unroll
       for (int r = 0; r < 4; r++) o[db][qb][r] = 0.0f;
-  float m_run[2] = {-3.0e38f, -3.0e38f};
+  float m_run[2] = {NO_REFERENCE, NO_REFERENCE};
   // The denominators come out of the second product too: one more block row of V^T, all ones,
   // sums P over the keys (every register of every lane then holds its query's denominator: the
   // sum of the very values, rounded to bf16, that O is made of).
@@ -629,7 +594,9 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
 
 // out[row][0 .. n_out) = sum_s O_s * 2^((m_s - M) log2 e) / sum_s l_s * 2^((m_s - M) log2 e), M = max_s m_s:
 // the parts formula of morello/src/spec.rs:107-132 over the splits' triples.  One thread per
-// output element; a split that saw no key has l = 0 and the smallest m, so it drops out.
+// output element; a split that saw no key has l = 0 and the smallest m, so it drops out.  The launch is one trip to
+// memory: the triples of U splits are all requested before the first is looked at, and the sums are kept against a running maximum.
+template <uint32_t U>
 __global__ __launch_bounds__(256) void k_attn_merge(const float *__restrict__ partials, float *__restrict__ out,
                                                     uint64_t rows, uint32_t splits, uint32_t d, uint32_t n_out) {
   const uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
@@ -638,50 +605,42 @@ __global__ __launch_bounds__(256) void k_attn_merge(const float *__restrict__ pa
   const uint32_t col = uint32_t(i % n_out);
   const float *part = partials + row * splits * (d + 4);
   const uint32_t stride = d + 4;
-  // Eight splits' loads in flight at a time: the loop is all latency otherwise (35 splits one
-  // after another took 20 us).
-  constexpr uint32_t U = 8;
-  float m = -3.0e38f;
-  for (uint32_t s0 = 0; s0 < splits; s0 += U) {
-    float ms[U];
-#pragma unroll
-    for (uint32_t u = 0; u < U; u++) {
-      const float v = part[(s0 + u < splits ? s0 + u : 0) * stride + d];  // always a valid address
-      ms[u] = s0 + u < splits ? v : -3.0e38f;
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < U; u++) m = fmaxf(m, ms[u]);
-  }
-  float num = 0.0f, den = 0.0f;
+  float m = -3.0e38f, num = 0.0f, den = 0.0f;
   for (uint32_t s0 = 0; s0 < splits; s0 += U) {
     float ms[U], ls[U], os[U];
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) {
-      const bool in = s0 + u < splits;
-      const float *p = part + (in ? s0 + u : 0) * stride;
-      const float mv = p[d], lv = p[d + 1], ov = p[col];
-      ms[u] = in ? mv : -3.0e38f, ls[u] = in ? lv : 0.0f, os[u] = in ? ov : 0.0f;
+      const float *p = part + (s0 + u < splits ? s0 + u : 0) * stride;  // always a valid address
+      ms[u] = p[d], ls[u] = p[d + 1], os[u] = p[col];
     }
+    float m_new = m;
 #pragma unroll
-    for (uint32_t u = 0; u < U; u++) {
-      const float w = __builtin_amdgcn_exp2f((ms[u] - m) * LOG2E);
-      num += os[u] * w;
-      den += ls[u] * w;
-    }
+    for (uint32_t u = 0; u < U; u++)
+      if (s0 + u < splits) m_new = fmaxf(m_new, ms[u]);
+    const float old = __builtin_amdgcn_exp2f((m - m_new) * LOG2E);
+    num *= old, den *= old, m = m_new;
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++)
+      if (s0 + u < splits) {
+        const float w = __builtin_amdgcn_exp2f((ms[u] - m) * LOG2E);
+        num += os[u] * w;
+        den += ls[u] * w;
+      }
   }
   out[row * n_out + col] = num / den;
 }
 
 }  // namespace
 
-// Key splits for a launch: 1 unless the (entry, query block) pairs fill at most half of the
+uint32_t g_compute_units = 256;   // set by mrl_init: planning makes no runtime call
+
+namespace {
+// Key splits of the form of 64 or 128 queries: 1 unless the (entry, query block) pairs fill at most half of the
 // compute units and there are keys enough to share out (four blocks of 64 per workgroup at
 // least, and more time saved than the partial results cost).  The workgroups then number at most one per compute unit: measured on 256 units, 256
 // workgroups stream K and V at 4.9-5.6 TB/s where 320 or 512 reach 3.6-4.8.
-uint32_t g_compute_units = 256;
-
-uint32_t attn_key_splits(const AttnArgs &a) {
-  const uint64_t units = g_compute_units;  // set by mrl_init: planning makes no runtime call
+uint32_t key_splits_of_blocks(const AttnArgs &a) {
+  const uint64_t units = g_compute_units;
   const uint64_t bq = a.query_block, groups = uint64_t((a.m + bq - 1) / bq) * a.b, blocks = (a.n2 + BKV - 1) / BKV;
   if (groups == 0) return 1;
   const uint64_t splits = std::min<uint64_t>({units / groups, blocks / 4, 256});
@@ -689,6 +648,95 @@ uint32_t attn_key_splits(const AttnArgs &a) {
   if (splits < 2 || blocks * (splits - 1) <= 8 * splits) return 1;
   return uint32_t(splits);
 }
+
+// Queries per workgroup of that form (tile_out over the Compose's rows): 64 where 128 would leave half of
+// the compute units or more without a workgroup, or pad a query dimension of 64 or less.
+// Unless the keys are many enough to share out instead: 128 queries with the keys in as many
+// parts as fill the chip measured faster once a part holds 4096 keys, or 1024 with at most a
+// quarter of the units taken (2 x 8192 x 8192 keys: 68.8 us against 77.1, 1 x 8192 x 8192 39.9
+// against 49.7, 2 x 4096 x 4096 30.6 against 34.1; 4 x 4096 x 4096 the other way, 47.2 against 42.8).
+uint32_t query_block_of(const AttnArgs &a) {
+  const uint64_t groups128 = uint64_t(a.b) * ((a.m + 127) / 128), units = g_compute_units;
+  bool few_groups = 2 * groups128 <= units;
+  if (few_groups && a.m > 64) {
+    const uint64_t parts = std::min<uint64_t>(units / groups128, ((a.n2 + 63) / 64) / 4);
+    const uint64_t keys = parts >= 2 ? a.n2 / parts : 0;
+    if (keys >= 4096 || (4 * groups128 <= units && keys >= 1024)) few_groups = false;
+  }
+  return (a.m <= 64 || few_groups) && a.m > 32 ? 64 : 128;
+}
+
+// Key splits of the form that deals keys to waves, `groups` workgroups without them: the cheapest by
+//   rounds of a workgroup's eight blocks of 32 keys, each 0.9 us at head dim 128 (131 KB a round), 0.35 at 64;
+//   K and V at what the workgroups stream together: each 140 bytes a nanosecond from L2, 100 from the memory-side cache, 42 from memory, 6500 at most;
+//   2.7 us for the merging launch and 0.02 a split that it reads.
+// (1 x 1 x 128 against 5536 keys: 1 split 22.7 us, 5 9.7, 10 7.9, 21 8.0; 16 x 1 against 32768 keys that no cache holds: 8 splits
+// 53.2, 16 50.8, 32 52.8; 20 x 1 x 64 against 872: 1 split 4.6, 3 6.9.)
+uint32_t key_splits_of_waves(const AttnArgs &a, uint64_t groups) {
+  const uint64_t blocks = (a.n2 + 31) / 32, most = std::min<uint64_t>(g_compute_units / groups, blocks / 8);
+  const double bytes = 4.0 * a.b * a.n2 * a.k, round_ns = a.k == 128 ? 900 : a.k == 64 ? 350 : 250,
+               share = bytes > 64e6 ? 42 : bytes > 16e6 ? 100 : 140;
+  auto ns = [&](uint64_t s) {
+    const uint64_t rounds = ((blocks + s - 1) / s + 7) / 8;
+    return std::max(double(rounds) * round_ns, bytes / std::min(double(groups * s) * share, 6500.0)) + (s > 1 ? 2700.0 + 20.0 * double(s) : 0.0);
+  };
+  uint64_t best = 1;
+  double least = ns(1);
+  auto consider = [&](uint64_t s) {
+    if (s < 2 || s > most) return;
+    const double t = ns(s);
+    if (t < least) best = s, least = t;
+  };
+  consider(most);
+  for (uint64_t rounds = 1; rounds <= 8; rounds++) consider((blocks + 8 * rounds - 1) / (8 * rounds));
+  return uint32_t(best);
+}
+
+// The form that deals keys to waves, where it is the faster one: always for up to 16 queries an entry; for more
+// while a round of workgroups holds them all (one of D = 128 to a compute unit, two of 64 or 32), of 16 queries or else of 32, and the
+// keys are not so many that the other form's larger share of queries per key read counts for more.  Measured
+// (us, this form / the other): 4 x 1 x 128 against 564 keys 5.4 / 10.1; 16 x 103 x 80 against 767 6.7 / 11.9; 40 x 90 x 128
+// against 1024 8.1 / 15.4; 13 x 346 x 80 against 1088 (32 queries) 9.6 / 15.4; 18 x 329 x 32 against 1810 6.4 / 12.8;
+// beyond: 47 x 192 x 128 against 1856 28.9 / 22.5, 16 x 2048 x 2048 58.9 / 33.8, 2 x 2048 against 4096 keys 21.2 / 22.4, 8192 31.7 / 26.8.
+bool by_waves(AttnArgs &a) {
+  if (a.kt_rows || a.m == 0 || a.b == 0) return false;
+  const uint64_t units = g_compute_units, room = a.k == 128 ? units : 2 * units;
+  const uint64_t g16 = uint64_t(a.b) * ((a.m + 15) / 16), g32 = uint64_t(a.b) * ((a.m + 31) / 32);
+  const uint64_t longest = a.k == 128 ? 2048 : 4096;
+  a.query_block = 16, a.waves = 8, a.key_splits = 1;
+  if (a.m <= 16) {
+    if (g16 < units) a.key_splits = key_splits_of_waves(a, g16);
+    return true;
+  }
+  if (g16 <= room && a.n2 <= longest) {
+    // (more than 16 queries share what a split streams, and its partial results are as many rows: only where less than half of the chip is at work)
+    if (2 * g16 <= units) a.key_splits = key_splits_of_waves(a, g16);
+    return true;
+  }
+  if (4 * g16 <= units && g16 * a.n2 <= 200 * longest) {   // longer ones in splits: 8 x 32 x 128 against 8192 keys 9.8 / 13.9, 2 x 512 against 4096 11.6 / 14.1, 8192 16.1 / 14.9
+    a.key_splits = key_splits_of_waves(a, g16);
+    return true;
+  }
+  // Up to 128 keys leave four of eight waves without a block: workgroups of four, two to a unit (8 x 640 x 128 against 68: 4.9 us, of eight 6.7, the other form 6.5).
+  if (a.k == 128 && g16 <= 2 * units && a.n2 <= 128) {
+    a.waves = 4;
+    return true;
+  }
+  a.query_block = 32;
+  if (a.n2 <= 2048 && (g32 <= units || (g32 <= room && a.n2 >= 384))) return true;
+  return false;
+}
+}  // namespace
+
+void attn_choose(AttnArgs &a) {
+  if (!a.query_block && !a.key_splits) {
+    if (by_waves(a)) return;
+    a.query_block = 0, a.key_splits = 0;
+  }
+  if (!a.query_block) a.query_block = query_block_of(a);
+  if (!a.key_splits) a.key_splits = key_splits_of_blocks(a);
+}
+
 size_t attn_partial_bytes(const AttnArgs &a, uint32_t splits) {
   return splits > 1 ? size_t(a.b) * a.m * splits * (a.k + 4) * sizeof(float) : 0;
 }
@@ -697,7 +745,7 @@ bool attn_applicable(const AttnArgs &a) {
   auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   return a.k == a.n && (a.k == 32 || a.k == 64 || a.k == 128) && a.n_out >= 1 && a.n_out <= a.n && a.m && a.n2 && a.b &&
          (!a.kt_rows || a.n2 % 8 == 0) && (a.k_in == 0 || (!a.kt_rows && a.k > 32 && a.k_in <= a.k && a.k_in % 8 == 0 && a.n_out % 8 == 0)) && (a.key_splits <= 1 || (a.partials && a.key_splits <= 65535)) &&
-         uint64_t(a.n2) * a.k * 2 < (1ull << 31) && (a.query_block == 64 || a.query_block == 128) &&
+         uint64_t(a.n2) * a.k * 2 < (1ull << 31) && (a.query_block == 64 || a.query_block == 128 || (!a.kt_rows && (a.query_block == 16 || a.query_block == 32))) &&
          uint64_t((a.m + a.query_block - 1) / a.query_block) * a.b < (1u << 31) &&
          al16(a.q) && al16(a.kt) && al16(a.v) && al16(a.out);
 }
@@ -723,12 +771,6 @@ hipError_t launch_one(const AttnArgs &a, hipStream_t stream) {
              3000.0);
   MRL_LAUNCH((k_attn<D, RAGGED, KT_ROWS, QG, NARROW>), grid, dim3(128 * QG), LDS, stream, a.q, a.kt, a.v, a.out, a.b, a.m, a.n2, a.n_out,
              a.key_splits, a.partials, a.k_in);
-  if (a.key_splits > 1) {
-    const uint64_t rows = uint64_t(a.b) * a.m, total = rows * a.n_out;
-    plan::work(plan::UNIT_STREAM, 0, double(attn_partial_bytes(a, a.key_splits)) + 4.0 * total);
-    MRL_LAUNCH(k_attn_merge, dim3(uint32_t((total + 255) / 256)), dim3(256), 0, stream, a.partials, a.out, rows,
-                       a.key_splits, uint32_t(D), a.n_out);
-  }
   return mrl::plan::last_error();
 }
 
@@ -742,8 +784,19 @@ hipError_t launch_for(const AttnArgs &a, hipStream_t stream) {
 }
 }  // namespace
 
-hipError_t launch_attn(const AttnArgs &a, hipStream_t stream) {
-  if (!attn_applicable(a)) return hipErrorInvalidValue;
+hipError_t launch_attn_merge(const AttnArgs &a, hipStream_t stream) {
+  const uint64_t rows = uint64_t(a.b) * a.m, total = rows * a.n_out;
+  plan::work(plan::UNIT_STREAM, 0, double(attn_partial_bytes(a, a.key_splits)) + 4.0 * total);
+  const dim3 grid(uint32_t((total + 255) / 256)), block(256);
+  if (a.key_splits <= 4) MRL_LAUNCH(k_attn_merge<4>, grid, block, 0, stream, a.partials, a.out, rows, a.key_splits, a.k, a.n_out);
+  else if (a.key_splits <= 8) MRL_LAUNCH(k_attn_merge<8>, grid, block, 0, stream, a.partials, a.out, rows, a.key_splits, a.k, a.n_out);
+  else MRL_LAUNCH(k_attn_merge<16>, grid, block, 0, stream, a.partials, a.out, rows, a.key_splits, a.k, a.n_out);
+  return plan::last_error();
+}
+
+namespace {
+hipError_t launch_products(const AttnArgs &a, hipStream_t stream) {
+  if (a.query_block < 64) return launch_attn_keys(a, stream);
   if (a.query_block == 64) {
     switch (a.k) {
       case 32: return launch_for<32, 2>(a, stream);
@@ -756,6 +809,13 @@ hipError_t launch_attn(const AttnArgs &a, hipStream_t stream) {
     case 64: return launch_for<64, 4>(a, stream);
     default: return launch_for<128, 4>(a, stream);
   }
+}
+}  // namespace
+
+hipError_t launch_attn(const AttnArgs &a, hipStream_t stream) {
+  if (!attn_applicable(a)) return hipErrorInvalidValue;
+  const hipError_t e = launch_products(a, stream);
+  return e != hipSuccess || a.key_splits <= 1 ? e : launch_attn_merge(a, stream);
 }
 
 }  // namespace mrl

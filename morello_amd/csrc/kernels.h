@@ -293,16 +293,19 @@ struct AttnArgs {
   // are taken as, zeros behind them).
   uint32_t k_in = 0;
   bool kt_rows = false;  // KT stored row-major, n2 fastest (n2 a multiple of 8)
-  // Queries per workgroup: 128 (eight waves) or 64 (four).
-  uint32_t query_block = 128;
+  // Queries per workgroup: 128 (eight waves) or 64 (four); 16 or 32: the form that deals the keys to the waves.
+  uint32_t query_block = 0;
+  uint32_t waves = 8;    // that form's waves per workgroup, 4 or 8
   // More than 1: the keys are shared out over that many workgroups per query block and the
   // partial results merged afterwards; `partials` holds attn_partial_bytes() of scratch.
-  uint32_t key_splits = 1;
+  uint32_t key_splits = 0;
   float *partials = nullptr;
 };
-uint32_t attn_key_splits(const AttnArgs &a);
+void attn_choose(AttnArgs &a);   // sets query_block, waves and key_splits where they are 0
 size_t attn_partial_bytes(const AttnArgs &a, uint32_t splits);
 bool attn_applicable(const AttnArgs &a);
 hipError_t launch_attn(const AttnArgs &a, hipStream_t stream);
+hipError_t launch_attn_keys(const AttnArgs &a, hipStream_t stream);   // attention_keys.hip
+hipError_t launch_attn_merge(const AttnArgs &a, hipStream_t stream);
 
 }  // namespace mrl

@@ -1,0 +1,81 @@
+"""The fused Matmul -> Softmax -> Matmul that deals the keys to a workgroup's waves (k_attn with W = 8 or 4), at the edges of
+its blocks: 16 or 32 queries, blocks of 32 keys, eight or four waves, key shares, head dims read in place."""
+import numpy as np
+import pytest
+
+import morello_amd as M
+from gpu_util import run_spec
+from morello_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+KT = M.layout(0, 2, 1)
+
+
+def _f64(bits):
+    return synth.bf16_bits_to_f32(bits).astype(np.float64)
+
+
+def _run(b, m, keys, d, seed=190, std=0.5, change=None):
+    v, q, k = (synth.normal_bf16(seed, i, s, std) for i, s in enumerate([(b, keys, d), (b, m, d), (b, keys, d)]))
+    if change:
+        change(v, q, k)
+    spec = M.ComposeMSM(b, m, d, keys, d, layouts=[None, None, KT, None])
+    got = run_spec(spec, [v, q, k, np.full((b, m, d), 7, np.float32)]).astype(np.float64)
+    s = _f64(q) @ _f64(k).transpose(0, 2, 1)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    return spec.plan(), got, p / p.sum(-1, keepdims=True) @ _f64(v)
+
+
+def _close(got, want):
+    # P is rounded to bf16 (2^-9 of each) and summed in f32: 4e-3 in the norm at most
+    assert np.linalg.norm(got - want) <= 4e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("d", [32, 64, 80, 128])
+@pytest.mark.parametrize("m", [1, 2, 15, 16, 17, 33])
+@pytest.mark.parametrize("keys", [1, 31, 32, 33, 255, 256, 257, 290, 1000])
+def test_block_edges(gpu, d, m, keys):
+    plan, got, want = _run(3, m, keys, d)
+    assert "QB = 1, W = 8" in plan.steps[0].kernel and plan.kernels == ["k_attn"]
+    _close(got, want)
+
+
+@pytest.mark.parametrize("b,m,keys,d", [(1, 1, 5000, 128), (2, 8, 9001, 64), (2, 16, 7777, 128), (5, 40, 4100, 64), (1, 3, 40000, 32), (7, 1, 6000, 72)])
+def test_key_shares(gpu, b, m, keys, d):
+    plan, got, want = _run(b, m, keys, d)
+    assert "W = 8" in plan.steps[0].kernel and plan.kernels == ["k_attn", "k_attn_merge"]
+    _close(got, want)
+
+
+@pytest.mark.parametrize("b,m,keys,d,form", [
+    (11, 400, 65, 128, "QB = 1, W = 4"), (11, 401, 128, 96, "QB = 1, W = 4"), (23, 345, 1, 128, "QB = 1, W = 4"),
+    (9, 620, 300, 128, "QB = 2, W = 8"), (9, 625, 129, 128, "QB = 2, W = 8"), (17, 950, 400, 64, "QB = 2, W = 8"), (17, 950, 385, 48, "QB = 2, W = 8"),
+    (300, 5, 40, 64, "QB = 1, W = 8"), (30, 250, 97, 32, "QB = 1, W = 8")])
+def test_other_widths(gpu, b, m, keys, d, form):
+    plan, got, want = _run(b, m, keys, d)
+    assert form in plan.steps[0].kernel and plan.kernels == ["k_attn"]
+    _close(got, want)
+
+
+@pytest.mark.parametrize("m", [1, 20])
+def test_scores_that_outgrow_the_reference(gpu, m):
+    """Scores rising by about 100 along the keys and back: every wave moves its reference several times, and whole waves drop out."""
+    def change(v, q, k):
+        q[:, :, 0] = 0x3f80                                               # 1
+        ramp = (np.abs((np.arange(3000) // 150) % 10 - 5) * 40.0).astype(np.float32)
+        k[:, :, 0] = (ramp.view(np.uint32) >> 16).astype(np.uint16)
+    _, got, want = _run(2, m, 3000, 64, change=change)
+    assert np.isfinite(got).all()
+    _close(got, want)
+
+
+def test_keys_of_minus_infinity(gpu):
+    def change(v, q, k):
+        q[:, :, 0] = 0x3f80
+        k[:, 3::5, 0] = 0xff80                                            # -inf: these keys drop out
+        k[:, :40, 0] = 0xff80
+        k[:, :, 1:] = np.where((k[:, :, 1:] & 0x7f80) == 0x7f80, 0, k[:, :, 1:])
+    _, got, want = _run(2, 4, 700, 128, change=change)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    _close(got, want)
