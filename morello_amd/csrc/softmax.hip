@@ -33,101 +33,83 @@ __device__ inline uint32_t bf16_bits(float f) {
   return (bits + 0x7fffu + ((bits >> 16) & 1u)) >> 16;
 }
 
-// NV float4 vectors per lane; cols is a multiple of 4 and <= NV * 256.  OUT_BF16: the result is
-// written as bf16 (the left operand of the product that follows a Softmax in a Compose whose
-// inputs are bf16).
-template <int NV, bool OUT_BF16>
-__global__ __launch_bounds__(256) void k_softmax_regs(const float *__restrict__ in,
-                                                      void *__restrict__ out_any, uint64_t rows,
-                                                      uint32_t cols) {
-  float *out = static_cast<float *>(out_any);
-  const uint64_t row = uint64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const uint32_t lane = threadIdx.x & 63;
-  const float4 *src = (const float4 *)(in + row * cols);
-  float4 *dst = (float4 *)(out + row * cols);
-  const uint32_t nvec = cols / 4;
-  float4 v[NV];
-  float mx = F32_MIN;
-  bool nan = false;
-#pragma unroll
-  for (int i = 0; i < NV; i++) {
-    const uint32_t idx = i * 64 + lane;
-    if (idx < nvec) {
-      const f4 t = MRL_LOAD_ONCE((const f4 *)src + idx);
-      v[i] = float4{t[0], t[1], t[2], t[3]};
-      nan |= (v[i].x != v[i].x) | (v[i].y != v[i].y) | (v[i].z != v[i].z) | (v[i].w != v[i].w);
-      mx = fmaxf(fmaxf(mx, fmaxf(v[i].x, v[i].y)), fmaxf(v[i].z, v[i].w));
-    }
-  }
-  mx = wave_max(mx);
-  if (__any(nan)) mx = __uint_as_float(0x7fc00000u);
-  float sum = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NV; i++) {
-    const uint32_t idx = i * 64 + lane;
-    if (idx < nvec) {
-      v[i].x = expf(v[i].x - mx);
-      v[i].y = expf(v[i].y - mx);
-      v[i].z = expf(v[i].z - mx);
-      v[i].w = expf(v[i].w - mx);
-      sum += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-    }
-  }
-  sum = wave_sum(sum);
-#pragma unroll
-  for (int i = 0; i < NV; i++) {
-    const uint32_t idx = i * 64 + lane;
-    if (idx < nvec) {
-      v[i].x /= sum, v[i].y /= sum, v[i].z /= sum, v[i].w /= sum;
-      if constexpr (OUT_BF16) {
-        typedef unsigned u2 __attribute__((ext_vector_type(2)));
-        u2 *dst16 = reinterpret_cast<u2 *>(static_cast<uint16_t *>(out_any) + row * cols);
-        __builtin_nontemporal_store(u2{bf16_bits(v[i].x) | (bf16_bits(v[i].y) << 16), bf16_bits(v[i].z) | (bf16_bits(v[i].w) << 16)},
-                                    dst16 + idx);
-      } else {
-        __builtin_nontemporal_store(f4{v[i].x, v[i].y, v[i].z, v[i].w}, (f4 *)dst + idx);
-      }
-    }
+// Vectors of rows that start on any element: a load or store of 16 (8) bytes at the elements' own alignment, which global
+// memory takes.
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned u2 __attribute__((ext_vector_type(2)));
+typedef unsigned u2_any __attribute__((ext_vector_type(2), aligned(2)));
+template <bool ODD>
+__device__ inline f4 load_quad(const float *row, uint32_t idx) {
+  if constexpr (ODD) return MRL_LOAD_ONCE((const f4_any *)row + idx);
+  else return MRL_LOAD_ONCE((const f4 *)row + idx);
+}
+template <bool ODD, bool OUT_BF16>
+__device__ inline void store_quad(f4 y, void *out, uint64_t row_start, uint32_t idx) {
+  if constexpr (OUT_BF16) {
+    const u2 bits = {bf16_bits(y[0]) | (bf16_bits(y[1]) << 16), bf16_bits(y[2]) | (bf16_bits(y[3]) << 16)};
+    uint16_t *to = static_cast<uint16_t *>(out) + row_start;
+    if constexpr (ODD) MRL_STORE_ONCE(bits, (u2_any *)to + idx);
+    else MRL_STORE_ONCE(bits, (u2 *)to + idx);
+  } else {
+    float *to = static_cast<float *>(out) + row_start;
+    if constexpr (ODD) MRL_STORE_ONCE(y, (f4_any *)to + idx);
+    else MRL_STORE_ONCE(y, (f4 *)to + idx);
   }
 }
+template <bool OUT_BF16>
+__device__ inline void store_one(float y, void *out, uint64_t at) {
+  if constexpr (OUT_BF16) static_cast<uint16_t *>(out)[at] = uint16_t(bf16_bits(y));
+  else MRL_STORE_ONCE(y, static_cast<float *>(out) + at);
+}
 
-// The same for rows that are not whole 16-byte vectors (cols not a multiple of 4, so rows start
-// on any 4 bytes): NE scalars per lane, element i * 64 + lane, cols <= NE * 64.
-template <int NE, bool OUT_BF16>
-__global__ __launch_bounds__(256) void k_softmax_regs1(const float *__restrict__ in, void *__restrict__ out_any,
-                                                       uint64_t rows, uint32_t cols) {
+// NV float4 vectors per lane; cols <= NV * 256, a multiple of 4 unless ODD: then the last one to three elements of a row
+// go to the first lanes, one each.  OUT_BF16: the result is
+// written as bf16 (the left operand of the product that follows a Softmax in a Compose whose
+// inputs are bf16).
+template <int NV, bool ODD, bool OUT_BF16>
+__global__ __launch_bounds__(256) void k_softmax_regs(const float *__restrict__ in, void *__restrict__ out, uint64_t rows, uint32_t cols) {
   const uint64_t row = uint64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const uint32_t lane = threadIdx.x & 63;
   const float *src = in + row * cols;
-  float v[NE];
+  const uint32_t nvec = cols / 4, last = nvec * 4 + lane;   // `last`: this lane's element behind the vectors
+  // All of a lane's loads go out before the first is looked at, without a branch around any: a vector past the row's end is
+  // the last one again.  (With `if (idx < nvec)` around each the compiler waits for every load before the next.)  What bounds
+  // the kernel is memory; 16 x 1501 rows, buffers taking turns, us before -> now: 1501 columns 54.6 -> 52.2 (5.5 TB/s; a plain
+  // copy runs at 5.9), 1500 54.4 -> 52.2, 2000 71.9 -> 67.0; 9 x 711 x 2157 31.3 -> 20.6, 64 x 1000 x 257 38.5 -> 23.8.
+  f4 v[NV];
+  float tail = F32_MIN;
   float mx = F32_MIN;
   bool nan = false;
 #pragma unroll
-  for (int i = 0; i < NE; i++) {
-    const uint32_t e = i * 64 + lane;
-    v[i] = e < cols ? MRL_LOAD_ONCE(src + e) : F32_MIN;
-    nan |= v[i] != v[i];
-    mx = fmaxf(mx, v[i]);
+  for (int i = 0; i < NV; i++) v[i] = load_quad<ODD>(src, min(uint32_t(i * 64 + lane), nvec - 1));
+  if (ODD && last < cols) tail = MRL_LOAD_ONCE(src + last);
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    nan |= (v[i][0] != v[i][0]) | (v[i][1] != v[i][1]) | (v[i][2] != v[i][2]) | (v[i][3] != v[i][3]);
+    mx = fmaxf(fmaxf(mx, fmaxf(v[i][0], v[i][1])), fmaxf(v[i][2], v[i][3]));
   }
+  if (ODD) nan |= tail != tail, mx = fmaxf(mx, tail);
   mx = wave_max(mx);
   if (__any(nan)) mx = __uint_as_float(0x7fc00000u);
   float sum = 0.0f;
 #pragma unroll
-  for (int i = 0; i < NE; i++) {
-    v[i] = expf(v[i] - mx);
-    sum += uint32_t(i * 64) + lane < cols ? v[i] : 0.0f;
+  for (int i = 0; i < NV; i++) {
+    const uint32_t idx = i * 64 + lane;
+    if (idx < nvec) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) v[i][j] = expf(v[i][j] - mx);
+      sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+    }
   }
+  if (ODD && last < cols) tail = expf(tail - mx), sum += tail;
   sum = wave_sum(sum);
 #pragma unroll
-  for (int i = 0; i < NE; i++) {
-    const uint32_t e = i * 64 + lane;
-    if (e >= cols) continue;
-    const float y = v[i] / sum;
-    if constexpr (OUT_BF16) (static_cast<uint16_t *>(out_any) + row * cols)[e] = uint16_t(bf16_bits(y));
-    else __builtin_nontemporal_store(y, static_cast<float *>(out_any) + row * cols + e);
+  for (int i = 0; i < NV; i++) {
+    const uint32_t idx = i * 64 + lane;
+    if (idx < nvec) store_quad<ODD, OUT_BF16>(v[i] / sum, out, row * cols, idx);
   }
+  if (ODD && last < cols) store_one<OUT_BF16>(tail / sum, out, row * cols + last);
 }
 
 // Rows of up to 256 elements: L lanes per row (a power of two, 64 / L rows per wavefront), up to
@@ -308,30 +290,31 @@ __global__ __launch_bounds__(256) void k_softmax_chunk_write(const float *__rest
   }
 }
 
-// Rows of 4096 < cols <= NV * 1024 (cols a multiple of 4) when there are rows enough to fill
-// the chip with a workgroup each: the row stays in the workgroup's registers between the passes,
-// as in k_softmax_regs, so it is read once.
-template <int NV, bool OUT_BF16>
-__global__ __launch_bounds__(256) void k_softmax_block(const float *__restrict__ in, void *__restrict__ out_any,
-                                                       uint32_t cols) {
+// A workgroup per row of up to NV * 1024 elements: rows of more than 4096 when there are rows enough to fill the chip with a
+// workgroup each, shorter ones when there are too few for a wavefront each.  The row stays in the workgroup's registers
+// between the passes, as in k_softmax_regs, so it is read once.
+template <int NV, bool ODD, bool OUT_BF16>
+__global__ __launch_bounds__(256) void k_softmax_block(const float *__restrict__ in, void *__restrict__ out, uint32_t cols) {
   __shared__ float lds[2][4];
   const uint64_t row = blockIdx.x;
-  const uint32_t nvec = cols / 4, w = threadIdx.x >> 6;
-  const f4 *src = (const f4 *)(in + row * cols);
+  const uint32_t nvec = cols / 4, w = threadIdx.x >> 6, last = nvec * 4 + threadIdx.x;
+  const float *src = in + row * cols;
   f4 v[NV];
+  float tail = F32_MIN;
   float mx = F32_MIN;
   bool nan = false;
 #pragma unroll
+  for (int i = 0; i < NV; i++) v[i] = load_quad<ODD>(src, min(uint32_t(i * 256 + threadIdx.x), nvec - 1));
+  if (ODD && last < cols) tail = MRL_LOAD_ONCE(src + last);
+#pragma unroll
   for (int i = 0; i < NV; i++) {
-    const uint32_t idx = i * 256 + threadIdx.x;
-    if (idx < nvec) {
-      v[i] = MRL_LOAD_ONCE(src + idx);
-      nan |= (v[i][0] != v[i][0]) | (v[i][1] != v[i][1]) | (v[i][2] != v[i][2]) | (v[i][3] != v[i][3]);
-      mx = fmaxf(fmaxf(mx, fmaxf(v[i][0], v[i][1])), fmaxf(v[i][2], v[i][3]));
-    }
+    nan |= (v[i][0] != v[i][0]) | (v[i][1] != v[i][1]) | (v[i][2] != v[i][2]) | (v[i][3] != v[i][3]);
+    mx = fmaxf(fmaxf(mx, fmaxf(v[i][0], v[i][1])), fmaxf(v[i][2], v[i][3]));
   }
+  if (ODD) nan |= tail != tail, mx = fmaxf(mx, tail);
   mx = wave_max(mx);
-  if ((threadIdx.x & 63) == 0) lds[0][w] = __any(nan) ? __uint_as_float(0x7fc00000u) : mx;
+  const bool any_nan = __any(nan);
+  if ((threadIdx.x & 63) == 0) lds[0][w] = any_nan ? __uint_as_float(0x7fc00000u) : mx;
   __syncthreads();
   {
     const float a = lds[0][0], b = lds[0][1], c = lds[0][2], d = lds[0][3];
@@ -347,6 +330,7 @@ __global__ __launch_bounds__(256) void k_softmax_block(const float *__restrict__
       sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
     }
   }
+  if (ODD && last < cols) tail = expf(tail - mx), sum += tail;
   sum = wave_sum(sum);
   if ((threadIdx.x & 63) == 0) lds[1][w] = sum;
   __syncthreads();
@@ -354,17 +338,9 @@ __global__ __launch_bounds__(256) void k_softmax_block(const float *__restrict__
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     const uint32_t idx = i * 256 + threadIdx.x;
-    if (idx < nvec) {
-      const f4 y = v[i] / sum;
-      if constexpr (OUT_BF16) {
-        typedef unsigned u2 __attribute__((ext_vector_type(2)));
-        __builtin_nontemporal_store(u2{bf16_bits(y[0]) | (bf16_bits(y[1]) << 16), bf16_bits(y[2]) | (bf16_bits(y[3]) << 16)},
-                                    reinterpret_cast<u2 *>(static_cast<uint16_t *>(out_any) + row * cols) + idx);
-      } else {
-        __builtin_nontemporal_store(y, (f4 *)(static_cast<float *>(out_any) + row * cols) + idx);
-      }
-    }
+    if (idx < nvec) store_quad<ODD, OUT_BF16>(v[i] / sum, out, row * cols, idx);
   }
+  if (ODD && last < cols) store_one<OUT_BF16>(tail / sum, out, row * cols + last);
 }
 
 template <int V, bool OUT_BF16>
@@ -381,6 +357,36 @@ hipError_t launch_chunks(const float *in, void *out, uint64_t rows, uint32_t col
 }  // namespace
 
 namespace {
+// ODD: rows of a length that is no multiple of 4.
+template <bool ODD, bool OUT_BF16>
+hipError_t launch_long_rows(const float *in, void *out, uint64_t rows, uint32_t cols, void *scratch, hipStream_t stream) {
+  // A workgroup per row with the row in registers: rows beyond the wavefront kernel's 4096
+  // columns when there are 256 of them or more, and rows of more than 1024 columns when there are
+  // too few of them to occupy the chip a wavefront each.
+  if (rows <= 0x7fffffffull && ((cols > 16 * 256 && cols <= 16 * 1024 && rows >= 256) || (cols > 1024 && cols <= 16 * 256 && rows < 2048))) {
+    plan::work(plan::UNIT_STREAM, 0, double(rows) * cols * (4 + (OUT_BF16 ? 2 : 4)));
+    if (cols <= 4 * 1024) MRL_LAUNCH((k_softmax_block<4, ODD, OUT_BF16>), dim3(uint32_t(rows)), dim3(256), 0, stream, in, out, cols);
+    else if (cols <= 8 * 1024) MRL_LAUNCH((k_softmax_block<8, ODD, OUT_BF16>), dim3(uint32_t(rows)), dim3(256), 0, stream, in, out, cols);
+    else MRL_LAUNCH((k_softmax_block<16, ODD, OUT_BF16>), dim3(uint32_t(rows)), dim3(256), 0, stream, in, out, cols);
+    return mrl::plan::last_error();
+  }
+  if (scratch && softmax_scratch_bytes(rows, cols))
+    return launch_chunks<ODD ? 1 : 4, OUT_BF16>(in, out, rows, cols, static_cast<float2 *>(scratch), stream);
+  const uint64_t blocks64 = (rows + 3) / 4;
+  if (blocks64 > 0x7fffffffull || cols > 16 * 256) return hipErrorInvalidValue;   // (longer rows go in chunks, and no scratch was passed for them)
+  const dim3 grid{uint32_t(blocks64)}, block{256};
+  plan::work(plan::UNIT_STREAM, 0, double(rows) * cols * (4 + (OUT_BF16 ? 2 : 4)));
+  const uint32_t nv = (cols / 4 + 63) / 64;
+  if (nv <= 1) MRL_LAUNCH((k_softmax_regs<1, ODD, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
+  else if (nv <= 2) MRL_LAUNCH((k_softmax_regs<2, ODD, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
+  else if (nv <= 4) MRL_LAUNCH((k_softmax_regs<4, ODD, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
+  else if (nv <= 6) MRL_LAUNCH((k_softmax_regs<6, ODD, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
+  else if (nv <= 8) MRL_LAUNCH((k_softmax_regs<8, ODD, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
+  else if (nv <= 12) MRL_LAUNCH((k_softmax_regs<12, ODD, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
+  else MRL_LAUNCH((k_softmax_regs<16, ODD, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
+  return mrl::plan::last_error();
+}
+
 template <bool OUT_BF16>
 hipError_t launch_rows(const float *in, void *out, uint64_t rows, uint32_t cols, void *scratch, hipStream_t stream) {
   if (rows == 0 || cols == 0) return hipSuccess;
@@ -393,51 +399,15 @@ hipError_t launch_rows(const float *in, void *out, uint64_t rows, uint32_t cols,
     if (cols <= 128) return launch_short<16, OUT_BF16>(in, out, rows, cols, stream);
     return launch_short<32, OUT_BF16>(in, out, rows, cols, stream);
   }
-  // A workgroup per row with the row in registers: rows beyond the wavefront kernel's 4096
-  // columns when there are 256 of them or more, and rows of more than 1024 columns when there are
-  // too few of them to occupy the chip a wavefront each.
-  if (cols % 4 == 0 && rows <= 0x7fffffffull &&
-      ((cols > 16 * 256 && cols <= 16 * 1024 && rows >= 256) || (cols > 1024 && cols <= 16 * 256 && rows < 2048))) {
-    plan::work(plan::UNIT_STREAM, 0, double(rows) * cols * (4 + (OUT_BF16 ? 2 : 4)));
-    if (cols <= 8 * 1024) MRL_LAUNCH((k_softmax_block<8, OUT_BF16>), dim3(uint32_t(rows)), dim3(256), 0, stream, in, out, cols);
-    else MRL_LAUNCH((k_softmax_block<16, OUT_BF16>), dim3(uint32_t(rows)), dim3(256), 0, stream, in, out, cols);
-    return mrl::plan::last_error();
-  }
-  if (cols % 4 != 0 && cols <= 64 * 64 && rows >= 512 && (rows + 3) / 4 <= 0x7fffffffull) {
-    const dim3 grid{uint32_t((rows + 3) / 4)}, block{256};
-    plan::work(plan::UNIT_STREAM, 0, double(rows) * cols * (4 + (OUT_BF16 ? 2 : 4)));
-    if (cols <= 16 * 64) MRL_LAUNCH((k_softmax_regs1<16, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
-    else if (cols <= 32 * 64) MRL_LAUNCH((k_softmax_regs1<32, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
-    else MRL_LAUNCH((k_softmax_regs1<64, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
-    return mrl::plan::last_error();
-  }
-  if (scratch && softmax_scratch_bytes(rows, cols)) {
-    if (cols % 4 == 0) return launch_chunks<4, OUT_BF16>(in, out, rows, cols, static_cast<float2 *>(scratch), stream);
-    return launch_chunks<1, OUT_BF16>(in, out, rows, cols, static_cast<float2 *>(scratch), stream);
-  }
-  const uint64_t blocks64 = (rows + 3) / 4;
-  if (blocks64 > 0x7fffffffull) return hipErrorInvalidValue;
-  const dim3 grid{uint32_t(blocks64)}, block{256};
-  plan::work(plan::UNIT_STREAM, 0, double(rows) * cols * (4 + (OUT_BF16 ? 2 : 4)));
-  if (cols % 4 == 0 && cols <= 16 * 256) {
-    const uint32_t nv = (cols / 4 + 63) / 64;
-    if (nv <= 1) MRL_LAUNCH((k_softmax_regs<1, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
-    else if (nv <= 2) MRL_LAUNCH((k_softmax_regs<2, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
-    else if (nv <= 4) MRL_LAUNCH((k_softmax_regs<4, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
-    else if (nv <= 8) MRL_LAUNCH((k_softmax_regs<8, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
-    else MRL_LAUNCH((k_softmax_regs<16, OUT_BF16>), grid, block, 0, stream, in, out, rows, cols);
-  } else {
-    return hipErrorInvalidValue;  // rows in chunks, and no scratch was passed for them
-  }
-  return mrl::plan::last_error();
+  return cols % 4 == 0 ? launch_long_rows<false, OUT_BF16>(in, out, rows, cols, scratch, stream)
+                       : launch_long_rows<true, OUT_BF16>(in, out, rows, cols, scratch, stream);
 }
 }  // namespace
 
 // Scratch the chunked kernels want for this shape (0: the shape runs without).
 size_t softmax_scratch_bytes(uint64_t rows, uint32_t cols) {
-  // Up to 4096 columns the register kernels serve; fewer than 512 rows that are not whole
-  // vectors go in chunks too (a single one), with scalar loads.
-  if (cols <= 16 * 256 && (cols % 4 == 0 || cols <= 256 || rows >= 512)) return 0;
+  // Up to 4096 columns the register kernels serve.
+  if (cols <= 16 * 256) return 0;
   const uint64_t chunks = (cols + SOFTMAX_CHUNK - 1) / SOFTMAX_CHUNK;
   if (rows * chunks > 0x7fffffffull) return 0;
   return size_t(rows * chunks * sizeof(float2));

@@ -480,3 +480,26 @@ def test_compose_msm_with_an_infinite_key(gpu, dims, where):
         assert np.array_equal(np.isnan(got), np.isnan(want)), target
         ok = ~np.isnan(want)
         assert np.abs(got[ok] - want[ok]).max() / np.abs(want[ok]).max() < 1e-2, target
+
+
+@pytest.mark.parametrize("rows,cols", [(3, 257), (5, 1023), (2100, 1025), (7, 1501), (2049, 2047), (2, 4093), (600, 4097), (258, 8190), (257, 16383), (2050, 4095)])
+def test_softmax_rows_of_odd_lengths(gpu, rows, cols):
+    """Rows that start on any element: whole vectors and one to three elements behind them, a wavefront or a workgroup a row."""
+    x = synth.normal_f32(208, 0, (rows, cols), std=3.0)
+    x[-1, -1] = 9.0
+    x[0, cols - 1] = np.nan
+    spec = M.Softmax([rows, cols], 1)
+    assert spec.plan().kernels in (["k_softmax_regs"], ["k_softmax_block"])
+    got = run_spec(spec, [x, np.full((rows, cols), 7, np.float32)])
+    e = np.exp(x[1:].astype(np.float64) - x[1:].max(-1, keepdims=True))
+    want = e / e.sum(-1, keepdims=True)
+    assert np.isnan(got[0]).all()
+    assert (np.abs(got[1:] - want) <= 1e-5 * want + 1e-12).all()
+
+
+@pytest.mark.parametrize("scan", [9, 16, 17, 63, 64, 65, 127, 128, 129, 256, 257, 511, 512, 513])
+@pytest.mark.parametrize("before,after", [(5, 3401), (300, 33)])
+def test_softmax_over_an_outer_dim_in_registers(gpu, scan, before, after):
+    """Scan dims on either side of what a workgroup holds, column tiles with a ragged end."""
+    assert M.Softmax([before, scan, after], 1).plan().kernels == ["k_softmax_cols"]
+    _softmax_outer((before, scan, after), 1)
