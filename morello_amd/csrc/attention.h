@@ -41,14 +41,6 @@ __device__ inline uint32_t lds_address(const void *p) {
   return uint32_t(reinterpret_cast<uintptr_t>((lds_void *)p));
 }
 
-// Workgroups go to the 8 XCDs round-robin.  All query blocks of a batch entry share its K and V, so they are kept on
-// one XCD (one L2): XCD x takes the x-th run of the `total` consecutive (entry, block) pairs, the first total % 8 runs
-// one pair longer.
-__device__ inline uint32_t xcd_run(uint32_t workgroup, uint32_t total) {
-  const uint32_t xcd = workgroup % 8;
-  return xcd * (total / 8) + min(xcd, total % 8) + workgroup / 8;
-}
-
 __device__ inline v2i read_tr16(const uint8_t *p) {
   const v4s r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)p);
   return __builtin_bit_cast(v2i, r);

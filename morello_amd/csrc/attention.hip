@@ -113,6 +113,7 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
   constexpr int BQ = 32 * QG;
   const int lr = lane & 15, lgp = lane >> 4;   // position within a block's 16 rows / columns, lane group
   const uint32_t nqb = (p.m + BQ - 1) / BQ;
+  // (all query blocks of a batch entry share its K and V)
   const uint32_t lin = xcd_run(blockIdx.x, nqb * p.b);
   const int64_t head = lin / nqb;
   const int q0 = int(lin % nqb) * BQ + qg * 32;

@@ -54,6 +54,7 @@ __global__ __launch_bounds__(64 * W) void k_attn(const void *q, const void *kt, 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lgp = lane >> 4;   // position in a block's 16 rows / columns, lane group
   const uint32_t nqb = (m + 16 * QB - 1) / (16 * QB);
+  // (all query blocks of a batch entry share its K and V)
   const uint32_t lin = xcd_run(blockIdx.x, nqb * b);
   const int64_t head = lin / nqb;
   const uint32_t q0 = (lin % nqb) * (16 * QB);

@@ -47,6 +47,13 @@ inline hipError_t raise_lds_limit(std::atomic<uint64_t> &done, const void *kerne
 #define MRL_STORE_ONCE(v, p) __builtin_nontemporal_store(v, p)
 #endif
 
+// Workgroups go to the 8 XCDs round-robin, each with an L2 of its own.  Of `total` workgroups in an order in which neighbours
+// share data, XCD x takes the x-th run, the first total % 8 runs one longer.
+__device__ inline uint32_t xcd_run(uint32_t workgroup, uint32_t total) {
+  const uint32_t xcd = workgroup % 8;
+  return xcd * (total / 8) + min(xcd, total % 8) + workgroup / 8;
+}
+
 struct Strided {
   void *ptr;
   int dtype;
