@@ -50,8 +50,8 @@ inline hipError_t raise_lds_limit(std::atomic<uint64_t> &done, const void *kerne
 // Workgroups go to the 8 XCDs round-robin, each with an L2 of its own.  Of `total` workgroups in an order in which neighbours
 // share data, XCD x takes the x-th run, the first total % 8 runs one longer.
 __device__ inline uint32_t xcd_run(uint32_t workgroup, uint32_t total) {
-  const uint32_t xcd = workgroup % 8;
-  return xcd * (total / 8) + min(xcd, total % 8) + workgroup / 8;
+  const uint32_t xcd = workgroup % 8, longer = total % 8;
+  return xcd * (total / 8) + (xcd < longer ? xcd : longer) + workgroup / 8;
 }
 
 struct Strided {
@@ -251,6 +251,7 @@ hipError_t launch_unfold(const void *image, void *rows, uint32_t batch, uint32_t
 // (hipErrorInvalidValue without it).  `out` may be `in`.
 constexpr uint32_t SOFTMAX_CHUNK = 4096;
 size_t softmax_scratch_bytes(uint64_t rows, uint32_t cols);
+size_t softmax_chunk_bytes(uint64_t rows, uint32_t cols);
 hipError_t launch_softmax_rows(const float *in, float *out, uint64_t rows, uint32_t cols, void *scratch,
                                hipStream_t stream);
 // The same with the result rounded to bf16 (rows of `cols` 16-bit values).
