@@ -495,7 +495,7 @@ __global__ __launch_bounds__(256) void k_move_tiled32(MoveStrided p) {
 // by memory, so what matters is the order: a workgroup's tile is long along the digit that
 // continues the destination's runs AND along the one that continues the source's, so that both
 // sides see whole cache lines (f32 2048 x 16384 into bf16 strips of 16 columns, runs of 64 and
-// 32 bytes: an element per thread in destination order 133 us, this 44).  UNROLL vectors a
+// 32 bytes: an element per thread in destination order 133 us, this 41).  UNROLL vectors a
 // thread, their loads in flight together.
 constexpr int MOVE_RUNS_ACT = 4;   // digits a tile extends along at most
 template <int SE, int DE, int V, int UNROLL>
@@ -1142,8 +1142,9 @@ uint32_t runs_tile(const MoveStrided &p, uint32_t shared, uint32_t vec, uint32_t
   };
   const int next_d = next(p.ds, -1), next_s = next(p.ss, -1);
   if (next_d >= 0 && next_s >= 0 && next_s != next_d) {
-    // 512 bytes of the source side, along two digits if need be, the rest of the tile along the destination's
-    const uint32_t want_s = std::min(std::max(1u, 512u / (ext[shared] * vec * se)), std::max(1u, tile_cap / tile));
+    // 512 bytes of the source side (of 32 a vector 1 KiB: 42.9 / 40.9 us at 2048 x 16384), along two digits if need be, the rest of the tile along the destination's
+    const uint32_t piece = vec * se == 32 ? 1024 : 512;
+    const uint32_t want_s = std::min(std::max(1u, piece / (ext[shared] * vec * se)), std::max(1u, tile_cap / tile));
     const int further = p.shape[next_s] < want_s ? next(p.ss, next_s) : -1;
     const bool two = further >= 0 && further != next_d;
     const uint32_t s1 = std::min(want_s, p.shape[next_s]), s2 = two ? std::min(want_s / s1, p.shape[further]) : 1;
@@ -1193,6 +1194,7 @@ hipError_t launch_move_runs(MoveStrided p, uint32_t shared, uint32_t vec, bool t
 #define MRL_RUNS(SE, DE)                                                                                            \
   if (se == SE && de == DE) {                                                                                      \
     constexpr int WIDE = 16 / (SE > DE ? SE : DE);                                                                  \
+    if constexpr (SE == 4 && DE == 2) MRL_RUNS_V(SE, DE, 8)                                                         \
     MRL_RUNS_V(SE, DE, WIDE)                                                                                        \
     else MRL_RUNS_V(SE, DE, WIDE / 2)                                                                               \
     else if constexpr (WIDE >= 8) MRL_RUNS_V(SE, DE, WIDE / 4)                                                      \
@@ -1292,11 +1294,17 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
     }
   }
   // A shared contiguous digit in whole vectors on both sides: 16, 8 or 4 bytes on the wider side.
+  // From 32-bit elements to 16-bit ones 16 bytes on the narrower side where the source's rows lie multiples of 8 KiB apart, on
+  // the same memory channels (us, buffers taking turns, before -> now: f32 2048 x 16384 into bf16 strips of 16 44.7 -> 42.0, 8192 x 8192 97.4 -> 81.4,
+  // 4096 x 8192 44.1 -> 40.9, 512 x 16384 11.3 -> 10.3; other rows either way: 7232 x 6800 56.9 -> 58.9, 8192 x 3072 30.6 -> 32.0).
   const size_t widest = std::max(se, de);
   uint32_t vec = 0;
+  uint64_t row = 0;   // bytes from one row of the source to the next: its longest stride
+  for (uint32_t d = 0; d < rank; d++) row = std::max(row, uint64_t(p.ss[d]) * se);
+  const bool pages = se == 4 && de == 2 && p.count > MOVE_SMALL && row % 8192 == 0;
   if (shared && rank > 1)
-    for (uint32_t v = uint32_t(16 / widest); vec == 0 && v >= 1 && v * widest >= 4; v /= 2) {
-      bool fits = v > 1 && p.shape[dim_s] % v == 0 && (reinterpret_cast<uintptr_t>(src) % (v * se)) == 0 &&
+    for (uint32_t v = uint32_t(16 / widest) * (pages ? 2 : 1); vec == 0 && v >= 1 && v * widest >= 4; v /= 2) {
+      bool fits = v > 1 && p.shape[dim_s] % v == 0 && (reinterpret_cast<uintptr_t>(src) % std::min<size_t>(16, v * se)) == 0 &&
                   (reinterpret_cast<uintptr_t>(dst) % (v * de)) == 0;
       for (uint32_t d = 0; fits && d < rank; d++) fits = int(d) == dim_s || (p.ss[d] % v == 0 && p.ds[d] % v == 0);
       if (fits) vec = v;

@@ -154,12 +154,18 @@ __device__ inline void tile_origin(const MoveTile &p, int64_t &base_s, int64_t &
 }
 
 // V elements of `size` bytes as zero-extended values <-> memory, one access of V * size bytes.
+// (32 bytes, eight 32-bit values: two accesses)
 template <int SIZE, int V>
 __device__ inline void load_run(const void *p, int64_t off, uint32_t (&raw)[V]) {
   constexpr int BYTES = SIZE * V;
   if constexpr (V == 1 || BYTES < 4) {
 #pragma unroll
     for (int e = 0; e < V; e++) raw[e] = load_sized<SIZE>(p, off + e);
+  } else if constexpr (BYTES == 32) {   // two of 16, at their alignment
+    const v4u_t *at = reinterpret_cast<const v4u_t *>(static_cast<const uint8_t *>(p) + off * SIZE);
+    const v4u_t lo = at[0], hi = at[1];
+#pragma unroll
+    for (int e = 0; e < V; e++) raw[e] = e < 4 ? lo[e] : hi[e - 4];
   } else {
     typedef uint32_t W __attribute__((ext_vector_type(BYTES / 4 == 1 ? 2 : BYTES / 4)));
     const uint8_t *at = static_cast<const uint8_t *>(p) + off * SIZE;

@@ -135,3 +135,14 @@ def test_gathered_runs_of_four_and_of_two(gpu, sdt, ddt, shape, src, dst):
 def test_gathered_runs_off_an_element(gpu, shift):
     _check(M.f32, M.f32, [20, 60004], None, (1, 0), "k_move_gather", shift)
     _check(M.bf16, M.bf16, [20, 60004], None, (1, 0), "k_move_gather", shift)
+
+
+@pytest.mark.parametrize("sdt,ddt", [(M.f32, M.bf16), (M.i32, M.u16), (M.f32, M.u16)])
+@pytest.mark.parametrize("rows,cols,strips,shift", [(1030, 2048, 16, (0, 0)), (513, 2048, 8, (0, 0)), (1030, 1024, 16, (0, 0)), (2049, 3072, 16, (0, 0)), (1025, 2048, 24, (0, 0)),
+                                                    (1030, 2048, 16, (4, 0)), (1030, 2048, 16, (0, 4)), (1030, 2048, 16, (2, 8))])
+def test_narrowing_rows_8_kib_apart(gpu, sdt, ddt, rows, cols, strips, shift):
+    """Rows of multiples of 8 KiB (and of 4 and 12), 32-bit elements to 16-bit ones: eight elements a vector where both buffers are aligned for it, four or two otherwise."""
+    if strips == 24:   # a digit between the strips and the rows
+        _check(sdt, ddt, [5, rows // 5, cols], None, (2, 1, 0, (2, "p", 8)), "k_move_runs", shift)
+    else:
+        _check(sdt, ddt, [1, rows, cols], None, (0, 2, 1, (2, "p", strips)), "k_move_runs", shift)
