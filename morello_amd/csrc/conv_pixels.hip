@@ -48,45 +48,99 @@ struct PixelsArgs {
   uint32_t chunks_log2;         // log2 of cpr
   uint32_t slots;               // pixels of a filter's row in LDS: steps * 64 / PB
   uint32_t patch_w, patch_h;    // pixels
+  int whole_lines;              // 32 filters of a pixel are a cache line of the output
   uint32_t patch_bytes;         // of LDS, rows that only a tail step's masked lanes read included
   FastDiv by_image, by_row, by_slots, by_patch_w;   // items of an image, of an image's row of them
+};
+
+// Pixels of four elements in LDS out of pixels of three or four in memory.
+template <int KIND>
+struct Pixels {
+  static constexpr bool HALVES = KIND == IMG_BF16;
+  static constexpr int ES = HALVES ? 2 : 1, PB = 4 * ES, PER_CHUNK = 16 / PB;   // bytes of a pixel in LDS, pixels of a chunk
+  typedef typename std::conditional<HALVES, float, int>::type Element;
+  typedef Element Acc __attribute__((ext_vector_type(4)));
+  struct Pixel { uint32_t v[ES]; };
+  struct Raw { uint32_t v[ES + 1]; uint32_t shift; };
+  __device__ static Acc mfma(v4i a, v4i b, Acc c) {
+    if constexpr (HALVES) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
+  }
+  // A pixel out of the aligned dwords it lies in (a dword without a byte of it is not read).
+  __device__ static Raw fetch(const uint8_t *at, uint32_t pixel_bytes) {
+    Raw r;
+    r.shift = uint32_t(reinterpret_cast<uintptr_t>(at)) & 3;
+    const uint32_t *from = reinterpret_cast<const uint32_t *>(at - r.shift);
+#pragma unroll
+    for (int i = 0; i < ES; i++) r.v[i] = from[i];
+    r.v[ES] = from[r.shift + pixel_bytes > 4 * ES ? ES : ES - 1];
+    return r;
+  }
+  __device__ static Pixel pixel(const Raw &r, uint32_t pixel_bytes) {
+    const uint32_t last_mask = pixel_bytes == PB ? 0xffffffffu : HALVES ? 0xffffu : 0xffffffu;
+    Pixel x;
+#pragma unroll
+    for (int i = 0; i < ES; i++) x.v[i] = __builtin_amdgcn_alignbyte(r.v[i + 1], r.v[i], r.shift);
+    x.v[ES - 1] &= last_mask;
+    return x;
+  }
+  __device__ static void put(uint8_t *to, const Pixel &x) {
+    if constexpr (HALVES) *(v2u *)to = v2u{x.v[0], x.v[ES - 1]};
+    else *(uint32_t *)to = x.v[0];
+  }
+  // The image's pixels as they are multiplied: u8 as a - 128.
+  __device__ static void put_image(uint8_t *to, const Raw &r, uint32_t pixel_bytes) {
+    Pixel x = pixel(r, pixel_bytes);
+    if (KIND == IMG_U8) x.v[0] ^= 0x80808080u;
+    put(to, x);
+  }
+  // This workgroup's filters, `nf` from f0 on, into rows of `filter_row` bytes at `filt` (`group` of them, zeros where no pixel
+  // is): their bytes are one contiguous piece of memory, fetched in whole chunks with the loads in flight together into
+  // the LDS behind, then spread out pixel by pixel.
+  __device__ static void stage_filters(const PixelsArgs &p, uint32_t group, uint32_t f0, uint32_t nf, uint32_t filter_row, uint8_t *filt) {
+    const int tid = threadIdx.x;
+    const uint32_t filter_bytes = p.fh * p.fw * p.pixel_bytes;
+    const uint8_t *from = p.filters + uint64_t(f0) * filter_bytes;
+    const uint32_t head = uint32_t(reinterpret_cast<uintptr_t>(from)) & 15, chunks = (head + nf * filter_bytes + 15) / 16;
+    const v4i *first = reinterpret_cast<const v4i *>(from - head);
+    v4i *raw = reinterpret_cast<v4i *>(filt + group * filter_row);
+    constexpr uint32_t BATCH = 3;
+    for (uint32_t c0 = 0; c0 < chunks; c0 += BATCH * 64 * WAVES) {
+      v4i got[BATCH];
+#pragma unroll
+      for (uint32_t j = 0; j < BATCH; j++) got[j] = first[min(c0 + j * 64 * WAVES + tid, chunks - 1)];
+#pragma unroll
+      for (uint32_t j = 0; j < BATCH; j++)
+        if (c0 + j * 64 * WAVES + tid < chunks) raw[c0 + j * 64 * WAVES + tid] = got[j];
+    }
+    __syncthreads();
+    const uint32_t *words = reinterpret_cast<const uint32_t *>(raw);
+    const uint32_t per_row = uint32_t(PER_CHUNK) << p.chunks_log2;   // pixels a window's row takes
+#pragma unroll 2
+    for (uint32_t i = tid; i < group * p.slots; i += 64 * WAVES) {
+      const uint32_t fi = p.by_slots.div(i), s = i - fi * p.slots;
+      const uint32_t r = s / PER_CHUNK >> p.chunks_log2, x = s & (per_row - 1);
+      const bool real = fi < nf && r < p.fh && x < p.fw;
+      const uint32_t at = real ? head + ((fi * p.fh + r) * p.fw + x) * p.pixel_bytes : head;
+      Raw px;
+#pragma unroll
+      for (int w = 0; w <= ES; w++) px.v[w] = words[at / 4 + w];
+      px.shift = at & 3;
+      put(filt + fi * filter_row + s * PB, real ? pixel(px, p.pixel_bytes) : Pixel{});
+    }
+    __syncthreads();   // the raw bytes are no longer needed
+  }
 };
 
 // KS: whole k steps of 64 bytes (a window's chunks / 4); the rest is a tail whose lanes past the
 // filter's last row count for nothing.  PIXELS: always true; tells this form from the other one in plans and profiles.
 template <int KS, int KIND, bool PIXELS>
 __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
-  constexpr bool HALVES = KIND == IMG_BF16;
-  constexpr int ES = HALVES ? 2 : 1, PB = 4 * ES, PER_CHUNK = 16 / PB;   // bytes of a pixel in LDS, pixels of a chunk
-  typedef typename std::conditional<HALVES, v4f, v4i>::type Acc;
-  auto mfma = [](v4i a, v4i b, Acc c) {
-    if constexpr (HALVES) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
-  };
-  struct Pixel { uint32_t v[ES]; };
-  struct Raw { uint32_t v[ES + 1]; uint32_t shift; };
-  // A pixel out of the aligned dwords it lies in (a dword without a byte of it is not read).
-  auto fetch = [&](const uint8_t *at) {
-    Raw r;
-    r.shift = uint32_t(reinterpret_cast<uintptr_t>(at)) & 3;
-    const uint32_t *from = reinterpret_cast<const uint32_t *>(at - r.shift);
-#pragma unroll
-    for (int i = 0; i < ES; i++) r.v[i] = from[i];
-    r.v[ES] = from[r.shift + p.pixel_bytes > 4 * ES ? ES : ES - 1];
-    return r;
-  };
-  const uint32_t last_mask = p.pixel_bytes == PB ? 0xffffffffu : HALVES ? 0xffffu : 0xffffffu;
-  auto pixel = [&](const Raw &r) {
-    Pixel x;
-#pragma unroll
-    for (int i = 0; i < ES; i++) x.v[i] = __builtin_amdgcn_alignbyte(r.v[i + 1], r.v[i], r.shift);
-    x.v[ES - 1] &= last_mask;
-    return x;
-  };
-  auto put = [&](uint8_t *to, const Pixel &x) {
-    if constexpr (HALVES) *(v2u *)to = v2u{x.v[0], x.v[ES - 1]};
-    else *(uint32_t *)to = x.v[0];
-  };
+  typedef Pixels<KIND> P;
+  typedef typename P::Acc Acc;
+  typedef typename P::Raw Raw;
+  constexpr bool HALVES = P::HALVES;
+  constexpr int PB = P::PB, PER_CHUNK = P::PER_CHUNK;
   extern __shared__ __attribute__((aligned(16))) uint8_t pix_lds[];
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -118,45 +172,12 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
   auto fetch_patch = [&](const Corner &at) {
 #pragma unroll
     for (int j = 0; j < HELD; j++)
-      if (lane + j * 64 < int(patch_pixels)) held[j] = fetch(source(at, held_y[j], held_x[j]));
+      if (lane + j * 64 < int(patch_pixels)) held[j] = P::fetch(source(at, held_y[j], held_x[j]), p.pixel_bytes);
   };
   const uint32_t stride = gridDim.x * WAVES;
   uint32_t item = blockIdx.x * WAVES + wave;
   if (item < p.items) fetch_patch(corner_of(item));   // in flight while the filters are staged
-  // The filters: their bytes are one contiguous piece of memory, fetched in whole chunks with the loads in
-  // flight together (into what will be the patches), then spread out pixel by pixel.
-  {
-    const uint32_t filter_bytes = p.fh * p.fw * p.pixel_bytes;
-    const uint8_t *from = p.filters + uint64_t(f0) * filter_bytes;
-    const uint32_t head = uint32_t(reinterpret_cast<uintptr_t>(from)) & 15, chunks = (head + nf * filter_bytes + 15) / 16;
-    const v4i *first = reinterpret_cast<const v4i *>(from - head);
-    v4i *raw = reinterpret_cast<v4i *>(filt + p.group * filter_row);
-    constexpr uint32_t BATCH = 3;
-    for (uint32_t c0 = 0; c0 < chunks; c0 += BATCH * 64 * WAVES) {
-      v4i got[BATCH];
-#pragma unroll
-      for (uint32_t j = 0; j < BATCH; j++) got[j] = first[min(c0 + j * 64 * WAVES + tid, chunks - 1)];
-#pragma unroll
-      for (uint32_t j = 0; j < BATCH; j++)
-        if (c0 + j * 64 * WAVES + tid < chunks) raw[c0 + j * 64 * WAVES + tid] = got[j];
-    }
-    __syncthreads();
-    const uint32_t *words = reinterpret_cast<const uint32_t *>(raw);
-    const uint32_t per_row = uint32_t(PER_CHUNK) << p.chunks_log2;   // pixels a window's row takes
-#pragma unroll 2
-    for (uint32_t i = tid; i < p.group * p.slots; i += 64 * WAVES) {
-      const uint32_t fi = p.by_slots.div(i), s = i - fi * p.slots;
-      const uint32_t r = s / PER_CHUNK >> p.chunks_log2, x = s & (per_row - 1);
-      const bool real = fi < nf && r < p.fh && x < p.fw;
-      const uint32_t at = real ? head + ((fi * p.fh + r) * p.fw + x) * p.pixel_bytes : head;
-      Raw px;
-#pragma unroll
-      for (int w = 0; w <= ES; w++) px.v[w] = words[at / 4 + w];
-      px.shift = at & 3;
-      put(filt + fi * filter_row + s * PB, real ? pixel(px) : Pixel{});
-    }
-    __syncthreads();   // the raw bytes are no longer needed
-  }
+  P::stage_filters(p, p.group, f0, nf, filter_row, filt);   // (the bytes as they lie in memory into what will be the patches)
   const uint8_t *my_filt = filt + li * filter_row + lg * 16;
   // u8 pixels are multiplied as a - 128: 128 times a filter's sum comes on top (kept in LDS, in the
   // 16 bytes between the filters' rows).
@@ -164,7 +185,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
     const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
     for (uint32_t fb = wave; fb < p.group / 16; fb += WAVES) {
       Acc sum = {};
-      for (uint32_t ks = 0; ks < p.steps; ks++) sum = mfma(*(const v4i *)(my_filt + fb * 16 * filter_row + ks * 64), ones, sum);
+      for (uint32_t ks = 0; ks < p.steps; ks++) sum = P::mfma(*(const v4i *)(my_filt + fb * 16 * filter_row + ks * 64), ones, sum);
       if (li == 0) *(v4i *)(filt + (fb * 16 + lg) * filter_row + p.steps * 64) = sum * 128;
     }
     __syncthreads();
@@ -188,16 +209,10 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
     const Corner at = corner_of(item);
 #pragma unroll
     for (int j = 0; j < HELD; j++)
-      if (lane + j * 64 < int(patch_pixels)) {
-        Pixel x = pixel(held[j]);
-        if (KIND == IMG_U8) x.v[0] ^= 0x80808080u;
-        put(patch + (lane + j * 64) * PB, x);
-      }
+      if (lane + j * 64 < int(patch_pixels)) P::put_image(patch + (lane + j * 64) * PB, held[j], p.pixel_bytes);
     for (uint32_t i = lane + HELD * 64; i < patch_pixels; i += 64) {
       const uint32_t r = p.by_patch_w.div(i);
-      Pixel x = pixel(fetch(source(at, r, i - r * p.patch_w)));
-      if (KIND == IMG_U8) x.v[0] ^= 0x80808080u;
-      put(patch + i * PB, x);
+      P::put_image(patch + i * PB, P::fetch(source(at, r, i - r * p.patch_w), p.pixel_bytes), p.pixel_bytes);
     }
     // The wave's LDS accesses complete in order: what is left is that the compiler keeps them so.
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -228,7 +243,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
 #pragma unroll
         for (int pb = 0; pb < ITEM_H; pb++)
 #pragma unroll
-          for (int fb = 0; fb < FB; fb++) acc[pb][fb] = mfma(a[fb], bop[pb], acc[pb][fb]);
+          for (int fb = 0; fb < FB; fb++) acc[pb][fb] = P::mfma(a[fb], bop[pb], acc[pb][fb]);
       };
 #pragma unroll 2
       for (int ks = 0; ks < KS; ks++) step(ks, true);
@@ -254,6 +269,151 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
   }
 }
 
+// The same with the filters' operands in registers, for filters of up to seven rows whose rows are RPS to a step (1, 2 or 4):
+// a workgroup takes 32 filters, and the operand of patch row r serves every pair of a step and an output row with
+// RPS * step + row = r.  What bounded the form above beside its stores was LDS, 56 KB read per 16 x 2 pixels and 64 filters of bf16
+// 7 x 7; here 16 KB are.  Bound now by the stores of the output and by the start (filters staged, a first patch: 4 us). us, the
+// form above / this: bf16 7 x 7 16 x 3 -> 64 x 109^2 16.7 / 15.2, 32 x 3 -> 96 x 224^2 152 / 127, u8 7 x 7 12 x 4 -> 96 x 76^2 12.6 / 9.9.
+template <int KS, int RPS, bool TAIL, int KIND, bool PIXELS>
+__global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
+  typedef Pixels<KIND> P;
+  typedef typename P::Acc Acc;
+  typedef typename P::Raw Raw;
+  constexpr bool HALVES = P::HALVES;
+  constexpr int PB = P::PB, PER_CHUNK = P::PER_CHUNK, STEPS = KS + TAIL, CHUNKS = 4 / RPS, GROUP = 16 * FB;
+  constexpr uint32_t filter_row = STEPS * 64 + 16, patch_w = ITEM_W - 1 + PER_CHUNK * CHUNKS, row_bytes = patch_w * PB;
+  constexpr int ROWS = RPS * (STEPS - 1) + ITEM_H;      // patch rows that operands start in
+  extern __shared__ __attribute__((aligned(16))) uint8_t pix_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint8_t *const patch = pix_lds + wave * p.patch_bytes;   // (where the filters lay while they were staged)
+  const uint32_t f0 = blockIdx.y * GROUP, nf = min(uint32_t(GROUP), p.f - f0);
+
+  const uint32_t patch_pixels = patch_w * p.patch_h;
+  struct Corner { uint32_t img, y0, x0; };
+  const uint32_t tiles_x = (p.ow + ITEM_W - 1) / ITEM_W, per_image = tiles_x * ((p.oh + ITEM_H - 1) / ITEM_H);
+  auto corner_of = [&](uint32_t item) {
+    const uint32_t img = p.by_image.div(item), in_img = item - img * per_image, ty = p.by_row.div(in_img);
+    return Corner{img, ty * ITEM_H, (in_img - ty * tiles_x) * ITEM_W};
+  };
+  auto source = [&](const Corner &at, uint32_t r, uint32_t x) {   // (past the image's edge: as above)
+    return p.image + ((uint64_t(at.img) * p.h + min(at.y0 + r, p.h - 1)) * p.w + min(at.x0 + x, p.w - 1)) * p.pixel_bytes;
+  };
+  Raw held[HELD];
+  auto fetch_patch = [&](const Corner &at) {
+#pragma unroll
+    for (int j = 0; j < HELD; j++) {
+      const uint32_t i = lane + j * 64, r = i / patch_w;
+      if (i < patch_pixels) held[j] = P::fetch(source(at, r, i - r * patch_w), p.pixel_bytes);
+    }
+  };
+  const uint32_t stride = gridDim.x * WAVES;
+  uint32_t item = blockIdx.x * WAVES + wave;
+  if (item < p.items) fetch_patch(corner_of(item));   // in flight while the filters are staged
+  P::stage_filters(p, GROUP, f0, nf, filter_row, pix_lds);
+  v4i a[STEPS][FB];
+#pragma unroll
+  for (int ks = 0; ks < STEPS; ks++)
+#pragma unroll
+    for (int fb = 0; fb < FB; fb++) a[ks][fb] = *(const v4i *)(pix_lds + (fb * 16 + li) * filter_row + lg * 16 + ks * 64);
+  Acc start[FB];   // u8 pixels are multiplied as a - 128: 128 times a filter's sum comes on top
+#pragma unroll
+  for (int fb = 0; fb < FB; fb++) {
+    start[fb] = Acc{};
+    if constexpr (KIND == IMG_U8) {
+      const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ks++) start[fb] = P::mfma(a[ks][fb], ones, start[fb]);
+      start[fb] *= 128;
+    }
+  }
+  __syncthreads();   // every wave holds its operands: the patches may lie there
+  const uint32_t chunk = lg & (CHUNKS - 1), row_of = uint32_t(lg) / CHUNKS;
+  const uint8_t *my_patch = patch + row_of * row_bytes + li * PB + chunk * 16;
+  const uint32_t keep_lo = chunk * PER_CHUNK < p.fw ? 0xffffffffu : 0u, keep_hi = chunk * PER_CHUNK + 1 < p.fw ? 0xffffffffu : 0u;
+  const bool inside = KS * RPS + row_of < p.fh;   // of the tail step
+  for (; item < p.items; item += stride) {
+    const Corner at = corner_of(item);
+#pragma unroll
+    for (int j = 0; j < HELD; j++)
+      if (lane + j * 64 < int(patch_pixels)) P::put_image(patch + (lane + j * 64) * PB, held[j], p.pixel_bytes);
+    // The wave's LDS accesses complete in order: what is left is that the compiler keeps them so.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (item + stride < p.items) fetch_patch(corner_of(item + stride));
+    Acc acc[ITEM_H][FB];
+#pragma unroll
+    for (int pb = 0; pb < ITEM_H; pb++)
+#pragma unroll
+      for (int fb = 0; fb < FB; fb++) acc[pb][fb] = start[fb];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+      v4i bop;
+      if constexpr (HALVES) {
+        const v2u lo = *(const v2u *)(my_patch + r * row_bytes) & keep_lo, hi = *(const v2u *)(my_patch + r * row_bytes + 8) & keep_hi;
+        bop = v4i{int(lo[0]), int(lo[1]), int(hi[0]), int(hi[1])};
+      } else {
+        const uint32_t *w = (const uint32_t *)(my_patch + r * row_bytes);
+        bop = v4i{int(w[0]), int(w[1]), int(w[2]), int(w[3])};
+      }
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ks++) {
+        const int pb = r - RPS * ks;
+        if (pb < 0 || pb >= ITEM_H) continue;
+        const v4i b = HALVES && TAIL && ks == KS && !inside ? v4i{0, 0, 0, 0} : bop;
+#pragma unroll
+        for (int fb = 0; fb < FB; fb++) acc[pb][fb] = P::mfma(a[ks][fb], b, acc[pb][fb]);
+      }
+    }
+    auto at_pixel = [&](int pb, uint32_t x) { return (Acc *)(p.out + ((uint64_t(at.img) * p.oh + at.y0 + pb) * p.ow + x) * p.f + f0 + 4 * lg); };
+    if (p.whole_lines) {
+      // A pixel's 32 filters are a cache line: lanes of pixels 0 .. 7 and 8 .. 15 exchange a block, so that a store is eight whole
+      // lines and not sixteen halves, and they go past the caches (32 x 3 -> 96 x 224^2 bf16 7 x 7: 156 us in halves, 148 in
+      // lines, 127 in lines past the caches; halves past the caches 197).
+      const bool low = li < 8;
+      const uint32_t x = at.x0 + (li & 7);
+#pragma unroll
+      for (int pb = 0; pb < ITEM_H; pb++) {
+        const Acc mine = low ? acc[pb][0] : acc[pb][1];
+        Acc theirs = low ? acc[pb][1] : acc[pb][0];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const typename P::Element own = theirs[i];
+          const int bits = __builtin_bit_cast(int, own), other = __builtin_amdgcn_update_dpp(bits, bits, 0x128, 0xf, 0xf, false);   // row_ror:8
+          theirs[i] = __builtin_bit_cast(typename P::Element, other);
+        }
+        if (at.y0 + pb >= p.oh) continue;
+        Acc *d = at_pixel(pb, x) + (low ? 0 : 4), *e = at_pixel(pb, x + 8) + (low ? 0 : 4);
+        Acc v = low ? mine : theirs, w = low ? theirs : mine;
+        if (x < p.ow) {
+          if (p.accum) v += *d;
+          MRL_STORE_ONCE(v, d);
+        }
+        if (x + 8 < p.ow) {
+          if (p.accum) w += *e;
+          MRL_STORE_ONCE(w, e);
+        }
+      }
+    } else {
+      const uint32_t x = at.x0 + li;
+#pragma unroll
+      for (int pb = 0; pb < ITEM_H; pb++)
+        if (at.y0 + pb < p.oh && x < p.ow) {
+          Acc *d = at_pixel(pb, x);
+#pragma unroll
+          for (int fb = 0; fb < FB; fb++)
+            if (fb * 16 < int(nf)) {
+              Acc v = acc[pb][fb];
+              if (p.accum) v += d[4 * fb];
+              d[4 * fb] = v;
+            }
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 template <int KS, int KIND, bool PIXELS = true>
 hipError_t launch(const PixelsArgs &p, dim3 grid, size_t lds, hipStream_t stream) {
   static std::atomic<uint64_t> limit{0};
@@ -271,6 +431,26 @@ hipError_t launch_ks(const PixelsArgs &p, int kind, dim3 grid, size_t lds, hipSt
     case IMG_U8: return launch<KS, IMG_U8>(p, grid, lds, stream);
     default: return launch<KS, IMG_BF16>(p, grid, lds, stream);
   }
+}
+
+// The form with the filters' operands in registers: `rows` filter rows, `rps` of them to a step.
+template <int KS, int RPS, bool TAIL, int KIND, bool PIXELS = true>
+hipError_t launch_held(const PixelsArgs &p, dim3 grid, size_t lds, hipStream_t stream) {
+  MRL_LAUNCH((k_conv_windows<KS, RPS, TAIL, KIND, PIXELS>), grid, dim3(64 * WAVES), lds, stream, p);
+  return plan::last_error();
+}
+template <int RPS, int KIND>
+hipError_t launch_rows(const PixelsArgs &p, dim3 grid, size_t lds, hipStream_t stream) {
+  switch (p.fh) {
+#define MRL_ROWS(N) case N: return launch_held<N / RPS, RPS, N % RPS != 0, KIND>(p, grid, lds, stream);
+    MRL_ROWS(1) MRL_ROWS(2) MRL_ROWS(3) MRL_ROWS(4) MRL_ROWS(5) MRL_ROWS(6)
+#undef MRL_ROWS
+    default: return launch_held<7 / RPS, RPS, 7 % RPS != 0, KIND>(p, grid, lds, stream);
+  }
+}
+// int8 rows of one or two chunks, bf16 ones of two or four.
+bool rows_held(const ConvArgs &c, int kind, uint32_t chunks_log2) {
+  return c.fh <= 7 && (kind == IMG_BF16 ? chunks_log2 >= 1 : chunks_log2 <= 1);
 }
 
 constexpr uint32_t MAX_KS = 7;
@@ -298,6 +478,7 @@ hipError_t launch_conv_pixels(const ConvArgs &c, int kind, hipStream_t stream) {
   p.image = (const uint8_t *)c.image, p.filters = (const uint8_t *)c.filters, p.out = (int32_t *)c.out;
   p.f = c.f, p.oh = c.oh, p.ow = c.ow, p.fh = c.fh, p.fw = c.fw, p.h = c.oh + c.fh - 1, p.w = c.ow + c.fw - 1;
   p.pixel_bytes = c.c * es, p.accum = c.accum;
+  p.whole_lines = c.f % 32 == 0 && (reinterpret_cast<uintptr_t>(c.out) & 127) == 0;
   p.chunks_log2 = chunks_log2_of(c, kind);
   const uint32_t rows_per_step = 4u >> p.chunks_log2, whole = c.fh / rows_per_step;
   p.steps = (c.fh + rows_per_step - 1) / rows_per_step;
@@ -307,20 +488,35 @@ hipError_t launch_conv_pixels(const ConvArgs &c, int kind, hipStream_t stream) {
   const uint32_t tiles_x = (c.ow + ITEM_W - 1) / ITEM_W, per_image = tiles_x * ((c.oh + ITEM_H - 1) / ITEM_H);
   p.items = c.b * per_image;
   p.by_image = FastDiv(per_image), p.by_row = FastDiv(tiles_x), p.by_slots = FastDiv(p.slots), p.by_patch_w = FastDiv(p.patch_w);
+  const double pixels = double(c.b) * c.oh * c.ow;
+  // (one or two steps under three or four groups of filters, past three rounds of waves: a patch staged once for all of them is
+  // the faster one, us, once / per group: 16 x 3 -> 128 x 100^2 3 x 3 16.9 / 19.4, 12 x 4 -> 96 x 134^2 17.7 / 18.5; 17 x 4 -> 96 x 80^2, two and a half rounds, 11.4 / 10.2)
+  const uint32_t groups = (c.f + 16 * FB - 1) / (16 * FB);
+  const bool shared_patch = p.steps <= 2 && groups > 2 && c.f <= 128 && uint64_t(p.items) * groups > 3 * 2 * uint64_t(g_compute_units) * WAVES;
+  if (!shared_patch && rows_held(c, kind, p.chunks_log2) && p.patch_w * p.patch_h <= HELD * 64) {
+    const size_t raw = size_t(std::min<uint32_t>(c.f, 16 * FB)) * c.fh * c.fw * p.pixel_bytes + 32;
+    const size_t lds = std::max(16 * FB * (p.steps * 64 + 16) + raw, WAVES * size_t(p.patch_bytes));
+    const uint32_t wgs = std::min<uint32_t>((p.items + WAVES - 1) / WAVES, std::max(1u, 2 * g_compute_units / groups));
+    plan::work(plan::UNIT_STREAM, 0, 1.5 * (pixels * c.f * 4 * (c.accum ? 2 : 1) + double(c.b) * p.h * p.w * p.pixel_bytes), 0,
+               4000.0 + (700.0 + 100.0 * p.steps) * double((p.items + wgs * WAVES - 1) / (wgs * WAVES)));
+    const dim3 grid(wgs, groups);
+    if (kind == IMG_BF16) return rows_per_step == 1 ? launch_rows<1, IMG_BF16>(p, grid, lds, stream) : launch_rows<2, IMG_BF16>(p, grid, lds, stream);
+    if (kind == IMG_U8) return rows_per_step == 2 ? launch_rows<2, IMG_U8>(p, grid, lds, stream) : launch_rows<4, IMG_U8>(p, grid, lds, stream);
+    return rows_per_step == 2 ? launch_rows<2, IMG_I8>(p, grid, lds, stream) : launch_rows<4, IMG_I8>(p, grid, lds, stream);
+  }
   // All filters of up to 128 in one workgroup, so that a pixel is staged once; 32 at a time where that
   // would leave compute units without work.
   const uint64_t wanted = (uint64_t(p.items) + WAVES - 1) / WAVES;
   p.group = c.f <= 32 || wanted * 2 <= g_compute_units ? 32 : c.f <= 128 ? (c.f + 31) & ~31u : 64;
-  const uint32_t groups = (c.f + p.group - 1) / p.group;
+  const uint32_t all_groups = (c.f + p.group - 1) / p.group;
   // behind the filters the patches, and before them the filters as they lie in memory (16 bytes more on either side)
   const size_t raw = size_t(std::min(c.f, p.group)) * c.fh * c.fw * p.pixel_bytes + 32;
   const size_t lds = p.group * (p.steps * 64 + 16) + std::max(raw, WAVES * size_t(p.patch_bytes));
   // Two workgroups to a compute unit walk the items, so that the filters are staged once each.
-  const uint32_t wgs = std::min<uint32_t>((p.items + WAVES - 1) / WAVES, std::max(1u, 2 * g_compute_units / groups));
-  const double pixels = double(c.b) * c.oh * c.ow;
+  const uint32_t wgs = std::min<uint32_t>((p.items + WAVES - 1) / WAVES, std::max(1u, 2 * g_compute_units / all_groups));
   plan::work(plan::UNIT_STREAM, 0, 1.5 * (pixels * c.f * 4 * (c.accum ? 2 : 1) + double(c.b) * p.h * p.w * p.pixel_bytes), 0,
              4000.0 + (1000.0 + 200.0 * p.steps) * double((p.items + wgs * WAVES - 1) / (wgs * WAVES)));   // staging the filters; an item
-  const dim3 grid(wgs, groups);
+  const dim3 grid(wgs, all_groups);
   switch (whole) {
     case 0: return launch_ks<0>(p, kind, grid, lds, stream);
     case 1: return launch_ks<1>(p, kind, grid, lds, stream);

@@ -327,7 +327,9 @@ bool conv_windows_applicable(const ConvArgs &c, int kind) {
 #else
   const bool c_ok = c_bytes % 16 != 0;
 #endif
-  return c.f % 16 == 0 && c.f / 64 < 65535 && c_ok && uint64_t(c.fh) * seg_padded <= 64 * (kind == 3 ? MAX_KS_F32 : MAX_KS) &&
+  // (the pixel form holds no windows: bf16 7 x 7 over four channels, 392 bytes, 13 x 4 -> 64 x 192^2 240 us unfolded, 28 there)
+  return c.f % 16 == 0 && c.f / 64 < 65535 && c_ok &&
+         (uint64_t(c.fh) * seg_padded <= 64 * (kind == 3 ? MAX_KS_F32 : MAX_KS) || conv_pixels_applicable(c, kind)) &&
          uint64_t(c.b) * ((c.oh + TILE_H - 1) / TILE_H) * ((c.ow + TILE_W - 1) / TILE_W) < (1ull << 31) &&
          (reinterpret_cast<uintptr_t>(c.out) & (c.out_planes ? 3 : 15)) == 0 && (reinterpret_cast<uintptr_t>(c.image) & (es - 1)) == 0 &&
          (reinterpret_cast<uintptr_t>(c.filters) & (es - 1)) == 0;

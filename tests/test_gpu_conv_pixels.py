@@ -68,3 +68,31 @@ def test_three_and_four_channels(gpu, shape, accum, types):
         assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
         ok = np.isfinite(want)
         assert not ok.any() or float(np.abs(got[ok].astype(np.float64) - want[ok]).max() / np.abs(want[ok]).max()) < 1e-5
+
+
+@pytest.mark.parametrize("types", ["u8", "i8", "bf16"])
+@pytest.mark.parametrize("fh,fw", [(1, 3), (2, 2), (3, 3), (4, 5), (5, 5), (6, 4), (7, 7), (7, 3), (3, 7)])
+@pytest.mark.parametrize("f,c", [(16, 3), (32, 4), (48, 3), (96, 4)])
+def test_filters_in_registers(gpu, types, fh, fw, f, c):
+    """Every number of filter rows that stays in registers, whole steps and tails, whole cache lines of the output and not; an
+    infinity and a NaN in a bf16 image reach the outputs whose windows hold them and no others."""
+    dts, codes = TYPES[types]
+    b, oh, ow = 2, 21, 37
+    shape = [b, f, c, oh, ow, fh, fw]
+    gen = {M.u8: synth.uniform_u8, M.i8: synth.uniform_i8, M.bf16: synth.normal_bf16}
+    img, filt = gen[dts[0]](161, 0, (b, oh + fh - 1, ow + fw - 1, c)), gen[dts[1]](161, 1, (f, fh, fw, c))
+    if types == "bf16":
+        img = img.copy()
+        img[0, 0, 0, 0], img[1, oh // 2, ow // 2, 1] = 0x7f80, 0x7fc0
+    out0 = synth.uniform_u8(161, 2, (b, oh, ow, f)).astype(np.float32 if types == "bf16" else np.int32) - 100
+    for accum in (False, True):
+        spec = M.Conv(shape, dts, accum=accum)
+        assert spec.plan().kernels == ["k_conv_windows"]
+        got = run_spec(spec, [img, filt, out0])
+        want = orc.conv(shape, codes, img, filt, out0.copy(), accum, layouts=[NHWC] * 3)
+        if types != "bf16":
+            assert np.array_equal(got, want)
+            continue
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        ok = np.isfinite(want)
+        assert float(np.abs(got[ok].astype(np.float64) - want[ok]).max() / np.abs(want[ok]).max()) < 1e-5
