@@ -12,9 +12,8 @@ namespace mrl {
 namespace {
 using gemm::v4i;
 
-// Rows of B per wavefront (up to four rows of A) and steps of K in flight: two and four measured
-// fastest (bf16 1 x 2048 x 16384: 10.5 us; four rows and two steps 12.4, eight rows 13.3, one row
-// 11.2); the switches are for such measurements.
+// Rows of B per wavefront (launch_rows says where one is taken) and steps of K in flight: two and four measured fastest where B comes
+// from memory (bf16 1 x 8192 x 8192 23.7 us; four rows 32.1). The switches are for such measurements.
 #ifndef MRL_GEMV_MAX_M
 #define MRL_GEMV_MAX_M 8
 #endif
@@ -60,8 +59,8 @@ __device__ inline typename Acc<KIND>::type dot16(v4i a, v4i b, typename Acc<KIND
   return acc;
 }
 
-// COLS: output columns (rows of B) per wavefront, all in flight together.
-template <int KIND, int ROWS, int COLS>
+// COLS: output columns (rows of B) per wavefront, all in flight together.  PAST: B is read past the caches.
+template <int KIND, int ROWS, int COLS, bool PAST>
 __global__ __launch_bounds__(64 * WAVES) void k_gemv(GemmArgs g) {
   typedef typename Acc<KIND>::type acc_t;
   constexpr int ES = KIND == 3 ? 4 : KIND == 2 ? 2 : 1;
@@ -92,7 +91,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemv(GemmArgs g) {
   for (int kb = lane * 16; kb < k_bytes; kb += 64 * 16) {
     v4i bv[COLS], av[ROWS];
 #pragma unroll
-    for (int c = 0; c < COLS; c++) bv[c] = __builtin_nontemporal_load((const v4i *)(b_row[c] + kb));
+    for (int c = 0; c < COLS; c++) bv[c] = PAST ? __builtin_nontemporal_load((const v4i *)(b_row[c] + kb)) : *(const v4i *)(b_row[c] + kb);
 #pragma unroll
     for (int r = 0; r < ROWS; r++) {
       av[r] = *(const v4i *)(a_row[r] + kb);
@@ -139,24 +138,27 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemv(GemmArgs g) {
       }
 }
 
-template <int KIND, int ROWS, int COLS>
+template <int KIND, int ROWS, int COLS, bool PAST = true>
 hipError_t launch_as(const GemmArgs &g, hipStream_t stream) {
   const dim3 grid(uint32_t((uint64_t(g.n) + COLS * WAVES - 1) / (COLS * WAVES)), g.batch), block(64 * WAVES);
   constexpr int ES = KIND == 3 ? 4 : KIND == 2 ? 2 : 1;
   plan::work(plan::UNIT_STREAM, 2.0 * g.m * g.n * g.k * g.batch,
              double(g.batch) * ((double(g.m) + g.n) * g.k * ES + (g.c_bf16 ? 2.0 : 4.0) * g.m * g.n));
-  MRL_LAUNCH((k_gemv<KIND, ROWS, COLS>), grid, block, 0, stream, g);
+  MRL_LAUNCH((k_gemv<KIND, ROWS, COLS, PAST>), grid, block, 0, stream, g);
   return mrl::plan::last_error();
 }
 
 template <int KIND>
 hipError_t launch_rows(const GemmArgs &g, hipStream_t stream) {
-  // One row of B per wavefront once B is some 200 MB (bf16 1 x 4096 x 32768: 39.6 us against 42.3
-  // with two; at 134 MB the same, at 67 MB 11.2 against 10.6).
-  constexpr int ES = KIND == 3 ? 4 : KIND == 2 ? 2 : 1;
-  if (g.m == 1 && double(g.n) * g.k * ES * g.batch >= 200e6) return launch_as<KIND, 1, 1>(g, stream);
-  if (g.m == 1) return launch_as<KIND, 1, MRL_GEMV_COLS>(g, stream);
-  if (g.m == 2) return launch_as<KIND, 2, MRL_GEMV_COLS>(g, stream);
+  // A B that the memory-side cache holds beside others stays there for the next launch, and goes one row to a wavefront; a larger one
+  // is streamed past it, two rows to a wavefront and one from some 200 MB on (us, buffers taking turns, one row through / two past: bf16 1 x 2048 x 16384, 67 MB, 11.4 / 12.3,
+  // u8 2 x 8192 x 8192 11.5 / 15.6, bf16 2 x 5056 x 5122 9.7 / 11.1; 2 x 10688 x 5120, 109 MB, 23.9 / 22.9; 100 MB in rows of no whole KB, one row past / two: 2 x 6528 x 7726 23.2 / 18.0).
+  const double bytes = double(g.n) * g.k * (KIND == 3 ? 4 : KIND == 2 ? 2 : 1) * g.batch;
+  if (g.m == 1) {
+    if (bytes <= 80e6) return launch_as<KIND, 1, 1, false>(g, stream);
+    return bytes >= 200e6 ? launch_as<KIND, 1, 1>(g, stream) : launch_as<KIND, 1, MRL_GEMV_COLS>(g, stream);
+  }
+  if (g.m == 2) return bytes <= 80e6 ? launch_as<KIND, 2, 1, false>(g, stream) : launch_as<KIND, 2, MRL_GEMV_COLS>(g, stream);
   if (g.m <= 4) return launch_as<KIND, 4, MRL_GEMV_COLS>(g, stream);
   return launch_as<KIND, MAX_ROWS, 2>(g, stream);
 }
