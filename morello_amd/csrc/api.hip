@@ -779,13 +779,15 @@ int run_conv(const mrl_spec &s, void *const *params, Workspace &ws) {
     // needs no window arithmetic: its image is the left operand of a plain Matmul, below.)
     // Few output tiles and long windows (deep layers on small images): slices of the window as
     // batch entries with partial results, summed in slice order, as for a Matmul.
-    const uint32_t splits = forced == 2 ? 1 : mrl::gemm_k_splits(conv_args, kind);
+    uint32_t slice_k = 0;
+    const uint32_t splits = forced == 2 ? 1 : mrl::conv_k_slices(conv_args, kind, &slice_k);
     if (splits > 1) {
       void *partial = nullptr;
       HIP_TRY(ws.alloc(&partial, size_t(splits) * conv_args.m * conv_args.n * 4));
       mrl::GemmArgs slices = conv_args;
-      slices.batch = splits, slices.k = conv_args.k / splits;
+      slices.batch = splits, slices.k = slice_k;
       slices.sb = int64_t(slices.k), slices.conv.slice_bytes = uint32_t(slices.k * img.elem);
+      slices.conv.window_bytes = uint32_t(conv_args.k * img.elem);
       slices.c = partial, slices.ldc = conv_args.n, slices.sc = int64_t(conv_args.m) * conv_args.n, slices.accum = 0;
       HIP_TRY(mrl::launch_conv_gemm(slices, kind, ws.stream, 64));
       HIP_TRY(mrl::launch_sum_splits(partial, conv_args.c, splits, conv_args.m, conv_args.n, conv_args.ldc,

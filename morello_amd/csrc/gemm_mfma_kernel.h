@@ -430,13 +430,15 @@ __global__ __launch_bounds__(TL::NT) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
   for (int tn = 0; tn < TN; tn++) colsum[tn] = 0;
 
   v4i a_reg[A_CH], b_reg[B_CH];
-  const int kt_count = int((g.k + BK - 1) / BK);
+  // K of this entry: a Conv's last slice of the windows may be a shorter one.
+  const int k = CONV && g.conv.slice_bytes != 0 ? int(min(g.conv.slice_bytes, g.conv.window_bytes - blockIdx.y * g.conv.slice_bytes)) / ES : int(g.k);
+  const int kt_count = (k + BK - 1) / BK;
   // EDGE bookkeeping.  The tiles are addressed relative to `a_tile` / `b_tile` (wave-uniform,
   // advanced by one k step per load) with per-thread 32-bit offsets; what lies past the last
   // row of the tile is out of the resource's range.  The end of K inside a row is not (the
   // next row follows), so a thread whose chunk starts at or past K asks for the
   // out-of-range offset instead.
-  const int k_bytes = int(g.k) * ES;
+  const int k_bytes = k * ES;
   const uint8_t *a_tile = A, *b_tile = B;
   const int a_rows = min(BM, int(g.m - m0)), b_rows = min(BN, int(g.n - n0));  // rows the tile owns
   const uint32_t a_off = uint32_t(tid / A_ROW_CH) * uint32_t(lda_b) + (tid % A_ROW_CH) * 16;

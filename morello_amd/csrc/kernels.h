@@ -151,7 +151,8 @@ struct GemmArgs {
     uint64_t image_bytes;   // all of `a`
     // K shared out over batch entries (each a slice of the windows, a partial result of its own):
     // bytes of a window a slice starts behind the previous one; 0 = one entry, the whole window.
-    uint32_t slice_bytes;
+    // `k` is then that of a whole slice, and the last entry has what is left of window_bytes.
+    uint32_t slice_bytes, window_bytes;
     // Filled in by launch_conv_gemm: the divisions of the window arithmetic.
     FastDiv by_ow, by_oh, by_c_bytes, by_fw;
   } conv = {};
@@ -175,6 +176,9 @@ uint32_t gemm_tile_side(const GemmArgs &g, int kind);
 // A single Matmul with few output tiles and a long K runs as `splits` batch entries over slices
 // of K whose partial results are summed afterwards (1: as it is).  The slices are whole k steps.
 uint32_t gemm_k_splits(const GemmArgs &g, int kind, uint32_t *remainder = nullptr);
+// The same for a Conv as an implicit Matmul, whose kernel takes a shorter last slice: the number of
+// slices, each of *slice_k elements but the last.
+uint32_t conv_k_slices(const GemmArgs &g, int kind, uint32_t *slice_k);
 // c[r][col] (+)= sum over s of partial[s][r][col]; partial is dense [splits][m][n], 32-bit
 // elements (int32 when `integers`, else f32), summed in order of s; c holds the same, or bf16.
 hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint32_t m, uint32_t n, int64_t ldc,
