@@ -467,6 +467,26 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     HIP_TRY(mrl::launch_gemm_skinny(g, kind, ws.stream));
     return finish_output(c, ws);
   }
+  // Rows that are not whole 16-byte chunks, in a problem small enough that copies of them would be a third of its time: read
+  // in place too.
+  const int64_t chunk = 16 / int64_t(a.elem);
+  if (!sched && rows && (g.lda % chunk != 0 || g.sa % chunk != 0 || g.ldb % chunk != 0 || g.sb % chunk != 0) && mrl::gemm_ring_rows_columns(g, kind)) {
+    uint32_t slice_k = 0;
+    const uint32_t splits = mrl::uneven_k_slices(g, kind, false, &slice_k);
+    if (splits == 1) {
+      HIP_TRY(mrl::launch_gemm_ring_rows(g, kind, ws.stream));
+    } else {
+      void *partial = nullptr;
+      HIP_TRY(ws.alloc(&partial, size_t(splits) * g.m * g.n * 4));
+      mrl::GemmArgs slices = g;
+      slices.batch = splits, slices.k = slice_k, slices.k_total = g.k;
+      slices.sa = slice_k, slices.sb = g.b_kmajor ? int64_t(slice_k) : int64_t(slice_k) * g.ldb;
+      slices.c = partial, slices.ldc = g.n, slices.sc = int64_t(g.m) * g.n, slices.accum = 0, slices.c_bf16 = false;
+      HIP_TRY(mrl::launch_gemm_ring_rows(slices, kind, ws.stream));
+      HIP_TRY(mrl::launch_sum_splits(partial, g.c, splits, g.m, g.n, g.ldc, g.accum != 0, kind <= 1, g.c_bf16, ws.stream));
+    }
+    return finish_output(c, ws);
+  }
   // Operands the matrix-core kernels cannot walk in place are copied with the strided Move
   // first when that opens the fast path: A or C stored column-major becomes row-major, and rows
   // that are not whole 16-byte chunks (K or N not a multiple of 16 bytes) are padded with zeros
@@ -780,14 +800,13 @@ int run_conv(const mrl_spec &s, void *const *params, Workspace &ws) {
     // Few output tiles and long windows (deep layers on small images): slices of the window as
     // batch entries with partial results, summed in slice order, as for a Matmul.
     uint32_t slice_k = 0;
-    const uint32_t splits = forced == 2 ? 1 : mrl::conv_k_slices(conv_args, kind, &slice_k);
+    const uint32_t splits = forced == 2 ? 1 : mrl::uneven_k_slices(conv_args, kind, true, &slice_k);
     if (splits > 1) {
       void *partial = nullptr;
       HIP_TRY(ws.alloc(&partial, size_t(splits) * conv_args.m * conv_args.n * 4));
       mrl::GemmArgs slices = conv_args;
-      slices.batch = splits, slices.k = slice_k;
+      slices.batch = splits, slices.k = slice_k, slices.k_total = conv_args.k;
       slices.sb = int64_t(slices.k), slices.conv.slice_bytes = uint32_t(slices.k * img.elem);
-      slices.conv.window_bytes = uint32_t(conv_args.k * img.elem);
       slices.c = partial, slices.ldc = conv_args.n, slices.sc = int64_t(conv_args.m) * conv_args.n, slices.accum = 0;
       HIP_TRY(mrl::launch_conv_gemm(slices, kind, ws.stream, 64));
       HIP_TRY(mrl::launch_sum_splits(partial, conv_args.c, splits, conv_args.m, conv_args.n, conv_args.ldc,

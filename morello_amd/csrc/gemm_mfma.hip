@@ -110,24 +110,27 @@ uint32_t gemm_k_splits(const GemmArgs &g, int kind, uint32_t *remainder) {
   return uint32_t(want);
 }
 
-uint32_t conv_k_slices(const GemmArgs &g, int kind, uint32_t *slice_k) {
+uint32_t uneven_k_slices(const GemmArgs &g, int kind, bool conv, uint32_t *slice_k) {
   // The slices need not be equal: windows are rarely a whole number of steps (5 x 5 over 272 bf16
   // channels: 106 and a quarter) or one with a divisor near the wanted count (3 x 3 over 352 int8
   // channels: 25), and in one piece a chain of 107 steps took 40.8 us on four tiles; in twelve
   // slices 8.3.
-  const uint64_t es = elem_size_of(kind);
-  const uint64_t steps = (uint64_t(g.k) * es + 127) / 128;
+  const uint64_t es = elem_size_of(kind), k_bytes = uint64_t(g.k) * es;
+  const uint64_t steps = (k_bytes + 127) / 128;
   const uint64_t tiles = uint64_t((g.m + 63) / 64) * ((g.n + 63) / 64);
   if (g.batch != 1 || tiles >= 384 || steps < 16) return 1;
-  const uint64_t wanted = std::min<uint64_t>({32, 768 / tiles, steps / 8});
-  const uint64_t per = (steps + wanted - 1) / wanted, count = (steps + per - 1) / per;
+  const uint64_t wanted = std::max<uint64_t>(1, std::min<uint64_t>({32, (conv ? 768 : 256) / tiles, steps / 8}));
+  uint64_t per = (steps + wanted - 1) / wanted;
+  while (k_bytes % (per * 128) != 0 && k_bytes % (per * 128) <= 128) per++;   // (gemm_ring_rows.hip wants two steps or more)
+  const uint64_t count = (steps + per - 1) / per;
   if (count <= 1) return 1;
-  // As in gemm_k_splits, with the step of each type (a chain of 66 int8 steps 30 us, of 107 bf16
+  // (Rows that start anywhere: one workgroup a compute unit, 292 x 6007 x 2192 bf16 in halves, 350 of them, 43.6 us, whole 35.)
+  // As in gemm_k_splits, with the step of each kernel and type (Conv: a chain of 66 int8 steps 30 us, of 107 bf16
   // steps 40) and the partials' traffic at the 3 TB/s that a sum of a few MB reaches: 2 x (48 -> 144) x 43^2 5 x 5
   // bf16, 174 tiles of 19 steps, 9.7 us whole, 11.4 in halves; 3 x (144 -> 128) x 34^2 3 x 3, 110
   // of 21, 10.2 and 11.1; 10 x (80 -> 64) x 19^2 5 x 5, 57 of 32, 14.2 and 9.5 in four.
-  const double spread = std::min<double>(double(count), 384.0 / double(tiles));
-  const double saved_us = double(steps) * (1.0 - 1.0 / spread) * (kind == 2 ? 0.36 : 0.46);
+  const double spread = std::min<double>(double(count), (conv ? 384.0 : 256.0) / double(tiles));
+  const double saved_us = double(steps) * (1.0 - 1.0 / spread) * (!conv ? 0.28 : kind == 2 ? 0.36 : 0.46);
   const double cost_us = 2.2 + (double(count) + 1.0) * double(g.m) * double(g.n) * 4.0 / 3.0e6;
   if (spread <= 1.0 || saved_us < 1.2 * cost_us) return 1;
   *slice_k = uint32_t(per * 128 / es);

@@ -431,7 +431,7 @@ __global__ __launch_bounds__(TL::NT) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
 
   v4i a_reg[A_CH], b_reg[B_CH];
   // K of this entry: a Conv's last slice of the windows may be a shorter one.
-  const int k = CONV && g.conv.slice_bytes != 0 ? int(min(g.conv.slice_bytes, g.conv.window_bytes - blockIdx.y * g.conv.slice_bytes)) / ES : int(g.k);
+  const int k = CONV && g.k_total != 0 ? int(min(g.k, g.k_total - blockIdx.y * g.k)) : int(g.k);
   const int kt_count = (k + BK - 1) / BK;
   // EDGE bookkeeping.  The tiles are addressed relative to `a_tile` / `b_tile` (wave-uniform,
   // advanced by one k step per load) with per-thread 32-bit offsets; what lies past the last

@@ -20,49 +20,16 @@
 // rows that one half of a wave reads at once lie in different banks.  Loads fill LDS in order, so
 // the swizzles are applied to the addresses in memory.
 // Semantics: morello/src/spec.rs:480-485; integers exact, bf16 summed in f32.
-#include <algorithm>
-
-#include "gemm_mfma_kernel.h"
+#include "gemm_ring.h"
 
 namespace mrl {
 namespace {
-using gemm::BF16;
-using gemm::I8;
-using gemm::v2i;
-using gemm::v4i;
-using gemm::v8bf;
+using namespace ring;
 using gemm::TileWalk;
-typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr uint32_t OUTSIDE = 0x80000000u;   // an offset no resource here holds
-constexpr int BM = 128, STEP = 128, WAVES = 8;   // bytes of K a step: two MFMAs deep, one for each half of the waves
-
-template <class T> struct Ring;
-template <> struct Ring<I8> {
-  typedef v4i Acc;
-  __device__ static Acc mfma(v4i a, v4i b, Acc c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }
-};
-template <> struct Ring<BF16> {
-  typedef v4f Acc;
-  __device__ static Acc mfma(v4i a, v4i b, Acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-  }
-};
-
-// Byte position of a row-major B's piece-and-rest `byte` of k row r <-> in memory (an involution).  Rows
-// of BN elements; a row's place relative to the 256 bytes of a bank line repeats every 256 / (pitch % 256).
-template <class T, int BN>
-__device__ inline int swizzle(int byte, int r) {
-  constexpr int PITCH = BN * T::ES, PIECE = 16 * T::ES;
-  // the bits of the row number that tell apart the rows half a wave reads at once: bf16 r & 3 and bit 3, int8 r & 7 and bit 4
-  const int rows = T::ES == 2 ? (r & 3) | ((r >> 3) & 1) << 2 : (r & 7) | ((r >> 4) & 1) << 3;
-  constexpr int OFF = PITCH % 256;   // 0: all rows start in the same bank; 128 (64, 192): the low bit (two bits) of the row already moves it
-  constexpr int MOVED = OFF == 0 ? 0 : OFF % 128 == 0 ? 1 : OFF % 64 == 0 ? 2 : 3;
-  constexpr int PIECES = (256 >> MOVED) / PIECE;   // of a group to exchange within
-  const int x = (rows >> MOVED) & (PIECES - 1);
-  return ((byte / PIECE) ^ x) * PIECE + byte % PIECE;
-}
+constexpr int BM = 128;
 
 // One load of 64 lanes x 16 bytes into the KiB at LDS address `lds_addr` + AT (wave-uniform), lane l to the l-th
 // 16 bytes; the instruction's offset AT is added to the address in memory too, so callers take it off
@@ -82,20 +49,9 @@ __device__ inline void wait_for_all_but() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 
-constexpr int min_of(int a, int b) { return a < b ? a : b; }
-// f(0), ..., f(N - 1) with the number as a type
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void each(F &&f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    each<N, I + 1>(f);
-  }
-}
-
 template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RB, int SLOTS>
 __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_WALK_PARAMS, GemmArgs g) {
   typedef typename Ring<T>::Acc Acc;
-  typedef typename T::Out Out;
   constexpr int ES = T::ES, BK = STEP / ES, RA = 4, BN = 32 * RB, WM = 64, WN = 16 * RB;
   constexpr int A_BYTES = BM * STEP, B_BYTES = BN * STEP, SLOT = A_BYTES + B_BYTES;
   constexpr int A_LOADS = A_BYTES / (1024 * WAVES), B_LOADS = (B_BYTES / 1024 + WAVES - 1) / WAVES, LOADS = A_LOADS + B_LOADS;   // a wave's, per step
@@ -247,75 +203,7 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
   if (steps & 1) each<RA * RB>([&](auto q) { multiply(even, q); });
   wait_for_all_but<0>();   // (requests past the last step write zeros)
 
-  // C.  Register i of a block: row 4 (l / 16) + i, column l % 16.  A wave's block row goes through its own
-  // piece of LDS and leaves in whole rows of WN columns.
-  if (A_UNSIGNED)
-#pragma unroll
-    for (int c = 0; c < RB; c++) {
-      colsum[c] += __shfl_xor(colsum[c], 16);
-      colsum[c] += __shfl_xor(colsum[c], 32);
-      colsum[c] *= 128;
-    }
-  constexpr int ROW = WN + 4;
-  Out *piece = (Out *)lds + (wave & 3) * (WM * ROW);
-  const int64_t row_first = m0 + wm * WM, col_first = n0 + wn * WN;
-  const int cols = int(min(int64_t(WN), int64_t(g.n) - col_first));
-  // (The loops stay loops: code that a launch runs once is fetched from memory, and unrolled it took longer to
-  // fetch than to run.)
-  auto store = [&](auto *C) {
-    typedef std::remove_pointer_t<decltype(C)> Stored;
-    typedef Stored four __attribute__((ext_vector_type(4)));
-    typedef Out out4 __attribute__((ext_vector_type(4)));
-    C += int64_t(blockIdx.y) * g.sc + row_first * g.ldc + col_first;
-    const int rows = int(min(int64_t(WM), int64_t(g.m) - row_first));
-    // four columns at a time where all of a row's are whole and aligned
-    if (cols % 4 == 0 && g.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % (4 * sizeof(Stored)) == 0) {
-#pragma unroll 4
-      for (int e = 0; e < WM * WN / 4 / 128; e++) {
-        const int at = (2 * e + kw) * 64 + lane, row = at / (WN / 4), col = at % (WN / 4) * 4;
-        if (row < rows && col < cols) {
-          out4 v = *(const out4 *)(piece + row * ROW + col);
-          four *d = (four *)(C + int64_t(row) * g.ldc + col);
-          if (g.accum) v += __builtin_convertvector(*d, out4);
-          *d = __builtin_convertvector(v, four);
-        }
-      }
-    } else {
-#pragma unroll 4
-      for (int e = 0; e < WM * WN / 128; e++) {
-        const int at = (2 * e + kw) * 64 + lane, row = at / WN, col = at % WN;
-        if (row < rows && col < cols) {
-          Out v = piece[row * ROW + col];
-          Stored *d = C + int64_t(row) * g.ldc + col;
-          if (g.accum) v += Out(*d);
-          *d = Stored(v);
-        }
-      }
-    }
-  };
-  // The two halves of K: the upper waves' sums through LDS onto the lower waves', and both store.
-  auto for_each_sum = [&](auto f) {
-#pragma unroll
-    for (int r = 0; r < RA; r++)
-#pragma unroll
-      for (int c = 0; c < RB; c++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          Out v = acc[r][c][i];
-          if (A_UNSIGNED) v += Out(colsum[c]);
-          f(piece[(r * 16 + 4 * lg + i) * ROW + c * 16 + li], v);
-        }
-  };
-  if (kw) for_each_sum([](Out &at, Out v) { at = v; });
-  __syncthreads();
-  if (!kw) for_each_sum([](Out &at, Out v) { at = v + at; });
-  __syncthreads();
-  if (cols > 0 && row_first < int64_t(g.m)) {
-    if constexpr (std::is_same<T, BF16>::value) {
-      if (g.c_bf16) store((__bf16 *)g.c);
-      else store((Out *)g.c);
-    } else store((Out *)g.c);
-  }
+  store_tile<T, A_UNSIGNED, RA, RB>(g, lds, acc, colsum, m0, n0, 0);
 }
 
 template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RB, int SLOTS>

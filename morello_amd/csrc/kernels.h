@@ -140,6 +140,9 @@ struct GemmArgs {
   // false: B rows run along N (`ldb` = elements between k rows); true: B rows run along K
   // (`ldb` = elements between n rows), as col_major / layout![0,2,1] store it.
   bool b_kmajor = false;
+  // K shared out over batch entries: each has `k` elements, the last what is left of k_total (0: `k` each).  The
+  // Conv build of k_gemm and gemm_ring_rows.hip take it.
+  uint32_t k_total = 0;
   // C is bf16 (bf16 operands only): the f32 sum, the old value included, is rounded once.
   bool c_bf16 = false;
   // Conv as an implicit Matmul (the CONV build of the kernel): `a` is a channels-last image
@@ -151,8 +154,7 @@ struct GemmArgs {
     uint64_t image_bytes;   // all of `a`
     // K shared out over batch entries (each a slice of the windows, a partial result of its own):
     // bytes of a window a slice starts behind the previous one; 0 = one entry, the whole window.
-    // `k` is then that of a whole slice, and the last entry has what is left of window_bytes.
-    uint32_t slice_bytes, window_bytes;
+    uint32_t slice_bytes;
     // Filled in by launch_conv_gemm: the divisions of the window arithmetic.
     FastDiv by_ow, by_oh, by_c_bytes, by_fw;
   } conv = {};
@@ -176,9 +178,9 @@ uint32_t gemm_tile_side(const GemmArgs &g, int kind);
 // A single Matmul with few output tiles and a long K runs as `splits` batch entries over slices
 // of K whose partial results are summed afterwards (1: as it is).  The slices are whole k steps.
 uint32_t gemm_k_splits(const GemmArgs &g, int kind, uint32_t *remainder = nullptr);
-// The same for a Conv as an implicit Matmul, whose kernel takes a shorter last slice: the number of
-// slices, each of *slice_k elements but the last.
-uint32_t conv_k_slices(const GemmArgs &g, int kind, uint32_t *slice_k);
+// The same for the kernels that take a shorter last slice (k_total): the number of slices, each of *slice_k elements but the
+// last.  conv: an implicit Matmul, else rows that start anywhere.
+uint32_t uneven_k_slices(const GemmArgs &g, int kind, bool conv, uint32_t *slice_k);
 // c[r][col] (+)= sum over s of partial[s][r][col]; partial is dense [splits][m][n], 32-bit
 // elements (int32 when `integers`, else f32), summed in order of s; c holds the same, or bf16.
 hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint32_t m, uint32_t n, int64_t ldc,
@@ -190,6 +192,10 @@ hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint
 // gemm_possible() takes with edge_addressable() leading dimensions.  gemm_ring_columns: the width for a problem, 0 for none.
 uint32_t gemm_ring_columns(const GemmArgs &g, int kind);
 hipError_t launch_gemm_ring(const GemmArgs &g, int kind, uint32_t bn, hipStream_t stream);
+// gemm_ring_rows.hip: such tiles for rows that start anywhere (K or N no whole 16-byte chunks), operands read in place.
+// gemm_ring_rows_columns: the width of its tiles for a problem, 0 for none.
+uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind);
+hipError_t launch_gemm_ring_rows(const GemmArgs &g, int kind, hipStream_t stream);
 // gemm_wide_edge.hip: the four-wave tile on ragged shapes and against a k-fastest B.
 hipError_t launch_gemm_wide_edge(const GemmArgs &g, int kind, hipStream_t stream);
 hipError_t launch_gemm_big(const GemmArgs &g, int kind, hipStream_t stream, uint32_t staging = 0);
