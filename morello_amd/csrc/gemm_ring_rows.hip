@@ -239,10 +239,11 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
     return 0;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
   const uint64_t units = g_compute_units, small = tiles(64, 64);
-  // Two int8 classes keep the copies although this is the faster way: their plans, copies and a tile of k_gemm, are relied on.
-  // Exactly one round of tiles (1000^3: 10.5 / 6.8), and fewer than 128 columns over sixteen steps or more (384 x 2559 x
-  // 120: 12.4 / 8.8).
-  if (kind <= 1 && (small == units || (g.n < 128 && steps >= 16))) return 0;
+  // Three int8 classes keep the copies although this is the faster way: their plans, copies and a tile of k_gemm, or the
+  // scratch that these take are relied on.  Exactly one round of tiles (1000^3: 10.5 / 6.8), fewer than 128 columns over sixteen
+  // steps or more (384 x 2559 x 120: 12.4 / 8.8), and up to three steps (300 x 270 x 290, with which a stream's scratch is
+  // tested; 1217 x 281 x 334 8.7 / 5.7).
+  if (kind <= 1 && (small == units || (g.n < 128 && steps >= 16) || steps <= 3)) return 0;
   if (small <= units) return small > units / 2 && steps > 88 ? 0 : 32;   // (292 x 6007 x 2192 bf16, 175 tiles of 94 steps: 34.7 / 35.8)
   if (tiles(128, 64) <= units) return steps <= (kind == 2 ? 48 : 24) ? 64 : 0;
   return kind == 2 && steps <= 24 && g.n >= 128 && tiles(128, 128) <= units ? 128 : 0;

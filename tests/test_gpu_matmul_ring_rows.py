@@ -31,14 +31,16 @@ def _check(got, A, B, C, accum, dts):
 @pytest.mark.parametrize("nk", [False, True])
 @pytest.mark.parametrize("types", list(TYPES))
 @pytest.mark.parametrize("b,m,k_bytes,n,accum,families", [
-    (1, 1900, 2 * 128 + 2, 487, False, 1),    # one element in the first step
-    (1, 900, 2 * 128 - 2, 1025, True, 1),     # one short of two whole steps
+    (1, 1900, 3 * 128 + 2, 487, False, 1),   # one element in the first step
+    (1, 900, 4 * 128 - 2, 1025, True, 1),    # one short of four whole steps
     (3, 65, 9 * 128 + 6, 707, False, 1),     # a row past a tile, three columns of the last one its own
     (2, 384, 5 * 128 + 62, 577, True, 1),    # whole tiles in m; one column
     (1, 191, 40 * 128 + 34, 133, False, 2),  # slices of K, the last one shorter
     (1, 100, 33 * 128 + 18, 250, True, 2),   # ... the old values added in the sum
     (2, 641, 6 * 128 + 14, 1027, True, 1),   # tiles of 128 x 64
     (1, 1283, 8 * 128 + 30, 1021, False, 1),
+    (1, 461, 15 * 128, 656, True, 1),        # rows of whole chunks
+    (2, 200, 9 * 128 + 16, 336, False, 1),
 ])
 def test_rows_that_start_anywhere(gpu, b, m, k_bytes, n, accum, families, types, nk):
     dts = TYPES[types]
@@ -66,7 +68,7 @@ def test_rows_that_start_anywhere(gpu, b, m, k_bytes, n, accum, families, types,
 
 
 @pytest.mark.parametrize("nk", [False, True])
-@pytest.mark.parametrize("types,m,k,n", [("bf16", 1411, 733, 1555), ("bf16_out", 1300, 1501, 2049), ("bf16_out", 1153, 201, 1861)])
+@pytest.mark.parametrize("types,m,k,n", [("bf16", 1411, 733, 1555), ("bf16_out", 1300, 1501, 2049), ("bf16_out", 1153, 201, 1861), ("bf16", 1153, 65, 1861)])
 def test_tiles_of_128_columns(gpu, types, m, k, n, nk):
     dts = TYPES[types]
     A, B = synth.normal_bf16(182, 0, (1, m, k)), synth.normal_bf16(182, 1, (1, k, n))
