@@ -468,9 +468,16 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     return finish_output(c, ws);
   }
   // Rows that are not whole 16-byte chunks, in a problem small enough that copies of them would be a third of its time: read
-  // in place too.
+  // in place too.  And any rows where its smallest tile steps through K faster than k_gemm's (0.25 to 0.33 us against 0.4 to 0.5:
+  // u8 1144 x 3952 x 672 16.2 / 13.6, bf16 221 x 1824 x 624 twice 12.9 / 11.2; up to eight steps they are even), unless K falls
+  // into equal slices, of which k_gemm's may go three to a compute unit (bf16 1721 x 4416 x 304 15.4 / 21.0), or is long beside
+  // int8 rows of N, of which a step takes half lines (139 x 4080 x 2288 twice 22.6 / 23.5).
   const int64_t chunk = 16 / int64_t(a.elem);
-  if (!sched && rows && (g.lda % chunk != 0 || g.sa % chunk != 0 || g.ldb % chunk != 0 || g.sb % chunk != 0) && mrl::gemm_ring_rows_columns(g, kind)) {
+  const bool ragged = g.lda % chunk != 0 || g.sa % chunk != 0 || g.ldb % chunk != 0 || g.sb % chunk != 0;
+  const uint32_t in_place = !sched && rows ? mrl::gemm_ring_rows_columns(g, kind) : 0;
+  uint32_t k_left = 0;
+  const bool steps_pay = in_place == 32 && uint64_t(g.k) * a.elem > 8 * 128 && (kind == 2 || g.b_kmajor || g.k <= 24 * 128);
+  if (in_place != 0 && (ragged || (steps_pay && (mrl::gemm_k_splits(g, kind, &k_left) == 1 || k_left != 0)))) {
     uint32_t slice_k = 0;
     const uint32_t splits = mrl::uneven_k_slices(g, kind, false, &slice_k);
     if (splits == 1) {

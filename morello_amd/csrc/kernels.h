@@ -192,7 +192,8 @@ hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint
 // gemm_possible() takes with edge_addressable() leading dimensions.  gemm_ring_columns: the width for a problem, 0 for none.
 uint32_t gemm_ring_columns(const GemmArgs &g, int kind);
 hipError_t launch_gemm_ring(const GemmArgs &g, int kind, uint32_t bn, hipStream_t stream);
-// gemm_ring_rows.hip: such tiles for rows that start anywhere (K or N no whole 16-byte chunks), operands read in place.
+// gemm_ring_rows.hip: such tiles for rows that start anywhere (K or N no whole 16-byte chunks), operands read in place; its
+// smallest, 64 x 64, is also the faster one for whole chunks.
 // gemm_ring_rows_columns: the width of its tiles for a problem, 0 for none.
 uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind);
 hipError_t launch_gemm_ring_rows(const GemmArgs &g, int kind, hipStream_t stream);
