@@ -5,7 +5,7 @@
 // bytes, ~0.45 us each, on four waves, and wants rows that are whole 16-byte chunks.  Here every one of
 // a workgroup's eight waves takes its own share of K (units of 128 bytes, dealt round) for the same
 // RT x CT blocks of 16 x 16 outputs, waits for nobody on the way, and the waves' partial sums
-// meet in LDS once.  Rows may start at any element.
+// meet in LDS once.  Rows may start at any element; those that start on words are read as they lie.
 //   semantics: morello/src/spec.rs:480-485; integers exact, bf16 and f32 summed in f32.
 #include "gemm_mfma_kernel.h"
 #include "row_chunks.h"
@@ -40,38 +40,58 @@ __device__ inline typename Kind<KIND>::Acc mfma(v4i a, v4i b, typename Kind<KIND
   }
 }
 
-// Sixteen bytes of a row of k_bytes, from a multiple of 16 on.  ALIGNED: rows start on 16-byte chunks
-// and K ends on one.  Otherwise they are cut out of the two aligned chunks they lie in: an access
-// that is not aligned runs at a fraction of the rate, and an aligned chunk that holds a valid byte
-// can be read whole wherever the allocation ends.
-template <bool ALIGNED>
+// Sixteen bytes of a row of k_bytes (64 or more), from a multiple of 16 on.  START: what rows start on, K ending on it for 16.
+//   4: an access on a word is nearly as fast as one on a chunk (bf16 13 x 2350 x 15509 15.9 us cut out of two chunks, 14.0;
+//      30 x 2244 x 7224 13.3, 10.4; u8 25 x 1720 x 5536 8.4, 5.6);
+//   1: cut out of the two aligned chunks they lie in: an access that is not on a word runs at a fraction of the
+//      rate (u8 4 x 7095 x 6144 14.5 us, cut 11.3), and an aligned chunk that holds a valid byte can be read whole
+//      wherever the allocation ends.
+typedef int chunk_on_word __attribute__((ext_vector_type(4), aligned(4)));
+template <int START>
 struct Row {
+  typedef v4i Raw;
+  const uint8_t *first;
+  int k_bytes;
+  __device__ void set(const uint8_t *row, int bytes) { first = row, k_bytes = bytes; }
+  // all sixteen inside the row
+  __device__ Raw fetch(int kb) const {
+    if constexpr (START == 16) return *(const v4i *)(first + kb);
+    return __builtin_bit_cast(v4i, *(const chunk_on_word *)(first + kb));
+  }
+  __device__ v4i value(const Raw &r) const { return r; }
+  // those behind the row's end are zeros
+  __device__ v4i tail(int kb) const {
+    const int left = k_bytes - kb;
+    if (left <= 0) return v4i{0, 0, 0, 0};
+    if constexpr (START == 16) return *(const v4i *)(first + kb);
+    // the sixteen that end with the word that holds the row's last byte, and of those the ones asked for
+    const int back = left >= 16 ? 0 : (16 - left) & ~3;
+    const v4i v = __builtin_bit_cast(v4i, *(const chunk_on_word *)(first + kb - back));
+    return left >= 16 ? v : keep_bytes(cut_chunk(v, v4i{0, 0, 0, 0}, uint32_t(back)), left);
+  }
+};
+template <>
+struct Row<1> {
   struct Raw { v4i lo, hi; };
   const uint8_t *first;   // the chunk the row's first byte lies in
   int shift;              // where in that chunk
   int k_bytes;
   __device__ void set(const uint8_t *row, int bytes) {
-    shift = ALIGNED ? 0 : int(uintptr_t(row) & 15);
+    shift = int(uintptr_t(row) & 15);
     first = row - shift, k_bytes = bytes;
   }
-  // all sixteen inside the row
   __device__ Raw fetch(int kb) const {
     Raw r;
     r.lo = *(const v4i *)(first + kb);
-    if constexpr (!ALIGNED) r.hi = *(const v4i *)(first + kb + (shift ? 16 : 0));
+    r.hi = *(const v4i *)(first + kb + (shift ? 16 : 0));
     return r;
   }
-  __device__ v4i value(const Raw &r) const {
-    if constexpr (ALIGNED) return r.lo;
-    return cut_chunk(r.lo, r.hi, uint32_t(shift));
-  }
-  // those behind the row's end are zeros
+  __device__ v4i value(const Raw &r) const { return cut_chunk(r.lo, r.hi, uint32_t(shift)); }
   __device__ v4i tail(int kb) const {
     const int left = k_bytes - kb;
     if (left <= 0) return v4i{0, 0, 0, 0};
     Raw r;
     r.lo = *(const v4i *)(first + kb);
-    if constexpr (ALIGNED) return r.lo;
     r.hi = *(const v4i *)(first + kb + (shift + min(left, 16) > 16 ? 16 : 0));
     return keep_bytes(value(r), left);
   }
@@ -168,7 +188,7 @@ constexpr int skinny_lds() {
 // the wave's own 2 KiB of LDS per block (no barrier: nobody else reads it).  Loads straight in the MFMA's form,
 // sixteen rows to every sixteen lanes, ask the cache for a line per lane: bf16 64 x 4096 x 4096 25 us that way.
 // The next unit is requested as soon as this one has left its registers.
-template <int KIND, bool ALIGNED, int RT, int CT>
+template <int KIND, int START, int RT, int CT>
 __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(GemmArgs g) {
   typedef typename Kind<KIND>::Acc Acc;
   typedef typename Kind<KIND>::Out Out;
@@ -183,7 +203,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(GemmArgs g) {
   // rows lane / 8 and lane / 8 + 8 of each.  Rows past M and columns past N repeat the last one;
   // their results are not stored.
   const int chunk = lane & 7;
-  Row<ALIGNED> src[TILES][2];
+  Row<START> src[TILES][2];
 #pragma unroll
   for (int t = 0; t < TILES; t++)
 #pragma unroll
@@ -219,7 +239,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(GemmArgs g) {
     }
   };
   const int units = k_bytes / UNIT, rest = k_bytes - units * UNIT;
-  typename Row<ALIGNED>::Raw raw[TILES][2];
+  typename Row<START>::Raw raw[TILES][2];
   auto fetch = [&](int u) {
 #pragma unroll
     for (int t = TILES - 1; t >= 0; t--)
@@ -263,7 +283,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_tiny(GemmArgs g) {
   const uint8_t *A = (const uint8_t *)g.a + int64_t(blockIdx.z) * g.sa * ES;
   const uint8_t *B = (const uint8_t *)g.b + int64_t(blockIdx.z) * g.sb * ES;
   const int k_bytes = int(g.k) * ES;
-  Row<false> a_row[RT];
+  Row<1> a_row[RT];
   Col<ES> b_col[CT];
 #pragma unroll
   for (int t = 0; t < RT; t++) a_row[t].set(A + min(row0 + t * 16 + in16, int64_t(g.m) - 1) * (g.lda * ES), k_bytes);
@@ -312,9 +332,9 @@ void declare_work(const GemmArgs &g) {
              800.0 + 400.0 * double(uint64_t(g.k) * ES / (UNIT * WAVES)));
 }
 
-template <int KIND, bool ALIGNED, int RT, int CT>
+template <int KIND, int START, int RT, int CT>
 hipError_t launch_skinny(const GemmArgs &g, hipStream_t stream) {
-  constexpr auto kern = k_gemm_skinny<KIND, ALIGNED, RT, CT>;
+  constexpr auto kern = k_gemm_skinny<KIND, START, RT, CT>;
   static std::atomic<uint64_t> lds_limit_set{0};
   if (!plan::recording() && skinny_lds<RT, CT>() > 65536) {
     hipError_t e = raise_lds_limit(lds_limit_set, (const void *)kern, skinny_lds<RT, CT>());
@@ -322,31 +342,32 @@ hipError_t launch_skinny(const GemmArgs &g, hipStream_t stream) {
   }
   declare_work<KIND, RT, CT>(g);
   const dim3 grid((g.n + 16 * CT - 1) / (16 * CT), (g.m + 16 * RT - 1) / (16 * RT), g.batch);
-  MRL_LAUNCH((k_gemm_skinny<KIND, ALIGNED, RT, CT>), grid, dim3(64 * WAVES), (skinny_lds<RT, CT>()), stream, g);
+  MRL_LAUNCH((k_gemm_skinny<KIND, START, RT, CT>), grid, dim3(64 * WAVES), (skinny_lds<RT, CT>()), stream, g);
   return mrl::plan::last_error();
 }
 
-template <int KIND, bool ALIGNED>
+template <int KIND, int START>
 hipError_t launch_rows(const GemmArgs &g, hipStream_t stream) {
   // A wider block re-reads A less often (a row block of A is read once per column block); narrower ones
   // give the chip more workgroups.  Up to 16 rows A is no more than B's block: narrow always (bf16
   // 4 x 4096 x 16384 26.4 us, two columns of blocks 34).  Rows that have to be cut out of two chunks are
   // dear on the A side: wide from 128 columns of blocks on (u8 40 x 4001 x 5000 14.1 against 22.4).
   const uint64_t cols = (uint64_t(g.n) + 15) / 16 * g.batch;
-  if (g.m <= 16) return launch_skinny<KIND, ALIGNED, 1, 1>(g, stream);
-  if (g.m <= 32) return cols >= 512 ? launch_skinny<KIND, ALIGNED, 2, 2>(g, stream) : launch_skinny<KIND, ALIGNED, 2, 1>(g, stream);
-  return cols >= (ALIGNED ? 512 : 128) ? launch_skinny<KIND, ALIGNED, 4, 2>(g, stream) : launch_skinny<KIND, ALIGNED, 4, 1>(g, stream);
+  if (g.m <= 16) return launch_skinny<KIND, START, 1, 1>(g, stream);
+  if (g.m <= 32) return cols >= 512 ? launch_skinny<KIND, START, 2, 2>(g, stream) : launch_skinny<KIND, START, 2, 1>(g, stream);
+  return cols >= (START == 16 ? 512 : 128) ? launch_skinny<KIND, START, 4, 2>(g, stream) : launch_skinny<KIND, START, 4, 1>(g, stream);
 }
 
 template <int KIND>
 hipError_t launch_kind(const GemmArgs &g, hipStream_t stream) {
   constexpr int ES = Kind<KIND>::ES;
   if (g.b_kmajor) {
-    auto chunks = [](const void *p, int64_t ld, int64_t stride) {
-      return ((reinterpret_cast<uintptr_t>(p) | uintptr_t(ld * ES) | uintptr_t(stride * ES)) & 15) == 0;
-    };
-    const bool aligned = uint64_t(g.k) * ES % 16 == 0 && chunks(g.a, g.lda, g.sa) && chunks(g.b, g.ldb, g.sb);
-    return aligned ? launch_rows<KIND, true>(g, stream) : launch_rows<KIND, false>(g, stream);
+    const uintptr_t starts = reinterpret_cast<uintptr_t>(g.a) | uintptr_t(g.lda * ES) | uintptr_t(g.sa * ES) |
+                             reinterpret_cast<uintptr_t>(g.b) | uintptr_t(g.ldb * ES) | uintptr_t(g.sb * ES);
+    if (starts % 16 == 0 && uint64_t(g.k) * ES % 16 == 0) return launch_rows<KIND, 16>(g, stream);
+    if constexpr (ES < 4)
+      if (starts % 4 != 0) return launch_rows<KIND, 1>(g, stream);
+    return launch_rows<KIND, 4>(g, stream);
   }
   const uint64_t blocks = (uint64_t(g.n) + 15) / 16 * ((uint64_t(g.m) + 15) / 16) * g.batch;
   if (g.m <= 16 || blocks <= 128) {
