@@ -463,7 +463,9 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
                                                                          : -1;
   g.c_bf16 = dc == MRL_BF16;
   // Few rows, or a small problem: read in place whatever the rows' alignment.
-  if (!sched && kind >= 0 && rows && mrl::gemm_skinny_applicable(g, kind)) {
+  const uint32_t in_place = !sched && rows ? mrl::gemm_ring_rows_columns(g, kind) : 0;
+  const bool few = in_place != 0 && g.m <= 64;   // (rows enough for the tiles below all the same)
+  if (!sched && kind >= 0 && rows && !few && mrl::gemm_skinny_applicable(g, kind)) {
     HIP_TRY(mrl::launch_gemm_skinny(g, kind, ws.stream));
     return finish_output(c, ws);
   }
@@ -474,10 +476,9 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   // int8 rows of N, of which a step takes half lines (139 x 4080 x 2288 twice 22.6 / 23.5).
   const int64_t chunk = 16 / int64_t(a.elem);
   const bool ragged = g.lda % chunk != 0 || g.sa % chunk != 0 || g.ldb % chunk != 0 || g.sb % chunk != 0;
-  const uint32_t in_place = !sched && rows ? mrl::gemm_ring_rows_columns(g, kind) : 0;
-  uint32_t k_left = 0;
   const bool steps_pay = in_place == 32 && uint64_t(g.k) * a.elem > 8 * 128 && (kind == 2 || g.b_kmajor || g.k <= 24 * 128);
-  if (in_place != 0 && (ragged || (steps_pay && (mrl::gemm_k_splits(g, kind, &k_left) == 1 || k_left != 0)))) {
+  uint32_t k_left = 0;
+  if (in_place != 0 && (ragged || few || (steps_pay && (mrl::gemm_k_splits(g, kind, &k_left) == 1 || k_left != 0)))) {
     uint32_t slice_k = 0;
     const uint32_t splits = mrl::uneven_k_slices(g, kind, false, &slice_k);
     if (splits == 1) {

@@ -234,7 +234,12 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
   if (kind < 0 || kind > 2) return 0;
   const int es = kind == 2 ? 2 : 1;
   const uint64_t steps = (uint64_t(g.k) * es + STEP - 1) / STEP;
-  if (g.m <= 64 || g.n <= 64 || steps < 2 || steps >= (1u << 22) || !gemm::edge_addressable(g, es) || g.batch > 65535 ||
+  // More than 32 rows against a large k-fastest B: half a tile or more, and K in slices fills the chip where gemm_skinny.hip
+  // and k_gemm have a workgroup for 16, 32 or 64 columns (bf16 38 x 10482 x 1472 24.0 / 11.7, 57 x 1856 x 4284 13.4 / 9.6, u8 41 x
+  // 6895 x 2728 17.3 / 11.5; below 10 MB of B they are the faster ones: u8 39 x 3840 x 1920 6.2 / 8.6).
+  const bool few = g.m <= 64;
+  if (few && !(g.m > 32 && g.b_kmajor && g.batch == 1 && uint64_t(g.n) * g.k * es > (10ull << 20))) return 0;
+  if (g.n <= 64 || steps < 2 || steps >= (1u << 22) || !gemm::edge_addressable(g, es) || g.batch > 65535 ||
       reinterpret_cast<uintptr_t>(g.c) % (g.c_bf16 ? 2 : 4) != 0)
     return 0;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };

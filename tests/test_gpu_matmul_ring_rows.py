@@ -67,6 +67,22 @@ def test_rows_that_start_anywhere(gpu, b, m, k_bytes, n, accum, families, types,
         d.free()
 
 
+@pytest.mark.parametrize("types", list(TYPES))
+@pytest.mark.parametrize("m,k_bytes,n,accum,families", [
+    (33, 61 * 128 + 22, 1475, True, 2),      # half a tile of rows, K in slices
+    (64, 9 * 128 + 16, 9999, False, 1),      # a whole one, in one piece; rows of whole chunks
+])
+def test_33_to_64_rows_against_a_large_b(gpu, types, m, k_bytes, n, accum, families):
+    dts = TYPES[types]
+    k = k_bytes // (2 if dts[0] == M.bf16 else 1)
+    A, B = GEN[dts[0]](184, 0, (1, m, k)), GEN[dts[1]](184, 1, (1, k, n))
+    C = {M.i32: lambda: synth.uniform_i8(184, 2, (1, m, n)).astype(np.int32) * 1001,
+         M.f32: lambda: synth.normal_f32(184, 2, (1, m, n)), M.bf16: lambda: synth.normal_bf16(184, 2, (1, m, n))}[dts[2]]()
+    spec = M.Matmul([1, m, k, n], dts, [None, KT, None], accum)
+    assert spec.plan().kernels == ["k_gemm_ring", "k_sum_splits"][:families]
+    _check(run_spec(spec, [A, np.ascontiguousarray(B.transpose(0, 2, 1)), C.copy()]), A, B, C, accum, dts)
+
+
 @pytest.mark.parametrize("nk", [False, True])
 @pytest.mark.parametrize("types,m,k,n", [("bf16", 1411, 733, 1555), ("bf16_out", 1300, 1501, 2049), ("bf16_out", 1153, 201, 1861), ("bf16", 1153, 65, 1861)])
 def test_tiles_of_128_columns(gpu, types, m, k, n, nk):
