@@ -271,7 +271,7 @@ constexpr int MAX_DEVICES = 64;
 void *g_scratch_ptr[MAX_DEVICES] = {};
 
 // Whether this thread's call makes the smallest copies there are (rows padded to 16 bytes and not to whole cache
-// lines, short columns turned): mrl_run_noalloc, for a Spec whose scratch does not fit otherwise.
+// lines, short columns turned) and no partial results of uneven slices or shares of keys: mrl_run_noalloc, for a Spec whose scratch does not fit otherwise.
 thread_local bool g_tight_scratch = false;
 
 struct Workspace {
@@ -480,7 +480,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   uint32_t k_left = 0;
   if (in_place != 0 && (ragged || few || (steps_pay && (mrl::gemm_k_splits(g, kind, &k_left) == 1 || k_left != 0)))) {
     uint32_t slice_k = 0;
-    const uint32_t splits = mrl::uneven_k_slices(g, kind, false, &slice_k);
+    const uint32_t splits = g_tight_scratch ? 1 : mrl::uneven_k_slices(g, kind, false, &slice_k);
     if (splits == 1) {
       HIP_TRY(mrl::launch_gemm_ring_rows(g, kind, ws.stream));
     } else {
@@ -808,7 +808,7 @@ int run_conv(const mrl_spec &s, void *const *params, Workspace &ws) {
     // Few output tiles and long windows (deep layers on small images): slices of the window as
     // batch entries with partial results, summed in slice order, as for a Matmul.
     uint32_t slice_k = 0;
-    const uint32_t splits = forced == 2 ? 1 : mrl::uneven_k_slices(conv_args, kind, true, &slice_k);
+    const uint32_t splits = forced == 2 || g_tight_scratch ? 1 : mrl::uneven_k_slices(conv_args, kind, true, &slice_k);
     if (splits > 1) {
       void *partial = nullptr;
       HIP_TRY(ws.alloc(&partial, size_t(splits) * conv_args.m * conv_args.n * 4));
@@ -1058,6 +1058,7 @@ int run_compose_msm(const mrl_spec &s, void *const *params, Workspace &ws) {
       if (!out_in_order) HIP_TRY(ws.alloc(&result, size_t(b) * m * n * sizeof(float)));
       at.out = static_cast<float *>(result);
       if (forced == 1) at.query_block = g_forced->query_block, at.key_splits = g_forced->key_splits;
+      else if (g_tight_scratch) at.key_splits = 1;
       mrl::attn_choose(at);
       if (at.key_splits > 1) {
         void *partials = nullptr;

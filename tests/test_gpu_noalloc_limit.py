@@ -36,3 +36,21 @@ def test_copies_fit_that_did(gpu, dts, shape, k_fastest):
     else:
         # the same kernel family over a K that ends elsewhere: f32 sums of 2817 products in another order
         assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+
+
+def test_conv_fits_without_partial_results(gpu):
+    """Windows shared out in slices of unequal length, 10 MB of partial results beside 30 MB of copies to channels-last."""
+    b, f, c, oh, fh = 4, 256, 3056, 36, 3
+    row_major = M.layout(0, 1, 2, 3)
+    spec = M.Conv([b, f, c, oh, oh, fh, fh], [M.u8, M.i8, M.i32], [row_major] * 3)
+    assert spec.plan().scratch_bytes > M.NOALLOC_SCRATCH_BYTES
+    ih = oh + fh - 1
+    arrays = [synth.uniform_u8(951, 0, (b, c, ih, ih)), synth.uniform_i8(951, 1, (f, c, fh, fh)), np.zeros((b, f, oh, oh), np.int32)]
+    want = run_spec(spec, arrays)
+    bufs = [M.DeviceBuffer.from_numpy(a) for a in arrays]
+    spec.run_noalloc([x.ptr for x in bufs])
+    M.synchronize()
+    got = bufs[2].to_numpy(np.int32, arrays[2].shape)
+    for x in bufs:
+        x.free()
+    assert np.array_equal(got, want)
