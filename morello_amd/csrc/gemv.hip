@@ -59,8 +59,8 @@ __device__ inline typename Acc<KIND>::type dot16(v4i a, v4i b, typename Acc<KIND
   return acc;
 }
 
-// COLS: output columns (rows of B) per wavefront, all in flight together.  PAST: B is read past the caches.
-template <int KIND, int ROWS, int COLS, bool PAST>
+// COLS: output columns (rows of B) per wavefront, all in flight together.
+template <int KIND, int ROWS, int COLS>
 __global__ __launch_bounds__(64 * WAVES) void k_gemv(GemmArgs g) {
   typedef typename Acc<KIND>::type acc_t;
   constexpr int ES = KIND == 3 ? 4 : KIND == 2 ? 2 : 1;
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemv(GemmArgs g) {
   for (int kb = lane * 16; kb < k_bytes; kb += 64 * 16) {
     v4i bv[COLS], av[ROWS];
 #pragma unroll
-    for (int c = 0; c < COLS; c++) bv[c] = PAST ? __builtin_nontemporal_load((const v4i *)(b_row[c] + kb)) : *(const v4i *)(b_row[c] + kb);
+    for (int c = 0; c < COLS; c++) bv[c] = __builtin_nontemporal_load((const v4i *)(b_row[c] + kb));
 #pragma unroll
     for (int r = 0; r < ROWS; r++) {
       av[r] = *(const v4i *)(a_row[r] + kb);
@@ -138,27 +138,26 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemv(GemmArgs g) {
       }
 }
 
-template <int KIND, int ROWS, int COLS, bool PAST = true>
+template <int KIND, int ROWS, int COLS>
 hipError_t launch_as(const GemmArgs &g, hipStream_t stream) {
   const dim3 grid(uint32_t((uint64_t(g.n) + COLS * WAVES - 1) / (COLS * WAVES)), g.batch), block(64 * WAVES);
   constexpr int ES = KIND == 3 ? 4 : KIND == 2 ? 2 : 1;
   plan::work(plan::UNIT_STREAM, 2.0 * g.m * g.n * g.k * g.batch,
              double(g.batch) * ((double(g.m) + g.n) * g.k * ES + (g.c_bf16 ? 2.0 : 4.0) * g.m * g.n));
-  MRL_LAUNCH((k_gemv<KIND, ROWS, COLS, PAST>), grid, block, 0, stream, g);
+  MRL_LAUNCH((k_gemv<KIND, ROWS, COLS>), grid, block, 0, stream, g);
   return mrl::plan::last_error();
 }
 
 template <int KIND>
 hipError_t launch_rows(const GemmArgs &g, hipStream_t stream) {
-  // A B that the memory-side cache holds beside others stays there for the next launch, and goes one row to a wavefront; a larger one
-  // is streamed past it, two rows to a wavefront and one from some 200 MB on (us, buffers taking turns, one row through / two past: bf16 1 x 2048 x 16384, 67 MB, 11.4 / 12.3,
-  // u8 2 x 8192 x 8192 11.5 / 15.6, bf16 2 x 5056 x 5122 9.7 / 11.1; 2 x 10688 x 5120, 109 MB, 23.9 / 22.9; 100 MB in rows of no whole KB, one row past / two: 2 x 6528 x 7726 23.2 / 18.0).
+  // One row of A: one row of B per wavefront from some 200 MB on (bf16 1 x 4096 x 32768 39.6 us against 42.3), two below (1 x 2048 x
+  // 16384 12.9 against 12.9, on one buffer again and again 10.8 against 11.3).  Two rows of A: one up to 80 MB (us, enough copies of
+  // B in turn that no cache holds them, two / one: u8 2 x 8192 x 8192 16.2 / 14.0, bf16 2 x 5056 x 5122 11.4 / 11.1; 2 x 6528 x 7726, 100 MB,
+  // 18.0 / 23.2; f32 2 x 2048 x 8192 14.8 / 14.0, but 11.9 / 12.9 on one buffer: two).  Loads through the caches, one row: 11.3 us for 1 x 2048 x 16384 while the 256 MB memory-side cache holds every B in
+  // use, 14.7 when a program goes through more of them, as one that decodes through its layers does.
   const double bytes = double(g.n) * g.k * (KIND == 3 ? 4 : KIND == 2 ? 2 : 1) * g.batch;
-  if (g.m == 1) {
-    if (bytes <= 80e6) return launch_as<KIND, 1, 1, false>(g, stream);
-    return bytes >= 200e6 ? launch_as<KIND, 1, 1>(g, stream) : launch_as<KIND, 1, MRL_GEMV_COLS>(g, stream);
-  }
-  if (g.m == 2) return bytes <= 80e6 ? launch_as<KIND, 2, 1, false>(g, stream) : launch_as<KIND, 2, MRL_GEMV_COLS>(g, stream);
+  if (g.m == 1) return bytes >= 200e6 ? launch_as<KIND, 1, 1>(g, stream) : launch_as<KIND, 1, MRL_GEMV_COLS>(g, stream);
+  if (g.m == 2) return KIND != 3 && bytes <= 80e6 ? launch_as<KIND, 2, 1>(g, stream) : launch_as<KIND, 2, MRL_GEMV_COLS>(g, stream);
   if (g.m <= 4) return launch_as<KIND, 4, MRL_GEMV_COLS>(g, stream);
   return launch_as<KIND, MAX_ROWS, 2>(g, stream);
 }
