@@ -25,6 +25,23 @@ namespace attn {
 namespace {
 
 constexpr int KEYS = 32;   // keys per block
+// Blocks of a wave whose maxima the reference follows (1024 keys a workgroup): the exponential of the largest score so far is then
+// exactly 1, and the largest weigh most in the rounding of P to bf16.  Error in the norm, the form of attention.hip / two
+// blocks / four: 19 x 64 x 64 against 1372 keys 1.13e-3 / 1.16e-3 / 0.86e-3, 4 x 700 x 32 against 2048 1.23 / 1.27 / 1.08, 22 x 2 x 64 against
+// 1938 1.14 / 1.25 / 1.06, 16 x 1 x 128 against 32768 1.26 / 1.40 / 1.11.  With the maxima over lanes exchanged in the vector unit
+// (over_lane_groups) and not through LDS four cost no more than two did: 0.96 of the time over 400 shapes.
+constexpr int FOLLOWED = 4;
+
+// The largest of a value over the four lane groups, in all of them.
+__device__ inline float over_lane_groups(float x) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  const unsigned own = __float_as_uint(x);
+  const u2 rows = __builtin_amdgcn_permlane16_swap(own, own, false, false);   // groups 0, 0, 2, 2 and 1, 1, 3, 3
+  const float pair = fmaxf(__uint_as_float(rows.x), __uint_as_float(rows.y));
+  const unsigned both = __float_as_uint(pair);
+  const u2 halves = __builtin_amdgcn_permlane32_swap(both, both, false, false);
+  return fmaxf(__uint_as_float(halves.x), __uint_as_float(halves.y));
+}
 
 template <int D>
 struct Tiles {
@@ -177,8 +194,7 @@ __global__ __launch_bounds__(64 * W) void k_attn(const void *q, const void *kt, 
           for (int kb = 0; kb < 2; kb++)
 #pragma unroll
             for (int r = 0; r < 4; r++) mx = fmaxf(mx, s[kb][qb][r]);
-          mx = fmaxf(mx, __shfl_xor(mx, 16));
-          mx = fmaxf(mx, __shfl_xor(mx, 32));
+          mx = over_lane_groups(mx);
           const float m_new = fmaxf(m_run[qb], mx);
           const float alpha = __builtin_amdgcn_exp2f((m_run[qb] - m_new) * LOG2E);
           m_run[qb] = m_new;
@@ -187,11 +203,9 @@ __global__ __launch_bounds__(64 * W) void k_attn(const void *q, const void *kt, 
           for (int db = 0; db < NDB; db++) o[db][qb] *= alpha;
         }
       };
-      // The reference follows a wave's first two blocks (512 keys a workgroup): the exponential of the largest score so far is
-      // exactly 1, and the largest weigh most in the rounding of P (13 x 346 x 80 against 1088 keys, error in the norm: 1.24e-3
-      // from the first block, 1.08e-3 from two, 1.17e-3 the other form).  Following every block's maximum would halve that and
-      // costs a second round of exponentials wherever some query's moves: up to 22 % of the time.
-      const bool fresh = block < first + wave + 2 * W;
+      // Beyond the followed blocks the reference moves where a score has outgrown it.  (Following every block's maximum would halve
+      // the error once more and costs a second round of exponentials wherever some query's moves.)
+      const bool fresh = block < first + wave + FOLLOWED * W;
       v8bf pb[QB];
       float pmax = 0.0f;
       auto exponentials = [&]() {
