@@ -699,23 +699,24 @@ uint32_t key_splits_of_waves(const AttnArgs &a, uint64_t groups) {
 // (us, this form / the other): 4 x 1 x 128 against 564 keys 5.4 / 10.1; 16 x 103 x 80 against 767 6.7 / 11.9; 40 x 90 x 128
 // against 1024 8.1 / 15.4; 13 x 346 x 80 against 1088 (32 queries) 9.6 / 15.4; 18 x 329 x 32 against 1810 6.4 / 12.8;
 // beyond: 47 x 192 x 128 against 1856 28.9 / 22.5, 16 x 2048 x 2048 58.9 / 33.8, 2 x 2048 against 4096 keys 21.2 / 22.4, 8192 31.7 / 26.8.
-bool by_waves(AttnArgs &a) {
+// `shares`: of the keys, where they are given (1: no scratch for partial results), else 0.
+bool by_waves(AttnArgs &a, uint32_t shares) {
   if (a.kt_rows || a.m == 0 || a.b == 0) return false;
   const uint64_t units = g_compute_units, room = a.k == 128 ? units : 2 * units;
   const uint64_t g16 = uint64_t(a.b) * ((a.m + 15) / 16), g32 = uint64_t(a.b) * ((a.m + 31) / 32);
   const uint64_t longest = a.k == 128 ? 2048 : 4096;
-  a.query_block = 16, a.waves = 8, a.key_splits = 1;
+  a.query_block = 16, a.waves = 8, a.key_splits = shares ? shares : 1;
   if (a.m <= 16) {
-    if (g16 < units) a.key_splits = key_splits_of_waves(a, g16);
+    if (!shares && g16 < units) a.key_splits = key_splits_of_waves(a, g16);
     return true;
   }
   if (g16 <= room && a.n2 <= longest) {
     // (more than 16 queries share what a split streams, and its partial results are as many rows: only where less than half of the chip is at work)
-    if (2 * g16 <= units) a.key_splits = key_splits_of_waves(a, g16);
+    if (!shares && 2 * g16 <= units) a.key_splits = key_splits_of_waves(a, g16);
     return true;
   }
-  if (4 * g16 <= units && g16 * a.n2 <= 200 * longest) {   // longer ones in splits: 8 x 32 x 128 against 8192 keys 9.8 / 13.9, 2 x 512 against 4096 11.6 / 14.1, 8192 16.1 / 14.9
-    a.key_splits = key_splits_of_waves(a, g16);
+  if (shares != 1 && 4 * g16 <= units && g16 * a.n2 <= 200 * longest) {   // longer ones in splits: 8 x 32 x 128 against 8192 keys 9.8 / 13.9, 2 x 512 against 4096 11.6 / 14.1, 8192 16.1 / 14.9
+    if (!shares) a.key_splits = key_splits_of_waves(a, g16);
     return true;
   }
   // Up to 128 keys leave four of eight waves without a block: workgroups of four, two to a unit (8 x 640 x 128 against 68: 4.9 us, of eight 6.7, the other form 6.5).
@@ -730,11 +731,11 @@ bool by_waves(AttnArgs &a) {
 }  // namespace
 
 void attn_choose(AttnArgs &a) {
-  if (!a.query_block && !a.key_splits) {
-    if (by_waves(a)) return;
-    a.query_block = 0, a.key_splits = 0;
+  if (!a.query_block) {
+    const uint32_t shares = a.key_splits;
+    if (by_waves(a, shares)) return;
+    a.query_block = query_block_of(a), a.key_splits = shares;
   }
-  if (!a.query_block) a.query_block = query_block_of(a);
   if (!a.key_splits) a.key_splits = key_splits_of_blocks(a);
 }
 

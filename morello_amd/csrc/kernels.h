@@ -320,7 +320,7 @@ struct AttnArgs {
   uint32_t key_splits = 0;
   float *partials = nullptr;
 };
-void attn_choose(AttnArgs &a);   // sets query_block, waves and key_splits where they are 0
+void attn_choose(AttnArgs &a);   // sets query_block with waves, and key_splits, where they are 0
 size_t attn_partial_bytes(const AttnArgs &a, uint32_t splits);
 bool attn_applicable(const AttnArgs &a);
 hipError_t launch_attn(const AttnArgs &a, hipStream_t stream);

@@ -54,3 +54,21 @@ def test_conv_fits_without_partial_results(gpu):
     for x in bufs:
         x.free()
     assert np.array_equal(got, want)
+
+
+def test_attention_of_few_queries_fits_without_partial_results(gpu):
+    """Padded copies of K and V (33 MB) leave no room for shares of the keys: the same form with one share, which needs none."""
+    b, m, keys, d = 8, 16, 8100, 100
+    spec = M.ComposeMSM(b, m, d, keys, d, layouts=[None, None, M.layout(0, 2, 1), None])
+    one_share = M.Action(spec, M._binding.ActionC(M.ActionKind.Fused, 0, 0, 0, 1, 0, 0, 0, 0.0))
+    assert "W = 8" in one_share.plan().steps[-1].kernel
+    assert spec.plan().scratch_bytes > M.NOALLOC_SCRATCH_BYTES >= one_share.plan().scratch_bytes
+    arrays = [synth.normal_bf16(952, i, s, 0.4) for i, s in enumerate([(b, keys, d), (b, m, d), (b, keys, d)])] + [np.zeros((b, m, d), np.float32)]
+    want = run_spec(one_share, arrays)
+    bufs = [M.DeviceBuffer.from_numpy(a) for a in arrays]
+    spec.run_noalloc([x.ptr for x in bufs])
+    M.synchronize()
+    got = bufs[3].to_numpy(np.float32, arrays[3].shape)
+    for x in bufs:
+        x.free()
+    assert np.array_equal(got, want)

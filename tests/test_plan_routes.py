@@ -120,3 +120,18 @@ def test_padded_copies_of_up_to_a_million_chunks_go_one_to_a_thread():
     assert step.family == "k_pad_rows_pair" and step.grid[0] == (1000 * 64 + 255) // 256
     step = M.Matmul([1, 5003, 4001, 5001], (M.bf16, M.bf16, M.f32)).plan().steps[0]
     assert step.family == "k_pad_rows_pair" and step.grid[0] <= 5003 * 632 // 1024 + 1
+
+
+def _fused(spec, tile_m, parts):
+    return M.Action(spec, M._binding.ActionC(M.ActionKind.Fused, tile_m, 0, 0, parts, 0, 0, 0, 0.0))
+
+
+@pytest.mark.parametrize("b,m,keys,d", [(4, 1, 564, 128), (16, 103, 767, 80), (13, 346, 1088, 80), (40, 90, 1024, 128), (16, 2048, 2048, 128)])
+def test_fused_without_a_query_block_is_the_rules_choice(b, m, keys, d):
+    """... of the form and its queries per workgroup, with the shares of the keys that the action names (none: one)."""
+    spec = M.ComposeMSM(b, m, d, keys, d, layouts=[None, None, KT, None])
+    rules = spec.plan().steps[0]
+    for parts in (0, 1, 2):
+        p = _fused(spec, 0, parts).plan()
+        assert p.steps[0].kernel == rules.kernel and p.steps[0].grid == (rules.grid[0], max(1, parts), 1)
+        assert p.kernels == ["k_attn", "k_attn_merge"][:max(1, parts)] and (p.scratch_bytes > 0) == (parts == 2)
