@@ -512,8 +512,9 @@ int mrl_compose_plan(const mrl_compose *c, mrl_plan *plan, mrl_plan_step *steps,
  *                   share the rows' pixels through LDS and take 16 filters each (64 channels);
  *                   Compose Matmul->Softmax->Matmul: the fused kernel
  *                   with tile_out over the rows (`tile_m` = 128 or 64 queries per workgroup, 0 = the
- *                   dispatch rules' choice) and the keys in `parts` shares (parallel_softmax.rs:31-223;
- *                   0 or 1 = one workgroup per query block, more = partial results merged with the parts formula)
+ *                   dispatch rules' choice, which may be 32 or 16 with the keys dealt to the workgroup's
+ *                   waves) and the keys in `parts` shares (parallel_softmax.rs:31-223; 0 or 1 = one
+ *                   workgroup per query block, more = partial results merged with the parts formula)
  *   SPATIAL_SPLIT   Conv as a Matmul over its windows read in place (spatial_split.rs:73-118),
  *                   tile_out([tile_m, tile_n]) on that Matmul
  *   UNFOLD          Conv: the windows materialised (a Move), then the Matmul

@@ -652,7 +652,7 @@ struct Forced {
   bool conv_rows = false;   // fused kernel: whole output rows per workgroup, pixels shared through LDS
   int msm_path = 0;         // 1 fused kernel (key_splits workgroups per query block), 2 staged
   uint32_t key_splits = 0;
-  uint32_t query_block = 0; // fused kernel: queries per workgroup (64 or 128), 0 = the rule below
+  uint32_t query_block = 0; // fused kernel: queries per workgroup (64 or 128), 0 = attn_choose's, with its form of the kernel
 };
 thread_local const Forced *g_forced = nullptr;
 
@@ -2334,6 +2334,9 @@ int dispatch_action(const mrl_spec &spec, void *const *params, Workspace &ws, co
   // A Compose's key shares: what mrl_target_actions lists, one share or at least two blocks of 64 keys each.
   if (a.kind == MRL_ACTION_FUSED && spec.kind == MRL_SPEC_COMPOSE_MSM && a.parts > 1 &&
       (a.parts > 64 || 2 * uint64_t(a.parts) > (uint64_t(spec.spec_shape[3]) + 63) / 64))
+    return MRL_ERR_UNSUPPORTED;
+  // Queries per workgroup: those of the form that walks its keys in halves (attn_choose alone takes the other one, of 16 or 32).
+  if (a.kind == MRL_ACTION_FUSED && spec.kind == MRL_SPEC_COMPOSE_MSM && a.tile_m != 0 && a.tile_m != 64 && a.tile_m != 128)
     return MRL_ERR_UNSUPPORTED;
   const bool conv_action = a.kind == MRL_ACTION_SPATIAL_SPLIT || a.kind == MRL_ACTION_UNFOLD || a.kind == MRL_ACTION_GENERIC;
   if ((conv_action && spec.kind != MRL_SPEC_CONV) || (a.kind == MRL_ACTION_BUFFERIZE && spec.kind != MRL_SPEC_COMPOSE_MSM) ||

@@ -135,3 +135,11 @@ def test_fused_without_a_query_block_is_the_rules_choice(b, m, keys, d):
         p = _fused(spec, 0, parts).plan()
         assert p.steps[0].kernel == rules.kernel and p.steps[0].grid == (rules.grid[0], max(1, parts), 1)
         assert p.kernels == ["k_attn", "k_attn_merge"][:max(1, parts)] and (p.scratch_bytes > 0) == (parts == 2)
+
+
+@pytest.mark.parametrize("tile_m", [16, 32, 48, 256])
+def test_fused_takes_the_query_blocks_it_documents(tile_m):
+    for m, keys in ((1, 564), (2048, 2048)):
+        spec = M.ComposeMSM(4, m, 128, keys, 128, layouts=[None, None, KT, None])
+        with pytest.raises(M.MorelloError):
+            _fused(spec, tile_m, 1).plan()
