@@ -1299,9 +1299,14 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
   // 4096 x 8192 44.1 -> 40.9, 512 x 16384 11.3 -> 10.3; other rows either way: 7232 x 6800 56.9 -> 58.9, 8192 x 3072 30.6 -> 32.0).
   const size_t widest = std::max(se, de);
   uint32_t vec = 0;
-  uint64_t row = 0;   // bytes from one row of the source to the next: its longest stride
-  for (uint32_t d = 0; d < rank; d++) row = std::max(row, uint64_t(p.ss[d]) * se);
-  const bool pages = se == 4 && de == 2 && p.count > MOVE_SMALL && row % 8192 == 0;
+  // `row`: bytes from one row of the source to the next, the source's step along the digit that continues the destination's runs:
+  // the one that a tile is long along.  (The longest stride of a batched Move is the entries': 2 x 8192 x 3072 63.7 us with eight
+  // elements a vector, 61.4 with four, 8 x 1024 x 1536 18.5 and 16.4.)
+  uint64_t row = 0;
+  int64_t least = 0;
+  for (uint32_t d = 0; d < rank; d++)
+    if (int(d) != dim_d && p.shape[d] > 1 && (row == 0 || p.ds[d] < least)) row = uint64_t(p.ss[d]) * se, least = p.ds[d];
+  const bool pages = se == 4 && de == 2 && p.count > MOVE_SMALL && row != 0 && row % 8192 == 0;
   if (shared && rank > 1)
     for (uint32_t v = uint32_t(16 / widest) * (pages ? 2 : 1); vec == 0 && v >= 1 && v * widest >= 4; v /= 2) {
       bool fits = v > 1 && p.shape[dim_s] % v == 0 && (reinterpret_cast<uintptr_t>(src) % std::min<size_t>(16, v * se)) == 0 &&

@@ -2,6 +2,7 @@
 take, or takes at many times the other's cost."""
 import math
 
+import numpy as np
 import pytest
 
 import morello_amd as M
@@ -143,3 +144,14 @@ def test_fused_takes_the_query_blocks_it_documents(tile_m):
         spec = M.ComposeMSM(4, m, 128, keys, 128, layouts=[None, None, KT, None])
         with pytest.raises(M.MorelloError):
             _fused(spec, tile_m, 1).plan()
+
+
+@pytest.mark.parametrize("shape,wide", [([1, 2048, 16384], True), ([1, 8192, 3072], False), ([2, 8192, 3072], False), ([2, 8192, 2048], True),
+                                        ([3, 4097, 2048], True), ([8, 1024, 1536], False), ([4, 1, 700, 4096], True)])
+def test_wide_narrowing_vectors_where_rows_lie_8_kib_apart(shape, wide):
+    """Rows, not the entries of a batch: two of 8192 x 3072 are a multiple of 8 KiB apart and their rows 12."""
+    r = len(shape)
+    strips = M.layout(*range(r - 2), r - 1, r - 2, (r - 1, M.Packed(16)))
+    p = M.Move(shape, (M.f32, M.bf16), layouts=[None, strips]).plan()
+    per_workgroup = np.prod(shape) / p.steps[0].grid[0]   # 1024 vectors of eight elements, or of four
+    assert p.kernels == ["k_move_runs"] and (per_workgroup > 5000) == wide, p
