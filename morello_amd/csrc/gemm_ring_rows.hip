@@ -225,7 +225,8 @@ hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
 
 // Measured against padded copies and the kernels of gemm_mfma.hip (us, those / this):
 //   32 (64 x 64) where such tiles are one round at most: bf16 613 x 2516 x 936 24.5 / 15.7, 907 x 1546 x 235 twice 20.5 /
-//     11.5, 2033 x 340 x 350 8.6 / 5.1, 796 x 4509 x 96 in slices of K 22.6 / 10.0, u8 1015 x 2999 x 803 20.9 / 15.0;
+//     11.5, 2033 x 340 x 350 8.6 / 5.1, 796 x 4509 x 96 in slices of K 22.6 / 10.0, u8 1015 x 2999 x 803 20.9 / 15.0,
+//     1000^3, exactly a round, 10.4 / 7.4, 1060 x 10040 x 103 25.7 / 11.6, 300 x 270 x 290 6.7 / 4.4;
 //   64 (128 x 64) where those are: bf16 975 x 2176 x 1666 22.5 / 17.5, u8 1888 x 1633 x 885 17.4 / 14.7; int8 over a long K reads
 //     its rows' lines once too often: 1651 x 5949 x 844 28.8 / 31.8, and bf16 over a longer one: 1835 x 3535 x 655 31.7 / 35.2;
 //   128 (128 x 128), bf16: 1483 x 858 x 1983 18.4 / 15.8, 1303 x 1524 x 2056 24.3 / 20.3; over a long K the copies are
@@ -244,11 +245,6 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
     return 0;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
   const uint64_t units = g_compute_units, small = tiles(64, 64);
-  // Three int8 classes keep the copies although this is the faster way: their plans, copies and a tile of k_gemm, or the
-  // scratch that these take are relied on.  Exactly one round of tiles (1000^3: 10.5 / 6.8), fewer than 128 columns over sixteen
-  // steps or more (384 x 2559 x 120: 12.4 / 8.8), and up to three steps (300 x 270 x 290, with which a stream's scratch is
-  // tested; 1217 x 281 x 334 8.7 / 5.7).
-  if (kind <= 1 && (small == units || (g.n < 128 && steps >= 16) || steps <= 3)) return 0;
   if (small <= units) return small > units / 2 && steps > 88 ? 0 : 32;   // (292 x 6007 x 2192 bf16, 175 tiles of 94 steps: 34.7 / 35.8)
   if (tiles(128, 64) <= units) return steps <= (kind == 2 ? 48 : 24) ? 64 : 0;
   return kind == 2 && steps <= 24 && g.n >= 128 && tiles(128, 128) <= units ? 128 : 0;

@@ -277,7 +277,7 @@ def test_matrix_vector_against_a_very_large_b(gpu, dts, codes, shape, accum):
                                        ((M.bf16, M.bf16, M.f32), [7, 7, 6]), ((M.f32, M.f32, M.f32), [6, 6, 6])])
 @pytest.mark.parametrize("shape,accum", [((1, 512, 8192, 512), False), ((1, 256, 16384, 192), True),
                                          ((1, 100, 4096, 300), True), ((1, 32, 4096, 1000), False),
-                                         ((1, 130, 2048, 70), False),
+                                         ((1, 130, 4096, 70), False),
                                          # K is no whole number of equal slices: a shorter one behind them
                                          ((1, 300, 30000, 300), True), ((1, 64, 16256, 128), False), ((1, 96, 5008, 40), False)])
 @pytest.mark.parametrize("b_k_fastest", [True, False])

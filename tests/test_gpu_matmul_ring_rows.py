@@ -41,6 +41,10 @@ def _check(got, A, B, C, accum, dts):
     (1, 1283, 8 * 128 + 30, 1021, False, 1),
     (1, 461, 15 * 128, 656, True, 1),        # rows of whole chunks
     (2, 200, 9 * 128 + 16, 336, False, 1),
+    (1, 1000, 1000, 1000, False, 1),         # one round of tiles to the last
+    (1, 384, 2558, 120, False, 1),           # fewer than 128 columns
+    (2, 1270, 130, 210, True, 1),            # two steps
+    (1, 1300, 270, 690, False, 1),           # three
 ])
 def test_rows_that_start_anywhere(gpu, b, m, k_bytes, n, accum, families, types, nk):
     dts = TYPES[types]

@@ -82,14 +82,15 @@ def test_async_launches_on_two_streams(gpu):
 
 
 def test_releasing_a_streams_arena(gpu):
-    """mrl_stream_release: a Spec that stages operands (ragged K and N) runs on a stream, the
+    """mrl_stream_release: a Spec that stages operands (ragged K and N, few columns) runs on a stream, the
     stream's scratch arena is given back while the stream lives on, and the next call on the same
     stream (it starts a new arena) still accumulates onto the first one's result."""
     stream = M.Stream()
-    b, m, k, n = 1, 300, 270, 290
+    b, m, k, n = 1, 3000, 270, 60
     A, Bm = synth.uniform_u8(830, 0, (b, m, k)), synth.uniform_i8(830, 1, (b, k, n))
     bufs = [M.DeviceBuffer.from_numpy(x) for x in (A, Bm, np.zeros((b, m, n), np.int32))]
     spec = M.MatmulAccum([b, m, k, n], (M.u8, M.i8, M.i32))
+    assert spec.plan().scratch_bytes > 0
     want = orc.matmul([b, m, k, n], [0, 1, 5], A, Bm, np.zeros((b, m, n), np.int32))
     free0 = M.device_free_bytes()
     spec.run_async([x.ptr for x in bufs], stream)
@@ -112,13 +113,14 @@ def test_host_threads_share_a_stream_and_its_scratch(gpu):
     result must still be its own thread's."""
     import threading
     stream = M.Stream()
-    shapes = [(1, 300, 270, 290), (2, 257, 333, 201), (1, 400, 250, 310), (1, 260, 267, 500)]
+    shapes = [(1, 3000, 270, 60), (2, 1257, 333, 61), (3, 500, 270, 59), (1, 2060, 267, 50)]
     jobs = []
     for t, (b, m, k, n) in enumerate(shapes):
         A, Bm = synth.uniform_u8(820 + t, 0, (b, m, k)), synth.uniform_i8(820 + t, 1, (b, k, n))
         bufs = [M.DeviceBuffer.from_numpy(x) for x in (A, Bm, np.zeros((b, m, n), np.int32))]
         want = orc.matmul([b, m, k, n], [0, 1, 5], A, Bm, np.zeros((b, m, n), np.int32))
         jobs.append((M.MatmulAccum([b, m, k, n], (M.u8, M.i8, M.i32)), bufs, want, (b, m, n)))
+        assert jobs[-1][0].plan().scratch_bytes > 0
     rounds, errors = 5, []
 
     def work(spec, bufs):

@@ -97,8 +97,9 @@ def test_plans_follow_shape_dtype_and_layout():
     p = M.ComposeMSM(16, 2048, 256, 2048, 256, layouts=[None, None, KT, None]).plan()
     assert p.kernels == ["k_gemm", "k_softmax_regs", "k_gemm_wide"] and "OUT_BF16 = true" in p.steps[1].kernel
     assert "B_KMAJOR = true" in p.steps[0].kernel
-    # Ragged sizes: zero-padded copies of A and B, then the edge build of a small tile.
-    p = M.Matmul([1, 1000, 1000, 1000], (M.u8, M.i8, M.i32)).plan()
+    # Ragged sizes: read in place up to a round of tiles, else zero-padded copies of A and B, then the edge build of a small tile.
+    assert M.Matmul([1, 1000, 1000, 1000], (M.u8, M.i8, M.i32)).plan().kernels == ["k_gemm_ring"]
+    p = M.Matmul([1, 1500, 1000, 1500], (M.u8, M.i8, M.i32)).plan()
     assert p.kernels == ["k_pad_rows_pair", "k_gemm"] and "EDGE = true" in p.steps[1].kernel   # both operands' padded copies in one launch
     # One row of A with a ragged K: padded, and still on the matrix cores.
     assert M.Matmul([4, 1, 3565, 256], (M.bf16, M.bf16, M.f32)).plan().kernels == ["k_pad_rows", "k_gemm"]

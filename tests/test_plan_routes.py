@@ -80,7 +80,7 @@ def test_copies_of_a_short_k_are_no_taller_than_it():
     assert p.kernels == ["k_pad_rows_pair", "k_gemm_ring"]
     assert M.Matmul([1, 4518, 3787, 4543], (M.u8, M.i8, M.i32)).plan().kernels == ["k_pad_rows_pair", "k_gemm_wide"]
     for layout in (None, KT):   # ... which falls into equal slices
-        assert M.Matmul([1, 384, 2559, 120], (M.u8, M.i8, M.i32), layouts=[None, layout, None]).plan().kernels == ["k_pad_rows_pair", "k_gemm", "k_sum_splits"]
+        assert M.Matmul([1, 384, 2559, 60], (M.u8, M.i8, M.i32), layouts=[None, layout, None]).plan().kernels == ["k_pad_rows_pair", "k_gemm", "k_sum_splits"]
 
 
 @pytest.mark.parametrize("layout", [None, KT])
@@ -117,8 +117,8 @@ def test_the_two_forms_of_k_conv_windows_are_told_apart():
 
 
 def test_padded_copies_of_up_to_a_million_chunks_go_one_to_a_thread():
-    step = M.Matmul([1, 1000, 1000, 1000], (M.u8, M.i8, M.i32)).plan().steps[0]
-    assert step.family == "k_pad_rows_pair" and step.grid[0] == (1000 * 64 + 255) // 256
+    step = M.Matmul([1, 1500, 1000, 1500], (M.u8, M.i8, M.i32)).plan().steps[0]
+    assert step.family == "k_pad_rows_pair" and step.grid[0] == (1500 * 64 + 255) // 256
     step = M.Matmul([1, 5003, 4001, 5001], (M.bf16, M.bf16, M.f32)).plan().steps[0]
     assert step.family == "k_pad_rows_pair" and step.grid[0] <= 5003 * 632 // 1024 + 1
 
@@ -155,3 +155,12 @@ def test_wide_narrowing_vectors_where_rows_lie_8_kib_apart(shape, wide):
     p = M.Move(shape, (M.f32, M.bf16), layouts=[None, strips]).plan()
     per_workgroup = np.prod(shape) / p.steps[0].grid[0]   # 1024 vectors of eight elements, or of four
     assert p.kernels == ["k_move_runs"] and (per_workgroup > 5000) == wide, p
+
+
+@pytest.mark.parametrize("layout", [None, KT])
+@pytest.mark.parametrize("shape", [[1, 960, 1000, 1000], [1, 1000, 1000, 1000], [2, 4089, 1000, 99], [1, 384, 2559, 120], [1, 3910, 10085, 125],
+                                   [1, 300, 270, 290], [1, 1217, 281, 334], [3, 770, 136, 132]])
+def test_int8_up_to_a_round_of_tiles_is_read_in_place(shape, layout):
+    """... the last tile of a round, few columns and a short K among them."""
+    p = M.Matmul(shape, (M.u8, M.i8, M.i32), layouts=[None, layout, None]).plan()
+    assert p.kernels[0] == "k_gemm_ring" and "RA = 2" in p.steps[0].kernel, p
