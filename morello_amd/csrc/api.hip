@@ -968,9 +968,7 @@ int run_softmax(const mrl_spec &s, void *const *params, Workspace &ws) {
     as_given.ptr = v.in.ptr, as_turned.ptr = turned;
     HIP_TRY(mrl::launch_move_strided(as_given, as_turned, ws.stream));
     const uint64_t rows = before * after;
-    // (fewer than 512 rows of an odd length: in chunks, one a row)
-    if (const size_t bytes = scan % 4 != 0 && scan > 256 && scan <= 4096 && rows < 512 ? mrl::softmax_chunk_bytes(rows, scan) : mrl::softmax_scratch_bytes(rows, scan))
-      HIP_TRY(ws.alloc(&scratch, bytes));
+    if (const size_t bytes = mrl::softmax_scratch_bytes(rows, scan)) HIP_TRY(ws.alloc(&scratch, bytes));
     HIP_TRY(mrl::launch_softmax_rows((const float *)turned, (float *)turned, rows, scan, scratch, ws.stream));
     as_given.ptr = v.out.ptr;
     HIP_TRY(mrl::launch_move_strided(as_turned, as_given, ws.stream));

@@ -262,7 +262,6 @@ hipError_t launch_unfold(const void *image, void *rows, uint32_t batch, uint32_t
 // (hipErrorInvalidValue without it).  `out` may be `in`.
 constexpr uint32_t SOFTMAX_CHUNK = 4096;
 size_t softmax_scratch_bytes(uint64_t rows, uint32_t cols);
-size_t softmax_chunk_bytes(uint64_t rows, uint32_t cols);
 hipError_t launch_softmax_rows(const float *in, float *out, uint64_t rows, uint32_t cols, void *scratch,
                                hipStream_t stream);
 // The same with the result rounded to bf16 (rows of `cols` 16-bit values).

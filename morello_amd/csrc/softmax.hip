@@ -360,7 +360,6 @@ namespace {
 // ODD: rows of a length that is no multiple of 4.
 template <bool ODD, bool OUT_BF16>
 hipError_t launch_long_rows(const float *in, void *out, uint64_t rows, uint32_t cols, void *scratch, hipStream_t stream) {
-  if (scratch && cols <= 16 * 256) return launch_chunks<ODD ? 1 : 4, OUT_BF16>(in, out, rows, cols, static_cast<float2 *>(scratch), stream);
   // A workgroup per row with the row in registers: rows beyond the wavefront kernel's 4096
   // columns when there are 256 of them or more, and rows of more than 1024 columns when there are
   // too few of them to occupy the chip a wavefront each.
@@ -407,12 +406,7 @@ hipError_t launch_rows(const float *in, void *out, uint64_t rows, uint32_t cols,
 
 // Scratch the chunked kernels want for this shape (0: the shape runs without).
 size_t softmax_scratch_bytes(uint64_t rows, uint32_t cols) {
-  // Up to 4096 columns the register kernels serve.
-  return cols <= 16 * 256 ? 0 : softmax_chunk_bytes(rows, cols);
-}
-
-// Scratch with which launch_softmax_rows takes rows of up to 4096 elements in chunks as well (one a row).
-size_t softmax_chunk_bytes(uint64_t rows, uint32_t cols) {
+  if (cols <= 16 * 256) return 0;   // the register kernels serve
   const uint64_t chunks = (cols + SOFTMAX_CHUNK - 1) / SOFTMAX_CHUNK;
   if (rows * chunks > 0x7fffffffull) return 0;
   return size_t(rows * chunks * sizeof(float2));

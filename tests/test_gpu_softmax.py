@@ -503,3 +503,14 @@ def test_softmax_over_an_outer_dim_in_registers(gpu, scan, before, after):
     """Scan dims on either side of what a workgroup holds, column tiles with a ragged end."""
     assert M.Softmax([before, scan, after], 1).plan().kernels == ["k_softmax_cols"]
     _softmax_outer((before, scan, after), 1)
+
+
+@pytest.mark.parametrize("shape", [(45, 1963, 4), (300, 963, 4), (1, 4093, 13), (23, 2857, 3), (100, 1303, 7)])
+def test_turned_rows_of_odd_lengths_in_one_launch(gpu, shape):
+    spec = M.Softmax(list(shape), 1)
+    assert len(spec.plan().kernels) == 3 and spec.plan().kernels[1] in ("k_softmax_block", "k_softmax_regs"), spec.plan()
+    x = synth.normal_f32(207, 0, shape, std=3.0)
+    x[0, 5, 1], x[0, shape[1] - 1, 2] = np.inf * -1, -3.40282347e38
+    got = run_spec(spec, [x, np.zeros(shape, np.float32)])
+    want = orc.softmax(list(shape), 1, x)
+    assert (np.abs(got - want) <= 1e-5 * np.abs(want) + 1e-12).all()

@@ -130,7 +130,9 @@ def test_plans_follow_shape_dtype_and_layout():
     assert p.steps[1].grid == (64, 16, 1) and p.steps[0].bytes == pytest.approx(5.2 * 2048 * 4096)
     assert p.scratch_bytes == 64 * 16 * 64 * 8
     # Fewer than 16 contiguous elements behind the scan dim: scan dim turned innermost and back.
-    assert M.Softmax([45, 1963, 4], 1).plan().kernels[0].startswith("k_move") and len(M.Softmax([45, 1963, 4], 1).plan().kernels) == 4
+    turned = M.Softmax([45, 1963, 4], 1).plan()
+    assert turned.kernels[1] == "k_softmax_block" and len(turned.kernels) == 3 and all(k.startswith("k_move") for k in turned.kernels[::2])
+    assert M.Softmax([300, 963, 4], 1).plan().kernels[1] == "k_softmax_regs"   # (rows of an odd length, few or many, in one launch)
     assert M.Softmax([100000, 67], 1).plan().kernels == ["k_softmax_short"]
     # Moves: transpose tiled through LDS, Packed destination gathered, plain copy.
     sq = [4096, 4096]
