@@ -123,7 +123,6 @@ uint32_t uneven_k_slices(const GemmArgs &g, int kind, bool conv, uint32_t *slice
   uint64_t per = (steps + wanted - 1) / wanted;
   while (k_bytes % (per * 128) != 0 && k_bytes % (per * 128) <= 128) per++;   // (gemm_ring_rows.hip wants two steps or more)
   const uint64_t count = (steps + per - 1) / per;
-  if (count <= 1) return 1;
   // (Rows that start anywhere: one workgroup a compute unit, 292 x 6007 x 2192 bf16 in halves, 350 of them, 43.6 us, whole 35.)
   // As in gemm_k_splits, with the step of each kernel and type (Conv: a chain of 66 int8 steps 30 us, of 107 bf16
   // steps 40) and the partials' traffic at the 3 TB/s that a sum of a few MB reaches: 2 x (48 -> 144) x 43^2 5 x 5
@@ -132,7 +131,22 @@ uint32_t uneven_k_slices(const GemmArgs &g, int kind, bool conv, uint32_t *slice
   const double spread = std::min<double>(double(count), (conv ? 384.0 : 256.0) / double(tiles));
   const double saved_us = double(steps) * (1.0 - 1.0 / spread) * (!conv ? 0.28 : kind == 2 ? 0.36 : 0.46);
   const double cost_us = 2.2 + (double(count) + 1.0) * double(g.m) * double(g.n) * 4.0 / 3.0e6;
-  if (spread <= 1.0 || saved_us < 1.2 * cost_us) return 1;
+  bool pays = spread > 1.0 && saved_us >= 1.2 * cost_us;
+  if (conv) {
+    // int8 in two slices of eight steps, over half of the units and more in one piece already: 10 x (224 -> 16) x 33^2 3 x 3, 171 tiles of
+    // 16 steps, 9.6 us whole, 10.2 in halves, 14 x (240 -> 16) x 30^2, 197 of 17, 10.4 and 11.0 (16 x (112 -> 16) x 26^2 5 x 5, 169 of 22, 12.0 and 11.5).
+    if (kind <= 1 && tiles > 128 && steps < 18) pays = false;
+    // Equal slices where there are about as many (they end together), and where the above finds none worth it for long chains, which it has
+    // too short for many tiles (up to 0.5 us a step): us, whole or in so many uneven ones / equal: bf16 24 x (320 -> 320) x 10^2 3 x 3, 190 tiles of 45
+    // steps, 22.9 / 17.7 in three, 4 x (256 -> 288) x 24^2 18.8 / 15.1, 14 x (384 -> 112) x 26^2 28.0 / 26.4; 3 x (384 -> 160) x 15^2 5 x 5, 13.0 in 17 / 12.1
+    // in 15; fewer of them: 5 x (320 -> 112) x 11^2 5 x 5 14 / 5, 1.45 times as long; chains of 18 steps: 5 x (144 -> 112) x 26^2 1.2 times.
+    const uint32_t equal = gemm_k_splits(g, kind);
+    if (equal > 1 && (pays ? 8 * equal >= 7 * count : steps >= 32)) {
+      *slice_k = g.k / equal;
+      return equal;
+    }
+  }
+  if (!pays) return 1;
   *slice_k = uint32_t(per * 128 / es);
   return uint32_t(count);
 }

@@ -164,3 +164,14 @@ def test_int8_up_to_a_round_of_tiles_is_read_in_place(shape, layout):
     """... the last tile of a round, few columns and a short K among them."""
     p = M.Matmul(shape, (M.u8, M.i8, M.i32), layouts=[None, layout, None]).plan()
     assert p.kernels[0] == "k_gemm_ring" and "RA = 2" in p.steps[0].kernel, p
+
+
+@pytest.mark.parametrize("dts,b,c,f,hw,fs,slices", [
+    ("bf16", 24, 320, 320, 10, 3, 3), ("bf16", 4, 256, 288, 24, 3, 4), ("bf16", 22, 256, 96, 19, 3, 3), ("bf16", 14, 384, 112, 26, 3, 2),   # long chains: equal slices
+    ("bf16", 3, 384, 160, 15, 5, 15), ("bf16", 14, 384, 64, 12, 5, 15),                        # as many equal ones but two
+    ("bf16", 5, 320, 112, 11, 5, 14), ("u8", 5, 384, 32, 13, 5, 9), ("bf16", 11, 128, 64, 15, 3, 1),   # many fewer; a short chain
+    ("u8", 10, 224, 16, 33, 3, 1), ("u8", 14, 240, 16, 30, 3, 1), ("u8", 8, 224, 32, 11, 3, 2)])        # int8: two short slices of many tiles, of few
+def test_slices_of_conv_windows(dts, b, c, f, hw, fs, slices):
+    types = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[dts]
+    p = M.Conv([b, f, c, hw, hw, fs, fs], types).plan()
+    assert p.kernels == ["k_gemm", "k_sum_splits"][:1 + (slices > 1)] and p.steps[0].grid[1] == slices, p
