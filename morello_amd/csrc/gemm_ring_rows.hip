@@ -221,6 +221,27 @@ hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
   }
 }
 
+// More than half of a round of 64 x 64 tiles and up to three quarters: K is not shared out here (a second round), and k_gemm's slices of
+// it, three workgroups to a unit, are the faster way over a long K where they come cheap (us, those / this, bf16 where not said):
+//   no operand to copy, from 61 steps on: 678 x 5488 x 755 22.8 / 30.3, 1086 x 3848 x 533 20.8 / 23.0, 492 x 4664 x 1414 23.7 / 27.3, u8 201 x 10320 x 2955
+//     25.1 / 31.8 (59 steps 20.1 / 21.1; 231 x 3872 x 3091, 196 tiles, 23.2 / 22.1);
+//   K, ending on a whole chunk, in three equal slices or more: 653 x 5434 x 782 24.6 / 31.2, 460 x 4031 x 1299 23.0 / 26.6;
+//   only B to copy, from 77 steps on: 755 x 4992 x 741 22.7 / 26.8, 1775 x 5520 x 268 27.3 / 29.1 (1415 x 4448 x 443 26.9 / 24.5);
+//   int8 rows of N, of which a step takes half lines, from 67 steps on: 905 x 9285 x 519 29.7 / 35.7.
+// Other ragged ones are faster here: 1150 x 4530 x 497 28.1 / 26.5, 265 x 4822 x 2236 34.0 / 29.9.
+bool slices_are_faster(const GemmArgs &g, int kind, int es, uint64_t steps, uint64_t small, uint64_t units) {
+  if (4 * small > 3 * units || steps <= 60) return false;
+  const int64_t chunk = 16 / es;
+  const bool a_whole = g.lda % chunk == 0, b_whole = g.ldb % chunk == 0;
+  if (a_whole && b_whole) return true;
+  GemmArgs copied = g;
+  copied.k = uint32_t((g.k + chunk - 1) / chunk * chunk);
+  uint32_t left = 0;
+  if (gemm_k_splits(copied, kind, &left) >= 3 && left == 0) return true;
+  const bool few_tiles = 8 * small <= 5 * units;
+  return few_tiles && ((steps > 76 && a_whole && uint64_t(g.n) * g.k * es <= (11u << 20)) || (steps > 66 && kind <= 1 && !g.b_kmajor));
+}
+
 }  // namespace
 
 // Measured against padded copies and the kernels of gemm_mfma.hip (us, those / this):
@@ -245,8 +266,16 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
     return 0;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
   const uint64_t units = g_compute_units, small = tiles(64, 64);
-  if (small <= units) return small > units / 2 && steps > 88 ? 0 : 32;   // (292 x 6007 x 2192 bf16, 175 tiles of 94 steps: 34.7 / 35.8)
-  if (tiles(128, 64) <= units) return steps <= (kind == 2 ? 48 : 24) ? 64 : 0;
+  if (small <= units) {
+    if (2 * small <= units) return 32;
+    if (steps > 88) return 0;   // (292 x 6007 x 2192 bf16, 175 tiles of 94 steps: 34.7 / 35.8)
+    return g.batch == 1 && !few && slices_are_faster(g, kind, es, steps, small, units) ? 0 : 32;
+  }
+  // bf16 rows of an odd number of elements along K, a pair of lines for every 128 bytes of either operand: in one entry the copies are
+  // the faster way from 41 steps on (1031 x 2937 x 1194 26.7 / 32.0, 407 x 2585 x 2924 24.4 / 26.9, 746 x 2925 x 1518 26.9 / 27.5; 231 x 2739 x 4310 27.5 / 26.5;
+  // fewer steps, or two entries, on either side of even: 2270 x 2473 x 710 26.5 / 24.5, 836 x 2455 x 1981 25.3 / 26.0, 791 x 2925 x 918 twice 29.2 / 31.1, 2295 x 2943 x 374 twice 30.8 / 29.4).
+  const bool odd_rows = kind == 2 && g.b_kmajor && (g.lda % 2 != 0 || g.ldb % 2 != 0);
+  if (tiles(128, 64) <= units) return steps <= (kind != 2 ? 24 : odd_rows && g.batch == 1 ? 40 : 48) ? 64 : 0;
   return kind == 2 && steps <= 24 && g.n >= 128 && tiles(128, 128) <= units ? 128 : 0;
 }
 

@@ -175,3 +175,16 @@ def test_slices_of_conv_windows(dts, b, c, f, hw, fs, slices):
     types = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[dts]
     p = M.Conv([b, f, c, hw, hw, fs, fs], types).plan()
     assert p.kernels == ["k_gemm", "k_sum_splits"][:1 + (slices > 1)] and p.steps[0].grid[1] == slices, p
+
+
+@pytest.mark.parametrize("types,m,k,n,nk,in_place", [
+    ("bf16", 678, 5488, 755, True, False), ("u8", 201, 10320, 2955, True, False), ("bf16", 474, 3768, 1108, True, True), ("bf16", 231, 3872, 3091, True, True),    # nothing to copy: 86, 81, 59 steps; 196 tiles
+    ("bf16", 653, 5434, 782, True, False), ("bf16", 460, 4031, 1299, False, False), ("bf16", 1150, 4530, 497, True, True),                                         # equal slices, none
+    ("bf16", 755, 4992, 741, False, False), ("bf16", 1415, 4448, 443, False, True),                                                                             # one copy: 78 and 70 steps
+    ("u8", 905, 9285, 519, False, False), ("u8", 204, 9048, 2539, True, True),                                                                                   # int8 rows of N, of K
+    ("bf16", 1031, 2937, 1194, True, False), ("bf16", 836, 2455, 1981, True, True), ("bf16", 1031, 2938, 1194, True, True), ("bf16", 1031, 2937, 1194, False, True),   # odd rows along K, words, along N
+])
+def test_long_k_of_more_than_half_a_round_of_tiles(types, m, k, n, nk, in_place):
+    dts = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[types]
+    p = M.Matmul([1, m, k, n], dts, layouts=[None, KT if nk else None, None]).plan()
+    assert (p.kernels == ["k_gemm_ring"] and "RA = " in p.steps[0].kernel) == in_place, p
