@@ -188,3 +188,12 @@ def test_long_k_of_more_than_half_a_round_of_tiles(types, m, k, n, nk, in_place)
     dts = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[types]
     p = M.Matmul([1, m, k, n], dts, layouts=[None, KT if nk else None, None]).plan()
     assert (p.kernels == ["k_gemm_ring"] and "RA = " in p.steps[0].kernel) == in_place, p
+
+
+@pytest.mark.parametrize("types,m,k,n,start", [("bf16", 45, 398, 408, 1), ("bf16", 45, 514, 325, 4), ("u8", 40, 1020, 2804, 1), ("u8", 40, 1028, 2804, 4),
+                                               ("bf16", 32, 398, 408, 4), ("bf16", 45, 399, 408, 1), ("bf16", 45, 400, 408, 16), ("f32", 45, 199, 408, 4)])
+def test_few_rows_on_words(types, m, k, n, start):
+    """One load a chunk, or for more than 32 rows over up to a unit of K a wave cut out of two."""
+    dts = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32), "f32": (M.f32,) * 3}[types]
+    p = M.Matmul([1, m, k, n], dts, layouts=[None, KT, None]).plan()
+    assert p.kernels == ["k_gemm_skinny"] and f"START = {start}," in p.steps[0].kernel, p
