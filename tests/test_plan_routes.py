@@ -197,3 +197,11 @@ def test_few_rows_on_words(types, m, k, n, start):
     dts = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32), "f32": (M.f32,) * 3}[types]
     p = M.Matmul([1, m, k, n], dts, layouts=[None, KT, None]).plan()
     assert p.kernels == ["k_gemm_skinny"] and f"START = {start}," in p.steps[0].kernel, p
+
+
+@pytest.mark.parametrize("b,m,keys,d,by_waves", [(8, 1651, 448, 64, False), (12, 1129, 534, 64, False), (25, 554, 640, 64, True), (29, 309, 832, 64, True), (43, 290, 443, 64, True),
+                                                 (45, 326, 325, 64, False), (5, 1770, 512, 32, True), (9, 1598, 323, 32, False), (9, 620, 300, 128, True)])
+def test_32_queries_a_workgroup(b, m, keys, d, by_waves):
+    """Two of them to a compute unit only where the keys are many enough."""
+    p = M.ComposeMSM(b, m, d, keys, d, layouts=[None, None, KT, None]).plan()
+    assert p.kernels == ["k_attn"] and ("QB = 2, W = 8" in p.steps[0].kernel) == by_waves, p
