@@ -136,12 +136,13 @@ uint32_t uneven_k_slices(const GemmArgs &g, int kind, bool conv, uint32_t *slice
     // int8 in two slices of eight steps, over half of the units and more in one piece already: 10 x (224 -> 16) x 33^2 3 x 3, 171 tiles of
     // 16 steps, 9.6 us whole, 10.2 in halves, 14 x (240 -> 16) x 30^2, 197 of 17, 10.4 and 11.0 (16 x (112 -> 16) x 26^2 5 x 5, 169 of 22, 12.0 and 11.5).
     if (kind <= 1 && tiles > 128 && steps < 18) pays = false;
-    // Equal slices where there are about as many (they end together), and where the above finds none worth it for long chains, which it has
-    // too short for many tiles (up to 0.5 us a step): us, whole or in so many uneven ones / equal: bf16 24 x (320 -> 320) x 10^2 3 x 3, 190 tiles of 45
-    // steps, 22.9 / 17.7 in three, 4 x (256 -> 288) x 24^2 18.8 / 15.1, 14 x (384 -> 112) x 26^2 28.0 / 26.4; 3 x (384 -> 160) x 15^2 5 x 5, 13.0 in 17 / 12.1
-    // in 15; fewer of them: 5 x (320 -> 112) x 11^2 5 x 5 14 / 5, 1.45 times as long; chains of 18 steps: 5 x (144 -> 112) x 26^2 1.2 times.
+    // Equal slices where there are about as many (they end together), and where the above finds none worth it, which has the steps
+    // too short for them (up to 0.5 us each), for long chains or few results: us, whole or in so many uneven ones / equal: bf16 24 x (320 -> 320) x 10^2 3 x 3, 190
+    // tiles of 45 steps, 22.9 / 17.7 in three, 4 x (256 -> 288) x 24^2 18.8 / 15.1, 14 x (384 -> 112) x 26^2 28.0 / 26.4, 9 x (192 -> 96) x 24^2, 27 steps,
+    // 14.8 / 12.2; 18 steps in two 4 x (128 -> 208) x 15^2, 187 thousand results, 10.7 / 9.6, 5 x (128 -> 48) x 40^2, 384 thousand, 10.7 / 10.8; 3 x (384 -> 160) x
+    // 15^2 5 x 5, 13.0 in 17 / 12.1 in 15; fewer of them: 5 x (320 -> 112) x 11^2 5 x 5 14 / 5, 1.45 times as long.
     const uint32_t equal = gemm_k_splits(g, kind);
-    if (equal > 1 && (pays ? 8 * equal >= 7 * count : steps >= 32)) {
+    if (equal > 1 && (pays ? 8 * equal >= 7 * count : steps >= 27 || (steps >= 18 && uint64_t(g.m) * g.n < 350000))) {
       *slice_k = g.k / equal;
       return equal;
     }

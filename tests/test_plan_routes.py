@@ -169,7 +169,9 @@ def test_int8_up_to_a_round_of_tiles_is_read_in_place(shape, layout):
 @pytest.mark.parametrize("dts,b,c,f,hw,fs,slices", [
     ("bf16", 24, 320, 320, 10, 3, 3), ("bf16", 4, 256, 288, 24, 3, 4), ("bf16", 22, 256, 96, 19, 3, 3), ("bf16", 14, 384, 112, 26, 3, 2),   # long chains: equal slices
     ("bf16", 3, 384, 160, 15, 5, 15), ("bf16", 14, 384, 64, 12, 5, 15),                        # as many equal ones but two
-    ("bf16", 5, 320, 112, 11, 5, 14), ("u8", 5, 384, 32, 13, 5, 9), ("bf16", 11, 128, 64, 15, 3, 1),   # many fewer; a short chain
+    ("bf16", 5, 320, 112, 11, 5, 14), ("u8", 5, 384, 32, 13, 5, 9),   # many fewer
+    ("bf16", 9, 192, 96, 24, 3, 3), ("bf16", 11, 128, 64, 15, 3, 2), ("bf16", 4, 128, 208, 15, 3, 2), ("u8", 4, 256, 48, 41, 3, 2),   # 27 steps, 18 under few results
+    ("bf16", 5, 128, 48, 40, 3, 1), ("bf16", 16, 128, 32, 27, 3, 1), ("u8", 6, 256, 64, 33, 3, 1),                                   # 18 under many
     ("u8", 10, 224, 16, 33, 3, 1), ("u8", 14, 240, 16, 30, 3, 1), ("u8", 8, 224, 32, 11, 3, 2)])        # int8: two short slices of many tiles, of few
 def test_slices_of_conv_windows(dts, b, c, f, hw, fs, slices):
     types = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[dts]
