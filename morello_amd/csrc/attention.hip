@@ -725,11 +725,13 @@ bool by_waves(AttnArgs &a, uint32_t shares) {
     return true;
   }
   a.query_block = 32;
-  // Two workgroups to a unit: from 384 keys on at head dim 32, from 640 on at 64, or from 384 where the other form would have 128 queries
-  // a workgroup (8 x 1651 x 64 against 448 keys 8.9 / 7.3, 12 x 1129 against 534 9.4 / 8.4, 25 x 554 against 640 9.7 / 10.1; 33 x 439 against 624, of
-  // 128, 9.8 / 10.8; 5 x 1770 x 32 against 512 5.9 / 6.5).
+  // Two workgroups to a unit: from 384 keys on at head dim 32.  At 64 from 1060 on, or 1300 where the other form has whole blocks on both sides
+  // (us, this / 64 queries in halves of the keys: 36 x 278 x 64 against 640 10.0 / 9.5, 9 x 955 against 1090 11.7 / 12.2, 17 x 580 against 1355 13.0 / 14.3;
+  // 14 x 960 against 1024 12.3 / 10.8, 12 x 960 against 1280 13.1 / 12.2), but from 384 where that one would have 128 queries (33 x 439 against 624
+  // 9.8 / 10.8; 5 x 1770 x 32 against 512 5.9 / 6.5).
   const uint64_t g128 = uint64_t(a.b) * ((a.m + 127) / 128);
-  if (a.n2 <= 2048 && (g32 <= units || (g32 <= room && a.n2 >= (a.k == 64 && 2 * g128 <= units ? 640u : 384u)))) return true;
+  const uint32_t enough = a.k != 64 || 2 * g128 > units ? 384 : a.m % 64 == 0 && a.n2 % 64 == 0 ? 1300 : 1060;
+  if (a.n2 <= 2048 && (g32 <= units || (g32 <= room && a.n2 >= enough))) return true;
   return false;
 }
 }  // namespace

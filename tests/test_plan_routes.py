@@ -201,7 +201,9 @@ def test_few_rows_on_words(types, m, k, n, start):
     assert p.kernels == ["k_gemm_skinny"] and f"START = {start}," in p.steps[0].kernel, p
 
 
-@pytest.mark.parametrize("b,m,keys,d,by_waves", [(8, 1651, 448, 64, False), (12, 1129, 534, 64, False), (25, 554, 640, 64, True), (29, 309, 832, 64, True), (43, 290, 443, 64, True),
+@pytest.mark.parametrize("b,m,keys,d,by_waves", [(8, 1651, 448, 64, False), (12, 1129, 534, 64, False), (25, 554, 640, 64, False), (29, 309, 832, 64, False), (8, 1046, 1030, 64, False),
+                                                 (9, 955, 1090, 64, True), (14, 960, 1024, 64, False), (12, 960, 1280, 64, False), (14, 704, 1344, 64, True),   # ragged, and whole blocks of 64
+                                                 (43, 290, 443, 64, True), (36, 398, 420, 64, True),                                                          # where the other form has 128 queries
                                                  (45, 326, 325, 64, False), (5, 1770, 512, 32, True), (9, 1598, 323, 32, False), (9, 620, 300, 128, True)])
 def test_32_queries_a_workgroup(b, m, keys, d, by_waves):
     """Two of them to a compute unit only where the keys are many enough."""
