@@ -209,3 +209,12 @@ def test_32_queries_a_workgroup(b, m, keys, d, by_waves):
     """Two of them to a compute unit only where the keys are many enough."""
     p = M.ComposeMSM(b, m, d, keys, d, layouts=[None, None, KT, None]).plan()
     assert p.kernels == ["k_attn"] and ("QB = 2, W = 8" in p.steps[0].kernel) == by_waves, p
+
+
+@pytest.mark.parametrize("b,m,keys,d,shares", [(34, 1, 3264, 128, 4), (18, 2, 5760, 128, 8), (20, 1, 4032, 128, 8), (51, 4, 2759, 64, 3), (124, 1, 1152, 64, 1),   # 25 to 64 MB of K and V
+                                               (47, 1, 896, 64, 1), (16, 1, 2800, 128, 6), (16, 1, 32768, 128, 16), (71, 2, 1885, 128, 3),                         # below, above
+                                               (6, 1, 8679, 128, 17)])                                                                                             # not 34: a third trip of the merge
+def test_shares_of_the_keys_in_decoding(b, m, keys, d, shares):
+    """Workgroups enough to stream K and V from memory, not from a cache that a model's other layers have been through."""
+    p = M.ComposeMSM(b, m, d, keys, d, layouts=[None, None, KT, None]).plan()
+    assert p.kernels == ["k_attn", "k_attn_merge"][:1 + (shares > 1)] and p.steps[0].grid == (b, shares, 1), p
