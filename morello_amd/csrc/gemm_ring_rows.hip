@@ -241,6 +241,23 @@ bool slices_are_faster(const GemmArgs &g, int kind, int es, uint64_t steps, uint
   const bool few_tiles = 8 * small <= 5 * units;
   return few_tiles && ((steps > 76 && a_whole && uint64_t(g.n) * g.k * es <= (11u << 20)) || (steps > 66 && kind <= 1 && !g.b_kmajor));
 }
+// 33 to 64 rows of whole chunks, which k_gemm reads in place too.  Its slices are the faster way (us, those / this):
+//   three equal ones or more against 30 MB of B or more: bf16 47 x 8192 x 5696 26.6 / 37.3, 56 x 4480 x 9721 25.5 / 33.7, 33 x 3456 x 14243 25.9 / 29.0,
+//     52 x 7040 x 2911 15.4 / 17.2, u8 41 x 10240 x 10752 31.0 / 40.2, 45 x 3840 x 8607 15.0 / 16.9 (less of B, or two slices, are even: bf16 50 x 5184 x 1329
+//     9.7 / 10.0, 63 x 4224 x 3216 13.2 / 12.8);
+//   with one left over, from 129 tiles to seven tenths of a round past 60 steps (u8 40 x 10496 x 8431 29.3 / 39.2, bf16 45 x 3904 x 8991 25.7 / 28.7; 63 x
+//     3904 x 12191, 191 tiles, 34.2 / 32.2); of whole steps, to five eighths past 52 as well, and past 110 steps and ten thousand of all tiles (bf16 35 x 8768
+//     x 5888 29.0 / 35.4, 39 x 11712 x 4800 32.2 / 33.8; 55 x 7736 x 4661, 73 tiles of 121, 32.3 / 29.0, 48 x 9520 x 5312, 148 and three quarters, 39.6 / 34.1).
+bool slices_are_faster_of_few(const GemmArgs &g, int kind, int es, uint64_t steps, uint64_t small, uint64_t units) {
+  const int64_t chunk = 16 / es;
+  if (g.lda % chunk != 0 || g.ldb % chunk != 0 || g.k % chunk != 0) return false;
+  uint32_t left = 0;
+  const uint32_t slices = gemm_k_splits(g, kind, &left);
+  if (left == 0) return slices >= 3 && uint64_t(g.n) * g.k * es >= 30000000;
+  if (2 * small > units && steps > 60) return 10 * small <= 7 * units;
+  if (uint64_t(g.k) * es % STEP != 0) return false;
+  return 2 * small > units ? steps > 52 && 8 * small <= 5 * units : steps > 110 && small * steps > 10000;
+}
 
 }  // namespace
 
@@ -267,6 +284,7 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
   const uint64_t units = g_compute_units, small = tiles(64, 64);
   if (small <= units) {
+    if (few && slices_are_faster_of_few(g, kind, es, steps, small, units)) return 0;
     if (2 * small <= units) return 32;
     if (steps > 88) return 0;   // (292 x 6007 x 2192 bf16, 175 tiles of 94 steps: 34.7 / 35.8)
     return g.batch == 1 && !few && slices_are_faster(g, kind, es, steps, small, units) ? 0 : 32;

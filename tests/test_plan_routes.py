@@ -218,3 +218,15 @@ def test_shares_of_the_keys_in_decoding(b, m, keys, d, shares):
     """Workgroups enough to stream K and V from memory, not from a cache that a model's other layers have been through."""
     p = M.ComposeMSM(b, m, d, keys, d, layouts=[None, None, KT, None]).plan()
     assert p.kernels == ["k_attn", "k_attn_merge"][:1 + (shares > 1)] and p.steps[0].grid == (b, shares, 1), p
+
+
+@pytest.mark.parametrize("types,m,k,n,in_place", [
+    ("bf16", 47, 8192, 5696, False), ("bf16", 33, 3456, 14243, False), ("u8", 45, 3840, 8607, False), ("bf16", 43, 4224, 14336, False),   # three equal slices of K or more
+    ("bf16", 50, 5184, 1329, True), ("bf16", 63, 4224, 3216, True), ("bf16", 56, 2816, 14053, True),                                      # ... of 14 and 27 MB of B; two
+    ("u8", 40, 10496, 8431, False), ("bf16", 45, 3904, 8991, False), ("bf16", 63, 3904, 12191, True), ("bf16", 46, 3904, 15168, True),    # one left over: 132, 141, 191, 237 tiles
+    ("bf16", 35, 8768, 5888, False), ("bf16", 55, 7736, 4661, True), ("bf16", 48, 9520, 5312, True), ("bf16", 52, 3712, 8704, False),     # many steps; whole ones
+    ("bf16", 57, 4478, 12288, True)])                                                                                                     # rows of no whole chunks
+def test_33_to_64_rows_over_a_long_k(types, m, k, n, in_place):
+    dts = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[types]
+    p = M.Matmul([1, m, k, n], dts, layouts=[None, KT, None]).plan()
+    assert p.kernels[0] == ("k_gemm_ring" if in_place else "k_gemm"), p
