@@ -150,14 +150,23 @@ hipError_t launch_as(const GemmArgs &g, hipStream_t stream) {
 
 template <int KIND>
 hipError_t launch_rows(const GemmArgs &g, hipStream_t stream) {
-  // One row of A: one row of B per wavefront from some 200 MB on (bf16 1 x 4096 x 32768 39.6 us against 42.3), two below (1 x 2048 x
-  // 16384 12.9 against 12.9, on one buffer again and again 10.8 against 11.3).  Two rows of A: one up to 80 MB (us, enough copies of
-  // B in turn that no cache holds them, two / one: u8 2 x 8192 x 8192 16.2 / 14.0, bf16 2 x 5056 x 5122 11.4 / 11.1; 2 x 6528 x 7726, 100 MB,
-  // 18.0 / 23.2; f32 2 x 2048 x 8192 14.8 / 14.0, but 11.9 / 12.9 on one buffer: two).  Loads through the caches, one row: 11.3 us for 1 x 2048 x 16384 while the 256 MB memory-side cache holds every B in
+  // Rows of B per wavefront (us, enough copies of B in turn that no cache holds them, two / one).
+  //   One row of A: one from some 200 MB on (bf16 1 x 4096 x 32768 42.3 / 39.6), two below (1 x 2048 x 16384 12.9 / 12.9, on one buffer again
+  //     and again 10.8 / 11.3).
+  //   Two rows of A, bf16: one up to 5200 rows of B, of which pairs are too few wavefronts (2 x 9144 x 3020 16.3 / 15.0, 2 x 5056 x 5122 11.4 / 11.1,
+  //     2 x 4592 x 5804 11.3 / 11.7, 2 x 3712 x 9142 15.5 / 20.3), or 6200 of 8 KiB, whole trips of the unrolled loop (2 x 4096 x 6144 11.8 / 10.9, x 6656 12.6 /
+  //     12.8), and up to 80 MB (2 x 6528 x 7726, 100 MB, 18.0 / 23.2).
+  //   Bytes: one up to 70 MB, of rows that are four trips of 1 KiB or more (2 x 11424 x 4800 18.7 / 15.4, 2 x 4448 x 10576 12.7 / 11.1, 2 x 8192 x 8192 16.2 / 14.0, 2 x 4096 x 11008 12.0 / 9.6;
+  //     2 x 3360 x 13907 13.8 / 16.4, 2 x 10144 x 7518 17.3 / 18.4).
+  //   f32: two (2 x 2048 x 8192 14.8 / 14.0, but 11.9 / 12.9 on one buffer).
+  // Loads through the caches, one row: 11.3 us for 1 x 2048 x 16384 while the 256 MB memory-side cache holds every B in
   // use, 14.7 when a program goes through more of them, as one that decodes through its layers does.
   const double bytes = double(g.n) * g.k * (KIND == 3 ? 4 : KIND == 2 ? 2 : 1) * g.batch;
   if (g.m == 1) return bytes >= 200e6 ? launch_as<KIND, 1, 1>(g, stream) : launch_as<KIND, 1, MRL_GEMV_COLS>(g, stream);
-  if (g.m == 2) return KIND != 3 && bytes <= 80e6 ? launch_as<KIND, 2, 1>(g, stream) : launch_as<KIND, 2, MRL_GEMV_COLS>(g, stream);
+  if (g.m == 2) {
+    const bool one = KIND == 2 ? uint64_t(g.n) * g.batch <= (g.k % 4096 == 0 ? 6200u : 5200u) && bytes <= 80e6 : KIND != 3 && g.k >= 4096 && bytes <= 70e6;
+    return one ? launch_as<KIND, 2, 1>(g, stream) : launch_as<KIND, 2, MRL_GEMV_COLS>(g, stream);
+  }
   if (g.m <= 4) return launch_as<KIND, 4, MRL_GEMV_COLS>(g, stream);
   return launch_as<KIND, MAX_ROWS, 2>(g, stream);
 }

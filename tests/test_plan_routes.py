@@ -230,3 +230,11 @@ def test_33_to_64_rows_over_a_long_k(types, m, k, n, in_place):
     dts = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[types]
     p = M.Matmul([1, m, k, n], dts, layouts=[None, KT, None]).plan()
     assert p.kernels[0] == ("k_gemm_ring" if in_place else "k_gemm"), p
+
+
+@pytest.mark.parametrize("types,k,n,rows", [("bf16", 9152, 3008, 1), ("bf16", 5056, 5122, 1), ("bf16", 4592, 5804, 2), ("bf16", 3712, 9142, 2), ("bf16", 4096, 6144, 1), ("bf16", 4096, 6656, 2),
+                                            ("bf16", 6528, 7726, 2), ("u8", 11424, 4800, 1), ("u8", 8192, 8192, 1), ("u8", 4096, 11008, 1), ("u8", 3360, 13907, 2), ("u8", 10144, 7518, 2)])
+def test_rows_of_b_a_wavefront_for_two_rows_of_a(types, k, n, rows):
+    dts = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[types]
+    p = M.Matmul([1, 2, k, n], dts, layouts=[None, KT, None]).plan()
+    assert p.kernels == ["k_gemv"] and f"ROWS = 2, COLS = {rows}]" in p.steps[0].kernel, p
