@@ -1294,9 +1294,9 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
     }
   }
   // A shared contiguous digit in whole vectors on both sides: 16, 8 or 4 bytes on the wider side.
-  // From 32-bit elements to 16-bit ones 16 bytes on the narrower side where the source's rows lie multiples of 8 KiB apart, on
-  // the same memory channels (us, buffers taking turns, before -> now: f32 2048 x 16384 into bf16 strips of 16 44.7 -> 42.0, 8192 x 8192 97.4 -> 81.4,
-  // 4096 x 8192 44.1 -> 40.9, 512 x 16384 11.3 -> 10.3; other rows either way: 7232 x 6800 56.9 -> 58.9, 8192 x 3072 30.6 -> 32.0).
+  // From 32-bit elements to 16-bit ones 16 bytes on the narrower side where the source's rows lie 8, 16, 32 or 64 KiB apart, on the
+  // same memory channels (us, four elements a vector / eight: f32 2048 x 16384 into bf16 strips of 16 44.9 / 42.2, 4096 x 16384 109 / 84, 8192 x 8192 98 / 82, 1024 x 4096 8.7 /
+  // 7.9, 2048 x 2048 9.0 / 8.0; other rows: 2048 x 12288 30.3 / 33.3, 2048 x 10240 25.3 / 28.0, 8192 x 6144 58.6 / 62.1, 1024 x 32768 39.7 / 41.6).
   const size_t widest = std::max(se, de);
   uint32_t vec = 0;
   // `row`: bytes from one row of the source to the next, the source's step along the digit that continues the destination's runs:
@@ -1306,7 +1306,7 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
   int64_t least = 0;
   for (uint32_t d = 0; d < rank; d++)
     if (int(d) != dim_d && p.shape[d] > 1 && (row == 0 || p.ds[d] < least)) row = uint64_t(p.ss[d]) * se, least = p.ds[d];
-  const bool pages = se == 4 && de == 2 && p.count > MOVE_SMALL && row != 0 && row % 8192 == 0;
+  const bool pages = se == 4 && de == 2 && p.count > MOVE_SMALL && (row == 8192 || row == 16384 || row == 32768 || row == 65536);
   if (shared && rank > 1)
     for (uint32_t v = uint32_t(16 / widest) * (pages ? 2 : 1); vec == 0 && v >= 1 && v * widest >= 4; v /= 2) {
       bool fits = v > 1 && p.shape[dim_s] % v == 0 && (reinterpret_cast<uintptr_t>(src) % std::min<size_t>(16, v * se)) == 0 &&

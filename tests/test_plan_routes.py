@@ -147,9 +147,10 @@ def test_fused_takes_the_query_blocks_it_documents(tile_m):
 
 
 @pytest.mark.parametrize("shape,wide", [([1, 2048, 16384], True), ([1, 8192, 3072], False), ([2, 8192, 3072], False), ([2, 8192, 2048], True),
-                                        ([3, 4097, 2048], True), ([8, 1024, 1536], False), ([4, 1, 700, 4096], True)])
+                                        ([3, 4097, 2048], True), ([8, 1024, 1536], False), ([4, 1, 700, 4096], True),
+                                        ([1, 2048, 6144], False), ([1, 2048, 10240], False), ([1, 2048, 12288], False), ([1, 8192, 8192], True), ([1, 1024, 32768], False)])
 def test_wide_narrowing_vectors_where_rows_lie_8_kib_apart(shape, wide):
-    """Rows, not the entries of a batch: two of 8192 x 3072 are a multiple of 8 KiB apart and their rows 12."""
+    """... or 16, 32 or 64.  Rows, not the entries of a batch: two of 8192 x 3072 are a multiple of 8 KiB apart and their rows 12."""
     r = len(shape)
     strips = M.layout(*range(r - 2), r - 1, r - 2, (r - 1, M.Packed(16)))
     p = M.Move(shape, (M.f32, M.bf16), layouts=[None, strips]).plan()
