@@ -239,3 +239,13 @@ def test_rows_of_b_a_wavefront_for_two_rows_of_a(types, k, n, rows):
     dts = {"bf16": (M.bf16, M.bf16, M.f32), "u8": (M.u8, M.i8, M.i32)}[types]
     p = M.Matmul([1, 2, k, n], dts, layouts=[None, KT, None]).plan()
     assert p.kernels == ["k_gemv"] and f"ROWS = 2, COLS = {rows}]" in p.steps[0].kernel, p
+
+
+@pytest.mark.parametrize("b,m,k,n,out,accum,in_place", [
+    (1, 43, 1273, 4452, M.f32, False, False), (1, 43, 1084, 5269, M.f32, False, True), (1, 35, 971, 8647, M.f32, False, True), (1, 39, 1603, 3436, M.f32, False, True),   # few rows: odd, words, 136 tiles, slices
+    (2, 581, 2761, 1178, M.bf16, False, False), (2, 887, 1961, 904, M.f32, False, False), (2, 1343, 1481, 639, M.f32, False, True), (2, 581, 2762, 1178, M.f32, False, True),   # 44, 31, 24 steps; words
+    (2, 789, 1007, 1167, M.f32, False, False), (1, 2399, 1307, 925, M.bf16, False, False), (2, 598, 1019, 3125, M.f32, False, True), (2, 1101, 829, 1540, M.bf16, False, True),   # 128 x 128: 16, 21 steps, 250 tiles, 13 steps
+    (1, 1749, 173, 1407, M.bf16, True, False), (1, 1749, 173, 1407, M.bf16, False, True), (1, 1749, 174, 1408, M.bf16, True, True)])                                          # onto bf16
+def test_odd_rows_of_bf16_along_k(b, m, k, n, out, accum, in_place):
+    p = M.Matmul([b, m, k, n], (M.bf16, M.bf16, out), accum=accum, layouts=[None, KT, None]).plan()
+    assert (p.kernels[0] == "k_gemm_ring" and "RA = " in p.steps[0].kernel) == in_place, p
