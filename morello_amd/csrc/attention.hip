@@ -669,8 +669,9 @@ uint32_t query_block_of(const AttnArgs &a) {
 
 // Key splits of the form that deals keys to waves, `groups` workgroups without them: the cheapest by
 //   rounds of a workgroup's eight blocks of 32 keys, each 0.9 us at head dim 128 (131 KB a round), 0.35 at 64;
-//   K and V at what the workgroups stream together: each 140 bytes a nanosecond from L2, 100 from the memory-side cache, 50 and, of
-//     much, 42 from memory, 6500 at most.  From 25 MB on they are taken to come from memory: a cache that grows by a token a
+//   K and V at what the workgroups stream together: each 140 bytes a nanosecond from L2 (up to 8 MB: 8 x 2 x 64
+//     against 1408 keys in 1 6.1, in 3 8.2; 16 x 1 x 64 against 2240 8.4 and 6.9), 100 from the memory-side cache, 50 and, of much, 42 from
+//     memory, 6500 at most.  From 25 MB on they are taken to come from memory: a cache that grows by a token a
 //     step is one of a model's many layers (us, at 100 a workgroup / at 50, buffers in turn that no cache holds: 34 x 1 x 128
 //     against 3264 keys in 2 splits 21.2, in 4 14.8; 18 x 2 x 128 against 5760 in 4 19.9, in 8 14.8; 49 x 1 x 64 against 2816 in 1 16.3, in 3 11.1;
 //     on one buffer again and again 20 x 1 x 128 against 4032 10.8 and 10.7, 73 x 1 x 64 against 2176 8.8 and 10.1);
@@ -680,7 +681,7 @@ uint32_t query_block_of(const AttnArgs &a) {
 uint32_t key_splits_of_waves(const AttnArgs &a, uint64_t groups) {
   const uint64_t blocks = (a.n2 + 31) / 32, most = std::min<uint64_t>(g_compute_units / groups, blocks / 8);
   const double bytes = 4.0 * a.b * a.n2 * a.k, round_ns = a.k == 128 ? 900 : a.k == 64 ? 350 : 250,
-               share = bytes > 64e6 ? 42 : bytes > 25e6 ? 50 : bytes > 16e6 ? 100 : 140;
+               share = bytes > 64e6 ? 42 : bytes > 25e6 ? 50 : bytes > 8e6 ? 100 : 140;
   auto ns = [&](uint64_t s) {
     const uint64_t rounds = ((blocks + s - 1) / s + 7) / 8;
     return std::max(double(rounds) * round_ns, bytes / std::min(double(groups * s) * share, 6500.0)) + (s > 1 ? 2700.0 + 20.0 * double(s) + 800.0 * double((s - 1) / 16) : 0.0);
