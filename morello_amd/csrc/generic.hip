@@ -1142,8 +1142,9 @@ uint32_t runs_tile(const MoveStrided &p, uint32_t shared, uint32_t vec, uint32_t
   };
   const int next_d = next(p.ds, -1), next_s = next(p.ss, -1);
   if (next_d >= 0 && next_s >= 0 && next_s != next_d) {
-    // 512 bytes of the source side (of 32 a vector 1 KiB: 42.9 / 40.9 us at 2048 x 16384), along two digits if need be, the rest of the tile along the destination's
-    const uint32_t piece = vec * se == 32 ? 1024 : 512;
+    // 512 bytes of the source side, along two digits if need be, the rest of the tile along the destination's (of 32 a vector from rows 32 KiB
+    // apart 1 KiB: f32 2048 x 16384 into bf16 strips of 16 43.9 / 42.0 us, 8192 x 8192 87.2 / 81.1; but 4096 x 4096 18.8 / 20.5)
+    const uint32_t piece = vec * se == 32 && p.ss[next_d] * int64_t(vec * se) >= 32768 ? 1024 : 512;
     const uint32_t want_s = std::min(std::max(1u, piece / (ext[shared] * vec * se)), std::max(1u, tile_cap / tile));
     const int further = p.shape[next_s] < want_s ? next(p.ss, next_s) : -1;
     const bool two = further >= 0 && further != next_d;
