@@ -461,7 +461,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
                    : (da == MRL_BF16 && db == MRL_BF16 && (dc == MRL_F32 || dc == MRL_BF16)) ? 2
                    : (da == MRL_F32 && db == MRL_F32 && dc == MRL_F32)   ? 3
                                                                          : -1;
-  g.c_bf16 = dc == MRL_BF16;
+  g.c_bf16 = dc == MRL_BF16, g.tight = g_tight_scratch;
   // Few rows, or a small problem: read in place whatever the rows' alignment.
   const uint32_t in_place = !sched && rows ? mrl::gemm_ring_rows_columns(g, kind) : 0;
   const bool few = in_place != 0 && g.m <= 64;   // (rows enough for the tiles below all the same)

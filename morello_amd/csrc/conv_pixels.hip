@@ -273,7 +273,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
 // a workgroup takes 32 filters, and the operand of patch row r serves every pair of a step and an output row with
 // RPS * step + row = r.  What bounded the form above beside its stores was LDS, 56 KB read per 16 x 2 pixels and 64 filters of bf16
 // 7 x 7; here 16 KB are.  Bound now by the stores of the output and by the start (filters staged, a first patch: 4 us). us, the
-// form above / this: bf16 7 x 7 16 x 3 -> 64 x 109^2 16.7 / 15.2, 32 x 3 -> 96 x 224^2 152 / 127, u8 7 x 7 12 x 4 -> 96 x 76^2 12.6 / 9.9.
+// form above / this: bf16 7 x 7 16 x 3 -> 64 x 109^2 17.2 / 15.5, 32 x 3 -> 96 x 224^2 154 / 131, u8 7 x 7 12 x 4 -> 96 x 76^2 12.5 / 8.8.
 template <int KS, int RPS, bool TAIL, int KIND, bool PIXELS>
 __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
   typedef Pixels<KIND> P;
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
     if (p.whole_lines) {
       // A pixel's 32 filters are a cache line: lanes of pixels 0 .. 7 and 8 .. 15 exchange a block, so that a store is eight whole
       // lines and not sixteen halves, and they go past the caches (32 x 3 -> 96 x 224^2 bf16 7 x 7: 156 us in halves, 148 in
-      // lines, 127 in lines past the caches; halves past the caches 197).
+      // lines, 131 in lines past the caches; halves past the caches 197).
       const bool low = li < 8;
       const uint32_t x = at.x0 + (li & 7);
 #pragma unroll

@@ -283,6 +283,8 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
     return 0;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
   const uint64_t units = g_compute_units, small = tiles(64, 64);
+  if (g.tight)   // no scratch for copies or partial results, whatever it costs
+    return small <= units ? 32 : tiles(128, 64) <= units ? 64 : kind == 2 && g.n >= 128 && tiles(128, 128) <= units ? 128 : 0;
   // bf16 rows of an odd number of elements along K, a pair of lines for every 128 bytes of either operand: most where the operands come
   // from memory (us, those / this, from memory and with three sets of operands in turn, which the memory-side cache keeps).
   const bool odd_rows = kind == 2 && g.b_kmajor && (g.lda % 2 != 0 || g.ldb % 2 != 0);
@@ -298,12 +300,12 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
   // In one entry from 41 steps on (1031 x 2937 x 1194 26.7 / 32.0, 407 x 2585 x 2924 24.4 / 26.9; 231 x 2739 x 4310 27.5 / 26.5, 2270 x 2473 x 710 26.5 / 24.5), in several
   // from 31 (twice 581 x 2761 x 1178 28.5 / 37.2, 27.0 / 29.4, 887 x 1961 x 904 24.6 / 28.3, 22.7 / 21.6; 1343 x 1481 x 639 24.6 / 25.5, 22.4 / 19.3).
   if (tiles(128, 64) <= units) return steps <= (kind != 2 ? 24u : !odd_rows ? 48u : g.batch == 1 ? 40u : 30u) ? 64 : 0;
-  // Of 128 x 128 up to three quarters of a round from 16 (twice 789 x 1007 x 1167 20.9 / 25.1, 19.0 / 21.1, 2399 x 1307 x 925 25.3 / 28.5, 23.5 / 22.6;
+  // Of 128 x 128 up to two thirds of a round from 16 (twice 789 x 1007 x 1167 20.9 / 25.1, 19.0 / 21.1, 2399 x 1307 x 925 25.3 / 28.5, 23.5 / 22.6;
   // twice 598 x 1019 x 3125, 250 tiles, 27.0 / 26.2, 24.1 / 20.4).
   // Onto bf16 results over up to five steps an element a lane, which odd rows leave, is the slower end (1749 x 173 x 1407 11.9 / 14.7, 11.2 / 12.2).
   const uint64_t large = tiles(128, 128);
   if (kind != 2 || g.n < 128 || large > units || (g.accum && g.c_bf16 && steps <= 5 && (g.lda % 2 != 0 || g.ldb % 2 != 0))) return 0;
-  return steps <= (odd_rows && 4 * large <= 3 * units ? 15u : 24u) ? 128 : 0;
+  return steps <= (odd_rows && 3 * large <= 2 * units ? 15u : 24u) ? 128 : 0;
 }
 
 hipError_t launch_gemm_ring_rows(const GemmArgs &g, int kind, hipStream_t stream) {

@@ -495,7 +495,7 @@ __global__ __launch_bounds__(256) void k_move_tiled32(MoveStrided p) {
 // by memory, so what matters is the order: a workgroup's tile is long along the digit that
 // continues the destination's runs AND along the one that continues the source's, so that both
 // sides see whole cache lines (f32 2048 x 16384 into bf16 strips of 16 columns, runs of 64 and
-// 32 bytes: an element per thread in destination order 133 us, this 41).  UNROLL vectors a
+// 32 bytes: an element per thread in destination order 133 us, this 42).  UNROLL vectors a
 // thread, their loads in flight together.
 constexpr int MOVE_RUNS_ACT = 4;   // digits a tile extends along at most
 template <int SE, int DE, int V, int UNROLL>

@@ -143,6 +143,8 @@ struct GemmArgs {
   // K shared out over batch entries: each has `k` elements, the last what is left of k_total (0: `k` each).  The
   // Conv build of k_gemm and gemm_ring_rows.hip take it.
   uint32_t k_total = 0;
+  // Scratch is short: rows are read in place wherever that is possible (gemm_ring_rows.hip).
+  bool tight = false;
   // C is bf16 (bf16 operands only): the f32 sum, the old value included, is rounded once.
   bool c_bf16 = false;
   // Conv as an implicit Matmul (the CONV build of the kernel): `a` is a channels-last image
