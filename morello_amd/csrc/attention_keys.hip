@@ -14,7 +14,7 @@
 // is in flight at any time and eight waves keep 64 to 128 KiB of a compute unit's requests under way.
 // What bounds it: the stream of K and V where they are large (16 x 1 x 128 against 32768 keys, 268 MB that no cache holds:
 // 53.6 us before, 50.7 now, of which the merging launch and its gap are 5 to 6), and otherwise the trip to memory of a round
-// of 256 keys (0.9 us at D = 128 from L2): 4 x 1 x 128 against 564 keys 10.1 -> 5.5 us, 16 x 103 x 80 against 767 11.9 -> 6.7,
+// of 256 keys (0.9 us at D = 128 from L2): 4 x 1 x 128 against 564 keys 10.1 -> 5.4 us, 16 x 103 x 80 against 767 11.9 -> 6.7,
 // 13 x 346 x 80 against 1088 15.4 -> 9.6.
 #include <algorithm>
 
