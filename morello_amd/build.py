@@ -18,7 +18,7 @@ GEN_DIR = os.path.join(OBJ_DIR, "gen")   # generated assembly (the k loops of th
 # generator -> the file the kernel header of the same tile includes
 GENERATED = {"gen_gemm_wide.py": "gemm_wide_gfx950.inc", "gen_gemm_loop.py": "gemm_loop_gfx950.inc"}
 
-SOURCES = ["api.hip", "generic.hip", "move_gather_1.hip", "move_gather_2.hip", "move_gather_4.hip", "gemm_mfma.hip", "gemm_sched.hip", "gemm_nt.hip", "gemm_wide_edge.hip", "gemm_ring.hip", "gemm_ring_rows.hip", "gemv.hip", "gemm_skinny.hip", "conv_gemm.hip", "conv_i8.hip", "conv_windows.hip", "conv_pixels.hip", "conv_small.hip", "unfold.hip", "softmax.hip", "parts.hip", "mfma_rate.hip", "attention.hip", "attention_keys.hip", "plan.hip", "host_stage.hip"]
+SOURCES = ["api.hip", "generic.hip", "move_gather_1.hip", "move_gather_2.hip", "move_gather_4.hip", "gemm_mfma.hip", "gemm_sched.hip", "gemm_nt.hip", "gemm_wide_edge.hip", "gemm_ring.hip", "gemm_ring_rows.hip", "gemm_f32.hip", "gemv.hip", "gemm_skinny.hip", "conv_gemm.hip", "conv_i8.hip", "conv_windows.hip", "conv_pixels.hip", "conv_small.hip", "unfold.hip", "softmax.hip", "parts.hip", "mfma_rate.hip", "attention.hip", "attention_keys.hip", "plan.hip", "host_stage.hip"]
 
 # -packed-fp32-ops off: the compiler must not form v_pk_{add,mul,fma}_f32.
 FLAGS = [

@@ -462,11 +462,33 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
                    : (da == MRL_F32 && db == MRL_F32 && dc == MRL_F32)   ? 3
                                                                          : -1;
   g.c_bf16 = dc == MRL_BF16, g.tight = g_tight_scratch;
+  // One launch, or slices of K as batch entries with partial results, summed into C in slice order.
+  auto in_slices = [&](uint32_t count, uint32_t slice_k, auto launch) -> int {
+    if (count == 1) {
+      HIP_TRY(launch(g));
+      return MRL_OK;
+    }
+    void *partial = nullptr;
+    HIP_TRY(ws.alloc(&partial, size_t(count) * g.m * g.n * 4));
+    mrl::GemmArgs slices = g;
+    slices.batch = count, slices.k = slice_k, slices.k_total = g.k;
+    slices.sa = slice_k, slices.sb = g.b_kmajor ? int64_t(slice_k) : int64_t(slice_k) * g.ldb;
+    slices.c = partial, slices.ldc = g.n, slices.sc = int64_t(g.m) * g.n, slices.accum = 0, slices.c_bf16 = false;
+    HIP_TRY(launch(slices));
+    HIP_TRY(mrl::launch_sum_splits(partial, g.c, count, g.m, g.n, g.ldc, g.accum != 0, kind <= 1, g.c_bf16, ws.stream));
+    return MRL_OK;
+  };
   // Few rows, or a small problem: read in place whatever the rows' alignment.
   const uint32_t in_place = !sched && rows ? mrl::gemm_ring_rows_columns(g, kind) : 0;
   const bool few = in_place != 0 && g.m <= 64;   // (rows enough for the tiles below all the same)
   if (!sched && kind >= 0 && rows && !few && mrl::gemm_skinny_applicable(g, kind)) {
     HIP_TRY(mrl::launch_gemm_skinny(g, kind, ws.stream));
+    return finish_output(c, ws);
+  }
+  if (!sched && rows && mrl::gemm_f32_applicable(g, kind)) {
+    uint32_t slice_k = 0;
+    const uint32_t count = mrl::gemm_f32_slices(g, &slice_k);
+    if ((rc = in_slices(count, slice_k, [&](const mrl::GemmArgs &a) { return mrl::launch_gemm_f32(a, ws.stream); })) != MRL_OK) return rc;
     return finish_output(c, ws);
   }
   // Rows that are not whole 16-byte chunks, in a problem small enough that copies of them would be a third of its time: read
@@ -481,18 +503,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   if (in_place != 0 && (ragged || few || (steps_pay && (mrl::gemm_k_splits(g, kind, &k_left) == 1 || k_left != 0)))) {
     uint32_t slice_k = 0;
     const uint32_t splits = g_tight_scratch ? 1 : mrl::uneven_k_slices(g, kind, false, &slice_k);
-    if (splits == 1) {
-      HIP_TRY(mrl::launch_gemm_ring_rows(g, kind, ws.stream));
-    } else {
-      void *partial = nullptr;
-      HIP_TRY(ws.alloc(&partial, size_t(splits) * g.m * g.n * 4));
-      mrl::GemmArgs slices = g;
-      slices.batch = splits, slices.k = slice_k, slices.k_total = g.k;
-      slices.sa = slice_k, slices.sb = g.b_kmajor ? int64_t(slice_k) : int64_t(slice_k) * g.ldb;
-      slices.c = partial, slices.ldc = g.n, slices.sc = int64_t(g.m) * g.n, slices.accum = 0, slices.c_bf16 = false;
-      HIP_TRY(mrl::launch_gemm_ring_rows(slices, kind, ws.stream));
-      HIP_TRY(mrl::launch_sum_splits(partial, g.c, splits, g.m, g.n, g.ldc, g.accum != 0, kind <= 1, g.c_bf16, ws.stream));
-    }
+    if ((rc = in_slices(splits, slice_k, [&](const mrl::GemmArgs &a) { return mrl::launch_gemm_ring_rows(a, kind, ws.stream); })) != MRL_OK) return rc;
     return finish_output(c, ws);
   }
   // Operands the matrix-core kernels cannot walk in place are copied with the strided Move
@@ -1767,7 +1778,7 @@ uint32_t mrl_target_layouts_for_shape(const uint32_t *shape, uint32_t rank, int 
 
 uint32_t mrl_target_kernels(const char **names, uint32_t cap) {
   static const char *const families[] = {
-      "k_gemm", "k_gemm_big", "k_gemm_wide", "k_gemv", "k_gemm_ring", "k_gemm_skinny", "k_gemm_tiny", "k_matmul_generic", "k_sum_splits", "k_conv_i8", "k_conv_rows_i8", "k_conv_windows", "k_conv_small", "k_conv_generic", "k_conv_generic_wave", "k_unfold",
+      "k_gemm", "k_gemm_big", "k_gemm_wide", "k_gemv", "k_gemm_ring", "k_gemm_skinny", "k_gemm_tiny", "k_gemm_f32", "k_gemm_f32_waves", "k_matmul_generic", "k_sum_splits", "k_conv_i8", "k_conv_rows_i8", "k_conv_windows", "k_conv_small", "k_conv_generic", "k_conv_generic_wave", "k_unfold",
       "k_unfold_gather", "k_attn", "k_attn_merge", "k_softmax_regs", "k_softmax_short", "k_softmax_block", "k_softmax_chunk_stats", "k_softmax_chunk_write",
       "k_softmax_cols",
       "k_softmax_generic", "k_softmax_cols_short", "k_parts", "k_parts_block", "k_parts_rows", "k_parts_cols", "k_broadcast", "k_broadcast_rows", "k_broadcast_fill_rows", "k_fill", "k_fill16", "k_fill_zero", "k_move_rows", "k_move_runs",

@@ -1,0 +1,539 @@
+// f32 Matmul through the bf16 matrix cores: every f32 as three bf16 that add up to it exactly.
+//
+// The f32 MFMA has a sixteenth of the bf16 one's rate.  A value's upper 16 bits are a bf16 (h); what is left has 16 bits, of
+// which the rounded upper half (m) and the rest (l) are bf16 too: x = h + m + l without error, and
+//   x y = h h' + (h m' + m h') + (m m' + h l' + l h') + the rest, below 2^-23 |x y| and of either sign:
+// six MFMAs for sixteen k where the f32 form takes eight of twice the time each.  The products but the first are summed on
+// their own.  The roundings of a sum, one to sixteen terms and not to two, then come to less than those of the f32 MFMA: relative
+// error in the norm for 0.5 x normal operands, f32 MFMA / this: K = 128 9.3e-8 / 6.5e-8, 1024 5.7e-7 / 1.3e-7, 2048 8.1e-7 / 1.9e-7.
+//
+// Where the parts would not do, the tile is computed again by the f32 MFMA: an infinity in A or B leaves a NaN (its m is inf - inf),
+// and so does an overflow on the way; and in a row of A or column of B of nothing but tiny values the l, then the m, are no
+// bf16 any more.  Each thread keeps the largest magnitude of what it cuts up, all of one row or column.  (All tiles twice: 2048^3 with
+// an infinity in every sixteenth row 370 us, 512^3 18.)
+//
+// What bounds it: the bf16 MFMAs at what the board's power lets them run at (4096^3 in 695 us is 1.19 PFLOP/s of them, where the 256 tile
+// reaches 1.42), for the smaller tiles the cutting, six vector instructions a value; below a round of tiles the chain of a step.
+//
+// Rows start on any element and are read in place.  The first step takes what K has over whole steps, zeros behind it, so that no
+// load but its leaves K and none is masked; rows past M and columns past N are the last one again and are not stored.
+// Semantics: morello/src/spec.rs:480-485.
+#include "gemm_ring.h"
+
+namespace mrl {
+namespace {
+using gemm::TileWalk;
+using gemm::v4i;
+using gemm::v8bf;
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef float four_on_word __attribute__((ext_vector_type(4), aligned(4)));
+
+// A row or column whose largest magnitude reaches it loses nothing that counts beside that value (its lowest bit is 2^-113, a bf16
+// goes down to 2^-126 without denormals).
+constexpr float TINY = 0x1p-90f;
+
+struct Parts { v4i h, m, l; };
+// Eight values as three chunks of eight bf16; `most`: the largest magnitude so far.
+__device__ inline Parts cut(const float *x, float &most) {
+  Parts p;
+  float r[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) r[i] = x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xffff0000u);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    p.h[i] = int(__builtin_amdgcn_perm(__float_as_uint(x[2 * i + 1]), __float_as_uint(x[2 * i]), 0x07060302));   // the upper halves
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(x[2 * i]), "v"(x[2 * i + 1]));
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) p.m[i] = __builtin_bit_cast(int, __builtin_convertvector((v2f{r[2 * i], r[2 * i + 1]}), v2bf));
+#pragma unroll
+  for (int i = 0; i < 4; i++) r[2 * i] -= __uint_as_float(uint32_t(p.m[i]) << 16), r[2 * i + 1] -= __uint_as_float(uint32_t(p.m[i]) & 0xffff0000u);
+#pragma unroll
+  for (int i = 0; i < 4; i++) p.l[i] = int(__builtin_amdgcn_perm(__float_as_uint(r[2 * i + 1]), __float_as_uint(r[2 * i]), 0x07060302));
+  return p;
+}
+
+__device__ inline v16f mfma(v4i a, v4i b, v16f c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+
+// Operands of one batch entry (or slice of K), in bytes where they are strides.
+struct Problem {
+  const uint8_t *a, *b;
+  float *c;
+  int64_t m, n;
+  uint32_t lda_b, ldb_b;
+  int k;
+  __device__ explicit Problem(const GemmArgs &g) {
+    a = (const uint8_t *)((const float *)g.a + int64_t(blockIdx.y) * g.sa), b = (const uint8_t *)((const float *)g.b + int64_t(blockIdx.y) * g.sb);
+    c = (float *)g.c + int64_t(blockIdx.y) * g.sc;
+    m = g.m, n = g.n, lda_b = uint32_t(g.lda) * 4, ldb_b = uint32_t(g.ldb) * 4;
+    k = g.k_total != 0 ? int(min(g.k, g.k_total - blockIdx.y * g.k)) : int(g.k);
+  }
+};
+
+// No number where one of the sums is none, or infinite.
+template <int N>
+__device__ inline float probe_of(const float (&sum)[N]) {
+  float probe = 0.0f;
+#pragma unroll
+  for (int e = 0; e < N; e++) probe = __builtin_fmaf(0.0f, sum[e], probe);
+  return probe;
+}
+
+// Whether a tile's parts did: no value that is infinite or no number among this thread's sums, and no row of A or column of B, whose
+// N largest magnitudes this thread keeps (`which`: numbers of theirs below `all`), of nothing but tiny values.  Of the workgroup.
+template <int N>
+__device__ inline bool parts_did(const float (&most)[N], const int (&which)[N], int all, float probe, uint32_t *seen) {
+  bool odd = probe != probe;
+#pragma unroll
+  for (int i = 0; i < N; i++) odd = odd || !(most[i] >= TINY);
+  if (!__syncthreads_or(odd)) return true;
+  if (__syncthreads_or(probe != probe)) return false;
+  for (int i = threadIdx.x; i < all; i += blockDim.x) seen[i] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; i++) atomicMax(seen + which[i], __float_as_uint(most[i]));
+  __syncthreads();
+  bool tiny = false;
+  for (int i = threadIdx.x; i < all; i += blockDim.x) tiny = tiny || (seen[i] != 0 && seen[i] < __float_as_uint(TINY));
+  return !__syncthreads_or(tiny);
+}
+
+// The `share`-th of SHARES parts of a wave's T x T blocks, block after block.  Register i of a block: row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32.
+template <int T, int SHARES>
+__device__ inline void store(const Problem &p, int64_t m0, int64_t n0, int share, bool accum, int64_t ldc, const float (&sum)[T * T * 16 / SHARES]) {
+  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
+#pragma unroll
+  for (int e = 0; e < T * T * 16 / SHARES; e++) {
+    const int reg = share * (T * T * 16 / SHARES) + e, block = reg / 16, i = reg % 16;
+    const int64_t row = m0 + block / T * 32 + 8 * (i / 4) + 4 * lh + i % 4, col = n0 + block % T * 32 + li;
+    if (row < p.m && col < p.n) {
+      float *at = p.c + row * ldc + col;
+      *at = accum ? sum[e] + *at : sum[e];
+    }
+  }
+}
+
+// The sums of PARTS waves that share T x T blocks meet in LDS, [part][wave of the tile][register][lane]; each wave takes its share.
+// `lds`: the first part's, `stride` floats before the next one's, which nobody reads any more once all are here.
+template <int T, int PARTS>
+__device__ inline void meet(float *lds, int stride, int wave_of_tile, int part, const v16f (&acc)[T][T], float (&sum)[T * T * 16 / PARTS]) {
+  constexpr int REGS = T * T * 16, MINE = REGS / PARTS;
+  if constexpr (PARTS == 1) {
+#pragma unroll
+    for (int e = 0; e < REGS; e++) sum[e] = acc[e / 16 / T][e / 16 % T][e % 16];
+  } else {
+    float *const at = lds + wave_of_tile * (REGS * 64) + (threadIdx.x & 63);
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < REGS; e++) at[part * stride + e * 64] = acc[e / 16 / T][e / 16 % T][e % 16];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < MINE; e++) {
+      sum[e] = at[(part * MINE + e) * 64];
+#pragma unroll
+      for (int q = 1; q < PARTS; q++) sum[e] += at[q * stride + (part * MINE + e) * 64];
+    }
+  }
+}
+
+// T x T blocks of 32 x 32 from (m0, n0) on by the f32 MFMA, every PARTS-th sixteen k: what the parts of a value cannot do.
+template <int T, int PARTS, bool B_KMAJOR>
+__device__ inline void multiply_f32(const Problem &p, int64_t m0, int64_t n0, int part, v16f (&acc)[T][T]) {
+  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
+  const float *a[T], *b[T];
+#pragma unroll
+  for (int t = 0; t < T; t++) {
+    const int64_t row = min(m0 + 32 * t + li, p.m - 1), col = min(n0 + 32 * t + li, p.n - 1);
+    a[t] = (const float *)(p.a + row * p.lda_b), b[t] = (const float *)(p.b + (B_KMAJOR ? col * p.ldb_b : col * 4));
+#pragma unroll
+    for (int c = 0; c < T; c++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[t][c][i] = 0.0f;
+  }
+  for (int k0 = 16 * part; k0 < p.k; k0 += 16 * PARTS) {
+    float x[8][T], y[8][T];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int at = min(k0 + 8 * lh + i, p.k - 1);
+#pragma unroll
+      for (int t = 0; t < T; t++) x[i][t] = a[t][at], y[i][t] = B_KMAJOR ? b[t][at] : *(const float *)((const uint8_t *)b[t] + int64_t(at) * p.ldb_b);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      if (k0 + 8 * lh + i >= p.k)
+#pragma unroll
+        for (int t = 0; t < T; t++) x[i][t] = y[i][t] = 0.0f;
+#pragma unroll
+      for (int r = 0; r < T; r++)
+#pragma unroll
+        for (int c = 0; c < T; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i][r], y[i][c], acc[r][c], 0, 0, 0);
+    }
+  }
+}
+
+// T x T blocks to a wave, four waves to a tile of 64 T x 64 T; G groups of four waves take every G-th step of 16 k.
+template <int T, int G>
+struct Staged {
+  static constexpr int BM = 64 * T, PART = BM * 32, OPERAND = 3 * PART, STAGE = 2 * OPERAND;
+  static constexpr int GROUP = G > 1 && BM * BM * 4 > 2 * STAGE ? BM * BM * 4 : 2 * STAGE;   // a group's two stages, or its sums
+};
+// A thread cuts eight k of a row of A or a column of B at a time and writes the parts to LDS as the MFMA takes them.  Step j's MFMAs,
+// the cutting of step j + 1's values and the loads of step j + 3 run between two barriers, dealt out by the scheduler hints.
+template <int T, int G, bool B_KMAJOR>
+__global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_PARAMS, GemmArgs g) {
+  typedef Staged<T, G> S;
+  constexpr int BM = S::BM, K = 16;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), group = wave >> 2, wm = wave >> 1 & 1, wn = wave & 1;
+  const int tid = threadIdx.x & 255;
+  MRL_WALK_TILE(tile_m, tile_n)
+  const int64_t m0 = int64_t(tile_m) * BM, n0 = int64_t(tile_n) * BM;
+  const Problem p(g);
+  const int steps = (p.k + K - 1) / K, mine = (steps + G - 1) / G, head = p.k - K * (steps - 1);   // (every group passes as many barriers)
+  uint8_t *const stages = lds + group * S::GROUP;
+  // Where a row's eight k of a half of the lanes lie: the halves change places every four rows, and again every eight, so that neither
+  // eight nor sixteen lanes that write both halves of their rows, or read one half of theirs, meet in a bank.
+  auto place = [](int row, int half) { return row * 32 + ((half ^ (row >> 2) ^ (row >> 3)) & 1) * 16; };
+
+  // What this thread cuts: of A and of B where T is 2, of A or (waves 2 and 3) of B where it is 1.
+  constexpr int OPERANDS = T == 2 ? 2 : 1;
+  const uint8_t *from[OPERANDS];
+  uint32_t off[OPERANDS];
+  int half[OPERANDS], at[OPERANDS], which[OPERANDS];
+  int next = min(group, steps - 1);   // the step that `from` is at
+  const bool second = T == 1 && __builtin_amdgcn_readfirstlane(tid >> 7);
+  auto across = [&](int o) { return !B_KMAJOR && (T == 2 ? o == 1 : second); };
+#pragma unroll
+  for (int o = 0; o < OPERANDS; o++) {
+    const bool is_b = T == 2 ? o == 1 : second;
+    const int t = T == 2 ? tid : tid & 127, k0 = next == 0 ? 0 : head + K * (next - 1);
+    const int row = across(o) ? t % BM : t >> 1;
+    half[o] = across(o) ? __builtin_amdgcn_readfirstlane(t / BM) : t & 1;
+    if (across(o)) {
+      from[o] = p.b + n0 * 4 + int64_t(k0 + 8 * half[o]) * p.ldb_b;
+      off[o] = uint32_t(min(row, int(p.n - n0) - 1)) * 4;
+    } else {
+      from[o] = (is_b ? p.b + n0 * p.ldb_b : p.a + m0 * p.lda_b) + int64_t(k0) * 4;
+      off[o] = uint32_t(min(row, int((is_b ? p.n - n0 : p.m - m0) - 1))) * (is_b ? p.ldb_b : p.lda_b) + 32 * half[o];
+    }
+    at[o] = (is_b ? S::OPERAND : 0) + place(row, half[o]);
+    which[o] = (is_b ? BM : 0) + row;
+  }
+  float most[OPERANDS];
+#pragma unroll
+  for (int o = 0; o < OPERANDS; o++) most[o] = 0.0f;
+
+  struct Values { float x[OPERANDS][8]; };
+  Values kept[2];
+  auto load = [&](Values &to) {   // this group's next step (past its last: that again)
+    const int ahead = next + G >= steps ? 0 : next == 0 ? head + K * (G - 1) : K * G;
+#pragma unroll
+    for (int o = 0; o < OPERANDS; o++) {
+      if (across(o)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) to.x[o][i] = *(const float *)(from[o] + i * int64_t(p.ldb_b) + off[o]);
+        from[o] += ahead * int64_t(p.ldb_b);
+      } else {
+        const four_on_word lo = *(const four_on_word *)(from[o] + off[o]), hi = *(const four_on_word *)(from[o] + off[o] + 16);
+#pragma unroll
+        for (int i = 0; i < 4; i++) to.x[o][i] = lo[i], to.x[o][4 + i] = hi[i];
+        from[o] += ahead * 4;
+      }
+    }
+    next += ahead ? G : 0;
+  };
+  auto put = [&](const Values &v, uint8_t *stage) {
+#pragma unroll
+    for (int o = 0; o < OPERANDS; o++) {
+      const Parts c = cut(v.x[o], most[o]);
+      uint8_t *to = stage + at[o];
+      *(v4i *)to = c.h, *(v4i *)(to + S::PART) = c.m, *(v4i *)(to + 2 * S::PART) = c.l;
+    }
+  };
+
+  v16f big[T][T], small[T][T];
+#pragma unroll
+  for (int r = 0; r < T; r++)
+#pragma unroll
+    for (int c = 0; c < T; c++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) big[r][c][i] = small[r][c][i] = 0.0f;
+  struct Operands { v4i a[3][T], b[3][T]; };
+  const int a_rd = wm * 1024 * T + place(li, lh), b_rd = S::OPERAND + wn * 1024 * T + place(li, lh);
+  auto read = [&](const uint8_t *stage, Operands &f) {
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int t = 0; t < T; t++) {
+        f.a[i][t] = *(const v4i *)(stage + a_rd + i * S::PART + t * 1024);
+        f.b[i][t] = *(const v4i *)(stage + b_rd + i * S::PART + t * 1024);
+      }
+  };
+  auto multiply = [&](const Operands &f) {
+    auto all = [&](int x, int y, v16f (&acc)[T][T]) {   // (one block after the other: no MFMA waits for the one before it)
+#pragma unroll
+      for (int r = 0; r < T; r++)
+#pragma unroll
+        for (int c = 0; c < T; c++) acc[r][c] = mfma(f.a[x][r], f.b[y][c], acc[r][c]);
+    };
+    all(0, 1, small), all(0, 0, big), all(1, 0, small), all(1, 1, small), all(0, 2, small), all(2, 0, small);
+  };
+  // All LDS reads and writes are done; loads stay under way.
+  auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
+  // Step j, whose parts lie in `stage`, while step j + 1's are cut.
+  auto step = [&](Values &v, const uint8_t *stage, uint8_t *next_stage) {
+    Operands f;
+    read(stage, f);
+    put(v, next_stage);
+    load(v);
+    multiply(f);
+    __builtin_amdgcn_sched_group_barrier(0x100, 6 * T, 0);   // the reads, then an MFMA and some of the cutting in turn
+#pragma unroll
+    for (int i = 0; i < 6 * T * T; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, T == 2 ? 5 : 10, 0);
+    }
+    barrier();
+  };
+  {
+    Values v;
+    load(v);
+    load(kept[1]);
+    load(kept[0]);
+    if (group == 0)
+#pragma unroll
+      for (int o = 0; o < OPERANDS; o++)
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          if (8 * half[o] + i >= head) v.x[o][i] = 0.0f;
+    put(v, stages);
+  }
+  barrier();
+  int j = 0;
+  for (; j + 2 < mine; j += 2) {
+    step(kept[1], stages, stages + S::STAGE);
+    step(kept[0], stages + S::STAGE, stages);
+  }
+  if (j + 1 < mine) step(kept[1], stages, stages + S::STAGE);
+  if ((mine - 1) * G + group < steps) {   // (behind K's end: nothing)
+    Operands f;
+    read(stages + ((mine - 1) & 1) * S::STAGE, f);
+    multiply(f);
+  }
+#pragma unroll
+  for (int r = 0; r < T; r++)
+#pragma unroll
+    for (int c = 0; c < T; c++) big[r][c] += small[r][c];
+
+  const int64_t row0 = m0 + wm * 32 * T, col0 = n0 + wn * 32 * T;
+  float sum[T * T * 16 / G];
+  meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
+  if (!parts_did(most, which, 2 * BM, probe_of(sum), (uint32_t *)lds)) {
+    multiply_f32<T, G, B_KMAJOR>(p, row0, col0, group, big);
+    meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
+  }
+  store<T, G>(p, row0, col0, group, g.accum, g.ldc, sum);
+}
+
+// A block of 32 x 32 on four waves that take every fourth step of 32 k, operands straight from memory into registers: no barrier and no
+// trip through LDS on the way.
+constexpr int DEAL = 4;
+template <bool B_KMAJOR>
+__global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS, GemmArgs g) {
+  constexpr int K = 32, D = 2;
+  __shared__ __attribute__((aligned(16))) float part[DEAL * 1024];
+  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  MRL_WALK_TILE(tile_m, tile_n)
+  const int64_t m0 = int64_t(tile_m) * 32, n0 = int64_t(tile_n) * 32;
+  const Problem p(g);
+  const int steps = (p.k + K - 1) / K, head = p.k - K * (steps - 1);
+  int next = min(wave, steps - 1);   // the step that the operands are at
+  const int k0 = next == 0 ? 0 : head + K * (next - 1);
+  const uint8_t *a = p.a + m0 * p.lda_b + int64_t(k0) * 4;
+  const uint8_t *b = B_KMAJOR ? p.b + n0 * p.ldb_b + int64_t(k0) * 4 : p.b + n0 * 4 + int64_t(k0) * p.ldb_b;
+  // Lane (l % 32, l / 32): 16 k, from 16 (l / 32) on, of row and column l % 32; eight of them to an MFMA.
+  const uint32_t a_off = uint32_t(min(li, int(p.m - m0) - 1)) * p.lda_b + lh * 64, col = uint32_t(min(li, int(p.n - n0) - 1));
+  const uint32_t b_off = B_KMAJOR ? col * p.ldb_b + lh * 64 : col * 4 + uint32_t(lh) * 16 * p.ldb_b;
+  struct Values { float a[16], b[16]; };
+  Values kept[D];
+  auto load = [&](Values &v) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const four_on_word x = *(const four_on_word *)(a + a_off + q * 16);
+#pragma unroll
+      for (int i = 0; i < 4; i++) v.a[q * 4 + i] = x[i];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if constexpr (B_KMAJOR) {
+        const four_on_word x = *(const four_on_word *)(b + b_off + q * 16);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v.b[q * 4 + i] = x[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) v.b[q * 4 + i] = *(const float *)(b + (q * 4 + i) * int64_t(p.ldb_b) + b_off);
+      }
+    }
+    const int ahead = next + DEAL >= steps ? 0 : next == 0 ? head + K * (DEAL - 1) : K * DEAL;   // (past the last: that again)
+    a += int64_t(ahead) * 4, b += B_KMAJOR ? int64_t(ahead) * 4 : int64_t(ahead) * p.ldb_b;
+    next += ahead ? DEAL : 0;
+  };
+  float most[2] = {0.0f, 0.0f};
+  v16f big[1][1], small;
+#pragma unroll
+  for (int i = 0; i < 16; i++) big[0][0][i] = small[i] = 0.0f;
+  auto multiply = [&](const Parts &x, const Parts &y) {
+    small = mfma(x.h, y.m, small);
+    big[0][0] = mfma(x.h, y.h, big[0][0]);
+    small = mfma(x.m, y.h, small);
+    small = mfma(x.m, y.m, small);
+    small = mfma(x.h, y.l, small);
+    small = mfma(x.l, y.h, small);
+  };
+  const int mine = steps > wave ? (steps - wave + DEAL - 1) / DEAL : 0;
+  if (mine > 0) {
+    ring::each<D>([&](auto d) { load(kept[decltype(d)::value]); });
+    if (wave == 0)
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        if (16 * lh + i >= head) kept[0].a[i] = kept[0].b[i] = 0.0f;
+    for (int left = mine; left > 0;) {
+      bool done = false;
+      ring::each<D>([&](auto d) {
+        Values &v = kept[decltype(d)::value];
+        if (!done) {
+          const Parts a0 = cut(v.a, most[0]), b0 = cut(v.b, most[1]);
+          multiply(a0, b0);
+          const Parts a1 = cut(v.a + 8, most[0]), b1 = cut(v.b + 8, most[1]);
+          load(v);
+          multiply(a1, b1);
+          done = --left == 0;
+        }
+      });
+    }
+  }
+  big[0][0] += small;
+  const int which[2] = {li, 32 + li};
+  float sum[16 / DEAL];
+  meet<1, DEAL>(part, 1024, 0, wave, big, sum);
+  // (a wave without a step has nothing to say)
+  const float known[2] = {mine ? most[0] : __builtin_inff(), mine ? most[1] : __builtin_inff()};
+  if (!parts_did(known, which, 64, probe_of(sum), (uint32_t *)part)) {
+    multiply_f32<1, DEAL, B_KMAJOR>(p, m0, n0, wave, big);
+    meet<1, DEAL>(part, 1024, 0, wave, big, sum);
+  }
+  store<1, DEAL>(p, m0, n0, wave, g.accum, g.ldc, sum);
+}
+
+void declare_work(const GemmArgs &g, int side, int k_step, double serial_ns) {
+  const double mn = double(g.m) * g.n * g.batch;
+  // (1.2 to 1.3 times the rate that the model takes for the f32 MFMA)
+  plan::work(plan::UNIT_MFMA_F32, 2.0 * mn * g.k, (double(g.m) * g.k + double(g.k) * g.n) * g.batch * 4 + mn * 4 * (g.accum ? 2 : 1),
+             2.0 * side * side * double((g.k + k_step - 1) / k_step * k_step), serial_ns, 1.4);
+}
+
+template <int T, int G, bool B_KMAJOR>
+hipError_t launch_staged(const GemmArgs &g, hipStream_t stream) {
+  typedef Staged<T, G> S;
+  constexpr int BM = S::BM, LDS = G * S::GROUP;
+  static std::atomic<uint64_t> lds_limit_set{0};
+  if (!plan::recording() && LDS > 65536) {
+    hipError_t e = raise_lds_limit(lds_limit_set, (const void *)k_gemm_f32<T, G, B_KMAJOR>, LDS);
+    if (e != hipSuccess) return e;
+  }
+  const int tiles_m = int((g.m + BM - 1) / BM), tiles_n = int((g.n + BM - 1) / BM);
+  declare_work(g, BM, 16, 2000.0 + (T == 2 ? 700.0 : 400.0) * ((g.k + 15) / 16) / G);
+  const TileWalk walk = gemm::tile_walk(tiles_m, tiles_n);
+  MRL_LAUNCH((k_gemm_f32<T, G, B_KMAJOR>), dim3(tiles_m * tiles_n, g.batch), dim3(256 * G), LDS, stream, MRL_WALK_ARGS(walk), g);
+  return plan::last_error();
+}
+
+template <bool B_KMAJOR>
+hipError_t launch_waves(const GemmArgs &g, hipStream_t stream) {
+  const int tiles_m = int((g.m + 31) / 32), tiles_n = int((g.n + 31) / 32);
+  declare_work(g, 32, 32, 2000.0 + 700.0 * ((g.k + 31) / 32) / DEAL);
+  const TileWalk walk = gemm::tile_walk(tiles_m, tiles_n);
+  MRL_LAUNCH((k_gemm_f32_waves<B_KMAJOR>), dim3(tiles_m * tiles_n, g.batch), dim3(64 * DEAL), 0, stream, MRL_WALK_ARGS(walk), g);
+  return plan::last_error();
+}
+
+template <int T, int G>
+hipError_t launch_either(const GemmArgs &g, hipStream_t stream) {
+  return g.b_kmajor ? launch_staged<T, G, true>(g, stream) : launch_staged<T, G, false>(g, stream);
+}
+
+}  // namespace
+
+// Workgroups of a form go to the compute units in rounds, each as long as a workgroup's steps.  Measured, on operands of 1 to 50 MB: a step of 4 x 32 k of a block of 32 x 32 0.75 us of its unit, however many share it; of 2 x 16 k of 64 x 64
+// 0.5; of 2 x 16 k of 128 x 128 1.05 to, on all units, 1.47; of 16 k of two such workgroups 1.35, of one 0.85.  Slices of K cost the launch that sums them, 2.5 us, and
+// their results at 3 TB/s.  (us, the f32 MFMA on copies of whole chunks / this, form and slices: 195 x 500 x 621 17.0 / 6.9, waves;
+// 192 x 2176 x 128 16.1 / 9.2, waves in 8; twice 382 x 226 x 1179 14.1 / 8.7, 64 wide; 537 x 1668 x 568 25.0 / 17.0, 64 wide in 3; 2048^3 162
+// / 98.9, 128 wide in two groups; 2070 x 389 x 3128 68.2 / 47.9, 128 wide in one; 4096^3 943 / 695.)
+namespace {
+enum Form : uint32_t { NONE, WAVES, WIDE_64, WIDE_128, WIDE_128_PAIR };
+struct Choice {
+  Form form;
+  uint32_t slices, slice_k;
+};
+Choice choose(const GemmArgs &g) {
+  const double units = g_compute_units;
+  auto tiles = [&](uint32_t side) { return double((g.m + side - 1) / side) * ((g.n + side - 1) / side) * g.batch; };
+  const double t32 = tiles(32), t64 = tiles(64), t128 = tiles(128);
+  auto rounds = [&](double n, double at_once) { return double(uint64_t((n + at_once - 1) / at_once)); };
+  Choice best{NONE, 1, g.k};
+  double least = 1e300;
+  auto consider = [&](Form form, uint32_t slices, uint32_t slice_k, double us) {
+    if (us < least) least = us, best = {form, slices, slice_k};
+  };
+  const uint32_t steps = (g.k + 15) / 16;
+  consider(WIDE_128, 1, g.k, 5.0 + std::max(1.05, 0.75 + 0.72 * std::min(1.0, t128 / units)) * rounds(t128, units) * ((steps + 1) / 2));
+  consider(WIDE_128_PAIR, 1, g.k, 5.0 + (t128 <= units ? 0.85 : 1.35 * rounds(t128, 2 * units)) * steps);
+  for (uint32_t want : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u}) {
+    uint32_t slice_k = want == 1 ? g.k : (g.k + want * 32 - 1) / (want * 32) * 32;
+    if (want > 1 && (g.batch != 1 || g.tight || slice_k < 128)) break;
+    if (g.k % slice_k != 0 && g.k % slice_k < 32) slice_k += 32;   // (no slice shorter than a step)
+    const uint32_t slices = (g.k + slice_k - 1) / slice_k;
+    const double sum = slices == 1 ? 0.0 : 2.5 + (slices + 1.0) * g.m * g.n * 4.0 / 3e6;
+    const uint32_t s16 = (slice_k + 15) / 16, s32 = (slice_k + 31) / 32;
+    if (g.k >= 32) consider(WAVES, slices, slice_k, 4.0 + 0.75 * rounds(t32 * slices, units) * ((s32 + DEAL - 1) / DEAL) + sum);
+    consider(WIDE_64, slices, slice_k, 3.8 + 0.5 * rounds(t64 * slices, units) * ((s16 + 1) / 2) + sum);
+  }
+  return best;
+}
+}  // namespace
+
+// Any rows of f32, from a step of K on.  Whole chunks over a short K, whose start and end are most of the time, stay with k_gemm
+// (1472 x 128 x 1472 10.5 us, here 12.1; 832 x 192 x 1088 7.2 and 7.1).
+bool gemm_f32_applicable(const GemmArgs &g, int kind) {
+  auto words = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 4 == 0; };
+  if (kind != 3 || g.k < 16 || !gemm::edge_addressable(g, 4) || g.batch > 65535 || !words(g.a) || !words(g.b) || !words(g.c)) return false;
+  const bool chunks = g.lda % 4 == 0 && g.ldb % 4 == 0 && g.sa % 4 == 0 && g.sb % 4 == 0 &&
+                      reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && reinterpret_cast<uintptr_t>(g.b) % 16 == 0;
+  return !(chunks && g.k <= 192) && gemm_pays(g, kind) && !gemv_applicable(g, kind);
+}
+
+uint32_t gemm_f32_slices(const GemmArgs &g, uint32_t *slice_k) {
+  const Choice c = choose(g);
+  *slice_k = c.slice_k;
+  return c.slices;
+}
+
+hipError_t launch_gemm_f32(const GemmArgs &g, hipStream_t stream) {
+  GemmArgs whole = g;
+  if (g.k_total != 0) whole.batch = 1, whole.k = g.k_total;   // the form goes by the whole problem
+  switch (choose(whole).form) {
+    case WAVES: return g.b_kmajor ? launch_waves<true>(g, stream) : launch_waves<false>(g, stream);
+    case WIDE_64: return launch_either<1, 2>(g, stream);
+    case WIDE_128: return launch_either<2, 2>(g, stream);
+    case WIDE_128_PAIR: return launch_either<2, 1>(g, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace mrl

@@ -141,7 +141,7 @@ struct GemmArgs {
   // (`ldb` = elements between n rows), as col_major / layout![0,2,1] store it.
   bool b_kmajor = false;
   // K shared out over batch entries: each has `k` elements, the last what is left of k_total (0: `k` each).  The
-  // Conv build of k_gemm and gemm_ring_rows.hip take it.
+  // Conv build of k_gemm, gemm_ring_rows.hip and gemm_f32.hip take it.
   uint32_t k_total = 0;
   // Scratch is short: rows are read in place wherever that is possible (gemm_ring_rows.hip).
   bool tight = false;
@@ -202,6 +202,11 @@ hipError_t launch_gemm_ring_rows(const GemmArgs &g, int kind, hipStream_t stream
 // gemm_wide_edge.hip: the four-wave tile on ragged shapes and against a k-fastest B.
 hipError_t launch_gemm_wide_edge(const GemmArgs &g, int kind, hipStream_t stream);
 hipError_t launch_gemm_big(const GemmArgs &g, int kind, hipStream_t stream, uint32_t staging = 0);
+
+// ---- gemm_f32.hip: f32 operands as three bf16 each, rows that start anywhere ----
+bool gemm_f32_applicable(const GemmArgs &g, int kind);
+uint32_t gemm_f32_slices(const GemmArgs &g, uint32_t *slice_k);   // of K, each of *slice_k but the last: k_total then says how long all are
+hipError_t launch_gemm_f32(const GemmArgs &g, hipStream_t stream);
 
 // ---- gemv.hip: at most four rows of A against a k-fastest B, as dot products (a stream over B) ----
 bool gemv_applicable(const GemmArgs &g, int kind);

@@ -1,0 +1,79 @@
+"""f32 Matmuls through the bf16 matrix cores (gemm_f32.hip), against float64."""
+import numpy as np
+import pytest
+
+import morello_amd as M
+from morello_amd import synth
+from gpu_util import run_spec
+
+pytestmark = pytest.mark.gpu
+KT = M.layout(0, 2, 1)
+F32 = (M.f32,) * 3
+FORMS = {"waves": "k_gemm_f32_waves", "64": "k_gemm_f32 [T = 1, G = 2", "128": "k_gemm_f32 [T = 2, G = 2", "pair": "k_gemm_f32 [T = 2, G = 1"}
+
+
+def _spec(b, m, k, n, nk, accum=False):
+    return M.Matmul([b, m, k, n], F32, [None, KT if nk else None, None], accum)
+
+
+def _run(spec, A, B, C, nk):
+    return run_spec(spec, [A, np.ascontiguousarray(B.transpose(0, 2, 1)) if nk else B, C.copy()])
+
+
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("b,m,k,n,accum,form,slices", [
+    (1, 511, 513, 261, False, "waves", 1),    # a step and one k, rows and columns short of a block and one past it
+    (1, 331, 385, 501, True, "waves", 1),
+    (2, 300, 543, 301, True, "waves", 1),     # 31 k in the first step; two entries
+    (1, 33, 4001, 97, False, "waves", 16),    # slices of K, the last one shorter
+    (1, 129, 1410, 65, True, "waves", 6),     # ... the old values added in the sum
+    (1, 2477, 129, 257, False, "64", 1),      # nine steps on two groups, one k in the first
+    (1, 641, 223, 1601, True, "64", 1),
+    (3, 130, 175, 1029, True, "64", 1),
+    (1, 537, 1667, 569, True, "64", 3),
+    (2, 555, 1907, 2969, False, "128", 1),
+    (1, 1740, 1751, 1637, True, "128", 1),
+    (1, 2071, 389, 3129, True, "pair", 1),
+    (1, 1697, 322, 4417, False, "pair", 1),
+    (1, 2048, 1024, 2048, False, "128", 1),   # whole tiles, rows of whole chunks
+])
+def test_f32_matmul_in_parts(gpu, b, m, k, n, accum, form, slices, nk):
+    """Within the error of a product's parts (2^-23) and of one rounding for every term; and in the norm below 4e-7, where sums
+    of two terms at a time come to 3e-7 at K = 500 and 8e-7 at 2048."""
+    spec = _spec(b, m, k, n, nk, accum)
+    plan = spec.plan()
+    assert plan.steps[0].kernel.startswith(FORMS[form]) and plan.kernels[1:] == ["k_sum_splits"] * (slices > 1), plan
+    assert plan.steps[0].grid[1] == b * slices
+    A, B, C = synth.normal_f32(191, 0, (b, m, k)), synth.normal_f32(191, 1, (b, k, n)), synth.normal_f32(191, 2, (b, m, n))
+    got = _run(spec, A, B, C, nk).astype(np.float64)
+    a64, b64 = A.astype(np.float64), B.astype(np.float64)
+    want = a64 @ b64 + (C if accum else 0)
+    assert (np.abs(got - want) <= (k + 4) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64) + 8)).all()
+    assert np.linalg.norm(got - want) <= 4e-7 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("m,k,n", [(511, 513, 261), (2477, 129, 257), (1740, 751, 1637), (2071, 389, 3129), (537, 1667, 569)])
+def test_f32_values_that_are_no_three_bf16(gpu, m, k, n, nk):
+    """Infinities, the largest finite values, rows and columns of tiny values beside ordinary ones, of zeros, and NaN: as f32
+    arithmetic has them, in the tiles that hold them and in the others."""
+    A, B = np.abs(synth.normal_f32(192, 0, (1, m, k))), np.abs(synth.normal_f32(192, 1, (1, k, n))) + np.float32(0.01)
+    A[0, 3, 7], A[0, 70, k - 1] = np.inf, -np.inf
+    A[0, 5] = 0
+    A[0, 9] = 0
+    A[0, 9, 11] = -3.40282347e38            # the lowest value beside zeros
+    B[0, 11] = np.float32(0.5)
+    A[0, 100] *= np.float32(1e-36)          # tiny, every one of them: the l and m would be lost
+    B[0, :, 20] *= np.float32(1e-35)
+    A[0, 130, 2] = np.nan
+    want = A[0].astype(np.float64) @ B[0].astype(np.float64)
+    spec = _spec(1, m, k, n, nk)
+    assert spec.plan().kernels[0].startswith("k_gemm_f32")
+    got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk)[0]
+    with np.errstate(over="ignore"):
+        want32 = want.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want32)) and np.array_equal(np.isinf(got), np.isinf(want32))
+    assert np.array_equal(got[np.isinf(got)], want32[np.isinf(want32)])
+    normal = np.isfinite(want) & (np.abs(want) >= 2.0 ** -120)   # (below: the products themselves are denormal)
+    assert (np.abs(got[normal] - want[normal]) <= 2e-6 * np.abs(want[normal])).all()
+    assert normal[100].sum() >= n - 1 and (got[5] == 0).all()
