@@ -827,7 +827,7 @@ int run_conv(const mrl_spec &s, void *const *params, Workspace &ws) {
       slices.batch = splits, slices.k = slice_k, slices.k_total = conv_args.k;
       slices.sb = int64_t(slices.k), slices.conv.slice_bytes = uint32_t(slices.k * img.elem);
       slices.c = partial, slices.ldc = conv_args.n, slices.sc = int64_t(conv_args.m) * conv_args.n, slices.accum = 0;
-      HIP_TRY(mrl::launch_conv_gemm(slices, kind, ws.stream, 64));
+      HIP_TRY(mrl::launch_conv_gemm(slices, kind, ws.stream));
       HIP_TRY(mrl::launch_sum_splits(partial, conv_args.c, splits, conv_args.m, conv_args.n, conv_args.ldc,
                                      s.accum != 0, kind <= 1, false, ws.stream));
     } else {

@@ -1,0 +1,194 @@
+// The tile of gemm_ring_rows.hip: rows that start anywhere, or (CONV) the windows of a channels-last image.
+#pragma once
+#include "gemm_ring.h"
+
+namespace mrl {
+namespace ring {
+typedef int chunk_anywhere __attribute__((ext_vector_type(4), aligned(1)));
+
+// The first `left` of v's bytes (none below 1, all from 16 on), zeros behind them.
+__device__ inline v4i first_bytes(v4i v, int left) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int n = left - 4 * i;
+    v[i] &= n >= 4 ? -1 : n <= 0 ? 0 : int((1u << (8 * n)) - 1);
+  }
+  return v;
+}
+
+// CONV (with B_KMAJOR): row p of A is the window of output pixel p, fh runs of fw * c contiguous elements of the image, whole 16-byte chunks each.
+template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RA, int RB, bool CONV = false>
+__device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_t tile_n, const GemmArgs &g) {
+  static_assert(!CONV || B_KMAJOR, "");
+  typedef typename Ring<T>::Acc Acc;
+  constexpr int ES = T::ES, BK = STEP / ES, BM = 32 * RA, BN = 32 * RB, WM = 16 * RA, WN = 16 * RB;
+  constexpr int A_BYTES = BM * STEP, B_BYTES = BN * STEP, SLOT = A_BYTES + B_BYTES;
+  constexpr int A_LOADS = A_BYTES / (1024 * WAVES), B_LOADS = (B_BYTES / 1024 + WAVES - 1) / WAVES, LOADS = A_LOADS + B_LOADS;   // a wave's, per step
+  constexpr int DEPTH = 2;   // (four to eight, on the smallest tile: 4 to 13 % slower, more to wait for at the start and nothing gained behind it)
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kw = wave >> 2, wm = wave >> 1 & 1, wn = wave & 1;
+  const int64_t m0 = int64_t(tile_m) * BM, n_tile = int64_t(tile_n) * BN;
+  const int64_t n0 = B_KMAJOR ? n_tile : min(n_tile, int64_t(g.n) - BN);
+  const uint8_t *A = (const uint8_t *)g.a + (CONV ? 0 : (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES);
+  const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : n0)) * ES;
+  const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = uint32_t(g.ldb) * ES;
+  const int a_last = min(BM, int(g.m - m0)) - 1, b_last = min(BN, int(g.n - n0)) - 1;
+  const int k = g.k_total != 0 ? int(min(g.k, g.k_total - blockIdx.y * g.k)) : int(g.k), steps = (k + BK - 1) / BK, head = k - (steps - 1) * BK;   // head: elements of K in the first step
+
+  // Where this lane's chunks of a step come from, as in gemm_ring.hip: lane l of a load has the l-th 16 bytes of a KiB of LDS.
+  auto b_load = [&](int i) { return i * WAVES + wave - (i * WAVES + wave < B_BYTES / 1024 ? 0 : WAVES / 2); };
+  constexpr int CHUNKS = STEP / 16, ROWS_PER_LOAD = 64 / CHUNKS, ROWS_PER_LINE = 256 / STEP;
+  const int row16 = lane / CHUNKS, chunk = (lane % CHUNKS) ^ (row16 / ROWS_PER_LINE % CHUNKS);
+  auto chunk_of = [&](int load) { return chunk ^ (load * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS); };
+  uint32_t off[LOADS];
+  int dst[LOADS], whole[LOADS];   // whole: of the chunk's 16 bytes, those the first step has
+#pragma unroll
+  for (int i = 0; i < A_LOADS; i++) {
+    const int load = wave * A_LOADS + i;
+    const int row = min(load * ROWS_PER_LOAD + row16, a_last);
+    if constexpr (CONV) {
+      const uint32_t p = uint32_t(m0) + row, line = g.conv.by_ow.div(p), img = g.conv.by_oh.div(line);
+      off[i] = ((img * g.conv.h + (line - img * g.conv.oh)) * g.conv.w + (p - line * g.conv.ow)) * g.conv.c_bytes;
+    } else {
+      off[i] = uint32_t(row) * lda_b + chunk_of(load) * 16;
+    }
+    dst[i] = load * 1024 + lane * 16;
+    whole[i] = head * ES - chunk_of(load) * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < B_LOADS; i++) {
+    const int load = b_load(i);
+    dst[A_LOADS + i] = A_BYTES + load * 1024 + lane * 16;
+    if constexpr (B_KMAJOR) {
+      off[A_LOADS + i] = uint32_t(min(load * ROWS_PER_LOAD + row16, b_last)) * ldb_b + chunk_of(load) * 16;
+      whole[A_LOADS + i] = head * ES - chunk_of(load) * 16;
+    } else {
+      constexpr int PITCH = BN * ES;
+      const int at = load * 1024 + lane * 16, r = at / PITCH;
+      off[A_LOADS + i] = uint32_t(r) * ldb_b + swizzle<T, BN>(at % PITCH, r);
+      whole[A_LOADS + i] = r < head ? 16 : 0;
+    }
+  }
+  const uint8_t *a_tile = A, *b_tile = B;
+  const int64_t b_step = B_KMAJOR ? int64_t(STEP) : int64_t(BK) * ldb_b;
+  // CONV: where the chunks of the step to load lie in a window, from its corner on; the step's first byte of the window.
+  uint32_t in_window[A_LOADS];
+  uint32_t window_byte = CONV ? blockIdx.y * g.conv.slice_bytes : 0;
+  auto find_chunks = [&]() {
+    if constexpr (CONV)
+#pragma unroll
+      for (int i = 0; i < A_LOADS; i++) {
+        const uint32_t kb = window_byte + chunk_of(wave * A_LOADS + i) * 16;
+        in_window[i] = kb + g.conv.by_run.div(kb) * g.conv.run_gap;
+      }
+  };
+  find_chunks();
+  auto load = [&](auto which) {
+    constexpr int I = decltype(which)::value;
+    if constexpr (CONV && I < A_LOADS) return __builtin_bit_cast(v4i, *(const chunk_anywhere *)(A + (off[I] + in_window[I])));
+    else return __builtin_bit_cast(v4i, *(const chunk_anywhere *)((I < A_LOADS ? a_tile : b_tile) + off[I]));
+  };
+  int loaded = 0;   // the step that the pointers are at
+  auto advance = [&]() {   // to the next one (past the last: nowhere)
+    const bool more = loaded + 1 < steps;
+    a_tile += !more ? 0 : loaded == 0 ? head * ES : STEP;
+    window_byte += !more ? 0 : loaded == 0 ? head * ES : STEP;
+    find_chunks();
+    b_tile += !more ? 0 : loaded == 0 ? (B_KMAJOR ? int64_t(head) * ES : int64_t(head) * ldb_b) : b_step;
+    loaded++;
+  };
+
+  // Operand addresses within a slot: lane (l % 16, l / 16) takes the l / 16-th 16 bytes of row l % 16.
+  const int in_rows = li * STEP + (((4 * kw + lg) ^ (li / ROWS_PER_LINE % CHUNKS)) << 4);
+  int b_rd[RB];
+  if constexpr (!B_KMAJOR) {
+    constexpr int LANES_PER_ROW = 2 * ES;   // of a group of sixteen: 8 bytes each of a row's sixteen columns
+    const int r = (64 / ES) * kw + (16 / ES) * lg + li / LANES_PER_ROW;
+#pragma unroll
+    for (int c = 0; c < RB; c++) b_rd[c] = A_BYTES + r * (BN * ES) + swizzle<T, BN>((wn * WN + c * 16) * ES + 8 * (li % LANES_PER_ROW), r);
+  }
+  v4i af[2][RA], bf[2][RB], kept[DEPTH][LOADS];
+  // The i-th operand read of 64 bytes of K (RA of A, then RB of B), out of the slot of the same parity.
+  auto read = [&](auto set, auto which) {
+    constexpr int S = decltype(set)::value, I = decltype(which)::value;
+    const uint8_t *slot = lds + S * SLOT;
+    if constexpr (I < RA) af[S][I] = *(const v4i *)(slot + wm * WM * STEP + in_rows + I * 16 * STEP);
+    else if constexpr (B_KMAJOR) bf[S][I - RA] = *(const v4i *)(slot + A_BYTES + wn * WN * STEP + in_rows + (I - RA) * 16 * STEP);
+    else {
+      const uint8_t *at = slot + b_rd[I - RA];
+      const v2i lo = T::read_tr(at), hi = T::read_tr(at + T::K_PER_READ * (BN * ES));
+      bf[S][I - RA] = v4i{lo[0], lo[1], hi[0], hi[1]};
+    }
+  };
+  Acc acc[RA][RB];
+  int colsum[RB];
+#pragma unroll
+  for (int c = 0; c < RB; c++) {
+    colsum[c] = 0;
+#pragma unroll
+    for (int r = 0; r < RA; r++) acc[r][c] = Acc{0, 0, 0, 0};
+  }
+  auto multiply = [&](auto set, auto which) {   // the which-th block
+    constexpr int S = decltype(set)::value, I = decltype(which)::value, R = I / RB, C = I % RB;
+    if constexpr (A_UNSIGNED && C == 0) af[S][R] ^= v4i{int(0x80808080), int(0x80808080), int(0x80808080), int(0x80808080)};
+    acc[R][C] = Ring<T>::mfma(af[S][R], bf[S][C], acc[R][C]);
+    if constexpr (A_UNSIGNED && R == 0)   // a - 128 was multiplied: 128 times the column sums of B come on top
+#pragma unroll
+      for (int w = 0; w < 4; w++) colsum[C] = __builtin_amdgcn_sdot4(bf[S][C][w], 0x01010101, colsum[C], false);
+  };
+  // All LDS reads and writes are done; loads stay under way.
+  auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
+  // A step of parity P whose successor but one waits in set K.
+  auto step = [&](auto parity, auto held) {
+    constexpr int P = decltype(parity)::value, K = decltype(held)::value;
+    barrier();
+    each<RA * RB>([&](auto q) {
+      constexpr int Q = decltype(q)::value, N = RA * RB, READS = RA + RB;
+      multiply(parity, q);
+      constexpr int R0 = min_of(READS, (Q * READS * 4 + N * 3 - 1) / (N * 3)), R1 = min_of(READS, ((Q + 1) * READS * 4 + N * 3 - 1) / (N * 3));   // in the first three quarters
+      each<R1 - R0>([&](auto i) { read(std::integral_constant<int, 1 - P>{}, std::integral_constant<int, R0 + decltype(i)::value>{}); });
+      constexpr int L0 = Q * LOADS / N, L1 = (Q + 1) * LOADS / N;
+      each<L1 - L0>([&](auto i) {
+        constexpr int I = L0 + decltype(i)::value;
+        *(v4i *)(lds + P * SLOT + dst[I]) = kept[K][I];
+        kept[K][I] = load(std::integral_constant<int, I>{});
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    advance();
+  };
+  {
+    v4i first[2][LOADS];
+    each<2>([&](auto s) {
+      each<LOADS>([&](auto i) { first[decltype(s)::value][decltype(i)::value] = load(i); });
+      advance();
+    });
+    each<DEPTH>([&](auto s) {
+      each<LOADS>([&](auto i) { kept[decltype(s)::value][decltype(i)::value] = load(i); });
+      advance();
+    });
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) {
+      *(v4i *)(lds + dst[i]) = first_bytes(first[0][i], whole[i]);
+      *(v4i *)(lds + SLOT + dst[i]) = first[1][i];
+    }
+  }
+  barrier();
+  each<RA + RB>([&](auto i) { read(std::integral_constant<int, 0>{}, i); });
+  // (what a step reads and writes for those behind the last one is not multiplied)
+  for (int left = steps;;) {
+    bool done = false;
+    each<DEPTH>([&](auto s) {
+      if (!done) {
+        step(std::integral_constant<int, decltype(s)::value % 2>{}, s);
+        done = --left == 0;
+      }
+    });
+    if (done) break;
+  }
+  barrier();
+  store_tile<T, A_UNSIGNED, RA, RB>(g, lds, acc, colsum, m0, n0, int(n_tile - n0));
+}
+
+}  // namespace ring
+}  // namespace mrl

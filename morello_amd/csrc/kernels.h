@@ -159,6 +159,9 @@ struct GemmArgs {
     uint32_t slice_bytes;
     // Filled in by launch_conv_gemm: the divisions of the window arithmetic.
     FastDiv by_ow, by_oh, by_c_bytes, by_fw;
+    // Bytes of the image between the end of a window's row and the start of its next one, and the division by the bytes of such a row.
+    uint32_t run_gap;
+    FastDiv by_run;
   } conv = {};
 };
 // kind: 0 = i8 x i8, 1 = u8 x i8, 2 = bf16 x bf16, 3 = f32 x f32; B stored k-fastest (gemm_nt.hip).
@@ -166,7 +169,7 @@ struct GemmArgs {
 hipError_t launch_gemm_nt(const GemmArgs &g, int kind, uint32_t tile, hipStream_t stream);
 // Conv as an implicit Matmul (g.conv filled in, B = the KRSC filters, k-fastest); tile chosen by size.
 bool conv_gemm_applicable(const GemmArgs &g, int kind);
-// `tile`: side of the workgroup tile (64, 128, 256), or 0 for the choice by problem size.
+// `tile`: side of k_gemm's square workgroup tile (64, 128, 256), or 0 for the choice by problem size, its tiles of gemm_ring_rows.h among them.
 hipError_t launch_conv_gemm(const GemmArgs &g, int kind, hipStream_t stream, uint32_t tile = 0);
 // kind: 0 = i8 x i8 -> i32, 1 = u8 x i8 -> i32, 2 = bf16 x bf16 -> f32, 3 = f32 x f32 -> f32.
 // Shapes, leading dimensions and alignment the kernel can walk.
