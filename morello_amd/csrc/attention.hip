@@ -521,6 +521,9 @@ __global__ __launch_bounds__(512) void k_attn(const void *q, const void *kt, con
   // Merge the two key halves: (m, d, O) of half 1 goes through LDS to the wave of half 0
   // that owns the same queries.  Layout [value][lane] keeps lanes on distinct banks.
   const float l_tot[2] = {den[0][0], den[1][0]};
+  // The fetches past the last block land in tiles that nobody reads, but must not land on what is exchanged here: beside copies across
+  // PCIe they took longer than the last matrix slot.
+  __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();  // all K/V reads are done: the staging area is free
   // [quad of values][lane], 16 bytes per lane: lanes on distinct banks, one instruction per quad.
   constexpr int MQ = DD::MERGE_ROWS / 4;   // a lane's quads: O^T's blocks, then (m, m, l, l)
