@@ -498,11 +498,11 @@ __global__ __launch_bounds__(256) void k_move_tiled32(MoveStrided p) {
 // 32 bytes: an element per thread in destination order 133 us, this 42).  UNROLL vectors a
 // thread, their loads in flight together.
 constexpr int MOVE_RUNS_ACT = 4;   // digits a tile extends along at most
-template <int SE, int DE, int V, int UNROLL>
+template <int SE, int DE, int V, int UNROLL, bool DIAGONAL = false>
 __global__ __launch_bounds__(256) void k_move_runs(MoveTile p) {
   int64_t base_s, base_d;
   uint32_t room[MOVE_MAX_RANK];
-  tile_origin(p, base_s, base_d, room);
+  tile_origin<DIAGONAL>(p, base_s, base_d, room);
   uint32_t raw[UNROLL][V], to[UNROLL];
   bool inside[UNROLL];
 #pragma unroll
@@ -1118,7 +1118,7 @@ void fill_tile(MoveTile *t, const MoveStrided &p, const uint32_t *ext, const uin
 
 // k_move_runs' tile over a view whose shared digit counts vectors of `vec` elements: how many vectors it
 // holds, and how many tiles there are.  0 where it would have more workgroups than a launch takes.
-uint32_t runs_tile(const MoveStrided &p, uint32_t shared, uint32_t vec, uint32_t se, MoveTile *t, uint64_t *blocks) {
+uint32_t runs_tile(const MoveStrided &p, uint32_t shared, uint32_t vec, uint32_t se, uint32_t de, MoveTile *t, uint64_t *blocks) {
   const uint32_t rank = p.rank;
   // Four vectors a thread once every compute unit gets two such workgroups.
   const uint32_t tile_cap = p.count >= 1024ull * 2 * g_compute_units ? 1024 : 256;
@@ -1166,6 +1166,15 @@ uint32_t runs_tile(const MoveStrided &p, uint32_t shared, uint32_t vec, uint32_t
   fill_tile(t, p, ext, nullptr, nullptr, first, &n_act, blocks);
   t->tile = tile;
   for (uint32_t e = 0; e < 4; e++) t->lds_step[e] = 0;
+  // In the destination's order, the second digit first: where that is 64 tiles and more of rows whole pages apart in the source, those under way read a narrow strip of
+  // every row, a few memory channels.  Along the source's rows, each one tile further on, both sides spread (us, before / after: f32 2048 x 16384 into
+  // bf16 strips of 16 41.9 / 39.8, 8192 x 8192 81.8 / 75.7, f32 to f32 120.2 / 100.1, bf16 4096 x 4096 15.2 / 12.5, 8192 x 128 x 32 turned to 128 x 8192 23.6 / 18.3).  Not for fewer
+  // tiles (f32 strips of 16 back into 8192 x 8192, 16 of them, 95.0 / 103.4), other rows (strips back into 1000 x 80000 116.0 / 121.8), where the caches hold the
+  // tensors (2000 x 3008 9.2 / 9.6), for runs of 16 bytes (bf16 4096 x 4096 strips of 8 15.3 / 15.9), or onto wider elements, where the writes are the larger part
+  // (bf16 2048 x 16384 into f32 strips of 16 31.5 / 34.6).
+  const int64_t apart = n_first > 1 ? p.ss[first[1]] * int64_t(vec * se) : 0;
+  t->diagonal = se >= de && vec * se >= 16 && ext[shared] * vec * se >= 32 && t->chunks[1] >= 64 && apart >= 8192 && apart % 4096 == 0 &&
+                p.count * vec * (se + de) >= 64000000;
   return *blocks < (1u << 24) ? tile : 0;
 }
 
@@ -1180,7 +1189,7 @@ hipError_t launch_move_runs(MoveStrided p, uint32_t shared, uint32_t vec, bool t
   MoveTile t;
   uint64_t blocks = 0;
   // (a tile that leaves threads of its workgroup without a vector: four short digits, the rest of the tensor elsewhere)
-  const uint32_t tile = tiled ? runs_tile(p, shared, vec, se, &t, &blocks) : 0;
+  const uint32_t tile = tiled ? runs_tile(p, shared, vec, se, de, &t, &blocks) : 0;
   if (tile < 192) {
     blocks = (p.count + 255) / 256;
     for (uint32_t o = 0; o < p.rank; o++) p.by_shape[o] = FastDiv(p.shape[p.order[o]]);
@@ -1189,7 +1198,9 @@ hipError_t launch_move_runs(MoveStrided p, uint32_t shared, uint32_t vec, bool t
 #define MRL_RUNS_V(SE, DE, V)                                                                                       \
   if (vec == V) {                                                                                                  \
     if (tile < 192) MRL_LAUNCH((k_move_runs<SE, DE, V>), grid, dim3(256), 0, stream, p);                            \
-    else if (tile > 256) MRL_LAUNCH((k_move_runs<SE, DE, V, 4>), grid, dim3(256), 0, stream, t);                    \
+    else if (tile > 256 && t.diagonal) {                                                                            \
+      if constexpr (SE >= DE && V * SE >= 16) MRL_LAUNCH((k_move_runs<SE, DE, V, 4, true>), grid, dim3(256), 0, stream, t); \
+    } else if (tile > 256) MRL_LAUNCH((k_move_runs<SE, DE, V, 4>), grid, dim3(256), 0, stream, t);                  \
     else MRL_LAUNCH((k_move_runs<SE, DE, V, 1>), grid, dim3(256), 0, stream, t);                                    \
   }
 #define MRL_RUNS(SE, DE)                                                                                            \

@@ -24,6 +24,7 @@ struct MoveTile {
   uint32_t inv_s[MOVE_MAX_RANK], inv_d[MOVE_MAX_RANK], inv_ext[MOVE_MAX_RANK];  // ceil(2^32 / x)
   uint32_t tile;  // elements (k_move_runs: vectors) per tile
   FastDiv by_chunks[MOVE_MAX_RANK];   // a block number into tile coordinates without dividing (blocks number below 2^31)
+  bool diagonal;         // k_move_runs: which of tile_origin's orders
   uint32_t lds_step[4];  // k_move_gather: where the elements of a destination run of four lie in source order, from its first
 };
 constexpr uint32_t MOVE_TILE_MAX = 4096;
@@ -140,13 +141,21 @@ __device__ inline uint32_t div_small(uint32_t n, uint32_t d, uint32_t inv) {
 
 // Coordinates of this workgroup's tile: the offsets of its origin on the two sides, and how much of
 // each digit is left from there on.
+// DIAGONAL: the tiles are numbered along the third digit before the second, each row of them one further on.
+template <bool DIAGONAL = false>
 __device__ inline void tile_origin(const MoveTile &p, int64_t &base_s, int64_t &base_d, uint32_t (&room)[MOVE_MAX_RANK]) {
   uint32_t blk = blockIdx.x;
   base_s = base_d = 0;
 #pragma unroll
-  for (uint32_t d = 0; d < MOVE_MAX_RANK; d++) {
+  for (uint32_t o = 0; o < MOVE_MAX_RANK; o++) {
+    const uint32_t d = DIAGONAL && (o == 1 || o == 2) ? 3 - o : o;
     const uint32_t rest = p.by_chunks[d].div(blk);
-    const uint32_t origin = (blk - rest * p.chunks[d]) * p.ext[d];
+    uint32_t at = blk - rest * p.chunks[d];
+    if (DIAGONAL && d == 2) {   // (the second digit's place is the next remainder)
+      at += rest - p.by_chunks[1].div(rest) * p.chunks[1];
+      at -= p.by_chunks[2].div(at) * p.chunks[2];
+    }
+    const uint32_t origin = at * p.ext[d];
     blk = rest;
     room[d] = p.shape[d] - origin;
     base_s += int64_t(origin) * p.ss[d], base_d += int64_t(origin) * p.ds[d];

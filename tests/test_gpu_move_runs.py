@@ -146,3 +146,12 @@ def test_narrowing_rows_8_kib_apart(gpu, sdt, ddt, rows, cols, strips, shift):
         _check(sdt, ddt, [5, rows // 5, cols], None, (2, 1, 0, (2, "p", 8)), "k_move_runs", shift)
     else:
         _check(sdt, ddt, [1, rows, cols], None, (0, 2, 1, (2, "p", strips)), "k_move_runs", shift)
+
+
+@pytest.mark.parametrize("sdt,ddt", [(M.f32, M.bf16), (M.f32, M.f32), (M.bf16, M.bf16)])
+@pytest.mark.parametrize("rows,cols", [(2051, 16 * 512), (4100, 16 * 256)])
+def test_packing_strips_along_diagonals(gpu, sdt, ddt, rows, cols):
+    """From 64 MB on, both sides together, with rows whole pages apart, tiles are numbered along the source's rows, each row one tile further on: whole and ragged
+    rows, more rows of tiles than columns and fewer."""
+    _check(sdt, ddt, [1, rows, cols], None, STRIPS, "k_move_runs")
+    _check(sdt, ddt, [rows, 128, cols // 128], None, (1, 0, 2), "k_move_runs")
