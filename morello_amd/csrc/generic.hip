@@ -904,12 +904,15 @@ __global__ __launch_bounds__(256) void k_softmax_cols_short(SMC q) {
 // R: not 0 where the scan dim is at most WAVES * R: PHASE 0 then keeps the columns in registers, R values a lane, and
 // reads each element once.  Bound by memory; over dim 1, us before -> now: 25 x 370 x 961 30.4 -> 23.5, 20 x 200 x 2000 20.7 -> 14.1,
 // 64 x 60 x 1000 10.1 -> 7.2, 6 x 120 x 135 13.1 -> 5.7.
-template <int WAVES, int PHASE, int R = 0>
+// RUNS: an XCD takes neighbouring tiles, which share the lines that rows of odd lengths cross, in its L2 (us, dealt over the XCDs / in runs: 16 x 1793 x 673 68.4 /
+// 51.3, 20 x 1500 x 700 65.4 / 52.8, 32 x 513 x 1000 40.6 / 33.0).  Rows of whole lines that are read twice are dealt over the XCDs (24 x 1160 x 2752 167 / 170, 6 x
+// 3000 x 4000 160 / 165).
+template <int WAVES, int PHASE, int R = 0, bool RUNS = (R > 0)>
 __global__ __launch_bounds__(64 * WAVES) void k_softmax_cols(SMC q) {
   const SM &p = q.s;
   __shared__ float sm_max[WAVES][64], sm_den[WAVES][64];
   const uint32_t lane = threadIdx.x % 64, w = threadIdx.x / 64;
-  uint64_t r = R > 0 ? xcd_run(blockIdx.x, gridDim.x) : blockIdx.x;   // (neighbouring tiles share the lines that rows of odd lengths cross)
+  uint64_t r = RUNS ? xcd_run(blockIdx.x, gridDim.x) : blockIdx.x;
   const uint32_t f = uint32_t(r % q.fast_tiles) * 64 + lane;
   r /= q.fast_tiles;
   int64_t ibase = 0, obase = 0;
@@ -1660,6 +1663,7 @@ hipError_t launch_softmax_generic(const Strided &in, const Strided &out, uint32_
       const uint64_t blocks = lines / in.shape[d] * q.fast_tiles;
       if (blocks > 0x7fffffffull) break;
       const uint32_t chunks = scratch ? softmax_cols_chunks(blocks, in.shape[scan_dim]) : 1;
+      const bool runs = in.stride[scan_dim] % 32 != 0 || out.stride[scan_dim] % 32 != 0;
       if (chunks > 1) {
         // Few columns: the scan dim shared out over blockIdx.y as well, in two launches.
         q.chunks = chunks, q.chunk_len = (in.shape[scan_dim] + chunks - 1) / chunks, q.pairs = (float2 *)scratch;
@@ -1668,9 +1672,11 @@ hipError_t launch_softmax_generic(const Strided &in, const Strided &out, uint32_
         // its piece (32 steps a pass) is what small problems take: 2149 x 172 11 us, 100000 x 64 45 us.
         const double chain_ns = 2500.0 + 700.0 * ((q.chunk_len + 31) / 32);
         plan::work(plan::UNIT_STREAM, 0, 5.2 * count, 0, chain_ns);
-        MRL_LAUNCH((k_softmax_cols<4, 1>), dim3(uint32_t(blocks), chunks), dim3(256), 0, stream, q);
+        if (runs) MRL_LAUNCH((k_softmax_cols<4, 1, 0, true>), dim3(uint32_t(blocks), chunks), dim3(256), 0, stream, q);
+        else MRL_LAUNCH((k_softmax_cols<4, 1>), dim3(uint32_t(blocks), chunks), dim3(256), 0, stream, q);
         plan::work(plan::UNIT_STREAM, 0, 10.4 * count, 0, chain_ns);
-        MRL_LAUNCH((k_softmax_cols<4, 2>), dim3(uint32_t(blocks), chunks), dim3(256), 0, stream, q);
+        if (runs) MRL_LAUNCH((k_softmax_cols<4, 2, 0, true>), dim3(uint32_t(blocks), chunks), dim3(256), 0, stream, q);
+        else MRL_LAUNCH((k_softmax_cols<4, 2>), dim3(uint32_t(blocks), chunks), dim3(256), 0, stream, q);
         return mrl::plan::last_error();
       }
       // Columns in registers while two workgroups of sixteen waves share a compute unit with them (32 values a lane); with 64 values
@@ -1681,6 +1687,7 @@ hipError_t launch_softmax_generic(const Strided &in, const Strided &out, uint32_
       else if (scan <= 128) MRL_LAUNCH((k_softmax_cols<4, 0, 32>), grid, dim3(256), 0, stream, q);
       else if (scan <= 256) MRL_LAUNCH((k_softmax_cols<8, 0, 32>), grid, dim3(512), 0, stream, q);
       else if (scan <= 512) MRL_LAUNCH((k_softmax_cols<16, 0, 32>), grid, dim3(1024), 0, stream, q);
+      else if (runs) MRL_LAUNCH((k_softmax_cols<16, 0, 0, true>), grid, dim3(1024), 0, stream, q);
       else MRL_LAUNCH((k_softmax_cols<16, 0>), grid, dim3(1024), 0, stream, q);
       return mrl::plan::last_error();
     }
