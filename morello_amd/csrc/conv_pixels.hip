@@ -35,6 +35,7 @@ enum { IMG_I8 = 0, IMG_U8 = 1, IMG_BF16 = 2 };
 
 constexpr int WAVES = 8, ITEM_W = 16, ITEM_H = 2;
 constexpr int HELD = 4;   // patch pixels a lane holds in flight
+constexpr int STRIP_CHUNKS = 6;   // of 64 pixels that a strip's patch may be
 constexpr int FB = 2;     // blocks of 16 filters multiplied at a time
 
 struct PixelsArgs {
@@ -51,6 +52,7 @@ struct PixelsArgs {
   int whole_lines;              // 32 filters of a pixel are a cache line of the output
   uint32_t patch_bytes;         // of LDS, rows that only a tail step's masked lanes read included
   FastDiv by_image, by_row, by_slots, by_patch_w;   // items of an image, of an image's row of them
+  uint32_t strip, per_image, image_bytes;           // strips: output rows of one, strips and bytes of an image
 };
 
 // Pixels of four elements in LDS out of pixels of three or four in memory.
@@ -96,7 +98,9 @@ struct Pixels {
   }
   // This workgroup's filters, `nf` from f0 on, into rows of `filter_row` bytes at `filt` (`group` of them, zeros where no pixel
   // is): their bytes are one contiguous piece of memory, fetched in whole chunks with the loads in flight together into
-  // the LDS behind, then spread out pixel by pixel.
+  // the LDS behind, then spread out pixel by pixel.  ONE_BATCH: no more than the loop's first round
+  // (32 filters are 12 KiB), whose loads are otherwise made to wait for a patch in flight.
+  template <bool ONE_BATCH = false>
   __device__ static void stage_filters(const PixelsArgs &p, uint32_t group, uint32_t f0, uint32_t nf, uint32_t filter_row, uint8_t *filt) {
     const int tid = threadIdx.x;
     const uint32_t filter_bytes = p.fh * p.fw * p.pixel_bytes;
@@ -112,6 +116,7 @@ struct Pixels {
 #pragma unroll
       for (uint32_t j = 0; j < BATCH; j++)
         if (c0 + j * 64 * WAVES + tid < chunks) raw[c0 + j * 64 * WAVES + tid] = got[j];
+      if (ONE_BATCH) break;
     }
     __syncthreads();
     const uint32_t *words = reinterpret_cast<const uint32_t *>(raw);
@@ -414,6 +419,179 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
   }
 }
 
+// The same over strips of `strip` output rows: a strip's patch is in LDS at once, where every two rows of the form above fetch theirs with all the rows that
+// the windows hang over, and how many rows it has is chosen so that the waves end together (strip_rows).  Two chunks of the next strip's patch are on
+// their way under every two rows, into a second patch.  Its start is 0.4 us longer.
+template <int KS, int RPS, bool TAIL, int KIND, bool PIXELS, bool STRIPS>
+__global__ __launch_bounds__(64 * WAVES, 4) void k_conv_windows(PixelsArgs p) {
+  typedef Pixels<KIND> P;
+  typedef typename P::Acc Acc;
+  typedef typename P::Raw Raw;
+  constexpr bool HALVES = P::HALVES;
+  constexpr int PB = P::PB, PER_CHUNK = P::PER_CHUNK, STEPS = KS + TAIL, CHUNKS = 4 / RPS, GROUP = 16 * FB;
+  constexpr uint32_t filter_row = STEPS * 64 + 16, patch_w = ITEM_W - 1 + PER_CHUNK * CHUNKS, row_bytes = patch_w * PB;
+  constexpr int ROWS = RPS * (STEPS - 1) + ITEM_H;      // patch rows that the operands of two output rows start in
+  extern __shared__ __attribute__((aligned(16))) uint8_t pix_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint8_t *patch = pix_lds + wave * p.patch_bytes, *other = patch + WAVES * p.patch_bytes;   // (the filters are staged where the other patches will be)
+  const uint32_t f0 = blockIdx.y * GROUP, nf = min(uint32_t(GROUP), p.f - f0);
+
+  const uint32_t patch_pixels = patch_w * p.patch_h;
+  struct Corner { uint32_t img, y0, x0; };
+  const uint32_t tiles_x = (p.ow + ITEM_W - 1) / ITEM_W, per_image = p.per_image;
+  auto corner_of = [&](uint32_t item) {
+    const uint32_t img = p.by_image.div(item), in_img = item - img * per_image, ty = p.by_row.div(in_img);
+    return Corner{img, ty * p.strip, (in_img - ty * tiles_x) * ITEM_W};
+  };
+  // The c-th 64 pixels of a patch (past the image's edge: as above; an image is below 2 GiB, so that a lane's offset is 32 bits).
+  auto fetch = [&](const Corner &at, int c, Raw &px) {
+    const uint8_t *const image = p.image + uint64_t(at.img) * p.image_bytes;
+    const uint32_t odd = uint32_t(reinterpret_cast<uintptr_t>(image)) & 3;
+    const uint32_t i = lane + c * 64, r = i / patch_w;
+    if (i >= patch_pixels) return;
+    const uint32_t off = (min(at.y0 + r, p.h - 1) * p.w + min(at.x0 + (i - r * patch_w), p.w - 1)) * p.pixel_bytes + odd;
+    px.shift = off & 3;
+    const uint32_t *from = reinterpret_cast<const uint32_t *>(image - odd + (off & ~3u));
+#pragma unroll
+    for (int e = 0; e < P::ES; e++) px.v[e] = from[e];
+    px.v[P::ES] = from[px.shift + p.pixel_bytes > 4 * P::ES ? P::ES : P::ES - 1];
+  };
+  auto put = [&](uint8_t *to, int c, const Raw &px) {
+    const uint32_t i = lane + c * 64;
+    if (i < patch_pixels) P::put_image(to + i * PB, px, p.pixel_bytes);
+  };
+  const uint32_t stride = gridDim.x * WAVES;
+  uint32_t item = blockIdx.x * WAVES + wave;
+  Raw first[STRIP_CHUNKS];   // in flight while the filters are staged
+  {
+    const Corner at = corner_of(min(item, p.items - 1));
+#pragma unroll
+    for (int c = 0; c < STRIP_CHUNKS; c++) fetch(at, c, first[c]);
+  }
+  P::template stage_filters<true>(p, GROUP, f0, nf, filter_row, pix_lds + WAVES * p.patch_bytes);
+  v4i a[STEPS][FB];
+#pragma unroll
+  for (int ks = 0; ks < STEPS; ks++)
+#pragma unroll
+    for (int fb = 0; fb < FB; fb++) a[ks][fb] = *(const v4i *)(pix_lds + WAVES * p.patch_bytes + (fb * 16 + li) * filter_row + lg * 16 + ks * 64);
+  Acc start[FB];   // u8 pixels are multiplied as a - 128: 128 times a filter's sum comes on top
+#pragma unroll
+  for (int fb = 0; fb < FB; fb++) {
+    start[fb] = Acc{};
+    if constexpr (KIND == IMG_U8) {
+      const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ks++) start[fb] = P::mfma(a[ks][fb], ones, start[fb]);
+      start[fb] *= 128;
+    }
+  }
+  __syncthreads();   // every wave holds its operands: the other patches may lie there
+#pragma unroll
+  for (int c = 0; c < STRIP_CHUNKS; c++)
+    if (c * 64 < int(patch_pixels)) put(patch, c, first[c]);
+  const uint32_t chunk = lg & (CHUNKS - 1), row_of = uint32_t(lg) / CHUNKS;
+  const uint32_t in_patch = row_of * row_bytes + li * PB + chunk * 16;
+  const uint32_t keep_lo = chunk * PER_CHUNK < p.fw ? 0xffffffffu : 0u, keep_hi = chunk * PER_CHUNK + 1 < p.fw ? 0xffffffffu : 0u;
+  const bool inside = KS * RPS + row_of < p.fh;   // of the tail step
+  for (; item < p.items; item += stride) {
+    const Corner at = corner_of(item);
+    const bool more = item + stride < p.items;
+    const Corner next = corner_of(more ? item + stride : item);
+    // The wave's LDS accesses complete in order: what is left is that the compiler keeps them so.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t end = min(p.oh, at.y0 + p.strip);
+    const uint8_t *operands = patch + in_patch;
+    int chunks = more ? 0 : STRIP_CHUNKS;   // of the next patch that are in LDS
+#pragma unroll 1
+    for (uint32_t y0 = at.y0; y0 < end; y0 += ITEM_H, operands += ITEM_H * row_bytes) {
+      // Two chunks of the next patch are on their way under every two rows.
+      Raw px[2];
+      const int c0 = chunks;
+      if (c0 < STRIP_CHUNKS) fetch(next, c0, px[0]), fetch(next, c0 + 1, px[1]);
+      Acc acc[ITEM_H][FB];
+#pragma unroll
+      for (int pb = 0; pb < ITEM_H; pb++)
+#pragma unroll
+        for (int fb = 0; fb < FB; fb++) acc[pb][fb] = start[fb];
+#pragma unroll
+      for (int r = 0; r < ROWS; r++) {
+        v4i bop;
+        if constexpr (HALVES) {
+          const v2u lo = *(const v2u *)(operands + r * row_bytes) & keep_lo, hi = *(const v2u *)(operands + r * row_bytes + 8) & keep_hi;
+          bop = v4i{int(lo[0]), int(lo[1]), int(hi[0]), int(hi[1])};
+        } else {
+          const uint32_t *w = (const uint32_t *)(operands + r * row_bytes);
+          bop = v4i{int(w[0]), int(w[1]), int(w[2]), int(w[3])};
+        }
+#pragma unroll
+        for (int ks = 0; ks < STEPS; ks++) {
+          const int pb = r - RPS * ks;
+          if (pb < 0 || pb >= ITEM_H) continue;
+          const v4i b = HALVES && TAIL && ks == KS && !inside ? v4i{0, 0, 0, 0} : bop;
+#pragma unroll
+          for (int fb = 0; fb < FB; fb++) acc[pb][fb] = P::mfma(a[ks][fb], b, acc[pb][fb]);
+        }
+      }
+      auto at_pixel = [&](int pb, uint32_t x) { return (Acc *)(p.out + ((uint64_t(at.img) * p.oh + y0 + pb) * p.ow + x) * p.f + f0 + 4 * lg); };
+      if (p.whole_lines) {
+        // A pixel's 32 filters are a cache line: lanes of pixels 0 .. 7 and 8 .. 15 exchange a block, so that a store is eight whole
+        // lines and not sixteen halves, and they go past the caches (32 x 3 -> 96 x 224^2 bf16 7 x 7: 156 us in halves, 148 in
+        // lines, 131 in lines past the caches; halves past the caches 197).
+        const bool low = li < 8;
+        const uint32_t x = at.x0 + (li & 7);
+#pragma unroll
+        for (int pb = 0; pb < ITEM_H; pb++) {
+          const Acc mine = low ? acc[pb][0] : acc[pb][1];
+          Acc theirs = low ? acc[pb][1] : acc[pb][0];
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const typename P::Element own = theirs[i];
+            const int bits = __builtin_bit_cast(int, own), other = __builtin_amdgcn_update_dpp(bits, bits, 0x128, 0xf, 0xf, false);   // row_ror:8
+            theirs[i] = __builtin_bit_cast(typename P::Element, other);
+          }
+          if (y0 + pb >= end) continue;
+          Acc *d = at_pixel(pb, x) + (low ? 0 : 4), *e = at_pixel(pb, x + 8) + (low ? 0 : 4);
+          Acc v = low ? mine : theirs, w = low ? theirs : mine;
+          if (x < p.ow) {
+            if (p.accum) v += *d;
+            MRL_STORE_ONCE(v, d);
+          }
+          if (x + 8 < p.ow) {
+            if (p.accum) w += *e;
+            MRL_STORE_ONCE(w, e);
+          }
+        }
+      } else {
+        const uint32_t x = at.x0 + li;
+#pragma unroll
+        for (int pb = 0; pb < ITEM_H; pb++)
+          if (y0 + pb < end && x < p.ow) {
+            Acc *d = at_pixel(pb, x);
+#pragma unroll
+            for (int fb = 0; fb < FB; fb++)
+              if (fb * 16 < int(nf)) {
+                Acc v = acc[pb][fb];
+                if (p.accum) v += d[4 * fb];
+                d[4 * fb] = v;
+              }
+          }
+      }
+      if (c0 < STRIP_CHUNKS) put(other, c0, px[0]), put(other, c0 + 1, px[1]), chunks = c0 + 2;
+    }
+    for (; chunks * 64 < int(patch_pixels) && chunks < STRIP_CHUNKS; chunks++) {
+      Raw px;
+      fetch(next, chunks, px);
+      put(other, chunks, px);
+    }
+    uint8_t *const t = patch;
+    patch = other, other = t;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 template <int KS, int KIND, bool PIXELS = true>
 hipError_t launch(const PixelsArgs &p, dim3 grid, size_t lds, hipStream_t stream) {
   static std::atomic<uint64_t> limit{0};
@@ -434,8 +612,14 @@ hipError_t launch_ks(const PixelsArgs &p, int kind, dim3 grid, size_t lds, hipSt
 }
 
 // The form with the filters' operands in registers: `rows` filter rows, `rps` of them to a step.
+template <int KS, int RPS, bool TAIL, int KIND, bool PIXELS = true, bool STRIPS = true>
+hipError_t launch_strips(const PixelsArgs &p, dim3 grid, size_t lds, hipStream_t stream) {
+  MRL_LAUNCH((k_conv_windows<KS, RPS, TAIL, KIND, PIXELS, STRIPS>), grid, dim3(64 * WAVES), lds, stream, p);
+  return plan::last_error();
+}
 template <int KS, int RPS, bool TAIL, int KIND, bool PIXELS = true>
 hipError_t launch_held(const PixelsArgs &p, dim3 grid, size_t lds, hipStream_t stream) {
+  if (p.strip) return launch_strips<KS, RPS, TAIL, KIND>(p, grid, lds, stream);
   MRL_LAUNCH((k_conv_windows<KS, RPS, TAIL, KIND, PIXELS>), grid, dim3(64 * WAVES), lds, stream, p);
   return plan::last_error();
 }
@@ -458,6 +642,27 @@ constexpr uint32_t MAX_KS = 7;
 uint32_t chunks_log2_of(const ConvArgs &c, int kind) {   // chunks of 16 bytes of a window's row, as 1, 2 or 4
   const uint32_t pixels = kind == IMG_BF16 ? 2 : 4, chunks = (c.fw + pixels - 1) / pixels;
   return chunks <= 1 ? 0 : chunks <= 2 ? 1 : chunks <= 4 ? 2 : 3;
+}
+
+// Output rows of a strip, 0: pairs of rows are faster.  A wave's first item waits for its patch and, longer, for the filters; a unit's second
+// workgroup adds to that, by their size; and what a round leaves over is a round.  In us, over those that no choice changes: 0.45 a row (an odd one's pair half), more
+// beside a second workgroup, 0.4 a round, and the strips' longer start and code 1.  (us, pairs / strips of so many rows: 16 x 3 -> 64 x 109^2 bf16 7 x 7, 6160 pairs on
+// 2048 waves, 15.4 / 13.7 (7), 9 x 4 -> 64 x 115^2 12.4 / 10.1, 11 x 3 -> 32 x 82^2 7.0 / 6.5 (3), u8 17 x 3 -> 16 x 151^2 3 x 3 8.1 / 7.3; 14 x 3 -> 64 x 60^2 bf16
+// 3 x 3 5.7, strips of four 6.0.)  From five rounds of pairs on these are the better ones (u8 27 x 3 -> 64 x 146^2 5 x 5 31.4, strips of ten 33.1).
+uint32_t strip_rows(const ConvArgs &c, uint32_t patch_w, uint32_t steps, uint32_t groups) {
+  const uint64_t units = g_compute_units, waves = std::max<uint64_t>(1, 2 * units / groups) * WAVES, across = (c.ow + ITEM_W - 1) / ITEM_W;
+  auto strips = [&](uint32_t rows) { return c.b * across * ((c.oh + rows - 1) / rows); };
+  if (strips(ITEM_H) > 4 * waves) return 0;
+  auto us = [&](uint32_t rows) {
+    const uint64_t n = strips(rows), rounds = (n + waves - 1) / waves;
+    const double strip = 0.45 * (rows + (rows & 1) * 0.5);
+    return (n + WAVES - 1) / WAVES * groups <= units ? strip : 0.6 + 0.16 * steps + (rounds > 1 ? 0.4 * double(rounds) : 0) + 1.35 * double(rounds) * strip;
+  };
+  uint32_t best = 0;
+  double least = us(ITEM_H) - 1.0;
+  for (uint32_t rows = 3; rows <= 12 && patch_w * (rows + c.fh - 1) <= STRIP_CHUNKS * 64; rows++)
+    if (us(rows) < least) best = rows, least = us(rows);
+  return best;
 }
 
 }  // namespace
@@ -483,7 +688,7 @@ hipError_t launch_conv_pixels(const ConvArgs &c, int kind, hipStream_t stream) {
   const uint32_t rows_per_step = 4u >> p.chunks_log2, whole = c.fh / rows_per_step;
   p.steps = (c.fh + rows_per_step - 1) / rows_per_step;
   p.slots = p.steps * 64 / pb;
-  p.patch_w = ITEM_W - 1 + ((16 / pb) << p.chunks_log2), p.patch_h = ITEM_H + c.fh - 1;
+  p.patch_w = ITEM_W - 1 + ((16 / pb) << p.chunks_log2), p.patch_h = ITEM_H + c.fh - 1, p.strip = p.per_image = p.image_bytes = 0;
   p.patch_bytes = ((ITEM_H + p.steps * rows_per_step - 1) * p.patch_w * pb + 15) & ~15u;
   const uint32_t tiles_x = (c.ow + ITEM_W - 1) / ITEM_W, per_image = tiles_x * ((c.oh + ITEM_H - 1) / ITEM_H);
   p.items = c.b * per_image;
@@ -494,8 +699,15 @@ hipError_t launch_conv_pixels(const ConvArgs &c, int kind, hipStream_t stream) {
   const uint32_t groups = (c.f + 16 * FB - 1) / (16 * FB);
   const bool shared_patch = p.steps <= 2 && groups > 2 && c.f <= 128 && uint64_t(p.items) * groups > 3 * 2 * uint64_t(g_compute_units) * WAVES;
   if (!shared_patch && rows_held(c, kind, p.chunks_log2) && p.patch_w * p.patch_h <= HELD * 64) {
+    p.strip = uint64_t(p.h) * p.w * p.pixel_bytes < (1ull << 31) ? strip_rows(c, p.patch_w, p.steps, groups) : 0;
+    if (p.strip) {
+      const uint32_t strips = tiles_x * ((c.oh + p.strip - 1) / p.strip);
+      p.patch_h = p.strip + c.fh - 1, p.image_bytes = p.h * p.w * p.pixel_bytes;
+      p.items = c.b * strips, p.by_image = FastDiv(strips), p.per_image = strips;
+      p.patch_bytes = (((p.strip + 1) / ITEM_H * ITEM_H + p.steps * rows_per_step - 1) * p.patch_w * pb + 15) & ~15u;
+    }
     const size_t raw = size_t(std::min<uint32_t>(c.f, 16 * FB)) * c.fh * c.fw * p.pixel_bytes + 32;
-    const size_t lds = std::max(16 * FB * (p.steps * 64 + 16) + raw, WAVES * size_t(p.patch_bytes));
+    const size_t patches = WAVES * size_t(p.patch_bytes), lds = (p.strip ? patches : 0) + std::max(16 * FB * (p.steps * 64 + 16) + raw, patches);
     const uint32_t wgs = std::min<uint32_t>((p.items + WAVES - 1) / WAVES, std::max(1u, 2 * g_compute_units / groups));
     plan::work(plan::UNIT_STREAM, 0, 1.5 * (pixels * c.f * 4 * (c.accum ? 2 : 1) + double(c.b) * p.h * p.w * p.pixel_bytes), 0,
                4000.0 + (700.0 + 100.0 * p.steps) * double((p.items + wgs * WAVES - 1) / (wgs * WAVES)));
