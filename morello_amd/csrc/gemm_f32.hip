@@ -9,8 +9,9 @@
 //
 // Where the parts would not do, the tile is computed again by the f32 MFMA: an infinity in A or B leaves a NaN (its m is inf - inf),
 // and so does an overflow on the way; and in a row of A or column of B of nothing but tiny values the l, then the m, are no
-// bf16 any more.  Each thread keeps the largest magnitude of what it cuts up, all of one row or column.  (All tiles twice: 2048^3 with
-// an infinity in every sixteenth row 370 us, 512^3 18.)
+// bf16 any more.  Each thread keeps the largest magnitude of what it cuts up, all of one row or column; one past 2^60 has its tile
+// computed again too, since it could bring the lost parts of a tiny value beside ordinary ones back to the size of a result.  (All
+// tiles twice: 2048^3 with an infinity in every sixteenth row 370 us, 512^3 18.)
 //
 // What bounds it: the bf16 MFMAs at what the board's power lets them run at (4096^3 in 695 us is 1.19 PFLOP/s of them, where the 256 tile
 // reaches 1.42), for the smaller tiles the cutting, six vector instructions a value; below a round of tiles the chain of a step.
@@ -33,6 +34,8 @@ typedef float four_on_word __attribute__((ext_vector_type(4), aligned(4)));
 // A row or column whose largest magnitude reaches it loses nothing that counts beside that value (its lowest bit is 2^-113, a bf16
 // goes down to 2^-126 without denormals).
 constexpr float TINY = 0x1p-90f;
+// What a value loses below 2^-126 stays below 2^-66 of a product as long as the other operand stays below this.
+constexpr float HUGE_VALUE = 0x1p60f;
 
 struct Parts { v4i h, m, l; };
 // Eight values as three chunks of eight bf16; `most`: the largest magnitude so far.
@@ -84,14 +87,18 @@ __device__ inline float probe_of(const float (&sum)[N]) {
 }
 
 // Whether a tile's parts did: no value that is infinite or no number among this thread's sums, and no row of A or column of B, whose
-// N largest magnitudes this thread keeps (`which`: numbers of theirs below `all`), of nothing but tiny values.  Of the workgroup.
+// N largest magnitudes this thread keeps (`which`: numbers of theirs below `all`), with a huge value or of nothing but tiny ones.  Of the
+// workgroup.
 template <int N>
 __device__ inline bool parts_did(const float (&most)[N], const int (&which)[N], int all, float probe, uint32_t *seen) {
-  bool odd = probe != probe;
+  bool never = probe != probe;
+#pragma unroll
+  for (int i = 0; i < N; i++) never = never || most[i] > HUGE_VALUE;
+  bool odd = never;
 #pragma unroll
   for (int i = 0; i < N; i++) odd = odd || !(most[i] >= TINY);
   if (!__syncthreads_or(odd)) return true;
-  if (__syncthreads_or(probe != probe)) return false;
+  if (__syncthreads_or(never)) return false;
   for (int i = threadIdx.x; i < all; i += blockDim.x) seen[i] = 0;
   __syncthreads();
 #pragma unroll
@@ -423,7 +430,7 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
   float sum[16 / DEAL];
   meet<1, DEAL>(part, 1024, 0, wave, big, sum);
   // (a wave without a step has nothing to say)
-  const float known[2] = {mine ? most[0] : __builtin_inff(), mine ? most[1] : __builtin_inff()};
+  const float known[2] = {mine ? most[0] : 1.0f, mine ? most[1] : 1.0f};
   if (!parts_did(known, which, 64, probe_of(sum), (uint32_t *)part)) {
     multiply_f32<1, DEAL, B_KMAJOR>(p, m0, n0, wave, big);
     meet<1, DEAL>(part, 1024, 0, wave, big, sum);

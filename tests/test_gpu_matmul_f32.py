@@ -77,3 +77,23 @@ def test_f32_values_that_are_no_three_bf16(gpu, m, k, n, nk):
     normal = np.isfinite(want) & (np.abs(want) >= 2.0 ** -120)   # (below: the products themselves are denormal)
     assert (np.abs(got[normal] - want[normal]) <= 2e-6 * np.abs(want[normal])).all()
     assert normal[100].sum() >= n - 1 and (got[5] == 0).all()
+
+
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("m,k,n", [(511, 513, 261), (2477, 129, 257), (1740, 751, 1637), (2071, 389, 3129), (537, 1667, 569)])
+def test_f32_tiny_values_that_huge_ones_bring_back(gpu, m, k, n, nk):
+    """A tiny value beside a one that meets a zero, times a huge one: the only product of its result, to one rounding."""
+    A, B = synth.normal_f32(193, 0, (1, m, k)), synth.normal_f32(193, 1, (1, k, n))
+    rows, cols = [50, m - 1], [30, n - 1]
+    for i, r in enumerate(rows):
+        A[0, r] = 0
+        A[0, r, 3], A[0, r, 17] = 1, np.float32(1.2345678e-36) * (i + 1)
+    for i, c in enumerate(cols):
+        B[0, 3, c], B[0, 17, c] = 0, np.float32(1.7654321e35) * (i + 1)
+    spec = _spec(1, m, k, n, nk)
+    assert spec.plan().kernels[0].startswith("k_gemm_f32")
+    got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk)[0].astype(np.float64)
+    want = A[0].astype(np.float64) @ B[0].astype(np.float64)
+    at = np.ix_(rows, cols)
+    assert (np.abs(got[at] - want[at]) <= 2.0 ** -22 * np.abs(want[at])).all(), (got[at], want[at])
+    assert np.linalg.norm(np.delete(got - want, cols, 1)) <= 4e-7 * np.linalg.norm(np.delete(want, cols, 1))
