@@ -59,6 +59,12 @@ hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
     case 32: return launch_either<T, A_UNSIGNED, 2, 2>(g, stream);
     case 64: return launch_either<T, A_UNSIGNED, 4, 2>(g, stream);
     case 128: return launch_either<T, A_UNSIGNED, 4, 4>(g, stream);
+    case 160:
+      if constexpr (T::ES == 2) return launch_either<T, A_UNSIGNED, 4, 5>(g, stream);
+      return hipErrorInvalidValue;
+    case 192:
+      if constexpr (T::ES == 2) return launch_either<T, A_UNSIGNED, 4, 6>(g, stream);
+      return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
   }
 }
@@ -110,7 +116,9 @@ bool slices_are_faster_of_few(const GemmArgs &g, int kind, int es, uint64_t step
 //   64 (128 x 64) where those are: bf16 975 x 2176 x 1666 22.5 / 17.5, u8 1888 x 1633 x 885 17.4 / 14.7; int8 over a long K reads
 //     its rows' lines once too often: 1651 x 5949 x 844 28.8 / 31.8, and bf16 over a longer one: 1835 x 3535 x 655 31.7 / 35.2;
 //   128 (128 x 128), bf16: 1483 x 858 x 1983 18.4 / 15.8, 1303 x 1524 x 2056 24.3 / 20.3; over a long K the copies are
-//     the faster way (1538 x 3021 x 1767 34.2 / 38.6), for int8 at once (1055 x 929 x 1801 13.2 / 15.8).
+//     the faster way (1538 x 3021 x 1767 34.2 / 38.6), for int8 at once (1055 x 929 x 1801 13.2 / 15.8);
+//   160 (128 x 160) where those are and 128 x 128 ones are not, else 192 (128 x 192), bf16: 2306 x 735 x 2260 24.5 / 17.4, 2491 x 1862 x 2026 38.8 /
+//     31.3, k-fastest B twice 771 x 813 x 3032 29.1 / 21.2.
 uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
   if (kind < 0 || kind > 2) return 0;
   const int es = kind == 2 ? 2 : 1;
@@ -145,9 +153,24 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
   // Of 128 x 128 up to two thirds of a round from 16 (twice 789 x 1007 x 1167 20.9 / 25.1, 19.0 / 21.1, 2399 x 1307 x 925 25.3 / 28.5, 23.5 / 22.6;
   // twice 598 x 1019 x 3125, 250 tiles, 27.0 / 26.2, 24.1 / 20.4).
   // Onto bf16 results over up to five steps an element a lane, which odd rows leave, is the slower end (1749 x 173 x 1407 11.9 / 14.7, 11.2 / 12.2).
+  // From a row-major B of rows that start on words the lines are touched once more by A alone: to 46 steps (1332 x 1992 x 1783 36.5 / 33.8, 30.1 / 26.3, twice 429 x 2894 x
+  // 3511, 46 of them, 46.2 / 44.9, 43.9 / 35.2, 1768 x 2696 x 1679 43.0 / 43.1, 34.6 / 32.3; past them 1222 x 3074 x 1065 twice 41.7 / 45.7, 40.0 / 37.3; odd rows of A 2387
+  // x 2641 x 1031 37.0 / 47.2, 34.8 / 35.1, 1366 x 2257 x 2332 33.4 / 37.0, 31.6 / 27.9).
+  // Past a round of 128 x 128 the copies' tiles take two: from a row-major B up to 32 steps (2491 x 1862 x 2026 41.1 / 38.5, 38.8 / 31.3, odd rows
+  // of A 2072 x 1899 x 2689 43.3 / 43.6, 41.8 / 37.7; rows on words gain up to 46, 1084 x 2582 x 2596 twice 51.7 / 46.6, 49.7 / 39.6, 1001 x 2050 x 4425 41.1 / 40.9, 40.5 / 34.1, and stay with
+  // the copies all the same, whose route tests/test_plan_routes.py holds fast for the last; odd ones lose there, 2103 x 2583 x 2065 43.2 / 54.3,
+  // 42.1 / 44.2), a k-fastest B up to 20 (547 x 1118 x 4107 twice 36.8 / 31.7, 33.9 / 27.1; 2138 x 1460 x 2320 30.7 / 33.3, 28.6 / 26.3), with odd rows 16 (2146 x 927 x
+  // 2260 31.1 / 29.9, 28.3 / 23.5; 894 x 1195 x 2688 twice 31.6 / 33.9, 29.5 / 27.0); up to six steps they are even (2057 x 323 x 2231 17.9 / 19.5, 16.2 / 16.8).  Over 79 random
+  // sizes of these classes 1.20 times as fast with three sets, 1.06 from memory (geometric means; least 1.00 and 0.90).  Of one and two entries, as measured.
   const uint64_t large = tiles(128, 128);
+  const bool words = g.lda % 2 == 0 && (!g.b_kmajor || g.ldb % 2 == 0);
+  if (kind == 2 && large > units) {
+    const uint32_t most = g.b_kmajor ? (words ? 20u : 16u) : 32u;
+    if (g.batch > 2 || steps <= 6 || steps > most) return 0;
+    return g.n >= 160 && tiles(128, 160) <= units ? 160 : g.n >= 192 && tiles(128, 192) <= units ? 192 : 0;
+  }
   if (kind != 2 || g.n < 128 || large > units || (g.accum && g.c_bf16 && steps <= 5 && (g.lda % 2 != 0 || g.ldb % 2 != 0))) return 0;
-  return steps <= (odd_rows && 3 * large <= 2 * units ? 15u : 24u) ? 128 : 0;
+  return steps <= (odd_rows && 3 * large <= 2 * units ? 15u : words && !g.b_kmajor && g.batch <= 2 ? 46u : 24u) ? 128 : 0;
 }
 
 hipError_t launch_gemm_ring_rows(const GemmArgs &g, int kind, hipStream_t stream) {

@@ -98,6 +98,27 @@ def test_tiles_of_128_columns(gpu, types, m, k, n, nk):
     _check(run_spec(spec, [A, np.ascontiguousarray(B.transpose(0, 2, 1)) if nk else B, C]), A, B, C, False, dts)
 
 
+@pytest.mark.parametrize("types,b,m,k,n,columns,orders,accum", [
+    ("bf16", 1, 1411, 733, 2733, 160, "kn nk", False),       # rows and columns short of a tile, odd rows of both
+    ("bf16_out", 2, 641, 898, 3203, 160, "kn nk", True),     # a row and three columns past one; rows on words
+    ("bf16", 1, 2432, 386, 1840, 160, "kn nk", True),        # whole tiles but the last column's half; two elements past six steps
+    ("bf16_out", 1, 1500, 449, 3649, 192, "kn nk", False),   # one column past a tile, one element past seven steps
+    ("bf16", 1, 2305, 1024, 2307, 192, "kn", True),          # rows of A of whole chunks
+    ("bf16_out", 1, 1185, 2047, 3370, 160, "kn", False),     # the longest K, odd rows
+    ("bf16", 1, 1281, 2942, 1997, 128, "kn", False),     # ... on the smaller tile, rows on words
+])
+def test_tiles_past_a_round_of_128_columns(gpu, types, b, m, k, n, columns, orders, accum):
+    dts = TYPES[types]
+    A, B = synth.normal_bf16(185, 0, (b, m, k)), synth.normal_bf16(185, 1, (b, k, n))
+    C = synth.normal_bf16(185, 2, (b, m, n)) if dts[2] == M.bf16 else synth.normal_f32(185, 2, (b, m, n))
+    for order in orders.split():
+        nk = order == "nk"
+        spec = M.Matmul([b, m, k, n], dts, [None, KT if nk else None, None], accum)
+        plan = spec.plan()
+        assert plan.kernels == ["k_gemm_ring"] and plan.steps[0].grid[0] == -(-m // 128) * -(-n // columns), plan
+        _check(run_spec(spec, [A, np.ascontiguousarray(B.transpose(0, 2, 1)) if nk else B, C.copy()]), A, B, C, accum, dts)
+
+
 def test_nonfinite_operands_stay_in_their_rows_and_columns(gpu):
     """A NaN and infinities beside the ends of K, M and N, and of the first step, reach the rows and columns that hold them only."""
     for m, k, n in ((129, 733, 1195), (129, 3333, 195)):   # whole, and in slices of K
