@@ -514,3 +514,21 @@ def test_turned_rows_of_odd_lengths_in_one_launch(gpu, shape):
     got = run_spec(spec, [x, np.zeros(shape, np.float32)])
     want = orc.softmax(list(shape), 1, x)
     assert (np.abs(got - want) <= 1e-5 * np.abs(want) + 1e-12).all()
+
+
+@pytest.mark.parametrize("shape,kernels", [
+    ((9, 513, 1793), 1),   # read twice, 261 tiles of 64 columns: not a multiple of the eight XCDs, the last one of a column
+    ((33, 700, 513), 1),
+    ((1, 1793, 673), 2),   # eleven tiles in pieces of the scan dim
+    ((3, 1001, 65), 2),
+    ((1, 2149, 63), 2),    # a single tile, fewer than XCDs
+    ((9, 640, 1824), 1),   # rows of whole lines
+])
+def test_neighbouring_column_tiles_on_one_xcd(gpu, shape, kernels):
+    x = synth.normal_f32(233, 0, shape, std=2.0)
+    spec = M.Softmax(list(shape), 1)
+    assert spec.plan().kernels == ["k_softmax_cols"] * kernels
+    got = run_spec(spec, [x, np.zeros(shape, np.float32)])
+    e = np.exp(x.astype(np.float64) - x.max(axis=1, keepdims=True))
+    want = e / e.sum(axis=1, keepdims=True)
+    assert (np.abs(got - want) <= 1e-5 * want + 1e-12).all()
