@@ -59,12 +59,8 @@ hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
     case 32: return launch_either<T, A_UNSIGNED, 2, 2>(g, stream);
     case 64: return launch_either<T, A_UNSIGNED, 4, 2>(g, stream);
     case 128: return launch_either<T, A_UNSIGNED, 4, 4>(g, stream);
-    case 160:
-      if constexpr (T::ES == 2) return launch_either<T, A_UNSIGNED, 4, 5>(g, stream);
-      return hipErrorInvalidValue;
-    case 192:
-      if constexpr (T::ES == 2) return launch_either<T, A_UNSIGNED, 4, 6>(g, stream);
-      return hipErrorInvalidValue;
+    case 160: return launch_either<T, A_UNSIGNED, 4, 5>(g, stream);
+    case 192: return launch_either<T, A_UNSIGNED, 4, 6>(g, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -116,9 +112,10 @@ bool slices_are_faster_of_few(const GemmArgs &g, int kind, int es, uint64_t step
 //   64 (128 x 64) where those are: bf16 975 x 2176 x 1666 22.5 / 17.5, u8 1888 x 1633 x 885 17.4 / 14.7; int8 over a long K reads
 //     its rows' lines once too often: 1651 x 5949 x 844 28.8 / 31.8, and bf16 over a longer one: 1835 x 3535 x 655 31.7 / 35.2;
 //   128 (128 x 128), bf16: 1483 x 858 x 1983 18.4 / 15.8, 1303 x 1524 x 2056 24.3 / 20.3; over a long K the copies are
-//     the faster way (1538 x 3021 x 1767 34.2 / 38.6), for int8 at once (1055 x 929 x 1801 13.2 / 15.8);
+//     the faster way (1538 x 3021 x 1767 34.2 / 38.6), for int8 rows of an odd number of bytes at once (1055 x 929 x 1801 13.2 / 15.8); k-fastest
+//     B of others 875 x 3964 x 2980 35.0 / 25.9, 726 x 996 x 4035 17.8 / 13.6;
 //   160 (128 x 160) where those are and 128 x 128 ones are not, else 192 (128 x 192), bf16: 2306 x 735 x 2260 24.5 / 17.4, 2491 x 1862 x 2026 38.8 /
-//     31.3, k-fastest B twice 771 x 813 x 3032 29.1 / 21.2.
+//     31.3, k-fastest B twice 771 x 813 x 3032 29.1 / 21.2; u8 2078 x 1500 x 2672 28.4 / 21.6.
 uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
   if (kind < 0 || kind > 2) return 0;
   const int es = kind == 2 ? 2 : 1;
@@ -164,12 +161,22 @@ uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind) {
   // sizes of these classes 1.20 times as fast with three sets, 1.06 from memory (geometric means; least 1.00 and 0.90).  Of one and two entries, as measured.
   const uint64_t large = tiles(128, 128);
   const bool words = g.lda % 2 == 0 && (!g.b_kmajor || g.ldb % 2 == 0);
-  if (kind == 2 && large > units) {
-    const uint32_t most = g.b_kmajor ? (words ? 20u : 16u) : 32u;
-    if (g.batch > 2 || steps <= 6 || steps > most) return 0;
+  // int8 rows on words, or on pairs of bytes up to 16 steps (from memory and with three sets): k-fastest B from five steps to 34, 875 x 3964 x 2980 35.6 / 31.6, 35.0 / 25.9, 1688 x
+  // 524 x 1292 14.5 / 12.3, 13.5 / 10.3, pairs 945 x 1058 x 3508 19.7 / 17.7, 18.9 / 15.1, 1247 x 1158 x 2125 19.7 / 20.3, 18.2 / 16.4; past those pairs 1329 x 4210 x 1494 33.4 / 39.7,
+  // 32.2 / 31.0; four steps 697 x 504 x 2771 13.4 / 14.1, 12.0 / 11.8.  A row-major B past a round of 128 x 128, of pairs too: 2225 x 1010 x 2684 26.4 / 23.7, 25.9 / 19.6, 2816 x 1812 x
+  // 1415 32.6 / 33.7, 31.7 / 27.7, 1291 x 4236 x 3778 52.4 / 50.7, 51.3 / 42.4.  Below, rows on pairs are as fast either way (2040 x 866 x 1246 15.2 / 17.3, 14.2 / 13.8); rows on words would gain (1857 x 2008 x 1725 26.9 / 26.4, 25.3 / 20.9) and stay with the copies, whose route tests/test_plan_routes.py holds fast for 1500 x 1000 x 1500.  Over 24 random sizes of these
+  // classes 1.10 times as fast from memory, 1.22 with three sets (geometric means; least 0.97 and 1.08).
+  if (kind != 2) {
+    const uint64_t either = uint64_t(g.lda) | (g.b_kmajor ? uint64_t(g.ldb) : 0);
+    if (g.batch > 2 || steps < 5 || either % 2 != 0 || steps > (g.b_kmajor && either % 4 != 0 ? 16u : 34u)) return 0;
+    if (large <= units) return g.b_kmajor && g.n >= 128 ? 128 : 0;
+  } else if (large > units) {
+    if (g.batch > 2 || steps <= 6 || steps > (g.b_kmajor ? (words ? 20u : 16u) : 32u)) return 0;
+  }
+  if (large > units) {
     return g.n >= 160 && tiles(128, 160) <= units ? 160 : g.n >= 192 && tiles(128, 192) <= units ? 192 : 0;
   }
-  if (kind != 2 || g.n < 128 || large > units || (g.accum && g.c_bf16 && steps <= 5 && (g.lda % 2 != 0 || g.ldb % 2 != 0))) return 0;
+  if (g.n < 128 || (g.accum && g.c_bf16 && steps <= 5 && (g.lda % 2 != 0 || g.ldb % 2 != 0))) return 0;
   return steps <= (odd_rows && 3 * large <= 2 * units ? 15u : words && !g.b_kmajor && g.batch <= 2 ? 46u : 24u) ? 128 : 0;
 }
 

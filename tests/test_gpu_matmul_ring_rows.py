@@ -119,6 +119,24 @@ def test_tiles_past_a_round_of_128_columns(gpu, types, b, m, k, n, columns, orde
         _check(run_spec(spec, [A, np.ascontiguousarray(B.transpose(0, 2, 1)) if nk else B, C.copy()]), A, B, C, accum, dts)
 
 
+@pytest.mark.parametrize("types,b,m,k,n,columns,nk,accum", [
+    ("u8", 1, 1285, 522, 1537, 128, True, False),    # ten bytes past four steps, rows on pairs of bytes
+    ("i8", 1, 1281, 4348, 1537, 128, True, True),    # the longest K, rows on words
+    ("u8", 2, 641, 770, 3203, 160, True, True),
+    ("u8", 1, 2432, 642, 1840, 160, False, True),    # whole tiles but the last column's half
+    ("i8", 1, 1500, 1030, 3649, 192, False, False),  # one column past a tile
+    ("u8", 1, 1500, 1030, 3649, 192, True, False),
+])
+def test_int8_tiles_past_a_round(gpu, types, b, m, k, n, columns, nk, accum):
+    dts = TYPES[types]
+    A, B = GEN[dts[0]](186, 0, (b, m, k)), GEN[dts[1]](186, 1, (b, k, n))
+    C = synth.uniform_i8(186, 2, (b, m, n)).astype(np.int32) * 1001
+    spec = M.Matmul([b, m, k, n], dts, [None, KT if nk else None, None], accum)
+    plan = spec.plan()
+    assert plan.kernels == ["k_gemm_ring"] and plan.steps[0].grid[0] == -(-m // 128) * -(-n // columns), plan
+    _check(run_spec(spec, [A, np.ascontiguousarray(B.transpose(0, 2, 1)) if nk else B, C.copy()]), A, B, C, accum, dts)
+
+
 def test_nonfinite_operands_stay_in_their_rows_and_columns(gpu):
     """A NaN and infinities beside the ends of K, M and N, and of the first step, reach the rows and columns that hold them only."""
     for m, k, n in ((129, 733, 1195), (129, 3333, 195)):   # whole, and in slices of K
