@@ -477,6 +477,15 @@ hipError_t launch_either(const GemmArgs &g, hipStream_t stream) {
 
 }  // namespace
 
+// About `want` slices of K, each of so many; 0: too short for it.  The kernels' first step loads as much of K as any other, in the last slice too: that has
+// a step of 32 or more.  (One more step to a slice may leave less than a step again: 1281 in twelve, 128, 160, 192.)
+uint32_t gemm_f32_slice_k(uint32_t k, uint32_t want) {
+  uint32_t slice_k = (k + want * 32 - 1) / (want * 32) * 32;
+  if (slice_k < 128) return 0;
+  while (slice_k < k && k % slice_k != 0 && k % slice_k < 32) slice_k += 32;
+  return slice_k;
+}
+
 // Workgroups of a form go to the compute units in rounds, each as long as a workgroup's steps.  Measured, on operands of 1 to 50 MB: a step of 4 x 32 k of a block of 32 x 32 0.75 us of its unit, however many share it; of 2 x 16 k of 64 x 64
 // 0.5; of 2 x 16 k of 128 x 128 1.05 to, on all units, 1.47; of 16 k of two such workgroups 1.35, of one 0.85.  Slices of K cost the launch that sums them, 2.5 us, and
 // their results at 3 TB/s.  (us, the f32 MFMA on copies of whole chunks / this, form and slices: 195 x 500 x 621 17.0 / 6.9, waves;
@@ -502,9 +511,9 @@ Choice choose(const GemmArgs &g) {
   consider(WIDE_128, 1, g.k, 5.0 + std::max(1.05, 0.75 + 0.72 * std::min(1.0, t128 / units)) * rounds(t128, units) * ((steps + 1) / 2));
   consider(WIDE_128_PAIR, 1, g.k, 5.0 + (t128 <= units ? 0.85 : 1.35 * rounds(t128, 2 * units)) * steps);
   for (uint32_t want : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u}) {
-    uint32_t slice_k = want == 1 ? g.k : (g.k + want * 32 - 1) / (want * 32) * 32;
-    if (want > 1 && (g.batch != 1 || g.tight || slice_k < 128)) break;
-    if (g.k % slice_k != 0 && g.k % slice_k < 32) slice_k += 32;   // (no slice shorter than a step)
+    const uint32_t slice_k = want == 1 ? g.k : gemm_f32_slice_k(g.k, want);
+    if (want > 1 && (g.batch != 1 || g.tight || slice_k == 0)) break;
+    if (want > 1 && slice_k >= g.k) continue;
     const uint32_t slices = (g.k + slice_k - 1) / slice_k;
     const double sum = slices == 1 ? 0.0 : 2.5 + (slices + 1.0) * g.m * g.n * 4.0 / 3e6;
     const uint32_t s16 = (slice_k + 15) / 16, s32 = (slice_k + 31) / 32;
@@ -534,7 +543,10 @@ uint32_t gemm_f32_slices(const GemmArgs &g, uint32_t *slice_k) {
 hipError_t launch_gemm_f32(const GemmArgs &g, hipStream_t stream) {
   GemmArgs whole = g;
   if (g.k_total != 0) whole.batch = 1, whole.k = g.k_total;   // the form goes by the whole problem
-  switch (choose(whole).form) {
+  const Form form = choose(whole).form;
+  const uint32_t last = g.k_total != 0 ? g.k_total - (g.batch - 1) * g.k : g.k;
+  if (last < (form == WAVES ? 32u : 16u)) return hipErrorInvalidValue;   // (the first step would leave K)
+  switch (form) {
     case WAVES: return g.b_kmajor ? launch_waves<true>(g, stream) : launch_waves<false>(g, stream);
     case WIDE_64: return launch_either<1, 2>(g, stream);
     case WIDE_128: return launch_either<2, 2>(g, stream);

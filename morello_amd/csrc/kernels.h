@@ -208,6 +208,7 @@ hipError_t launch_gemm_big(const GemmArgs &g, int kind, hipStream_t stream, uint
 
 // ---- gemm_f32.hip: f32 operands as three bf16 each, rows that start anywhere ----
 bool gemm_f32_applicable(const GemmArgs &g, int kind);
+uint32_t gemm_f32_slice_k(uint32_t k, uint32_t want);
 uint32_t gemm_f32_slices(const GemmArgs &g, uint32_t *slice_k);   // of K, each of *slice_k but the last: k_total then says how long all are
 hipError_t launch_gemm_f32(const GemmArgs &g, hipStream_t stream);
 

@@ -52,3 +52,15 @@ def test_outputs_the_matrix_cores_take(tmp_path):
     assert res.returncode == 0, res.stderr
     run = subprocess.run([str(exe)], capture_output=True, text=True)
     assert run.returncode == 0 and "dispatch ok" in run.stdout, run.stdout[-2000:] + run.stderr
+
+
+def test_slices_of_f32_matmuls_are_no_shorter_than_a_step(tmp_path):
+    """A last slice of 1 to 31 was loaded as a whole step: past A's last row, and up to 31 rows past B's end."""
+    exe = tmp_path / "f32_slices_check"
+    lib_dir = os.path.join(ROOT, "morello_amd")
+    cmd = ["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-isystem", "/opt/rocm/include", os.path.join(ROOT, "tests", "f32_slices_check.cpp"),
+           "-o", str(exe), "-L", lib_dir, "-lmorello_amd", f"-Wl,-rpath,{lib_dir}", "-Wl,-rpath,/opt/rocm/lib"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    run = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert run.returncode == 0 and "f32 slices ok" in run.stdout, run.stdout[-2000:] + run.stderr

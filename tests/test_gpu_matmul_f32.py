@@ -97,3 +97,15 @@ def test_f32_tiny_values_that_huge_ones_bring_back(gpu, m, k, n, nk):
     at = np.ix_(rows, cols)
     assert (np.abs(got[at] - want[at]) <= 2.0 ** -22 * np.abs(want[at])).all(), (got[at], want[at])
     assert np.linalg.norm(np.delete(got - want, cols, 1)) <= 4e-7 * np.linalg.norm(np.delete(want, cols, 1))
+
+
+@pytest.mark.parametrize("m,k,n,nk", [(48, 1281, 1040, False), (272, 1293, 304, True), (400, 1345, 272, False), (112, 1921, 464, False), (144, 2689, 304, True), (112, 3531, 144, False), (720, 3540, 16, True)])
+def test_f32_slices_that_nearly_divide_k(gpu, m, k, n, nk):
+    """K a little over a number of slices, whose last one was loaded past the operands' ends."""
+    spec = _spec(1, m, k, n, nk)
+    plan = spec.plan()
+    assert plan.kernels == [plan.steps[0].family, "k_sum_splits"] and plan.steps[0].family.startswith("k_gemm_f32"), plan
+    A, B = synth.normal_f32(194, 0, (1, m, k)), synth.normal_f32(194, 1, (1, k, n))
+    got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk).astype(np.float64)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    assert np.linalg.norm(got - want) <= 4e-7 * np.linalg.norm(want)
