@@ -87,16 +87,16 @@ __device__ inline float probe_of(const float (&sum)[N]) {
 }
 
 // Whether a tile's parts did: no value that is infinite or no number among this thread's sums, and no row of A or column of B, whose
-// N largest magnitudes this thread keeps (`which`: numbers of theirs below `all`), with a huge value or of nothing but tiny ones.  Of the
-// workgroup.
+// N largest magnitudes this thread keeps (`which`: numbers of theirs below `all`; zeros where it `had` no values), with a huge value or of
+// nothing but tiny ones.  Of the workgroup.
 template <int N>
-__device__ inline bool parts_did(const float (&most)[N], const int (&which)[N], int all, float probe, uint32_t *seen) {
+__device__ inline bool parts_did(const float (&most)[N], const int (&which)[N], int all, bool had, float probe, uint32_t *seen) {
   bool never = probe != probe;
 #pragma unroll
   for (int i = 0; i < N; i++) never = never || most[i] > HUGE_VALUE;
   bool odd = never;
 #pragma unroll
-  for (int i = 0; i < N; i++) odd = odd || !(most[i] >= TINY);
+  for (int i = 0; i < N; i++) odd = odd || (had && !(most[i] >= TINY));
   if (!__syncthreads_or(odd)) return true;
   if (__syncthreads_or(never)) return false;
   for (int i = threadIdx.x; i < all; i += blockDim.x) seen[i] = 0;
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
   const int64_t row0 = m0 + wm * 32 * T, col0 = n0 + wn * 32 * T;
   float sum[T * T * 16 / G];
   meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
-  if (!parts_did(most, which, 2 * BM, probe_of(sum), (uint32_t *)lds)) {
+  if (!parts_did(most, which, 2 * BM, true, probe_of(sum), (uint32_t *)lds)) {
     multiply_f32<T, G, B_KMAJOR>(p, row0, col0, group, big);
     meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
   }
@@ -429,9 +429,7 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
   const int which[2] = {li, 32 + li};
   float sum[16 / DEAL];
   meet<1, DEAL>(part, 1024, 0, wave, big, sum);
-  // (a wave without a step has nothing to say)
-  const float known[2] = {mine ? most[0] : 1.0f, mine ? most[1] : 1.0f};
-  if (!parts_did(known, which, 64, probe_of(sum), (uint32_t *)part)) {
+  if (!parts_did(most, which, 64, mine > 0, probe_of(sum), (uint32_t *)part)) {
     multiply_f32<1, DEAL, B_KMAJOR>(p, m0, n0, wave, big);
     meet<1, DEAL>(part, 1024, 0, wave, big, sum);
   }

@@ -109,3 +109,20 @@ def test_f32_slices_that_nearly_divide_k(gpu, m, k, n, nk):
     got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk).astype(np.float64)
     want = A.astype(np.float64) @ B.astype(np.float64)
     assert np.linalg.norm(got - want) <= 4e-7 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("m,k,n,nk,last", [(500, 95, 500, True, 95), (511, 65, 261, True, 65), (300, 47, 301, True, 47), (300, 33, 301, True, 33), (160, 675, 197, False, 35), (150, 816, 420, True, 48)])
+def test_f32_tiny_rows_over_fewer_steps_than_waves(gpu, m, k, n, nk, last):
+    """A row and a column of nothing but tiny values where some of a tile's waves have no step of K, or of its last slice."""
+    A, B = np.abs(synth.normal_f32(195, 0, (1, m, k))), np.abs(synth.normal_f32(195, 1, (1, k, n))) + np.float32(0.01)
+    A[0, 100, :k - last] = B[0, :k - last, 20] = 0
+    A[0, 100] *= np.float32(1e-36)
+    B[0, :, 20] *= np.float32(1e-36)
+    spec = _spec(1, m, k, n, nk)
+    assert spec.plan().kernels[0] == "k_gemm_f32_waves"
+    got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk)[0].astype(np.float64)
+    want = A[0].astype(np.float64) @ B[0].astype(np.float64)
+    normal = want >= 2.0 ** -120   # (below: the products themselves are denormal)
+    for at in (np.s_[100, :], np.s_[:, 20]):   # (sums of `last` terms)
+        assert (np.abs(got - want)[at] <= (last + 4) * 2.0 ** -24 * want[at])[normal[at]].all()
+    assert normal[100].sum() >= n - 1 and normal[:, 20].sum() >= m - 1
