@@ -1,11 +1,13 @@
 // f32 Matmul through the bf16 matrix cores: every f32 as three bf16 that add up to it exactly.
 //
 // The f32 MFMA has a sixteenth of the bf16 one's rate.  A value's upper 16 bits are a bf16 (h); what is left has 16 bits, of
-// which the rounded upper half (m) and the rest (l) are bf16 too: x = h + m + l without error, and
-//   x y = h h' + (h m' + m h') + (m m' + h l' + l h') + the rest, below 2^-23 |x y| and of either sign:
-// six MFMAs for sixteen k where the f32 form takes eight of twice the time each.  The products but the first are summed on
-// their own.  The roundings of a sum, one to sixteen terms and not to two, then come to less than those of the f32 MFMA: relative
-// error in the norm for 0.5 x normal operands, f32 MFMA / this: K = 128 9.3e-8 / 6.5e-8, 1024 5.7e-7 / 1.3e-7, 2048 8.1e-7 / 1.9e-7.
+// which the rounded upper half (m) and the rest (l) are bf16 too: x = h + m + l without error, m below 2^-7 |x| and l at most 2^-16 |x|, and
+//   x y = h h' + (h m' + m h') + (m m' + h l' + l h') + (m l' + l m') + l l', the last at most 2^-32 |x y| and left out:
+// eight MFMAs for sixteen k where the f32 form takes eight of twice the time each.  The products but the first are summed on
+// their own, 2^-6 of the first and less, so that a sum of one term is rounded as once (within 2^-24 and a sixteenth of that; without m l' + l m', 3 to 18 % faster, 2^-22).
+// The roundings of a longer sum, one to sixteen terms and not to two, come to less than those of the f32 MFMA: relative
+// error in the norm for 0.5 x normal operands, f32 MFMA / this: K = 226 2.7e-7 / 6.7e-8, 1024 5.7e-7 / 1.3e-7, 1500 6.9e-7 / 1.6e-7.
+// (The three parts: G. Henry, P. Tang and A. Heinecke, Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations, 2019.)
 //
 // Where the parts would not do, the tile is computed again by the f32 MFMA: an infinity in A or B leaves a NaN (its m is inf - inf),
 // and so does an overflow on the way; and in a row of A or column of B of nothing but tiny values the l, then the m, are no
@@ -13,7 +15,7 @@
 // computed again too, since it could bring the lost parts of a tiny value beside ordinary ones back to the size of a result.  (All
 // tiles twice: 2048^3 with an infinity in every sixteenth row 370 us, 512^3 18.)
 //
-// What bounds it: the bf16 MFMAs at what the board's power lets them run at (4096^3 in 695 us is 1.19 PFLOP/s of them, where the 256 tile
+// What bounds it: the bf16 MFMAs at what the board's power lets them run at (4096^3 in 838 us is 1.31 PFLOP/s of them, where the 256 tile
 // reaches 1.42), for the smaller tiles the cutting, six vector instructions a value; below a round of tiles the chain of a step.
 //
 // Rows start on any element and are read in place.  The first step takes what K has over whole steps, zeros behind it, so that no
@@ -288,7 +290,7 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
 #pragma unroll
         for (int c = 0; c < T; c++) acc[r][c] = mfma(f.a[x][r], f.b[y][c], acc[r][c]);
     };
-    all(0, 1, small), all(0, 0, big), all(1, 0, small), all(1, 1, small), all(0, 2, small), all(2, 0, small);
+    all(0, 1, small), all(0, 0, big), all(1, 0, small), all(1, 1, small), all(0, 2, small), all(2, 0, small), all(1, 2, small), all(2, 1, small);
   };
   // All LDS reads and writes are done; loads stay under way.
   auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
@@ -301,9 +303,9 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
     multiply(f);
     __builtin_amdgcn_sched_group_barrier(0x100, 6 * T, 0);   // the reads, then an MFMA and some of the cutting in turn
 #pragma unroll
-    for (int i = 0; i < 6 * T * T; i++) {
+    for (int i = 0; i < 8 * T * T; i++) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, T == 2 ? 5 : 10, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, T == 2 ? 4 : 8, 0);
     }
     barrier();
   };
@@ -402,6 +404,8 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
     small = mfma(x.m, y.m, small);
     small = mfma(x.h, y.l, small);
     small = mfma(x.l, y.h, small);
+    small = mfma(x.m, y.l, small);
+    small = mfma(x.l, y.m, small);
   };
   const int mine = steps > wave ? (steps - wave + DEAL - 1) / DEAL : 0;
   if (mine > 0) {
@@ -438,9 +442,9 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
 
 void declare_work(const GemmArgs &g, int side, int k_step, double serial_ns) {
   const double mn = double(g.m) * g.n * g.batch;
-  // (1.2 to 1.3 times the rate that the model takes for the f32 MFMA)
+  // (1.1 to 1.3 times the rate that the model takes for the f32 MFMA)
   plan::work(plan::UNIT_MFMA_F32, 2.0 * mn * g.k, (double(g.m) * g.k + double(g.k) * g.n) * g.batch * 4 + mn * 4 * (g.accum ? 2 : 1),
-             2.0 * side * side * double((g.k + k_step - 1) / k_step * k_step), serial_ns, 1.4);
+             2.0 * side * side * double((g.k + k_step - 1) / k_step * k_step), serial_ns, 1.3);
 }
 
 template <int T, int G, bool B_KMAJOR>
@@ -486,9 +490,9 @@ uint32_t gemm_f32_slice_k(uint32_t k, uint32_t want) {
 
 // Workgroups of a form go to the compute units in rounds, each as long as a workgroup's steps.  Measured, on operands of 1 to 50 MB: a step of 4 x 32 k of a block of 32 x 32 0.75 us of its unit, however many share it; of 2 x 16 k of 64 x 64
 // 0.5; of 2 x 16 k of 128 x 128 1.05 to, on all units, 1.47; of 16 k of two such workgroups 1.35, of one 0.85.  Slices of K cost the launch that sums them, 2.5 us, and
-// their results at 3 TB/s.  (us, the f32 MFMA on copies of whole chunks / this, form and slices: 195 x 500 x 621 17.0 / 6.9, waves;
-// 192 x 2176 x 128 16.1 / 9.2, waves in 8; twice 382 x 226 x 1179 14.1 / 8.7, 64 wide; 537 x 1668 x 568 25.0 / 17.0, 64 wide in 3; 2048^3 162
-// / 98.9, 128 wide in two groups; 2070 x 389 x 3128 68.2 / 47.9, 128 wide in one; 4096^3 943 / 695.)
+// their results at 3 TB/s.  (us, the f32 MFMA on copies of whole chunks / this, form and slices: 195 x 500 x 621 17.0 / 7.4, waves;
+// 192 x 2176 x 128 16.4 / 8.8, waves in 8; twice 382 x 226 x 1179 14.2 / 9.3, 64 wide; 537 x 1668 x 568 23.1 / 17.8, 64 wide in 3; 2048^3 153
+// / 121, 128 wide in two groups; 2070 x 389 x 3128 57.7 / 47.6, 128 wide in one; 4096^3 959 / 838.)
 namespace {
 enum Form : uint32_t { NONE, WAVES, WIDE_64, WIDE_128, WIDE_128_PAIR };
 struct Choice {
