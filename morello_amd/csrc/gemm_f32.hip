@@ -9,14 +9,16 @@
 // error in the norm for 0.5 x normal operands, f32 MFMA / this: K = 226 2.7e-7 / 6.7e-8, 1024 5.7e-7 / 1.3e-7, 1500 6.9e-7 / 1.6e-7.
 // (The three parts: G. Henry, P. Tang and A. Heinecke, Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations, 2019.)
 //
-// Where the parts would not do, the tile is computed again by the f32 MFMA: an infinity in A or B leaves a NaN (its m is inf - inf),
-// and so does an overflow on the way; and in a row of A or column of B of nothing but tiny values the l, then the m, are no
-// bf16 any more.  Each thread keeps the largest magnitude of what it cuts up, all of one row or column; one past 2^60 has its tile
-// computed again too, since it could bring the lost parts of a tiny value beside ordinary ones back to the size of a result.  (All
-// tiles twice: 2048^3 with an infinity in every sixteenth row 370 us, 512^3 18.)
+// Where the parts would not do, the tile is computed again by the f32 MFMA:
+//   - an infinity in A or B leaves a NaN (its m is inf - inf), and so does an overflow on the way;
+//   - below 2^-110 the lowest bits of a value may lie below 2^-133, the lowest of a bf16 (the MFMA takes and makes denormals): each thread notes whether it cut
+//     such bits off, and the largest magnitude of what it cuts up.  K such losses times that magnitude have to be below half of the last bit of every sum
+//     of the tile: beside values of ordinary size they are unless those meet nothing but zeros;
+//   - sums below 2^-120, whose parts' products are rounded at 2^-149 more often than the f32 MFMA would.
+// (All tiles twice: 2048^3 with an infinity in every sixteenth row 370 us, 512^3 18.)
 //
 // What bounds it: the bf16 MFMAs at what the board's power lets them run at (4096^3 in 838 us is 1.31 PFLOP/s of them, where the 256 tile
-// reaches 1.42), for the smaller tiles the cutting, six vector instructions a value; below a round of tiles the chain of a step.
+// reaches 1.42), for the smaller tiles the cutting, six and a half vector instructions a value; below a round of tiles the chain of a step.
 //
 // Rows start on any element and are read in place.  The first step takes what K has over whole steps, zeros behind it, so that no
 // load but its leaves K and none is masked; rows past M and columns past N are the last one again and are not stored.
@@ -33,15 +35,14 @@ typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float four_on_word __attribute__((ext_vector_type(4), aligned(4)));
 
-// A row or column whose largest magnitude reaches it loses nothing that counts beside that value (its lowest bit is 2^-113, a bf16
-// goes down to 2^-126 without denormals).
-constexpr float TINY = 0x1p-90f;
-// What a value loses below 2^-126 stays below 2^-66 of a product as long as the other operand stays below this.
-constexpr float HUGE_VALUE = 0x1p60f;
-
 struct Parts { v4i h, m, l; };
-// Eight values as three chunks of eight bf16; `most`: the largest magnitude so far.
-__device__ inline Parts cut(const float *x, float &most) {
+// What a thread has cut up so far: the largest magnitude; and, in the lower half, bits that no part has.
+struct Seen {
+  float most = 0.0f;
+  uint32_t lost = 0;
+};
+// Eight values as three chunks of eight bf16.
+__device__ inline Parts cut(const float *x, Seen &seen) {
   Parts p;
   float r[8];
 #pragma unroll
@@ -49,14 +50,16 @@ __device__ inline Parts cut(const float *x, float &most) {
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     p.h[i] = int(__builtin_amdgcn_perm(__float_as_uint(x[2 * i + 1]), __float_as_uint(x[2 * i]), 0x07060302));   // the upper halves
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(x[2 * i]), "v"(x[2 * i + 1]));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(seen.most) : "v"(x[2 * i]), "v"(x[2 * i + 1]));
   }
 #pragma unroll
   for (int i = 0; i < 4; i++) p.m[i] = __builtin_bit_cast(int, __builtin_convertvector((v2f{r[2 * i], r[2 * i + 1]}), v2bf));
 #pragma unroll
-  for (int i = 0; i < 4; i++) r[2 * i] -= __uint_as_float(uint32_t(p.m[i]) << 16), r[2 * i + 1] -= __uint_as_float(uint32_t(p.m[i]) & 0xffff0000u);
-#pragma unroll
-  for (int i = 0; i < 4; i++) p.l[i] = int(__builtin_amdgcn_perm(__float_as_uint(r[2 * i + 1]), __float_as_uint(r[2 * i]), 0x07060302));
+  for (int i = 0; i < 4; i++) {
+    r[2 * i] -= __uint_as_float(uint32_t(p.m[i]) << 16), r[2 * i + 1] -= __uint_as_float(uint32_t(p.m[i]) & 0xffff0000u);
+    asm("v_or3_b32 %0, %0, %1, %2" : "+v"(seen.lost) : "v"(r[2 * i]), "v"(r[2 * i + 1]));
+    p.l[i] = int(__builtin_amdgcn_perm(__float_as_uint(r[2 * i + 1]), __float_as_uint(r[2 * i]), 0x07060302));
+  }
   return p;
 }
 
@@ -79,36 +82,26 @@ struct Problem {
   }
 };
 
-// No number where one of the sums is none, or infinite.
+// Whether a tile's parts did, of the workgroup: `sum`, this thread's of `k` terms, holds nothing infinite, no NaN and no sum below 2^-120 but zeros; and
+// what the threads lost counts for nothing in any of them.  (A loss is below 2^-133, so that of a product's two values below 2^-132 times the largest.)
 template <int N>
-__device__ inline float probe_of(const float (&sum)[N]) {
+__device__ inline bool parts_did(const Seen &seen, const float (&sum)[N], int k, uint32_t *largest) {
   float probe = 0.0f;
+  uint32_t least = ~0u;   // twice the smallest magnitude's bits less one, zeros left out
 #pragma unroll
-  for (int e = 0; e < N; e++) probe = __builtin_fmaf(0.0f, sum[e], probe);
-  return probe;
-}
-
-// Whether a tile's parts did: no value that is infinite or no number among this thread's sums, and no row of A or column of B, whose
-// N largest magnitudes this thread keeps (`which`: numbers of theirs below `all`; zeros where it `had` no values), with a huge value or of
-// nothing but tiny ones.  Of the workgroup.
-template <int N>
-__device__ inline bool parts_did(const float (&most)[N], const int (&which)[N], int all, bool had, float probe, uint32_t *seen) {
-  bool never = probe != probe;
-#pragma unroll
-  for (int i = 0; i < N; i++) never = never || most[i] > HUGE_VALUE;
-  bool odd = never;
-#pragma unroll
-  for (int i = 0; i < N; i++) odd = odd || (had && !(most[i] >= TINY));
-  if (!__syncthreads_or(odd)) return true;
+  for (int e = 0; e < N; e++) probe = __builtin_fmaf(0.0f, sum[e], probe), least = min(least, 2 * __float_as_uint(sum[e]) - 1);
+  const bool never = probe != probe || least < 2 * __float_as_uint(0x1p-120f) - 1, lost = (seen.lost & 0xffff) != 0;
+  if (!__syncthreads_or(never || lost)) return true;
   if (__syncthreads_or(never)) return false;
-  for (int i = threadIdx.x; i < all; i += blockDim.x) seen[i] = 0;
+  if (threadIdx.x == 0) *largest = 0;
   __syncthreads();
+  atomicMax(largest, __float_as_uint(seen.most));
+  __syncthreads();
+  const float counts = __uint_as_float(*largest) * (float(k) * 0x1p-107f);
+  bool below = false;
 #pragma unroll
-  for (int i = 0; i < N; i++) atomicMax(seen + which[i], __float_as_uint(most[i]));
-  __syncthreads();
-  bool tiny = false;
-  for (int i = threadIdx.x; i < all; i += blockDim.x) tiny = tiny || (seen[i] != 0 && seen[i] < __float_as_uint(TINY));
-  return !__syncthreads_or(tiny);
+  for (int e = 0; e < N; e++) below = below || !(__builtin_fabsf(sum[e]) >= counts);
+  return !__syncthreads_or(below);
 }
 
 // The `share`-th of SHARES parts of a wave's T x T blocks, block after block.  Register i of a block: row 8 (i / 4) + 4 (l / 32) + i % 4, column l % 32.
@@ -213,7 +206,7 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
   constexpr int OPERANDS = T == 2 ? 2 : 1;
   const uint8_t *from[OPERANDS];
   uint32_t off[OPERANDS];
-  int half[OPERANDS], at[OPERANDS], which[OPERANDS];
+  int half[OPERANDS], at[OPERANDS];
   int next = min(group, steps - 1);   // the step that `from` is at
   const bool second = T == 1 && __builtin_amdgcn_readfirstlane(tid >> 7);
   auto across = [&](int o) { return !B_KMAJOR && (T == 2 ? o == 1 : second); };
@@ -231,11 +224,8 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
       off[o] = uint32_t(min(row, int((is_b ? p.n - n0 : p.m - m0) - 1))) * (is_b ? p.ldb_b : p.lda_b) + 32 * half[o];
     }
     at[o] = (is_b ? S::OPERAND : 0) + place(row, half[o]);
-    which[o] = (is_b ? BM : 0) + row;
   }
-  float most[OPERANDS];
-#pragma unroll
-  for (int o = 0; o < OPERANDS; o++) most[o] = 0.0f;
+  Seen seen;
 
   struct Values { float x[OPERANDS][8]; };
   Values kept[2];
@@ -259,7 +249,7 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
   auto put = [&](const Values &v, uint8_t *stage) {
 #pragma unroll
     for (int o = 0; o < OPERANDS; o++) {
-      const Parts c = cut(v.x[o], most[o]);
+      const Parts c = cut(v.x[o], seen);
       uint8_t *to = stage + at[o];
       *(v4i *)to = c.h, *(v4i *)(to + S::PART) = c.m, *(v4i *)(to + 2 * S::PART) = c.l;
     }
@@ -342,7 +332,7 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
   const int64_t row0 = m0 + wm * 32 * T, col0 = n0 + wn * 32 * T;
   float sum[T * T * 16 / G];
   meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
-  if (!parts_did(most, which, 2 * BM, true, probe_of(sum), (uint32_t *)lds)) {
+  if (!parts_did(seen, sum, p.k, (uint32_t *)lds)) {
     multiply_f32<T, G, B_KMAJOR>(p, row0, col0, group, big);
     meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
   }
@@ -393,7 +383,7 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
     a += int64_t(ahead) * 4, b += B_KMAJOR ? int64_t(ahead) * 4 : int64_t(ahead) * p.ldb_b;
     next += ahead ? DEAL : 0;
   };
-  float most[2] = {0.0f, 0.0f};
+  Seen seen;
   v16f big[1][1], small;
 #pragma unroll
   for (int i = 0; i < 16; i++) big[0][0][i] = small[i] = 0.0f;
@@ -419,9 +409,9 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
       ring::each<D>([&](auto d) {
         Values &v = kept[decltype(d)::value];
         if (!done) {
-          const Parts a0 = cut(v.a, most[0]), b0 = cut(v.b, most[1]);
+          const Parts a0 = cut(v.a, seen), b0 = cut(v.b, seen);
           multiply(a0, b0);
-          const Parts a1 = cut(v.a + 8, most[0]), b1 = cut(v.b + 8, most[1]);
+          const Parts a1 = cut(v.a + 8, seen), b1 = cut(v.b + 8, seen);
           load(v);
           multiply(a1, b1);
           done = --left == 0;
@@ -430,10 +420,9 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
     }
   }
   big[0][0] += small;
-  const int which[2] = {li, 32 + li};
   float sum[16 / DEAL];
   meet<1, DEAL>(part, 1024, 0, wave, big, sum);
-  if (!parts_did(most, which, 64, mine > 0, probe_of(sum), (uint32_t *)part)) {
+  if (!parts_did(seen, sum, p.k, (uint32_t *)part)) {
     multiply_f32<1, DEAL, B_KMAJOR>(p, m0, n0, wave, big);
     meet<1, DEAL>(part, 1024, 0, wave, big, sum);
   }

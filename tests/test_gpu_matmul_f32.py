@@ -143,3 +143,41 @@ def test_f32_sums_of_one_term_are_rounded_once(gpu, m, k, n, nk):
     want = values[:, None].astype(np.float64) * B[0, at].astype(np.float64)
     assert (np.abs(got - want) <= (1 + 2.0 ** -4) * 2.0 ** -24 * np.abs(want)).all()
     assert (got != want.astype(np.float32)).mean() < 0.02   # (near a tie)
+
+
+def _of_all_sizes(index, shape, lo, hi):
+    """Values of magnitudes from 2^lo to 2^hi, all 24 bits of them in use (fewer below 2^-126)."""
+    x = synth.normal_f32(197, index, shape)
+    mantissa, _ = np.frexp(np.where(x == 0, np.float32(1), x))
+    exponents = lo + (np.abs(synth.normal_f32(198, index, shape)) * 1e6).astype(np.int64) % (hi - lo)
+    return np.ldexp(mantissa, (exponents + 1).astype(np.int32)).astype(np.float32)
+
+
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("m,k", [(511, 501), (2477, 257), (1340, 1637), (6071, 1029), (137, 1667)])
+def test_f32_values_down_to_the_smallest_beside_ones(gpu, m, k, nk):
+    """Times the identity every value is itself, denormals too, also where a part of it is below the smallest bf16; with a one in every row."""
+    A, B = _of_all_sizes(0, (1, m, k), -149, 10), np.eye(k, dtype=np.float32)[None]
+    A[0, :, 5] = 1
+    spec = _spec(1, m, k, k, nk)
+    assert spec.plan().kernels[0].startswith("k_gemm_f32")
+    got = _run(spec, A, B, np.zeros((1, m, k), np.float32), nk)
+    assert np.array_equal(got, A)
+
+
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("lo_a,hi_a,lo_b,hi_b", [(-130, 0, 0, 60), (-70, -50, -80, -50), (-149, 1, -20, 100), (-1, 1, -126, 1), (20, 100, -149, -90)])
+@pytest.mark.parametrize("m,k,n", [(511, 513, 261), (2477, 129, 257), (1740, 751, 1637), (2071, 389, 3129), (537, 1667, 569)])
+def test_f32_one_term_of_any_size_beside_zeros(gpu, m, k, n, lo_a, hi_a, lo_b, hi_b, nk):
+    """A row of A has a one that meets a zero and one value of any size that meets one of any size: the product, rounded once; or, among
+    the denormals, within one of the smallest."""
+    values, others = _of_all_sizes(1, (m,), lo_a, hi_a), _of_all_sizes(2, (1, k, n), lo_b, hi_b)
+    A, B = np.zeros((1, m, k), np.float32), others
+    at = 1 + np.arange(m) * 7 % (k - 1)
+    A[0, :, 0], B[0, 0] = 1, 0
+    A[0, np.arange(m), at] = values
+    spec = _spec(1, m, k, n, nk)
+    assert spec.plan().kernels[0].startswith("k_gemm_f32")
+    got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk)[0].astype(np.float64)
+    want = values[:, None].astype(np.float64) * B[0, at].astype(np.float64)
+    assert (np.abs(got - want) <= (1 + 2.0 ** -4) * 2.0 ** -24 * np.abs(want) + np.where(np.abs(want) < 2.0 ** -120, 2.0 ** -149, 0)).all()
