@@ -15,7 +15,9 @@
 //     such bits off, and the largest magnitude of what it cuts up.  K such losses times that magnitude have to be below half of the last bit of every sum
 //     of the tile: beside values of ordinary size they are unless those meet nothing but zeros;
 //   - sums below 2^-120, whose parts' products are rounded at 2^-149 more often than the f32 MFMA would.
-// (All tiles twice: 2048^3 with an infinity in every sixteenth row 370 us, 512^3 18.)
+// The second pass stages the values as they are.  (us, nothing of the kind / an infinity in every sixteenth row / -3.4e38 in every row / all of A below
+// 2^-119, beside them the f32 MFMA's own kernel: 2048^3 118 / 159 / 150 / 241, 140; 1000^3 22 / 39 / 26 / 39, 25; 512^3 6.8 / 11.3 / 11.3 / 11.3, 11.5.  From memory without staging, and with
+// all values past 2^60 counted among these: 2048^3 328, with a k-fastest B 534, 1000^3 126, 512^3 18.)
 //
 // What bounds it: the bf16 MFMAs at what the board's power lets them run at (4096^3 in 838 us is 1.31 PFLOP/s of them, where the 256 tile
 // reaches 1.42), for the smaller tiles the cutting, six and a half vector instructions a value; below a round of tiles the chain of a step.
@@ -31,6 +33,7 @@ using gemm::TileWalk;
 using gemm::v4i;
 using gemm::v8bf;
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float four_on_word __attribute__((ext_vector_type(4), aligned(4)));
@@ -92,6 +95,11 @@ __device__ inline bool parts_did(const Seen &seen, const float (&sum)[N], int k,
   for (int e = 0; e < N; e++) probe = __builtin_fmaf(0.0f, sum[e], probe), least = min(least, 2 * __float_as_uint(sum[e]) - 1);
   const bool never = probe != probe || least < 2 * __float_as_uint(0x1p-120f) - 1, lost = (seen.lost & 0xffff) != 0;
   if (!__syncthreads_or(never || lost)) return true;
+  // (nothing large and no small result, as it mostly is: two barriers, not the largest magnitude's five)
+  bool small = seen.most > 0x1p20f;
+#pragma unroll
+  for (int e = 0; e < N; e++) small = small || !(__builtin_fabsf(sum[e]) >= float(k) * 0x1p-87f);
+  if (!__syncthreads_or(never || small)) return true;
   if (__syncthreads_or(never)) return false;
   if (threadIdx.x == 0) *largest = 0;
   __syncthreads();
@@ -142,41 +150,6 @@ __device__ inline void meet(float *lds, int stride, int wave_of_tile, int part, 
   }
 }
 
-// T x T blocks of 32 x 32 from (m0, n0) on by the f32 MFMA, every PARTS-th sixteen k: what the parts of a value cannot do.
-template <int T, int PARTS, bool B_KMAJOR>
-__device__ inline void multiply_f32(const Problem &p, int64_t m0, int64_t n0, int part, v16f (&acc)[T][T]) {
-  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
-  const float *a[T], *b[T];
-#pragma unroll
-  for (int t = 0; t < T; t++) {
-    const int64_t row = min(m0 + 32 * t + li, p.m - 1), col = min(n0 + 32 * t + li, p.n - 1);
-    a[t] = (const float *)(p.a + row * p.lda_b), b[t] = (const float *)(p.b + (B_KMAJOR ? col * p.ldb_b : col * 4));
-#pragma unroll
-    for (int c = 0; c < T; c++)
-#pragma unroll
-      for (int i = 0; i < 16; i++) acc[t][c][i] = 0.0f;
-  }
-  for (int k0 = 16 * part; k0 < p.k; k0 += 16 * PARTS) {
-    float x[8][T], y[8][T];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int at = min(k0 + 8 * lh + i, p.k - 1);
-#pragma unroll
-      for (int t = 0; t < T; t++) x[i][t] = a[t][at], y[i][t] = B_KMAJOR ? b[t][at] : *(const float *)((const uint8_t *)b[t] + int64_t(at) * p.ldb_b);
-    }
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      if (k0 + 8 * lh + i >= p.k)
-#pragma unroll
-        for (int t = 0; t < T; t++) x[i][t] = y[i][t] = 0.0f;
-#pragma unroll
-      for (int r = 0; r < T; r++)
-#pragma unroll
-        for (int c = 0; c < T; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i][r], y[i][c], acc[r][c], 0, 0, 0);
-    }
-  }
-}
-
 // T x T blocks to a wave, four waves to a tile of 64 T x 64 T; G groups of four waves take every G-th step of 16 k.
 template <int T, int G>
 struct Staged {
@@ -184,7 +157,8 @@ struct Staged {
   static constexpr int GROUP = G > 1 && BM * BM * 4 > 2 * STAGE ? BM * BM * 4 : 2 * STAGE;   // a group's two stages, or its sums
 };
 // A thread cuts eight k of a row of A or a column of B at a time and writes the parts to LDS as the MFMA takes them.  Step j's MFMAs,
-// the cutting of step j + 1's values and the loads of step j + 3 run between two barriers, dealt out by the scheduler hints.
+// the cutting of step j + 1's values and the loads of step j + 3 run between two barriers, dealt out by the scheduler hints.  Computed again, the same pass
+// takes the values to LDS as they are, for the f32 MFMA.
 template <int T, int G, bool B_KMAJOR>
 __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_PARAMS, GemmArgs g) {
   typedef Staged<T, G> S;
@@ -206,34 +180,39 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
   constexpr int OPERANDS = T == 2 ? 2 : 1;
   const uint8_t *from[OPERANDS];
   uint32_t off[OPERANDS];
-  int half[OPERANDS], at[OPERANDS];
-  int next = min(group, steps - 1);   // the step that `from` is at
-  const bool second = T == 1 && __builtin_amdgcn_readfirstlane(tid >> 7);
-  auto across = [&](int o) { return !B_KMAJOR && (T == 2 ? o == 1 : second); };
+  int half[OPERANDS], row[OPERANDS], at[OPERANDS];
+  int next;   // the step that `from` is at
+  const bool second = T == 1 && __builtin_amdgcn_readfirstlane(tid >> 7);   // (a type below, so that no step branches on it)
+  auto is_b = [](auto second, int o) { return T == 2 ? o == 1 : decltype(second)::value; };
+  auto across = [&](auto second, int o) { return !B_KMAJOR && is_b(second, o); };
+  auto begin = [&](auto second) {
+    next = min(group, steps - 1);
+    asm volatile("" : "+s"(next));   // (or the second pass keeps the first one's addresses, in scratch)
+    const int k0 = next == 0 ? 0 : head + K * (next - 1);
 #pragma unroll
-  for (int o = 0; o < OPERANDS; o++) {
-    const bool is_b = T == 2 ? o == 1 : second;
-    const int t = T == 2 ? tid : tid & 127, k0 = next == 0 ? 0 : head + K * (next - 1);
-    const int row = across(o) ? t % BM : t >> 1;
-    half[o] = across(o) ? __builtin_amdgcn_readfirstlane(t / BM) : t & 1;
-    if (across(o)) {
-      from[o] = p.b + n0 * 4 + int64_t(k0 + 8 * half[o]) * p.ldb_b;
-      off[o] = uint32_t(min(row, int(p.n - n0) - 1)) * 4;
-    } else {
-      from[o] = (is_b ? p.b + n0 * p.ldb_b : p.a + m0 * p.lda_b) + int64_t(k0) * 4;
-      off[o] = uint32_t(min(row, int((is_b ? p.n - n0 : p.m - m0) - 1))) * (is_b ? p.ldb_b : p.lda_b) + 32 * half[o];
+    for (int o = 0; o < OPERANDS; o++) {
+      const int t = T == 2 ? tid : tid & 127;
+      row[o] = across(second, o) ? t % BM : t >> 1;
+      half[o] = across(second, o) ? __builtin_amdgcn_readfirstlane(t / BM) : t & 1;
+      at[o] = (is_b(second, o) ? S::OPERAND : 0) + place(row[o], half[o]);
+      if (across(second, o)) {
+        from[o] = p.b + n0 * 4 + int64_t(k0 + 8 * half[o]) * p.ldb_b;
+        off[o] = uint32_t(min(row[o], int(p.n - n0) - 1)) * 4;
+      } else {
+        from[o] = (is_b(second, o) ? p.b + n0 * p.ldb_b : p.a + m0 * p.lda_b) + int64_t(k0) * 4;
+        off[o] = uint32_t(min(row[o], int((is_b(second, o) ? p.n - n0 : p.m - m0) - 1))) * (is_b(second, o) ? p.ldb_b : p.lda_b) + 32 * half[o];
+      }
     }
-    at[o] = (is_b ? S::OPERAND : 0) + place(row, half[o]);
-  }
+  };
   Seen seen;
 
   struct Values { float x[OPERANDS][8]; };
   Values kept[2];
-  auto load = [&](Values &to) {   // this group's next step (past its last: that again)
+  auto load = [&](auto second, Values &to) {   // this group's next step (past its last: that again)
     const int ahead = next + G >= steps ? 0 : next == 0 ? head + K * (G - 1) : K * G;
 #pragma unroll
     for (int o = 0; o < OPERANDS; o++) {
-      if (across(o)) {
+      if (across(second, o)) {
 #pragma unroll
         for (int i = 0; i < 8; i++) to.x[o][i] = *(const float *)(from[o] + i * int64_t(p.ldb_b) + off[o]);
         from[o] += ahead * int64_t(p.ldb_b);
@@ -282,58 +261,127 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
     };
     all(0, 1, small), all(0, 0, big), all(1, 0, small), all(1, 1, small), all(0, 2, small), all(2, 0, small), all(1, 2, small), all(2, 1, small);
   };
+  // The same for the f32 MFMA: 64 bytes of a row, the four chunks of which change places every four rows.
+  auto place_f32 = [](int row, int chunk) { return row * 64 + ((chunk ^ (row >> 2)) & 3) * 16; };
+  auto put_f32 = [&](auto second, const Values &v, uint8_t *stage) {
+#pragma unroll
+    for (int o = 0; o < OPERANDS; o++)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        *(v4f *)(stage + (is_b(second, o) ? BM * 64 : 0) + place_f32(row[o], 2 * half[o] + q)) = v4f{v.x[o][4 * q], v.x[o][4 * q + 1], v.x[o][4 * q + 2], v.x[o][4 * q + 3]};
+  };
+  struct OperandsF32 { v4f a[T][2], b[T][2]; };   // lane (l % 32, l / 32): eight k of a row, from 8 (l / 32) on, one to an MFMA
+  auto read_f32 = [&](const uint8_t *stage, OperandsF32 &f) {
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        f.a[t][q] = *(const v4f *)(stage + place_f32(32 * (wm * T + t) + li, 2 * lh + q));
+        f.b[t][q] = *(const v4f *)(stage + BM * 64 + place_f32(32 * (wn * T + t) + li, 2 * lh + q));
+      }
+  };
+  auto multiply_f32 = [&](const OperandsF32 &f) {
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+      for (int r = 0; r < T; r++)
+#pragma unroll
+        for (int c = 0; c < T; c++) big[r][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[r][i / 4][i % 4], f.b[c][i / 4][i % 4], big[r][c], 0, 0, 0);
+  };
   // All LDS reads and writes are done; loads stay under way.
   auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
-  // Step j, whose parts lie in `stage`, while step j + 1's are cut.
-  auto step = [&](Values &v, const uint8_t *stage, uint8_t *next_stage) {
-    Operands f;
-    read(stage, f);
-    put(v, next_stage);
-    load(v);
-    multiply(f);
-    __builtin_amdgcn_sched_group_barrier(0x100, 6 * T, 0);   // the reads, then an MFMA and some of the cutting in turn
+  // Step j, whose parts (or values) lie in `stage`, while step j + 1's are cut.
+  auto step = [&](auto f32, auto second, Values &v, const uint8_t *stage, uint8_t *next_stage) {
+    if constexpr (decltype(f32)::value) {
+      OperandsF32 f;
+      read_f32(stage, f);
+      put_f32(second, v, next_stage);
+      load(second, v);
+      multiply_f32(f);
+    } else {
+      Operands f;
+      read(stage, f);
+      put(v, next_stage);
+      load(second, v);
+      multiply(f);
+      __builtin_amdgcn_sched_group_barrier(0x100, 6 * T, 0);   // the reads, then an MFMA and some of the cutting in turn
 #pragma unroll
-    for (int i = 0; i < 8 * T * T; i++) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, T == 2 ? 4 : 8, 0);
+      for (int i = 0; i < 8 * T * T; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, T == 2 ? 4 : 8, 0);
+      }
     }
     barrier();
   };
-  {
-    Values v;
-    load(v);
-    load(kept[1]);
-    load(kept[0]);
-    if (group == 0)
+  // False where the parts may not do: a value of this size may make an infinite sum, and so be computed again.  Looked at when 8 steps, 16, 32 and so on are
+  // done, so that little is thrown away.  (Not so for rows of tiny values, which a row of probabilities is for most of its way.)
+  uint32_t *const given_up = (uint32_t *)(lds + G * S::GROUP);
+  auto pass_of = [&](auto f32, auto second) {
+    begin(second);
+    {
+      Values v;
+      load(second, v);
+      load(second, kept[1]);
+      load(second, kept[0]);
+      if (group == 0)
 #pragma unroll
-      for (int o = 0; o < OPERANDS; o++)
+        for (int o = 0; o < OPERANDS; o++)
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-          if (8 * half[o] + i >= head) v.x[o][i] = 0.0f;
-    put(v, stages);
-  }
-  barrier();
-  int j = 0;
-  for (; j + 2 < mine; j += 2) {
-    step(kept[1], stages, stages + S::STAGE);
-    step(kept[0], stages + S::STAGE, stages);
-  }
-  if (j + 1 < mine) step(kept[1], stages, stages + S::STAGE);
-  if ((mine - 1) * G + group < steps) {   // (behind K's end: nothing)
-    Operands f;
-    read(stages + ((mine - 1) & 1) * S::STAGE, f);
-    multiply(f);
-  }
-#pragma unroll
-  for (int r = 0; r < T; r++)
-#pragma unroll
-    for (int c = 0; c < T; c++) big[r][c] += small[r][c];
+          for (int i = 0; i < 8; i++)
+            if (8 * half[o] + i >= head) v.x[o][i] = 0.0f;
+      if constexpr (decltype(f32)::value) put_f32(second, v, stages);
+      else put(v, stages);
+    }
+    if (!decltype(f32)::value && threadIdx.x == 0) *given_up = 0;   // (never while others may be about to read it)
+    barrier();
+    int j = 0;
+    for (int look = decltype(f32)::value ? mine : 8;; look *= 2) {
+      for (; j + 2 < min(mine, look); j += 2) {
+        step(f32, second, kept[1], stages, stages + S::STAGE);
+        step(f32, second, kept[0], stages + S::STAGE, stages);
+      }
+      if (j + 2 >= mine) break;
+      // (read before the next step's barrier, and written again many steps later)
+      if (seen.most > 0x1p100f) *given_up = 1;
+      barrier();
+      if (__builtin_amdgcn_readfirstlane(*given_up)) return false;
+    }
+    if (j + 1 < mine) step(f32, second, kept[1], stages, stages + S::STAGE);
+    if ((mine - 1) * G + group < steps) {   // (behind K's end: nothing)
+      const uint8_t *stage = stages + ((mine - 1) & 1) * S::STAGE;
+      if constexpr (decltype(f32)::value) {
+        OperandsF32 f;
+        read_f32(stage, f);
+        multiply_f32(f);
+      } else {
+        Operands f;
+        read(stage, f);
+        multiply(f);
+      }
+    }
+    return true;
+  };
+  auto pass = [&](auto f32) { return second ? pass_of(f32, std::true_type{}) : pass_of(f32, std::false_type{}); };
 
   const int64_t row0 = m0 + wm * 32 * T, col0 = n0 + wn * 32 * T;
   float sum[T * T * 16 / G];
-  meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
-  if (!parts_did(seen, sum, p.k, (uint32_t *)lds)) {
-    multiply_f32<T, G, B_KMAJOR>(p, row0, col0, group, big);
+  bool did = pass(std::false_type{});
+  if (did) {
+#pragma unroll
+    for (int r = 0; r < T; r++)
+#pragma unroll
+      for (int c = 0; c < T; c++) big[r][c] += small[r][c];
+    meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
+    did = parts_did(seen, sum, p.k, (uint32_t *)lds);
+  }
+  if (!did) {
+#pragma unroll
+    for (int r = 0; r < T; r++)
+#pragma unroll
+      for (int c = 0; c < T; c++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) big[r][c][i] = 0.0f;
+    pass(std::true_type{});
     meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
   }
   store<T, G>(p, row0, col0, group, g.accum, g.ldc, sum);
@@ -352,10 +400,8 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
   const int64_t m0 = int64_t(tile_m) * 32, n0 = int64_t(tile_n) * 32;
   const Problem p(g);
   const int steps = (p.k + K - 1) / K, head = p.k - K * (steps - 1);
-  int next = min(wave, steps - 1);   // the step that the operands are at
-  const int k0 = next == 0 ? 0 : head + K * (next - 1);
-  const uint8_t *a = p.a + m0 * p.lda_b + int64_t(k0) * 4;
-  const uint8_t *b = B_KMAJOR ? p.b + n0 * p.ldb_b + int64_t(k0) * 4 : p.b + n0 * 4 + int64_t(k0) * p.ldb_b;
+  int next;   // the step that the operands are at
+  const uint8_t *a, *b;
   // Lane (l % 32, l / 32): 16 k, from 16 (l / 32) on, of row and column l % 32; eight of them to an MFMA.
   const uint32_t a_off = uint32_t(min(li, int(p.m - m0) - 1)) * p.lda_b + lh * 64, col = uint32_t(min(li, int(p.n - n0) - 1));
   const uint32_t b_off = B_KMAJOR ? col * p.ldb_b + lh * 64 : col * 4 + uint32_t(lh) * 16 * p.ldb_b;
@@ -398,7 +444,11 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
     small = mfma(x.l, y.m, small);
   };
   const int mine = steps > wave ? (steps - wave + DEAL - 1) / DEAL : 0;
-  if (mine > 0) {
+  auto pass = [&](auto f32) {
+    next = min(wave, steps - 1);
+    const int k0 = next == 0 ? 0 : head + K * (next - 1);
+    a = p.a + m0 * p.lda_b + int64_t(k0) * 4;
+    b = B_KMAJOR ? p.b + n0 * p.ldb_b + int64_t(k0) * 4 : p.b + n0 * 4 + int64_t(k0) * p.ldb_b;
     ring::each<D>([&](auto d) { load(kept[decltype(d)::value]); });
     if (wave == 0)
 #pragma unroll
@@ -409,21 +459,30 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
       ring::each<D>([&](auto d) {
         Values &v = kept[decltype(d)::value];
         if (!done) {
-          const Parts a0 = cut(v.a, seen), b0 = cut(v.b, seen);
-          multiply(a0, b0);
-          const Parts a1 = cut(v.a + 8, seen), b1 = cut(v.b + 8, seen);
-          load(v);
-          multiply(a1, b1);
+          if constexpr (decltype(f32)::value) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) big[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(v.a[i], v.b[i], big[0][0], 0, 0, 0);
+            load(v);
+          } else {
+            const Parts a0 = cut(v.a, seen), b0 = cut(v.b, seen);
+            multiply(a0, b0);
+            const Parts a1 = cut(v.a + 8, seen), b1 = cut(v.b + 8, seen);
+            load(v);
+            multiply(a1, b1);
+          }
           done = --left == 0;
         }
       });
     }
-  }
+  };
+  if (mine > 0) pass(std::false_type{});
   big[0][0] += small;
   float sum[16 / DEAL];
   meet<1, DEAL>(part, 1024, 0, wave, big, sum);
   if (!parts_did(seen, sum, p.k, (uint32_t *)part)) {
-    multiply_f32<1, DEAL, B_KMAJOR>(p, m0, n0, wave, big);
+#pragma unroll
+    for (int i = 0; i < 16; i++) big[0][0][i] = 0.0f;
+    if (mine > 0) pass(std::true_type{});
     meet<1, DEAL>(part, 1024, 0, wave, big, sum);
   }
   store<1, DEAL>(p, m0, n0, wave, g.accum, g.ldc, sum);
@@ -439,7 +498,7 @@ void declare_work(const GemmArgs &g, int side, int k_step, double serial_ns) {
 template <int T, int G, bool B_KMAJOR>
 hipError_t launch_staged(const GemmArgs &g, hipStream_t stream) {
   typedef Staged<T, G> S;
-  constexpr int BM = S::BM, LDS = G * S::GROUP;
+  constexpr int BM = S::BM, LDS = G * S::GROUP + 16;
   static std::atomic<uint64_t> lds_limit_set{0};
   if (!plan::recording() && LDS > 65536) {
     hipError_t e = raise_lds_limit(lds_limit_set, (const void *)k_gemm_f32<T, G, B_KMAJOR>, LDS);

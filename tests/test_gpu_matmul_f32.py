@@ -181,3 +181,26 @@ def test_f32_one_term_of_any_size_beside_zeros(gpu, m, k, n, lo_a, hi_a, lo_b, h
     got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk)[0].astype(np.float64)
     want = values[:, None].astype(np.float64) * B[0, at].astype(np.float64)
     assert (np.abs(got - want) <= (1 + 2.0 ** -4) * 2.0 ** -24 * np.abs(want) + np.where(np.abs(want) < 2.0 ** -120, 2.0 ** -149, 0)).all()
+
+
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("where", ["early", "late", "last"])
+@pytest.mark.parametrize("m,k,n", [(511, 513, 261), (2477, 129, 257), (1740, 1751, 1637), (2071, 389, 3129), (537, 1667, 569)])
+def test_f32_values_that_make_infinite_sums(gpu, m, k, n, where, nk):
+    """The lowest value once in every third row, met at the start of K, behind its middle or at its end: sums as f32 has them, in the tiles that
+    give up on the way and in those that find an infinite one in the end."""
+    A, B = synth.normal_f32(199, 0, (1, m, k)), synth.normal_f32(199, 1, (1, k, n))
+    rows = np.arange(0, m, 3)
+    at = {"early": rows % 11, "late": k // 2 + rows % (k // 2), "last": np.full(rows.size, k - 1)}[where]
+    A[0, rows, at] = -3.4e38
+    spec = _spec(1, m, k, n, nk)
+    assert spec.plan().kernels[0].startswith("k_gemm_f32")
+    got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk)[0].astype(np.float64)
+    a64, b64 = A[0].astype(np.float64), B[0].astype(np.float64)
+    want, scale = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    largest = float(np.finfo(np.float32).max)
+    sure = np.abs(np.abs(want) - largest) > 1e-5 * largest
+    infinite = sure & (np.abs(want) > largest)
+    assert infinite.any() and (got[infinite] == np.sign(want[infinite]) * np.inf).all()
+    finite = sure & (np.abs(want) < largest)
+    assert (np.abs(got - want)[finite] <= (k + 4) * 2.0 ** -24 * scale[finite]).all()
