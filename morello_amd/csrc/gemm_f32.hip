@@ -536,52 +536,65 @@ uint32_t gemm_f32_slice_k(uint32_t k, uint32_t want) {
   return slice_k;
 }
 
-// Workgroups of a form go to the compute units in rounds, each as long as a workgroup's steps.  Measured, on operands of 1 to 50 MB: a step of 4 x 32 k of a block of 32 x 32 0.75 us of its unit, however many share it; of 2 x 16 k of 64 x 64
-// 0.5; of 2 x 16 k of 128 x 128 1.05 to, on all units, 1.47; of 16 k of two such workgroups 1.35, of one 0.85.  Slices of K cost the launch that sums them, 2.5 us, and
-// their results at 3 TB/s.  (us, the f32 MFMA on copies of whole chunks / this, form and slices: 195 x 500 x 621 17.0 / 7.4, waves;
+// Workgroups of a form go to the compute units in rounds, each as long as a workgroup's steps.  Measured on operands of 1 to 50 MB, B row-major / k-fastest: a
+// step of 4 x 32 k of a block of 32 x 32 0.8 / 0.87 us of its unit, however many share it (lines per load, not bytes: the second touches 64 of them), of 2 x 16 k of
+// 64 x 64 0.49 / 0.455, of 2 x 16 k of 128 x 128 1.14 / 1.07 to, on all units, 0.4 more; of 16 k of two such workgroups 1.5, of one 0.82; and what a round costs beside its steps.
+// Slices of K cost the launch that sums them and their results at 3.1 TB/s.  (us, the f32 MFMA on copies of whole chunks / this, form and slices: 195 x 500 x 621 17.1 / 7.4, waves;
 // 192 x 2176 x 128 16.4 / 8.8, waves in 8; twice 382 x 226 x 1179 14.2 / 9.3, 64 wide; 537 x 1668 x 568 23.1 / 17.8, 64 wide in 3; 2048^3 153
-// / 121, 128 wide in two groups; 2070 x 389 x 3128 57.7 / 47.6, 128 wide in one; 4096^3 959 / 838.)
+// / 122, 128 wide in two groups; 2070 x 389 x 3128 57.7 / 48.6, 128 wide in one; 4096^3 959 / 880.  Over 3100 random sizes 1.35 times as fast, the form chosen within 1.3 % of
+// the fastest, geometric means.)
 namespace {
 enum Form : uint32_t { NONE, WAVES, WIDE_64, WIDE_128, WIDE_128_PAIR };
 struct Choice {
   Form form;
   uint32_t slices, slice_k;
+  double us;
 };
 Choice choose(const GemmArgs &g) {
   const double units = g_compute_units;
+  const bool nk = g.b_kmajor;
   auto tiles = [&](uint32_t side) { return double((g.m + side - 1) / side) * ((g.n + side - 1) / side) * g.batch; };
   const double t32 = tiles(32), t64 = tiles(64), t128 = tiles(128);
   auto rounds = [&](double n, double at_once) { return double(uint64_t((n + at_once - 1) / at_once)); };
-  Choice best{NONE, 1, g.k};
-  double least = 1e300;
+  Choice best{NONE, 1, g.k, 1e300};
   auto consider = [&](Form form, uint32_t slices, uint32_t slice_k, double us) {
-    if (us < least) least = us, best = {form, slices, slice_k};
+    if (us < best.us) best = {form, slices, slice_k, us};
   };
-  const uint32_t steps = (g.k + 15) / 16;
-  consider(WIDE_128, 1, g.k, 5.0 + std::max(1.05, 0.75 + 0.72 * std::min(1.0, t128 / units)) * rounds(t128, units) * ((steps + 1) / 2));
-  consider(WIDE_128_PAIR, 1, g.k, 5.0 + (t128 <= units ? 0.85 : 1.35 * rounds(t128, 2 * units)) * steps);
+  const double steps = (g.k + 15) / 16, pairs = (g.k + 31) / 32, r128 = rounds(t128, units), r_pair = rounds(t128, 2 * units);
+  consider(WIDE_128, 1, g.k, 7.0 + 5.0 * (r128 - 1) + ((nk ? 1.07 : 1.14) + 0.4 * std::min(1.0, t128 / units)) * r128 * pairs);
+  consider(WIDE_128_PAIR, 1, g.k, 7.0 + (t128 <= units ? 0.82 * steps : (1.5 * steps + 3.0) * r_pair));
+  // (k-fastest rows 512 bytes or a multiple of that apart share the sets of the first cache)
+  const double between = nk && g.k % 128 == 0 ? 1.5 : 0.9;
   for (uint32_t want : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u}) {
     const uint32_t slice_k = want == 1 ? g.k : gemm_f32_slice_k(g.k, want);
     if (want > 1 && (g.batch != 1 || g.tight || slice_k == 0)) break;
     if (want > 1 && slice_k >= g.k) continue;
-    const uint32_t slices = (g.k + slice_k - 1) / slice_k;
-    const double sum = slices == 1 ? 0.0 : 2.5 + (slices + 1.0) * g.m * g.n * 4.0 / 3e6;
-    const uint32_t s16 = (slice_k + 15) / 16, s32 = (slice_k + 31) / 32;
-    if (g.k >= 32) consider(WAVES, slices, slice_k, 4.0 + 0.75 * rounds(t32 * slices, units) * ((s32 + DEAL - 1) / DEAL) + sum);
-    consider(WIDE_64, slices, slice_k, 3.8 + 0.5 * rounds(t64 * slices, units) * ((s16 + 1) / 2) + sum);
+    const uint32_t slices = (g.k + slice_k - 1) / slice_k, s32 = (slice_k + 31) / 32;
+    const double sum = slices == 1 ? 0.0 : 2.6 + slices * (0.03 + double(g.m) * g.n * 4.0 / 3.1e6);
+    const double r32 = rounds(t32 * slices, units), r64 = rounds(t64 * slices, units);
+    if (g.k >= 32) consider(WAVES, slices, slice_k, 3.85 + between * (r32 - 1) + (nk ? 0.87 : 0.8) * r32 * ((s32 + DEAL - 1) / DEAL) + sum);
+    consider(WIDE_64, slices, slice_k, 4.4 + 1.2 * (r64 - 1) + (nk ? 0.455 : 0.49) * r64 * s32 + sum);
   }
   return best;
 }
+// k_gemm's 64 x 64 tiles with the f32 MFMA, on rows of whole chunks.
+double k_gemm_us(const GemmArgs &g) {
+  const double a_unit = double((g.m + 63) / 64) * ((g.n + 63) / 64) * g.batch / g_compute_units, steps = (g.k + 31) / 32;
+  return a_unit <= 1 ? 3.4 + 0.68 * steps : a_unit <= 2 ? 4.2 + 1.18 * steps : 5.5 + (0.35 + 0.5 * a_unit) * steps;
+}
 }  // namespace
 
-// Any rows of f32, from a step of K on.  Whole chunks over a short K, whose start and end are most of the time, stay with k_gemm
-// (1472 x 128 x 1472 10.5 us, here 12.1; 832 x 192 x 1088 7.2 and 7.1).
+// Any rows of f32, from a step of K on.  Whole chunks over a short K, whose start and end are most of the time, stay with k_gemm (640 x 128 x 1632 8.0 us, here
+// 8.9, 288 x 128 x 1696 5.6 and 6.3; of a few tiles 160 k and more would gain, 256 x 168 x 768 6.7 and 5.2), and so do those whose tiles its smaller rounds suit better (1472 x
+// 256 x 1472 16.8, here 18.8, 2304 x 224 x 2048 25.4 and 27.3, 2 x 576 x 320 x 2176 19.8 and 21.9).
 bool gemm_f32_applicable(const GemmArgs &g, int kind) {
   auto words = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 4 == 0; };
   if (kind != 3 || g.k < 16 || !gemm::edge_addressable(g, 4) || g.batch > 65535 || !words(g.a) || !words(g.b) || !words(g.c)) return false;
+  if (!gemm_pays(g, kind) || gemv_applicable(g, kind)) return false;
   const bool chunks = g.lda % 4 == 0 && g.ldb % 4 == 0 && g.sa % 4 == 0 && g.sb % 4 == 0 &&
                       reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && reinterpret_cast<uintptr_t>(g.b) % 16 == 0;
-  return !(chunks && g.k <= 192) && gemm_pays(g, kind) && !gemv_applicable(g, kind);
+  uint32_t left = 0;
+  return !chunks || (g.k > 192 && (gemm_tile_side(g, kind) != 64 || gemm_k_splits(g, kind, &left) != 1 || k_gemm_us(g) >= 1.05 * choose(g).us));
 }
 
 uint32_t gemm_f32_slices(const GemmArgs &g, uint32_t *slice_k) {

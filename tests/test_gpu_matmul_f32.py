@@ -111,7 +111,7 @@ def test_f32_slices_that_nearly_divide_k(gpu, m, k, n, nk):
     assert np.linalg.norm(got - want) <= 4e-7 * np.linalg.norm(want)
 
 
-@pytest.mark.parametrize("m,k,n,nk,last", [(500, 95, 500, True, 95), (511, 65, 261, True, 65), (300, 47, 301, True, 47), (300, 33, 301, True, 33), (160, 675, 197, False, 35), (150, 816, 420, True, 48)])
+@pytest.mark.parametrize("m,k,n,nk,last", [(500, 95, 500, True, 95), (511, 65, 261, True, 65), (300, 47, 301, True, 47), (300, 33, 301, True, 33), (160, 675, 197, False, 35), (157, 689, 194, True, 49)])
 def test_f32_tiny_rows_over_fewer_steps_than_waves(gpu, m, k, n, nk, last):
     """A row and a column of nothing but tiny values where some of a tile's waves have no step of K, or of its last slice."""
     A, B = np.abs(synth.normal_f32(195, 0, (1, m, k))), np.abs(synth.normal_f32(195, 1, (1, k, n))) + np.float32(0.01)
