@@ -5,8 +5,9 @@
 //   x y = h h' + (h m' + m h') + (m m' + h l' + l h') + (m l' + l m') + l l', the last at most 2^-32 |x y| and left out:
 // eight MFMAs for sixteen k where the f32 form takes eight of twice the time each.  The products but the first are summed on
 // their own, 2^-6 of the first and less, so that a sum of one term is rounded as once (within 2^-24 and a sixteenth of that; without m l' + l m', 3 to 18 % faster, 2^-22).
-// The roundings of a longer sum, one to sixteen terms and not to two, come to less than those of the f32 MFMA: relative
-// error in the norm for 0.5 x normal operands, f32 MFMA / this: K = 226 2.7e-7 / 6.7e-8, 1024 5.7e-7 / 1.3e-7, 1500 6.9e-7 / 1.6e-7.
+// Waves that share K add up their first products and their others apart, so that a sum of some terms is rounded at its size about as often (1 to 2 % of the time).
+// The roundings of a longer sum, one to sixteen terms and not to two, come to less than those of the f32 MFMA: relative error in the norm for 0.5 x normal
+// operands, f32 MFMA / this: two values a row 3.1e-8 / 2.6e-8, four 4.0e-8 / 2.6e-8, 16 7.4e-8 / 3.3e-8, K = 226 2.7e-7 / 6.7e-8, 1024 5.7e-7 / 1.3e-7, 1500 6.9e-7 / 1.6e-7.
 // (The three parts: G. Henry, P. Tang and A. Heinecke, Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations, 2019.)
 //
 // Where the parts would not do, the tile is computed again by the f32 MFMA:
@@ -19,8 +20,9 @@
 // 2^-119, beside them the f32 MFMA's own kernel: 2048^3 118 / 159 / 150 / 241, 140; 1000^3 22 / 39 / 26 / 39, 25; 512^3 6.8 / 11.3 / 11.3 / 11.3, 11.5.  From memory without staging, and with
 // all values past 2^60 counted among these: 2048^3 328, with a k-fastest B 534, 1000^3 126, 512^3 18.)
 //
-// What bounds it: the bf16 MFMAs at what the board's power lets them run at (4096^3 in 838 us is 1.31 PFLOP/s of them, where the 256 tile
-// reaches 1.42), for the smaller tiles the cutting, six and a half vector instructions a value; below a round of tiles the chain of a step.
+// What bounds it: of large ones the bf16 MFMAs at what the board's power lets them run at (4096^3 in 848 us is 1.30 PFLOP/s of them, the matrix cores busy 72 % of the
+// cycles, where bf16 operands reach 1.42); 64-wide tiles as much by the cutting, six and a half vector instructions a value (37 and 41 % of the cycles, a third in waits); blocks of
+// 32 x 32 by the chain of a step (14 and 31 %).
 //
 // Rows start on any element and are read in place.  The first step takes what K has over whole steps, zeros behind it, so that no
 // load but its leaves K and none is masked; rows past M and columns past N are the last one again and are not stored.
@@ -367,11 +369,11 @@ __global__ __launch_bounds__(256 * G, T == 2 ? 2 : 4) void k_gemm_f32(MRL_WALK_P
   float sum[T * T * 16 / G];
   bool did = pass(std::false_type{});
   if (did) {
-#pragma unroll
-    for (int r = 0; r < T; r++)
-#pragma unroll
-      for (int c = 0; c < T; c++) big[r][c] += small[r][c];
+    float rest[T * T * 16 / G];
     meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, big, sum);
+    meet<T, G>((float *)lds, S::GROUP / 4, wave & 3, group, small, rest);
+#pragma unroll
+    for (int e = 0; e < T * T * 16 / G; e++) sum[e] += rest[e];
     did = parts_did(seen, sum, p.k, (uint32_t *)lds);
   }
   if (!did) {
@@ -430,18 +432,18 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
     next += ahead ? DEAL : 0;
   };
   Seen seen;
-  v16f big[1][1], small;
+  v16f big[1][1], small[1][1];
 #pragma unroll
-  for (int i = 0; i < 16; i++) big[0][0][i] = small[i] = 0.0f;
+  for (int i = 0; i < 16; i++) big[0][0][i] = small[0][0][i] = 0.0f;
   auto multiply = [&](const Parts &x, const Parts &y) {
-    small = mfma(x.h, y.m, small);
+    small[0][0] = mfma(x.h, y.m, small[0][0]);
     big[0][0] = mfma(x.h, y.h, big[0][0]);
-    small = mfma(x.m, y.h, small);
-    small = mfma(x.m, y.m, small);
-    small = mfma(x.h, y.l, small);
-    small = mfma(x.l, y.h, small);
-    small = mfma(x.m, y.l, small);
-    small = mfma(x.l, y.m, small);
+    small[0][0] = mfma(x.m, y.h, small[0][0]);
+    small[0][0] = mfma(x.m, y.m, small[0][0]);
+    small[0][0] = mfma(x.h, y.l, small[0][0]);
+    small[0][0] = mfma(x.l, y.h, small[0][0]);
+    small[0][0] = mfma(x.m, y.l, small[0][0]);
+    small[0][0] = mfma(x.l, y.m, small[0][0]);
   };
   const int mine = steps > wave ? (steps - wave + DEAL - 1) / DEAL : 0;
   auto pass = [&](auto f32) {
@@ -476,9 +478,11 @@ __global__ __launch_bounds__(64 * DEAL, 2) void k_gemm_f32_waves(MRL_WALK_PARAMS
     }
   };
   if (mine > 0) pass(std::false_type{});
-  big[0][0] += small;
-  float sum[16 / DEAL];
+  float sum[16 / DEAL], rest[16 / DEAL];
   meet<1, DEAL>(part, 1024, 0, wave, big, sum);
+  meet<1, DEAL>(part, 1024, 0, wave, small, rest);
+#pragma unroll
+  for (int e = 0; e < 16 / DEAL; e++) sum[e] += rest[e];
   if (!parts_did(seen, sum, p.k, (uint32_t *)part)) {
 #pragma unroll
     for (int i = 0; i < 16; i++) big[0][0][i] = 0.0f;

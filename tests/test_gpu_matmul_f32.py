@@ -204,3 +204,19 @@ def test_f32_values_that_make_infinite_sums(gpu, m, k, n, where, nk):
     assert infinite.any() and (got[infinite] == np.sign(want[infinite]) * np.inf).all()
     finite = sure & (np.abs(want) < largest)
     assert (np.abs(got - want)[finite] <= (k + 4) * 2.0 ** -24 * scale[finite]).all()
+
+
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("m,k,n", [(511, 513, 261), (2477, 129, 257), (1740, 751, 1637), (2071, 389, 3129)])   # (slices of K round each part of a sum once more, as those of the other kernels do)
+def test_f32_sums_of_two_terms(gpu, m, k, n, nk):
+    """Two values a row, wherever in K: below 2.9e-8 in the norm, where one rounding of each sum comes to 2.5e-8 (2^-24 over the square root of three, times what a
+    significand's distribution makes of it), the f32 MFMA's two to 3.1e-8, and a rounding for every wave that has one of the terms to 3.4e-8."""
+    A, B = np.zeros((1, m, k), np.float32), synth.normal_f32(201, 1, (1, k, n))
+    rows, first = np.arange(m), np.arange(m) * 13 % k
+    A[0, rows, first] = synth.normal_f32(201, 2, (m,))
+    A[0, rows, (first + 1 + np.arange(m) * 29 % (k - 1)) % k] = synth.normal_f32(201, 3, (m,))
+    spec = _spec(1, m, k, n, nk)
+    assert len(spec.plan().kernels) == 1 and spec.plan().kernels[0].startswith("k_gemm_f32")
+    got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk).astype(np.float64)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    assert np.linalg.norm(got - want) <= 2.9e-8 * np.linalg.norm(want)
