@@ -220,3 +220,16 @@ def test_f32_sums_of_two_terms(gpu, m, k, n, nk):
     got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk).astype(np.float64)
     want = A.astype(np.float64) @ B.astype(np.float64)
     assert np.linalg.norm(got - want) <= 2.9e-8 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("nk", [False, True])
+@pytest.mark.parametrize("m,n", [(2477, 657), (2471, 1257), (3477, 3257)])
+@pytest.mark.parametrize("k", [17, 18, 31, 33, 47, 49])
+def test_f32_matmul_over_the_fewest_steps(gpu, m, k, n, nk):
+    """One to four steps of 16 k on one or two groups of waves, the first of one to sixteen."""
+    spec = _spec(1, m, k, n, nk)
+    assert spec.plan().kernels == ["k_gemm_f32"]
+    A, B = synth.normal_f32(202, 0, (1, m, k)), synth.normal_f32(202, 1, (1, k, n))
+    got = _run(spec, A, B, np.zeros((1, m, n), np.float32), nk).astype(np.float64)
+    a64, b64 = A.astype(np.float64), B.astype(np.float64)
+    assert (np.abs(got - a64 @ b64) <= (k + 4) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64))).all()
