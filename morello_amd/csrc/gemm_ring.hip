@@ -12,7 +12,12 @@
 //   - eight waves: four blocks of 64 x BN / 2 outputs, each once for the first and once for the second 64 bytes of
 //     every step, whose sums meet in LDS at the end: two waves on a SIMD, one issuing while the other's MFMAs
 //     run, and an operand read still serves BN / 32 or four MFMAs;
-//   - widths chosen so that the tiles fill one round (gemm_ring_columns).
+//   - widths chosen so that the tiles fill one round (gemm_ring_columns);
+//   - nothing but the barrier between a step's last MFMA and the next one's first: what the next step's reads and requests start from
+//     is worked out behind the MFMAs of the step before.  (Some 35 scalar instructions in one go behind the last MFMA, while both waves of a SIMD had
+//     none under way: bf16 2048^3 22.0 us, now 21.0, u8 1472 x 2304 x 2752 21.0 / 19.2, 1546 x 5000 x 2560 41.3 / 37.8.)
+// What bounds the loop now is the way into LDS: a step of the 128 x 128 tile takes 0.36 us, its loads by themselves 0.31 (105 bytes a
+// nanosecond and unit), its MFMAs 0.21.
 // The loads are buffer loads: rows past M or N and chunks past K come as zeros, without a branch.
 //
 // LDS: A as [row][128 bytes], 16-byte chunks XOR-ed with (row / 2) & 7; a k-fastest B likewise; a
@@ -27,6 +32,8 @@ namespace {
 using namespace ring;
 using gemm::TileWalk;
 typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) const uint8_t lds_u8;
+typedef __attribute__((address_space(3))) const v4i lds_v4i;
 
 constexpr uint32_t OUTSIDE = 0x80000000u;   // an offset no resource here holds
 constexpr int BM = 128;
@@ -37,16 +44,19 @@ constexpr int BM = 128;
 // the same statement, with the wait state it needs: the compiler sets that reserved register right before its own
 // uses and keeps nothing in it, and may do so between any two statements.
 template <int AT>
-__device__ inline void dma16(__amdgpu_buffer_rsrc_t from, uint32_t off, uint32_t lds_addr) {
+__device__ inline void dma16(v4i from, uint32_t off, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen offset:%3 lds" : : "v"(off), "s"(from), "s"(lds_addr), "n"(AT) : "memory");
 }
-__device__ inline __amdgpu_buffer_rsrc_t resource(const void *base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, int(bytes), 0x00020000);
-}
+// (of addresses below 2^48, as all are: the bits above belong to the stride)
+__device__ inline v4i resource(uint64_t base, uint32_t bytes) { return v4i{int(uint32_t(base)), int(uint32_t(base >> 32)), int(bytes), 0x00020000}; }
 // All but the newest N loads have landed, and every LDS read is done.
+// (A builtin wait, which the compiler sees: it adds none of its own for the operands that are in.)
 template <int N>
 __device__ inline void wait_for_all_but() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
+  asm volatile("" : : : "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 7 << 4);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" : : : "memory");
 }
 
 template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RB, int SLOTS>
@@ -92,40 +102,44 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
   for (int i = 0; i < A_LOADS; i++) a_off[i] += 4096 - i * 1024;
 #pragma unroll
   for (int i = 0; i < B_LOADS; i++) b_off[i] += 4096;
-  const uint8_t *a_tile = A - 4096, *b_tile = B - 4096;
+  // Where the step to request starts: the resources' bases.  Their sizes do not change from step to step (an offset past them is a
+  // row's that does not exist), but for the steps that hold K's end and lie behind it.
+  uint64_t a_tile = reinterpret_cast<uintptr_t>(A) - 4096, b_tile = reinterpret_cast<uintptr_t>(B) - 4096;
+  uint32_t a_bytes = uint32_t(a_end) + 4096, b_bytes = (B_KMAJOR ? b_end : uint32_t(BK) * ldb_b - n0_b) + 4096;
   int left = k_bytes;   // of K from the step to request on
-  uint32_t a_dst = lds0 + wave * (A_LOADS * 1024), b_dst = lds0 + A_BYTES;
-  const uint32_t a_dst_end = a_dst + SLOTS * SLOT;
-  __amdgpu_buffer_rsrc_t a_buf, b_buf;
-  const int64_t b_step = B_KMAJOR ? int64_t(STEP) : int64_t(BK) * ldb_b;
-  // The resources of the step to request, and its offsets: chunks past K, in the step that holds K's end,
-  // become ones outside (the steps behind it are empty, so for good).
-  auto prepare = [&]() {
-    const bool some = left > 0;
-    a_buf = resource(a_tile, some ? uint32_t(a_end - (k_bytes - left) + 4096) : 0u);
-    const uint32_t b_bytes = B_KMAJOR ? b_end - uint32_t(k_bytes - left) : uint32_t(min(left / ES, BK)) * ldb_b - n0_b;
-    b_buf = resource(b_tile, some ? b_bytes + 4096 : 0u);
-    if (some && left < STEP) {
-#pragma unroll
-      for (int i = 0; i < A_LOADS; i++)
-        if ((chunk ^ ((wave * A_LOADS + i) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16 >= left) a_off[i] = OUTSIDE;
-      if constexpr (B_KMAJOR)
-#pragma unroll
-        for (int i = 0; i < B_LOADS; i++)
-          if ((chunk ^ ((b_load(i)) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16 >= left) b_off[i] = OUTSIDE;
+  const uint32_t a_dst = lds0 + wave * (A_LOADS * 1024), b_dst = lds0 + A_BYTES;
+  uint32_t fill = 0;   // the slot that it goes to
+  const uint64_t b_step = B_KMAJOR ? uint64_t(STEP) : uint64_t(BK) * ldb_b;
+  // Of the step that holds K's end, chunks past it become ones outside (the steps behind it are empty, so for good).
+  auto end_of_k = [&]() __attribute__((always_inline)) {
+    if (left <= 0) {
+      a_bytes = b_bytes = 0;
+      return;
     }
+    if constexpr (!B_KMAJOR) b_bytes = uint32_t(left / ES) * ldb_b - n0_b + 4096;
+    each<A_LOADS>([&](auto i) { a_off[i] = (chunk ^ ((wave * A_LOADS + i) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16 >= left ? OUTSIDE : a_off[i]; });
+    if constexpr (B_KMAJOR) each<B_LOADS>([&](auto i) { b_off[i] = (chunk ^ (b_load(i) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16 >= left ? OUTSIDE : b_off[i]; });
   };
   // Its i-th load of this wave.
   auto load = [&](auto which) {
     constexpr int I = decltype(which)::value;
-    if constexpr (I < A_LOADS) dma16<I * 1024>(a_buf, a_off[I], a_dst);
-    else dma16<0>(b_buf, b_off[I - A_LOADS], b_dst + b_load(I - A_LOADS) * 1024);
+    if constexpr (I < A_LOADS) dma16<I * 1024>(resource(a_tile, a_bytes), a_off[I], fill + a_dst);
+    else dma16<0>(resource(b_tile, b_bytes), b_off[I - A_LOADS], fill + (b_dst + b_load(I - A_LOADS) * 1024));
   };
-  auto advance = [&]() {
-    left -= STEP;
-    a_tile += STEP, b_tile += b_step;
-    a_dst += SLOT, b_dst += SLOT;
-    if (a_dst == a_dst_end) a_dst -= SLOTS * SLOT, b_dst -= SLOTS * SLOT;
+  auto next_slot = [&](uint32_t at) { return at + SLOT == SLOTS * SLOT ? 0u : at + SLOT; };
+  // To the next step, in three parts.
+  auto advance = [&](auto part) {
+    constexpr int P = decltype(part)::value;
+    if constexpr (P == 0) {
+      a_tile += STEP, left -= STEP;
+      asm("" : "+s"(a_tile));   // (one sum a step, not an induction of the compiler's and three)
+    }
+    if constexpr (P == 1) {
+      b_tile += b_step;
+      asm("" : "+s"(b_tile));
+    }
+    if constexpr (P == 2)
+      if (left < STEP) end_of_k();
   };
 
   // Operand addresses within a slot: lane (l % 16, l / 16) takes the l / 16-th 16 bytes of row l % 16.
@@ -138,15 +152,24 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
     for (int c = 0; c < RB; c++) b_rd[c] = A_BYTES + r * (BN * ES) + swizzle<T, BN>((wn * WN + c * 16) * ES + 8 * (li % LANES_PER_ROW), r);
   }
   v4i af[2][RA], bf[2][RB];
-  int at_slot = 0;
-  const uint8_t *slot = lds;   // the one that operands are read from
+  // The addresses of a step's operands, in the slot `from`.
+  const int a_rd = wm * WM * STEP + in_rows;
+  constexpr int B_ADDRESSES = B_KMAJOR ? 1 : RB;
+  if constexpr (B_KMAJOR) b_rd[0] = A_BYTES + wn * WN * STEP + in_rows;
+  uint32_t a_at, b_at[B_ADDRESSES];
+  auto locate = [&](uint32_t from, auto which) {
+    constexpr int I = decltype(which)::value;
+    uint32_t &at = I == 0 ? a_at : b_at[I == 0 ? 0 : I - 1];
+    at = lds0 + from + (I == 0 ? a_rd : b_rd[I == 0 ? 0 : I - 1]);
+    asm("" : "+v"(at));   // here, and not behind the barrier
+  };
   // The i-th operand read of 64 bytes of K (RA of A, then RB of B).
   auto read = [&](auto set, auto which) {
     constexpr int S = decltype(set)::value, I = decltype(which)::value;
-    if constexpr (I < RA) af[S][I] = *(const v4i *)(slot + wm * WM * STEP + in_rows + I * 16 * STEP);
-    else if constexpr (B_KMAJOR) bf[S][I - RA] = *(const v4i *)(slot + A_BYTES + wn * WN * STEP + in_rows + (I - RA) * 16 * STEP);
+    if constexpr (I < RA) af[S][I] = *(lds_v4i *)uintptr_t(a_at + I * 16 * STEP);
+    else if constexpr (B_KMAJOR) bf[S][I - RA] = *(lds_v4i *)uintptr_t(b_at[0] + (I - RA) * 16 * STEP);
     else {
-      const uint8_t *at = slot + b_rd[I - RA];
+      const uint8_t *at = (const uint8_t *)(lds_u8 *)uintptr_t(b_at[I - RA]);
       const v2i lo = T::read_tr(at), hi = T::read_tr(at + T::K_PER_READ * (BN * ES));
       bf[S][I - RA] = v4i{lo[0], lo[1], hi[0], hi[1]};
     }
@@ -170,32 +193,40 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
   std::integral_constant<int, 0> even;
   std::integral_constant<int, 1> odd;
   // One MFMA after the other with a read or a load, if there are any to issue, behind it: what a wave
-  // issues in one go its MFMAs wait for.
+  // issues in one go its MFMAs wait for.  The last quarter has what the next step's reads and requests start from, so that no
+  // arithmetic stands between the barrier and the first of either.
   auto step = [&](auto multiplied, auto fetched) {
     wait_for_all_but<(SLOTS - 2) * LOADS>();
-    at_slot = at_slot + 1 == SLOTS ? 0 : at_slot + 1;
-    slot = lds + at_slot * SLOT;
     each<RA * RB>([&](auto q) {
-      constexpr int Q = decltype(q)::value, N = RA * RB, READS = RA + RB;
+      constexpr int Q = decltype(q)::value, N = RA * RB, READS = RA + RB, AHEAD = 3 + 1 + B_ADDRESSES;
       multiply(multiplied, q);
       constexpr int R0 = min_of(READS, (Q * READS * 4 + N * 3 - 1) / (N * 3)), R1 = min_of(READS, ((Q + 1) * READS * 4 + N * 3 - 1) / (N * 3));   // in the first three quarters
       each<R1 - R0>([&](auto i) { read(fetched, std::integral_constant<int, R0 + decltype(i)::value>{}); });   // (behind the last step: zeros)
-      constexpr int L0 = Q * LOADS / N, L1 = (Q + 1) * LOADS / N;
+      constexpr int L0 = min_of(LOADS, Q * LOADS * 4 / (N * 3)), L1 = Q == N - 1 ? LOADS : min_of(LOADS, (Q + 1) * LOADS * 4 / (N * 3));
       each<L1 - L0>([&](auto i) { load(std::integral_constant<int, L0 + decltype(i)::value>{}); });
+      constexpr int FROM = N - (N + 3) / 4, S0 = Q < FROM ? 0 : (Q - FROM) * AHEAD / (N - FROM), S1 = Q < FROM ? 0 : (Q + 1 - FROM) * AHEAD / (N - FROM);
+      static_assert(N % 4 == 0, "the step's reads and loads are out by FROM");
+      if constexpr (Q == FROM) fill = next_slot(fill);
+      each<S1 - S0>([&](auto i) {
+        constexpr int I = S0 + decltype(i)::value;
+        if constexpr (I < 3) advance(std::integral_constant<int, I>{});
+        else locate(next_slot(fill), std::integral_constant<int, I - 3>{});
+      });
       __builtin_amdgcn_sched_barrier(0);
     });
-    advance();
-    prepare();
   };
+  auto advance_whole = [&]() { each<3>([&](auto i) { advance(i); }); };
+  if (left < STEP) end_of_k();
 #pragma unroll 1
   for (int s = 0; s < SLOTS; s++) {
-    prepare();
     each<LOADS>([&](auto i) { load(i); });
-    advance();
+    advance_whole();
+    fill = next_slot(fill);
   }
+  each<1 + B_ADDRESSES>([&](auto i) { locate(0, i); });
   wait_for_all_but<(SLOTS - 1) * LOADS>();
   each<RA + RB>([&](auto i) { read(even, i); });
-  prepare();
+  each<1 + B_ADDRESSES>([&](auto i) { locate(SLOT, i); });
   for (int k = 0; k + 2 <= steps; k += 2) {
     step(even, odd);
     step(odd, even);
@@ -230,12 +261,12 @@ template <class T, bool A_UNSIGNED, int RB, int SLOTS>
 hipError_t launch_either(const GemmArgs &g, hipStream_t stream) {
   return g.b_kmajor ? launch_ring<T, A_UNSIGNED, true, RB, SLOTS>(g, stream) : launch_ring<T, A_UNSIGNED, false, RB, SLOTS>(g, stream);
 }
-// As many slots as a compute unit's LDS holds of the wider ones, which run one to a unit (of the 64-wide tile's,
-// five instead of three measured within 4 % either way).
+// As many slots as a compute unit's LDS holds of the wider ones, and four of the 64-wide tile's as well: all run one to a unit (of the
+// last, three / four / six: bf16 1024 x 7040 x 1344 35.7 / 33.2 / 33.4 us, 1664 x 6720 x 1152 34.6 / 33.0 / 33.2; of 128, five instead of four are within 1 %).
 template <class T, bool A_UNSIGNED>
 hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
   switch (bn) {
-    case 64: return launch_either<T, A_UNSIGNED, 2, 3>(g, stream);
+    case 64: return launch_either<T, A_UNSIGNED, 2, 4>(g, stream);
     case 128:
       if constexpr (T::ES == 2) return launch_either<T, A_UNSIGNED, 4, 4>(g, stream);
       return hipErrorInvalidValue;
