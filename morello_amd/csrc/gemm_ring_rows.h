@@ -5,6 +5,8 @@
 namespace mrl {
 namespace ring {
 typedef int chunk_anywhere __attribute__((ext_vector_type(4), aligned(1)));
+typedef __attribute__((address_space(1))) const uint8_t global_u8;
+typedef __attribute__((address_space(1))) const chunk_anywhere global_chunk;
 
 // The first `left` of v's bytes (none below 1, all from 16 on), zeros behind them.
 __device__ inline v4i first_bytes(v4i v, int left) {
@@ -24,7 +26,15 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
   constexpr int ES = T::ES, BK = STEP / ES, BM = 32 * RA, BN = 32 * RB, WM = 16 * RA, WN = 16 * RB;
   constexpr int A_BYTES = BM * STEP, B_BYTES = BN * STEP, SLOT = A_BYTES + B_BYTES;
   constexpr int A_LOADS = A_BYTES / (1024 * WAVES), B_LOADS = (B_BYTES / 1024 + WAVES - 1) / WAVES, LOADS = A_LOADS + B_LOADS;   // a wave's, per step
-  constexpr int DEPTH = 2;   // (four to eight, on the smallest tile: 4 to 13 % slower, more to wait for at the start and nothing gained behind it)
+  // The k loop in pairs of steps and one more.  With an exit between the two, the other form, the compiler sees a way from the first to itself and makes
+  // it wait for all but half a step's loads: less code, and as good as or better than two whole steps under way for small tiles of windows (u8
+  // 10 x (16 -> 224) x 10^2 5 x 5, five steps: 4.5 us, in pairs 4.7) and for rows on 128 x 128 tiles and, of int8 along K, wider ones (u8 726 x 996 x 4035
+  // 12.9 / 13.4, 2432 x 1702 x 2069 25.2 / 25.6).  Else worse: bf16 33 x 1664 x 12928 10.6 / 9.3, 138 x 699 x 368 6.6 / 6.2, 394 x 139 x 145 5.0 / 4.5,
+  // 8 x (256 -> 256) x 28^2 3 x 3 15.6 / 14.8.
+  constexpr bool PAIRS = CONV ? RA * RB > 4 : RB < 4 || (RB > 4 && !(ES == 1 && B_KMAJOR));
+  // Steps of loads under way (four to eight, on the smallest tile: 4 to 13 % slower, more to wait for at the start and nothing gained behind it).  In
+  // pairs on the widest tiles rows of any alignment lose by the second (bf16 2306 x 735 x 2260 17.3 us, with one 17.0; 3456 x 1909 x 1221 32.9 / 32.4).
+  constexpr int DEPTH = !CONV && PAIRS && RB >= 5 ? 1 : 2;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kw = wave >> 2, wm = wave >> 1 & 1, wn = wave & 1;
   const int64_t m0 = int64_t(tile_m) * BM, n_tile = int64_t(tile_n) * BN;
@@ -69,34 +79,36 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
       whole[A_LOADS + i] = r < head ? 16 : 0;
     }
   }
-  const uint8_t *a_tile = A, *b_tile = B;
+  const global_u8 *a_tile = (const global_u8 *)A, *b_tile = (const global_u8 *)B;
   const int64_t b_step = B_KMAJOR ? int64_t(STEP) : int64_t(BK) * ldb_b;
   // CONV: where the chunks of the step to load lie in a window, from its corner on; the step's first byte of the window.
   uint32_t in_window[A_LOADS];
   uint32_t window_byte = CONV ? blockIdx.y * g.conv.slice_bytes : 0;
-  auto find_chunks = [&]() {
-    if constexpr (CONV)
-#pragma unroll
-      for (int i = 0; i < A_LOADS; i++) {
-        const uint32_t kb = window_byte + chunk_of(wave * A_LOADS + i) * 16;
-        in_window[i] = kb + g.conv.by_run.div(kb) * g.conv.run_gap;
-      }
+  auto find_chunk = [&](auto which) {
+    constexpr int I = decltype(which)::value;
+    const uint32_t kb = window_byte + chunk_of(wave * A_LOADS + I) * 16;
+    in_window[I] = kb + g.conv.by_run.div(kb) * g.conv.run_gap;
+    asm("" : "+v"(in_window[I]));   // here, and not behind the next barrier
   };
-  find_chunks();
   auto load = [&](auto which) {
     constexpr int I = decltype(which)::value;
-    if constexpr (CONV && I < A_LOADS) return __builtin_bit_cast(v4i, *(const chunk_anywhere *)(A + (off[I] + in_window[I])));
-    else return __builtin_bit_cast(v4i, *(const chunk_anywhere *)((I < A_LOADS ? a_tile : b_tile) + off[I]));
+    if constexpr (CONV && I < A_LOADS) return __builtin_bit_cast(v4i, *(const global_chunk *)(a_tile + (off[I] + in_window[I])));
+    else return __builtin_bit_cast(v4i, *(const global_chunk *)((I < A_LOADS ? a_tile : b_tile) + off[I]));
   };
-  int loaded = 0;   // the step that the pointers are at
-  auto advance = [&]() {   // to the next one (past the last: nowhere)
-    const bool more = loaded + 1 < steps;
-    a_tile += !more ? 0 : loaded == 0 ? head * ES : STEP;
-    window_byte += !more ? 0 : loaded == 0 ? head * ES : STEP;
-    find_chunks();
-    b_tile += !more ? 0 : loaded == 0 ? (B_KMAJOR ? int64_t(head) * ES : int64_t(head) * ldb_b) : b_step;
-    loaded++;
+  int behind = steps;   // steps from the one that the pointers are at on
+  // To the next one (past the last: nowhere); `first`: from the first step, which has `head` elements.
+  auto advance = [&](auto first) {
+    const bool more = --behind > 0;
+    const int a_step = !more ? 0 : decltype(first)::value ? head * ES : STEP;
+    if constexpr (CONV) window_byte += a_step;
+    else {
+      a_tile += a_step;
+      if constexpr (PAIRS) asm("" : "+s"(a_tile));   // (scalar bases, not sums of each lane's)
+    }
+    b_tile += !more ? 0 : !decltype(first)::value ? b_step : B_KMAJOR ? int64_t(head) * ES : int64_t(head) * ldb_b;
+    if constexpr (PAIRS) asm("" : "+s"(b_tile));
   };
+  if constexpr (CONV) each<A_LOADS>([&](auto i) { find_chunk(i); });
 
   // Operand addresses within a slot: lane (l % 16, l / 16) takes the l / 16-th 16 bytes of row l % 16.
   const int in_rows = li * STEP + (((4 * kw + lg) ^ (li / ROWS_PER_LINE % CHUNKS)) << 4);
@@ -136,8 +148,13 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
 #pragma unroll
       for (int w = 0; w < 4; w++) colsum[C] = __builtin_amdgcn_sdot4(bf[S][C][w], 0x01010101, colsum[C], false);
   };
-  // All LDS reads and writes are done; loads stay under way.
-  auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); };
+  // All LDS reads and writes are done; loads stay under way.  (A builtin wait, which the compiler sees: it adds none of its own for the operands that are in.)
+  auto barrier = [] {
+    asm volatile("" : : : "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
+  };
   // A step of parity P whose successor but one waits in set K.
   auto step = [&](auto parity, auto held) {
     constexpr int P = decltype(parity)::value, K = decltype(held)::value;
@@ -153,19 +170,26 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
         *(v4i *)(lds + P * SLOT + dst[I]) = kept[K][I];
         kept[K][I] = load(std::integral_constant<int, I>{});
       });
+      if constexpr (Q == N - 1) advance(std::false_type{});
+      if constexpr (CONV && Q == N - 1) each<A_LOADS>([&](auto i) { find_chunk(i); });
       __builtin_amdgcn_sched_barrier(0);
     });
-    advance();
   };
   {
     v4i first[2][LOADS];
     each<2>([&](auto s) {
       each<LOADS>([&](auto i) { first[decltype(s)::value][decltype(i)::value] = load(i); });
-      advance();
+      if constexpr (PAIRS) __builtin_amdgcn_sched_barrier(0);
+      advance(std::integral_constant<bool, decltype(s)::value == 0>{});
+      if constexpr (CONV) each<A_LOADS>([&](auto i) { find_chunk(i); });
     });
     each<DEPTH>([&](auto s) {
-      each<LOADS>([&](auto i) { kept[decltype(s)::value][decltype(i)::value] = load(i); });
-      advance();
+      each<LOADS>([&](auto i) {
+        kept[decltype(s)::value][decltype(i)::value] = load(i);
+        if constexpr (PAIRS) __builtin_amdgcn_sched_barrier(0);   // in this order, which the loop's waits count on
+      });
+      advance(std::false_type{});
+      if constexpr (CONV) each<A_LOADS>([&](auto i) { find_chunk(i); });
     });
 #pragma unroll
     for (int i = 0; i < LOADS; i++) {
@@ -175,16 +199,27 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
   }
   barrier();
   each<RA + RB>([&](auto i) { read(std::integral_constant<int, 0>{}, i); });
-  // (what a step reads and writes for those behind the last one is not multiplied)
-  for (int left = steps;;) {
-    bool done = false;
-    each<DEPTH>([&](auto s) {
-      if (!done) {
-        step(std::integral_constant<int, decltype(s)::value % 2>{}, s);
-        done = --left == 0;
-      }
-    });
-    if (done) break;
+  // (What a step reads and writes for those behind the last one is not multiplied.)
+  const std::integral_constant<int, 0> even;
+  const std::integral_constant<int, 1> odd;
+  const std::integral_constant<int, DEPTH - 1> second;
+  if constexpr (!PAIRS) {
+    for (int left = steps;;) {
+      bool done = false;
+      each<2>([&](auto s) {
+        if (!done) {
+          step(s, std::integral_constant<int, decltype(s)::value % DEPTH>{});
+          done = --left == 0;
+        }
+      });
+      if (done) break;
+    }
+  } else {
+    for (int left = steps; left >= 2; left -= 2) {
+      step(even, even);
+      step(odd, second);
+    }
+    if (steps & 1) step(even, even);
   }
   barrier();
   store_tile<T, A_UNSIGNED, RA, RB>(g, lds, acc, colsum, m0, n0, int(n_tile - n0));
