@@ -83,12 +83,16 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, uint8_t *lds, type
     C += int64_t(blockIdx.y) * g.sc + row_first * g.ldc + col_first;
     const int rows = int(min(int64_t(WM), int64_t(g.m) - row_first));
     const int some = max(from, 0);   // a place of this wave's: read, not written, by lanes that have none
-    // An element a lane, or four where all of a row's columns are whole and aligned.  Old values come in batches: one at a
-    // time, each behind the store before it, they took longer than a short K (bf16 2163 x 420 x 513).
+    // An element a lane, or four where all of a row's columns are whole and aligned.  Of bf16 eight where they are not, wherever rows start: two bytes a
+    // lane take as many accesses to an eighth of the bytes (us, by elements / eights: 1501 x 1001 x 2001 18.5 / 17.2, 2072 x 1899 x 2689 36.4 / 33.9, 179 x 142
+    // x 2617 4.3 / 4.0, 1001 x 2050 x 4425 with its copies 35.8 / 33.9; onto old values, eights read from anywhere too, 1500 x 300 x 1501 11.0 / 14.6).
+    // Old values come in batches: one at a time, each behind the store before it, they took longer than a short K (bf16 2163 x 420 x 513).
     auto rows_of = [&](auto at_once) {
-      constexpr int V = decltype(at_once)::value, COUNT = WM * WN / V / 128, BATCH = divisor_up_to(8, COUNT);
+      constexpr int V = decltype(at_once)::value, COUNT = (WM * WN / V + 127) / 128, BATCH = divisor_up_to(8, COUNT);
       typedef Stored stored_v __attribute__((ext_vector_type(V)));
+      typedef stored_v stored_there __attribute__((aligned(V == 8 ? sizeof(Stored) : V * sizeof(Stored))));
       typedef Out out_v __attribute__((ext_vector_type(V)));
+      typedef out_v out_there __attribute__((aligned(V < 4 ? 4 : 16)));
 #pragma unroll 1
       for (int e = 0; e < COUNT; e += BATCH) {
         int64_t to[BATCH];
@@ -98,22 +102,27 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, uint8_t *lds, type
 #pragma unroll
         for (int u = 0; u < BATCH; u++) {
           const int at = (2 * (e + u) + kw) * 64 + lane, row = at / (WN / V), col = at % (WN / V) * V;
-          mine[u] = row < rows && col >= from && col < cols;
+          mine[u] = row < rows && col >= from && (V == 8 ? col + V <= cols : col < cols);
           to[u] = mine[u] ? int64_t(row) * g.ldc + col : some;
-          v[u] = *(const out_v *)(piece + row * ROW + col);
+          v[u] = *(const out_there *)(piece + (V == 8 ? min(row, WM - 1) : row) * ROW + col);
+          if constexpr (V == 8)
+            if (!mine[u] && row < rows)   // what an edge cuts
+#pragma unroll 1
+              for (int c = max(col, from); c < min(col + V, cols); c++) C[int64_t(row) * g.ldc + c] = Stored(piece[row * ROW + c]);
         }
-        if (g.accum) {
+        if (V < 8 && g.accum) {
 #pragma unroll
-          for (int u = 0; u < BATCH; u++) old[u] = *(const stored_v *)(C + to[u]);
+          for (int u = 0; u < BATCH; u++) old[u] = *(const stored_there *)(C + to[u]);
 #pragma unroll
           for (int u = 0; u < BATCH; u++) v[u] += __builtin_convertvector(old[u], out_v);
         }
 #pragma unroll
         for (int u = 0; u < BATCH; u++)
-          if (mine[u]) *(stored_v *)(C + to[u]) = __builtin_convertvector(v[u], stored_v);
+          if (mine[u]) *(stored_there *)(C + to[u]) = __builtin_convertvector(v[u], stored_v);
       }
     };
     if (cols % 4 == 0 && from % 4 == 0 && g.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % (4 * sizeof(Stored)) == 0) rows_of(std::integral_constant<int, 4>{});
+    else if (sizeof(Stored) == 2 && !g.accum) rows_of(std::integral_constant<int, sizeof(Stored) == 2 ? 8 : 1>{});
     else rows_of(std::integral_constant<int, 1>{});
   };
   // The two halves of K: the upper waves' sums through LDS onto the lower waves', and both store.
