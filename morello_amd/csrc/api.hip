@@ -546,11 +546,12 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     // A and B as rows, whichever way B's run; an operand with no rows at all is turned by a Move.
     mrl::PadRows pads[2];
     int n_pads = 0;
-    auto make_rows = [&](Prepared &p, mrl::Strided &t, uint32_t rows, bool *padded) -> int {
+    auto make_rows = [&](Prepared &p, mrl::Strided &t, uint32_t rows, uint32_t panel, bool *padded) -> int {
       *padded = false;
       if (walkable(t)) return MRL_OK;
       mrl::Strided dense = rows_of(t);
       *padded = as_rows(t, &any_ld, &any_bs);
+      if (panel != 0) dense.stride[1] = (int64_t(t.shape[2]) + panel - 1) / panel * panel;
       if (*padded) dense.stride[0] = int64_t(rows) * dense.stride[1];
       // (a copy that cannot be: the operand stays as it is, for the generic kernel)
       if (*padded && !mrl::pad_rows_possible({t, nullptr, uint32_t(dense.stride[1]), rows, p.elem})) {
@@ -560,7 +561,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
       const size_t bytes = size_t(t.shape[0]) * dense.stride[0] * p.elem;
       HIP_TRY(ws.alloc(&dense.ptr, bytes));
       if (*padded) {
-        pads[n_pads++] = {t, dense.ptr, uint32_t(dense.stride[1]), rows, p.elem};
+        pads[n_pads++] = {t, dense.ptr, uint32_t(dense.stride[1]), rows, p.elem, panel};
       } else {
         if (dense.stride[1] != int64_t(t.shape[2])) HIP_TRY(mrl::launch_fill_zero(dense.ptr, bytes, ws.stream));
         HIP_TRY(mrl::launch_move_strided(t, dense, ws.stream));
@@ -569,7 +570,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
       return MRL_OK;
     };
     bool a_padded, b_padded;
-    if ((rc = make_rows(a, a.t, a.t.shape[1], &a_padded)) != MRL_OK) return rc;
+    if ((rc = make_rows(a, a.t, a.t.shape[1], 0, &a_padded)) != MRL_OK) return rc;
     // A right operand of one column (or one row) has rows either way: read in place where one of them allows it, else
     // copied as the fewer bytes (f32 20000 x (3 x 16 x 1): one row of K, or sixteen of an element each).
     auto copied = [&](const mrl::Strided &t) { return double(t.shape[1]) * double(rows_of(t).stride[1]); };
@@ -585,8 +586,23 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     // steps or more; a short row-major operand would only get a copy of many times its rows (u8 16 x 3 x 4825541: 77 MB for 14).
     const uint32_t whole_k = uint32_t((g.k + per16 - 1) / per16 * per16);
     const bool end_whole = a_padded && !g_tight_scratch && (g.b_kmajor || uint64_t(whole_k) * a.elem >= 16 * 128);
-    if ((rc = make_rows(b, b_rows, g.b_kmajor ? b_rows.shape[1] : end_whole ? whole_k : g.k, &b_padded)) != MRL_OK) return rc;
+    // The copy of a row-major B for a tile of gemm_ring.hip is cut into that tile's columns: what a step takes of it is then contiguous, whole
+    // lines of few pages, and not 64 to 384 bytes of each of 64 or 128 rows (us, rows / panels: u8 1408 x 6001 x 1409 33.5 / 30.7, 1546 x 5000 x 2561 45.5 /
+    // 43.9, bf16 750 x 3001 x 2900 twice 52.6 / 50.7, 1100 x 4000 x 1101 30.7 / 29.8, 1001 x 2050 x 4425 33.3 / 33.1).
+    const uint32_t b_rows_count = g.b_kmajor ? b_rows.shape[1] : end_whole ? whole_k : g.k;
+    uint32_t panel = 0;
+    if (!g.b_kmajor && kind <= 2 && !g_tight_scratch && !walkable(b_rows) && as_rows(b_rows, &any_ld, &any_bs)) {
+      mrl::GemmArgs then = g;
+      then.a = a.t.ptr, then.b = nullptr, then.k = b_rows_count;
+      then.ldb = rows_of(b_rows).stride[1], then.sb = int64_t(b_rows_count) * then.ldb;
+      uint32_t k_rest = 0;
+      if (as_rows(a.t, &then.lda, &then.sa) && mrl::gemm_possible(then, kind) && mrl::gemm_pays(then, kind) &&
+          mrl::gemm_k_splits(then, kind, &k_rest) == 1)
+        panel = mrl::gemm_goes_to_ring(then, kind);
+    }
+    if ((rc = make_rows(b, b_rows, b_rows_count, panel, &b_padded)) != MRL_OK) return rc;
     if (end_whole && b_padded) g.k = whole_k;
+    if (panel != 0 && b_padded) g.b_panel_rows = b_rows_count;
     b.t = g.b_kmajor ? transposed(b_rows) : b_rows;
     if (n_pads == 2) HIP_TRY(mrl::launch_pad_rows_pair(pads[0], pads[1], ws.stream));
     else if (n_pads == 1) HIP_TRY(mrl::launch_pad_rows(pads[0], ws.stream));

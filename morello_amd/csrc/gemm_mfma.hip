@@ -194,13 +194,20 @@ hipError_t launch_gemm_big(const GemmArgs &g, int kind, hipStream_t stream, uint
   return hipErrorInvalidValue;
 }
 
+// Only the 256 tile has a build without the EDGE kernels' limit on leading dimensions.
+static uint32_t side_of(const GemmArgs &g, int es) { return edge_addressable(g, es) ? tile_side(g, es) : 256; }
+
+uint32_t gemm_goes_to_ring(const GemmArgs &g, int kind) {
+  return gemv_applicable(g, kind) || side_of(g, elem_size_of(kind)) == 256 ? 0 : gemm_ring_columns(g, kind);
+}
+
 hipError_t launch_gemm(const GemmArgs &g, int kind, hipStream_t stream) {
+  if (const uint32_t bn = gemm_goes_to_ring(g, kind)) return launch_gemm_ring(g, kind, bn, stream);
+  if (g.b_panel_rows != 0) return hipErrorInvalidValue;   // (laid out for that kernel)
   if (gemv_applicable(g, kind)) return launch_gemv(g, kind, stream);
   const int es = elem_size_of(kind);
-  // Only the 256 tile has a build without the EDGE kernels' limit on leading dimensions.
-  const uint32_t side = edge_addressable(g, es) ? tile_side(g, es) : 256;
+  const uint32_t side = side_of(g, es);
   if (side == 256) return launch_gemm_big(g, kind, stream);
-  if (const uint32_t bn = gemm_ring_columns(g, kind)) return launch_gemm_ring(g, kind, bn, stream);
   if (g.b_kmajor) return launch_gemm_nt(g, kind, side, stream);
   return launch_gemm_scheduled(g, kind, side, side, 128 / es, stream);
 }

@@ -72,10 +72,11 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
   MRL_WALK_TILE(tile_m, tile_n)
   const int64_t m0 = int64_t(tile_m) * BM, n0 = int64_t(tile_n) * BN;
   const uint8_t *A = (const uint8_t *)g.a + (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES;
-  const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : n0)) * ES;
-  const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = uint32_t(g.ldb) * ES;
+  const bool panels = !B_KMAJOR && g.b_panel_rows != 0;
+  const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : panels ? n0 * g.b_panel_rows : n0)) * ES;
+  const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = panels ? BN * ES : uint32_t(g.ldb) * ES;
   // Bytes of the tile's rows (leading dimensions stay below 2^24 bytes); what of a row-major B's lies left of the tile.
-  const int a_end = min(BM, int(g.m - m0)) * int(lda_b), n0_b = int(n0) * ES;
+  const int a_end = min(BM, int(g.m - m0)) * int(lda_b), n0_b = panels ? 0 : int(n0) * ES;
   const uint32_t b_end = uint32_t(min(BN, int(g.n - n0))) * ldb_b;
   const int k_bytes = int(g.k) * ES, steps = (k_bytes + STEP - 1) / STEP;
 

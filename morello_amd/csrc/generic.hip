@@ -597,6 +597,8 @@ struct PadJob {
   uint32_t chunks;                        // destination chunks in all
   int64_t src_batch, src_ld;                        // bytes
   FastDiv by_row_chunks, by_dst_rows;
+  uint32_t panel_chunks;                  // of a row of a panel (0: no panels)
+  FastDiv by_panel_chunks;
 };
 constexpr int PAD_UNROLL = 4;
 template <int UNROLL>
@@ -604,13 +606,18 @@ __device__ inline void pad_chunks(const PadJob &j) {
   const uint32_t first = blockIdx.x * (256 * UNROLL) + threadIdx.x;
   chunk_t lo[UNROLL], hi[UNROLL];
   int left[UNROLL];
-  uint32_t shift[UNROLL];
+  uint32_t shift[UNROLL], to[UNROLL];
 #pragma unroll
   for (int u = 0; u < UNROLL; u++) {
     const uint32_t i = min(first + u * 256, j.chunks - 1);
     const uint32_t line = j.by_row_chunks.div(i), entry = j.by_dst_rows.div(line), row = line - entry * j.dst_rows;
     const PadChunk c = pad_chunk(i - line * j.row_chunks, row < j.rows ? j.row_bytes : 0);
     left[u] = c.left;
+    to[u] = i;
+    if (j.panel_chunks != 0) {
+      const uint32_t in_row = i - line * j.row_chunks, panel = j.by_panel_chunks.div(in_row);
+      to[u] = (entry * j.row_chunks + panel * j.panel_chunks) * j.dst_rows + row * j.panel_chunks + in_row - panel * j.panel_chunks;
+    }
     // (a chunk with nothing in it reads the row's first instead)
     const uint8_t *from = j.src + int64_t(entry) * j.src_batch + int64_t(min(row, j.rows - 1)) * j.src_ld + c.at;
     shift[u] = uint32_t(uintptr_t(from) & 15);
@@ -620,7 +627,7 @@ __device__ inline void pad_chunks(const PadJob &j) {
   }
 #pragma unroll
   for (int u = 0; u < UNROLL; u++)
-    if (first + u * 256 < j.chunks) j.dst[first + u * 256] = keep_bytes(cut_chunk(lo[u], hi[u], shift[u]), left[u]);
+    if (first + u * 256 < j.chunks) j.dst[to[u]] = keep_bytes(cut_chunk(lo[u], hi[u], shift[u]), left[u]);
 }
 template <int UNROLL>
 __global__ __launch_bounds__(256) void k_pad_rows(PadJob j) { pad_chunks<UNROLL>(j); }
@@ -1534,6 +1541,7 @@ bool pad_job(const PadRows &p, PadJob *j) {
   j->chunks = batch * p.dst_rows * j->row_chunks;
   j->src_batch = (batch == 1 ? 0 : src.stride[0]) * int64_t(es), j->src_ld = (rows == 1 ? 0 : src.stride[1]) * int64_t(es);
   j->by_row_chunks = FastDiv(j->row_chunks), j->by_dst_rows = FastDiv(j->dst_rows);
+  j->panel_chunks = p.panel * es / 16, j->by_panel_chunks = FastDiv(std::max(1u, j->panel_chunks));
   return true;
 }
 // Four chunks a thread, their loads in flight together, for copies that fill the chip several times over; below, one a
@@ -1555,6 +1563,8 @@ hipError_t launch_pad_rows(const PadRows &p, hipStream_t stream) {
 hipError_t launch_pad_rows_pair(const PadRows &p0, const PadRows &p1, hipStream_t stream) {
   PadJob j0, j1;
   if (!pad_job(p0, &j0) || !pad_job(p1, &j1)) return hipErrorInvalidValue;
+  // The larger first: workgroups of the smaller that have nothing to copy then stand at the launch's end (bf16 1344 x 1111 x 5021 33.7 / 33.0 us).
+  if (j0.chunks < j1.chunks) std::swap(j0, j1);
   plan::work(plan::UNIT_STREAM, 0, pad_bytes(j0) + pad_bytes(j1));
   const uint32_t most = std::max(j0.chunks, j1.chunks);
   if (pad_in_fours(most)) MRL_LAUNCH((k_pad_rows_pair<PAD_UNROLL>), dim3((most + 256 * PAD_UNROLL - 1) / (256 * PAD_UNROLL), 2), dim3(256), 0, stream, j0, j1);

@@ -92,10 +92,12 @@ hipError_t launch_move_view(const void *src, int src_dtype, void *dst, int dst_d
 // Copy of a [batch][rows][cols] tensor with contiguous rows (starting on any element) into dense rows of
 // `dst_ld` elements (whole 16-byte chunks), `dst_rows` per batch entry; zeros from each row's end to
 // `dst_ld` and in the rows past the source's.
+// panel not 0 (whole chunks, a divisor of dst_ld): an entry's rows are cut into panels of that many elements, which
+// follow each other, dst_rows rows of `panel` each.
 struct PadRows {
   Strided src;
   void *dst;
-  uint32_t dst_ld, dst_rows, elem_size;
+  uint32_t dst_ld, dst_rows, elem_size, panel = 0;
 };
 bool pad_rows_possible(const PadRows &p);   // (`dst` not looked at) fewer than 2^31 chunks, which the kernel numbers in 32 bits
 hipError_t launch_pad_rows(const PadRows &p, hipStream_t stream);
@@ -145,6 +147,8 @@ struct GemmArgs {
   uint32_t k_total = 0;
   // Scratch is short: rows are read in place wherever that is possible (gemm_ring_rows.hip).
   bool tight = false;
+  // Not 0 (gemm_ring.hip, a row-major B): B's copy is in panels as wide as the tile, this many rows each (PadRows).
+  uint32_t b_panel_rows = 0;
   // C is bf16 (bf16 operands only): the f32 sum, the old value included, is rounded once.
   bool c_bf16 = false;
   // Conv as an implicit Matmul (the CONV build of the kernel): `a` is a channels-last image
@@ -196,6 +200,7 @@ hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint
 // gemm_ring.hip: tiles of 128 rows by `bn` (64, 128, 160 or 192) columns, operands straight into a ring of LDS slots; what
 // gemm_possible() takes with edge_addressable() leading dimensions.  gemm_ring_columns: the width for a problem, 0 for none.
 uint32_t gemm_ring_columns(const GemmArgs &g, int kind);
+uint32_t gemm_goes_to_ring(const GemmArgs &g, int kind);   // its width where launch_gemm takes it, else 0
 hipError_t launch_gemm_ring(const GemmArgs &g, int kind, uint32_t bn, hipStream_t stream);
 // gemm_ring_rows.hip: such tiles for rows that start anywhere (K or N no whole 16-byte chunks), operands read in place; its
 // smallest, 64 x 64, is also the faster one for whole chunks.
