@@ -595,6 +595,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
       mrl::GemmArgs then = g;
       then.a = a.t.ptr, then.b = nullptr, then.k = b_rows_count;
       then.ldb = rows_of(b_rows).stride[1], then.sb = int64_t(b_rows_count) * then.ldb;
+      if (!as_rows(c.t, &then.ldc, &then.sc)) then.ldc = g.n;   // (made dense below)
       uint32_t k_rest = 0;
       if (as_rows(a.t, &then.lda, &then.sa) && mrl::gemm_possible(then, kind) && mrl::gemm_pays(then, kind) &&
           mrl::gemm_k_splits(then, kind, &k_rest) == 1)

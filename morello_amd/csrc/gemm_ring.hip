@@ -268,9 +268,7 @@ template <class T, bool A_UNSIGNED>
 hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
   switch (bn) {
     case 64: return launch_either<T, A_UNSIGNED, 2, 4>(g, stream);
-    case 128:
-      if constexpr (T::ES == 2) return launch_either<T, A_UNSIGNED, 4, 4>(g, stream);
-      return hipErrorInvalidValue;
+    case 128: return launch_either<T, A_UNSIGNED, 4, 4>(g, stream);
     case 160: return launch_either<T, A_UNSIGNED, 5, 4>(g, stream);
     case 192: return launch_either<T, A_UNSIGNED, 6, 4>(g, stream);
     default: return hipErrorInvalidValue;
@@ -279,24 +277,31 @@ hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
 
 }  // namespace
 
-// Measured against k_gemm's tiles (us, k_gemm / this), on rounds of one tile per compute unit:
+// Measured against k_gemm's tiles (us, k_gemm / this; means of 520 random sizes, of three sets of operands in turn), on rounds of one
+// tile per compute unit:
 //   64 where k_gemm's 64 tile would go two to a unit (257 of them on) and this one at most one: bf16 1100 x 3001 x
-//     1100 35.1 / 28.0, 1280 x 1024 x 1600 11.2 / 10.6, u8 1408 x 3001 x 1408 23.6 / 20.9; two to a unit it loses (400 x
-//     3001 x 4400 35.7 / 46.4);
+//     1100 35.1 / 28.0, u8 1408 x 3001 x 1408 23.6 / 20.9; two to a unit it loses (400 x 3001 x 4400 35.7 / 46.4).  bf16 from 13
+//     steps on (13 to 15 1.13 times as fast, 1.11 with operands from memory; 11 and 12 1.05 and from memory 0.85 at the least, nine and ten 1.02 and
+//     0.91), integers from 14 (14 to 16 1.11, from memory 1.09; 11 to 13 1.04 and 0.97, seven and eight 0.98);
+//   128 for more than half a round of 128 x 128.  Integers from 28 steps on: 4054 x 4352 x 832 26.6 / 24.1 (28 and 29 1.07, 30 to 34 1.06, from memory
+//     1.03; 23 to 25 1.02 and from memory 0.97, 11 to 16 0.94).  bf16 too: 2048^3 22.9 / 22.2 (28 and 29 1.04, 30 to 34 1.09, from memory 1.07;
+//     23 to 26 1.06, but 0.93 for one in six; 9 to 16 0.95).  Where 64 x 64 tiles are 512 at most, which k_gemm runs two to a unit, both from 36
+//     (integers 35 to 44 1.08, bf16 45 on 1.22; 30 to 34 1.02 and from memory 0.95, 11 to 19 0.89);
 //   160, else 192, where the 128 tile needs a second round and they do not: bf16 1001 x 2050 x 4425 47.2 / 38.9, 1800 x 2001
-//     x 3000 41.0 / 35.3, u8 1000 x 2001 x 4500 34.6 / 30.1;
-//   128, bf16, within one round: 1984 x 5171 x 1536 55.6 / 50.0, 2048^3 22.9 / 22.2 (u8 2048 x 2001 x 1792 20.0 / 22.1).
-// Short K leaves the start of the ring and the summing of the two halves of K dominant: bf16 1408 x 320 x 1408 5.9 /
-// 6.7, 2048 x 512 x 2560 12.0 / 13.2, 1500 x 512 x 2500 15.9 / 16.5.
+//     x 3000 41.0 / 35.3, u8 1000 x 2001 x 4500 34.6 / 30.1.  (128 in two rounds: 0.92 to 1.03, and 0.90 with operands from memory.)
+// Short K leaves the start of the ring and the summing of the two halves of K dominant: bf16 1408 x 320 x 1408 5.9 / 6.7.
 uint32_t gemm_ring_columns(const GemmArgs &g, int kind) {
   if (kind < 0 || kind > 2) return 0;
   const uint64_t es = kind == 2 ? 2 : 1, steps = (uint64_t(g.k) * es + STEP - 1) / STEP;
-  if (steps < 16 || g.m <= 128 || g.n <= 128) return 0;
+  if (steps < (kind == 2 ? 13 : 14) || g.m <= 128 || g.n <= 128) return 0;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
-  const uint64_t units = g_compute_units, small = tiles(64, 64);
-  if (small <= 512) return small > units && tiles(BM, 64) <= units ? 64 : 0;
-  const uint64_t whole = tiles(BM, 128);
-  if (whole <= units) return kind == 2 && steps >= 32 && 2 * whole > units ? 128 : 0;
+  const uint64_t units = g_compute_units, small = tiles(64, 64), whole = tiles(BM, 128);
+  if (small <= 512) {
+    if (small <= units) return 0;
+    return tiles(BM, 64) <= units ? 64 : 2 * whole > units && steps >= 36 ? 128 : 0;
+  }
+  if (whole <= units) return 2 * whole > units && steps >= 28 ? 128 : 0;
+  if (steps < 16) return 0;
   return tiles(BM, 160) <= units ? 160 : tiles(BM, 192) <= units ? 192 : 0;
 }
 
