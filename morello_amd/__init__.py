@@ -34,6 +34,17 @@ def _check(status: int, where: str):
         raise MorelloError(status, where)
 
 
+class _PointerArrays(dict):
+    """The ctypes array type of n pointers: forming it anew costs a call as much as checking its Spec."""
+
+    def __missing__(self, n: int):
+        self[n] = C.c_void_p * n
+        return self[n]
+
+
+_pointers = _PointerArrays()
+
+
 class Dtype(enum.IntEnum):
     """morello/src/common.rs:15-24."""
     Uint8 = 0
@@ -273,19 +284,19 @@ class Spec:
     # -- execution -------------------------------------------------------------------
     def run_device(self, ptrs: Sequence[int]):
         """`ptrs`: device pointers in Spec parameter order.  Synchronous."""
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         _check(B.load().mrl_run(C.byref(self._c), arr), "mrl_run")
 
     def run_async(self, ptrs: Sequence[int], stream: "Stream"):
         """Enqueues the Spec on `stream` and returns; `stream.synchronize()` waits for it."""
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         _check(B.load().mrl_run_async(C.byref(self._c), arr, stream.handle), "mrl_run_async")
 
     def run_noalloc(self, ptrs: Sequence[int], stream: "Stream | None" = None):
         """As run_async without any device allocation: scratch comes from the library's fixed
         per-GPU array (NOALLOC_SCRATCH_BYTES); MorelloError (tensor too large) if the Spec needs more
         even with the smallest copies of its operands."""
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         _check(B.load().mrl_run_noalloc(C.byref(self._c), arr, stream.handle if stream else None), "mrl_run_noalloc")
 
     def run_host(self, *arrays: np.ndarray):
@@ -303,7 +314,7 @@ class Spec:
 
     def run_timed(self, ptrs: Sequence[int], steps: int) -> float:
         """`steps` back-to-back launches between two HIP events; total device milliseconds."""
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         ms = C.c_double()
         _check(B.load().mrl_run_timed(C.byref(self._c), arr, steps, C.byref(ms)), "mrl_run_timed")
         return ms.value
@@ -340,7 +351,7 @@ class Spec:
 
     def bench(self, ptrs: Sequence[int], iters: int, repeats: int = 10):
         """CodeGen::bench protocol (codegen/mod.rs:133-169): (best, mean) ns per launch."""
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         best, mean = C.c_double(), C.c_double()
         _check(B.load().mrl_bench(C.byref(self._c), arr, iters, repeats, C.byref(best), C.byref(mean)),
                "mrl_bench")
@@ -382,7 +393,7 @@ class ScheduledMatmul:
         if self.split_k is None:
             raise MorelloError(1, "schedule needs .split(k)")
         sched = B.MatmulScheduleC(self.tile_m, self.tile_n, self.split_k, int(self.staging))
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         lib = B.load()
         synchronize()
         t0 = time.perf_counter()
@@ -396,7 +407,7 @@ class ScheduledMatmul:
         if self.split_k is None:
             raise MorelloError(1, "schedule needs .split(k)")
         sched = B.MatmulScheduleC(self.tile_m, self.tile_n, self.split_k, int(self.staging))
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         _check(B.load().mrl_run_matmul_scheduled(C.byref(self.spec._c), arr, C.byref(sched), None),
                "mrl_run_matmul_scheduled")
         synchronize()
@@ -560,7 +571,7 @@ class Compose:
         return _plan_of(B.load().mrl_compose_plan, self._c, "mrl_compose_plan")
 
     def run_device(self, ptrs: Sequence[int]):
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         _check(B.load().mrl_run_compose(C.byref(self._c), arr, None), "mrl_run_compose")
         synchronize()
 
@@ -644,13 +655,13 @@ class Action:
         return Plan([PlanStep(steps[i]) for i in range(min(cap, head.n_steps))], head.cost_ns, int(head.scratch_bytes))
 
     def run_device(self, ptrs: Sequence[int]):
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         _check(B.load().mrl_run_action(C.byref(self.spec._c), arr, C.byref(self._c), None), "mrl_run_action")
         synchronize()
 
     def run_timed(self, ptrs: Sequence[int], steps: int) -> float:
         """`steps` back-to-back launches of this action between two HIP events; total device milliseconds."""
-        arr = (C.c_void_p * len(ptrs))(*ptrs)
+        arr = _pointers[len(ptrs)](*ptrs)
         ms = C.c_double()
         _check(B.load().mrl_run_action_timed(C.byref(self.spec._c), arr, C.byref(self._c), steps, C.byref(ms)),
                "mrl_run_action_timed")

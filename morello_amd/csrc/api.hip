@@ -350,7 +350,7 @@ struct Workspace {
 // per element.
 int relayout(const void *src, void *dst, bool to_dense, const Prepared &p, Workspace &ws) {
   const mrl_layout &from = to_dense ? p.user_desc : p.dense_desc, &to = to_dense ? p.dense_desc : p.user_desc;
-  std::vector<mrl::MoveDim> view;
+  mrl::MoveView view;
   if (mrl::common_view(from, to, p.t.shape, p.t.rank, &view)) {
     const hipError_t e = mrl::launch_move_view(src, p.t.dtype, dst, p.t.dtype, view.data(), uint32_t(view.size()), ws.stream);
     if (e == hipSuccess) return MRL_OK;
@@ -377,7 +377,7 @@ int prepare(const mrl_spec &s, uint32_t idx, void *ptr, bool needs_read, Workspa
   mrl_layout dense;
   mrl_layout_row_major(shape, rank, &dense);
   // A layout with Packed dims can still be row-major order (layout![0, 1, 1p16], say).
-  std::vector<mrl::MoveDim> view;
+  mrl::MoveView view;
   if (mrl::common_view(s.layouts[idx], dense, shape, rank, &view) &&
       mrl::same_order(view)) {
     out->t.ptr = ptr;
@@ -1033,7 +1033,7 @@ int run_compose_msm(const mrl_spec &s, void *const *params, Workspace &ws) {
     {
       mrl_layout rows_kt;
       mrl_layout_row_major(kt_shape, 3, &rows_kt);
-      std::vector<mrl::MoveDim> view;
+      mrl::MoveView view;
       at.kt_rows = k == dp && n2 % 8 == 0 && (reinterpret_cast<uintptr_t>(params[2]) & 15) == 0 &&
                    mrl::common_view(s.layouts[2], rows_kt, kt_shape, 3, &view) && mrl::same_order(view);
     }
@@ -1045,7 +1045,7 @@ int run_compose_msm(const mrl_spec &s, void *const *params, Workspace &ws) {
     auto operand = [&](uint32_t i, const uint32_t *shape, const mrl_layout &want, uint32_t rows, uint32_t cols,
                        const void **result) -> int {
       const void *dense = params[i];
-      std::vector<mrl::MoveDim> view;
+      mrl::MoveView view;
       if (!mrl::common_view(s.layouts[i], want, shape, 3, &view)) return MRL_ERR_UNSUPPORTED;
       const bool in_order = mrl::same_order(view);
       if (!in_order) {
@@ -1073,7 +1073,7 @@ int run_compose_msm(const mrl_spec &s, void *const *params, Workspace &ws) {
       at.kt = params[2];
       return MRL_OK;
     };
-    std::vector<mrl::MoveDim> out_view;
+    mrl::MoveView out_view;
     int rc = MRL_OK;
     if (mrl::common_view(rows_o, s.layouts[3], o_shape, 3, &out_view) &&
         (rc = operand(0, v_shape, rows_v, n2, n, &at.v)) == MRL_OK &&
@@ -1160,7 +1160,7 @@ int run_move(const mrl_spec &s, void *const *params, Workspace &ws) {
   }
   // Layouts with a common strided view (permutations of the logical dims; Packed and OddEven
   // dims whose sizes refine each other): strided kernels, coalesced on both sides.
-  std::vector<mrl::MoveDim> view;
+  mrl::MoveView view;
   if (mrl::common_view(li, lo, shape, rank, &view)) {
     const hipError_t e = mrl::launch_move_view(params[0], s.dtypes[0], params[1], s.dtypes[1], view.data(),
                                                uint32_t(view.size()), ws.stream);
@@ -1685,7 +1685,7 @@ size_t mrl_spec_workspace_bytes(const mrl_spec *spec) {
     if (mrl::layout_strides(spec->layouts[i], shape, rank, strides)) continue;
     mrl_layout dense;
     mrl_layout_row_major(shape, rank, &dense);
-    std::vector<mrl::MoveDim> view;
+    mrl::MoveView view;
     if (mrl::common_view(spec->layouts[i], dense, shape, rank, &view) && mrl::same_order(view))
       continue;  // Packed dims in row-major order
     total += size_t(volume(shape, rank)) * mrl_dtype_size(spec->dtypes[i]);
