@@ -13,6 +13,7 @@
 
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace mrl {
@@ -71,6 +72,17 @@ double step_ns(const Step &s, uint32_t compute_units);
 
 inline hipError_t last_error() { return g_recorder ? hipSuccess : hipGetLastError(); }
 
+// The kernel's own stub would store the launch's shape, fetch it back and do this (2.43 us of host time a launch with 240 bytes
+// of arguments, 2.25 without the detour).  Arguments take the kernel's own types here as they do there; an error is left where the stub leaves
+// it, for last_error.
+template <class... P, class... A>
+inline void launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds_bytes, hipStream_t stream, A &&...a) {
+  [&](P... p) {
+    void *args[] = {(void *)&p...};
+    (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, args, lds_bytes, stream);
+  }(std::forward<A>(a)...);
+}
+
 }  // namespace plan
 }  // namespace mrl
 
@@ -79,6 +91,6 @@ inline hipError_t last_error() { return g_recorder ? hipSuccess : hipGetLastErro
     if (mrl::plan::recording()) mrl::plan::note(#kernel, __PRETTY_FUNCTION__, grid, block, lds);            \
     else {                                                                                             \
       mrl::plan::g_launches++;                                                                         \
-      hipLaunchKernelGGL(kernel, grid, block, lds, stream, __VA_ARGS__);                               \
+      mrl::plan::launch(kernel, grid, block, lds, stream, __VA_ARGS__);                                \
     }                                                                                                  \
   } while (0)
