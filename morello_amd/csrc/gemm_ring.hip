@@ -1,4 +1,4 @@
-// Matmul tiles of 128 rows by 64 to 192 columns for problems that do not fill the chip with 256 x 256 ones: operands
+// Matmul tiles of 128 rows by 64 to 192 columns, and of 64 x 64, for problems that do not fill the chip with 256 x 256 ones: operands
 // straight from memory into a ring of LDS slots of 128 bytes of K.
 //
 // What bounds a middling Matmul is less the MFMAs than everything around them: k_gemm's waves spend two
@@ -36,7 +36,6 @@ typedef __attribute__((address_space(3))) const uint8_t lds_u8;
 typedef __attribute__((address_space(3))) const v4i lds_v4i;
 
 constexpr uint32_t OUTSIDE = 0x80000000u;   // an offset no resource here holds
-constexpr int BM = 128;
 
 // One load of 64 lanes x 16 bytes into the KiB at LDS address `lds_addr` + AT (wave-uniform), lane l to the l-th
 // 16 bytes; the instruction's offset AT is added to the address in memory too, so callers take it off
@@ -59,10 +58,10 @@ __device__ inline void wait_for_all_but() {
   asm volatile("" : : : "memory");
 }
 
-template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RB, int SLOTS>
+template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RA, int RB, int SLOTS>
 __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_WALK_PARAMS, GemmArgs g) {
   typedef typename Ring<T>::Acc Acc;
-  constexpr int ES = T::ES, BK = STEP / ES, RA = 4, BN = 32 * RB, WM = 64, WN = 16 * RB;
+  constexpr int ES = T::ES, BK = STEP / ES, BM = 32 * RA, BN = 32 * RB, WM = 16 * RA, WN = 16 * RB;
   constexpr int A_BYTES = BM * STEP, B_BYTES = BN * STEP, SLOT = A_BYTES + B_BYTES;
   constexpr int A_LOADS = A_BYTES / (1024 * WAVES), B_LOADS = (B_BYTES / 1024 + WAVES - 1) / WAVES, LOADS = A_LOADS + B_LOADS;   // a wave's, per step
   static_assert((SLOTS - 1) * LOADS < 64 && A_LOADS <= 4 && B_LOADS <= 4, "");
@@ -78,7 +77,7 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
   // Bytes of the tile's rows (leading dimensions stay below 2^24 bytes); what of a row-major B's lies left of the tile.
   const int a_end = min(BM, int(g.m - m0)) * int(lda_b), n0_b = panels ? 0 : int(n0) * ES;
   const uint32_t b_end = uint32_t(min(BN, int(g.n - n0))) * ldb_b;
-  const int k_bytes = int(g.k) * ES, steps = (k_bytes + STEP - 1) / STEP;
+  const int k = g.k_total != 0 ? int(min(g.k, g.k_total - blockIdx.y * g.k)) : int(g.k), k_bytes = k * ES, steps = (k_bytes + STEP - 1) / STEP;
 
   // Where this lane's chunks of a step come from.  Rows of 64 bytes: sixteen to a load.
   uint32_t a_off[A_LOADS], b_off[B_LOADS];
@@ -238,11 +237,11 @@ __global__ __launch_bounds__(64 * WAVES, RB <= 2 ? 4 : 2) void k_gemm_ring(MRL_W
   store_tile<T, A_UNSIGNED, RA, RB>(g, lds, acc, colsum, m0, n0, 0);
 }
 
-template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RB, int SLOTS>
+template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RA, int RB, int SLOTS>
 hipError_t launch_ring(const GemmArgs &g, hipStream_t stream) {
-  constexpr auto kern = k_gemm_ring<T, A_UNSIGNED, B_KMAJOR, RB, SLOTS>;
-  constexpr int BN = 32 * RB, LDS = SLOTS * (BM + BN) * STEP;
-  static_assert(LDS >= 4 * 64 * (16 * RB + 4) * 4, "the waves' pieces of C fit");
+  constexpr auto kern = k_gemm_ring<T, A_UNSIGNED, B_KMAJOR, RA, RB, SLOTS>;
+  constexpr int BM = 32 * RA, BN = 32 * RB, LDS = SLOTS * (BM + BN) * STEP;
+  static_assert(LDS >= 4 * 16 * RA * (16 * RB + 4) * 4, "the waves' pieces of C fit");
   static std::atomic<uint64_t> lds_limit_set{0};
   if (!plan::recording() && LDS > 65536) {
     hipError_t e = raise_lds_limit(lds_limit_set, (const void *)kern, LDS);
@@ -254,23 +253,26 @@ hipError_t launch_ring(const GemmArgs &g, hipStream_t stream) {
              (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * (g.c_bf16 ? 2 : 4) * (g.accum ? 2 : 1),
              2.0 * BM * BN * steps * (STEP / T::ES), 2500.0 + 300.0 * steps);
   const TileWalk walk = gemm::tile_walk(tiles_m, tiles_n);
-  MRL_LAUNCH((k_gemm_ring<T, A_UNSIGNED, B_KMAJOR, RB, SLOTS>), dim3(tiles_m * tiles_n, g.batch), dim3(64 * WAVES), LDS, stream, MRL_WALK_ARGS(walk), g);
+  MRL_LAUNCH((k_gemm_ring<T, A_UNSIGNED, B_KMAJOR, RA, RB, SLOTS>), dim3(tiles_m * tiles_n, g.batch), dim3(64 * WAVES), LDS, stream, MRL_WALK_ARGS(walk), g);
   return plan::last_error();
 }
 
-template <class T, bool A_UNSIGNED, int RB, int SLOTS>
+template <class T, bool A_UNSIGNED, int RA, int RB, int SLOTS>
 hipError_t launch_either(const GemmArgs &g, hipStream_t stream) {
-  return g.b_kmajor ? launch_ring<T, A_UNSIGNED, true, RB, SLOTS>(g, stream) : launch_ring<T, A_UNSIGNED, false, RB, SLOTS>(g, stream);
+  return g.b_kmajor ? launch_ring<T, A_UNSIGNED, true, RA, RB, SLOTS>(g, stream) : launch_ring<T, A_UNSIGNED, false, RA, RB, SLOTS>(g, stream);
 }
 // As many slots as a compute unit's LDS holds of the wider ones, and four of the 64-wide tile's as well: all run one to a unit (of the
-// last, three / four / six: bf16 1024 x 7040 x 1344 35.7 / 33.2 / 33.4 us, 1664 x 6720 x 1152 34.6 / 33.0 / 33.2; of 128, five instead of four are within 1 %).
+// last, three / four / six: bf16 1024 x 7040 x 1344 35.7 / 33.2 / 33.4 us, 1664 x 6720 x 1152 34.6 / 33.0 / 33.2; of 128, five instead of four are within 1 %).  Four of the 64 x 64
+// tile, two of which share a unit (us, three / four / six / eight: bf16 192 x 768 x 384 4.74 / 4.81 / 4.9 / 5.2, 313 x 2176 x 267 twice 10.7 / 9.3 / 9.2 /
+// 9.5, u8 600 x 2496 x 236 7.3 / 7.3 / 7.6 / 7.9, 693 x 4352 x 817 11.9 / 10.8).
 template <class T, bool A_UNSIGNED>
 hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
   switch (bn) {
-    case 64: return launch_either<T, A_UNSIGNED, 2, 4>(g, stream);
-    case 128: return launch_either<T, A_UNSIGNED, 4, 4>(g, stream);
-    case 160: return launch_either<T, A_UNSIGNED, 5, 4>(g, stream);
-    case 192: return launch_either<T, A_UNSIGNED, 6, 4>(g, stream);
+    case 32: return launch_either<T, A_UNSIGNED, 2, 2, 4>(g, stream);
+    case 64: return launch_either<T, A_UNSIGNED, 4, 2, 4>(g, stream);
+    case 128: return launch_either<T, A_UNSIGNED, 4, 4, 4>(g, stream);
+    case 160: return launch_either<T, A_UNSIGNED, 4, 5, 4>(g, stream);
+    case 192: return launch_either<T, A_UNSIGNED, 4, 6, 4>(g, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -293,16 +295,16 @@ hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
 uint32_t gemm_ring_columns(const GemmArgs &g, int kind) {
   if (kind < 0 || kind > 2) return 0;
   const uint64_t es = kind == 2 ? 2 : 1, steps = (uint64_t(g.k) * es + STEP - 1) / STEP;
-  if (steps < (kind == 2 ? 13 : 14) || g.m <= 128 || g.n <= 128) return 0;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
-  const uint64_t units = g_compute_units, small = tiles(64, 64), whole = tiles(BM, 128);
+  const uint64_t units = g_compute_units, small = tiles(64, 64), whole = tiles(128, 128);
+  if (steps < (kind == 2 ? 13 : 14) || g.m <= 128 || g.n <= 128) return 0;
   if (small <= 512) {
     if (small <= units) return 0;
-    return tiles(BM, 64) <= units ? 64 : 2 * whole > units && steps >= 36 ? 128 : 0;
+    return tiles(128, 64) <= units ? 64 : 2 * whole > units && steps >= 36 ? 128 : 0;
   }
   if (whole <= units) return 2 * whole > units && steps >= 28 ? 128 : 0;
   if (steps < 16) return 0;
-  return tiles(BM, 160) <= units ? 160 : tiles(BM, 192) <= units ? 192 : 0;
+  return tiles(128, 160) <= units ? 160 : tiles(128, 192) <= units ? 192 : 0;
 }
 
 hipError_t launch_gemm_ring(const GemmArgs &g, int kind, uint32_t bn, hipStream_t stream) {

@@ -13,7 +13,7 @@
 //   - rows past M (or N) are the last one again, and a row-major B's last tile starts BN columns before B's end and
 //     leaves those its neighbour has: no load leaves the operands, and none is masked but the first step's.
 // What bounds it is the step's chain of barrier, operand reads and MFMAs, 0.25 to 0.33 us on the smallest tile (k_gemm's
-// step: 0.4 to 0.5), and past one workgroup a unit the cache lines that unaligned rows touch twice.
+// step: 0.4 to 0.5; gemm_ring.hip's, of whole chunks, 0.17 to 0.2), and past one workgroup a unit the cache lines that unaligned rows touch twice.
 // Everything else as in gemm_ring.hip.
 // Semantics: morello/src/spec.rs:480-485; integers exact, bf16 summed in f32.
 #include "gemm_ring_rows.h"

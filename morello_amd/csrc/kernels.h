@@ -197,13 +197,12 @@ hipError_t launch_sum_splits(const void *partial, void *c, uint32_t splits, uint
 // Always the 256 x 256 tile, 128 bytes of K per step.
 // staging: 0 = whichever of the 256 x 256 kernels applies (four waves, eight waves, compiler-scheduled),
 // 1 / 2 / 3 = mrl_staging's REGISTERS / DIRECT_B / DIRECT_B_WIDE only (hipErrorInvalidValue where that one does not apply).
-// gemm_ring.hip: tiles of 128 rows by `bn` (64, 128, 160 or 192) columns, operands straight into a ring of LDS slots; what
-// gemm_possible() takes with edge_addressable() leading dimensions.  gemm_ring_columns: the width for a problem, 0 for none.
+// gemm_ring.hip: tiles of 128 rows by `bn` (64, 128, 160 or 192) columns, or (32) of 64 x 64, operands straight into a ring of LDS slots; what
+// gemm_possible() takes with edge_addressable() leading dimensions.  gemm_ring_columns: the width for a problem, 0 for none; 32 is the caller's choice.
 uint32_t gemm_ring_columns(const GemmArgs &g, int kind);
 uint32_t gemm_goes_to_ring(const GemmArgs &g, int kind);   // its width where launch_gemm takes it, else 0
 hipError_t launch_gemm_ring(const GemmArgs &g, int kind, uint32_t bn, hipStream_t stream);
-// gemm_ring_rows.hip: such tiles for rows that start anywhere (K or N no whole 16-byte chunks), operands read in place; its
-// smallest, 64 x 64, is also the faster one for whole chunks.
+// gemm_ring_rows.hip: such tiles for rows that start anywhere (K or N no whole 16-byte chunks), operands read in place.
 // gemm_ring_rows_columns: the width of its tiles for a problem, 0 for none.
 uint32_t gemm_ring_rows_columns(const GemmArgs &g, int kind);
 hipError_t launch_gemm_ring_rows(const GemmArgs &g, int kind, hipStream_t stream);
