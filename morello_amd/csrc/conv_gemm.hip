@@ -1,10 +1,10 @@
 // Conv as an implicit Matmul on the matrix cores: the kernels of gemm_mfma_kernel.h and of
-// gemm_ring_rows.h with their left operand addressed as the windows of a channels-last image (the CONV build) and the KRSC
+// gemm_ring_tile.h with their left operand addressed as the windows of a channels-last image (the CONV build) and the KRSC
 // filters as a B operand stored k-fastest.  Takes any Conv whose channel vectors are whole
 // 16-byte chunks (morello/src/spec.rs:486-494: no stride, no padding); nothing is unfolded in
 // memory.  Its own translation unit so that the instantiations compile beside the others.
 #include "gemm_mfma_kernel.h"
-#include "gemm_ring_rows.h"
+#include "gemm_ring_tile.h"
 
 namespace mrl {
 namespace {
@@ -19,19 +19,20 @@ hipError_t launch_for(const GemmArgs &g, uint32_t tile, hipStream_t stream) {
   return launch<T, A_UNSIGNED, TileBig, true, true, true>(g, stream);
 }
 
-// The tiles of gemm_ring_rows.h on windows: 32 RA pixels by 32 RB filters on eight waves, two to a SIMD, each with half of every step.
-template <class T, bool A_UNSIGNED, int RA, int RB, bool CONV>
+// The tiles of gemm_ring_tile.h on windows: 32 RA pixels by 32 RB filters on eight waves, two to a SIMD, each with half of every step.
+template <class T, bool A_UNSIGNED, int RA, int RB, bool CONV, int SLOTS>
 __global__ __launch_bounds__(64 * ring::WAVES, RA * RB <= 8 ? 4 : 2) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   MRL_WALK_TILE(tile_m, tile_n)
-  ring::rows_tile<T, A_UNSIGNED, true, RA, RB, CONV>(lds, tile_m, tile_n, g);
+  ring::ring_tile<T, A_UNSIGNED, true, RA, RB, SLOTS, CONV>(lds, tile_m, tile_n, g);
 }
-template <class T, bool A_UNSIGNED, int RA, int RB, bool CONV = true>
+template <class T, bool A_UNSIGNED, int RA, int RB, bool CONV, int SLOTS>
 hipError_t launch_ring_tile(const GemmArgs &g, hipStream_t stream) {
-  constexpr int BM = 32 * RA, BN = 32 * RB, LDS = std::max(2 * (BM + BN) * ring::STEP, 4 * 16 * RA * (16 * RB + 4) * 4);
+  constexpr int BM = 32 * RA, BN = 32 * RB, LDS = SLOTS * (BM + BN) * ring::STEP;
+  static_assert(LDS >= 4 * 16 * RA * (16 * RB + 4) * 4, "the waves' pieces of C fit");
   static std::atomic<uint64_t> lds_limit_set{0};
   if (!plan::recording() && LDS > 65536) {
-    hipError_t e = raise_lds_limit(lds_limit_set, (const void *)k_gemm<T, A_UNSIGNED, RA, RB, CONV>, LDS);
+    hipError_t e = raise_lds_limit(lds_limit_set, (const void *)k_gemm<T, A_UNSIGNED, RA, RB, CONV, SLOTS>, LDS);
     if (e != hipSuccess) return e;
   }
   const int tiles_m = int((g.m + BM - 1) / BM), tiles_n = int((g.n + BN - 1) / BN);
@@ -40,26 +41,29 @@ hipError_t launch_ring_tile(const GemmArgs &g, hipStream_t stream) {
              double(g.conv.image_bytes) + double(g.n) * (g.k_total ? g.k_total : g.k) * T::ES + mn * 4 * (g.accum ? 2 : 1),
              2.0 * BM * BN * steps * (ring::STEP / T::ES), 2500.0 + 300.0 * steps);
   const TileWalk walk = gemm::tile_walk(tiles_m, tiles_n);
-  MRL_LAUNCH((k_gemm<T, A_UNSIGNED, RA, RB, CONV>), dim3(tiles_m * tiles_n, g.batch), dim3(64 * ring::WAVES), LDS, stream, MRL_WALK_ARGS(walk), g);
+  MRL_LAUNCH((k_gemm<T, A_UNSIGNED, RA, RB, CONV, SLOTS>), dim3(tiles_m * tiles_n, g.batch), dim3(64 * ring::WAVES), LDS, stream, MRL_WALK_ARGS(walk), g);
   return plan::last_error();
 }
 
 // Where those tiles are the faster ones.  A launch's time is taken as a fixed part and, for every round of its workgroups over the compute
 // units, the steps of a workgroup (128 bytes of the windows).  Measured (us; a step and round, int8 / bf16):
-//   these tiles: 64 x 32 3.5 + 0.26 / 0.24, 64 x 64 3.5 + 0.26 / 0.25, 128 x 32 4 + 0.30 / 0.29, 128 x 64 4.5 + 0.43 / 0.33, 128 x 128 5.5 +
-//     0.66 / 0.53, 128 x 192 6.5 + 0.89 / 0.70,
+//   these tiles: 64 x 32 3.5 + 0.25 / 0.24 (a single round 0.18 / 0.13), 64 x 64 3.5 + 0.26 / 0.25 (0.22 / 0.15), 128 x 32 4 + 0.30 / 0.29, 128 x 64 4.5 + 0.31 /
+//     0.32 (a single round of bf16 0.25), 128 x 128 5.5 + 0.48 / 0.50, 128 x 192 6.5 + 0.66 / 0.67,
 //   k_gemm's: 64 3.5 + 0.30 / 0.245, 128 4 + 0.69 / 0.57, 256 5 + 2.15 / 1.83;
-// past the third round those of which several share a unit even out the last one.  (us, k_gemm / this: bf16 12 x (352 -> 192) x 68^2 5 x 5 265.7 /
-// 190.5, u8 18 x (272 -> 192) x 42^2 5 x 5 101.9 / 55.2, bf16 7 x (288 -> 16) x 58^2 5 x 5 55.9 / 36.1, 29 x (224 -> 48) x 58^2 3 x 3 57.1 / 42.5, 11 x (144 -> 208) x
-// 14^2 3 x 3 10.3 / 7.5, u8 5 x (192 -> 224) x 10^2 8.4 / 7.0; over 200 random layers 1.08 times as fast, geometric mean.)
+// past the third round those of which several share a unit even out the last one.  What bounds a single round is the wait for what the step after next
+// asked of memory, past one the way into LDS.  (us, k_gemm / this: bf16 12 x (352 -> 192) x 68^2 5 x 5 265.7 / 190.5, u8 18 x (272 -> 192) x 42^2 5 x 5 101.9 /
+// 55.2, 9 x (224 -> 304) x 27^2 5 x 5 33.0 / 27.1, 5 x (144 -> 112) x 64^2 5 x 5 23.1 / 19.4, bf16 11 x (144 -> 208) x 14^2 3 x 3 10.3 / 7.5.  Windows by way of
+// registers, two slots of LDS / straight to LDS, three or four: bf16 21 x (144 -> 64) x 17^2 3 x 3 7.5 / 6.4, 2 x (96 -> 48) x 69^2 6.3 / 5.6, u8 31 x (240 -> 144) x
+// 14^2 5 x 5 23.2 / 19.6, 1 x (64 -> 48) x 21^2 5 x 5 6.1 / 5.7; over 140 random layers 1.035 times as fast, no one slower.)
 // Up to three steps, two of them what the start of a workgroup fetches, and up to seven past one round, k_gemm's start is the shorter one: u8 4 x
-// (16 -> 176) x 57^2 3 x 3, two steps, 5.7 / 7.4; 28 x (48 -> 336) x 11^2, four, 318 tiles, 5.7 / 6.3.
+// (16 -> 176) x 57^2 3 x 3, two steps, 5.7 / 7.4; 28 x (48 -> 336) x 11^2, four, 318 tiles, 5.7 / 6.3.  But for its 256 x 256 tile, whose end is the longer one:
+// 7 x (16 -> 272) x 72^2 3 x 3, two steps, 27.6 / 19.1, bf16 17 x (16 -> 176) x 70^2 5 x 5, seven, 36.6 / 28.7.
 enum Tiles : uint32_t { SQUARE, T64x32, T64x64, T128x32, T128x64, T128x128, T128x192 };
 Tiles choose_tiles(const GemmArgs &g, int kind) {
   if (kind > 2) return SQUARE;
   const uint64_t es = kind == 2 ? 2 : 1, step = ring::STEP, steps = (uint64_t(g.k) * es + step - 1) / step;
   const uint64_t last = g.k_total != 0 ? g.k_total - uint64_t(g.batch - 1) * g.k : g.k;
-  if (last * es <= step) return SQUARE;   // (rows_tile wants two steps)
+  if (last * es <= step) return SQUARE;   // (a step has no successor to fetch)
   const uint64_t units = g_compute_units;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
   const uint64_t small = tiles(64, 64);
@@ -68,7 +72,8 @@ Tiles choose_tiles(const GemmArgs &g, int kind) {
     // (two columns of 32 for up to 48 filters where the chip has room for both: u8 3 x (272 -> 48) x 8^2 5 x 5 8.7 / 7.7)
     return g.n <= 32 || (g.n <= 48 && 2 * small <= units) ? T64x32 : T64x64;
   }
-  if (g.batch > 1 || steps < 8) return SQUARE;   // (slices three to a unit: bf16 26 x (336 -> 80) x 11^2 in six 13.5 / 14.4)
+  const uint32_t side = gemm_tile_side(g, kind);
+  if (g.batch > 1 || (steps < 8 && side != 256)) return SQUARE;   // (slices three to a unit: bf16 26 x (336 -> 80) x 11^2 in six 13.5 / 14.4)
   const bool i8 = kind != 2;
   auto us = [&](uint32_t bm, uint32_t bn, bool shared, double fixed, double step_us) {
     const double r = double(tiles(bm, bn)) / double(units), whole = double((tiles(bm, bn) + units - 1) / units);
@@ -81,16 +86,15 @@ Tiles choose_tiles(const GemmArgs &g, int kind) {
   };
   if (g.n <= 32) {
     consider(T128x32, us(128, 32, true, 4.0, i8 ? 0.30 : 0.29));
-    consider(T64x32, us(64, 32, true, 3.5, (i8 ? 0.26 : 0.24) * (tiles(64, 32) > 3 * units ? 0.8 : 1.0)));
+    consider(T64x32, us(64, 32, true, 3.5, (i8 ? 0.25 : 0.24) * (tiles(64, 32) > 3 * units ? 0.8 : 1.0)));
   } else {
     if (g.n <= 64) consider(T64x64, us(64, 64, true, 3.5, i8 ? 0.26 : 0.25));
-    consider(T128x64, us(128, 64, true, 4.5, (i8 ? 0.43 : 0.33) * (tiles(128, 64) > 2 * units ? 1.08 : 1.0)));
+    consider(T128x64, us(128, 64, true, 4.5, (i8 ? 0.31 : tiles(128, 64) > units ? 0.32 : 0.25) * (tiles(128, 64) > 2 * units ? 1.08 : 1.0)));
     if (g.n > 64 && steps >= 12) {
-      consider(T128x128, us(128, 128, false, 5.5, i8 ? 0.66 : 0.53));
-      consider(T128x192, us(128, 192, false, 6.5, i8 ? 0.89 : 0.70));
+      consider(T128x128, us(128, 128, false, 5.5, i8 ? 0.48 : 0.50));
+      consider(T128x192, us(128, 192, false, 6.5, i8 ? 0.66 : 0.67));
     }
   }
-  const uint32_t side = gemm_tile_side(g, kind);
   const double square = side == 64    ? us(64, 64, true, 3.5, i8 ? 0.30 : 0.245)
                         : side == 128 ? us(128, 128, true, 4.0, (i8 ? 0.69 : 0.57) * (tiles(128, 128) > units ? 0.87 : 1.0))
                                       : us(256, 256, false, 5.0, i8 ? 2.15 : 1.83);
@@ -100,12 +104,12 @@ Tiles choose_tiles(const GemmArgs &g, int kind) {
 template <class T, bool A_UNSIGNED>
 hipError_t launch_tiles(const GemmArgs &g, Tiles tiles, hipStream_t stream) {
   switch (tiles) {
-    case T64x32: return launch_ring_tile<T, A_UNSIGNED, 2, 1>(g, stream);
-    case T64x64: return launch_ring_tile<T, A_UNSIGNED, 2, 2>(g, stream);
-    case T128x32: return launch_ring_tile<T, A_UNSIGNED, 4, 1>(g, stream);
-    case T128x64: return launch_ring_tile<T, A_UNSIGNED, 4, 2>(g, stream);
-    case T128x128: return launch_ring_tile<T, A_UNSIGNED, 4, 4>(g, stream);
-    default: return launch_ring_tile<T, A_UNSIGNED, 4, 6>(g, stream);
+    case T64x32: return launch_ring_tile<T, A_UNSIGNED, 2, 1, true, 4>(g, stream);
+    case T64x64: return launch_ring_tile<T, A_UNSIGNED, 2, 2, true, 4>(g, stream);
+    case T128x32: return launch_ring_tile<T, A_UNSIGNED, 4, 1, true, 4>(g, stream);
+    case T128x64: return launch_ring_tile<T, A_UNSIGNED, 4, 2, true, 3>(g, stream);
+    case T128x128: return launch_ring_tile<T, A_UNSIGNED, 4, 4, true, 4>(g, stream);
+    default: return launch_ring_tile<T, A_UNSIGNED, 4, 6, true, 4>(g, stream);
   }
 }
 

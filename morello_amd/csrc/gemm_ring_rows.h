@@ -1,4 +1,4 @@
-// The tile of gemm_ring_rows.hip: rows that start anywhere, or (CONV) the windows of a channels-last image.
+// The tile of gemm_ring_rows.hip: rows that start anywhere.
 #pragma once
 #include "gemm_ring.h"
 
@@ -18,28 +18,24 @@ __device__ inline v4i first_bytes(v4i v, int left) {
   return v;
 }
 
-// CONV (with B_KMAJOR): row p of A is the window of output pixel p, fh runs of fw * c contiguous elements of the image, whole 16-byte chunks each.
-template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RA, int RB, bool CONV = false>
+template <class T, bool A_UNSIGNED, bool B_KMAJOR, int RA, int RB>
 __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_t tile_n, const GemmArgs &g) {
-  static_assert(!CONV || B_KMAJOR, "");
   typedef typename Ring<T>::Acc Acc;
   constexpr int ES = T::ES, BK = STEP / ES, BM = 32 * RA, BN = 32 * RB, WM = 16 * RA, WN = 16 * RB;
   constexpr int A_BYTES = BM * STEP, B_BYTES = BN * STEP, SLOT = A_BYTES + B_BYTES;
   constexpr int A_LOADS = A_BYTES / (1024 * WAVES), B_LOADS = (B_BYTES / 1024 + WAVES - 1) / WAVES, LOADS = A_LOADS + B_LOADS;   // a wave's, per step
   // The k loop in pairs of steps and one more.  With an exit between the two, the other form, the compiler sees a way from the first to itself and makes
-  // it wait for all but half a step's loads: less code, and as good as or better than two whole steps under way for small tiles of windows (u8
-  // 10 x (16 -> 224) x 10^2 5 x 5, five steps: 4.5 us, in pairs 4.7) and for rows on 128 x 128 tiles and, of int8 along K, wider ones (u8 726 x 996 x 4035
-  // 12.9 / 13.4, 2432 x 1702 x 2069 25.2 / 25.6).  Else worse: bf16 33 x 1664 x 12928 10.6 / 9.3, 138 x 699 x 368 6.6 / 6.2, 394 x 139 x 145 5.0 / 4.5,
-  // 8 x (256 -> 256) x 28^2 3 x 3 15.6 / 14.8.
-  constexpr bool PAIRS = CONV ? RA * RB > 4 : RB < 4 || (RB > 4 && !(ES == 1 && B_KMAJOR));
+  // it wait for all but half a step's loads: less code, and as good as or better than two whole steps under way on 128 x 128 tiles and, of int8 along K,
+  // wider ones (u8 726 x 996 x 4035 12.9 / 13.4, 2432 x 1702 x 2069 25.2 / 25.6).  Else worse: bf16 138 x 699 x 368 6.6 / 6.2, 394 x 139 x 145 5.0 / 4.5.
+  constexpr bool PAIRS = RB < 4 || (RB > 4 && !(ES == 1 && B_KMAJOR));
   // Steps of loads under way (four to eight, on the smallest tile: 4 to 13 % slower, more to wait for at the start and nothing gained behind it).  In
   // pairs on the widest tiles rows of any alignment lose by the second (bf16 2306 x 735 x 2260 17.3 us, with one 17.0; 3456 x 1909 x 1221 32.9 / 32.4).
-  constexpr int DEPTH = !CONV && PAIRS && RB >= 5 ? 1 : 2;
+  constexpr int DEPTH = PAIRS && RB >= 5 ? 1 : 2;
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kw = wave >> 2, wm = wave >> 1 & 1, wn = wave & 1;
   const int64_t m0 = int64_t(tile_m) * BM, n_tile = int64_t(tile_n) * BN;
   const int64_t n0 = B_KMAJOR ? n_tile : min(n_tile, int64_t(g.n) - BN);
-  const uint8_t *A = (const uint8_t *)g.a + (CONV ? 0 : (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES);
+  const uint8_t *A = (const uint8_t *)g.a + (int64_t(blockIdx.y) * g.sa + m0 * g.lda) * ES;
   const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : n0)) * ES;
   const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = uint32_t(g.ldb) * ES;
   const int a_last = min(BM, int(g.m - m0)) - 1, b_last = min(BN, int(g.n - n0)) - 1;
@@ -55,13 +51,7 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
 #pragma unroll
   for (int i = 0; i < A_LOADS; i++) {
     const int load = wave * A_LOADS + i;
-    const int row = min(load * ROWS_PER_LOAD + row16, a_last);
-    if constexpr (CONV) {
-      const uint32_t p = uint32_t(m0) + row, line = g.conv.by_ow.div(p), img = g.conv.by_oh.div(line);
-      off[i] = ((img * g.conv.h + (line - img * g.conv.oh)) * g.conv.w + (p - line * g.conv.ow)) * g.conv.c_bytes;
-    } else {
-      off[i] = uint32_t(row) * lda_b + chunk_of(load) * 16;
-    }
+    off[i] = uint32_t(min(load * ROWS_PER_LOAD + row16, a_last)) * lda_b + chunk_of(load) * 16;
     dst[i] = load * 1024 + lane * 16;
     whole[i] = head * ES - chunk_of(load) * 16;
   }
@@ -81,34 +71,20 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
   }
   const global_u8 *a_tile = (const global_u8 *)A, *b_tile = (const global_u8 *)B;
   const int64_t b_step = B_KMAJOR ? int64_t(STEP) : int64_t(BK) * ldb_b;
-  // CONV: where the chunks of the step to load lie in a window, from its corner on; the step's first byte of the window.
-  uint32_t in_window[A_LOADS];
-  uint32_t window_byte = CONV ? blockIdx.y * g.conv.slice_bytes : 0;
-  auto find_chunk = [&](auto which) {
-    constexpr int I = decltype(which)::value;
-    const uint32_t kb = window_byte + chunk_of(wave * A_LOADS + I) * 16;
-    in_window[I] = kb + g.conv.by_run.div(kb) * g.conv.run_gap;
-    asm("" : "+v"(in_window[I]));   // here, and not behind the next barrier
-  };
   auto load = [&](auto which) {
     constexpr int I = decltype(which)::value;
-    if constexpr (CONV && I < A_LOADS) return __builtin_bit_cast(v4i, *(const global_chunk *)(a_tile + (off[I] + in_window[I])));
-    else return __builtin_bit_cast(v4i, *(const global_chunk *)((I < A_LOADS ? a_tile : b_tile) + off[I]));
+    return __builtin_bit_cast(v4i, *(const global_chunk *)((I < A_LOADS ? a_tile : b_tile) + off[I]));
   };
   int behind = steps;   // steps from the one that the pointers are at on
   // To the next one (past the last: nowhere); `first`: from the first step, which has `head` elements.
   auto advance = [&](auto first) {
     const bool more = --behind > 0;
     const int a_step = !more ? 0 : decltype(first)::value ? head * ES : STEP;
-    if constexpr (CONV) window_byte += a_step;
-    else {
-      a_tile += a_step;
-      if constexpr (PAIRS) asm("" : "+s"(a_tile));   // (scalar bases, not sums of each lane's)
-    }
+    a_tile += a_step;
+    if constexpr (PAIRS) asm("" : "+s"(a_tile));   // (scalar bases, not sums of each lane's)
     b_tile += !more ? 0 : !decltype(first)::value ? b_step : B_KMAJOR ? int64_t(head) * ES : int64_t(head) * ldb_b;
     if constexpr (PAIRS) asm("" : "+s"(b_tile));
   };
-  if constexpr (CONV) each<A_LOADS>([&](auto i) { find_chunk(i); });
 
   // Operand addresses within a slot: lane (l % 16, l / 16) takes the l / 16-th 16 bytes of row l % 16.
   const int in_rows = li * STEP + (((4 * kw + lg) ^ (li / ROWS_PER_LINE % CHUNKS)) << 4);
@@ -171,7 +147,6 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
         kept[K][I] = load(std::integral_constant<int, I>{});
       });
       if constexpr (Q == N - 1) advance(std::false_type{});
-      if constexpr (CONV && Q == N - 1) each<A_LOADS>([&](auto i) { find_chunk(i); });
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -181,7 +156,6 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
       each<LOADS>([&](auto i) { first[decltype(s)::value][decltype(i)::value] = load(i); });
       if constexpr (PAIRS) __builtin_amdgcn_sched_barrier(0);
       advance(std::integral_constant<bool, decltype(s)::value == 0>{});
-      if constexpr (CONV) each<A_LOADS>([&](auto i) { find_chunk(i); });
     });
     each<DEPTH>([&](auto s) {
       each<LOADS>([&](auto i) {
@@ -189,7 +163,6 @@ __device__ __forceinline__ void rows_tile(uint8_t *lds, uint32_t tile_m, uint32_
         if constexpr (PAIRS) __builtin_amdgcn_sched_barrier(0);   // in this order, which the loop's waits count on
       });
       advance(std::false_type{});
-      if constexpr (CONV) each<A_LOADS>([&](auto i) { find_chunk(i); });
     });
 #pragma unroll
     for (int i = 0; i < LOADS; i++) {

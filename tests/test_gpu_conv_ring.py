@@ -82,3 +82,13 @@ def test_windows_on_ring_tiles_and_on_squares_agree(gpu, types, shape):
     for x in bufs:
         x.free()
     assert np.array_equal(got, other) if dts[2] == M.i32 else np.allclose(got, other, rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("types,shape,tiles", [
+    ("u8", [7, 272, 16, 72, 72, 3, 3], "RA = 4, RB = 2"),     # two steps, the second an eighth full; 256 x 256 tiles otherwise
+    ("i8", [9, 258, 48, 61, 67, 1, 3], "RA = 4, RB = 2"),     # filters lower than wide, two past a tile
+    ("u8", [1, 48, 64, 21, 21, 5, 5], "RA = 2, RB = 1"),
+    ("bf16", [21, 61, 144, 17, 17, 3, 3], "RA = 2, RB = 2"),  # the last row of tiles 53 pixels, its last column 61 filters
+])
+def test_windows_straight_into_lds(gpu, types, shape, tiles):
+    test_windows_on_ring_tiles(gpu, types, shape, tiles, 1, True)
