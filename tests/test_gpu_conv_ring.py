@@ -1,4 +1,4 @@
-"""Conv as an implicit Matmul on the tiles of gemm_ring_rows.h (conv_gemm.hip), against float64."""
+"""Conv as an implicit Matmul on the tiles of gemm_ring_tile.h (conv_gemm.hip), against float64."""
 import numpy as np
 import pytest
 
