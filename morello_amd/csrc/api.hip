@@ -496,8 +496,8 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   // u8 1144 x 3952 x 672 16.2 / 13.6, bf16 221 x 1824 x 624 twice 12.9 / 11.2; up to eight steps they are even), unless K falls
   // into equal slices, of which k_gemm's may go three to a compute unit (bf16 1721 x 4416 x 304 15.4 / 21.0), or is long beside
   // int8 rows of N, of which a step takes half lines (139 x 4080 x 2288 twice 22.6 / 23.5).
-  // Rows of whole chunks take that tile by way of LDS alone (gemm_ring.hip), which is the faster one throughout (us, through registers / this: bf16 1024^3 8.0 / 7.0, 86 x
-  // 2144 x 262 twice 12.4 / 10.5, 33 x 1664 x 12928 10.7 / 9.4, u8 693 x 4352 x 817 14.2 / 10.8, 51 x 1600 x 9152 7.4 / 6.2, 1383 x 5744 x 184 in three slices 12.3 / 11.5; over 60
+  // Rows of whole chunks take that tile by way of LDS alone (gemm_ring.hip), which is the faster one throughout (us, through registers / this: bf16 1024^3 8.0 / 7.0, 33 x
+  // 1664 x 12928 10.7 / 9.4, k-fastest B: 86 x 2144 x 262 twice 12.4 / 10.5, u8 693 x 4352 x 817 14.2 / 10.8, 51 x 1600 x 9152 7.4 / 6.2; 1383 x 5744 x 184 in three slices 12.3 / 11.5; over 60
   // random sizes 1.13 times as fast) and faster than k_gemm's from six steps on (192 x 896 x 320 5.05 / 4.55, 384 x 448 x 192 4.6 / 4.2, int8 rows of N over a long K too, 1144 x
   // 3952 x 672 16.9 / 13.7, 615 x 5760 x 112 twice 21.5 / 13.1), bf16 rows of N from nine (422 x 448 x 880 twice, seven, 5.3 / 5.6; 1005 x 576 x 336 5.2 / 4.7).
   const int64_t chunk = 16 / int64_t(a.elem);

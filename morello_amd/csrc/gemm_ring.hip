@@ -65,7 +65,7 @@ hipError_t launch_either(const GemmArgs &g, hipStream_t stream) {
 // As many slots as a compute unit's LDS holds of the wider ones, and four of the 64-wide tile's as well: all run one to a unit (of the
 // last, three / four / six: bf16 1024 x 7040 x 1344 35.7 / 33.2 / 33.4 us, 1664 x 6720 x 1152 34.6 / 33.0 / 33.2; of 128, five instead of four are within 1 %).  Four of the 64 x 64
 // tile, two of which share a unit (us, three / four / six / eight: bf16 192 x 768 x 384 4.74 / 4.81 / 4.9 / 5.2, 313 x 2176 x 267 twice 10.7 / 9.3 / 9.2 /
-// 9.5, u8 600 x 2496 x 236 7.3 / 7.3 / 7.6 / 7.9, 693 x 4352 x 817 11.9 / 10.8).
+// 9.5, u8 600 x 2496 x 236 7.3 / 7.3 / 7.6 / 7.9, 693 x 4352 x 817 with a k-fastest B 11.9 / 10.8).
 template <class T, bool A_UNSIGNED>
 hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
   switch (bn) {
