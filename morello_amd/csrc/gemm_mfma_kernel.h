@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "tile_bounds.h"
 
 
 namespace mrl {
@@ -333,7 +334,7 @@ __device__ inline void sched_slots(bool staging) {
 // epilogue stay free of branches.  A chunk that straddles the end of K brings along the bytes
 // between the row's end and its leading dimension: the caller keeps those zero (they are its
 // own padding whenever K is not a whole number of chunks).  Chunks to the right of B's last
-// column hold whatever follows in memory: they only reach columns of C that are not stored.
+// column hold the rows that follow, or zeros behind the last row: they only reach columns of C that are not stored.
 // B_KMAJOR: B is stored with k fastest (each of its n rows runs along K, `ldb` elements apart:
 // Morello's col_major / batched_col_major layouts, or layout![0,2,1]).  Its tile is then staged
 // and read exactly like A's, and no transposing read is involved.
@@ -440,7 +441,7 @@ __global__ __launch_bounds__(TL::NT) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
   // out-of-range offset instead.
   const int k_bytes = k * ES;
   const uint8_t *a_tile = A, *b_tile = B;
-  const int a_rows = min(BM, int(g.m - m0)), b_rows = min(BN, int(g.n - n0));  // rows the tile owns
+  const int a_rows = min(BM, int(g.m - m0)), b_rows = min(BN, int(g.n - n0));  // rows (of a row-major B: columns) the tile owns
   const uint32_t a_off = uint32_t(tid / A_ROW_CH) * uint32_t(lda_b) + (tid % A_ROW_CH) * 16;
   // CONV: byte offset of the window corner of each of the thread's rows (out of range past M).
   uint32_t a_corner[A_CH];
@@ -485,8 +486,8 @@ __global__ __launch_bounds__(TL::NT) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
           b_reg[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
                                                  b_buf, b_in ? b_off + i * uint32_t(b_step_i) : OUT_OF_RANGE, 0, 0));
       } else {
-        // k rows left from this tile's first on, each up to its leading dimension.
-        const auto b_buf = buffer_of(b_tile, (int64_t(g.k) - ld_kb / ES) * ldb_b - n0 * ES);
+        // k rows left from this tile's first on (none: a size below one).
+        const auto b_buf = buffer_of(b_tile, tile_bytes(int64_t(g.k) - ld_kb / ES, ldb_b, b_rows * ES));
 #pragma unroll
         for (int i = 0; i < B_CH; i++)
           b_reg[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(

@@ -1,6 +1,7 @@
 // The tile of gemm_ring.hip: rows of whole 16-byte chunks, or (CONV) the windows of a channels-last image of such pixels.
 #pragma once
 #include "gemm_ring.h"
+#include "tile_bounds.h"
 
 namespace mrl {
 namespace ring {
@@ -47,9 +48,10 @@ __device__ __forceinline__ void ring_tile(uint8_t *lds, uint32_t tile_m, uint32_
   const bool panels = !B_KMAJOR && g.b_panel_rows != 0;
   const uint8_t *B = (const uint8_t *)g.b + (int64_t(blockIdx.y) * g.sb + (B_KMAJOR ? n0 * g.ldb : panels ? n0 * g.b_panel_rows : n0)) * ES;
   const uint32_t lda_b = uint32_t(g.lda) * ES, ldb_b = panels ? BN * ES : uint32_t(g.ldb) * ES;
-  // Bytes of the tile's rows (leading dimensions stay below 2^24 bytes); what of a row-major B's lies left of the tile.
-  const int a_end = min(BM, int(g.m - m0)) * int(lda_b), n0_b = panels ? 0 : int(n0) * ES;
-  const uint32_t b_end = uint32_t(min(BN, int(g.n - n0))) * ldb_b;
+  // Bytes of the tile's rows (leading dimensions stay below 2^24 bytes); of `rows` rows of a row-major B (tile_bounds.h).
+  const int a_end = min(BM, int(g.m - m0)) * int(lda_b), n_left = min(BN, int(g.n - n0));
+  const uint32_t b_end = uint32_t(n_left) * ldb_b;
+  auto b_rows = [&](int rows) { return uint32_t(tile_bytes(rows, ldb_b, n_left * ES)); };
   const int k = g.k_total != 0 ? int(min(g.k, g.k_total - blockIdx.y * g.k)) : int(g.k), k_bytes = k * ES, steps = (k_bytes + STEP - 1) / STEP;
 
   // Where this lane's chunks of a step come from.  Rows of 64 bytes: sixteen to a load.
@@ -87,7 +89,7 @@ __device__ __forceinline__ void ring_tile(uint8_t *lds, uint32_t tile_m, uint32_
   // Where the step to request starts: the resources' bases.  Their sizes do not change from step to step (an offset past them is a
   // row's that does not exist), but for the steps that hold K's end and lie behind it.
   uint64_t a_tile = reinterpret_cast<uintptr_t>(A) - 4096, b_tile = reinterpret_cast<uintptr_t>(B) - 4096;
-  uint32_t a_bytes = (CONV ? uint32_t(g.conv.image_bytes) : uint32_t(a_end)) + 4096, b_bytes = (B_KMAJOR ? b_end : uint32_t(BK) * ldb_b - n0_b) + 4096;
+  uint32_t a_bytes = (CONV ? uint32_t(g.conv.image_bytes) : uint32_t(a_end)) + 4096, b_bytes = (B_KMAJOR ? b_end : b_rows(BK)) + 4096;
   int left = k_bytes;   // of K from the step to request on
   const uint32_t a_dst = lds0 + wave * (A_LOADS * 1024), b_dst = lds0 + A_BYTES;
   uint32_t fill = 0;   // the slot that it goes to
@@ -98,7 +100,7 @@ __device__ __forceinline__ void ring_tile(uint8_t *lds, uint32_t tile_m, uint32_
       a_bytes = b_bytes = 0;
       return;
     }
-    if constexpr (!B_KMAJOR) b_bytes = uint32_t(left / ES) * ldb_b - n0_b + 4096;
+    if constexpr (!B_KMAJOR) b_bytes = b_rows(left / ES) + 4096;
     if constexpr (!CONV) each<A_LOADS>([&](auto i) { a_off[i] = chunk_of(i) * 16 >= left ? OUTSIDE : a_off[i]; });
     if constexpr (B_KMAJOR) each<B_LOADS>([&](auto i) { b_off[i] = (chunk ^ (b_load(i) * ROWS_PER_LOAD / ROWS_PER_LINE % CHUNKS)) * 16 >= left ? OUTSIDE : b_off[i]; });
   };
