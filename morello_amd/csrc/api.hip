@@ -273,6 +273,11 @@ void *g_scratch_ptr[MAX_DEVICES] = {};
 // Whether this thread's call makes the smallest copies there are (rows padded to 16 bytes and not to whole cache
 // lines, short columns turned) and no partial results of uneven slices or shares of keys: mrl_run_noalloc, for a Spec whose scratch does not fit otherwise.
 thread_local bool g_tight_scratch = false;
+// And before that, for one whose scratch fits but for the columns that panels round a right operand's copy up by: copies as plain rows.
+thread_local bool g_copies_in_panels = true, g_made_panels = false;   // (the latter: since it was last cleared)
+struct ScratchChoices {   // for one call
+  ~ScratchChoices() { g_tight_scratch = false, g_copies_in_panels = true; }
+};
 
 struct Workspace {
   hipStream_t stream;
@@ -599,7 +604,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
     // 43.9, bf16 750 x 3001 x 2900 twice 52.6 / 50.7, 1100 x 4000 x 1101 30.7 / 29.8, 1001 x 2050 x 4425 33.3 / 33.1).
     const uint32_t b_rows_count = g.b_kmajor ? b_rows.shape[1] : end_whole ? whole_k : g.k;
     uint32_t panel = 0;
-    if (!g.b_kmajor && kind <= 2 && !g_tight_scratch && !walkable(b_rows) && as_rows(b_rows, &any_ld, &any_bs)) {
+    if (!g.b_kmajor && kind <= 2 && !g_tight_scratch && g_copies_in_panels && !walkable(b_rows) && as_rows(b_rows, &any_ld, &any_bs)) {
       mrl::GemmArgs then = g;
       then.a = a.t.ptr, then.b = nullptr, then.k = b_rows_count;
       then.ldb = rows_of(b_rows).stride[1], then.sb = int64_t(b_rows_count) * then.ldb;
@@ -609,6 +614,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
           mrl::gemm_k_splits(then, kind, &k_rest) == 1)
         panel = mrl::gemm_goes_to_ring(then, kind);
     }
+    if (panel != 0) g_made_panels = true;
     if ((rc = make_rows(b, b_rows, b_rows_count, panel, &b_padded)) != MRL_OK) return rc;
     if (end_whole && b_padded) g.k = whole_k;
     if (panel != 0 && b_padded) g.b_panel_rows = b_rows_count;
@@ -1835,6 +1841,29 @@ int mrl_run_async(const mrl_spec *spec, void *const *params, void *stream) {
   return run_async_impl(spec, params, (hipStream_t)stream);
 }
 
+}  // extern "C"
+
+// The first plan whose scratch fits the fixed array, or the one with the smallest copies; this thread's calls go by it until `ScratchChoices` ends.
+static int plan_for_fixed_scratch(const mrl_spec *spec, mrl_plan *plan, mrl_plan_step *steps = nullptr, uint32_t cap = 0) {
+  g_made_panels = false;
+  int rc = mrl_spec_plan(spec, plan, steps, cap);
+  if (rc == MRL_OK && plan->scratch_bytes > NOALLOC_SCRATCH_BYTES && g_made_panels) {
+    g_copies_in_panels = false;
+    rc = mrl_spec_plan(spec, plan, steps, cap);
+  }
+  if (rc == MRL_OK && plan->scratch_bytes > NOALLOC_SCRATCH_BYTES) {
+    g_tight_scratch = true;
+    rc = mrl_spec_plan(spec, plan, steps, cap);
+  }
+  return rc;
+}
+int mrl::noalloc_plan(const mrl_spec *spec, mrl_plan *plan, mrl_plan_step *steps, uint32_t cap) {
+  ScratchChoices until_return;
+  return plan_for_fixed_scratch(spec, plan, steps, cap);
+}
+
+extern "C" {
+
 int mrl_run_noalloc(const mrl_spec *spec, void *const *params, void *stream) {
   if (g_device < 0 || g_device >= MAX_DEVICES || !g_scratch_ptr[g_device]) {
     g_last_error = "mrl_run_noalloc: call mrl_init first (it looks up the device's scratch array)";
@@ -1863,15 +1892,9 @@ int mrl_run_noalloc(const mrl_spec *spec, void *const *params, void *stream) {
   }
   // What the call would take, from the plan (host arithmetic only), so that a Spec that does not
   // fit is turned down before anything is launched.
-  struct Tight {
-    ~Tight() { g_tight_scratch = false; }
-  } until_return;
+  ScratchChoices until_return;
   mrl_plan plan;
-  if ((rc = mrl_spec_plan(spec, &plan, nullptr, 0)) != MRL_OK) return rc;
-  if (plan.scratch_bytes > NOALLOC_SCRATCH_BYTES) {   // with the smallest copies
-    g_tight_scratch = true;
-    if ((rc = mrl_spec_plan(spec, &plan, nullptr, 0)) != MRL_OK) return rc;
-  }
+  if ((rc = plan_for_fixed_scratch(spec, &plan)) != MRL_OK) return rc;
   const std::string too_large = "mrl_run_noalloc: the Spec needs " + std::to_string(plan.scratch_bytes) +
                                 " bytes of scratch, the fixed array holds " + std::to_string(NOALLOC_SCRATCH_BYTES);
   if (plan.scratch_bytes > NOALLOC_SCRATCH_BYTES) {

@@ -341,4 +341,7 @@ hipError_t launch_attn(const AttnArgs &a, hipStream_t stream);
 hipError_t launch_attn_keys(const AttnArgs &a, hipStream_t stream);   // attention_keys.hip
 hipError_t launch_attn_merge(const AttnArgs &a, hipStream_t stream);
 
+// ---- api.hip: what mrl_run_noalloc would do ----
+int noalloc_plan(const mrl_spec *spec, mrl_plan *plan, mrl_plan_step *steps, uint32_t cap);
+
 }  // namespace mrl
