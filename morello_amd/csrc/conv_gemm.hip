@@ -48,7 +48,9 @@ hipError_t launch_ring_tile(const GemmArgs &g, hipStream_t stream) {
 // Where those tiles are the faster ones.  A launch's time is taken as a fixed part and, for every round of its workgroups over the compute
 // units, the steps of a workgroup (128 bytes of the windows).  Measured (us; a step and round, int8 / bf16):
 //   these tiles: 64 x 32 3.5 + 0.25 / 0.24 (a single round 0.18 / 0.13), 64 x 64 3.5 + 0.26 / 0.25 (0.22 / 0.15), 128 x 32 4 + 0.30 / 0.29, 128 x 64 4.5 + 0.31 /
-//     0.32 (a single round of bf16 0.25), 128 x 128 5.5 + 0.48 / 0.50, 128 x 192 6.5 + 0.66 / 0.67,
+//     0.32 (a single round of bf16 0.25), 128 x 128 5.5 + 0.48 / 0.50, 128 x 192 6.5 + 0.66 / 0.67; int8 past one round of the last two 0.66 and 0.89, to one and a half
+//     of 128 x 64 0.43, and the same beside the 256 x 256 tile: nothing is under way while a round's results leave, which a short int8 step does not make up for
+//     (u8 18 x (208 -> 240) x 71^2 3 x 3 74.5 / 91.3, 18 x (176 -> 192) x 79^2 65.1 / 73.1, 22 x (208 -> 64) x 46^2 15.6 / 17.7, 16 x (112 -> 160) x 55^2 20.8 / 25.1),
 //   k_gemm's: 64 3.5 + 0.30 / 0.245, 128 4 + 0.69 / 0.57, 256 5 + 2.15 / 1.83;
 // past the third round those of which several share a unit even out the last one.  What bounds a single round is the wait for what the step after next
 // asked of memory, past one the way into LDS.  (us, k_gemm / this: bf16 12 x (352 -> 192) x 68^2 5 x 5 265.7 / 190.5, u8 18 x (272 -> 192) x 42^2 5 x 5 101.9 /
@@ -57,7 +59,9 @@ hipError_t launch_ring_tile(const GemmArgs &g, hipStream_t stream) {
 // 14^2 5 x 5 23.2 / 19.6, 1 x (64 -> 48) x 21^2 5 x 5 6.1 / 5.7; over 140 random layers 1.035 times as fast, no one slower.)
 // Up to three steps, two of them what the start of a workgroup fetches, and up to seven past one round, k_gemm's start is the shorter one: u8 4 x
 // (16 -> 176) x 57^2 3 x 3, two steps, 5.7 / 7.4; 28 x (48 -> 336) x 11^2, four, 318 tiles, 5.7 / 6.3.  But for its 256 x 256 tile, whose end is the longer one:
-// 7 x (16 -> 272) x 72^2 3 x 3, two steps, 27.6 / 19.1, bf16 17 x (16 -> 176) x 70^2 5 x 5, seven, 36.6 / 28.7.
+// 7 x (16 -> 272) x 72^2 3 x 3, two steps, 27.6 / 19.1, bf16 17 x (16 -> 176) x 70^2 5 x 5, seven, 36.6 / 28.7.  Of int8 where that tile pads the filters half as much again
+// (without, 22 x (16 -> 176) x 114^2 3 x 3 61.4 / 84.4, 22 x (48 -> 208) x 40^2 15.3 / 19.1), and not for two steps past fourteen rounds, which the results bound
+// (27 x (16 -> 288) x 71^2 53.0 / 60.9).
 enum Tiles : uint32_t { SQUARE, T64x32, T64x64, T128x32, T128x64, T128x128, T128x192 };
 Tiles choose_tiles(const GemmArgs &g, int kind) {
   if (kind > 2) return SQUARE;
@@ -75,6 +79,7 @@ Tiles choose_tiles(const GemmArgs &g, int kind) {
   const uint32_t side = gemm_tile_side(g, kind);
   if (g.batch > 1 || (steps < 8 && side != 256)) return SQUARE;   // (slices three to a unit: bf16 26 x (336 -> 80) x 11^2 in six 13.5 / 14.4)
   const bool i8 = kind != 2;
+  if (i8 && steps < 8 && (16 * tiles(256, 256) <= 3 * tiles(128, 64) || (steps == 2 && tiles(128, 64) > 14 * units))) return SQUARE;
   auto us = [&](uint32_t bm, uint32_t bn, bool shared, double fixed, double step_us) {
     const double r = double(tiles(bm, bn)) / double(units), whole = double((tiles(bm, bn) + units - 1) / units);
     return fixed + double(steps) * step_us * (shared && r > 3.0 ? (r + whole) / 2 : whole);
@@ -89,10 +94,12 @@ Tiles choose_tiles(const GemmArgs &g, int kind) {
     consider(T64x32, us(64, 32, true, 3.5, (i8 ? 0.25 : 0.24) * (tiles(64, 32) > 3 * units ? 0.8 : 1.0)));
   } else {
     if (g.n <= 64) consider(T64x64, us(64, 64, true, 3.5, i8 ? 0.26 : 0.25));
-    consider(T128x64, us(128, 64, true, 4.5, (i8 ? 0.31 : tiles(128, 64) > units ? 0.32 : 0.25) * (tiles(128, 64) > 2 * units ? 1.08 : 1.0)));
+    const uint64_t t = tiles(128, 64);
+    const bool slow = (side == 256 && steps >= 8) || (t > units && 2 * t <= 3 * units);   // (int8)
+    consider(T128x64, us(128, 64, true, 4.5, (i8 ? (slow ? 0.43 : 0.31) : t > units ? 0.32 : 0.25) * (t > 2 * units ? 1.08 : 1.0)));
     if (g.n > 64 && steps >= 12) {
-      consider(T128x128, us(128, 128, false, 5.5, i8 ? 0.48 : 0.50));
-      consider(T128x192, us(128, 192, false, 6.5, i8 ? 0.66 : 0.67));
+      consider(T128x128, us(128, 128, false, 5.5, !i8 ? 0.50 : tiles(128, 128) > units ? 0.66 : 0.48));
+      consider(T128x192, us(128, 192, false, 6.5, !i8 ? 0.67 : tiles(128, 192) > units ? 0.89 : 0.66));
     }
   }
   const double square = side == 64    ? us(64, 64, true, 3.5, i8 ? 0.30 : 0.245)

@@ -1,0 +1,27 @@
+"""Which tiles the matrix-core kernels run on where two were measured against each other: sizes on both sides of a line.  No GPU needed."""
+import pytest
+
+import morello_amd as M
+
+TYPES = {"u8": (M.u8, M.i8, M.i32), "i8": (M.i8, M.i8, M.i32), "bf16": (M.bf16, M.bf16, M.f32)}
+
+
+@pytest.mark.parametrize("types,b,c,f,hw,fs,tile", [
+    ("u8", 22, 16, 176, 114, 3, "Tile<256, 256"),     # two steps; 256 x 256 pads the filters by 80, 128 x 64 by 16
+    ("u8", 22, 48, 208, 40, 3, "Tile<256, 256"),
+    ("u8", 7, 16, 272, 72, 3, "RA = 4, RB = 2"),      # ... by 240, 48
+    ("u8", 27, 16, 288, 71, 3, "Tile<256, 256"),      # two steps, twenty rounds of 128 x 64
+    ("u8", 27, 32, 288, 71, 3, "RA = 4, RB = 2"),     # three
+    ("bf16", 22, 16, 176, 60, 5, "RA = 4, RB = 2"),
+    ("u8", 16, 112, 160, 55, 3, "Tile<256, 256"),     # eight steps
+    ("u8", 18, 208, 240, 71, 3, "Tile<256, 256"),     # several rounds of 128 x 128
+    ("i8", 18, 176, 192, 79, 3, "Tile<256, 256"),     # ... of 128 x 192
+    ("u8", 5, 208, 96, 85, 5, "Tile<128, 128"),       # 283 tiles of 128 x 128
+    ("u8", 10, 288, 320, 28, 5, "RA = 4, RB = 4"),    # 186
+    ("u8", 22, 208, 64, 46, 3, "Tile<64, 64"),        # 364 tiles of 128 x 64
+    ("u8", 20, 208, 64, 40, 3, "RA = 4, RB = 2"),     # 250
+    ("u8", 26, 208, 64, 46, 3, "RA = 4, RB = 2"),     # 430
+])
+def test_windows(types, b, c, f, hw, fs, tile):
+    p = M.Conv([b, f, c, hw, hw, fs, fs], TYPES[types]).plan()
+    assert p.kernels == ["k_gemm"] and tile in p.steps[0].kernel, p
