@@ -92,6 +92,11 @@ hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
 //     (integers 35 to 44 1.08, bf16 45 on 1.22; 30 to 34 1.02 and from memory 0.95, 11 to 19 0.89);
 //   160, else 192, where the 128 tile needs a second round and they do not: bf16 1001 x 2050 x 4425 47.2 / 38.9, 1800 x 2001
 //     x 3000 41.0 / 35.3, u8 1000 x 2001 x 4500 34.6 / 30.1.  (128 in two rounds: 0.92 to 1.03, and 0.90 with operands from memory.)
+// Rows of K that are no whole cache lines, of which a step's 128 bytes lie in two, cost the 128-wide tile that much more than k_gemm's: i8 from 60 steps on, a
+// k-fastest bf16 B from 32, and where 64 x 64 tiles are 512 at most a k-fastest B of either not at all (one set of operands / three in turn / B from memory /
+// all of it, means: i8 below 60 0.97 / 0.96 / 0.96 / 0.93, from there 1.02 / 1.01 / 1.00 / 0.96, of whole lines 1.09 / 1.09 / 1.04 / 0.99; bf16 0.93 / 0.94 / 0.94 / 0.92,
+// of whole lines 1.09 / 1.09 / 1.04 / 1.00; i8 883 x 4928 x 2336 26.0 / 27.0, twice 792 x 3552 x 1760 21.7 / 24.6, bf16 twice 1109 x 1768 x 1504 21.1 / 23.5).  u8 pays k_gemm
+// for its columns' sums (1.04 / 1.04 / 1.03 / 1.00).  Where 128 x 128 pads much more than 64 x 64 the other choice is k_gemm's 64 tile, 1.8 times as slow.
 // Short K leaves the start of the ring and the summing of the two halves of K dominant: bf16 1408 x 320 x 1408 5.9 / 6.7.
 uint32_t gemm_ring_columns(const GemmArgs &g, int kind) {
   if (kind < 0 || kind > 2) return 0;
@@ -99,11 +104,17 @@ uint32_t gemm_ring_columns(const GemmArgs &g, int kind) {
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
   const uint64_t units = g_compute_units, small = tiles(64, 64), whole = tiles(128, 128);
   if (steps < (kind == 2 ? 13 : 14) || g.m <= 128 || g.n <= 128) return 0;
+  const bool k_lines = g.lda * es % STEP == 0;
   if (small <= 512) {
     if (small <= units) return 0;
-    return tiles(128, 64) <= units ? 64 : 2 * whole > units && steps >= 36 ? 128 : 0;
+    if (tiles(128, 64) <= units) return 64;
+    return 2 * whole > units && steps >= 36 && (k_lines || !g.b_kmajor || kind == 1) ? 128 : 0;
   }
-  if (whole <= units) return 2 * whole > units && steps >= 28 ? 128 : 0;
+  if (whole <= units) {
+    // (i8 of other rows stays for a whole round, whose route tests/test_gpu_matmul_ring_widths.py holds fast for 2048 x 3472 x 2048, 21.4 / 22.5)
+    const bool as_lines = k_lines || gemm_tile_side(g, kind) == 64 || (kind == 0 ? whole == units : kind == 1 || !g.b_kmajor);
+    return 2 * whole > units && steps >= (as_lines ? 28 : kind == 2 ? 32 : 60) ? 128 : 0;
+  }
   if (steps < 16) return 0;
   return tiles(128, 160) <= units ? 160 : tiles(128, 192) <= units ? 192 : 0;
 }

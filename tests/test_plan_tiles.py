@@ -25,3 +25,29 @@ TYPES = {"u8": (M.u8, M.i8, M.i32), "i8": (M.i8, M.i8, M.i32), "bf16": (M.bf16, 
 def test_windows(types, b, c, f, hw, fs, tile):
     p = M.Conv([b, f, c, hw, hw, fs, fs], TYPES[types]).plan()
     assert p.kernels == ["k_gemm"] and tile in p.steps[0].kernel, p
+
+
+KT = M.layout(0, 2, 1)
+
+
+@pytest.mark.parametrize("types,b,m,k,n,nk,tile", [
+    # 128 x 128: rows of K in whole cache lines, and not
+    ("i8", 1, 1985, 3584, 1264, False, "RB = 4, SLOTS"),
+    ("i8", 1, 1985, 3600, 1280, False, "Tile<128, 128"),
+    ("i8", 3, 626, 3584, 2144, True, "RB = 4, SLOTS"),
+    ("i8", 3, 626, 3600, 2144, True, "Tile<128, 128"),
+    ("i8", 3, 626, 3600, 2144, False, "Tile<128, 128"),
+    ("i8", 3, 626, 7600, 2144, False, "RB = 4, SLOTS"),
+    ("i8", 3, 184, 4112, 3664, False, "RB = 4, SLOTS"),    # (the other choice is 64 x 64)
+    ("u8", 3, 626, 3600, 2144, False, "RB = 4, SLOTS"),
+    ("bf16", 2, 1109, 1792, 1504, True, "RB = 4, SLOTS"),
+    ("bf16", 2, 1109, 1768, 1504, True, "Tile<128, 128"),
+    ("bf16", 2, 1109, 1768, 1504, False, "RB = 4, SLOTS"),
+    ("bf16", 2, 1109, 2024, 1504, True, "RB = 4, SLOTS"),
+    ("i8", 1, 814, 7296, 2400, True, "RB = 4, SLOTS"),     # at most 512 tiles of 64 x 64
+    ("i8", 1, 814, 7312, 2400, True, "Tile<64, 64"),
+    ("u8", 1, 814, 7312, 2400, True, "RB = 4, SLOTS"),
+])
+def test_middling_matmuls(types, b, m, k, n, nk, tile):
+    p = M.Matmul([b, m, k, n], TYPES[types], [None, KT if nk else None, None]).plan()
+    assert len(p.steps) == 1 and tile in p.steps[0].kernel, p
