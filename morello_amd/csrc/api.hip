@@ -504,13 +504,28 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   // Rows of whole chunks take that tile by way of LDS alone (gemm_ring.hip), which is the faster one throughout (us, through registers / this: bf16 1024^3 8.0 / 7.0, 33 x
   // 1664 x 12928 10.7 / 9.4, k-fastest B: 86 x 2144 x 262 twice 12.4 / 10.5, u8 693 x 4352 x 817 14.2 / 10.8, 51 x 1600 x 9152 7.4 / 6.2; 1383 x 5744 x 184 in three slices 12.3 / 11.5; over 60
   // random sizes 1.13 times as fast) and faster than k_gemm's from six steps on (192 x 896 x 320 5.05 / 4.55, 384 x 448 x 192 4.6 / 4.2, int8 rows of N over a long K too, 1144 x
-  // 3952 x 672 16.9 / 13.7, 615 x 5760 x 112 twice 21.5 / 13.1), bf16 rows of N from nine (422 x 448 x 880 twice, seven, 5.3 / 5.6; 1005 x 576 x 336 5.2 / 4.7).
+  // 3952 x 672 16.9 / 13.7, 615 x 5760 x 112 twice 21.5 / 13.1), bf16 rows of N from nine (422 x 448 x 880 twice, seven, 5.3 / 5.6; 1005 x 576 x 336 5.2 / 4.7), i8 rows of N
+  // from seven (six, 25 sizes, B from memory: 0.94).  Over a long K of int8 rows of N, slices on k_gemm's 128 tile, which takes whole lines of them, the last a shorter one, are
+  // the faster way where that tile reads B once and this one twice, and where this one runs K in one or two pieces (us, those / this: u8 106 x 9264 x 2960 18.9 / 27.3, i8 262 x
+  // 9584 x 2900 27.5 / 38.5, u8 932 x 13392 x 336 21.3 / 24.7; one set of operands, three, B and all of it from memory, means of 27 to 58 sizes: up to 128 rows, from 57 steps, 0.92 / 0.93 / 0.97 / 0.96; in one
+  // piece past 48 0.98 / 0.98 / 0.85 / 0.83, up to 48 1.14 / 1.11 / 0.96 / 0.91; in two past 80 0.97 / 0.97 / 0.87 / 0.83, 60 to 80 1.09 / 1.09 / 0.98 / 0.95; in more past 80 1.20 / 1.20 / 1.13 / 1.08).
   const int64_t chunk = 16 / int64_t(a.elem);
   const bool ragged = g.lda % chunk != 0 || g.sa % chunk != 0 || g.ldb % chunk != 0 || g.sb % chunk != 0;
   const bool aligned = in_place == 32 && !ragged && g.k % chunk == 0 && mrl::gemm_possible(g, kind);
-  const bool steps_pay = aligned ? uint64_t(g.k) * a.elem > (kind == 2 && !g.b_kmajor ? 8 : 5) * 128 : in_place == 32 && uint64_t(g.k) * a.elem > 8 * 128 && (kind == 2 || g.b_kmajor || g.k <= 24 * 128);
+  const bool steps_pay = aligned ? uint64_t(g.k) * a.elem > (g.b_kmajor || kind == 1 ? 5 : kind == 0 ? 6 : 8) * 128 : in_place == 32 && uint64_t(g.k) * a.elem > 8 * 128 && (kind == 2 || g.b_kmajor || g.k <= 24 * 128);
   uint32_t k_left = 0;
-  if (in_place != 0 && (ragged || few || (steps_pay && (mrl::gemm_k_splits(g, kind, &k_left) == 1 || k_left != 0)))) {
+  auto wide_slices = [&](uint32_t count) {
+    mrl::GemmArgs s = g;
+    s.batch = count, s.k = (g.k - k_left) / count;
+    const uint64_t tiles = uint64_t((g.m + 63) / 64) * ((g.n + 63) / 64);
+    return kind <= 1 && !g.b_kmajor && (g.m <= 128 || 3 * tiles > mrl::g_compute_units) &&
+           g.k > (g.m <= 128 || 2 * tiles > mrl::g_compute_units ? 48 : 80) * 128 && mrl::gemm_tile_side(s, kind) == 128;
+  };
+  auto not_in_k_gemms_slices = [&] {
+    const uint32_t count = mrl::gemm_k_splits(g, kind, &k_left);
+    return count == 1 || (k_left != 0 && !(aligned && wide_slices(count)));
+  };
+  if (in_place != 0 && (ragged || few || (steps_pay && not_in_k_gemms_slices()))) {
     uint32_t slice_k = 0;
     const uint32_t splits = g_tight_scratch ? 1 : mrl::uneven_k_slices(g, kind, false, &slice_k);
     if ((rc = in_slices(splits, slice_k, [&](const mrl::GemmArgs &a) {

@@ -51,3 +51,16 @@ KT = M.layout(0, 2, 1)
 def test_middling_matmuls(types, b, m, k, n, nk, tile):
     p = M.Matmul([b, m, k, n], TYPES[types], [None, KT if nk else None, None]).plan()
     assert len(p.steps) == 1 and tile in p.steps[0].kernel, p
+
+
+@pytest.mark.parametrize("types,m,k,n,kernel", [
+    # Rows of N on the 64 x 64 tile fed straight into LDS, from seven steps of i8, six of u8, nine of bf16
+    ("i8", 193, 768, 208, "k_gemm"), ("i8", 193, 896, 208, "k_gemm_ring"), ("u8", 193, 768, 208, "k_gemm_ring"), ("u8", 193, 640, 208, "k_gemm"),
+    ("bf16", 422, 512, 880, "k_gemm"), ("bf16", 422, 520, 880, "k_gemm_ring"),
+    # Slices of a long K that are not all equal: 230 tiles of 64 x 64, 90 and 75; two rows of tiles
+    ("i8", 262, 9584, 2896, "k_gemm"), ("i8", 262, 6128, 2896, "k_gemm_ring"), ("u8", 932, 13392, 336, "k_gemm"), ("u8", 932, 10128, 336, "k_gemm_ring"),
+    ("i8", 932, 13392, 304, "k_gemm_ring"), ("u8", 106, 9264, 2960, "k_gemm"), ("i8", 77, 11536, 2464, "k_gemm"), ("i8", 66, 9264, 640, "k_gemm_ring"),
+])
+def test_rows_of_n(types, m, k, n, kernel):
+    p = M.Matmul([1, m, k, n], TYPES[types]).plan()
+    assert p.kernels[0] == kernel, p
