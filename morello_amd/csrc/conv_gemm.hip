@@ -39,7 +39,7 @@ hipError_t launch_ring_tile(const GemmArgs &g, hipStream_t stream) {
   const double mn = double(g.m) * g.n * g.batch, steps = double((uint64_t(g.k) * T::ES + ring::STEP - 1) / ring::STEP);
   plan::work(T::ES == 1 ? plan::UNIT_MFMA_I8 : plan::UNIT_MFMA_BF16, 2.0 * mn * g.k,
              double(g.conv.image_bytes) + double(g.n) * (g.k_total ? g.k_total : g.k) * T::ES + mn * 4 * (g.accum ? 2 : 1),
-             2.0 * BM * BN * steps * (ring::STEP / T::ES), 2500.0 + 300.0 * steps);
+             2.0 * BM * BN * steps * (ring::STEP / T::ES), RA * RB > 4 ? 2500.0 + 300.0 * steps : 1300.0 + (T::ES == 2 ? 145.0 : 210.0) * steps);
   const TileWalk walk = gemm::tile_walk(tiles_m, tiles_n);
   MRL_LAUNCH((k_gemm<T, A_UNSIGNED, RA, RB, CONV, SLOTS>), dim3(tiles_m * tiles_n, g.batch), dim3(64 * ring::WAVES), LDS, stream, MRL_WALK_ARGS(walk), g);
   return plan::last_error();

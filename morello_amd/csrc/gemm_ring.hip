@@ -52,7 +52,7 @@ hipError_t launch_ring(const GemmArgs &g, hipStream_t stream) {
   const double mn = double(g.m) * g.n * g.batch, steps = double((uint64_t(g.k) * T::ES + STEP - 1) / STEP);
   plan::work(T::ES == 1 ? plan::UNIT_MFMA_I8 : plan::UNIT_MFMA_BF16, 2.0 * mn * g.k,
              (double(g.m) * g.k + double(g.k) * g.n) * g.batch * T::ES + mn * (g.c_bf16 ? 2 : 4) * (g.accum ? 2 : 1),
-             2.0 * BM * BN * steps * (STEP / T::ES), 2500.0 + 300.0 * steps);
+             2.0 * BM * BN * steps * (STEP / T::ES), RA * RB > 4 ? 2500.0 + 300.0 * steps : 900.0 + (B_KMAJOR ? (T::ES == 2 ? 155.0 : 185.0) : T::ES == 2 ? 220.0 : 275.0) * steps);
   const TileWalk walk = gemm::tile_walk(tiles_m, tiles_n);
   MRL_LAUNCH((k_gemm_ring<T, A_UNSIGNED, B_KMAJOR, RA, RB, SLOTS>), dim3(tiles_m * tiles_n, g.batch), dim3(64 * WAVES), LDS, stream, MRL_WALK_ARGS(walk), g);
   return plan::last_error();
