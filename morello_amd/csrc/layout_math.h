@@ -94,7 +94,9 @@ inline bool make_layout_eval(const mrl_layout &l, const uint32_t *shape, uint32_
     ev->psize[i] = phys[i];
     ev->mod[i] = prev != shape[ld] ? prev : 0;
     ev->next[i] = next;
-    ev->oddeven[i] = l.dims[i].kind == MRL_ODDEVEN;
+    // (A strip that is one element, inside it what other dims of the logical dim hold, has no odd ones: taken as a strip all the same, those
+    // would go past the buffer: [1, 1o4, 1p2] over two elements has offsets 0 and 3.)
+    ev->oddeven[i] = l.dims[i].kind == MRL_ODDEVEN && phys[i] != 1;
     ev->strip[i] = l.dims[i].size;
     ev->divide[i] = ev->oddeven[i] || shape[ld] != phys[i];
   }
