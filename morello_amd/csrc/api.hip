@@ -499,7 +499,8 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   // Rows that are not whole 16-byte chunks, in a problem small enough that copies of them would be a third of its time: read
   // in place too.  And any rows where its smallest tile steps through K faster than k_gemm's (0.25 to 0.33 us against 0.4 to 0.5:
   // u8 1144 x 3952 x 672 16.2 / 13.6, bf16 221 x 1824 x 624 twice 12.9 / 11.2; up to eight steps they are even), unless K falls
-  // into equal slices, of which k_gemm's may go three to a compute unit (bf16 1721 x 4416 x 304 15.4 / 21.0), or is long beside
+  // into equal slices, of which k_gemm's may go three to a compute unit (bf16 1721 x 4416 x 304 15.8 / 18.9; the line is the tile's through registers, on the one below 512 x
+  // 4096 x 512 12.7 / 11.1, 256 x 2048 x 1024 8.8 / 8.7, u8 512 x 4096 x 512 10.6 / 10.1), or is long beside
   // int8 rows of N, of which a step takes half lines (139 x 4080 x 2288 twice 22.6 / 23.5).
   // Rows of whole chunks take that tile by way of LDS alone (gemm_ring.hip), which is the faster one throughout (us, through registers / this: bf16 1024^3 8.0 / 7.0, 33 x
   // 1664 x 12928 10.7 / 9.4, k-fastest B: 86 x 2144 x 262 twice 12.4 / 10.5, u8 693 x 4352 x 817 14.2 / 10.8, 51 x 1600 x 9152 7.4 / 6.2; 1383 x 5744 x 184 in three slices 12.3 / 11.5; over 60

@@ -19,7 +19,8 @@ hipError_t launch_for(const GemmArgs &g, uint32_t tile, hipStream_t stream) {
   return launch<T, A_UNSIGNED, TileBig, true, true, true>(g, stream);
 }
 
-// The tiles of gemm_ring_tile.h on windows: 32 RA pixels by 32 RB filters on eight waves, two to a SIMD, each with half of every step.
+// The tiles of gemm_ring_tile.h on windows: 32 RA pixels by 32 RB filters on eight waves, two to a SIMD, each with
+// half of every step.
 template <class T, bool A_UNSIGNED, int RA, int RB, bool CONV, int SLOTS>
 __global__ __launch_bounds__(64 * ring::WAVES, RA * RB <= 8 ? 4 : 2) void k_gemm(MRL_WALK_PARAMS, GemmArgs g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
@@ -45,29 +46,39 @@ hipError_t launch_ring_tile(const GemmArgs &g, hipStream_t stream) {
   return plan::last_error();
 }
 
-// Where those tiles are the faster ones.  A launch's time is taken as a fixed part and, for every round of its workgroups over the compute
-// units, the steps of a workgroup (128 bytes of the windows).  Measured (us; a step and round, int8 / bf16):
-//   these tiles: 64 x 32 3.5 + 0.25 / 0.24 (a single round 0.18 / 0.13), 64 x 64 3.5 + 0.26 / 0.25 (0.22 / 0.15), 128 x 32 4 + 0.30 / 0.29, 128 x 64 4.5 + 0.31 /
-//     0.32 (a single round of bf16 0.25), 128 x 128 5.5 + 0.48 / 0.50, 128 x 192 6.5 + 0.66 / 0.67; int8 past one round of the last two 0.66 and 0.89, to one and a half
-//     of 128 x 64 0.43, and the same beside the 256 x 256 tile: nothing is under way while a round's results leave, which a short int8 step does not make up for
-//     (u8 18 x (208 -> 240) x 71^2 3 x 3 74.5 / 91.3, 18 x (176 -> 192) x 79^2 65.1 / 73.1, 22 x (208 -> 64) x 46^2 15.6 / 17.7, 16 x (112 -> 160) x 55^2 20.8 / 25.1),
+// Where those tiles are the faster ones.  A launch's time is taken as a fixed part and, for every round of its
+// workgroups over the compute units, the steps of a workgroup (128 bytes of the windows).  Measured (us; a step and
+// round, int8 / bf16):
+//   these tiles: 64 x 32 3.5 + 0.25 / 0.24 (a single round 0.18 / 0.13), 64 x 64 3.5 + 0.26 / 0.25 (0.22 / 0.15), 128
+//     x 32 4 + 0.30 / 0.29, 128 x 64 4.5 + 0.31 / 0.32 (a single round of bf16 0.25), 128 x 128 5.5 + 0.48 / 0.50,
+//     128 x 192 6.5 + 0.66 / 0.67; int8 past one round of the last two 0.66 and 0.89, to one and a half of 128 x 64
+//     0.43, and the same beside the 256 x 256 tile: nothing is under way while a round's results leave, which a short
+//     int8 step does not make up for (u8 18 x (208 -> 240) x 71^2 3 x 3 74.5 / 91.3, 18 x (176 -> 192) x 79^2 65.1 /
+//     73.1, 22 x (208 -> 64) x 46^2 15.6 / 17.7, 16 x (112 -> 160) x 55^2 20.8 / 25.1),
 //   k_gemm's: 64 3.5 + 0.30 / 0.245, 128 4 + 0.69 / 0.57, 256 5 + 2.15 / 1.83;
-// past the third round those of which several share a unit even out the last one.  What bounds a single round is the wait for what the step after next
-// asked of memory, past one the way into LDS.  (us, k_gemm / this: bf16 12 x (352 -> 192) x 68^2 5 x 5 265.7 / 190.5, u8 18 x (272 -> 192) x 42^2 5 x 5 101.9 /
-// 55.2, 9 x (224 -> 304) x 27^2 5 x 5 33.0 / 27.1, 5 x (144 -> 112) x 64^2 5 x 5 23.1 / 19.4, bf16 11 x (144 -> 208) x 14^2 3 x 3 10.3 / 7.5.  Windows by way of
-// registers, two slots of LDS / straight to LDS, three or four: bf16 21 x (144 -> 64) x 17^2 3 x 3 7.5 / 6.4, 2 x (96 -> 48) x 69^2 6.3 / 5.6, u8 31 x (240 -> 144) x
-// 14^2 5 x 5 23.2 / 19.6, 1 x (64 -> 48) x 21^2 5 x 5 6.1 / 5.7; over 140 random layers 1.035 times as fast, no one slower.)
-// Up to three steps, two of them what the start of a workgroup fetches, and up to seven past one round, k_gemm's start is the shorter one: u8 4 x
-// (16 -> 176) x 57^2 3 x 3, two steps, 5.7 / 7.4; 28 x (48 -> 336) x 11^2, four, 318 tiles, 5.7 / 6.3.  But for its 256 x 256 tile, whose end is the longer one:
-// 7 x (16 -> 272) x 72^2 3 x 3, two steps, 27.6 / 19.1, bf16 17 x (16 -> 176) x 70^2 5 x 5, seven, 36.6 / 28.7.  Of int8 where that tile pads the filters half as much again
-// (without, 22 x (16 -> 176) x 114^2 3 x 3 61.4 / 84.4, 22 x (48 -> 208) x 40^2 15.3 / 19.1), and not for two steps past fourteen rounds, which the results bound
-// (27 x (16 -> 288) x 71^2 53.0 / 60.9).
+// past the third round those of which several share a unit even out the last one.  What bounds a single round is the
+// wait for what the step after next asked of memory, past one the way into LDS.  (us, k_gemm / this: bf16 12 x (352
+// -> 192) x 68^2 5 x 5 265.7 / 190.5, u8 18 x (272 -> 192) x 42^2 5 x 5 101.9 / 55.2, 9 x (224 -> 304) x 27^2 5 x 5
+// 33.0 / 27.1, 5 x (144 -> 112) x 64^2 5 x 5 23.1 / 19.4, bf16 11 x (144 -> 208) x 14^2 3 x 3 10.3 / 7.5.  Windows by
+// way of registers, two slots of LDS / straight to LDS, three or four: bf16 21 x (144 -> 64) x 17^2 3 x 3 7.5 / 6.4,
+// 2 x (96 -> 48) x 69^2 6.3 / 5.6, u8 31 x (240 -> 144) x 14^2 5 x 5 23.2 / 19.6, 1 x (64 -> 48) x 21^2 5 x 5 6.1 /
+// 5.7; over 140 random layers 1.035 times as fast.)
+// Few steps leave the start and the end of a workgroup, and k_gemm's are the shorter ones (us, k_gemm / 64 x 64 or
+// 128 x 64 of these, whichever is the faster): one step, whatever the number of tiles, u8 4 x (32 -> 128) x 28^2 2 x
+// 2 3.3 / 3.9, bf16 8 x (8 -> 128) x 40^2 2 x 2 3.6 / 5.2; up to three in one round, where it is even at the last (u8
+// 2 x (32 -> 64) x 28^2 3 x 3 4.0 / 4.1), u8 4 x (16 -> 176) x 57^2 3 x 3, two, 6.0 / 7.7; up to seven past one, 28 x
+// (48 -> 336) x 11^2, four, 5.8 / 6.1, bf16 30 x (32 -> 96) x 18^2, five, 5.1 / 5.5, 20 x (16 -> 128) x 28^2, three,
+// 4.7 / 5.9.  But for its 256 x 256 tile, whose end is the longer one: u8 7 x (16 -> 272) x 72^2 3 x 3, two steps,
+// 27.6 / 19.1, bf16 17 x (16 -> 176) x 70^2 5 x 5, seven, 36.6 / 28.7.
+// Of int8 where that tile pads the filters half as much again (without, 22 x (16 -> 176) x 114^2 3 x 3 61.4 / 84.4,
+// 22 x (48 -> 208) x 40^2 15.3 / 19.1), and not for two steps past fourteen rounds, which the results bound (27 x (16
+// -> 288) x 71^2 53.0 / 60.9).
 enum Tiles : uint32_t { SQUARE, T64x32, T64x64, T128x32, T128x64, T128x128, T128x192 };
 Tiles choose_tiles(const GemmArgs &g, int kind) {
   if (kind > 2) return SQUARE;
   const uint64_t es = kind == 2 ? 2 : 1, step = ring::STEP, steps = (uint64_t(g.k) * es + step - 1) / step;
   const uint64_t last = g.k_total != 0 ? g.k_total - uint64_t(g.batch - 1) * g.k : g.k;
-  if (last * es <= step) return SQUARE;   // (a step has no successor to fetch)
+  if (last * es <= step) return SQUARE;
   const uint64_t units = g_compute_units;
   auto tiles = [&](uint32_t bm, uint32_t bn) { return uint64_t((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn) * g.batch; };
   const uint64_t small = tiles(64, 64);

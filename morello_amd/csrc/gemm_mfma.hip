@@ -123,24 +123,33 @@ uint32_t uneven_k_slices(const GemmArgs &g, int kind, bool conv, uint32_t *slice
   uint64_t per = (steps + wanted - 1) / wanted;
   while (k_bytes % (per * 128) != 0 && k_bytes % (per * 128) <= 128) per++;   // (gemm_ring_rows.hip wants two steps or more)
   const uint64_t count = (steps + per - 1) / per;
-  // (Rows that start anywhere: one workgroup a compute unit, 292 x 6007 x 2192 bf16 in halves, 350 of them, 43.6 us, whole 35.)
+  // (Rows that start anywhere: one workgroup a compute unit, 292 x 6007 x 2192 bf16 in halves, 350 of them, 43.6 us,
+  // whole 35.)
   // As in gemm_k_splits, with the step of each kernel and type (Conv: a chain of 66 int8 steps 30 us, of 107 bf16
   // steps 40) and the partials' traffic at the 3 TB/s that a sum of a few MB reaches: 2 x (48 -> 144) x 43^2 5 x 5
-  // bf16, 174 tiles of 19 steps, 9.7 us whole, 11.4 in halves; 3 x (144 -> 128) x 34^2 3 x 3, 110
-  // of 21, 10.2 and 11.1; 10 x (80 -> 64) x 19^2 5 x 5, 57 of 32, 14.2 and 9.5 in four.
+  // bf16, 174 tiles of 19 steps, 9.7 us whole, 11.4 in halves; 3 x (144 -> 128) x 34^2 3 x 3, 110 of 21, 10.2 and
+  // 11.1; 10 x (80 -> 64) x 19^2 5 x 5, 57 of 32, 14.2 and 9.5 in four.
+  // These are the times of tiles that went through registers.  Straight into LDS a single round's step takes 0.13 to
+  // 0.22 us (conv_gemm.hip, gemm_ring.hip), so that slices save half of what is reckoned here and cost the same.  (us
+  // now, in these slices / whole: bf16 1 x (352 -> 64) x 10^2 3 x 3 in six 6.7 / 10.3, 1 x (272 -> 64) x 14^2 5 x 5
+  // in twelve 7.1 / 18.5; 1 x (128 -> 64) x 30^2 in two 6.9 / 6.0, 10 x (80 -> 64) x 19^2 5 x 5 in four 8.9 / 8.2, 24
+  // x (320 -> 320) x 10^2 in three 18.2 / 11.3, u8 16 x (112 -> 16) x 26^2 5 x 5 in two 11.5 / 8.0.)
   const double spread = std::min<double>(double(count), (conv ? 384.0 : 256.0) / double(tiles));
   const double saved_us = double(steps) * (1.0 - 1.0 / spread) * (!conv ? 0.28 : kind == 2 ? 0.36 : 0.46);
   const double cost_us = 2.2 + (double(count) + 1.0) * double(g.m) * double(g.n) * 4.0 / 3.0e6;
   bool pays = spread > 1.0 && saved_us >= 1.2 * cost_us;
   if (conv) {
-    // int8 in two slices of eight steps, over half of the units and more in one piece already: 10 x (224 -> 16) x 33^2 3 x 3, 171 tiles of
-    // 16 steps, 9.6 us whole, 10.2 in halves, 14 x (240 -> 16) x 30^2, 197 of 17, 10.4 and 11.0 (16 x (112 -> 16) x 26^2 5 x 5, 169 of 22, 12.0 and 11.5).
+    // int8 in two slices of eight steps, over half of the units and more in one piece already: 10 x (224 -> 16) x
+    // 33^2 3 x 3, 171 tiles of 16 steps, 9.6 us whole, 10.2 in halves, 14 x (240 -> 16) x 30^2, 197 of 17, 10.4 and
+    // 11.0 (16 x (112 -> 16) x 26^2 5 x 5, 169 of 22, 12.0 and 11.5).
     if (kind <= 1 && tiles > 128 && steps < 18) pays = false;
-    // Equal slices where there are about as many (they end together), and where the above finds none worth it, which has the steps
-    // too short for them (up to 0.5 us each), for long chains or few results: us, whole or in so many uneven ones / equal: bf16 24 x (320 -> 320) x 10^2 3 x 3, 190
-    // tiles of 45 steps, 22.9 / 17.7 in three, 4 x (256 -> 288) x 24^2 18.8 / 15.1, 14 x (384 -> 112) x 26^2 28.0 / 26.4, 9 x (192 -> 96) x 24^2, 27 steps,
-    // 14.8 / 12.2; 18 steps in two 4 x (128 -> 208) x 15^2, 187 thousand results, 10.7 / 9.6, 5 x (128 -> 48) x 40^2, 384 thousand, 10.7 / 10.8; 3 x (384 -> 160) x
-    // 15^2 5 x 5, 13.0 in 17 / 12.1 in 15; fewer of them: 5 x (320 -> 112) x 11^2 5 x 5 14 / 5, 1.45 times as long.
+    // (As measured then.)  Equal slices where there are about as many (they end together), and where the above finds
+    // none worth it, which has the steps too short for them (up to 0.5 us each), for long chains or few results: us,
+    // whole or in so many uneven ones / equal: bf16 24 x (320 -> 320) x 10^2 3 x 3, 190 tiles of 45 steps, 22.9 /
+    // 17.7 in three, 4 x (256 -> 288) x 24^2 18.8 / 15.1, 14 x (384 -> 112) x 26^2 28.0 / 26.4, 9 x (192 -> 96) x
+    // 24^2, 27 steps, 14.8 / 12.2; 18 steps in two 4 x (128 -> 208) x 15^2, 187 thousand results, 10.7 / 9.6, 5 x
+    // (128 -> 48) x 40^2, 384 thousand, 10.7 / 10.8; 3 x (384 -> 160) x 15^2 5 x 5, 13.0 in 17 / 12.1 in 15; fewer of
+    // them: 5 x (320 -> 112) x 11^2 5 x 5 14 / 5, 1.45 times as long.
     const uint32_t equal = gemm_k_splits(g, kind);
     if (equal > 1 && (pays ? 8 * equal >= 7 * count : steps >= 27 || (steps >= 18 && uint64_t(g.m) * g.n < 350000))) {
       *slice_k = g.k / equal;

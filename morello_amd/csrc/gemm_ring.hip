@@ -62,10 +62,11 @@ template <class T, bool A_UNSIGNED, int RA, int RB, int SLOTS>
 hipError_t launch_either(const GemmArgs &g, hipStream_t stream) {
   return g.b_kmajor ? launch_ring<T, A_UNSIGNED, true, RA, RB, SLOTS>(g, stream) : launch_ring<T, A_UNSIGNED, false, RA, RB, SLOTS>(g, stream);
 }
-// As many slots as a compute unit's LDS holds of the wider ones, and four of the 64-wide tile's as well: all run one to a unit (of the
-// last, three / four / six: bf16 1024 x 7040 x 1344 35.7 / 33.2 / 33.4 us, 1664 x 6720 x 1152 34.6 / 33.0 / 33.2; of 128, five instead of four are within 1 %).  Four of the 64 x 64
-// tile, two of which share a unit (us, three / four / six / eight: bf16 192 x 768 x 384 4.74 / 4.81 / 4.9 / 5.2, 313 x 2176 x 267 twice 10.7 / 9.3 / 9.2 /
-// 9.5, u8 600 x 2496 x 236 7.3 / 7.3 / 7.6 / 7.9, 693 x 4352 x 817 with a k-fastest B 11.9 / 10.8).
+// As many slots as a compute unit's LDS holds of the wider ones, and four of the 64-wide tile's as well: all run one
+// to a unit (of the last, three / four / six: bf16 1024 x 7040 x 1344 35.7 / 33.2 / 33.4 us, 1664 x 6720 x 1152 34.6
+// / 33.0 / 33.2; of 128, five instead of four are within 1 %).  Four of the 64 x 64 tile, two of which share a unit
+// (us, three / four / six / eight: bf16 192 x 768 x 384 4.74 / 4.81 / 4.9 / 5.2, 313 x 2176 x 267 twice 10.7 / 9.3 /
+// 9.2 / 9.5, u8 600 x 2496 x 236 7.3 / 7.3 / 7.6 / 7.9, 693 x 4352 x 817 with a k-fastest B 11.9 / 10.8).
 template <class T, bool A_UNSIGNED>
 hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
   switch (bn) {
@@ -80,24 +81,32 @@ hipError_t launch_kind(const GemmArgs &g, uint32_t bn, hipStream_t stream) {
 
 }  // namespace
 
-// Measured against k_gemm's tiles (us, k_gemm / this; means of 520 random sizes, of three sets of operands in turn), on rounds of one
-// tile per compute unit:
+// Measured against k_gemm's tiles (us, k_gemm / this; means of 520 random sizes, of three sets of operands in turn),
+// on rounds of one tile per compute unit:
 //   64 where k_gemm's 64 tile would go two to a unit (257 of them on) and this one at most one: bf16 1100 x 3001 x
-//     1100 35.1 / 28.0, u8 1408 x 3001 x 1408 23.6 / 20.9; two to a unit it loses (400 x 3001 x 4400 35.7 / 46.4).  bf16 from 13
-//     steps on (13 to 15 1.13 times as fast, 1.11 with operands from memory; 11 and 12 1.05 and from memory 0.85 at the least, nine and ten 1.02 and
-//     0.91), integers from 14 (14 to 16 1.11, from memory 1.09; 11 to 13 1.04 and 0.97, seven and eight 0.98);
-//   128 for more than half a round of 128 x 128.  Integers from 28 steps on: 4054 x 4352 x 832 26.6 / 24.1 (28 and 29 1.07, 30 to 34 1.06, from memory
-//     1.03; 23 to 25 1.02 and from memory 0.97, 11 to 16 0.94).  bf16 too: 2048^3 22.9 / 22.2 (28 and 29 1.04, 30 to 34 1.09, from memory 1.07;
-//     23 to 26 1.06, but 0.93 for one in six; 9 to 16 0.95).  Where 64 x 64 tiles are 512 at most, which k_gemm runs two to a unit, both from 36
-//     (integers 35 to 44 1.08, bf16 45 on 1.22; 30 to 34 1.02 and from memory 0.95, 11 to 19 0.89);
-//   160, else 192, where the 128 tile needs a second round and they do not: bf16 1001 x 2050 x 4425 47.2 / 38.9, 1800 x 2001
-//     x 3000 41.0 / 35.3, u8 1000 x 2001 x 4500 34.6 / 30.1.  (128 in two rounds: 0.92 to 1.03, and 0.90 with operands from memory.)
-// Rows of K that are no whole cache lines, of which a step's 128 bytes lie in two, cost the 128-wide tile that much more than k_gemm's: i8 from 60 steps on, a
-// k-fastest bf16 B from 32, and where 64 x 64 tiles are 512 at most a k-fastest B of either not at all (one set of operands / three in turn / B from memory /
-// all of it, means: i8 below 60 0.97 / 0.96 / 0.96 / 0.93, from there 1.02 / 1.01 / 1.00 / 0.96, of whole lines 1.09 / 1.09 / 1.04 / 0.99; bf16 0.93 / 0.94 / 0.94 / 0.92,
-// of whole lines 1.09 / 1.09 / 1.04 / 1.00; i8 883 x 4928 x 2336 26.0 / 27.0, twice 792 x 3552 x 1760 21.7 / 24.6, bf16 twice 1109 x 1768 x 1504 21.1 / 23.5).  u8 pays k_gemm
-// for its columns' sums (1.04 / 1.04 / 1.03 / 1.00).  Where 128 x 128 pads much more than 64 x 64 the other choice is k_gemm's 64 tile, 1.8 times as slow.
-// Short K leaves the start of the ring and the summing of the two halves of K dominant: bf16 1408 x 320 x 1408 5.9 / 6.7.
+//     1100 35.1 / 28.0, u8 1408 x 3001 x 1408 23.6 / 20.9; two to a unit it loses (400 x 3001 x 4400 35.7 / 46.4).
+//     bf16 from 13 steps on, integers from 14 (335 sizes up to 15, one set of operands / three in turn / B from
+//     memory / all of it: rows of whole cache lines 1.23 / 1.11 / 1.11 / 1.04, others of a k-fastest B 1.16 / 1.04 /
+//     1.04 / 0.97, of a row-major one 1.11 / 1.02 / 1.00 / 0.93; bf16 of 11 and 12 1.05 and from memory 0.85 at the
+//     least, integers of 11 to 13 1.04 and 0.97);
+//   128 for more than half a round of 128 x 128.  Integers from 28 steps on: 4054 x 4352 x 832 26.6 / 24.1 (28 and 29
+//     1.07, 30 to 34 1.06, from memory 1.03; 23 to 25 1.02 and from memory 0.97, 11 to 16 0.94).  bf16 too: 2048^3
+//     22.9 / 22.2 (28 and 29 1.04, 30 to 34 1.09, from memory 1.07; 23 to 26 1.06, but 0.93 for one in six; 9 to 16
+//     0.95).  Where 64 x 64 tiles are 512 at most, which k_gemm runs two to a unit, both from 36 (integers 35 to 44
+//     1.08, bf16 45 on 1.22; 30 to 34 1.02 and from memory 0.95, 11 to 19 0.89);
+//   160, else 192, where the 128 tile needs a second round and they do not: bf16 1001 x 2050 x 4425 47.2 / 38.9, 1800
+//     x 2001 x 3000 41.0 / 35.3, u8 1000 x 2001 x 4500 34.6 / 30.1.  (128 in two rounds: 0.92 to 1.03, and 0.90 with
+//     operands from memory.)
+// Rows of K that are no whole cache lines, of which a step's 128 bytes lie in two, cost the 128-wide tile that much
+// more than k_gemm's: i8 from 60 steps on, a k-fastest bf16 B from 32, and where 64 x 64 tiles are 512 at most a
+// k-fastest B of either not at all (one set of operands / three in turn / B from memory / all of it, means: i8 below
+// 60 0.97 / 0.96 / 0.96 / 0.93, from there 1.02 / 1.01 / 1.00 / 0.96, of whole lines 1.09 / 1.09 / 1.04 / 0.99; bf16
+// 0.93 / 0.94 / 0.94 / 0.92, of whole lines 1.09 / 1.09 / 1.04 / 1.00; i8 883 x 4928 x 2336 26.0 / 27.0, twice 792 x
+// 3552 x 1760 21.7 / 24.6, bf16 twice 1109 x 1768 x 1504 21.1 / 23.5).  u8 pays k_gemm for its columns' sums (1.04 /
+// 1.04 / 1.03 / 1.00).  Where 128 x 128 pads much more than 64 x 64 the other choice is k_gemm's 64 tile, 1.8 times
+// as slow.
+// Short K leaves the start of the ring and the summing of the two halves of K dominant: bf16 1408 x 320 x 1408 5.9 /
+// 6.7.
 uint32_t gemm_ring_columns(const GemmArgs &g, int kind) {
   if (kind < 0 || kind > 2) return 0;
   const uint64_t es = kind == 2 ? 2 : 1, steps = (uint64_t(g.k) * es + STEP - 1) / STEP;
@@ -111,7 +120,8 @@ uint32_t gemm_ring_columns(const GemmArgs &g, int kind) {
     return 2 * whole > units && steps >= 36 && (k_lines || !g.b_kmajor || kind == 1) ? 128 : 0;
   }
   if (whole <= units) {
-    // (i8 of other rows stays for a whole round, whose route tests/test_gpu_matmul_ring_widths.py holds fast for 2048 x 3472 x 2048, 21.4 / 22.5)
+    // (i8 of other rows stays for a whole round, whose route tests/test_gpu_matmul_ring_widths.py holds fast for 2048
+    // x 3472 x 2048, 21.4 / 22.5)
     const bool as_lines = k_lines || gemm_tile_side(g, kind) == 64 || (kind == 0 ? whole == units : kind == 1 || !g.b_kmajor);
     return 2 * whole > units && steps >= (as_lines ? 28 : kind == 2 ? 32 : 60) ? 128 : 0;
   }

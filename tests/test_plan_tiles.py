@@ -31,6 +31,17 @@ KT = M.layout(0, 2, 1)
 
 
 @pytest.mark.parametrize("types,b,m,k,n,nk,tile", [
+    # 128 x 64 and 128 x 128 of row-major operands, the last column of tiles 8 or 16 wide
+    ("bf16", 1, 1153, 832, 904, False, "RB = 2, SLOTS"),
+    ("bf16", 1, 1153, 768, 904, False, "Tile<64, 64"),
+    ("bf16", 2, 1153, 776, 456, False, "RB = 2, SLOTS"),
+    ("u8", 2, 1153, 1680, 464, False, "RB = 2, SLOTS"),
+    ("u8", 2, 1153, 1664, 464, False, "Tile<64, 64"),
+    ("bf16", 1, 1985, 1792, 1160, False, "RB = 4, SLOTS"),
+    ("bf16", 1, 1985, 1728, 1160, False, "Tile<128, 128"),
+    ("u8", 1, 1985, 3584, 1168, False, "RB = 4, SLOTS"),
+    ("u8", 1, 1985, 3456, 1168, False, "Tile<128, 128"),
+    ("u8", 3, 300, 4608, 1808, False, "RB = 4, SLOTS"),
     # 128 x 128: rows of K in whole cache lines, and not
     ("i8", 1, 1985, 3584, 1264, False, "RB = 4, SLOTS"),
     ("i8", 1, 1985, 3600, 1280, False, "Tile<128, 128"),
