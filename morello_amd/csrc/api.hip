@@ -524,7 +524,7 @@ int run_matmul(const mrl_spec &s, void *const *params, Workspace &ws,
   };
   auto not_in_k_gemms_slices = [&] {
     const uint32_t count = mrl::gemm_k_splits(g, kind, &k_left);
-    return count == 1 || (k_left != 0 && !(aligned && wide_slices(count)));
+    return count == 1 || (k_left != 0 && !(aligned && !g_tight_scratch && wide_slices(count)));
   };
   if (in_place != 0 && (ragged || few || (steps_pay && not_in_k_gemms_slices()))) {
     uint32_t slice_k = 0;
